@@ -42,7 +42,8 @@ enum mdcn_dtype {
 
 /* Which device path runs. */
 enum mdcn_path {
-  MDCN_PATH_AUTO = 0,   /* fused MFMA kernel when the shape allows, else direct */
+  MDCN_PATH_AUTO = 0,   /* fused MFMA kernel when the shape allows, else the segment kernel (see
+                           mdcn_workspace_wanted()), else direct */
   MDCN_PATH_FUSED = 1,  /* fused implicit-GEMM MFMA kernel; error if not eligible */
   MDCN_PATH_DIRECT = 2, /* one thread per output element; any shape */
   MDCN_PATH_FUSED_SPLIT = 3, /* forward only: as MDCN_PATH_FUSED, but always the fused kernel with specialised
@@ -151,7 +152,7 @@ int mdcn_fused_eligible(const mdcn_params *p);
 /* Which device kernels mdcn_forward() launches for the main stage of the call described by *p (shape,
  * dtype, path, no_k_split; of the pointers only `input` and `output` are looked at, for their alignment):
  * a static string such as "fused3_kernel", "fused3_kernel+fused2_kernel", "fused2_kernel", "fused_kernel",
- * "direct_kernel", "f64_forward_kernel"; "" for an invalid *p.  The first name is the kernel that does
+ * "segment_kernel" (given the scratch of mdcn_workspace_wanted()), "direct_kernel", "f64_forward_kernel"; "" for an invalid *p.  The first name is the kernel that does
  * most of the work.  For reports and tests (no counterpart in the reference). */
 const char *mdcn_forward_kernels(const mdcn_params *p);
 
@@ -166,6 +167,13 @@ const char *mdcn_forward_kernels(const mdcn_params *p);
  * is accepted too and only runs that last round unshared.  Returns 0 for an invalid *p
  * (mdcn_forward then reports the error). */
 size_t mdcn_workspace_bytes(const mdcn_params *p);
+
+/* Bytes of device scratch with which mdcn_forward() runs its fastest kernels: at least
+ * mdcn_workspace_bytes().  It is more for shapes the fused path does not cover (channels of
+ * a deformable group that do not fill 128 bytes, say): with this much scratch a matrix-core kernel
+ * made for them runs on a re-laid copy of the input, with less the one-thread-per-output
+ * kernel, which needs none. */
+size_t mdcn_workspace_wanted(const mdcn_params *p);
 
 /* Enqueue the forward on `hip_stream` (a hipStream_t; NULL = the null stream).
  * Returns an mdcn_status.  Replaces the body of

@@ -21,7 +21,7 @@ EXT_LIB = os.path.join(PKG, '_ext' + sysconfig.get_config_var('EXT_SUFFIX'))
 ROCM = os.environ.get('ROCM_PATH', '/opt/rocm')
 
 HIPCC_FLAGS = [
-    '--offload-arch=gfx950', '-O3', '-std=c++17', '-fPIC', '-shared',
+    '--offload-arch=gfx950', '-O3', '-std=c++17', '-fPIC',
     # packed-fp32 VALU forms are kept out of the generated code
     '-Xclang', '-target-feature', '-Xclang', '-packed-fp32-ops',
     # '#pragma unroll' loops whose bodies index register arrays must unroll whatever their size
@@ -30,41 +30,52 @@ HIPCC_FLAGS = [
 ]
 
 
-def _run(cmd):
+def _run(cmd, cwd=None):
     print(' '.join(cmd), flush=True)
-    subprocess.check_call(cmd)
+    subprocess.check_call(cmd, cwd=cwd)
+
+
+SOURCES = ['mdcn_api.hip', 'mdcn_segment.hip']
 
 
 def build_hip(extra=(), check=True):
-    """Compile the library; with `check`, keep the device assembly of the compile
-    and scan it (asm_check.py) before the library is accepted."""
+    """Compile the library, its sources side by side; with `check`, keep the device
+    assembly of the compile and scan it (asm_check.py) before the library is accepted."""
     import shutil
     import tempfile
+    from concurrent.futures import ThreadPoolExecutor
     os.makedirs(LIBDIR, exist_ok=True)
     hipcc = os.path.join(ROCM, 'bin', 'hipcc')
     cmd = [hipcc, *HIPCC_FLAGS, *extra, '-I', os.path.join(ROOT, 'include')]
-    src = os.path.join(CSRC, 'mdcn_api.hip')
-    if not check:
-        _run([*cmd, '-o', HIP_LIB, src])
-        return HIP_LIB
-    from . import asm_check
     tmp = tempfile.mkdtemp(prefix='mdcn_build_')
+
+    def compile_one(name):
+        obj = os.path.join(tmp, name + '.o')
+        _run([*cmd, *(['-save-temps=obj'] if check else []), '-c', '-o', obj, os.path.join(CSRC, name)], cwd=tmp)
+        return obj
+
     try:
+        with ThreadPoolExecutor(min(8, len(SOURCES))) as pool:
+            objs = list(pool.map(compile_one, SOURCES))
+        asm = []
+        if check:
+            from . import asm_check
+            asm = sorted(os.path.join(tmp, f) for f in os.listdir(tmp) if f.endswith('.s') and 'gfx950' in f)
+            if len(asm) != len(SOURCES):
+                raise RuntimeError('no device assembly found to check')
+            bad = sum(asm_check.check_file(f) for f in asm)
+            if bad:
+                raise RuntimeError(f'{bad} finding(s) in the device assembly around inline-asm memory instructions '
+                                   '(see above and asm_check.py)')
+            print(f'asm_check: {len(asm)} device assembly file(s) clean', flush=True)
         out = os.path.join(tmp, 'libmdcn_hip.so')
-        print(' '.join([*cmd, '-save-temps=obj', '-o', out, src]), flush=True)
-        subprocess.check_call([*cmd, '-save-temps=obj', '-o', out, src], cwd=tmp)
-        asm = [os.path.join(tmp, f) for f in os.listdir(tmp) if f.endswith('.s') and 'gfx950' in f]
-        if not asm:
-            raise RuntimeError('no device assembly found to check')
-        bad = sum(asm_check.check_file(f) for f in asm)
-        if bad:
-            raise RuntimeError(f'{bad} finding(s) in the device assembly around inline-asm memory instructions '
-                               '(see above and asm_check.py)')
-        print(f'asm_check: {len(asm)} device assembly file(s) clean', flush=True)
+        _run([hipcc, '--offload-arch=gfx950', '-shared', '-o', out, *objs])
         shutil.move(out, HIP_LIB)
         # the assembly the library was built from stays beside it (git-ignored): tests scan it again
-        for f in asm:
-            shutil.copy(f, os.path.join(LIBDIR, 'libmdcn_hip.s' if len(asm) == 1 else os.path.basename(f)))
+        if asm:
+            with open(os.path.join(LIBDIR, 'libmdcn_hip.s'), 'w') as f:
+                for part in asm:
+                    f.write(open(part).read())
     finally:
         shutil.rmtree(tmp, ignore_errors=True)
     return HIP_LIB

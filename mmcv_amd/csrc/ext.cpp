@@ -142,7 +142,7 @@ bool prepare(Prepared &pr, const Tensor &input, const Tensor &weight,
   p.bias = with_bias ? dense(bias) : nullptr;
   p.output = output.data_ptr();
 
-  const size_t ws = mdcn_workspace_bytes(&p);
+  const size_t ws = mdcn_workspace_wanted(&p);
   if (ws > 0) {
     // torch's caching allocator: stream-ordered with the launches below
     pr.keep.push_back(at::empty({(int64_t)ws}, input.options().dtype(at::kByte)));
@@ -372,7 +372,7 @@ void deform_conv_forward(Tensor input, Tensor weight, Tensor offset, Tensor outp
   p.weight = keep[2].data_ptr();
   p.bias = nullptr;
   p.output = output.data_ptr();
-  const size_t ws = mdcn_workspace_bytes(&p);
+  const size_t ws = mdcn_workspace_wanted(&p);
   if (ws > 0) {
     keep.push_back(at::empty({(int64_t)ws}, input.options().dtype(at::kByte)));
     p.workspace = keep.back().data_ptr();

@@ -21,6 +21,7 @@
 #include "mdcn_fused3.h"
 #include "mdcn_oconv.h"
 #include "mdcn_prepass.h"
+#include "mdcn_segment.h"
 
 namespace {
 
@@ -155,6 +156,8 @@ struct Plan {
   size_t wp_bytes;   // packed weights
   size_t cut_bytes;  // eight-wave kernel: buffers and counters of the tiles it cuts along K (may be left out)
   int cut_wgs;     // ... one buffer and one counter per workgroup of its grid
+  bool seg;          // segment kernel: the shapes the fused kernels do not cover
+  SegPlan sp;
   // pack-level call only
   int CO, CO_pad;    // conv_offset channels: 3 (2 when unmodulated) * DG * taps, rounded up to 32
   int mask_kind;     // kMaskLogit, or kMaskNone when unmodulated
@@ -244,18 +247,40 @@ long wide_tiles_of_call(const mdcn_params *p, const Geom &g, const Plan &pl, lon
                     wide_tile_cost(pl.CT, g.sh == 1 && g.sw == 1));
 }
 
+// The segment kernel for a call the fused kernels do not take, in passes of n_chunk images.
+void plan_segments(const mdcn_params *p, const Geom &g, Plan *pl) {
+  pl->seg = false;
+  if (p->path == MDCN_PATH_DIRECT || p->dtype == MDCN_F64 || p->input_nhwc) return;
+  const int es = (int)elem_size(p->dtype);
+  if ((uint64_t)g.N * g.Ho * g.Wo > 0x7fffffffull || !seg_plan(g, es, 1, false, num_cus(), &pl->sp)) return;
+  pl->n_chunk = (int)std::min<uint64_t>((uint64_t)g.N, std::max<uint64_t>(1, g_fwd_pass_bytes.load() / pl->sp.xt_bytes));
+  pl->seg = seg_plan(g, es, pl->n_chunk, !p->no_k_split, num_cus(), &pl->sp);
+  pl->xt_bytes = align_up(pl->sp.xt_bytes);
+  pl->wp_bytes = align_up(pl->sp.wp_bytes);
+}
+
+// ... without it: one thread per output element, no workspace of its own
+void drop_segments(Plan *pl) {
+  pl->seg = false;
+  pl->xt_bytes = pl->wp_bytes = 0;
+}
+
 int make_plan(const mdcn_params *p, const Geom &g, Plan *pl) {
   const bool ok = fused_ok(p, g);
   if (forced_fused(p->path) && !ok) return MDCN_ERR_PATH;
   if (p->input_nhwc && (!ok || p->path == MDCN_PATH_DIRECT)) return MDCN_ERR_PATH;  // in-place reads: fused kernel only
   pl->fused = ok && p->path != MDCN_PATH_DIRECT;
+  pl->seg = false;
   pl->CT = pl->KC = pl->n_ctiles = pl->slabs = pl->n_chunk = 0;
   pl->xt_bytes = pl->wp_bytes = pl->owp_bytes = pl->raw_bytes = pl->cut_bytes = 0;
   pl->cut_wgs = 0;
   pl->CO = 3 * g.DG * g.taps;
   pl->CO_pad = (pl->CO + 31) / 32 * 32;
   pl->mask_kind = kMaskLogit;
-  if (!pl->fused) return MDCN_OK;
+  if (!pl->fused) {
+    plan_segments(p, g, pl);
+    return MDCN_OK;
+  }
   const size_t es = elem_size(p->dtype);
   pl->KC = slab_channels(p->dtype);
   pl->CT = pick_ct(g.cout_g, g.taps);
@@ -334,6 +359,7 @@ int make_pack_plan(const mdcn_pack_params *pp, const Geom &g, Plan *pl) {
         pl->fused = false;
         pl->xt_bytes = pl->wp_bytes = pl->cut_bytes = 0;
         pl->cut_wgs = 0;
+        plan_segments(p, g, pl);
       } else {
         pl->owp_bytes = align_up((size_t)(g.Cin / pl->KC) * g.taps * 4 * (pl->CO_pad / 32) * 64 * 16);
         pl->raw_bytes = align_up((size_t)pl->n_chunk * plane * pl->CO_pad * es);
@@ -496,7 +522,7 @@ int run_typed(const mdcn_params *p, const Geom &g, const Plan &pl, hipStream_t s
     if (px) {
       E *raw = (E *)px->raw;
       if (px->offset_weight) {
-        if (!raw) raw = (E *)p->workspace;
+        if (!raw) raw = (E *)((unsigned char *)p->workspace + pl.xt_bytes + pl.wp_bytes);
         const long total = (long)g.N * pl.CO * plane_out;
         const int grid = (int)std::min<long>((total + 255) / 256, 1L << 20);
         tic();
@@ -508,6 +534,35 @@ int run_typed(const mdcn_params *p, const Geom &g, const Plan &pl, hipStream_t s
       }
       om = nchw_raw_view(raw);
     }
+    if (pl.seg) {
+      SegArgs sa;
+      sa.s = pl.sp;
+      sa.xt = p->workspace;
+      sa.wp = (unsigned char *)p->workspace + pl.xt_bytes;
+      sa.bias = p->bias;
+      sa.row_bytes = (uint32_t)g.Wp * 16u;
+      sa.plane_bytes = (uint32_t)g.Hp * sa.row_bytes;
+      sa.img_bytes = (uint32_t)(g.G * pl.sp.nseg_g * pl.sp.cps) * sa.plane_bytes;
+      for (int n0 = 0; n0 < g.N && rc == MDCN_OK; n0 += pl.n_chunk) {
+        sa.g = g;
+        sa.g.N = std::min(pl.n_chunk, g.N - n0);
+        sa.om = om;
+        sa.om.off = (const E *)om.off + (long)n0 * om.off_n;
+        sa.om.msk = (const E *)om.msk + (long)n0 * om.msk_n;
+        sa.out = (E *)p->output + (size_t)n0 * g.Cout * plane_out;
+        sa.total_px = (long)sa.g.N * plane_out;
+        const long tile_px = 32 * (4 / pl.sp.kshare);
+        sa.n_work = (sa.total_px + tile_px - 1) / tile_px * pl.sp.n_ctiles * g.G;
+        tic();
+        if (seg_prepass(p->dtype, sa, (const E *)p->input + (size_t)n0 * g.Cin * g.H * g.W, n0 ? nullptr : p->weight,
+                        st) != hipSuccess)
+          rc = MDCN_ERR_LAUNCH;
+        toc(0);
+        tic();
+        if (rc == MDCN_OK && seg_forward(p->dtype, sa, st) != hipSuccess) rc = MDCN_ERR_LAUNCH;
+        toc(2);
+      }
+    } else {
     const long total = (long)g.N * g.Cout * plane_out;
     const int grid = (int)std::min<long>((total + 255) / 256, 1L << 20);
     tic();
@@ -516,6 +571,7 @@ int run_typed(const mdcn_params *p, const Geom &g, const Plan &pl, hipStream_t s
                        (const E *)p->bias, (E *)p->output, total);
     if (hipGetLastError() != hipSuccess) rc = MDCN_ERR_LAUNCH;
     toc(2);
+    }
   } else {
     unsigned char *ws = (unsigned char *)p->workspace;
     E *xt = (E *)ws;
@@ -720,6 +776,10 @@ int run(const mdcn_params *p, void *stream, float *ms, const mdcn_pack_params *p
     return run_f64(p, g, (hipStream_t)stream, ms);
   }
   // (the split-tile buffers come last and are optional: a workspace without them runs unsplit)
+  // a call whose workspace does not hold the segment kernel's copies runs without that kernel, as it may
+  if (pl.seg && (p->workspace_bytes < pl.xt_bytes + pl.wp_bytes + pl.raw_bytes || !p->workspace ||
+                 ((uintptr_t)p->workspace % kAlign) != 0))
+    drop_segments(&pl);
   const size_t need = pl.xt_bytes + pl.wp_bytes + pl.owp_bytes + pl.raw_bytes;
   if (need > 0 && (!p->workspace || p->workspace_bytes < need ||
                    ((uintptr_t)p->workspace % kAlign) != 0))
@@ -1251,6 +1311,7 @@ const char *mdcn_forward_kernels(const mdcn_params *p) {
   Plan pl;
   if (make_plan(p, g, &pl) != MDCN_OK) return "";
   if (p->dtype == MDCN_F64) return "f64_forward_kernel";
+  if (pl.seg) return "segment_kernel";
   if (!pl.fused) return "direct_kernel";
   if (!uses_fused2(p, g, pl)) return "fused_kernel";
   const size_t es = elem_size(p->dtype);
@@ -1267,7 +1328,15 @@ size_t mdcn_workspace_bytes(const mdcn_params *p) {
   if (check_params(p, &g, false) != MDCN_OK) return 0;
   Plan pl;
   if (make_plan(p, g, &pl) != MDCN_OK) return 0;
-  return pl.fused ? pl.xt_bytes + pl.wp_bytes + pl.cut_bytes : 0;
+  return pl.seg ? 0 : pl.xt_bytes + pl.wp_bytes + pl.cut_bytes;
+}
+
+size_t mdcn_workspace_wanted(const mdcn_params *p) {
+  Geom g;
+  if (check_params(p, &g, false) != MDCN_OK) return 0;
+  Plan pl;
+  if (make_plan(p, g, &pl) != MDCN_OK) return 0;
+  return pl.xt_bytes + pl.wp_bytes + pl.cut_bytes;
 }
 
 int mdcn_forward(const mdcn_params *p, void *hip_stream) {
@@ -1281,11 +1350,16 @@ int mdcn_forward_noalloc(const mdcn_params *p, void *hip_stream) {
   Plan pl;
   rc = make_plan(p, g, &pl);
   if (rc != MDCN_OK) return rc;
+  mdcn_params q = *p;
+  if (pl.seg) {  // needs no scratch: the kernel, and the bits, of a mdcn_forward() with mdcn_workspace_bytes()
+    q.workspace = nullptr;
+    q.workspace_bytes = 0;
+    return run(&q, hip_stream, nullptr);
+  }
   if (pl.xt_bytes + pl.wp_bytes > (size_t)MDCN_NOALLOC_SCRATCH_BYTES) return MDCN_ERR_SCRATCH_LIMIT;
   void *ptr = nullptr;
   rc = scratch_of_current_device(&ptr);
   if (rc != MDCN_OK) return rc;
-  mdcn_params q = *p;
   q.workspace = ptr;
   q.workspace_bytes = (size_t)MDCN_NOALLOC_SCRATCH_BYTES;
   return run(&q, hip_stream, nullptr);

@@ -31,19 +31,6 @@ namespace mdcn {
 constexpr int kCgTile = 128;
 constexpr int kCgTileBig = 256;
 
-// Work index of a workgroup of a 1-D launch of 8 * ceil(total / 8) workgroups, or
-// -1 for the few that have none.  Consecutive workgroup ids sit on different
-// XCDs (each with its own L2); this hands every XCD one contiguous run of work
-// indices, so that neighbours in the work order -- made to share an operand tile
-// -- run on the same XCD at about the same time and fetch that tile from HBM
-// once instead of once per XCD.
-__device__ __forceinline__ long xcd_work_index(long total) {
-  const long chunk = (total + 7) >> 3;
-  const long xcd = blockIdx.x & 7, i = blockIdx.x >> 3;
-  const long L = xcd * chunk + i;
-  return (i < chunk && L < total) ? L : -1;
-}
-
 // weight[Cout][cin_g][taps] -> wT[G][M_pad][cout_g], row m = tap * cin_g + c,
 // zero rows from taps * cin_g up to M_pad (a multiple of kCgTile).
 template <typename E>

@@ -39,6 +39,19 @@ __device__ __forceinline__ E from_f32(float v) {
   return (E)v;
 }
 
+// Work index of a workgroup of a 1-D launch of 8 * ceil(total / 8) workgroups, or
+// -1 for the few that have none.  Consecutive workgroup ids sit on different
+// XCDs (each with its own L2); this hands every XCD one contiguous run of work
+// indices, so that neighbours in the work order -- made to share an operand tile
+// -- run on the same XCD at about the same time and fetch that tile from HBM
+// once instead of once per XCD.
+__device__ __forceinline__ long xcd_work_index(long total) {
+  const long chunk = (total + 7) >> 3;
+  const long xcd = blockIdx.x & 7, i = blockIdx.x >> 3;
+  const long L = xcd * chunk + i;
+  return (i < chunk && L < total) ? L : -1;
+}
+
 // Sampling position of one (pixel, tap) and its four mask-scaled bilinear
 // weights; same arithmetic order as the reference's CPU sampler
 // (mmcv/ops/csrc/pytorch/cpu/modulated_deform_conv.cpp:5-33,158-163) in fp32,

@@ -1,0 +1,372 @@
+// Segment kernel: implicit GEMM  out[cout, pixel] = W[cout, k] * S[k, pixel]  for
+// channel counts that do not fill 128-byte slabs of one deformable group.
+//
+// The channels of a convolution group fall into segments that belong to one
+// deformable group; a segment is padded to whole 16-byte chunks and the input
+// copy is chunk-major ([N][chunk][H+2][W+2][16 bytes], zero border).  K runs over
+// "pairs" (cq neighbouring chunks of a segment, tap).  A wavefront owns 32
+// pixels x up to 256 output channels and keeps everything in registers: its lower
+// 32 lanes take the even pairs of the pixels and the upper 32 the odd ones,
+// each lane reads its pixel's offsets and mask from the NCHW tensors (32 lanes =
+// 32 neighbouring pixels), gathers the four corners of cq chunks and blends them,
+// and what comes out is a B operand of the 32x32 MFMA as it stands (column =
+// lane % 32, K half = lane / 32: K may be walked in any order as long as the
+// packed weights follow it).  No LDS tile, no barrier in the K loop; a position
+// is computed once per pair and used for cq chunks.  Neighbouring lanes sample
+// neighbouring pixels and a 16-byte pixel lets eight of them share a cache line.
+// The weights are packed in A-operand order and read from L1/L2.
+//
+// Few pixels: `kshare` waves of the workgroup split the pairs of a pixel block
+// among them and add their accumulators up through LDS, in a fixed order.
+//
+// What bounds it: the vector-memory path of the CU, 64 bytes of corner data per
+// 16 bytes of S; with fp32 tensors the MFMAs (32x32x2) are close behind.  Measured against the
+// one-thread-per-output kernel that these shapes had before: N=2, 64 -> 64 channels, 8 deformable groups,
+// 180x320, fp32 23.9 ms -> 0.15 ms + 0.013 ms of pre-pass; N=4, 96 -> 72 channels, 2 deformable groups,
+// 37x53, bf16 1 733 us -> 15 + 5 us.
+#include "mdcn_segment.h"
+
+#include <algorithm>
+
+#include "../../include/mdcn.h"
+#include "mdcn_fused.h"
+
+namespace mdcn {
+
+namespace {
+
+// Weights to A-operand order and the input to chunk planes, one launch: the first
+// pack_blocks workgroups repack, the others copy 256 pixels of the bordered plane
+// of one chunk each.
+template <typename E>
+__global__ __launch_bounds__(256) void seg_prepass_kernel(SegArgs a, const E *__restrict__ in,
+                                                          const E *__restrict__ w, int pack_blocks, int px_blocks) {
+  constexpr int VC = 16 / (int)sizeof(E);
+  const Geom &g = a.g;
+  const SegPlan &s = a.s;
+  if ((int)blockIdx.x < pack_blocks) {
+    const long total = (long)g.G * s.n_ctiles * s.iters * s.cq * s.nb * 64;
+    const int grp_per_seg = s.cps / s.cq;
+    for (long idx = (long)blockIdx.x * 256 + threadIdx.x; idx < total; idx += (long)pack_blocks * 256) {
+      long r = idx;
+      const int lane = (int)(r & 63);
+      r >>= 6;
+      const int nb = (int)(r % s.nb);
+      r /= s.nb;
+      const int q = (int)(r % s.cq);
+      r /= s.cq;
+      const int it = (int)(r % s.iters);
+      r /= s.iters;
+      const int ct = (int)(r % s.n_ctiles);
+      const int grp = (int)(r / s.n_ctiles);
+      const int p = 2 * it + (lane >> 5);
+      const int col = (ct * s.nb + nb) * 32 + (lane & 31);
+      const int sg = p / g.taps, tap = p - sg * g.taps;
+      const int sl = sg / grp_per_seg;                                   // segment of the group
+      const int c0 = ((sg - sl * grp_per_seg) * s.cq + q) * VC;           // first channel of the chunk in it
+      E v[VC];
+#pragma unroll
+      for (int i = 0; i < VC; ++i) {
+        const bool ok = p < s.pairs && col < g.cout_g && c0 + i < s.seg;
+        const E *src = w + ((long)(grp * g.cout_g + (ok ? col : 0)) * g.cin_g + (ok ? sl * s.seg + c0 + i : 0)) * g.taps +
+                       (ok ? tap : 0);
+        v[i] = ok ? *src : from_f32<E>(0.0f);
+      }
+      uint4 o;
+      __builtin_memcpy(&o, v, 16);
+      ((uint4 *)a.wp)[idx] = o;
+    }
+    return;
+  }
+  int b = (int)blockIdx.x - pack_blocks;
+  const int pb = b % px_blocks;
+  b /= px_blocks;
+  const int chunks = g.G * s.nseg_g * s.cps;
+  const int ch = b % chunks, n = b / chunks;
+  const int q = pb * 256 + (int)threadIdx.x;
+  if (q >= g.Hp * g.Wp) return;
+  const int yp = q / g.Wp, y = yp - 1, x = q - yp * g.Wp - 1;
+  const int sl = ch / s.cps, c0 = (ch - sl * s.cps) * VC;
+  const bool inside = y >= 0 && y < g.H && x >= 0 && x < g.W;
+  const long plane = (long)g.H * g.W;
+  const E *src = in + ((long)n * g.Cin + (long)sl * s.seg) * plane + (inside ? (long)y * g.W + x : 0);
+  E v[VC];
+#pragma unroll
+  for (int i = 0; i < VC; ++i) v[i] = src[(long)min(c0 + i, s.seg - 1) * plane];
+#pragma unroll
+  for (int i = 0; i < VC; ++i)
+    if (!inside || c0 + i >= s.seg) v[i] = from_f32<E>(0.0f);
+  uint4 o;
+  __builtin_memcpy(&o, v, 16);
+  *(uint4 *)((unsigned char *)const_cast<void *>(a.xt) + (size_t)n * a.img_bytes + (size_t)ch * a.plane_bytes +
+             (size_t)q * 16) = o;
+}
+
+// Waves per SIMD the register budget is cut for.
+constexpr int seg_occupancy(int NB, int CQ) { return CQ * NB <= 4 && NB <= 2 ? 4 : (NB <= 4 && CQ * NB <= 8 ? 3 : 2); }
+
+template <typename E, int NB, int CQ>
+__global__ __launch_bounds__(256, seg_occupancy(NB, CQ)) void segment_kernel(SegArgs a) {
+  using TR = ElemTraits<E>;
+  const Geom &g = a.g;
+  const SegPlan &s = a.s;
+  extern __shared__ __align__(16) unsigned char smem[];
+  // {offset channel of dy, mask channel, ti * dh << 16 | tj * dw, first chunk} of every pair
+  uint4 *tab = (uint4 *)smem;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int pxl = lane & 31, half = lane >> 5;
+
+  long L = xcd_work_index(a.n_work);
+  if (L < 0) return;
+  const int ct = (int)(L % s.n_ctiles);
+  L /= s.n_ctiles;
+  const int grp = (int)(L % g.G);
+  const int ptile = (int)(L / g.G);
+  const int wpx = 4 / s.kshare;                 // pixel blocks of the workgroup
+  const int ks = wave & (s.kshare - 1);
+  const long p0 = ((long)ptile * wpx + wave / s.kshare) * 32;
+
+  const int grp_per_seg = s.cps / s.cq;
+  for (int p = tid; p < s.pairs; p += 256) {
+    const int sg = p / g.taps, tap = p - sg * g.taps;
+    const int sl = sg / grp_per_seg;
+    const int ti = tap / g.kw, tj = tap - ti * g.kw;
+    const int dgi = ((grp * s.nseg_g + sl) * s.seg) / g.ch_per_dg;
+    tab[p] = make_uint4((uint32_t)((dgi * g.taps + tap) * 2), (uint32_t)(dgi * g.taps + tap),
+                        ((uint32_t)(ti * g.dh) << 16) | (uint32_t)(tj * g.dw),
+                        (uint32_t)((grp * s.nseg_g + sl) * s.cps + (sg - sl * grp_per_seg) * s.cq));
+  }
+  __syncthreads();
+
+  const int plane_out = g.Ho * g.Wo;
+  const long pp = min(p0 + pxl, a.total_px - 1);
+  const int n = (int)(pp / plane_out);
+  const int rem = (int)(pp - (long)n * plane_out);
+  const int ho = rem / g.Wo, wo = rem - ho * g.Wo;
+  const int by = ho * g.sh - g.ph, bx = wo * g.sw - g.pw;
+  const E *off = (const E *)a.om.off + (long)n * a.om.off_n + (long)rem * a.om.off_px;
+  const E *msk = (const E *)a.om.msk + (long)n * a.om.msk_n + (long)rem * a.om.msk_px;
+  const unsigned char *xt = (const unsigned char *)a.xt;
+  const uint32_t img = (uint32_t)n * a.img_bytes;
+
+  struct Raw {
+    E dy, dx, m;
+    uint32_t tij, chunk;
+  };
+  auto load_om = [&](int i, Raw &r) {
+    const int p = 2 * i + half;
+    const uint4 t = tab[min(p, s.pairs - 1)];
+    const E *o = off + (long)t.x * a.om.off_ch;
+    r.dy = o[0];
+    r.dx = o[a.om.off_ch];
+    r.m = msk[(long)t.y * a.om.msk_ch];
+    // (the odd pair out: a position outside, i.e. zeros, and not a second copy of the last pair)
+    r.tij = p < s.pairs ? t.z : 0x7fff0000u;
+    r.chunk = t.w;
+  };
+  struct Gather {
+    uint4 v[CQ][4];
+    uint4 w;
+  };
+  auto gather = [&](const Raw &r, Gather &v) {
+    const TapSample sm = make_tap_sample(by + (int)(r.tij >> 16), bx + (int)(r.tij & 0xffffu), to_f32(r.dy), to_f32(r.dx),
+                                         mask_value<E>(r.m, a.om.logit), g.H, g.W);
+    // (a position outside reads border pixels: see corner_offset())
+    const uint32_t pix = sm.inside ? (uint32_t)((sm.y0 + 1) * g.Wp + sm.x0 + 1) : (uint32_t)(g.Wp - 1);
+    uint32_t o = img + r.chunk * a.plane_bytes + pix * 16u;
+    uint32_t tw[4];
+    TR::table_weights(sm, tw);
+    v.w = make_uint4(tw[0], tw[1], tw[2], tw[3]);
+#pragma unroll
+    for (int q = 0; q < CQ; ++q) {
+      const unsigned char *top = xt + o, *bot = xt + (o + a.row_bytes);
+      v.v[q][0] = *(const uint4 *)top;
+      v.v[q][1] = *(const uint4 *)(top + 16);
+      v.v[q][2] = *(const uint4 *)bot;
+      v.v[q][3] = *(const uint4 *)(bot + 16);
+      o += a.plane_bytes;
+    }
+  };
+  const uint4 *wp = (const uint4 *)a.wp + (size_t)(grp * s.n_ctiles + ct) * s.iters * (CQ * NB * 64) + lane;
+  auto load_w = [&](int i, uint4 (&wf)[CQ][NB]) {
+    const uint4 *src = wp + (size_t)i * (CQ * NB * 64);
+#pragma unroll
+    for (int q = 0; q < CQ; ++q)
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) wf[q][nb] = src[(q * NB + nb) * 64];
+  };
+
+  f32x16 acc[NB];
+#pragma unroll
+  for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[nb][r] = 0.0f;
+
+  const int i0 = s.iters * ks / s.kshare, i1 = s.iters * (ks + 1) / s.kshare;
+  if (i0 < i1) {
+    Raw raw;
+    Gather gv;
+    uint4 wf[CQ][NB];
+    load_om(i0, raw);
+    gather(raw, gv);
+    load_w(i0, wf);
+    load_om(min(i0 + 1, i1 - 1), raw);
+    for (int i = i0; i < i1; ++i) {
+      uint4 x[CQ];
+#pragma unroll
+      for (int q = 0; q < CQ; ++q) x[q] = TR::blend(gv.v[q][0], gv.v[q][1], gv.v[q][2], gv.v[q][3], gv.w);
+      uint4 wc[CQ][NB];
+#pragma unroll
+      for (int q = 0; q < CQ; ++q)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) wc[q][nb] = wf[q][nb];
+      // (the last iteration fetches its own data again: nobody reads it)
+      gather(raw, gv);
+      load_om(min(i + 2, i1 - 1), raw);
+#pragma unroll
+      for (int q = 0; q < CQ; ++q)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) TR::mma(acc[nb], wc[q][nb], x[q]);
+      load_w(min(i + 1, i1 - 1), wf);
+    }
+  }
+
+  // register r of lane l: output channel (r/4)*8 + (l/32)*4 + r%4 of the block, pixel l%32
+  E *out = (E *)a.out;
+  const bool px_ok = p0 + pxl < a.total_px;
+  E *dst = out + ((long)n * g.Cout + (long)grp * g.cout_g) * plane_out + rem;
+  auto put = [&](int nb, int r, float v) {
+    const int col = (ct * NB + nb) * 32 + (r >> 2) * 8 + half * 4 + (r & 3);
+    if (px_ok && col < g.cout_g) {
+      if (a.bias) v += to_f32(((const E *)a.bias)[grp * g.cout_g + col]);
+      dst[(long)col * plane_out] = from_f32<E>(v);
+    }
+  };
+  if (s.kshare == 1) {
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) put(nb, r, acc[nb][r]);
+  } else {
+    float *red = (float *)(smem + (size_t)s.pairs * 16);  // [wave][16][64 lanes]
+    const int w0 = wave - ks;
+    const int per = 16 / s.kshare;
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      __syncthreads();
+#pragma unroll
+      for (int r = 0; r < 16; ++r) red[(wave * 16 + r) * 64 + lane] = acc[nb][r];
+      __syncthreads();
+      for (int r = ks * per; r < (ks + 1) * per; ++r) {
+        float v = 0.0f;
+        for (int k = 0; k < s.kshare; ++k) v += red[((w0 + k) * 16 + r) * 64 + lane];
+        put(nb, r, v);
+      }
+    }
+  }
+}
+
+template <typename E, int NB, int CQ>
+hipError_t launch(const SegArgs &a, hipStream_t st) {
+  const size_t lds = (size_t)a.s.pairs * 16 + (a.s.kshare > 1 ? 4 * 16 * 64 * 4 : 0);
+  hipLaunchKernelGGL((segment_kernel<E, NB, CQ>), dim3((unsigned)((a.n_work + 7) / 8 * 8)), dim3(256), lds, st, a);
+  return hipGetLastError();
+}
+
+template <typename E, int CQ>
+hipError_t launch_nb(const SegArgs &a, hipStream_t st) {
+  switch (a.s.nb) {
+    case 1: return launch<E, 1, CQ>(a, st);
+    case 2: return launch<E, 2, CQ>(a, st);
+    case 3: return launch<E, 3, CQ>(a, st);
+    default: break;
+  }
+  if constexpr (CQ <= 2) {
+    if (a.s.nb == 4) return launch<E, 4, CQ>(a, st);
+    if (a.s.nb == 6) return launch<E, 6, CQ>(a, st);
+  }
+  if constexpr (CQ == 1) {
+    if (a.s.nb == 8) return launch<E, 8, CQ>(a, st);
+  }
+  return hipErrorInvalidValue;
+}
+
+template <typename E>
+hipError_t launch_e(const SegArgs &a, hipStream_t st) {
+  return a.s.cq == 1 ? launch_nb<E, 1>(a, st) : a.s.cq == 2 ? launch_nb<E, 2>(a, st) : launch_nb<E, 4>(a, st);
+}
+
+template <typename E>
+hipError_t prepass_e(const SegArgs &a, const void *in, const void *weight, hipStream_t st) {
+  const int px_blocks = (a.g.Hp * a.g.Wp + 255) / 256;
+  const long blocks = (long)a.g.N * a.g.G * a.s.nseg_g * a.s.cps * px_blocks;
+  const long wtotal = (long)a.s.wp_bytes / 16;
+  const int pack_blocks = weight ? (int)std::max<long>(1, std::min<long>(wtotal / 256, 512)) : 0;
+  hipLaunchKernelGGL(seg_prepass_kernel<E>, dim3((unsigned)(blocks + pack_blocks)), dim3(256), 0, st, a, (const E *)in,
+                     (const E *)weight, pack_blocks, px_blocks);
+  return hipGetLastError();
+}
+
+}  // namespace
+
+bool seg_plan(const Geom &g, int es, int n_images, bool may_share, int cus, SegPlan *s) {
+  const int VC = 16 / es;
+  int u = g.cin_g, v = g.ch_per_dg;
+  while (v) {
+    const int t = u % v;
+    u = v;
+    v = t;
+  }
+  s->seg = u;
+  s->nseg_g = g.cin_g / s->seg;
+  const int cps0 = (s->seg + VC - 1) / VC;
+  const int blocks = (g.cout_g + 31) / 32;
+  s->n_ctiles = (blocks + 7) / 8;
+  s->nb = (blocks + s->n_ctiles - 1) / s->n_ctiles;
+  if (s->nb == 5) s->nb = 6;
+  if (s->nb == 7) s->nb = 8;
+  // Chunks per position: as many as share one without padding much.  A chunk costs its gather and
+  // blend, a position about one and a half of that.
+  double best = 0.0;
+  s->cq = 0;
+  for (int cq = 4; cq >= 1; cq /= 2) {
+    if (cq * s->nb > kSegFragsMax) continue;
+    const int groups = (cps0 + cq - 1) / cq;
+    const double cost = groups * 1.5 + groups * cq;
+    if (s->cq == 0 || cost < best) best = cost, s->cq = cq;
+  }
+  s->cps = (cps0 + s->cq - 1) / s->cq * s->cq;
+  const long pairs = (long)s->nseg_g * (s->cps / s->cq) * g.taps;
+  if (pairs > kSegPairsMax) return false;
+  if ((long)(g.kh - 1) * g.dh > 0xffff || (long)(g.kw - 1) * g.dw > 0xffff) return false;
+  s->pairs = (int)pairs;
+  s->iters = (s->pairs + 1) / 2;
+  const uint64_t img = (uint64_t)g.G * s->nseg_g * s->cps * g.Hp * g.Wp * 16;
+  if (img * (uint64_t)n_images > 0xF0000000ull) return false;
+  s->xt_bytes = (size_t)(img * (uint64_t)n_images);
+  s->wp_bytes = (size_t)g.G * s->n_ctiles * s->iters * s->cq * s->nb * 1024;
+  // Waves of a workgroup share a pixel block's K range while that leaves the chip's SIMDs short of two waves.
+  const long waves = ((long)n_images * g.Ho * g.Wo + 31) / 32 * s->n_ctiles * g.G;
+  s->kshare = 1;
+  while (may_share && s->kshare < 4 && waves * s->kshare < 8L * cus && s->iters >= 4 * s->kshare) s->kshare *= 2;
+  return true;
+}
+
+hipError_t seg_prepass(int dtype, const SegArgs &a, const void *in, const void *weight, hipStream_t st) {
+  switch (dtype) {
+    case MDCN_F32: return prepass_e<float>(a, in, weight, st);
+    case MDCN_F16: return prepass_e<f16_t>(a, in, weight, st);
+    default: return prepass_e<bf16_t>(a, in, weight, st);
+  }
+}
+
+hipError_t seg_forward(int dtype, const SegArgs &a, hipStream_t st) {
+  switch (dtype) {
+    case MDCN_F32: return launch_e<float>(a, st);
+    case MDCN_F16: return launch_e<f16_t>(a, st);
+    default: return launch_e<bf16_t>(a, st);
+  }
+}
+
+}  // namespace mdcn
