@@ -14,32 +14,43 @@
 #include "mdcn_common.h"
 #include "mdcn_direct.h"
 #include "mdcn_f64.h"
-#include "mdcn_backward.h"
-#include "mdcn_backward_gemm.h"
 #include "mdcn_fused.h"
 #include "mdcn_fused2.h"
 #include "mdcn_fused3.h"
 #include "mdcn_oconv.h"
+#include "mdcn_host.h"
 #include "mdcn_prepass.h"
 #include "mdcn_segment.h"
+
+namespace mdcn {
+
+int num_cus() {
+  static int cached[64] = {0};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  if (cached[dev] == 0) {
+    int n = 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
+      n = 256;
+    cached[dev] = n;
+  }
+  return cached[dev];
+}
+
+}  // namespace mdcn
 
 namespace {
 
 using namespace mdcn;
 
-constexpr size_t kAlign = 256;
 constexpr size_t kMaxLds = 160 * 1024;
 // Device byte offsets into the channels-last copy are 32-bit.
 constexpr uint64_t kMaxXtBytes = 0xF0000000ull;
-// Column gradient (and columns) held in memory per pass of the backward's matrix-core paths.
-constexpr uint64_t kBwdColGradCap = (uint64_t)3 << 29;  // 1.5 GiB each
 // Per-pass limits in force (mdcn_set_pass_limits lowers them; process wide).  Atomic, so that a
 // call that runs while another thread changes them reads one of the two values; a workspace that was
 // sized under one value and used under another is still the caller's to avoid.
 std::atomic<uint64_t> g_fwd_pass_bytes{kMaxXtBytes};
 std::atomic<uint64_t> g_bwd_pass_bytes{kBwdColGradCap};
-
-inline size_t align_up(size_t v) { return (v + kAlign - 1) / kAlign * kAlign; }
 
 // Scratch of mdcn_forward_noalloc(): the input copy and the packed weights of one
 // call, held by every device the library runs on until the process ends.  Host
@@ -63,8 +74,6 @@ int scratch_of_current_device(void **out) {
   *out = g_scratch_ptr[dev];
   return MDCN_OK;
 }
-
-inline size_t elem_size(int dtype) { return dtype == MDCN_F64 ? 8 : dtype == MDCN_F32 ? 4 : 2; }
 
 int check_params(const mdcn_params *p, Geom *g, bool need_ptrs, bool need_offsets = true) {
   if (!p) return MDCN_ERR_NULL;
@@ -122,19 +131,6 @@ bool fused_ok(const mdcn_params *p, const Geom &g) {
   return true;
 }
 
-int num_cus() {
-  static int cached[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (cached[dev] == 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-      n = 256;
-    cached[dev] = n;
-  }
-  return cached[dev];
-}
-
 // Length of the persistent schedule of `tiles` tiles of nk K steps in tile times, as UnitSchedule lays it
 // out: whole rounds, then the last round's tiles whole or cut into parts.
 double schedule_rounds(long tiles, int nk, bool may_cut) {
@@ -170,11 +166,6 @@ struct PackExtra {
   const void *offset_weight, *offset_bias;
   void *raw;
 };
-
-inline bool forced_fused(int path) {
-  return path == MDCN_PATH_FUSED || path == MDCN_PATH_FUSED_SPLIT || path == MDCN_PATH_FUSED_WIDE ||
-         path == MDCN_PATH_FUSED_NARROW;
-}
 
 // 16-bit tensors, 256- or 128-channel tiles, one deformable group, enough K steps: the eight-wave
 // kernels (mdcn_fused2.h; mdcn_fused3.h beside it where wide_ok() says so)
@@ -793,455 +784,6 @@ int run(const mdcn_params *p, void *stream, float *ms, const mdcn_pack_params *p
   }
 }
 
-// Largest margin R (up to 8) for which the LDS window of a th x tw output-pixel
-// tile fits max_px pixels; -1 if even R = 0 does not.
-int window_margin(const Geom &g, int th, int tw, long max_px, int *WH, int *WW) {
-  const long base_h = (long)(th - 1) * g.sh + (long)(g.kh - 1) * g.dh + 2;
-  const long base_w = (long)(tw - 1) * g.sw + (long)(g.kw - 1) * g.dw + 2;
-  int R = -1;
-  while (R < 8 && (base_h + 2 * (R + 1)) * (base_w + 2 * (R + 1)) <= max_px) ++R;
-  *WH = (int)base_h + 2 * std::max(R, 0);
-  *WW = (int)base_w + 2 * std::max(R, 0);
-  return R;
-}
-
-struct BwdPlan {
-  size_t gin_bytes, gw_bytes;  // fp32 staging (0 for fp32 tensors)
-  // grad_input / grad_offset / grad_mask by bwd_data_tiled_kernel (else, without
-  // `gemm`, one workgroup per tap):
-  bool tiled;
-  int R, WH, WW;   // its window margin and size
-  // matrix-core paths (bwd_colgrad_kernel + bwd_scatter_kernel, bwd_wgrad_kernel):
-  bool gemm;       // data gradients
-  bool wgemm;      // grad_weight from stored columns
-  int sR, sWH, sWW;  // window of the scatter kernel
-  int sCH;         // channels per pass over that window
-  int n_chunk;     // images per pass
-  int cg_tile;     // tile of the column-gradient product (kCgTile or kCgTileBig)
-  int M_pad;       // rows of the transposed weight matrix per group
-  long P_pad;      // row pitch of the columns matrix
-  int parts;       // workgroups of the scatter kernel per tile (shares of the channels)
-  size_t xt_bytes, gt_bytes, wt_bytes, d_bytes, col_bytes, part_bytes;
-  int w_tile, w_splits;  // weight-gradient product: tile, shares of the K range
-  size_t wpart_bytes;    // ... and their partial sums
-  size_t gpad_bytes;     // grad_output with padded rows, when its own rows cannot be copied 16 bytes at a time
-  size_t gb_bytes;  // fp32 sum of grad_bias (16-bit tensors)
-  size_t mx_bytes;  // the two maxima that scale the fixed-point window (16-bit tensors)
-  size_t total() const {
-    return gin_bytes + gw_bytes + gb_bytes + mx_bytes + xt_bytes + gt_bytes + wt_bytes + d_bytes + col_bytes + part_bytes +
-           wpart_bytes + gpad_bytes;
-  }
-};
-
-void make_bwd_plan(const mdcn_bwd_params *bp, const Geom &g, BwdPlan *pl) {
-  const bool f64 = bp->conv.dtype == MDCN_F64;
-  const bool staged = bp->conv.dtype != MDCN_F32 && !f64;
-  const size_t es = elem_size(bp->conv.dtype);
-  pl->gin_bytes = (staged && bp->grad_input) ? align_up((size_t)g.N * g.Cin * g.H * g.W * 4) : 0;
-  pl->gw_bytes = (staged && bp->grad_weight) ? align_up((size_t)g.Cout * g.cin_g * g.taps * 4) : 0;
-  pl->gb_bytes = (staged && bp->grad_bias) ? align_up((size_t)g.Cout * 4) : 0;
-  pl->mx_bytes = 0;
-  pl->tiled = pl->gemm = pl->wgemm = false;
-  pl->xt_bytes = pl->gt_bytes = pl->wt_bytes = pl->d_bytes = pl->col_bytes = pl->part_bytes = pl->wpart_bytes = 0;
-  pl->w_tile = kCgTile;
-  pl->w_splits = 1;
-  pl->gpad_bytes = 0;
-  pl->parts = 1;
-  pl->n_chunk = g.N;
-  pl->M_pad = 0;
-  pl->cg_tile = kCgTile;
-  pl->P_pad = 0;
-  pl->R = pl->sR = -1;
-  pl->WH = pl->WW = pl->sWH = pl->sWW = 0;
-  const int path = forced_fused(bp->conv.path) ? MDCN_PATH_FUSED : bp->conv.path;
-  if (path == MDCN_PATH_DIRECT || g.taps > kBwdTapsMax || f64) return;
-  const bool forced = path == MDCN_PATH_FUSED;
-  const size_t plane_out = (size_t)g.Ho * g.Wo;
-
-  // matrix-core paths: channels in whole 128-byte slabs, 32-channel blocks per tap
-  const int KC = (int)(128 / es);
-  const size_t d_img = (size_t)g.taps * g.Cin * plane_out * es;
-  // channels per pass: 16 / 8 of 32-bit fixed point (16-bit tensors), 8 / 4 doubles (fp32)
-  const int ch_big = es == 2 ? 16 : 8;
-  pl->sCH = ch_big;
-  pl->sR = window_margin(g, kScTH, kScTW, kScWindowPx, &pl->sWH, &pl->sWW);
-  if (pl->sR < 2 || g.ch_per_dg % ch_big) {  // fewer channels at a time buy a wider window
-    int wh, ww;
-    const int r = window_margin(g, kScTH, kScTW, 2 * kScWindowPx, &wh, &ww);
-    if (r > pl->sR || g.ch_per_dg % ch_big) {
-      pl->sCH = ch_big / 2;
-      pl->sR = r;
-      pl->sWH = wh;
-      pl->sWW = ww;
-    }
-  }
-  const long s_tiles = (long)g.N * g.DG * ((g.Ho + kScTH - 1) / kScTH) * ((g.Wo + kScTW - 1) / kScTW);
-  const bool mfma_ok = g.Cin % KC == 0 && g.cout_g % KC == 0 && g.cin_g % 32 == 0 &&
-                       g.ch_per_dg % pl->sCH == 0 && pl->sR >= 1 && (s_tiles >= 64 || forced) &&
-                       d_img <= kBwdColGradCap && plane_out <= ((size_t)1 << 30) &&
-                       (size_t)g.H * g.W <= ((size_t)1 << 30);  // (plane offsets held in 32 bits)
-  if (mfma_ok) {
-    pl->gemm = bp->grad_input != nullptr;
-    pl->wgemm = bp->grad_weight != nullptr;
-  }
-  if (pl->gemm || pl->wgemm) {
-    pl->n_chunk = (int)std::min<uint64_t>((uint64_t)g.N, std::max<uint64_t>(1, g_bwd_pass_bytes.load() / d_img));
-    pl->xt_bytes = align_up((size_t)g.N * (g.Cin / KC) * g.Hp * g.Wp * 128);
-  }
-  if (pl->gemm) {
-    pl->cg_tile = (g.taps * g.cin_g >= kCgTileBig && plane_out >= (size_t)kCgTileBig) ? kCgTileBig : kCgTile;
-    pl->M_pad = (g.taps * g.cin_g + pl->cg_tile - 1) / pl->cg_tile * pl->cg_tile;
-    pl->gt_bytes = align_up((size_t)g.N * (g.Cout / KC) * plane_out * 128);
-    pl->wt_bytes = align_up((size_t)g.G * pl->M_pad * g.cout_g * es);
-    pl->d_bytes = align_up(d_img * pl->n_chunk);
-    // enough workgroups for eight rounds or so of the chip's 2 x CUs slots
-    while (pl->parts < 8 && s_tiles * pl->parts < 4096 && g.ch_per_dg % (2 * pl->parts * pl->sCH) == 0)
-      pl->parts *= 2;
-    if (staged) pl->mx_bytes = kAlign;
-    if (pl->parts > 1) pl->part_bytes = align_up((size_t)pl->parts * g.N * g.DG * 3 * g.taps * plane_out * 4);
-  }
-  if (pl->wgemm) {
-    const long kpx = 128 / (long)es;  // pixels per K step
-    pl->P_pad = ((long)plane_out + kpx - 1) / kpx * kpx;
-    pl->col_bytes = align_up((size_t)pl->n_chunk * g.taps * g.Cin * pl->P_pad * es);
-    const int M = g.taps * g.cin_g;
-    pl->w_tile = (g.cout_g >= 192 && M >= kCgTileBig) ? kCgTileBig : kCgTile;
-    const long tiles = (long)g.G * ((g.cout_g + pl->w_tile - 1) / pl->w_tile) * ((M + pl->w_tile - 1) / pl->w_tile);
-    // one round of workgroups (256-tiles: one per CU, 128-tiles: two), shares of at least 8 K steps
-    const long slots = pl->w_tile == kCgTileBig ? 256 : 512;
-    const long work = (long)pl->n_chunk * (pl->P_pad / kpx);
-    pl->w_splits = (int)std::max<long>(1, std::min<long>(std::min<long>(work / 8, 64), slots / tiles));
-    pl->wpart_bytes = align_up((size_t)pl->w_splits * g.Cout * M * 4);
-    // grad_output rows go to LDS 16 bytes at a time: in place when they start aligned
-    if (plane_out % (16 / es) != 0 || ((uintptr_t)bp->grad_output % 16) != 0)
-      pl->gpad_bytes = align_up((size_t)g.N * g.Cout * pl->P_pad * es);
-  }
-  if (bp->grad_input && !pl->gemm) {
-    // (small problems keep the per-tap kernel: it has taps x more workgroups)
-    pl->R = window_margin(g, kBwdTile, kBwdTile, kBwdWindowBytes / (4 * kBwdChunk), &pl->WH, &pl->WW);
-    const long n_tiles = (long)g.N * g.DG * ((g.Ho + kBwdTile - 1) / kBwdTile) * ((g.Wo + kBwdTile - 1) / kBwdTile);
-    pl->tiled = pl->R >= 1 && (n_tiles >= 512 || forced);
-  }
-}
-
-template <typename E>
-int run_backward_typed(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan &pl, hipStream_t st) {
-  const mdcn_params *p = &bp->conv;
-  constexpr int KC = 128 / (int)sizeof(E);
-  const long plane_out = (long)g.Ho * g.Wo;
-  const OffMaskView om = dense_view(p->offset, p->mask, g);
-  unsigned char *ws = (unsigned char *)p->workspace;
-  auto blocks_for = [](long n) { return (int)std::max<long>(1, std::min<long>((n + 255) / 256, 1L << 20)); };
-  int rc = MDCN_OK;
-  auto check = [&]() { if (hipGetLastError() != hipSuccess) rc = MDCN_ERR_LAUNCH; };
-
-  const long n_in = (long)g.N * g.Cin * g.H * g.W;
-  const long n_w = (long)g.Cout * g.cin_g * g.taps;
-  float *gin32 = pl.gin_bytes ? (float *)ws : (float *)bp->grad_input;
-  float *gw32 = pl.gw_bytes ? (float *)(ws + pl.gin_bytes) : (float *)bp->grad_weight;
-  float *gb32 = pl.gb_bytes ? (float *)(ws + pl.gin_bytes + pl.gw_bytes) : (float *)bp->grad_bias;
-  uint32_t *maxima = (uint32_t *)(ws + pl.gin_bytes + pl.gw_bytes + pl.gb_bytes);  // [0] |d|, [1] |mask|
-  unsigned char *xt = ws + pl.gin_bytes + pl.gw_bytes + pl.gb_bytes + pl.mx_bytes;
-  unsigned char *gT = xt + pl.xt_bytes;
-  unsigned char *wT = gT + pl.gt_bytes;
-  unsigned char *D = wT + pl.wt_bytes;
-  unsigned char *col = D + pl.d_bytes;
-  const long off_total = (long)g.N * g.DG * 2 * g.taps * plane_out, mask_total = off_total / 2;
-  float *poff = (float *)(col + pl.col_bytes);
-  float *pmask = poff + (long)pl.parts * off_total;
-  float *wpart = (float *)(col + pl.col_bytes + pl.part_bytes);
-  const bool wgemm = pl.wgemm;
-  unsigned char *gpad = (unsigned char *)wpart + pl.wpart_bytes;
-  const bool gemm = pl.gemm;
-
-  if (bp->grad_input) {
-    hipLaunchKernelGGL(fill_zero_kernel<float>, dim3(blocks_for(n_in / 4 + 1)), dim3(256), 0, st, gin32, n_in);  // (16 bytes per thread)
-    check();
-  }
-  if (bp->grad_weight) {
-    hipLaunchKernelGGL(fill_zero_kernel<float>, dim3(blocks_for(n_w / 4 + 1)), dim3(256), 0, st, gw32, n_w);
-    check();
-  }
-
-  if (gemm || wgemm) {
-    {  // zero-bordered copy of the input in 32-byte records (what the scatter kernel reads per corner)
-      constexpr int EPV = 16 / (int)sizeof(E);
-      const int n_pchunks = (g.H * g.W + 32 * EPV - 1) / (32 * EPV);
-      hipLaunchKernelGGL((relayout_vec_kernel<E, true, 32>), dim3((unsigned)((long)g.N * (g.Cin / KC) * n_pchunks)),
-                         dim3(256), 0, st, g, (const E *)p->input, (E *)xt, n_pchunks);
-      check();
-    }
-    if (gemm) {  // pixel-major grad_output, transposed weights
-      Geom gg = g;
-      gg.Cin = g.Cout;
-      gg.H = g.Ho;
-      gg.W = g.Wo;
-      constexpr int EPV = 16 / (int)sizeof(E);
-      const int o_pchunks = (int)((plane_out + 32 * EPV - 1) / (32 * EPV));
-      hipLaunchKernelGGL((relayout_vec_kernel<E, false>), dim3((unsigned)((long)g.N * (g.Cout / KC) * o_pchunks)),
-                         dim3(256), 0, st, gg, (const E *)bp->grad_output, (E *)gT, o_pchunks);
-      check();
-      if (pl.mx_bytes) {
-        hipLaunchKernelGGL(fill_zero_kernel<uint32_t>, dim3(1), dim3(256), 0, st, maxima, 2L);
-        check();
-        if (p->mask) {
-          const long n_mask = (long)g.N * g.DG * g.taps * plane_out;
-          hipLaunchKernelGGL(absmax_kernel<E>, dim3(std::min(blocks_for(n_mask / 8), 256)), dim3(256), 0, st,
-                             (const E *)p->mask, n_mask, maxima + 1);
-          check();
-        }
-      }
-      const long wtotal = (long)g.G * pl.M_pad * g.cout_g;
-      hipLaunchKernelGGL(pack_weight_t_kernel<E>, dim3(blocks_for(wtotal)), dim3(256), 0, st, g,
-                         (const E *)p->weight, (E *)wT, pl.M_pad, wtotal);
-      check();
-    }
-    if (wgemm && pl.gpad_bytes) {
-      const long rows = (long)g.N * g.Cout;
-      hipLaunchKernelGGL(pad_rows_kernel<E>, dim3(blocks_for(rows * pl.P_pad)), dim3(256), 0, st,
-                         (const E *)bp->grad_output, (E *)gpad, rows, (int)plane_out, pl.P_pad);
-      check();
-    }
-    if (wgemm && pl.P_pad > plane_out) {
-      const long rows = (long)pl.n_chunk * g.taps * g.Cin;
-      hipLaunchKernelGGL(zero_col_pad_kernel<E>, dim3(blocks_for(rows * (pl.P_pad - plane_out))), dim3(256), 0, st,
-                         (E *)col, rows, (int)plane_out, pl.P_pad);
-      check();
-    }
-    for (int n0 = 0; n0 < g.N; n0 += pl.n_chunk) {
-      const int nb = std::min(pl.n_chunk, g.N - n0);
-      if (gemm) {
-        ColGradArgs ca;
-        ca.wT = wT;
-        ca.gT = gT;
-        ca.D = D;
-        ca.P = (int)plane_out;
-        ca.px_tiles = (int)((plane_out + pl.cg_tile - 1) / pl.cg_tile);
-        ca.m_tiles = pl.M_pad / pl.cg_tile;
-        ca.M = g.taps * g.cin_g;
-        ca.M_pad = pl.M_pad;
-        ca.cin_g = g.cin_g;
-        ca.cout_g = g.cout_g;
-        ca.taps = g.taps;
-        ca.G = g.G;
-        ca.Cin = g.Cin;
-        ca.Cout = g.Cout;
-        ca.kslabs = g.cout_g / KC;
-        ca.n0 = n0;
-        ca.dmax = pl.mx_bytes ? maxima : nullptr;
-        ca.total = (long)nb * g.G * ca.px_tiles * ca.m_tiles;
-        if (pl.cg_tile == kCgTileBig)
-          hipLaunchKernelGGL((bwd_colgrad_kernel<E, kCgTileBig>), dim3((unsigned)((ca.total + 7) / 8 * 8)),
-                             dim3(2 * kCgTileBig), 0, st, ca);
-        else
-          hipLaunchKernelGGL((bwd_colgrad_kernel<E, kCgTile>), dim3((unsigned)((ca.total + 7) / 8 * 8)),
-                             dim3(2 * kCgTile), 0, st, ca);
-        check();
-      }
-      BwdScatterArgs sa;
-      sa.g = g;
-      sa.xt = xt;
-      sa.om = om;
-      sa.D = gemm ? D : nullptr;
-      sa.gin32 = gin32;
-      sa.goff = bp->grad_offset;
-      sa.gmask = bp->grad_mask;
-      sa.col = wgemm ? col : nullptr;
-      sa.P_pad = pl.P_pad;
-      sa.tiles_x = (g.Wo + kScTW - 1) / kScTW;
-      sa.tiles_y = (g.Ho + kScTH - 1) / kScTH;
-      sa.R = pl.sR;
-      sa.WH = pl.sWH;
-      sa.WW = pl.sWW;
-      sa.n0 = n0;
-      sa.parts = gemm ? pl.parts : 1;
-      sa.poff = poff;
-      sa.pmask = pmask;
-      sa.off_total = off_total;
-      sa.mask_total = mask_total;
-      sa.dmax = maxima;
-      sa.mmax = p->mask ? maxima + 1 : nullptr;
-      const long sblocks = (long)nb * g.DG * sa.tiles_y * sa.tiles_x;
-      {
-        // 16-bit tensors: 32-bit fixed-point window (needs the maxima the data path computes;
-        // a columns-only call adds nothing to the window); fp32 tensors: doubles
-        constexpr bool k16 = sizeof(E) == 2;
-        using WT = typename std::conditional<k16, int32_t, double>::type;
-        constexpr int CHB = k16 ? 16 : 8;
-        const dim3 sgrid((unsigned)sblocks, (unsigned)sa.parts);
-        auto launch = [&](auto chv) {
-          constexpr int CHS = decltype(chv)::value;
-          if (gemm && wgemm)
-            hipLaunchKernelGGL((bwd_scatter_kernel<E, CHS, WT, true, true>), sgrid, dim3(256), 0, st, sa);
-          else if (gemm)
-            hipLaunchKernelGGL((bwd_scatter_kernel<E, CHS, WT, true, false>), sgrid, dim3(256), 0, st, sa);
-          else
-            hipLaunchKernelGGL((bwd_scatter_kernel<E, CHS, WT, false, true>), sgrid, dim3(256), 0, st, sa);
-        };
-        if (pl.sCH == CHB)
-          launch(std::integral_constant<int, CHB>());
-        else
-          launch(std::integral_constant<int, CHB / 2>());
-      }
-      check();
-      if (wgemm) {
-        WGradArgs wa;
-        wa.gout = pl.gpad_bytes ? (const void *)gpad : bp->grad_output;
-        wa.a_pitch = pl.gpad_bytes ? pl.P_pad : plane_out;
-        wa.col = col;
-        wa.part = wpart;
-        wa.P = (int)plane_out;
-        wa.P_pad = pl.P_pad;
-        wa.ksteps = (int)(pl.P_pad / KC);
-        wa.nb = nb;
-        wa.n0 = n0;
-        wa.M = g.taps * g.cin_g;
-        wa.cin_g = g.cin_g;
-        wa.cout_g = g.cout_g;
-        wa.taps = g.taps;
-        wa.G = g.G;
-        wa.Cin = g.Cin;
-        wa.Cout = g.Cout;
-        const int wtile = pl.w_tile;
-        wa.co_tiles = (g.cout_g + wtile - 1) / wtile;
-        wa.m_tiles = (wa.M + wtile - 1) / wtile;
-        const long tiles = (long)g.G * wa.co_tiles * wa.m_tiles;
-        wa.splits = pl.w_splits;
-        wa.total = tiles * wa.splits;
-        if (wtile == kCgTileBig)
-          hipLaunchKernelGGL((bwd_wgrad_kernel<E, kCgTileBig>), dim3((unsigned)((wa.total + 7) / 8 * 8)),
-                             dim3(2 * kCgTileBig), 0, st, wa);
-        else
-          hipLaunchKernelGGL((bwd_wgrad_kernel<E, kCgTile>), dim3((unsigned)((wa.total + 7) / 8 * 8)),
-                             dim3(2 * kCgTile), 0, st, wa);
-        check();
-        hipLaunchKernelGGL(wgrad_reduce_kernel, dim3(blocks_for(n_w / 4 + 1)), dim3(256), 0, st, wpart, gw32, wa.splits,
-                           g.cin_g, g.taps, n_w);
-        check();
-      }
-    }
-  }
-
-  if (bp->grad_input) {
-    if (gemm) {
-      if (pl.parts > 1) {
-        hipLaunchKernelGGL(combine_parts_kernel<E>, dim3(blocks_for(off_total / 4 + 1)), dim3(256), 0, st, poff,
-                           (E *)bp->grad_offset, off_total, pl.parts);
-        check();
-        if (bp->grad_mask) {
-          hipLaunchKernelGGL(combine_parts_kernel<E>, dim3(blocks_for(mask_total / 4 + 1)), dim3(256), 0, st, pmask,
-                             (E *)bp->grad_mask, mask_total, pl.parts);
-          check();
-        }
-      }
-    } else if (pl.tiled) {
-      BwdDataTiledArgs da;
-      da.g = g;
-      da.input = p->input;
-      da.om = om;
-      da.weight = p->weight;
-      da.gout = bp->grad_output;
-      da.gin32 = gin32;
-      da.goff = bp->grad_offset;
-      da.gmask = bp->grad_mask;
-      da.tiles_x = (g.Wo + kBwdTile - 1) / kBwdTile;
-      da.tiles_y = (g.Ho + kBwdTile - 1) / kBwdTile;
-      da.R = pl.R;
-      da.WH = pl.WH;
-      da.WW = pl.WW;
-      const long blocks = (long)g.N * g.DG * da.tiles_y * da.tiles_x;
-      hipLaunchKernelGGL(bwd_data_tiled_kernel<E>, dim3((unsigned)blocks), dim3(256), 0, st, da);
-      check();
-    } else {
-      const int rows = g.N * g.DG * g.taps;  // (image, deformable group, tap)
-      const dim3 grid((unsigned)((plane_out + 255) / 256), (unsigned)std::min(rows, 65535));
-      hipLaunchKernelGGL(bwd_data_kernel<E>, grid, dim3(256), 0, st, g, (const E *)p->input, om,
-                         (const E *)p->weight, (const E *)bp->grad_output, gin32,
-                         (E *)bp->grad_offset, (E *)bp->grad_mask, rows);
-      check();
-    }
-    if (pl.gin_bytes) {
-      hipLaunchKernelGGL(round_kernel<E>, dim3(blocks_for(n_in / 8 + 1)), dim3(256), 0, st, gin32,  // (8 elements per thread)
-                         (E *)bp->grad_input, n_in);
-      check();
-    }
-  }
-  if (bp->grad_weight) {
-    if (!wgemm) {
-      BwdWeightArgs wa;
-      wa.g = g;
-      wa.input = p->input;
-      wa.om = om;
-      wa.gout = bp->grad_output;
-      wa.gw32 = gw32;
-      wa.k_tiles = (g.cin_g * g.taps + 63) / 64;
-      wa.co_tiles = (g.cout_g + 255) / 256;
-      wa.px_chunks = (int)((plane_out + 63) / 64);
-      const long tiles = (long)wa.k_tiles * wa.co_tiles * g.G;
-      const long work = (long)g.N * wa.px_chunks;
-      wa.splits = (int)std::max<long>(1, std::min<long>(work, (4L * num_cus() + tiles - 1) / tiles));
-      wa.g_vec_ok = (plane_out % (16 / (long)sizeof(E)) == 0) && (((uintptr_t)bp->grad_output % 16) == 0);
-      hipLaunchKernelGGL(bwd_weight_kernel<E>, dim3((unsigned)tiles, (unsigned)wa.splits), dim3(256), 0,
-                         st, wa);
-      check();
-    }
-    if (pl.gw_bytes) {
-      hipLaunchKernelGGL(round_kernel<E>, dim3(blocks_for(n_w / 8 + 1)), dim3(256), 0, st, gw32,
-                         (E *)bp->grad_weight, n_w);
-      check();
-    }
-  }
-  if (bp->grad_bias) {
-    hipLaunchKernelGGL(fill_zero_kernel<float>, dim3(blocks_for(g.Cout)), dim3(256), 0, st, gb32, (long)g.Cout);
-    check();
-    const int runs = (int)((plane_out + kBiasRun - 1) / kBiasRun);
-    const int splits = (int)std::min<long>((long)g.N * runs, 64);
-    hipLaunchKernelGGL(bwd_bias_kernel<E>, dim3(g.Cout, splits), dim3(256), 0, st, g,
-                       (const E *)bp->grad_output, gb32, runs, splits);
-    check();
-    if (pl.gb_bytes) {
-      hipLaunchKernelGGL(round_kernel<E>, dim3(blocks_for(g.Cout)), dim3(256), 0, st, gb32,
-                         (E *)bp->grad_bias, (long)g.Cout);
-      check();
-    }
-  }
-  return rc;
-}
-
-// Double precision: grad_input by atomics into the zeroed tensor, everything else
-// has one owner; no workspace.
-int run_backward_f64(const mdcn_bwd_params *bp, const Geom &g, hipStream_t st) {
-  const mdcn_params *p = &bp->conv;
-  const long plane_out = (long)g.Ho * g.Wo;
-  auto blocks_for = [](long n) { return (int)std::max<long>(1, std::min<long>((n + 255) / 256, 1L << 20)); };
-  int rc = MDCN_OK;
-  auto check = [&]() { if (hipGetLastError() != hipSuccess) rc = MDCN_ERR_LAUNCH; };
-  if (bp->grad_input) {
-    const long n_in = (long)g.N * g.Cin * g.H * g.W;
-    hipLaunchKernelGGL(f64_zero_kernel, dim3(blocks_for(n_in)), dim3(256), 0, st, (double *)bp->grad_input, n_in);
-    check();
-    const long total = (long)g.N * g.DG * g.taps * plane_out;
-    hipLaunchKernelGGL(f64_bwd_data_kernel, dim3(blocks_for(total)), dim3(256), 0, st, g, (const double *)p->input,
-                       (const double *)p->offset, (const double *)p->mask, (const double *)p->weight,
-                       (const double *)bp->grad_output, (double *)bp->grad_input, (double *)bp->grad_offset,
-                       (double *)bp->grad_mask, total);
-    check();
-  }
-  if (bp->grad_weight) {
-    const long n_w = (long)g.Cout * g.cin_g * g.taps;
-    hipLaunchKernelGGL(f64_bwd_weight_kernel, dim3((unsigned)std::min<long>(n_w, 1L << 20)), dim3(256), 0, st, g,
-                       (const double *)p->input, (const double *)p->offset, (const double *)p->mask,
-                       (const double *)bp->grad_output, (double *)bp->grad_weight);
-    check();
-  }
-  if (bp->grad_bias) {
-    hipLaunchKernelGGL(f64_bwd_bias_kernel, dim3((unsigned)std::min(g.Cout, 65535)), dim3(256), 0, st, g,
-                       (const double *)bp->grad_output, (double *)bp->grad_bias);
-    check();
-  }
-  return rc;
-}
-
 int check_bwd(const mdcn_bwd_params *bp, Geom *g, bool need_ptrs) {
   if (!bp) return MDCN_ERR_NULL;
   const mdcn_params *p = &bp->conv;
@@ -1258,7 +800,7 @@ int check_bwd(const mdcn_bwd_params *bp, Geom *g, bool need_ptrs) {
   if (p->dtype == MDCN_F64 && forced_fused(p->path)) return MDCN_ERR_PATH;
   if (forced_fused(p->path)) {  // asked for the tiled kernels: the shape must allow them
     BwdPlan pl;
-    make_bwd_plan(bp, *g, &pl);
+    make_bwd_plan(bp, *g, g_bwd_pass_bytes.load(), &pl);
     if ((data && !pl.tiled && !pl.gemm) || (!data && bp->grad_weight && !pl.wgemm)) return MDCN_ERR_PATH;
   }
   return MDCN_OK;
@@ -1387,7 +929,7 @@ size_t mdcn_backward_workspace_bytes(const mdcn_bwd_params *bp) {
   Geom g;
   if (check_bwd(bp, &g, false) != MDCN_OK) return 0;
   BwdPlan pl;
-  make_bwd_plan(bp, g, &pl);
+  make_bwd_plan(bp, g, g_bwd_pass_bytes.load(), &pl);
   return pl.total();
 }
 
@@ -1396,18 +938,12 @@ int mdcn_backward(const mdcn_bwd_params *bp, void *hip_stream) {
   const int rc = check_bwd(bp, &g, true);
   if (rc != MDCN_OK) return rc;
   BwdPlan pl;
-  make_bwd_plan(bp, g, &pl);
+  make_bwd_plan(bp, g, g_bwd_pass_bytes.load(), &pl);
   const size_t need = pl.total();
   const mdcn_params *p = &bp->conv;
   if (need > 0 && (!p->workspace || p->workspace_bytes < need || ((uintptr_t)p->workspace % kAlign) != 0))
     return MDCN_ERR_WORKSPACE;
-  hipStream_t st = (hipStream_t)hip_stream;
-  switch (p->dtype) {
-    case MDCN_F64: return run_backward_f64(bp, g, st);
-    case MDCN_F32: return run_backward_typed<float>(bp, g, pl, st);
-    case MDCN_F16: return run_backward_typed<f16_t>(bp, g, pl, st);
-    default: return run_backward_typed<bf16_t>(bp, g, pl, st);
-  }
+  return run_backward(bp, g, pl, (hipStream_t)hip_stream);
 }
 
 int mdcn_pack_forward_timed(const mdcn_pack_params *pp, void *hip_stream, float ms[5]) {

@@ -1,0 +1,535 @@
+// Backward: plan, workspace carving and kernel launches.
+#include <algorithm>
+#include <type_traits>
+
+#include "mdcn_backward.h"
+#include "mdcn_backward_ends.h"
+#include "mdcn_backward_gemm.h"
+#include "mdcn_f64.h"
+#include "mdcn_fused.h"
+#include "mdcn_host.h"
+#include "mdcn_prepass.h"
+
+namespace mdcn {
+
+namespace {
+
+// Largest margin R (up to 8) for which the LDS window of a th x tw output-pixel
+// tile fits max_px pixels; -1 if even R = 0 does not.
+int window_margin(const Geom &g, int th, int tw, long max_px, int *WH, int *WW) {
+  const long base_h = (long)(th - 1) * g.sh + (long)(g.kh - 1) * g.dh + 2;
+  const long base_w = (long)(tw - 1) * g.sw + (long)(g.kw - 1) * g.dw + 2;
+  int R = -1;
+  while (R < 8 && (base_h + 2 * (R + 1)) * (base_w + 2 * (R + 1)) <= max_px) ++R;
+  *WH = (int)base_h + 2 * std::max(R, 0);
+  *WW = (int)base_w + 2 * std::max(R, 0);
+  return R;
+}
+
+}  // namespace
+
+void make_bwd_plan(const mdcn_bwd_params *bp, const Geom &g, uint64_t pass_bytes, BwdPlan *pl) {
+  const bool f64 = bp->conv.dtype == MDCN_F64;
+  const bool staged = bp->conv.dtype != MDCN_F32 && !f64;
+  const size_t es = elem_size(bp->conv.dtype);
+  pl->gin_bytes = (staged && bp->grad_input) ? align_up((size_t)g.N * g.Cin * g.H * g.W * 4) : 0;
+  pl->gw_bytes = (staged && bp->grad_weight) ? align_up((size_t)g.Cout * g.cin_g * g.taps * 4) : 0;
+  pl->gb_bytes = (staged && bp->grad_bias) ? align_up((size_t)g.Cout * 4) : 0;
+  pl->mx_bytes = 0;
+  pl->tiled = pl->gemm = pl->wgemm = false;
+  pl->xt_bytes = pl->gt_bytes = pl->wt_bytes = pl->d_bytes = pl->col_bytes = pl->part_bytes = pl->wpart_bytes = 0;
+  pl->w_tile = kCgTile;
+  pl->w_splits = 1;
+  pl->gpad_bytes = 0;
+  pl->bsplits = 0;
+  pl->im = pl->om = ChanMap{1, 1, 1, 1, 1};
+  pl->parts = 1;
+  pl->n_chunk = g.N;
+  pl->M_pad = 0;
+  pl->cg_tile = kCgTile;
+  pl->P_pad = 0;
+  pl->R = pl->sR = -1;
+  pl->WH = pl->WW = pl->sWH = pl->sWW = 0;
+  const int path = forced_fused(bp->conv.path) ? MDCN_PATH_FUSED : bp->conv.path;
+  if (path == MDCN_PATH_DIRECT || g.taps > kBwdTapsMax || f64) return;
+  const bool forced = path == MDCN_PATH_FUSED;
+  const size_t plane_out = (size_t)g.Ho * g.Wo;
+
+  // Matrix-core paths, for every channel count (padded in the copies) and any number of tiles: a call of 42
+  // tiles (fp32, N=2, 256 channels, 50x84) takes 0.41 ms here and took 2.57 ms with a workgroup per tap, one
+  // whose channels fill nothing (bf16, N=4, 96 -> 72, 37x53) 0.12 ms instead of 0.90.  Channels per pass over the window: 16 / 8 of 32-bit fixed point (16-bit tensors),
+  // 8 / 4 doubles (fp32)
+  const int KC = (int)(128 / es);
+  const int ch_big = es == 2 ? 16 : 8;
+  int u = g.cin_g, v = g.ch_per_dg;
+  while (v) {
+    const int t = u % v;
+    u = v;
+    v = t;
+  }
+  const int seg = u;
+  auto padded = [](int n, int to) { return (n + to - 1) / to * to; };
+  pl->sCH = ch_big;
+  pl->sR = window_margin(g, kScTH, kScTW, kScWindowPx, &pl->sWH, &pl->sWW);
+  // fewer channels at a time buy a wider window, and less padding where segments are short
+  const bool pads_less = 4 * padded(seg, ch_big) > 5 * padded(seg, ch_big / 2);
+  if (pl->sR < 2 || pads_less) {
+    int wh, ww;
+    const int r = window_margin(g, kScTH, kScTW, 2 * kScWindowPx, &wh, &ww);
+    if (r > pl->sR || pads_less) {
+      pl->sCH = ch_big / 2;
+      pl->sR = r;
+      pl->sWH = wh;
+      pl->sWW = ww;
+    }
+  }
+  ChanMap &im = pl->im, &om = pl->om;
+  im.seg = seg;
+  im.segp = padded(seg, pl->sCH);
+  im.nseg = g.cin_g / seg;
+  im.cg = g.cin_g;
+  im.cgp = padded(im.nseg * im.segp, 32);
+  om.seg = om.cg = g.cout_g;
+  om.nseg = 1;
+  om.segp = om.cgp = padded(g.cout_g, KC);
+  const long s_tiles = (long)g.N * g.DG * ((g.Ho + kScTH - 1) / kScTH) * ((g.Wo + kScTW - 1) / kScTW);
+  const int cin_p = g.G * im.cgp;
+  const size_t d_img = (size_t)g.taps * cin_p * plane_out * es;
+  const bool mfma_ok = pl->sR >= 1 && d_img <= kBwdColGradCap && plane_out <= ((size_t)1 << 30) &&
+                       (size_t)g.H * g.W <= ((size_t)1 << 30);  // (plane offsets held in 32 bits)
+  if (mfma_ok) {
+    pl->gemm = bp->grad_input != nullptr;
+    pl->wgemm = bp->grad_weight != nullptr;
+  }
+  if (pl->gemm || pl->wgemm) {
+    pl->n_chunk = (int)std::min<uint64_t>((uint64_t)g.N, std::max<uint64_t>(1, pass_bytes / d_img));
+    pl->xt_bytes = align_up((size_t)g.N * cin_p * g.Hp * g.Wp * es);
+    pl->gw_bytes = 0;
+    // Workgroups per tile: enough for eight rounds or so of the chip's 2 x CUs slots
+    const int passes = g.ch_per_dg / seg * (im.segp / pl->sCH);
+    while (pl->parts < 8 && s_tiles * pl->parts < 4096 && 2 * pl->parts <= passes) pl->parts *= 2;
+    pl->bsplits = 1;
+    if (bp->grad_bias) {
+      const long runs = (long)g.N * (((long)plane_out + kBiasRun - 1) / kBiasRun);
+      pl->bsplits = (int)std::min<long>(runs, 64);
+      pl->gb_bytes = align_up((size_t)g.Cout * pl->bsplits * 4);
+    }
+  }
+  if (pl->gemm) {
+    pl->cg_tile = (g.taps * im.cgp >= kCgTileBig && plane_out >= (size_t)kCgTileBig) ? kCgTileBig : kCgTile;
+    pl->M_pad = padded(g.taps * im.cgp, pl->cg_tile);
+    pl->gt_bytes = align_up((size_t)g.N * g.G * om.cgp * plane_out * es);
+    pl->wt_bytes = align_up((size_t)g.G * pl->M_pad * om.cgp * es);
+    pl->d_bytes = align_up(d_img * pl->n_chunk);
+    pl->mx_bytes = 2 * kAlign;
+    if (pl->parts > 1) pl->part_bytes = align_up((size_t)pl->parts * g.N * g.DG * 3 * g.taps * plane_out * 4);
+  }
+  if (pl->wgemm) {
+    const long kpx = 128 / (long)es;  // pixels per K step
+    pl->P_pad = ((long)plane_out + kpx - 1) / kpx * kpx;
+    pl->col_bytes = align_up((size_t)pl->n_chunk * g.taps * cin_p * pl->P_pad * es);
+    const int M = g.taps * im.cgp;
+    pl->w_tile = (g.cout_g >= 192 && M >= kCgTileBig) ? kCgTileBig : kCgTile;
+    const long tiles = (long)g.G * ((g.cout_g + pl->w_tile - 1) / pl->w_tile) * ((M + pl->w_tile - 1) / pl->w_tile);
+    // one round of workgroups (256-tiles: one per CU, 128-tiles: two), shares of at least 8 K steps
+    const long slots = pl->w_tile == kCgTileBig ? 256 : 512;
+    const long work = (long)pl->n_chunk * (pl->P_pad / kpx);
+    pl->w_splits = (int)std::max<long>(1, std::min<long>(std::min<long>(work / 8, 64), slots / tiles));
+    pl->wpart_bytes = align_up((size_t)pl->w_splits * g.Cout * M * 4);
+    // grad_output rows go to LDS 16 bytes at a time: in place when they start aligned
+    if (plane_out % (16 / es) != 0 || ((uintptr_t)bp->grad_output % 16) != 0)
+      pl->gpad_bytes = align_up((size_t)g.N * g.Cout * pl->P_pad * es);
+  }
+  if (bp->grad_input && !pl->gemm) {
+    // (small problems keep the per-tap kernel: it has taps x more workgroups)
+    pl->R = window_margin(g, kBwdTile, kBwdTile, kBwdWindowBytes / (4 * kBwdChunk), &pl->WH, &pl->WW);
+    const long n_tiles = (long)g.N * g.DG * ((g.Ho + kBwdTile - 1) / kBwdTile) * ((g.Wo + kBwdTile - 1) / kBwdTile);
+    pl->tiled = pl->R >= 1 && (n_tiles >= 512 || forced);
+  }
+}
+
+namespace {
+
+// Any shape: tiled or per-tap kernels on the VALU, grad_weight by sampling on the fly.
+template <typename E>
+int run_backward_general(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan &pl, hipStream_t st) {
+  const mdcn_params *p = &bp->conv;
+  const long plane_out = (long)g.Ho * g.Wo;
+  const OffMaskView om = dense_view(p->offset, p->mask, g);
+  unsigned char *ws = (unsigned char *)p->workspace;
+  auto blocks_for = [](long n) { return (int)std::max<long>(1, std::min<long>((n + 255) / 256, 1L << 20)); };
+  int rc = MDCN_OK;
+  auto check = [&]() { if (hipGetLastError() != hipSuccess) rc = MDCN_ERR_LAUNCH; };
+
+  const long n_in = (long)g.N * g.Cin * g.H * g.W;
+  const long n_w = (long)g.Cout * g.cin_g * g.taps;
+  float *gin32 = pl.gin_bytes ? (float *)ws : (float *)bp->grad_input;
+  float *gw32 = pl.gw_bytes ? (float *)(ws + pl.gin_bytes) : (float *)bp->grad_weight;
+  float *gb32 = pl.gb_bytes ? (float *)(ws + pl.gin_bytes + pl.gw_bytes) : (float *)bp->grad_bias;
+
+  if (bp->grad_input) {
+    hipLaunchKernelGGL(fill_zero_kernel<float>, dim3(blocks_for(n_in / 4 + 1)), dim3(256), 0, st, gin32, n_in);  // (16 bytes per thread)
+    check();
+  }
+  if (bp->grad_weight) {
+    hipLaunchKernelGGL(fill_zero_kernel<float>, dim3(blocks_for(n_w / 4 + 1)), dim3(256), 0, st, gw32, n_w);
+    check();
+  }
+
+  if (bp->grad_input) {
+    if (pl.tiled) {
+      BwdDataTiledArgs da;
+      da.g = g;
+      da.input = p->input;
+      da.om = om;
+      da.weight = p->weight;
+      da.gout = bp->grad_output;
+      da.gin32 = gin32;
+      da.goff = bp->grad_offset;
+      da.gmask = bp->grad_mask;
+      da.tiles_x = (g.Wo + kBwdTile - 1) / kBwdTile;
+      da.tiles_y = (g.Ho + kBwdTile - 1) / kBwdTile;
+      da.R = pl.R;
+      da.WH = pl.WH;
+      da.WW = pl.WW;
+      const long blocks = (long)g.N * g.DG * da.tiles_y * da.tiles_x;
+      hipLaunchKernelGGL(bwd_data_tiled_kernel<E>, dim3((unsigned)blocks), dim3(256), 0, st, da);
+      check();
+    } else {
+      const int rows = g.N * g.DG * g.taps;  // (image, deformable group, tap)
+      const dim3 grid((unsigned)((plane_out + 255) / 256), (unsigned)std::min(rows, 65535));
+      hipLaunchKernelGGL(bwd_data_kernel<E>, grid, dim3(256), 0, st, g, (const E *)p->input, om,
+                         (const E *)p->weight, (const E *)bp->grad_output, gin32,
+                         (E *)bp->grad_offset, (E *)bp->grad_mask, rows);
+      check();
+    }
+    if (pl.gin_bytes) {
+      hipLaunchKernelGGL(round_kernel<E>, dim3(blocks_for(n_in / 8 + 1)), dim3(256), 0, st, gin32,  // (8 elements per thread)
+                         (E *)bp->grad_input, n_in);
+      check();
+    }
+  }
+  if (bp->grad_weight) {
+    {
+      BwdWeightArgs wa;
+      wa.g = g;
+      wa.input = p->input;
+      wa.om = om;
+      wa.gout = bp->grad_output;
+      wa.gw32 = gw32;
+      wa.k_tiles = (g.cin_g * g.taps + 63) / 64;
+      wa.co_tiles = (g.cout_g + 255) / 256;
+      wa.px_chunks = (int)((plane_out + 63) / 64);
+      const long tiles = (long)wa.k_tiles * wa.co_tiles * g.G;
+      const long work = (long)g.N * wa.px_chunks;
+      wa.splits = (int)std::max<long>(1, std::min<long>(work, (4L * num_cus() + tiles - 1) / tiles));
+      wa.g_vec_ok = (plane_out % (16 / (long)sizeof(E)) == 0) && (((uintptr_t)bp->grad_output % 16) == 0);
+      hipLaunchKernelGGL(bwd_weight_kernel<E>, dim3((unsigned)tiles, (unsigned)wa.splits), dim3(256), 0,
+                         st, wa);
+      check();
+    }
+    if (pl.gw_bytes) {
+      hipLaunchKernelGGL(round_kernel<E>, dim3(blocks_for(n_w / 8 + 1)), dim3(256), 0, st, gw32,
+                         (E *)bp->grad_weight, n_w);
+      check();
+    }
+  }
+  if (bp->grad_bias) {
+    hipLaunchKernelGGL(fill_zero_kernel<float>, dim3(blocks_for(g.Cout)), dim3(256), 0, st, gb32, (long)g.Cout);
+    check();
+    const int runs = (int)((plane_out + kBiasRun - 1) / kBiasRun);
+    const int splits = (int)std::min<long>((long)g.N * runs, 64);
+    hipLaunchKernelGGL(bwd_bias_kernel<E>, dim3(g.Cout, splits), dim3(256), 0, st, g,
+                       (const E *)bp->grad_output, gb32, runs, splits);
+    check();
+    if (pl.gb_bytes) {
+      hipLaunchKernelGGL(round_kernel<E>, dim3(blocks_for(g.Cout)), dim3(256), 0, st, gb32,
+                         (E *)bp->grad_bias, (long)g.Cout);
+      check();
+    }
+  }
+  return rc;
+}
+
+// The matrix-core path: pre-pass, then per pass of images column gradient, scatter / columns and weight product, then the
+// finishing pass.
+template <typename E>
+int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan &pl, hipStream_t st) {
+  const mdcn_params *p = &bp->conv;
+  constexpr int KC = 128 / (int)sizeof(E);
+  constexpr int EPV = 16 / (int)sizeof(E);
+  constexpr bool staged = sizeof(E) == 2;  // grad_input is summed in fp32 and rounded at the end
+  const long plane_out = (long)g.Ho * g.Wo;
+  const OffMaskView om = dense_view(p->offset, p->mask, g);
+  unsigned char *ws = (unsigned char *)p->workspace;
+  auto take = [&](size_t bytes) {
+    unsigned char *q = ws;
+    ws += bytes;
+    return q;
+  };
+  int rc = MDCN_OK;
+  auto check = [&]() { if (hipGetLastError() != hipSuccess) rc = MDCN_ERR_LAUNCH; };
+  const bool gemm = pl.gemm, wgemm = pl.wgemm;
+  const int cin_p = g.G * pl.im.cgp, cout_p = g.G * pl.om.cgp;
+
+  float *gin_staging = (float *)take(pl.gin_bytes);
+  float *gin32 = staged ? gin_staging : (float *)bp->grad_input;
+  float *bpart = (float *)take(pl.gb_bytes);
+  uint32_t *dmax = (uint32_t *)take(pl.mx_bytes);
+  float *mmax = (float *)dmax + kAlign / 4;
+  unsigned char *xt = take(pl.xt_bytes), *gT = take(pl.gt_bytes), *wT = take(pl.wt_bytes);
+  unsigned char *D = take(pl.d_bytes), *col = take(pl.col_bytes);
+  const long off_total = (long)g.N * g.DG * 2 * g.taps * plane_out, mask_total = off_total / 2;
+  float *poff = (float *)take(pl.part_bytes);
+  float *pmask = poff + (long)pl.parts * off_total;
+  float *wpart = (float *)take(pl.wpart_bytes);
+  unsigned char *gpad = take(pl.gpad_bytes);
+  const long n_in = (long)g.N * g.Cin * g.H * g.W;
+  const int mask_blocks = (int)std::max<long>(1, std::min<long>(mask_total / (256 * EPV), 64));
+
+  auto up = [](long n, long per) { return (int)((n + per - 1) / per); };
+  {
+    BwdPreArgs a;
+    a.g = g;
+    a.im = pl.im;
+    a.om = pl.om;
+    a.cin_p = cin_p;
+    a.cout_p = cout_p;
+    a.in = p->input;
+    a.gout = bp->grad_output;
+    a.w = p->weight;
+    a.mask = p->mask;
+    a.xt = xt;
+    a.gT = gT;
+    a.wT = wT;
+    a.gpad = gpad;
+    a.col = col;
+    a.gin32 = gin32;
+    a.n_in = n_in;
+    a.x_chunks = up((long)g.H * g.W, 32 * EPV);
+    a.g_chunks = up(plane_out, 32 * EPV);
+    a.P_pad = pl.P_pad;
+    a.col_rows = (long)pl.n_chunk * g.taps * cin_p;
+    a.M_pad = pl.M_pad;
+    a.dmax = dmax;
+    a.mmax = mmax;
+    a.n_mask = mask_total;
+    a.bpart = bpart;
+    a.bsplits = pl.bsplits;
+    const int jobs[kPreJobs] = {
+        g.N * up(cin_p, KC) * a.x_chunks,
+        gemm ? g.N * (cout_p / KC) * a.g_chunks : 0,
+        pl.gpad_bytes ? up((long)g.N * g.Cout * (pl.P_pad / EPV), 256) : 0,
+        gemm ? up(n_in, kPreZeroPerBlock) : 0,
+        wgemm && pl.P_pad > plane_out ? up(a.col_rows * (pl.P_pad - plane_out), kPrePadPerBlock) : 0,
+        gemm ? up((long)g.G * pl.M_pad * pl.om.cgp, 256) : 0,
+        gemm && staged ? mask_blocks : 0,
+        bp->grad_bias ? g.Cout * pl.bsplits : 0,
+    };
+    int total = 0;
+    for (int j = 0; j < kPreJobs; ++j) a.end[j] = total += jobs[j];
+    hipLaunchKernelGGL(bwd_prepass_kernel<E>, dim3((unsigned)total), dim3(256), 0, st, a);
+    check();
+  }
+  for (int n0 = 0; n0 < g.N; n0 += pl.n_chunk) {
+    const int nb = std::min(pl.n_chunk, g.N - n0);
+    if (gemm) {
+      ColGradArgs ca;
+      ca.wT = wT;
+      ca.gT = gT;
+      ca.D = D;
+      ca.P = (int)plane_out;
+      ca.px_tiles = (int)((plane_out + pl.cg_tile - 1) / pl.cg_tile);
+      ca.m_tiles = pl.M_pad / pl.cg_tile;
+      ca.M = g.taps * pl.im.cgp;
+      ca.M_pad = pl.M_pad;
+      ca.cin_g = pl.im.cgp;
+      ca.cout_g = pl.om.cgp;
+      ca.taps = g.taps;
+      ca.G = g.G;
+      ca.Cin = cin_p;
+      ca.Cout = cout_p;
+      ca.kslabs = pl.om.cgp / KC;
+      ca.n0 = n0;
+      ca.dmax = staged ? dmax : nullptr;
+      ca.total = (long)nb * g.G * ca.px_tiles * ca.m_tiles;
+      if (pl.cg_tile == kCgTileBig)
+        hipLaunchKernelGGL((bwd_colgrad_kernel<E, kCgTileBig>), dim3((unsigned)((ca.total + 7) / 8 * 8)),
+                           dim3(2 * kCgTileBig), 0, st, ca);
+      else
+        hipLaunchKernelGGL((bwd_colgrad_kernel<E, kCgTile>), dim3((unsigned)((ca.total + 7) / 8 * 8)),
+                           dim3(2 * kCgTile), 0, st, ca);
+      check();
+    }
+    BwdScatterArgs sa;
+    sa.g = g;
+    sa.xt = xt;
+    sa.om = om;
+    sa.D = gemm ? D : nullptr;
+    sa.gin32 = gin32;
+    sa.goff = bp->grad_offset;
+    sa.gmask = bp->grad_mask;
+    sa.col = wgemm ? col : nullptr;
+    sa.P_pad = pl.P_pad;
+    sa.tiles_x = (g.Wo + kScTW - 1) / kScTW;
+    sa.tiles_y = (g.Ho + kScTH - 1) / kScTH;
+    sa.R = pl.sR;
+    sa.WH = pl.sWH;
+    sa.WW = pl.sWW;
+    sa.n0 = n0;
+    sa.parts = pl.parts;
+    sa.im = pl.im;
+    sa.cin_p = cin_p;
+    sa.passes = g.ch_per_dg / pl.im.seg * (pl.im.segp / pl.sCH);
+    sa.poff = poff;
+    sa.pmask = pmask;
+    sa.off_total = off_total;
+    sa.mask_total = mask_total;
+    sa.dmax = dmax;
+    sa.mmax = p->mask ? mmax : nullptr;
+    sa.n_mmax = mask_blocks;
+    const long sblocks = (long)nb * g.DG * sa.tiles_y * sa.tiles_x;
+    {
+      // 16-bit tensors: 32-bit fixed-point window (needs the maxima the data path computes;
+      // a columns-only call adds nothing to the window); fp32 tensors: doubles
+      constexpr bool k16 = sizeof(E) == 2;
+      using WT = typename std::conditional<k16, int32_t, double>::type;
+      constexpr int CHB = k16 ? 16 : 8;
+      const dim3 sgrid((unsigned)sblocks, (unsigned)sa.parts);
+      auto launch = [&](auto chv) {
+        constexpr int CHS = decltype(chv)::value;
+        if (gemm && wgemm)
+          hipLaunchKernelGGL((bwd_scatter_kernel<E, CHS, WT, true, true>), sgrid, dim3(256), 0, st, sa);
+        else if (gemm)
+          hipLaunchKernelGGL((bwd_scatter_kernel<E, CHS, WT, true, false>), sgrid, dim3(256), 0, st, sa);
+        else
+          hipLaunchKernelGGL((bwd_scatter_kernel<E, CHS, WT, false, true>), sgrid, dim3(256), 0, st, sa);
+      };
+      if (pl.sCH == CHB)
+        launch(std::integral_constant<int, CHB>());
+      else
+        launch(std::integral_constant<int, CHB / 2>());
+    }
+    check();
+    if (wgemm) {
+      WGradArgs wa;
+      wa.gout = pl.gpad_bytes ? (const void *)gpad : bp->grad_output;
+      wa.a_pitch = pl.gpad_bytes ? pl.P_pad : plane_out;
+      wa.col = col;
+      wa.part = wpart;
+      wa.P = (int)plane_out;
+      wa.P_pad = pl.P_pad;
+      wa.ksteps = (int)(pl.P_pad / KC);
+      wa.nb = nb;
+      wa.n0 = n0;
+      wa.M = g.taps * pl.im.cgp;
+      wa.accumulate = n0 > 0;
+      wa.cout_g = g.cout_g;
+      wa.taps = g.taps;
+      wa.G = g.G;
+      wa.Cin = cin_p;
+      wa.Cout = g.Cout;
+      const int wtile = pl.w_tile;
+      wa.co_tiles = (g.cout_g + wtile - 1) / wtile;
+      wa.m_tiles = (wa.M + wtile - 1) / wtile;
+      const long tiles = (long)g.G * wa.co_tiles * wa.m_tiles;
+      wa.splits = pl.w_splits;
+      wa.total = tiles * wa.splits;
+      if (wtile == kCgTileBig)
+        hipLaunchKernelGGL((bwd_wgrad_kernel<E, kCgTileBig>), dim3((unsigned)((wa.total + 7) / 8 * 8)),
+                           dim3(2 * kCgTileBig), 0, st, wa);
+      else
+        hipLaunchKernelGGL((bwd_wgrad_kernel<E, kCgTile>), dim3((unsigned)((wa.total + 7) / 8 * 8)),
+                           dim3(2 * kCgTile), 0, st, wa);
+      check();
+    }
+  }
+
+  {
+    BwdFinArgs a;
+    a.g = g;
+    a.im = pl.im;
+    a.gin32 = gin32;
+    a.gin = bp->grad_input;
+    a.n_in = n_in;
+    a.poff = poff;
+    a.pmask = pmask;
+    a.goff = bp->grad_offset;
+    a.gmask = bp->grad_mask;
+    a.off_total = off_total;
+    a.mask_total = mask_total;
+    a.parts = pl.parts;
+    a.wpart = wpart;
+    a.gw = bp->grad_weight;
+    a.splits = pl.w_splits;
+    a.bpart = bpart;
+    a.gb = bp->grad_bias;
+    a.bsplits = pl.bsplits;
+    const int jobs[kFinJobs] = {
+        gemm && staged ? up(n_in, 1024) : 0,
+        gemm && pl.parts > 1 ? up(off_total, 1024) : 0,
+        gemm && pl.parts > 1 && bp->grad_mask ? up(mask_total, 1024) : 0,
+        wgemm ? g.Cout * up(pl.im.cgp, kFinWeightCh) : 0,
+        bp->grad_bias ? up(g.Cout, 256) : 0,
+    };
+    int total = 0;
+    for (int j = 0; j < kFinJobs; ++j) a.end[j] = total += jobs[j];
+    if (total > 0) {
+      hipLaunchKernelGGL(bwd_finish_kernel<E>, dim3((unsigned)total), dim3(256), 0, st, a);
+      check();
+    }
+  }
+  return rc;
+}
+
+template <typename E>
+int run_backward_typed(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan &pl, hipStream_t st) {
+  return pl.gemm || pl.wgemm ? run_backward_matrix<E>(bp, g, pl, st) : run_backward_general<E>(bp, g, pl, st);
+}
+
+// Double precision: grad_input by atomics into the zeroed tensor, everything else
+// has one owner; no workspace.
+int run_backward_f64(const mdcn_bwd_params *bp, const Geom &g, hipStream_t st) {
+  const mdcn_params *p = &bp->conv;
+  const long plane_out = (long)g.Ho * g.Wo;
+  auto blocks_for = [](long n) { return (int)std::max<long>(1, std::min<long>((n + 255) / 256, 1L << 20)); };
+  int rc = MDCN_OK;
+  auto check = [&]() { if (hipGetLastError() != hipSuccess) rc = MDCN_ERR_LAUNCH; };
+  if (bp->grad_input) {
+    const long n_in = (long)g.N * g.Cin * g.H * g.W;
+    hipLaunchKernelGGL(f64_zero_kernel, dim3(blocks_for(n_in)), dim3(256), 0, st, (double *)bp->grad_input, n_in);
+    check();
+    const long total = (long)g.N * g.DG * g.taps * plane_out;
+    hipLaunchKernelGGL(f64_bwd_data_kernel, dim3(blocks_for(total)), dim3(256), 0, st, g, (const double *)p->input,
+                       (const double *)p->offset, (const double *)p->mask, (const double *)p->weight,
+                       (const double *)bp->grad_output, (double *)bp->grad_input, (double *)bp->grad_offset,
+                       (double *)bp->grad_mask, total);
+    check();
+  }
+  if (bp->grad_weight) {
+    const long n_w = (long)g.Cout * g.cin_g * g.taps;
+    hipLaunchKernelGGL(f64_bwd_weight_kernel, dim3((unsigned)std::min<long>(n_w, 1L << 20)), dim3(256), 0, st, g,
+                       (const double *)p->input, (const double *)p->offset, (const double *)p->mask,
+                       (const double *)bp->grad_output, (double *)bp->grad_weight);
+    check();
+  }
+  if (bp->grad_bias) {
+    hipLaunchKernelGGL(f64_bwd_bias_kernel, dim3((unsigned)std::min(g.Cout, 65535)), dim3(256), 0, st, g,
+                       (const double *)bp->grad_output, (double *)bp->grad_bias);
+    check();
+  }
+  return rc;
+}
+
+}  // namespace
+
+int run_backward(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan &pl, hipStream_t st) {
+  switch (bp->conv.dtype) {
+    case MDCN_F64: return run_backward_f64(bp, g, st);
+    case MDCN_F32: return run_backward_typed<float>(bp, g, pl, st);
+    case MDCN_F16: return run_backward_typed<f16_t>(bp, g, pl, st);
+    default: return run_backward_typed<bf16_t>(bp, g, pl, st);
+  }
+}
+
+}  // namespace mdcn

@@ -1,0 +1,281 @@
+// The two launches at the ends of the matrix-core backward: everything its three
+// main kernels read that is not an input of the call (pre-pass), and everything
+// they leave as fp32 or partial sums turned into the gradients (finish).  Each is
+// one launch whose workgroups are dealt out to the jobs by ranges of the block
+// index: the jobs are independent, most are small, and a launch of its own costs
+// each some four microseconds on the device and as much on the host.
+#pragma once
+
+#include "mdcn_backward_gemm.h"
+#include "mdcn_prepass.h"
+
+namespace mdcn {
+
+constexpr int kPreJobs = 8;
+enum { kPreX, kPreG, kPreRows, kPreZero, kPreColPad, kPreWeight, kPreMask, kPreBias };
+
+struct BwdPreArgs {
+  Geom g;
+  ChanMap im, om;          // padded orders of the input and output channels
+  int cin_p, cout_p;
+  int end[kPreJobs];       // job j has the blocks from end[j - 1] on
+  const void *in, *gout, *w, *mask;
+  void *xt, *gT, *wT, *gpad, *col;
+  float *gin32;
+  long n_in;               // elements of gin32
+  int x_chunks, g_chunks;  // pixel chunks of the re-layouts
+  long P_pad;
+  long col_rows;           // rows of col whose padding is cleared
+  int M_pad;
+  uint32_t *dmax;          // cleared
+  float *mmax;             // one value per block of the mask job
+  long n_mask;
+  float *bpart;            // [Cout][bsplits]
+  int bsplits;
+};
+
+constexpr int kPreZeroPerBlock = 256 * 32;   // floats a block of the zero job clears
+constexpr int kPrePadPerBlock = 256 * 8;     // elements a block of the col-pad job clears
+
+template <typename E>
+__global__ __launch_bounds__(256) void bwd_prepass_kernel(BwdPreArgs a) {
+  constexpr int EPV = 16 / (int)sizeof(E);
+  const Geom &g = a.g;
+  const int tid = threadIdx.x;
+  const long plane = (long)g.Ho * g.Wo;
+  int b = (int)blockIdx.x;
+  if (b < a.end[kPreX]) {  // zero-bordered copy of the input in 32-byte records (what the scatter kernel reads per corner)
+    relayout_vec_block<E, true, 32, true>(g, (const E *)a.in, (E *)a.xt, a.x_chunks, b, a.im, a.cin_p);
+    return;
+  }
+  if (b < a.end[kPreG]) {  // pixel-major grad_output
+    Geom gg = g;
+    gg.Cin = g.Cout;
+    gg.H = g.Ho;
+    gg.W = g.Wo;
+    relayout_vec_block<E, false, 128, true>(gg, (const E *)a.gout, (E *)a.gT, a.g_chunks, b - a.end[kPreX], a.om, a.cout_p);
+    return;
+  }
+  if (b < a.end[kPreRows]) {  // grad_output with rows that start 16-byte aligned, zeros behind the image
+    const long per_row = a.P_pad / EPV;
+    const long i = (long)(b - a.end[kPreG]) * 256 + tid;
+    const long r = i / per_row;
+    const int p = (int)(i - r * per_row) * EPV;
+    if (r >= (long)g.N * g.Cout) return;
+    const E *src = (const E *)a.gout + r * plane + p;
+    uint4 v;
+    if (p + EPV <= plane) {
+      __builtin_memcpy(&v, src, 16);
+    } else {
+      E e[EPV];
+#pragma unroll
+      for (int k = 0; k < EPV; ++k) e[k] = p + k < plane ? src[k] : from_f32<E>(0.0f);
+      __builtin_memcpy(&v, e, 16);
+    }
+    *(uint4 *)((E *)a.gpad + i * EPV) = v;
+    return;
+  }
+  if (b < a.end[kPreZero]) {  // the fp32 grad_input the scatter kernel adds into
+    const long i0 = (long)(b - a.end[kPreRows]) * kPreZeroPerBlock;
+    const bool vec = ((uintptr_t)a.gin32 % 16) == 0;
+    for (int k = 0; k < kPreZeroPerBlock / 1024; ++k) {
+      const long i = i0 + (long)k * 1024 + tid * 4;
+      if (vec && i + 4 <= a.n_in) {
+        *(float4 *)(a.gin32 + i) = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      } else {
+        for (int j = 0; j < 4; ++j)
+          if (i + j < a.n_in) a.gin32[i + j] = 0.0f;
+      }
+    }
+    return;
+  }
+  if (b < a.end[kPreColPad]) {  // padding columns [P, P_pad) of the rows of the columns matrix
+    const int padn = (int)(a.P_pad - plane);
+    const long i0 = (long)(b - a.end[kPreZero]) * kPrePadPerBlock;
+    for (int k = 0; k < kPrePadPerBlock / 256; ++k) {
+      const long i = i0 + k * 256 + tid, r = i / padn;
+      if (r < a.col_rows) ((E *)a.col)[r * a.P_pad + plane + (i - r * padn)] = from_f32<E>(0.0f);
+    }
+    return;
+  }
+  if (b < a.end[kPreWeight]) {
+    // weight[Cout][cin_g][taps] -> wT[G][M_pad][om.cgp], row m = tap * im.cgp + padded channel, zero where
+    // either channel is padding and in the rows up to M_pad
+    const long total = (long)g.G * a.M_pad * a.om.cgp;
+    const long idx = (long)(b - a.end[kPreColPad]) * 256 + tid;
+    if (idx >= total) return;
+    long r = idx;
+    const int co = (int)(r % a.om.cgp);
+    r /= a.om.cgp;
+    const int m = (int)(r % a.M_pad);
+    const int grp = (int)(r / a.M_pad);
+    const int tap = m / a.im.cgp;
+    int room;
+    const int c = chan_source(a.im, m - tap * a.im.cgp, room);  // (of the first group: channel within a group)
+    E v = from_f32<E>(0.0f);
+    if (tap < g.taps && room > 0 && co < g.cout_g)
+      v = ((const E *)a.w)[((long)(grp * g.cout_g + co) * g.cin_g + c) * g.taps + tap];
+    ((E *)a.wT)[idx] = v;
+    return;
+  }
+  __shared__ float red[4];
+  if (b < a.end[kPreMask]) {  // largest |mask|, a share per block
+    const int nb = a.end[kPreMask] - a.end[kPreWeight], bi = b - a.end[kPreWeight];
+    if (bi == 0 && tid == 0) *a.dmax = 0u;
+    const E *x = (const E *)a.mask;
+    float mx = 0.0f;
+    if (x) {
+      const long nv = ((uintptr_t)x % 16) == 0 ? a.n_mask / EPV : 0;
+      for (long v = (long)bi * 256 + tid; v < nv; v += (long)nb * 256) {
+        const uint4 q = ((const uint4 *)x)[v];
+        const E *e = (const E *)&q;
+#pragma unroll
+        for (int i = 0; i < EPV; ++i) mx = fmaxf(mx, fabsf(to_f32(e[i])));
+      }
+      for (long i = nv * EPV + (long)bi * 256 + tid; i < a.n_mask; i += (long)nb * 256) mx = fmaxf(mx, fabsf(to_f32(x[i])));
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+    if ((tid & 63) == 0) red[tid >> 6] = mx;
+    __syncthreads();
+    if (tid == 0) a.mmax[bi] = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    return;
+  }
+  {  // sums of grad_output over the pixels, a share of an output channel's runs per block
+    const int bi = b - a.end[kPreMask];
+    const int co = bi / a.bsplits, split = bi - co * a.bsplits;
+    const int runs = (int)((plane + kBiasRun - 1) / kBiasRun);
+    float s = 0.0f;
+    for (int w = split; w < g.N * runs; w += a.bsplits) {
+      const int n = w / runs, p0 = (w - n * runs) * kBiasRun;
+      const int len = (int)min((long)kBiasRun, plane - p0);
+      const E *src = (const E *)a.gout + ((long)n * g.Cout + co) * plane + p0;
+      const int nv = len / EPV;
+#pragma unroll 4
+      for (int v = tid; v < nv; v += 256) {
+        uint4 q;
+        __builtin_memcpy(&q, src + (long)v * EPV, 16);
+        const E *e = (const E *)&q;
+#pragma unroll
+        for (int i = 0; i < EPV; ++i) s += to_f32(e[i]);
+      }
+      for (int i = nv * EPV + tid; i < len; i += 256) s += to_f32(src[i]);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+    if ((tid & 63) == 0) red[tid >> 6] = s;
+    __syncthreads();
+    if (tid == 0) a.bpart[(long)co * a.bsplits + split] = (red[0] + red[1]) + (red[2] + red[3]);
+  }
+}
+
+constexpr int kFinJobs = 5;
+enum { kFinInput, kFinOffset, kFinMask, kFinWeight, kFinBias };
+
+struct BwdFinArgs {
+  Geom g;
+  ChanMap im;
+  int end[kFinJobs];
+  const float *gin32;   // 16-bit tensors: fp32 grad_input
+  void *gin;
+  long n_in;
+  const float *poff, *pmask;   // [parts][...]
+  void *goff, *gmask;
+  long off_total, mask_total;
+  int parts;
+  const float *wpart;   // [splits][G][cout_g][taps * im.cgp]
+  void *gw;
+  int splits;
+  const float *bpart;   // [Cout][bsplits]
+  void *gb;
+  int bsplits;
+};
+
+// dst[0 .. n) = sum over `parts` of src[part][0 .. n), rounded once; four elements per thread.
+template <typename E>
+__device__ __forceinline__ void sum_parts_block(const float *__restrict__ src, E *__restrict__ dst, long n, int parts, int b) {
+  const long i = ((long)b * 256 + threadIdx.x) * 4;
+  if (i >= n) return;
+  if (n % 4 == 0 && (uintptr_t)src % 16 == 0) {
+    float4 s = *(const float4 *)(src + i);
+    for (int p = 1; p < parts; ++p) {
+      const float4 t = *(const float4 *)(src + (long)p * n + i);
+      s.x += t.x; s.y += t.y; s.z += t.z; s.w += t.w;
+    }
+    struct Out4 { E v[4]; } o;
+    o.v[0] = from_f32<E>(s.x); o.v[1] = from_f32<E>(s.y); o.v[2] = from_f32<E>(s.z); o.v[3] = from_f32<E>(s.w);
+    __builtin_memcpy(dst + i, &o, sizeof(o));
+    return;
+  }
+  for (int k = 0; k < 4 && i + k < n; ++k) {
+    float s = 0.0f;
+    for (int p = 0; p < parts; ++p) s += src[(long)p * n + i + k];
+    dst[i + k] = from_f32<E>(s);
+  }
+}
+
+constexpr int kFinWeightCh = 64;   // padded channels of a row a block of the weight job handles
+
+template <typename E>
+__global__ __launch_bounds__(256) void bwd_finish_kernel(BwdFinArgs a) {
+  const Geom &g = a.g;
+  const int tid = threadIdx.x;
+  const int b = (int)blockIdx.x;
+  if (b < a.end[kFinInput]) {
+    sum_parts_block<E>(a.gin32, (E *)a.gin, a.n_in, 1, b);
+    return;
+  }
+  if (b < a.end[kFinOffset]) {
+    sum_parts_block<E>(a.poff, (E *)a.goff, a.off_total, a.parts, b - a.end[kFinInput]);
+    return;
+  }
+  if (b < a.end[kFinMask]) {
+    sum_parts_block<E>(a.pmask, (E *)a.gmask, a.mask_total, a.parts, b - a.end[kFinOffset]);
+    return;
+  }
+  if (b < a.end[kFinWeight]) {
+    // A row (group, output channel), kFinWeightCh of its padded channels: the partial sums are read along the
+    // channels of a tap, summed in a fixed order and written along the taps of a channel.
+    __shared__ float tile[kBwdTapsMax * kFinWeightCh];
+    const int cblocks = (a.im.cgp + kFinWeightCh - 1) / kFinWeightCh;
+    const int bi = b - a.end[kFinMask];
+    const int row = bi / cblocks, c0 = (bi - row * cblocks) * kFinWeightCh;
+    const int nc = min(kFinWeightCh, a.im.cgp - c0);
+    const long M = (long)g.taps * a.im.cgp;
+    const long split_stride = (long)g.Cout * M;
+    for (int i = tid; i < g.taps * kFinWeightCh; i += 256) {
+      const int tap = i / kFinWeightCh, c = i - tap * kFinWeightCh;
+      float s = 0.0f;
+      if (c < nc) {
+        const float *src = a.wpart + (long)row * M + (long)tap * a.im.cgp + c0 + c;
+        int sp = 0;
+        for (; sp + 4 <= a.splits; sp += 4) {
+          float v[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) v[u] = src[(long)(sp + u) * split_stride];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) s += v[u];
+        }
+        for (; sp < a.splits; ++sp) s += src[(long)sp * split_stride];
+      }
+      tile[i] = s;
+    }
+    __syncthreads();
+    E *dst = (E *)a.gw + (long)row * g.cin_g * g.taps;
+    for (int i = tid; i < g.taps * nc; i += 256) {
+      const int c = i / g.taps, tap = i - c * g.taps;
+      int room;
+      const int cs = chan_source(a.im, c0 + c, room);  // (of the first group: channel within a group)
+      if (room > 0) dst[(long)cs * g.taps + tap] = from_f32<E>(tile[tap * kFinWeightCh + c]);
+    }
+    return;
+  }
+  const int co = (b - a.end[kFinWeight]) * 256 + tid;
+  if (co < g.Cout) {
+    float s = 0.0f;
+    for (int i = 0; i < a.bsplits; ++i) s += a.bpart[(long)co * a.bsplits + i];
+    ((E *)a.gb)[co] = from_f32<E>(s);
+  }
+}
+
+}  // namespace mdcn

@@ -15,8 +15,14 @@
 // store the forward's columns, from which grad_weight is a second plain product
 // (bwd_wgrad_kernel).
 // Both operands of the product are pixel-major / K-contiguous copies written by
-// small pre-passes (relayout_vec_kernel<E, false> for grad_output,
-// pack_weight_t_kernel for the weights).
+// the pre-pass (mdcn_backward_ends.h), which with the finishing pass holds
+// everything else a call needs: five launches in all.
+//
+// Channels that do not fill the tiles are padded in these copies: a segment of
+// the input's channels (those of one group and one deformable group) to whole
+// passes of the scatter kernel, a group's to a multiple of 32, the output
+// channels of a group to 128 bytes.  Padding is zero in every copy, so it adds nothing
+// and its gradients are zero and never written.
 #pragma once
 
 #include "mdcn_backward.h"
@@ -31,28 +37,8 @@ namespace mdcn {
 constexpr int kCgTile = 128;
 constexpr int kCgTileBig = 256;
 
-// weight[Cout][cin_g][taps] -> wT[G][M_pad][cout_g], row m = tap * cin_g + c,
-// zero rows from taps * cin_g up to M_pad (a multiple of kCgTile).
-template <typename E>
-__global__ __launch_bounds__(256) void pack_weight_t_kernel(Geom g, const E *__restrict__ w,
-                                                            E *__restrict__ wT, int M_pad, long total) {
-  for (long idx = (long)blockIdx.x * blockDim.x + threadIdx.x; idx < total;
-       idx += (long)gridDim.x * blockDim.x) {
-    long r = idx;
-    const int co = (int)(r % g.cout_g);
-    r /= g.cout_g;
-    const int m = (int)(r % M_pad);
-    const int grp = (int)(r / M_pad);
-    E v = from_f32<E>(0.0f);
-    if (m < g.taps * g.cin_g) {
-      const int tap = m / g.cin_g, c = m - tap * g.cin_g;
-      v = w[((long)(grp * g.cout_g + co) * g.cin_g + c) * g.taps + tap];
-    }
-    wT[idx] = v;
-  }
-}
-
 struct ColGradArgs {
+  // (channel counts are those of the padded orders, see BwdPlan)
   const void *wT;  // [G][M_pad][cout_g]
   const void *gT;  // [N][Cout / KC][P][KC], KC = 128 bytes of channels
   void *D;         // [images of the pass][Cin / 16][taps][P][16]
@@ -230,29 +216,6 @@ constexpr int kScWindowPx = kScWindowBytes / 64;
 // tile touches an entry at most once per channel.
 constexpr int kScMaxAdds = 256 * 9;
 
-// largest |x| of a tensor, as the bit pattern of a non-negative float
-template <typename E>
-__global__ __launch_bounds__(256) void absmax_kernel(const E *__restrict__ x, long n, uint32_t *out) {
-  float mx = 0.0f;
-  constexpr int EPV = 16 / (int)sizeof(E);  // elements per 16-byte load
-  const long nv = (((uintptr_t)x % 16) == 0) ? n / EPV : 0;
-  for (long v = (long)blockIdx.x * blockDim.x + threadIdx.x; v < nv; v += (long)gridDim.x * blockDim.x) {
-    const uint4 q = ((const uint4 *)x)[v];
-    const E *e = (const E *)&q;
-#pragma unroll
-    for (int i = 0; i < EPV; ++i) mx = fmaxf(mx, fabsf(to_f32(e[i])));
-  }
-  for (long i = nv * EPV + (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
-    mx = fmaxf(mx, fabsf(to_f32(x[i])));
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
-  __shared__ float wmax[4];
-  if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = mx;
-  __syncthreads();
-  if (threadIdx.x == 0)  // one atomic per workgroup: they all queue on one address
-    atomicMax(out, __float_as_uint(fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]))));
-}
-
 // CH consecutive channels (8 to 32 bytes) as floats.
 template <typename E, int CH>
 struct VecCh {
@@ -318,7 +281,10 @@ struct BwdScatterArgs {
   float *gin32;
   void *goff;
   void *gmask;     // null when unmodulated
-  void *col;       // columns of the pass [image][group][tap][channel of the group][P_pad], or null
+  void *col;       // columns of the pass [image][group][tap][padded channel of the group][P_pad], or null
+  ChanMap im;      // padded order of the input channels
+  int cin_p;       // ... how many there are
+  int passes;      // passes of CH channels over a deformable group's segments
   long P_pad;      // row pitch of col in elements
   int tiles_x, tiles_y;
   int WH, WW;      // window size in input pixels
@@ -328,38 +294,15 @@ struct BwdScatterArgs {
   // (blockIdx.y), so that the launch has several times more workgroups than the
   // chip has room for and its last round is short; with parts > 1 each writes its
   // share of the offset / mask sums as floats to poff / pmask ([part][layout of
-  // grad_offset / grad_mask]), which combine_parts_kernel adds up.
+  // grad_offset / grad_mask]), which bwd_finish_kernel adds up.
   int parts;
   float *poff, *pmask;
   long off_total, mask_total;  // elements of grad_offset / grad_mask
-  // fixed-point window (16-bit tensors): largest |d| and largest |mask| (null: 1)
-  const uint32_t *dmax, *mmax;
+  // fixed-point window (16-bit tensors): largest |d|, and n_mmax values whose largest is that of |mask| (null: 1)
+  const uint32_t *dmax;
+  const float *mmax;
+  int n_mmax;
 };
-
-// out[i] = sum over parts of part[p][i], rounded once.  Four elements per thread
-// and step where the parts start at multiples of 16 bytes (total a multiple of 4).
-template <typename E>
-__global__ __launch_bounds__(256) void combine_parts_kernel(const float *__restrict__ part, E *__restrict__ out,
-                                                            long total, int parts) {
-  const long first = (long)blockIdx.x * blockDim.x + threadIdx.x, stride = (long)gridDim.x * blockDim.x;
-  const long nv = (total % 4 == 0 && (uintptr_t)part % 16 == 0) ? total / 4 : 0;
-  struct Out4 { E v[4]; };
-  for (long i = first; i < nv; i += stride) {
-    float4 s = ((const float4 *)part)[i];
-    for (int p = 1; p < parts; ++p) {
-      const float4 t = ((const float4 *)(part + (long)p * total))[i];
-      s.x += t.x; s.y += t.y; s.z += t.z; s.w += t.w;
-    }
-    Out4 o;
-    o.v[0] = from_f32<E>(s.x); o.v[1] = from_f32<E>(s.y); o.v[2] = from_f32<E>(s.z); o.v[3] = from_f32<E>(s.w);
-    __builtin_memcpy(out + 4 * i, &o, sizeof(o));
-  }
-  for (long i = nv * 4 + first; i < total; i += stride) {
-    float s = 0.0f;
-    for (int p = 0; p < parts; ++p) s += part[(long)p * total + i];
-    out[i] = from_f32<E>(s);
-  }
-}
 
 // The window is not fp32: LDS single-precision atomic adds are slow on this
 // hardware (measured per wavefront instruction per CU: ds_add_f32 170 clocks,
@@ -392,7 +335,13 @@ __global__ __launch_bounds__(256, 2) void bwd_scatter_kernel(BwdScatterArgs a) {
   __shared__ __align__(16) WT win[DATA ? kScWindowBytes / sizeof(WT) : 4];
   float fx_scale = 1.0f, fx_inv = 1.0f;
   if (kFixed && DATA) {
-    const float bound = __uint_as_float(*a.dmax) * (a.mmax ? __uint_as_float(*a.mmax) : 1.0f) * (float)kScMaxAdds;
+    float mm = 1.0f;
+    if (a.mmax) {
+      mm = (int)(threadIdx.x & 63) < a.n_mmax ? a.mmax[threadIdx.x & 63] : 0.0f;
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) mm = fmaxf(mm, __shfl_xor(mm, o));
+    }
+    const float bound = __uint_as_float(*a.dmax) * mm * (float)kScMaxAdds;
     // largest power of two not above 2^30 / bound (any scale will do when everything is zero)
     const int e = (bound > 0.0f && bound < 3.0e38f) ? 29 - ilogbf(bound) : 0;
     fx_scale = ldexpf(1.0f, max(-120, min(120, e)));
@@ -436,9 +385,24 @@ __global__ __launch_bounds__(256, 2) void bwd_scatter_kernel(BwdScatterArgs a) {
     t_m[t] = msk[(long)tc * a.om.msk_ch];
   }
 
+  // This workgroup's passes of CH channels.  Pass i of the deformable group: segment i / (segp / CH) of the
+  // group, from padded channel c0 on; the tensor's channel cs, of which `room` are left in the segment.
   const int part = blockIdx.y;
-  const int ch_per_part = g.ch_per_dg / a.parts;
-  const int c_begin = dgi * g.ch_per_dg + part * ch_per_part, c_end = c_begin + ch_per_part;
+  const int ps_begin = (int)((long)a.passes * part / a.parts), ps_end = (int)((long)a.passes * (part + 1) / a.parts);
+  struct Pass {
+    int c0, cs, room, grp;
+  };
+  auto pass_at = [&](int i) {
+    const int per = a.im.segp / CH;
+    const int k = i / per, w = (i - k * per) * CH;
+    const int S = dgi * (g.ch_per_dg / a.im.seg) + k;   // segment of the tensor
+    Pass p;
+    p.grp = S / a.im.nseg;
+    p.c0 = p.grp * a.im.cgp + (S - p.grp * a.im.nseg) * a.im.segp + w;
+    p.cs = S * a.im.seg + w;
+    p.room = a.im.seg - w;
+    return p;
+  };
 
   // Window pixels this thread flushes (tid, tid + 256, ...) as offsets into an image plane, the same
   // in every pass; -1 for one outside the image or past the window (it only ever receives zeros).
@@ -485,28 +449,31 @@ __global__ __launch_bounds__(256, 2) void bwd_scatter_kernel(BwdScatterArgs a) {
     s.lx = s.inside ? px - fx : 0.0f;
     s.m = s.inside ? mask_value<E>(e_m, a.om.logit) : 0.0f;
     // corners outside the image read the copy's zero border
-    const E *xp = (const E *)a.xt + (((long)n * (g.Cin / RC) + c0 / RC) * slab_px) * RC + (c0 % RC) +
+    const E *xp = (const E *)a.xt + (((long)n * (a.cin_p / RC) + c0 / RC) * slab_px) * RC + (c0 % RC) +
                   ((long)(s.y0 + 1) * g.Wp + (s.x0 + 1)) * RC;
     s.r00.load(xp);
     s.r01.load(xp + RC);
     s.r10.load(xp + (long)g.Wp * RC);
     s.r11.load(xp + (long)(g.Wp + 1) * RC);
     if constexpr (DATA)
-      s.rd.load((const E *)a.D + (((long)nl * (g.Cin / 16) + (c0 >> 4)) * g.taps + tap) * plane_out * 16 + pix * 16 +
+      s.rd.load((const E *)a.D + (((long)nl * (a.cin_p / 16) + (c0 >> 4)) * g.taps + tap) * plane_out * 16 + pix * 16 +
                 (c0 & 15));
   };
   // A tap's loads are issued one tap ahead, in front of the previous tap's stores and atomics
   // (a wait for loads also waits for every older store, and the compiler cannot move a load
   // above a store that might alias it); the last tap of a pass fetches the first of the next.
   Sample cur;
-  fetch(c_begin, 0, t_dy[0], t_dx[0], t_m[0], cur);
+  Pass ps = pass_at(ps_begin);
+  fetch(ps.c0, 0, t_dy[0], t_dx[0], t_m[0], cur);
 
-  for (int c0 = c_begin; c0 < c_end; c0 += CH) {
+  for (int pi = ps_begin; pi < ps_end; ++pi) {
     if constexpr (DATA) __syncthreads();  // the window is zero: first fill or the previous pass's flush
+    const int c0 = ps.c0, cs = ps.cs;
     // row of the columns matrix of channel c0 at tap 0 (a chunk stays inside one group)
-    const int grp = c0 / g.cin_g;
-    E *cbase = (E *)a.col + (((long)nl * g.Cin + (long)grp * g.cin_g) * g.taps + (c0 - grp * g.cin_g)) * a.P_pad + pix;
-    const int c_next = min(c0 + CH, c_end - CH);  // (the last pass fetches its own first tap again: unused)
+    E *cbase = (E *)a.col +
+               (((long)nl * a.cin_p + (long)ps.grp * a.im.cgp) * g.taps + (c0 - ps.grp * a.im.cgp)) * a.P_pad + pix;
+    const Pass nps = pass_at(min(pi + 1, ps_end - 1));  // (the last pass fetches its own first tap again: unused)
+    const int c_next = nps.c0;
 #pragma unroll
     for (int tap = 0; tap < kBwdTapsMax; ++tap) {
       if (tap < g.taps) {
@@ -594,7 +561,7 @@ __global__ __launch_bounds__(256, 2) void bwd_scatter_kernel(BwdScatterArgs a) {
         }
         if constexpr (COL) {
           if (valid) {
-            E *crow = cbase + (long)tap * g.cin_g * a.P_pad;
+            E *crow = cbase + (long)tap * a.im.cgp * a.P_pad;
 #pragma unroll
             for (int cc = 0; cc < CH; ++cc) crow[(long)cc * a.P_pad] = cv[cc];
           }
@@ -609,8 +576,9 @@ __global__ __launch_bounds__(256, 2) void bwd_scatter_kernel(BwdScatterArgs a) {
             rd.unpack(d);
 #pragma unroll
             for (int cc = 0; cc < CH; ++cc) {
+              if (cc >= ps.room) break;
               const float t = d[cc] * m;
-              float *gi = a.gin32 + ((long)n * g.Cin + c0 + cc) * plane_in;
+              float *gi = a.gin32 + ((long)n * g.Cin + cs + cc) * plane_in;
               if (ok00) unsafeAtomicAdd(gi + o00, w00 * t);
               if (ok01) unsafeAtomicAdd(gi + o01, w01 * t);
               if (ok10) unsafeAtomicAdd(gi + o10, w10 * t);
@@ -623,7 +591,8 @@ __global__ __launch_bounds__(256, 2) void bwd_scatter_kernel(BwdScatterArgs a) {
     }
     if constexpr (DATA) {
       __syncthreads();  // every add into the window has landed
-      float *gplane = a.gin32 + ((long)n * g.Cin + c0) * plane_in;
+      // (padding channels only ever receive zeros, and zeros are not written)
+      float *gplane = a.gin32 + ((long)n * g.Cin + cs) * plane_in;
 #pragma unroll
       for (int j = 0; j < kSlots; ++j) {
         if (flush_at[j] >= 0) {
@@ -655,6 +624,7 @@ __global__ __launch_bounds__(256, 2) void bwd_scatter_kernel(BwdScatterArgs a) {
         }
       }
     }
+    ps = nps;
   }
   if constexpr (DATA) {
     if (valid) {
@@ -686,41 +656,18 @@ __global__ __launch_bounds__(256, 2) void bwd_scatter_kernel(BwdScatterArgs a) {
   }
 }
 
-// Zeroes the padding columns [P, P_pad) of every row of the columns matrix.
-template <typename E>
-__global__ __launch_bounds__(256) void zero_col_pad_kernel(E *col, long rows, int P, long P_pad) {
-  const int padn = (int)(P_pad - P);
-  const long total = rows * padn;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (long)gridDim.x * blockDim.x) {
-    const long r = i / padn;
-    col[r * P_pad + P + (i - r * padn)] = from_f32<E>(0.0f);
-  }
-}
-
-// dst[row][0 .. P_pad) = src[row][0 .. P), zeros behind: grad_output with rows that start 16-byte
-// aligned, for images whose pixel count is not a multiple of the copy granule.
-template <typename E>
-__global__ __launch_bounds__(256) void pad_rows_kernel(const E *__restrict__ src, E *__restrict__ dst, long rows,
-                                                       int P, long P_pad) {
-  const long total = rows * P_pad;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (long)gridDim.x * blockDim.x) {
-    const long r = i / P_pad;
-    const long p = i - r * P_pad;
-    dst[i] = p < P ? src[r * P + p] : from_f32<E>(0.0f);
-  }
-}
-
 struct WGradArgs {
   const void *gout;  // [N][Cout][a_pitch]: grad_output in place (a_pitch = P) or its padded copy (P_pad)
   long a_pitch;
-  const void *col;   // [images of the pass][G][taps][cin_g][P_pad]
+  const void *col;   // [images of the pass][G][taps][padded channels of a group][P_pad]
   float *part;       // partial sums [split][G][cout_g][M], every element written
+  int accumulate;    // 0: the first pass writes them; 1: a later one adds to them
   int P;
   long P_pad;
   int ksteps;        // P_pad / (pixels per 128 bytes)
   int nb, n0;        // images of the pass, first image
-  int M;             // taps * cin_g
-  int cin_g, cout_g, taps, G, Cin, Cout;
+  int M;             // taps * padded channels of a group
+  int cout_g, taps, G, Cin, Cout;   // (Cin: padded)
   int co_tiles, m_tiles;
   int splits;        // workgroups sharing the (image, K step) range of one tile
   long total;        // workgroups with work: G x co_tiles x m_tiles x splits
@@ -849,40 +796,12 @@ __global__ __launch_bounds__(TILE * 2, TILE == 128 ? 2 : 1) void bwd_wgrad_kerne
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int co = ct * TILE + wm * (TILE / 2) + mb * 32 + (r >> 2) * 8 + fhalf * 4 + (r & 3);
-        if (co < a.cout_g) part[(long)co * a.M + m] = acc[mb][nb][r];
+        if (co < a.cout_g) {
+          float *p = part + (long)co * a.M + m;
+          *p = a.accumulate ? *p + acc[mb][nb][r] : acc[mb][nb][r];
+        }
       }
     }
-}
-
-// gw32[(grp, co), (c, tap)] += sum over the shares of part[share][grp][co][m = tap * cin_g + c].
-__global__ __launch_bounds__(256) void wgrad_reduce_kernel(const float *__restrict__ part, float *__restrict__ gw32,
-                                                           int splits, int cin_g, int taps, long n_w) {
-  const int M = cin_g * taps;
-  // four consecutive elements per thread (M is a multiple of 32 here: they share a row and a tap), the shares
-  // in a fixed order with four loads in flight
-  for (long i = 4 * ((long)blockIdx.x * blockDim.x + threadIdx.x); i < n_w; i += 4 * (long)gridDim.x * blockDim.x) {
-    const long row = i / M;  // (grp, co)
-    const int m = (int)(i - row * M);
-    float4 sum = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    int sp = 0;
-    for (; sp + 4 <= splits; sp += 4) {
-      float4 v[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) v[u] = *(const float4 *)(part + (long)(sp + u) * n_w + i);
-#pragma unroll
-      for (int u = 0; u < 4; ++u) sum.x += v[u].x, sum.y += v[u].y, sum.z += v[u].z, sum.w += v[u].w;
-    }
-    for (; sp < splits; ++sp) {
-      const float4 v = *(const float4 *)(part + (long)sp * n_w + i);
-      sum.x += v.x, sum.y += v.y, sum.z += v.z, sum.w += v.w;
-    }
-    const int tap = m / cin_g, cl = m - tap * cin_g;
-    float *dst = gw32 + row * M + (long)cl * taps + tap;
-    dst[0] += sum.x;
-    dst[taps] += sum.y;
-    dst[2 * taps] += sum.z;
-    dst[3 * taps] += sum.w;
-  }
 }
 
 }  // namespace mdcn

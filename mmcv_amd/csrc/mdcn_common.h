@@ -30,6 +30,21 @@ struct Geom {
   int Hp, Wp;     // H + 2, W + 2: the zero-bordered channels-last copy
 };
 
+// Channels of a tensor in a padded order: `nseg` segments of `seg` channels per group (nseg * seg = cg
+// channels), each padded to `segp`, the group to `cgp`.
+struct ChanMap {
+  int seg, segp, nseg, cg, cgp;
+};
+
+// Tensor channel of padded channel c; room: how many channels from there on are left in its segment (0 or
+// less: c is padding).
+__device__ __forceinline__ int chan_source(const ChanMap &m, int c, int &room) {
+  const int grp = c / m.cgp, r = c - grp * m.cgp;
+  const int s = r / m.segp, w = r - s * m.segp;
+  room = s < m.nseg ? m.seg - w : 0;
+  return grp * m.cg + s * m.seg + w;
+}
+
 __device__ __forceinline__ float to_f32(float v) { return v; }
 __device__ __forceinline__ float to_f32(f16_t v) { return (float)v; }
 __device__ __forceinline__ float to_f32(bf16_t v) { return (float)v; }

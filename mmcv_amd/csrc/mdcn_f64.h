@@ -41,7 +41,7 @@ __device__ __forceinline__ TapD make_tap_d(int base_y, int base_x, double dy, do
 }
 
 // One thread per output element.  mask == nullptr: no modulation (DCNv1).
-__global__ __launch_bounds__(256) void f64_forward_kernel(Geom g, const double *__restrict__ input,
+static __global__ __launch_bounds__(256) void f64_forward_kernel(Geom g, const double *__restrict__ input,
                                                           const double *__restrict__ offset,
                                                           const double *__restrict__ mask,
                                                           const double *__restrict__ weight,
@@ -84,7 +84,7 @@ __global__ __launch_bounds__(256) void f64_forward_kernel(Geom g, const double *
 // per (image, deformable group, tap, output pixel); the column gradient of each of
 // the group's channels, d = sum_co weight[co, c, tap] * grad_output[n, co, pixel],
 // is formed on the fly.
-__global__ __launch_bounds__(256) void f64_bwd_data_kernel(Geom g, const double *__restrict__ input,
+static __global__ __launch_bounds__(256) void f64_bwd_data_kernel(Geom g, const double *__restrict__ input,
                                                            const double *__restrict__ offset,
                                                            const double *__restrict__ mask,
                                                            const double *__restrict__ weight,
@@ -151,7 +151,7 @@ __device__ __forceinline__ double block_sum_d(double v, double *part) {
 // grad_weight: one workgroup per weight element (co, c, tap) sums
 // grad_output[n, co, pixel] * column[n, c, tap, pixel] over images and pixels; plain
 // store, so the result does not depend on the order workgroups run in.
-__global__ __launch_bounds__(256) void f64_bwd_weight_kernel(Geom g, const double *__restrict__ input,
+static __global__ __launch_bounds__(256) void f64_bwd_weight_kernel(Geom g, const double *__restrict__ input,
                                                              const double *__restrict__ offset,
                                                              const double *__restrict__ mask,
                                                              const double *__restrict__ gout,
@@ -189,7 +189,7 @@ __global__ __launch_bounds__(256) void f64_bwd_weight_kernel(Geom g, const doubl
 }
 
 // grad_bias[co] = sum over images and pixels of grad_output[:, co].
-__global__ __launch_bounds__(256) void f64_bwd_bias_kernel(Geom g, const double *__restrict__ gout,
+static __global__ __launch_bounds__(256) void f64_bwd_bias_kernel(Geom g, const double *__restrict__ gout,
                                                            double *__restrict__ gbias) {
   __shared__ double part[256];
   const long plane_out = (long)g.Ho * g.Wo;
@@ -204,7 +204,7 @@ __global__ __launch_bounds__(256) void f64_bwd_bias_kernel(Geom g, const double 
   }
 }
 
-__global__ __launch_bounds__(256) void f64_zero_kernel(double *p, long n) {
+static __global__ __launch_bounds__(256) void f64_zero_kernel(double *p, long n) {
   for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) p[i] = 0.0;
 }
 

@@ -34,24 +34,32 @@ namespace mdcn {
 // of channels, i.e. each 128-byte slab as four planes -- for a reader that takes 32 bytes of a pixel at a
 // time and whose neighbouring lanes read neighbouring pixels (the backward's scatter kernel): four pixels
 // share a cache line there, where the 128-byte records give every lane a line of its own.
-template <typename E, bool BORDER, int REC = 128>
+// MAPPED: the copy's channels are those of `cm`, cp of them (a multiple of RC elements for REC = 32, of KC for
+// REC = 128); padding channels are zero.
+template <typename E, bool BORDER, int REC = 128, bool MAPPED = false>
 __device__ __forceinline__ void relayout_vec_block(const Geom &g, const E *__restrict__ in, E *__restrict__ xt,
-                                                   int n_pchunks, int b) {
+                                                   int n_pchunks, int b, const ChanMap &cm = ChanMap(), int cp = 0) {
   static_assert(REC == 128 || REC == 32, "whole slabs or quarters of them");
   constexpr int EPV = 16 / (int)sizeof(E);
   constexpr int KC = 128 / (int)sizeof(E);
   constexpr int PXB = 32 * EPV;  // pixels per block
   const int pc = b % n_pchunks;
   b /= n_pchunks;
-  const int slabs_total = g.Cin / KC;
+  const int slabs_total = MAPPED ? (cp + KC - 1) / KC : g.Cin / KC;
   const int slab = b % slabs_total;
   const int n = b / slabs_total;
   const int tid = threadIdx.x;
   const int cg = tid & 7, pg = tid >> 3;
+  // planes of the copy this slab has (the last slab of a mapped copy may have fewer)
+  constexpr int NPL = 128 / REC;
+  const int planes = MAPPED && REC == 32 ? min(NPL, cp / (32 / (int)sizeof(E)) - slab * NPL) : NPL;
   const int plane = g.H * g.W;
   const int p0 = pc * PXB + pg * EPV;
   const long plane_px = BORDER ? (long)g.Hp * g.Wp : (long)plane;   // pixels of a plane of the copy
-  unsigned char *dst_slab = (unsigned char *)xt + (((long)n * slabs_total + slab) * plane_px) * 128;
+  unsigned char *dst_slab =
+      (unsigned char *)xt +
+      (MAPPED && REC == 32 ? ((long)n * (cp / (32 / (int)sizeof(E))) + slab * NPL) * plane_px * 32
+                           : (((long)n * slabs_total + slab) * plane_px) * 128);
   // where this thread's 16 bytes of pixel 0 go
   unsigned char *dst_cg = REC == 128 ? dst_slab + cg * 16 : dst_slab + (long)(cg >> 1) * plane_px * 32 + (cg & 1) * 16;
   const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
@@ -59,10 +67,13 @@ __device__ __forceinline__ void relayout_vec_block(const Geom &g, const E *__res
 #pragma unroll
   for (int i = 0; i < EPV; ++i) o[i] = zero;
   const int np = max(0, min(EPV, plane - p0));  // pixels of the run that exist
-  if (p0 < plane) {
-    const E *src = in + ((long)n * g.Cin + slab * KC + cg * EPV) * plane + p0;
+  int room = EPV;                               // channels of the thread's EPV that exist
+  int c_src = slab * KC + cg * EPV;
+  if constexpr (MAPPED) c_src = c_src < cp ? chan_source(cm, c_src, room) : (room = 0);
+  if (p0 < plane && room > 0) {
+    const E *src = in + ((long)n * g.Cin + c_src) * plane + p0;
     uint4 r[EPV];
-    if (np == EPV) {  // (16 bytes at the alignment of an element: one load instruction all the same)
+    if (np == EPV && room >= EPV) {  // (16 bytes at the alignment of an element: one load instruction all the same)
 #pragma unroll
       for (int j = 0; j < EPV; ++j) __builtin_memcpy(&r[j], src + (long)j * plane, 16);
     } else {
@@ -70,7 +81,7 @@ __device__ __forceinline__ void relayout_vec_block(const Geom &g, const E *__res
       for (int j = 0; j < EPV; ++j) {
         E e[EPV];
 #pragma unroll
-        for (int i = 0; i < EPV; ++i) e[i] = i < np ? src[(long)j * plane + i] : from_f32<E>(0.0f);
+        for (int i = 0; i < EPV; ++i) e[i] = i < np && j < room ? src[(long)j * plane + i] : from_f32<E>(0.0f);
         __builtin_memcpy(&r[j], e, 16);
       }
     }
@@ -148,7 +159,7 @@ __device__ __forceinline__ void relayout_vec_block(const Geom &g, const E *__res
       const int src_pg = (pg & ~6) | (((i >> 1) & 1) << 2) | ((i & 1) << 1);
       const int src_i = (i & ~3) | (b5 << 1) | b4;
       const int q = pc * PXB + src_pg * EPV + src_i;
-      if (q < plane) {
+      if (q < plane && (!MAPPED || (cg >> 1) < planes)) {
         const int y = q / g.W, x = q - y * g.W;
         unsigned char *d = dst_cg + (BORDER ? (long)(y + 1) * g.Wp + (x + 1) : (long)q) * REC;
         *(uint4 *)d = o[i];
@@ -160,16 +171,15 @@ __device__ __forceinline__ void relayout_vec_block(const Geom &g, const E *__res
     }
   }
   if (!BORDER) return;
-  constexpr int NPL = 128 / REC;       // planes of the copy per slab
   constexpr int QPP = REC / 16;        // 16-byte pieces per pixel of a plane
   if (pc == 0) {  // top border row and the left border pixel of the first image row
     const int per = (g.Wp + 1) * QPP;
-    for (int i = tid; i < per * NPL; i += 256)
+    for (int i = tid; i < per * planes; i += 256)
       *(uint4 *)(dst_slab + (long)(i / per) * plane_px * REC + (long)(i % per) * 16) = zero;
   }
   if (pc == n_pchunks - 1) {  // bottom border row
     const int per = g.Wp * QPP;
-    for (int i = tid; i < per * NPL; i += 256)
+    for (int i = tid; i < per * planes; i += 256)
       *(uint4 *)(dst_slab + (long)(i / per) * plane_px * REC + ((long)(g.Hp - 1) * g.Wp) * REC + (long)(i % per) * 16) = zero;
   }
 }

@@ -1,0 +1,56 @@
+"""The matrix-core backward where channels are padded: segments that are no whole pass of the scatter kernel,
+groups that are no multiple of 32 channels, output channels that are no multiple of 128 bytes, few tiles; all
+five gradients, and the weight or data gradients alone, against the CPU oracle."""
+import pytest
+import torch
+
+import oracle
+from mmcv_amd import capi
+from common import TOL, capi_backward, cast_case, make_case, rel_err
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    ('seg1_dg3', dict(N=1, Cin=3, Cout=2, H=9, W=7, deform_groups=3)),
+    ('seg4_dg8', dict(N=2, Cin=32, Cout=32, H=11, W=35, deform_groups=8)),
+    ('seg8_dg8', dict(N=1, Cin=64, Cout=64, H=17, W=33, deform_groups=8)),
+    ('seg20', dict(N=1, Cin=20, Cout=33, H=8, W=32)),
+    ('seg48_dg2', dict(N=2, Cin=96, Cout=72, H=13, W=19, deform_groups=2)),
+    ('gcd', dict(N=1, Cin=48, Cout=34, H=9, W=12, groups=2, deform_groups=3)),
+    ('groups_finer', dict(N=1, Cin=40, Cout=20, H=10, W=9, groups=2)),
+    ('s2', dict(N=2, Cin=24, Cout=40, H=19, W=23, stride=2)),
+    ('dil2_co200', dict(N=1, Cin=40, Cout=200, H=12, W=11, dilation=2, padding=2)),
+    ('one_pixel', dict(N=1, Cin=8, Cout=8, H=3, W=3, padding=0)),
+]
+NAMES = ('grad_input', 'grad_offset', 'grad_mask', 'grad_weight', 'grad_bias')
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16, torch.float16], ids=['f32', 'bf16', 'f16'])
+@pytest.mark.parametrize('name,kw', CASES, ids=[c[0] for c in CASES])
+def test_padded_backward(name, kw, dtype):
+    print(f'case={name} dtype={dtype}', flush=True)
+    case = cast_case(make_case(51, **kw), dtype)
+    Ho, Wo = case['offset'].shape[2:]
+    gy = torch.randn(kw['N'], kw['Cout'], Ho, Wo, generator=torch.Generator().manual_seed(3)).to(dtype)
+    geo = dict(stride=case['stride'], padding=case['padding'], dilation=case['dilation'],
+               groups=case['groups'], deform_groups=case['deform_groups'])
+    ref = oracle.backward(*[case[k].float().numpy() for k in ('input', 'offset', 'mask', 'weight')],
+                          gy.float().numpy(), True, **geo)
+    dev, gyd = cast_case(case, dtype, 'cuda'), gy.cuda()
+    for want in (dict(), dict(want_data=False, want_bias=False), dict(want_weight=False)):
+        got = capi_backward(dev, gyd, **want)
+        for nm, r, o in zip(NAMES, ref, got):
+            if o is None or (nm == 'grad_weight' and want.get('want_weight') is False) or (
+                    nm in NAMES[:3] and want.get('want_data') is False):
+                continue
+            err = rel_err(o.float().cpu().numpy(), r)
+            assert err <= TOL[dtype], (nm, want, err)
+    # images in passes of one: the weight gradient is summed over the passes
+    lib = capi.load()
+    lib.mdcn_set_pass_limits(0, 1)
+    try:
+        got = capi_backward(dev, gyd)
+    finally:
+        lib.mdcn_set_pass_limits(0, 0)
+    for nm, r, o in zip(NAMES, ref, got):
+        assert rel_err(o.float().cpu().numpy(), r) <= TOL[dtype], nm
