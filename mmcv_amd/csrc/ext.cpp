@@ -8,6 +8,8 @@
 // raises, the way the reference's device registry does for a device nobody
 // registered (mmcv/ops/csrc/common/pytorch_device_registry.hpp:120-126).
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/extension.h>
 
 #include <string>
@@ -533,6 +535,145 @@ void deform_conv_backward_parameters(Tensor input, Tensor offset, Tensor gradOut
   gradWeight.add_(gw, scale);
 }
 
+// ---- the layers' calls: one crossing from Python, autograd in C++ ----
+// What ModulatedDeformConv2dFunction / DeformConv2dFunction do
+// (mmcv/ops/modulated_deform_conv.py:104-214, mmcv/ops/deform_conv.py:60-200) for
+// device tensors outside of tracing and export: a call that needs no gradient is the
+// forward op and nothing else, one that does records a node whose backward is a
+// single call for the gradients that are asked for.  A small layer's time is the host's: the Python
+// Function cost 21 us a call (forward) and some 220 us (forward + backward) with its placeholders,
+// zero-filled gradients and keyword dictionaries.
+
+// offset's dtype decides the compute dtype (mmcv/ops/modulated_deform_conv.py:129-139)
+Tensor like(const Tensor &t, const Tensor &ref) {
+  return t.scalar_type() == ref.scalar_type() && t.device() == ref.device() ? t : t.to(ref.options());
+}
+
+struct LayerGeo {
+  int64_t kh, kw, sh, sw, ph, pw, dh, dw, groups, dgroups, step;
+  std::vector<int64_t> pack() const { return {sh, sw, ph, pw, dh, dw, groups, dgroups, step}; }
+  LayerGeo(const Tensor &weight, const std::vector<int64_t> &v)
+      : kh(weight.size(2)), kw(weight.size(3)), sh(v[0]), sw(v[1]), ph(v[2]), pw(v[3]), dh(v[4]), dw(v[5]),
+        groups(v[6]), dgroups(v[7]), step(v[8]) {}
+};
+
+// (N, Cout, Ho, Wo), not initialised; ValueError when a size is not positive
+// (mmcv/ops/modulated_deform_conv.py:216-230)
+Tensor new_output(const Tensor &input, const Tensor &weight, const LayerGeo &q) {
+  auto out = [](int64_t in, int64_t pad, int64_t dil, int64_t k, int64_t stride) {
+    const int64_t v = in + 2 * pad - (dil * (k - 1) + 1);
+    return (v >= 0 ? v / stride : -((-v + stride - 1) / stride)) + 1;  // rounds down, as Python's // does
+  };
+  TORCH_CHECK_VALUE(q.sh > 0 && q.sw > 0, "stride must be positive");
+  const int64_t n = input.size(0), co = weight.size(0);
+  const int64_t ho = out(input.size(2), q.ph, q.dh, q.kh, q.sh), wo = out(input.size(3), q.pw, q.dw, q.kw, q.sw);
+  TORCH_CHECK_VALUE(n > 0 && co > 0 && ho > 0 && wo > 0, "convolution input is too small (output would be ", n, "x", co,
+                    "x", ho, "x", wo, ")");
+  return at::empty({n, co, ho, wo}, input.options().memory_format(at::MemoryFormat::Contiguous));
+}
+
+// mask undefined: the unmodulated convolution.  bias may be undefined.
+Tensor layer_forward(const Tensor &input, const Tensor &offset, const Tensor &mask, const Tensor &weight,
+                     const Tensor &bias, const LayerGeo &q) {
+  Tensor output = new_output(input, weight, q);
+  if (mask.defined()) {
+    modulated_deform_conv_forward(input, weight, bias.defined() ? bias : weight, weight, offset, mask, output, weight,
+                                  q.kh, q.kw, q.sh, q.sw, q.ph, q.pw, q.dh, q.dw, q.groups, q.dgroups, bias.defined());
+  } else {
+    deform_conv_forward(input, weight, offset, output, weight, weight, q.kw, q.kh, q.sw, q.sh, q.pw, q.ph, q.dw, q.dh,
+                        q.groups, q.dgroups, q.step);
+  }
+  return output;
+}
+
+struct LayerFunction : public torch::autograd::Function<LayerFunction> {
+  static Tensor forward(torch::autograd::AutogradContext *ctx, const Tensor &input_, const Tensor &offset,
+                        const c10::optional<Tensor> &mask_, const Tensor &weight_, const c10::optional<Tensor> &bias_,
+                        std::vector<int64_t> geo) {
+    const Tensor input = like(input_, offset), weight = like(weight_, offset);
+    const Tensor mask = mask_.has_value() ? like(*mask_, offset) : Tensor();
+    const Tensor bias = bias_.has_value() ? like(*bias_, offset) : Tensor();
+    Tensor output = layer_forward(input, offset, mask, weight, bias, LayerGeo(weight, geo));
+    ctx->save_for_backward({input, offset, mask, weight});
+    geo.push_back(bias.defined() ? 1 : 0);
+    ctx->saved_data["geo"] = geo;
+    return output;
+  }
+
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx,
+                                                 torch::autograd::variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    const Tensor &input = saved[0], &offset = saved[1], &mask = saved[2], &weight = saved[3];
+    const std::vector<int64_t> geo = ctx->saved_data["geo"].toIntVector();
+    const LayerGeo q(weight, geo);
+    // (needs_input_grad counts the tensors that were given)
+    const size_t iw = mask.defined() ? 3 : 2;
+    const bool data = ctx->needs_input_grad(0) || ctx->needs_input_grad(1) || (mask.defined() && ctx->needs_input_grad(2));
+    const bool want_w = ctx->needs_input_grad(iw), want_b = geo.back() != 0 && ctx->needs_input_grad(iw + 1);
+    const bool twice = at::GradMode::is_enabled() && grads[0].requires_grad();
+    torch::autograd::variable_list out(6);
+    {
+      at::AutoGradMode no_grad(false);
+      const Tensor none = at::empty({0}, input.options());
+      auto fresh = [&](const Tensor &t) { return at::empty_like(t, t.options(), at::MemoryFormat::Contiguous); };
+      if (data) {
+        out[0] = fresh(input);
+        out[1] = fresh(offset);
+        if (mask.defined()) out[2] = fresh(mask);
+      }
+      if (want_w) out[3] = fresh(weight);
+      if (want_b) out[4] = at::empty({weight.size(0)}, weight.options());
+      auto or_none = [&](const Tensor &t) { return t.defined() ? t : none; };
+      if (data || want_w || want_b)
+        run_backward(mask.defined() ? "modulated_deform_conv_backward" : "deform_conv_backward", input, weight, offset,
+                     or_none(mask), grads[0], or_none(out[0]), or_none(out[1]), or_none(out[2]), or_none(out[3]),
+                     or_none(out[4]), q.kh, q.kw, q.sh, q.sw, q.ph, q.pw, q.dh, q.dw, q.groups, q.dgroups);
+    }
+    if (twice) {  // what torch.autograd.function.once_differentiable does
+      torch::autograd::variable_list defined;
+      for (auto &t : out)
+        if (t.defined()) defined.push_back(t.detach().set_requires_grad(true));
+      const int64_t n = (int64_t)defined.size();
+      auto err = std::make_shared<torch::autograd::DelayedError>(
+          "trying to differentiate twice a function that was marked with @once_differentiable", n);
+      defined = (*err)(std::move(defined));
+      size_t i = 0;
+      for (auto &t : out)
+        if (t.defined()) t = defined[i++];
+    }
+    return out;
+  }
+};
+
+Tensor layer_call(const Tensor &input, const Tensor &offset, const c10::optional<Tensor> &mask, const Tensor &weight,
+                  const c10::optional<Tensor> &bias, int64_t sh, int64_t sw, int64_t ph, int64_t pw, int64_t dh,
+                  int64_t dw, int64_t groups, int64_t dgroups, int64_t step) {
+  const Tensor m = mask.has_value() ? *mask : Tensor(), b = bias.has_value() ? *bias : Tensor();
+  const std::vector<int64_t> geo = {sh, sw, ph, pw, dh, dw, groups, dgroups, step};
+  const bool grad = at::GradMode::is_enabled() &&
+                    (input.requires_grad() || offset.requires_grad() || weight.requires_grad() ||
+                     (m.defined() && m.requires_grad()) || (b.defined() && b.requires_grad()));
+  if (grad) return LayerFunction::apply(input, offset, mask, weight, bias, geo);
+  const Tensor w = like(weight, offset);
+  return layer_forward(like(input, offset), offset, m.defined() ? like(m, offset) : m, w,
+                       b.defined() ? like(b, offset) : b, LayerGeo(w, geo));
+}
+
+// The Pack's forward without gradients: conv_offset, split, sigmoid and the convolution.
+Tensor pack_call(const Tensor &x_, const Tensor &offset_weight, const c10::optional<Tensor> &offset_bias,
+                 const Tensor &weight_, const c10::optional<Tensor> &bias_, int64_t sh, int64_t sw, int64_t ph, int64_t pw,
+                 int64_t dh, int64_t dw, int64_t groups, int64_t dgroups, bool unmodulated) {
+  const Tensor x = like(x_, offset_weight), weight = like(weight_, offset_weight);
+  const LayerGeo q(weight, {sh, sw, ph, pw, dh, dw, groups, dgroups, 1});
+  Tensor output = new_output(x, weight, q);
+  const Tensor none = at::empty({0}, x.options());
+  const bool with_bias = bias_.has_value();
+  modulated_deform_conv_pack_forward(x, offset_weight, offset_bias.has_value() ? *offset_bias : none, none, weight,
+                                     with_bias ? like(*bias_, offset_weight) : none, output, q.kh, q.kw, sh, sw, ph, pw,
+                                     dh, dw, groups, dgroups, with_bias, false, unmodulated);
+  return output;
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -584,6 +725,13 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("stride_h"), py::arg("stride_w"), py::arg("pad_h"), py::arg("pad_w"),
         py::arg("dilation_h"), py::arg("dilation_w"), py::arg("group"),
         py::arg("deformable_group"), py::arg("with_bias"));
+  // (positional: keyword matching costs a microsecond)
+  m.def("layer_call", &layer_call,
+        "layer_call(input, offset, mask | None, weight, bias | None, sh, sw, ph, pw, dh, dw, groups, deform_groups, "
+        "im2col_step): the layers' forward with autograd; without a mask the unmodulated convolution");
+  m.def("pack_call", &pack_call,
+        "pack_call(x, offset_weight, offset_bias | None, weight, bias | None, sh, sw, ph, pw, dh, dw, groups, "
+        "deform_groups, unmodulated): the Pack layers' forward, no autograd");
   m.def("set_path", [](int path) {
           TORCH_CHECK(path >= MDCN_PATH_AUTO && path <= MDCN_PATH_FUSED_NARROW,
                       "path must be 0 (auto), 1 (fused), 2 (direct), 3 (fused, specialised-wave kernel only), "

@@ -20,12 +20,13 @@ from torch.autograd.function import once_differentiable
 from torch.nn.modules.utils import _pair, _single
 
 from ..utils import ext_loader
-from .modulated_deform_conv import _conv_output_size, _renamed_kwargs
+from .modulated_deform_conv import (_conv_output_size, _in_one_call,
+                                    _renamed_kwargs)
 from .registry import MODELS
 
 ext_module = ext_loader.load_ext('_ext', [
     'deform_conv_forward', 'deform_conv_backward_input',
-    'deform_conv_backward_parameters'
+    'deform_conv_backward_parameters', 'layer_call', 'pack_call'
 ])
 
 
@@ -111,8 +112,8 @@ class DeformConv2dFunction(Function):
             'batch size must be divisible by im2col_step'
         grad_output = grad_output.contiguous()
         if ctx.needs_input_grad[0] or ctx.needs_input_grad[1]:
-            grad_input = torch.zeros_like(input, memory_format=torch.contiguous_format)
-            grad_offset = torch.zeros_like(offset, memory_format=torch.contiguous_format)
+            grad_input = torch.empty_like(input, memory_format=torch.contiguous_format)
+            grad_offset = torch.empty_like(offset, memory_format=torch.contiguous_format)
             ext_module.deform_conv_backward_input(
                 input, offset, grad_output, grad_input, grad_offset, weight,
                 ctx.bufs_[0], **_ext_kwargs(ctx, weight, step))
@@ -125,7 +126,18 @@ class DeformConv2dFunction(Function):
                 None, None, None)
 
 
-deform_conv2d = DeformConv2dFunction.apply
+def deform_conv2d(input, offset, weight, stride=1, padding=0, dilation=1, groups=1, deform_groups=1, bias=False,
+                  im2col_step=32):
+    if bias is False and _in_one_call(input) and input.size(0) > 0:
+        step = min(im2col_step, input.size(0))
+        assert input.size(0) % step == 0, 'batch size must be divisible by im2col_step'
+        sh, sw = _pair(stride)
+        ph, pw = _pair(padding)
+        dh, dw = _pair(dilation)
+        return ext_module.layer_call(input, offset, None, weight, None, sh, sw, ph, pw, dh, dw, groups,
+                                     deform_groups, step)
+    return DeformConv2dFunction.apply(input, offset, weight, stride, padding, dilation, groups, deform_groups, bias,
+                                      im2col_step)
 
 
 class DeformConv2d(nn.Module):
@@ -284,6 +296,10 @@ def deform_conv2d_pack(x, conv_offset, weight, stride, padding, dilation, groups
     output is read in place as the offsets.  No autograd."""
     stride, padding, dilation = _pair(stride), _pair(padding), _pair(dilation)
     cw, cb = conv_offset.weight, conv_offset.bias
+    if not return_raw and x.dim() == 4:
+        with torch.no_grad():
+            return ext_module.pack_call(x, cw, cb, weight, None, *stride, *padding, *dilation, groups, deform_groups,
+                                        True)
     x = x.type_as(cw)
     weight = weight.type_as(x)
     output = x.new_empty(_conv_output_size(x, weight, stride, padding, dilation))
