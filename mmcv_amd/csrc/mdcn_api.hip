@@ -17,6 +17,7 @@
 #include "mdcn_fused.h"
 #include "mdcn_fused2.h"
 #include "mdcn_fused3.h"
+#include "mdcn_fused_f32.h"
 #include "mdcn_oconv.h"
 #include "mdcn_host.h"
 #include "mdcn_prepass.h"
@@ -123,7 +124,8 @@ bool fused_ok(const mdcn_params *p, const Geom &g) {
   if (p->input_nhwc && (g.H < 2 || g.W < 2 || ((uintptr_t)p->input % 16) != 0)) return false;
   if (g.cin_g % KC || g.ch_per_dg % KC) return false;
   if (g.taps > kTapsLarge) return false;
-  if (fused_lds_bytes(pick_ct(g.cout_g, g.taps), table_capacity(g.taps)) > kMaxLds) return false;
+  const int ct = pick_ct(g.cout_g, g.taps), tmax = table_capacity(g.taps);
+  if ((p->dtype == MDCN_F32 ? fused_f32_lds_bytes(tmax) : fused_lds_bytes(ct, tmax)) > kMaxLds) return false;
   // one padded image must fit the 32-bit offsets
   const uint64_t img = (uint64_t)g.Hp * g.Wp * g.Cin * elem_size(p->dtype);
   if (img > kMaxXtBytes) return false;
@@ -279,20 +281,21 @@ int make_plan(const mdcn_params *p, const Geom &g, Plan *pl) {
   const uint64_t img = (uint64_t)g.Hp * g.Wp * g.Cin * es;
   pl->n_chunk = (int)std::min<uint64_t>((uint64_t)g.N, std::max<uint64_t>(1, g_fwd_pass_bytes.load() / img));
   if (p->dtype == MDCN_F32 && pl->CT == 256) {
-    // fp32 tiles are bound by the matrix pipe (a K step of a 128 x 256 tile is some 7 000 clocks of
-    // 32x32x2 MFMAs against 3 000 of sampling), so a tile's time goes with its width and what counts is
-    // how evenly the tiles fill the workgroups: take the 128-wide tile when its schedule is shorter
+    // an fp32 tile's time goes with its width: a 128-channel tile takes 0.56 of a 256-channel one (N=8, 256
+    // channels, 64x64: 240 us as 512 tiles of 128 channels, 213 us as 256 of 256), so what counts is how
+    // evenly the tiles fill the workgroups
     const long px_tiles = ((long)pl->n_chunk * g.Ho * g.Wo + kPT - 1) / kPT;
     const int nk = pl->slabs * g.taps;
     auto cost = [&](int ct) {
       const long tiles = px_tiles * ((g.cout_g + ct - 1) / ct) * g.G;
-      return schedule_rounds(tiles, nk, !p->no_k_split) * std::max(7000.0 * ct / 256, 3000.0);
+      return schedule_rounds(tiles, nk, !p->no_k_split) * (ct == 256 ? 1.0 : 0.56);
     };
     if (cost(128) < 0.95 * cost(256)) pl->CT = 128;
   }
   pl->n_ctiles = (g.cout_g + pl->CT - 1) / pl->CT;
   pl->xt_bytes = p->input_nhwc ? 0 : align_up((size_t)img * pl->n_chunk);
-  pl->wp_bytes = align_up((size_t)g.G * pl->n_ctiles * pl->slabs * g.taps * pl->CT * pl->KC * es);
+  // (fp32: three bf16 planes, 6 bytes an element)
+  pl->wp_bytes = align_up((size_t)g.G * pl->n_ctiles * pl->slabs * g.taps * pl->CT * pl->KC * (es == 4 ? 6 : es));
   // Tiles of the 128-pixel kernels' last round are cut along K where workgroups would otherwise idle: one
   // 128 x 256 fp32 tile and a counter per workgroup of the persistent grid -- asked for only when a launch
   // of this call has such a round (the 256-pixel kernel never cuts; what it leaves to the 128-pixel one may)
@@ -403,12 +406,18 @@ hipError_t launch_fused_ct(const FusedArgs &fa, bool unbordered, hipStream_t st)
   const int total_wg = fa.n_ptiles * fa.n_ctiles * fa.g.G;
   const int per_xcd = fa.cut_max > 1 ? std::max(1, num_cus() / 8)
                                        : std::max(1, std::min((total_wg + 7) / 8, num_cus() / 8));
-  if (unbordered)
-    hipLaunchKernelGGL((fused_kernel<E, CT, TMAX, MULTI_DG, true>), dim3(per_xcd * 8), dim3(kThreads),
-                       0, st, fa);
-  else
-    hipLaunchKernelGGL((fused_kernel<E, CT, TMAX, MULTI_DG, false>), dim3(per_xcd * 8), dim3(kThreads),
-                       0, st, fa);
+  const dim3 grid(per_xcd * 8), block(kThreads);
+  if constexpr (sizeof(E) == 4) {
+    if (unbordered)
+      hipLaunchKernelGGL((fused_f32_kernel<CT, TMAX, MULTI_DG, true>), grid, block, 0, st, fa);
+    else
+      hipLaunchKernelGGL((fused_f32_kernel<CT, TMAX, MULTI_DG, false>), grid, block, 0, st, fa);
+  } else {
+    if (unbordered)
+      hipLaunchKernelGGL((fused_kernel<E, CT, TMAX, MULTI_DG, true>), grid, block, 0, st, fa);
+    else
+      hipLaunchKernelGGL((fused_kernel<E, CT, TMAX, MULTI_DG, false>), grid, block, 0, st, fa);
+  }
   return hipGetLastError();
 }
 

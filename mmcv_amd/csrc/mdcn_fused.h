@@ -256,13 +256,15 @@ struct ElemTraits<float> {
     const float ww[4] = {__uint_as_float(w.x), __uint_as_float(w.y), __uint_as_float(w.z),
                          __uint_as_float(w.w)};
     const uint4 v[4] = {v0, v1, v2, v3};
+    // (the fused operations are written out: left to the compiler, copies of this code contract differently and a
+    // pixel's result depends on which of a lane's pixels it is)
     float acc[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const float d[4] = {__uint_as_float(v[q].x), __uint_as_float(v[q].y),
                           __uint_as_float(v[q].z), __uint_as_float(v[q].w)};
 #pragma unroll
-      for (int j = 0; j < 4; ++j) acc[j] = (q == 0) ? ww[q] * d[j] : acc[j] + ww[q] * d[j];
+      for (int j = 0; j < 4; ++j) acc[j] = (q == 0) ? ww[q] * d[j] : fmaf(ww[q], d[j], acc[j]);
     }
     return make_uint4(__float_as_uint(acc[0]), __float_as_uint(acc[1]), __float_as_uint(acc[2]),
                       __float_as_uint(acc[3]));

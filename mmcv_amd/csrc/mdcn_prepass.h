@@ -2,6 +2,7 @@
 #pragma once
 
 #include "mdcn_common.h"
+#include "mdcn_fused_f32.h"
 
 namespace mdcn {
 
@@ -199,6 +200,10 @@ template <typename E>
 __device__ __forceinline__ void pack_weight_elems(const Geom &g, const E *__restrict__ w, E *__restrict__ wp, int CT,
                                                   int KC, int n_ctiles, int slabs, long total, long first,
                                                   long stride, uint32_t *__restrict__ zero_ptr, int zero_n) {
+  if constexpr (sizeof(E) == 4) {  // the fp32 kernel's split planes
+    pack_weight_split(g, w, wp, CT, n_ctiles, slabs, first, stride, zero_ptr, zero_n);
+    return;
+  }
   for (long i = first; i < zero_n; i += stride) zero_ptr[i] = 0u;
   // one 16-byte run of a row (EPV consecutive input channels of one output channel and tap) per step: the
   // index arithmetic is paid once per run and the store is whole
