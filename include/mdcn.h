@@ -59,7 +59,9 @@ enum mdcn_path {
                                kernel all tiles or whole rounds of tiles, whichever its measured tile cost
                                says is shorter, and the rest of the pixels to the 128-pixel kernel.  Error if
                                the shape has no such kernel. */
-  MDCN_PATH_FUSED_NARROW = 5 /* forward only: as MDCN_PATH_FUSED, never the 256-pixel kernel */
+  MDCN_PATH_FUSED_NARROW = 5, /* forward only: as MDCN_PATH_FUSED, never the 256-pixel kernel */
+  MDCN_PATH_SEGMENT = 6 /* forward only: the segment kernel wherever it covers the shape (given the scratch of
+                           mdcn_workspace_wanted()), else direct; for comparisons and tests */
 };
 
 enum mdcn_status {

@@ -261,8 +261,8 @@ void drop_segments(Plan *pl) {
 int make_plan(const mdcn_params *p, const Geom &g, Plan *pl) {
   const bool ok = fused_ok(p, g);
   if (forced_fused(p->path) && !ok) return MDCN_ERR_PATH;
-  if (p->input_nhwc && (!ok || p->path == MDCN_PATH_DIRECT)) return MDCN_ERR_PATH;  // in-place reads: fused kernel only
-  pl->fused = ok && p->path != MDCN_PATH_DIRECT;
+  if (p->input_nhwc && (!ok || p->path == MDCN_PATH_DIRECT || p->path == MDCN_PATH_SEGMENT)) return MDCN_ERR_PATH;  // in-place reads: fused kernel only
+  pl->fused = ok && p->path != MDCN_PATH_DIRECT && p->path != MDCN_PATH_SEGMENT;
   pl->seg = false;
   pl->CT = pl->KC = pl->n_ctiles = pl->slabs = pl->n_chunk = 0;
   pl->xt_bytes = pl->wp_bytes = pl->owp_bytes = pl->raw_bytes = pl->cut_bytes = 0;

@@ -14,13 +14,13 @@ namespace mdcn {
 
 namespace {
 
-// Largest margin R (up to 8) for which the LDS window of a th x tw output-pixel
+// Largest margin R (up to `most`) for which the LDS window of a th x tw output-pixel
 // tile fits max_px pixels; -1 if even R = 0 does not.
-int window_margin(const Geom &g, int th, int tw, long max_px, int *WH, int *WW) {
+int window_margin(const Geom &g, int th, int tw, long max_px, int *WH, int *WW, int most = 8) {
   const long base_h = (long)(th - 1) * g.sh + (long)(g.kh - 1) * g.dh + 2;
   const long base_w = (long)(tw - 1) * g.sw + (long)(g.kw - 1) * g.dw + 2;
   int R = -1;
-  while (R < 8 && (base_h + 2 * (R + 1)) * (base_w + 2 * (R + 1)) <= max_px) ++R;
+  while (R < most && (base_h + 2 * (R + 1)) * (base_w + 2 * (R + 1)) <= max_px) ++R;
   *WH = (int)base_h + 2 * std::max(R, 0);
   *WW = (int)base_w + 2 * std::max(R, 0);
   return R;
@@ -50,6 +50,7 @@ void make_bwd_plan(const mdcn_bwd_params *bp, const Geom &g, uint64_t pass_bytes
   pl->P_pad = 0;
   pl->R = pl->sR = -1;
   pl->WH = pl->WW = pl->sWH = pl->sWW = 0;
+  pl->fR = pl->fWH = pl->fWW = 0;
   const int path = forced_fused(bp->conv.path) ? MDCN_PATH_FUSED : bp->conv.path;
   if (path == MDCN_PATH_DIRECT || g.taps > kBwdTapsMax || f64) return;
   const bool forced = path == MDCN_PATH_FUSED;
@@ -83,6 +84,8 @@ void make_bwd_plan(const mdcn_bwd_params *bp, const Geom &g, uint64_t pass_bytes
       pl->sWW = ww;
     }
   }
+  pl->fR = window_margin(g, kScTH, kScTW, (long)kScWindowPx * (2 * ch_big / pl->sCH), &pl->fWH, &pl->fWW, kScFarMargin);
+  if (pl->fR <= pl->sR) pl->fWH = 0;
   ChanMap &im = pl->im, &om = pl->om;
   im.seg = seg;
   im.segp = padded(seg, pl->sCH);
@@ -121,7 +124,7 @@ void make_bwd_plan(const mdcn_bwd_params *bp, const Geom &g, uint64_t pass_bytes
     pl->gt_bytes = align_up((size_t)g.N * g.G * om.cgp * plane_out * es);
     pl->wt_bytes = align_up((size_t)g.G * pl->M_pad * om.cgp * es);
     pl->d_bytes = align_up(d_img * pl->n_chunk);
-    pl->mx_bytes = 2 * kAlign;
+    pl->mx_bytes = 3 * kAlign;
     if (pl->parts > 1) pl->part_bytes = align_up((size_t)pl->parts * g.N * g.DG * 3 * g.taps * plane_out * 4);
   }
   if (pl->wgemm) {
@@ -277,6 +280,7 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
   float *bpart = (float *)take(pl.gb_bytes);
   uint32_t *dmax = (uint32_t *)take(pl.mx_bytes);
   float *mmax = (float *)dmax + kAlign / 4;
+  uint32_t *far = dmax + 2 * kAlign / 4;
   unsigned char *xt = take(pl.xt_bytes), *gT = take(pl.gt_bytes), *wT = take(pl.wt_bytes);
   unsigned char *D = take(pl.d_bytes), *col = take(pl.col_bytes);
   const long off_total = (long)g.N * g.DG * 2 * g.taps * plane_out, mask_total = off_total / 2;
@@ -287,6 +291,15 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
   const long n_in = (long)g.N * g.Cin * g.H * g.W;
   const int mask_blocks = (int)std::max<long>(1, std::min<long>(mask_total / (256 * EPV), 64));
 
+  // a sample of the offsets, 64 Ki of them at most, decides which window the scatter kernel uses
+  const long off_step = std::max<long>(1, (off_total >> 16) | 1);
+  const int far_blocks = (int)std::max<long>(1, std::min<long>(off_total / off_step / 1024, 64));
+
+  // Share of offset components beyond the margin from which the far window is the better one.  Half of 16 (fp32: 8)
+  // channels a pass cost next to nothing (bf16, N=2 C=256 135x224, margins 5 and 11: sigma 1.0 0.77 ms with either,
+  // 2.5 0.87 / 0.86, 4.0 1.63 / 0.94), half of 8 do: fp16, N=7 C=128 118x196 stride 2, margins 3 and 12: sigma
+  // 2.0 0.56 / 0.59, 2.5 0.60 / 0.60, 4.0 0.94 / 0.65.
+  const uint32_t far_min = (uint32_t)(off_total / off_step / (pl.sCH * (int)sizeof(E) == 32 ? 32 : 5));
   auto up = [](long n, long per) { return (int)((n + per - 1) / per); };
   {
     BwdPreArgs a;
@@ -314,6 +327,11 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
     a.dmax = dmax;
     a.mmax = mmax;
     a.n_mask = mask_total;
+    a.off = p->offset;
+    a.n_off = off_total;
+    a.off_step = off_step;
+    a.far_from = (float)pl.sR;
+    a.far = far;
     a.bpart = bpart;
     a.bsplits = pl.bsplits;
     const int jobs[kPreJobs] = {
@@ -324,6 +342,7 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
         wgemm && pl.P_pad > plane_out ? up(a.col_rows * (pl.P_pad - plane_out), kPrePadPerBlock) : 0,
         gemm ? up((long)g.G * pl.M_pad * pl.om.cgp, 256) : 0,
         gemm && staged ? mask_blocks : 0,
+        gemm && pl.fWH ? far_blocks : 0,
         bp->grad_bias ? g.Cout * pl.bsplits : 0,
     };
     int total = 0;
@@ -373,14 +392,15 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
     sa.P_pad = pl.P_pad;
     sa.tiles_x = (g.Wo + kScTW - 1) / kScTW;
     sa.tiles_y = (g.Ho + kScTH - 1) / kScTH;
-    sa.R = pl.sR;
-    sa.WH = pl.sWH;
-    sa.WW = pl.sWW;
+    sa.win = ScatterWindow{pl.sR, pl.sWH, pl.sWW};
+    sa.win_far = ScatterWindow{pl.fR, pl.fWH, pl.fWW};
+    sa.far = far;
+    sa.n_far = far_blocks;
+    sa.far_min = far_min;
     sa.n0 = n0;
     sa.parts = pl.parts;
     sa.im = pl.im;
     sa.cin_p = cin_p;
-    sa.passes = g.ch_per_dg / pl.im.seg * (pl.im.segp / pl.sCH);
     sa.poff = poff;
     sa.pmask = pmask;
     sa.off_total = off_total;

@@ -11,8 +11,8 @@
 
 namespace mdcn {
 
-constexpr int kPreJobs = 8;
-enum { kPreX, kPreG, kPreRows, kPreZero, kPreColPad, kPreWeight, kPreMask, kPreBias };
+constexpr int kPreJobs = 9;
+enum { kPreX, kPreG, kPreRows, kPreZero, kPreColPad, kPreWeight, kPreMask, kPreFar, kPreBias };
 
 struct BwdPreArgs {
   Geom g;
@@ -30,6 +30,10 @@ struct BwdPreArgs {
   uint32_t *dmax;          // cleared
   float *mmax;             // one value per block of the mask job
   long n_mask;
+  const void *off;
+  long n_off, off_step;    // one offset in off_step is looked at
+  float far_from;          // ... and counted when it is larger than this
+  uint32_t *far;           // one count per block of the job
   float *bpart;            // [Cout][bsplits]
   int bsplits;
 };
@@ -141,8 +145,20 @@ __global__ __launch_bounds__(256) void bwd_prepass_kernel(BwdPreArgs a) {
     if (tid == 0) a.mmax[bi] = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
     return;
   }
+  if (b < a.end[kPreFar]) {  // offsets that leave the scatter kernel's window, counted in a sample
+    const int nb = a.end[kPreFar] - a.end[kPreMask], bi = b - a.end[kPreMask];
+    float cnt = 0.0f;  // (64 Ki samples at most: exact)
+    for (long i = ((long)bi * 256 + tid) * a.off_step; i < a.n_off; i += (long)nb * 256 * a.off_step)
+      cnt += fabsf(to_f32(((const E *)a.off)[i])) > a.far_from ? 1.0f : 0.0f;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) cnt += __shfl_xor(cnt, o);
+    if ((tid & 63) == 0) red[tid >> 6] = cnt;
+    __syncthreads();
+    if (tid == 0) a.far[bi] = (uint32_t)((red[0] + red[1]) + (red[2] + red[3]));
+    return;
+  }
   {  // sums of grad_output over the pixels, a share of an output channel's runs per block
-    const int bi = b - a.end[kPreMask];
+    const int bi = b - a.end[kPreFar];
     const int co = bi / a.bsplits, split = bi - co * a.bsplits;
     const int runs = (int)((plane + kBiasRun - 1) / kBiasRun);
     float s = 0.0f;

@@ -212,6 +212,8 @@ __global__ __launch_bounds__(TILE * 2, TILE == 128 ? 2 : 1) void bwd_colgrad_ker
 // workgroups per CU was slower: the passes over the window double.)
 constexpr int kScWindowBytes = 60 * 1024;
 constexpr int kScWindowPx = kScWindowBytes / 64;
+// Largest margin of the window for far offsets.
+constexpr int kScFarMargin = 12;
 // Contributions one window entry can receive at most: every (pixel, tap) of the
 // tile touches an entry at most once per channel.
 constexpr int kScMaxAdds = 256 * 9;
@@ -273,6 +275,11 @@ struct VecCh {
 constexpr int kScTH = 8;
 constexpr int kScTW = 32;
 
+// A workgroup's window of grad_input in LDS: WH x WW input pixels, R of margin around the tile's undeformed footprint.
+struct ScatterWindow {
+  int R, WH, WW;
+};
+
 struct BwdScatterArgs {
   Geom g;
   const void *xt;  // zero-bordered input copy in 32-byte records [N][Cin / RC][H + 2][W + 2][RC], RC = 32 bytes of channels
@@ -284,11 +291,13 @@ struct BwdScatterArgs {
   void *col;       // columns of the pass [image][group][tap][padded channel of the group][P_pad], or null
   ChanMap im;      // padded order of the input channels
   int cin_p;       // ... how many there are
-  int passes;      // passes of CH channels over a deformable group's segments
   long P_pad;      // row pitch of col in elements
   int tiles_x, tiles_y;
-  int WH, WW;      // window size in input pixels
-  int R;           // margin of the window around the tile's undeformed footprint
+  ScatterWindow win;      // with CH channels a pass
+  ScatterWindow win_far;  // with CH / 2: twice the pixels, for offsets that leave the other one (WH = 0: none)
+  const uint32_t *far;    // n_far counts of sampled offsets beyond win's margin; above far_min in all, win_far is used
+  int n_far;
+  uint32_t far_min;
   int n0;          // first image of the pass
   // A deformable group's channels are shared among `parts` workgroups per tile
   // (blockIdx.y), so that the launch has several times more workgroups than the
@@ -324,7 +333,7 @@ struct BwdScatterArgs {
 // reference's columns tensor is) to a.col for the weight-gradient product.  At
 // least one of the two.
 template <typename E, int CH, typename WT, bool DATA, bool COL>
-__global__ __launch_bounds__(256, 2) void bwd_scatter_kernel(BwdScatterArgs a) {
+__device__ __forceinline__ void scatter_tile(const BwdScatterArgs &a, const ScatterWindow &wd, WT *win) {
   constexpr int RC = 32 / (int)sizeof(E);   // channels per record of the input copy
   static_assert(DATA || COL, "nothing to do");
   static_assert(CH <= RC && RC % CH == 0, "a pass reads a record or a whole fraction of one");
@@ -332,7 +341,6 @@ __global__ __launch_bounds__(256, 2) void bwd_scatter_kernel(BwdScatterArgs a) {
   constexpr bool kFixed = sizeof(WT) == 4;
   static_assert(kScTH * kScTW == 256, "one thread per pixel of the tile");
   static_assert(kScTH * kScTW * kBwdTapsMax <= kScMaxAdds, "bound on the adds per window entry");
-  __shared__ __align__(16) WT win[DATA ? kScWindowBytes / sizeof(WT) : 4];
   float fx_scale = 1.0f, fx_inv = 1.0f;
   if (kFixed && DATA) {
     float mm = 1.0f;
@@ -363,8 +371,8 @@ __global__ __launch_bounds__(256, 2) void bwd_scatter_kernel(BwdScatterArgs a) {
   const int ho = ty * kScTH + tid / kScTW, wo = tx * kScTW + tid % kScTW;
   const bool valid = ho < g.Ho && wo < g.Wo;
   const long pix = valid ? (long)ho * g.Wo + wo : 0;
-  const int wy0 = ty * kScTH * g.sh - g.ph - a.R, wx0 = tx * kScTW * g.sw - g.pw - a.R;
-  const int win_px = a.WH * a.WW;
+  const int wy0 = ty * kScTH * g.sh - g.ph - wd.R, wx0 = tx * kScTW * g.sw - g.pw - wd.R;
+  const int win_px = wd.WH * wd.WW;
 
   const E *off = (const E *)a.om.off + (long)n * a.om.off_n + pix * a.om.off_px +
                  (long)(dgi * 2 * g.taps) * a.om.off_ch;
@@ -388,7 +396,8 @@ __global__ __launch_bounds__(256, 2) void bwd_scatter_kernel(BwdScatterArgs a) {
   // This workgroup's passes of CH channels.  Pass i of the deformable group: segment i / (segp / CH) of the
   // group, from padded channel c0 on; the tensor's channel cs, of which `room` are left in the segment.
   const int part = blockIdx.y;
-  const int ps_begin = (int)((long)a.passes * part / a.parts), ps_end = (int)((long)a.passes * (part + 1) / a.parts);
+  const int passes = g.ch_per_dg / a.im.seg * (a.im.segp / CH);
+  const int ps_begin = (int)((long)passes * part / a.parts), ps_end = (int)((long)passes * (part + 1) / a.parts);
   struct Pass {
     int c0, cs, room, grp;
   };
@@ -413,7 +422,7 @@ __global__ __launch_bounds__(256, 2) void bwd_scatter_kernel(BwdScatterArgs a) {
 #pragma unroll
     for (int j = 0; j < kSlots; ++j) {
       const int q = tid + 256 * j;
-      const int y = wy0 + q / a.WW, x = wx0 + q % a.WW;
+      const int y = wy0 + q / wd.WW, x = wx0 + q % wd.WW;
       flush_at[j] = (q < win_px && y >= 0 && y < g.H && x >= 0 && x < g.W) ? y * g.W + x : -1;
     }
     // (the flush leaves the window zeroed for the next pass)
@@ -497,11 +506,11 @@ __global__ __launch_bounds__(256, 2) void bwd_scatter_kernel(BwdScatterArgs a) {
           for (int i = 0; i < VecCh<E, CH>::NW; ++i) rd.raw[i] &= keep;
         }
         const int ry = y0 - wy0, rx = x0 - wx0;
-        const bool in_win = ry >= 0 && ry + 1 < a.WH && rx >= 0 && rx + 1 < a.WW;
+        const bool in_win = ry >= 0 && ry + 1 < wd.WH && rx >= 0 && rx + 1 < wd.WW;
         const bool to_win = inside && in_win;
         // window is [channel][WH][WW]: neighbouring pixels, neighbouring banks; a lane with nothing
         // for the window adds its zeros at an entry of its own
-        const int wbase = to_win ? ry * a.WW + rx : (tid & 63);
+        const int wbase = to_win ? ry * wd.WW + rx : (tid & 63);
         const float s00 = (to_win && ok00) ? w00 : 0.0f, s01 = (to_win && ok01) ? w01 : 0.0f;
         const float s10 = (to_win && ok10) ? w10 : 0.0f, s11 = (to_win && ok11) ? w11 : 0.0f;
         const float mts = m * fx_scale;
@@ -544,8 +553,8 @@ __global__ __launch_bounds__(256, 2) void bwd_scatter_kernel(BwdScatterArgs a) {
               unsigned long long *wp = (unsigned long long *)win + cp * win_px + wbase;
               atomicAdd(wp, entry(s00, tl, th));
               atomicAdd(wp + 1, entry(s01, tl, th));
-              atomicAdd(wp + a.WW, entry(s10, tl, th));
-              atomicAdd(wp + a.WW + 1, entry(s11, tl, th));
+              atomicAdd(wp + wd.WW, entry(s10, tl, th));
+              atomicAdd(wp + wd.WW + 1, entry(s11, tl, th));
             } else {
 #pragma unroll
               for (int h = 0; h < 2; ++h) {
@@ -553,8 +562,8 @@ __global__ __launch_bounds__(256, 2) void bwd_scatter_kernel(BwdScatterArgs a) {
                 WT *wp = win + (2 * cp + h) * win_px + wbase;
                 atomicAdd(wp, (WT)(s00 * t));
                 atomicAdd(wp + 1, (WT)(s01 * t));
-                atomicAdd(wp + a.WW, (WT)(s10 * t));
-                atomicAdd(wp + a.WW + 1, (WT)(s11 * t));
+                atomicAdd(wp + wd.WW, (WT)(s10 * t));
+                atomicAdd(wp + wd.WW + 1, (WT)(s11 * t));
               }
             }
           }
@@ -654,6 +663,26 @@ __global__ __launch_bounds__(256, 2) void bwd_scatter_kernel(BwdScatterArgs a) {
       }
     }
   }
+}
+
+// Few offsets beyond the margin of the wide pass's window: CH channels a pass.  Many: half as many channels over a
+// window twice as large, since a corner outside the window costs CH global atomics.  (Which of the two is
+// decided on the device, from a sample of the offsets that the pre-pass has looked at.)
+template <typename E, int CH, typename WT, bool DATA, bool COL>
+__global__ __launch_bounds__(256, 2) void bwd_scatter_kernel(BwdScatterArgs a) {
+  __shared__ __align__(16) WT win[DATA ? kScWindowBytes / sizeof(WT) : 4];
+  if constexpr (DATA && CH * (int)sizeof(E) >= 16) {
+    if (a.win_far.WH > 0) {
+      uint32_t n = (int)(threadIdx.x & 63) < a.n_far ? a.far[threadIdx.x & 63] : 0u;
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o);
+      if (__builtin_amdgcn_readfirstlane((int)n) > (int)a.far_min) {
+        scatter_tile<E, CH / 2, WT, DATA, COL>(a, a.win_far, win);
+        return;
+      }
+    }
+  }
+  scatter_tile<E, CH, WT, DATA, COL>(a, a.win, win);
 }
 
 struct WGradArgs {

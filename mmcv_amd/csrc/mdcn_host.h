@@ -33,6 +33,7 @@ struct BwdPlan {
   bool wgemm;      // grad_weight from stored columns
   int sR, sWH, sWW;  // window of the scatter kernel
   int sCH;         // channels per pass over that window
+  int fR, fWH, fWW;  // window with half as many channels a pass, for far offsets (fWH = 0: none)
   int n_chunk;     // images per pass
   int cg_tile;     // tile of the column-gradient product (kCgTile or kCgTileBig)
   // Padded channel orders of its copies: segments of the input's channels to whole passes of sCH, a group's to

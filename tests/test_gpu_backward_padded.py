@@ -20,6 +20,9 @@ CASES = [
     ('groups_finer', dict(N=1, Cin=40, Cout=20, H=10, W=9, groups=2)),
     ('s2', dict(N=2, Cin=24, Cout=40, H=19, W=23, stride=2)),
     ('dil2_co200', dict(N=1, Cin=40, Cout=200, H=12, W=11, dilation=2, padding=2)),
+    # offsets beyond the scatter kernel's window: the window for far offsets, and past that one too
+    ('far', dict(N=1, Cin=64, Cout=32, H=21, W=39, sigma=6.0)),
+    ('far_s2', dict(N=1, Cin=64, Cout=32, H=37, W=69, stride=2, sigma=7.0)),
     ('one_pixel', dict(N=1, Cin=8, Cout=8, H=3, W=3, padding=0)),
 ]
 NAMES = ('grad_input', 'grad_offset', 'grad_mask', 'grad_weight', 'grad_bias')

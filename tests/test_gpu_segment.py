@@ -86,3 +86,18 @@ def test_segment_kernel(name, dtype):
         assert rel_err(yp.float().cpu().numpy(), ref) <= TOL[dtype]
         # a workspace one byte short: the kernel that needs none
         assert torch.equal(segment_forward(dev, short=True), capi_forward(dev, path=capi.PATH_DIRECT))
+
+
+def test_segment_path_on_a_shape_of_the_fused_kernels():
+    dev = cast_case(make_case(32, N=1, Cin=64, Cout=96, H=14, W=15), torch.bfloat16, 'cuda')
+    lib = capi.load()
+    p = capi.make_params(capi.MDCN_BF16, 1, 64, 14, 15, 96, 3, 3, (1, 1), (1, 1), (1, 1), 1, 1, capi.PATH_SEGMENT)
+    assert lib.mdcn_forward_kernels(ctypes.byref(p)) == b'segment_kernel'
+    ref = capi_forward(dev, path=capi.PATH_FUSED).float()
+    out = torch.empty(1, 96, 14, 15, dtype=torch.bfloat16, device='cuda')
+    ws = torch.empty(lib.mdcn_workspace_wanted(ctypes.byref(p)), dtype=torch.uint8, device='cuda')
+    p.input, p.offset, p.mask, p.weight, p.bias = (dev[k].data_ptr() for k in ('input', 'offset', 'mask', 'weight', 'bias'))
+    p.output, p.workspace, p.workspace_bytes = out.data_ptr(), ws.data_ptr(), ws.numel()
+    assert lib.mdcn_forward(ctypes.byref(p), None) == 0
+    torch.cuda.synchronize()
+    assert float((out.float() - ref).abs().max() / ref.abs().max()) <= TOL[torch.bfloat16]
