@@ -15,7 +15,7 @@ PROBE_LIB = os.path.join(HERE, 'libmfma_probe.so')
 
 def build():
     from mmcv_amd.build import HIPCC_FLAGS, ROCM
-    cmd = [os.path.join(ROCM, 'bin', 'hipcc'), *HIPCC_FLAGS, '-I', os.path.join(ROOT, 'include'),
+    cmd = [os.path.join(ROCM, 'bin', 'hipcc'), *HIPCC_FLAGS, '-shared', '-I', os.path.join(ROOT, 'include'),
            '-o', PROBE_LIB, os.path.join(HERE, 'mfma_probe.hip')]
     print(' '.join(cmd), flush=True)
     subprocess.check_call(cmd)
