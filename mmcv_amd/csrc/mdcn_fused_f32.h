@@ -45,6 +45,26 @@ constexpr size_t fused_f32_lds_bytes(int tmax) {
   return (size_t)kF32Tiles * kPT * 192 + (size_t)kPT * tmax * 20 + 16;
 }
 
+// Half `half` of the words h, m, l for an x whose first plane cannot be a rounded one.  Infinity and NaN go to
+// the last plane alone: of the products that are summed it meets the other operand's first plane only, which has that
+// operand's sign and is zero when it is, so that the result is what an fp32 product gives.  (In the first plane it would
+// meet the lower planes too, zeros and numbers of the other sign among them.)  Finite: a first plane that is cut off.
+__device__ __forceinline__ void split3_not_rounded(float x, int half, uint32_t &h, uint32_t &m, uint32_t &l) {
+  const uint32_t b = __float_as_uint(x);
+  uint32_t hb = 0u, mb = 0u, lb = (b >> 16) | ((b & 0x7fffffu) ? 0x40u : 0u);
+  if ((b & 0x7f800000u) != 0x7f800000u) {
+    hb = b >> 16;
+    const float r = x - __uint_as_float(b & 0xffff0000u);
+    mb = ElemTraits<bf16_t>::pack2(r, 0.0f) & 0xffffu;
+    lb = ElemTraits<bf16_t>::pack2(r - __uint_as_float(mb << 16), 0.0f) & 0xffffu;
+  }
+  const int sh = half * 16;
+  const uint32_t keep = 0xffff0000u >> sh;
+  h = (h & keep) | (hb << sh);
+  m = (m & keep) | (mb << sh);
+  l = (l & keep) | (lb << sh);
+}
+
 // Four floats as three bf16 planes of 8 bytes each.
 __device__ __forceinline__ void split3(const float (&x)[4], uint2 (&p)[3]) {
   float r[4] = {x[0], x[1], x[2], x[3]};
@@ -59,6 +79,12 @@ __device__ __forceinline__ void split3(const float (&x)[4], uint2 (&p)[3]) {
       r[2] -= __uint_as_float(hi << 16);
       r[3] -= __uint_as_float(hi & 0xffff0000u);
     }
+  }
+  // What is not finite, or rounds to infinity (from 2^128 (1 - 2^-9) on), has left NaN behind.
+  if (__builtin_expect(__builtin_isunordered(r[0], r[1]) || __builtin_isunordered(r[2], r[3]), 0)) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (r[i] != r[i]) split3_not_rounded(x[i], i & 1, i < 2 ? p[0].x : p[0].y, i < 2 ? p[1].x : p[1].y, i < 2 ? p[2].x : p[2].y);
   }
 }
 

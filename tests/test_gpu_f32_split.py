@@ -29,3 +29,33 @@ def test_split_products_are_fp32(cout, scale_x, scale_w):
     ref = capi_forward(wide)
     # sums of 864 products by fp32 adds: sqrt(864) * 2^-24 = 1.8e-6 of the terms' 2-norm for random roundings
     assert float((y - ref).norm() / ref.norm()) <= 1.8e-6
+
+
+def test_what_is_not_finite_stays_what_it_is():
+    """Infinities, NaN and the largest numbers, in either operand, against one thread per output."""
+    g = torch.Generator().manual_seed(9)
+    n, c, h, w = 1, 64, 12, 14
+    x, wt = torch.randn(n, c, h, w, generator=g), torch.randn(96, c, 3, 3, generator=g)
+    # some weights are bf16 numbers, whose lower planes are zero
+    wt[:, ::2] = wt[:, ::2].bfloat16().float()
+    big = torch.finfo(torch.float32).max
+    x[0, 3, 2, 2], x[0, 4, 5, 9], x[0, 5, 9, 3] = float('inf'), -float('inf'), float('nan')
+    x[0, 6, 10, 11], x[0, 7, 10, 2] = big, -big
+    wt *= 1e-3
+    wt[5, 8, 1, 1], wt[6, 9, 0, 2], wt[7, 10, 2, 0] = float('inf'), float('nan'), big
+    # no position on a pixel (no corner has weight zero) and none outside (where one path multiplies zeros, the other nothing)
+    off = torch.rand(n, 18, h - 2, w - 2, generator=g) * 0.4 + 0.3
+    case = dict(input=x, offset=off, mask=torch.rand(n, 9, h - 2, w - 2, generator=g) * 0.5 + 0.1, weight=wt,
+                bias=None, stride=(1, 1), padding=(0, 0), dilation=(1, 1), groups=1, deform_groups=1)
+    dev = {k: v.cuda() if torch.is_tensor(v) else v for k, v in case.items()}
+    got, ref = capi_forward(dev, path=capi.PATH_FUSED), capi_forward(dev, path=capi.PATH_DIRECT)
+    assert torch.equal(got.isnan(), ref.isnan()), (int(got.isnan().sum()), int(ref.isnan().sum()))
+    assert torch.equal(got == float('inf'), ref == float('inf'))
+    assert torch.equal(got == -float('inf'), ref == -float('inf'))
+    ok = ref.isfinite()
+    assert 0 < int(ok.sum()) < ok.numel() and int((ref.abs() == float('inf')).sum()) > 100
+    # (sums that hold a product with the largest numbers are as coarse as those)
+    small = ok & (ref.abs() < 1e30)
+    assert float((got[small] - ref[small]).norm() / ref[small].norm()) <= 1e-6
+    large = ok & (ref.abs() >= 1e30)
+    assert int(large.sum()) > 100 and float(((got[large] - ref[large]) / ref[large]).abs().max()) <= 1e-5
