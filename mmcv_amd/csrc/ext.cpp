@@ -132,7 +132,7 @@ bool prepare(Prepared &pr, const Tensor &input, const Tensor &weight,
   if (!input.is_contiguous() && input.is_contiguous(at::MemoryFormat::ChannelsLast)) {
     p.input = input.data_ptr();
     p.input_nhwc = 1;
-    if (!mdcn_fused_eligible(&p) || p.path == MDCN_PATH_DIRECT) {
+    if (!mdcn_fused_eligible(&p) || p.path == MDCN_PATH_DIRECT || p.path == MDCN_PATH_SEGMENT) {
       p.input = nullptr;
       p.input_nhwc = 0;
     }
@@ -650,6 +650,10 @@ Tensor layer_call(const Tensor &input, const Tensor &offset, const c10::optional
                   int64_t dw, int64_t groups, int64_t dgroups, int64_t step) {
   const Tensor m = mask.has_value() ? *mask : Tensor(), b = bias.has_value() ? *bias : Tensor();
   const std::vector<int64_t> geo = {sh, sw, ph, pw, dh, dw, groups, dgroups, step};
+  // (a Function without a jvp refuses these, also where no gradient is recorded)
+  for (const Tensor *t : {&input, &offset, &m, &weight, &b})
+    TORCH_CHECK_NOT_IMPLEMENTED(!t->defined() || !t->_fw_grad(0).defined(),
+                                "the deformable convolutions have no forward-mode derivative");
   const bool grad = at::GradMode::is_enabled() &&
                     (input.requires_grad() || offset.requires_grad() || weight.requires_grad() ||
                      (m.defined() && m.requires_grad()) || (b.defined() && b.requires_grad()));
@@ -733,13 +737,13 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "pack_call(x, offset_weight, offset_bias | None, weight, bias | None, sh, sw, ph, pw, dh, dw, groups, "
         "deform_groups, unmodulated): the Pack layers' forward, no autograd");
   m.def("set_path", [](int path) {
-          TORCH_CHECK(path >= MDCN_PATH_AUTO && path <= MDCN_PATH_FUSED_NARROW,
+          TORCH_CHECK(path >= MDCN_PATH_AUTO && path <= MDCN_PATH_SEGMENT,
                       "path must be 0 (auto), 1 (fused), 2 (direct), 3 (fused, specialised-wave kernel only), "
-                      "4 (fused, 256-pixel kernel on every whole tile) or 5 (fused, without the 256-pixel kernel)");
+                      "4 (fused, 256-pixel kernel on every whole tile), 5 (fused, without the 256-pixel kernel) or 6 (segment kernel)");
           g_path.store(path);
         }, "choose the device path of forward and backward: 0 auto, 1 fused / matrix-core kernels, 2 direct kernels, "
            "3 fused with the specialised-wave forward kernel, 4 fused with the 256-pixel forward kernel on every "
-           "whole tile, 5 fused without that kernel", py::arg("path"));
+           "whole tile, 5 fused without that kernel, 6 the segment kernel wherever it covers the shape", py::arg("path"));
   m.def("get_path", []() { return g_path.load(); });
   m.def("set_k_split", [](bool on) { g_no_k_split.store(on ? 0 : 1); },
         "true (default): idle workgroups of the fused forward kernel's last round take parts of the K range of its "

@@ -59,3 +59,17 @@ def test_too_small_input_is_a_value_error():
     z = lambda *s: torch.zeros(*s, device='cuda')
     with pytest.raises(ValueError, match='too small'):
         modulated_deform_conv2d(z(1, 4, 2, 2), z(1, 18, 1, 1), z(1, 9, 1, 1), z(4, 4, 3, 3), None)
+
+
+def test_function_transforms_and_forward_mode_are_refused():
+    """A Function without setup_context, vmap rule and jvp refuses them; so does the one call."""
+    from mmcv_amd.ops import modulated_deform_conv2d
+    t = _leaves(torch.float32, ())
+    rest = [t[k] for k in ('offset', 'mask', 'weight', 'bias')]
+    with pytest.raises(RuntimeError):
+        torch.func.vmap(lambda x: modulated_deform_conv2d(x, *rest, 1, 1))(t['input'][None])
+    with pytest.raises(RuntimeError):
+        torch.func.grad(lambda x: modulated_deform_conv2d(x, *rest, 1, 1).sum())(t['input'])
+    with torch.autograd.forward_ad.dual_level(), pytest.raises(RuntimeError):
+        x = torch.autograd.forward_ad.make_dual(t['input'], torch.ones_like(t['input']))
+        modulated_deform_conv2d(x, *rest, 1, 1)
