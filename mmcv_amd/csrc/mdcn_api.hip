@@ -364,41 +364,6 @@ int make_pack_plan(const mdcn_pack_params *pp, const Geom &g, Plan *pl) {
   return MDCN_OK;
 }
 
-// conv_offset of one batch chunk: the tiled kernel when its input patch and one
-// slab of weights fit an LDS budget, else the gather variant.
-template <typename E, int COF>
-hipError_t launch_oconv(OconvArgs oa, hipStream_t st) {
-  const Geom &g = oa.g;
-  const int PW = 31 * g.sw + (g.kw - 1) * g.dw + 1;
-  const long wbytes = (long)g.taps * 4 * COF * 1024;
-  auto lds_bytes = [&](int th) {
-    return (long)((th - 1) * g.sh + (g.kh - 1) * g.dh + 1) * PW * kRowB + wbytes;
-  };
-  oa.tiles_x = (g.Wo + 31) / 32;
-  oa.PW = PW;
-  auto tiled = [&](int th, auto kernel) {
-    oa.TH = th;
-    oa.tiles_y = (g.Ho + th - 1) / th;
-    oa.PH = (th - 1) * g.sh + (g.kh - 1) * g.dh + 1;
-    const long tiles = (long)g.N * oa.tiles_y * oa.tiles_x;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)tiles), dim3(256), 0, st, oa);
-    return hipGetLastError();
-  };
-  // 8 rows per workgroup when that still fills the chip, else 4
-  if constexpr (COF <= 2) {
-    const long tiles8 = (long)g.N * ((g.Ho + 7) / 8) * oa.tiles_x;
-    if (lds_bytes(8) <= kOconvLdsSmall && tiles8 >= 2L * num_cus())
-      return tiled(8, oconv_tiled_kernel<E, COF, 2, kOconvLdsSmall>);
-  }
-  if (lds_bytes(4) <= kOconvLdsSmall) return tiled(4, oconv_tiled_kernel<E, COF, 1, kOconvLdsSmall>);
-  if (lds_bytes(4) <= kOconvLdsLarge) return tiled(4, oconv_tiled_kernel<E, COF, 1, kOconvLdsLarge>);
-  constexpr int PXF = COF == 1 ? 4 : (COF == 2 ? 2 : 1);
-  const long px_per_block = 4L * 32 * PXF;
-  const long blocks = (oa.total_px + px_per_block - 1) / px_per_block;
-  hipLaunchKernelGGL((oconv_gather_kernel<E, COF, PXF>), dim3((unsigned)blocks), dim3(256), 0, st, oa);
-  return hipGetLastError();
-}
-
 template <typename E, int CT, int TMAX, bool MULTI_DG>
 hipError_t launch_fused_ct(const FusedArgs &fa, bool unbordered, hipStream_t st) {
   // persistent workgroups: one per CU, a multiple of the 8 XCDs
@@ -600,13 +565,6 @@ int run_typed(const mdcn_params *p, const Geom &g, const Plan &pl, hipStream_t s
         if (hipGetLastError() != hipSuccess) rc = MDCN_ERR_LAUNCH;
         packed = true;
       }
-      if (own_oconv) {
-        const long ototal = (long)(g.Cin / pl.KC) * g.taps * 4 * cof * 64 * (16 / (long)es);
-        const int ogrid = (int)std::min<long>((ototal + 255) / 256, 1L << 16);
-        hipLaunchKernelGGL(pack_offset_weight_kernel<E>, dim3(ogrid), dim3(256), 0, st, g,
-                           (const E *)px->offset_weight, owp, pl.CO, cof, ototal);
-        if (hipGetLastError() != hipSuccess) rc = MDCN_ERR_LAUNCH;
-      }
       toc(1);
     }
     for (int n0 = 0; n0 < g.N && rc == MDCN_OK; n0 += pl.n_chunk) {
@@ -620,9 +578,14 @@ int run_typed(const mdcn_params *p, const Geom &g, const Plan &pl, hipStream_t s
         tic();
         if (!packed) {
           const int pack_blocks = (int)std::max<long>(1, std::min<long>(wtotal / (256 * 8), 512));
-          hipLaunchKernelGGL(prepass_kernel<E>, dim3((unsigned)(blocks + pack_blocks)), dim3(256), 0, st, gc, in, xt,
-                             n_pchunks, g, (const E *)p->weight, wp, pl.CT, pl.KC, pl.n_ctiles, pl.slabs, wtotal,
-                             pack_blocks, cut_cnt, pl.cut_wgs);
+          OffsetPack op = {nullptr, nullptr, 0, 1, 0, 0};
+          if (own_oconv) {
+            const long chunks = (long)(g.Cin / pl.KC) * g.taps * 4 * cof * 64;
+            op = OffsetPack{px->offset_weight, owp, pl.CO, cof, chunks, (int)std::min<long>((chunks + 255) / 256, 512)};
+          }
+          hipLaunchKernelGGL(prepass_kernel<E>, dim3((unsigned)(blocks + pack_blocks + op.blocks)), dim3(256), 0, st, gc,
+                             in, xt, n_pchunks, g, (const E *)p->weight, wp, pl.CT, pl.KC, pl.n_ctiles, pl.slabs, wtotal,
+                             pack_blocks, cut_cnt, pl.cut_wgs, op);
           packed = true;
         } else {
           hipLaunchKernelGGL((relayout_vec_kernel<E, true>), dim3((unsigned)blocks), dim3(256), 0, st, gc, in, xt,
@@ -659,10 +622,7 @@ int run_typed(const mdcn_params *p, const Geom &g, const Plan &pl, hipStream_t s
         oa.slabs_total = g.Cin / pl.KC;
         oa.plane_px = g.Hp * g.Wp;
         tic();
-        hipError_t e = cof == 1 ? launch_oconv<E, 1>(oa, st)
-                     : cof == 2 ? launch_oconv<E, 2>(oa, st)
-                     : cof == 3 ? launch_oconv<E, 3>(oa, st)
-                                : launch_oconv<E, 4>(oa, st);
+        const hipError_t e = oconv_forward(p->dtype, oa, st);
         if (e != hipSuccess) rc = MDCN_ERR_LAUNCH;
         if (px->raw) {
           const long total = (long)gc.N * pl.CO * plane_out;

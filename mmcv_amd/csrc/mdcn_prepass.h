@@ -3,6 +3,7 @@
 
 #include "mdcn_common.h"
 #include "mdcn_fused_f32.h"
+#include "mdcn_oconv.h"
 
 namespace mdcn {
 
@@ -246,22 +247,28 @@ __global__ __launch_bounds__(256) void pack_weight_kernel(
                        (long)gridDim.x * blockDim.x, zero_ptr, zero_n);
 }
 
-// Both pre-passes of a forward call in one launch: the first `pack_blocks`
-// workgroups repack the weights (geometry gw: that of the whole call), the others
+// The pre-passes of a forward call in one launch: the first `pack_blocks`
+// workgroups repack the weights (geometry gw: that of the whole call), the next
+// op.blocks (none but in a pack-level call) those of conv_offset, the others
 // re-lay the input of one batch chunk (geometry g) as relayout_vec_kernel does.
-// The two are independent, and the small weight repack hides under the copy.
+// They are independent, and the small weight repacks hide under the copy.
 template <typename E>
 __global__ __launch_bounds__(256) void prepass_kernel(Geom g, const E *__restrict__ in, E *__restrict__ xt,
                                                       int n_pchunks, Geom gw, const E *__restrict__ w,
                                                       E *__restrict__ wp, int CT, int KC, int n_ctiles, int slabs,
                                                       long wtotal, int pack_blocks,
-                                                      uint32_t *__restrict__ zero_ptr, int zero_n) {
+                                                      uint32_t *__restrict__ zero_ptr, int zero_n, OffsetPack op) {
   if ((int)blockIdx.x < pack_blocks) {
     pack_weight_elems<E>(gw, w, wp, CT, KC, n_ctiles, slabs, wtotal, (long)blockIdx.x * 256 + threadIdx.x,
                          (long)pack_blocks * 256, zero_ptr, zero_n);
     return;
   }
-  relayout_vec_block<E, true>(g, in, xt, n_pchunks, (int)blockIdx.x - pack_blocks);
+  const int b = (int)blockIdx.x - pack_blocks;
+  if (b < op.blocks) {
+    pack_offset_chunks<E>(gw, op, (long)b * 256 + threadIdx.x, (long)op.blocks * 256);
+    return;
+  }
+  relayout_vec_block<E, true>(g, in, xt, n_pchunks, b - op.blocks);
 }
 
 }  // namespace mdcn
