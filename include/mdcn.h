@@ -42,8 +42,9 @@ enum mdcn_dtype {
 
 /* Which device path runs. */
 enum mdcn_path {
-  MDCN_PATH_AUTO = 0,   /* fused MFMA kernel when the shape allows, else the segment kernel (see
-                           mdcn_workspace_wanted()), else direct */
+  MDCN_PATH_AUTO = 0,   /* fused MFMA kernel when the shape allows (the segment kernel for small calls of few
+                           channels, with the workspace of mdcn_workspace_bytes() like the fused one), else the
+                           segment kernel (see mdcn_workspace_wanted()), else direct */
   MDCN_PATH_FUSED = 1,  /* fused implicit-GEMM MFMA kernel; error if not eligible */
   MDCN_PATH_DIRECT = 2, /* one thread per output element; any shape */
   MDCN_PATH_FUSED_SPLIT = 3, /* forward only: as MDCN_PATH_FUSED, but always the fused kernel with specialised

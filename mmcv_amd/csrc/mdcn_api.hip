@@ -133,8 +133,8 @@ bool fused_ok(const mdcn_params *p, const Geom &g) {
   return true;
 }
 
-// Length of the persistent schedule of `tiles` tiles of nk K steps in tile times, as UnitSchedule lays it
-// out: whole rounds, then the last round's tiles whole or cut into parts.
+// Length of the fp32 kernel's persistent schedule of `tiles` tiles of nk K steps in tile times, as UnitSchedule lays
+// it out: whole rounds, then the last round's tiles whole or cut into parts.
 double schedule_rounds(long tiles, int nk, bool may_cut) {
   const int stride = std::max(1, num_cus() / 8);
   const long chunk = (tiles + 7) / 8;  // the fullest XCD
@@ -142,7 +142,7 @@ double schedule_rounds(long tiles, int nk, bool may_cut) {
   if (rest == 0) return (double)full;
   const int rounds = (nk + kGatherAhead - 1) / kGatherAhead;
   long parts = 1;
-  if (may_cut) parts = std::max<long>(1, std::min<long>(std::min<long>(stride / rest, kCutMax), rounds / (8 / kGatherAhead)));
+  if (may_cut) parts = std::max<long>(1, std::min<long>(std::min<long>(stride / rest, kF32CutMax), rounds / (8 / kGatherAhead)));
   return (double)full + 1.0 / (double)parts;
 }
 
@@ -155,6 +155,7 @@ struct Plan {
   size_t cut_bytes;  // eight-wave kernel: buffers and counters of the tiles it cuts along K (may be left out)
   int cut_wgs;     // ... one buffer and one counter per workgroup of its grid
   bool seg;          // segment kernel: the shapes the fused kernels do not cover
+  bool seg_small;    // ... or small calls of those they do
   SegPlan sp;
   // pack-level call only
   int CO, CO_pad;    // conv_offset channels: 3 (2 when unmodulated) * DG * taps, rounded up to 32
@@ -192,7 +193,7 @@ bool wide_ok(const mdcn_params *p, const Geom &g, const Plan &pl) {
 }
 
 // Rounds of the 128-pixel kernel's schedule for `tiles` tiles of nk K steps, in tile times (its last round's
-// tiles are cut along K when that is allowed).
+// tiles are cut along K when that is allowed; the sixth part of a tile and the sum of all six take a quarter of its time).
 double narrow_rounds(long tiles, int nk, bool may_cut) {
   if (tiles <= 0) return 0.0;
   const int stride = std::max(1, num_cus() / 8);
@@ -201,7 +202,7 @@ double narrow_rounds(long tiles, int nk, bool may_cut) {
   if (rest == 0) return (double)full;
   const long steps6 = (nk + kF2Unroll - 1) / kF2Unroll;
   long parts = 1;
-  if (may_cut) parts = std::max<long>(1, std::min<long>(std::min<long>(stride / rest, kCutMax), steps6));
+  if (may_cut) parts = std::max<long>(1, std::min<long>(std::min<long>(stride / rest, 4), steps6));
   return (double)full + 1.0 / (double)parts;
 }
 
@@ -258,12 +259,33 @@ void drop_segments(Plan *pl) {
   pl->xt_bytes = pl->wp_bytes = 0;
 }
 
-int make_plan(const mdcn_params *p, const Geom &g, Plan *pl) {
+// Small calls of few terms, which the fused kernels cover too: there a tile's table, its first gathers and the sum
+// of its parts are most of the time, and a wavefront of the segment kernel has none of these.  Up to 18 iterations
+// (64 input channels of 3x3) and 64 output channels, until it has three waves per CU before they share K.  Whole
+// call, us, fused / segment kernel: fp32 64 -> 64 28x28 23.7 / 21.6, 56x56 26.9 / 22.9, 120x120 37.4 / 30.0, 150x150
+// 42.5 / 38.4, 200x200 64 / 64; 64 -> 256 56x56 37 / 44, 128 -> 64 32.1 / 34.8; bf16 64 -> 64 56x56 19.5 / 14.4, 150x150
+// 26.2 / 21.5, 200x200 34.1 / 34.5.
+// Never with more scratch than the fused kernels ask for.
+bool small_call(const mdcn_params *p, const Geom &g, const Plan &fused, Plan *alt) {
+  if (p->path != MDCN_PATH_AUTO || p->input_nhwc || !fused.fused) return false;
+  *alt = fused;
+  alt->fused = false;
+  plan_segments(p, g, alt);
+  if (!alt->seg || alt->n_chunk != g.N || alt->sp.iters > 18 || alt->sp.nb > 2) return false;
+  const long waves = ((long)g.N * g.Ho * g.Wo + 31) / 32 * alt->sp.n_ctiles * g.G;
+  if (waves > 3L * num_cus() || alt->xt_bytes + alt->wp_bytes > fused.xt_bytes + fused.wp_bytes) return false;
+  alt->seg_small = true;
+  alt->cut_bytes = 0;
+  alt->cut_wgs = 0;
+  return true;
+}
+
+int make_plan(const mdcn_params *p, const Geom &g, Plan *pl, bool may_be_small = true) {
   const bool ok = fused_ok(p, g);
   if (forced_fused(p->path) && !ok) return MDCN_ERR_PATH;
   if (p->input_nhwc && (!ok || p->path == MDCN_PATH_DIRECT || p->path == MDCN_PATH_SEGMENT)) return MDCN_ERR_PATH;  // in-place reads: fused kernel only
   pl->fused = ok && p->path != MDCN_PATH_DIRECT && p->path != MDCN_PATH_SEGMENT;
-  pl->seg = false;
+  pl->seg = pl->seg_small = false;
   pl->CT = pl->KC = pl->n_ctiles = pl->slabs = pl->n_chunk = 0;
   pl->xt_bytes = pl->wp_bytes = pl->owp_bytes = pl->raw_bytes = pl->cut_bytes = 0;
   pl->cut_wgs = 0;
@@ -291,6 +313,23 @@ int make_plan(const mdcn_params *p, const Geom &g, Plan *pl) {
       return schedule_rounds(tiles, nk, !p->no_k_split) * (ct == 256 ? 1.0 : 0.56);
     };
     if (cost(128) < 0.95 * cost(256)) pl->CT = 128;
+  }
+  // Few tiles: narrower ones, so that more workgroups have a part of one and its sum is shorter.  16 bits: the narrowest
+  // that still leaves two workgroups a tile (eight-wave kernel: 128 channels at least).  fp32, whose waves
+  // split the samples again for every tile of channels: 64, where that leaves four.  Whole call, us, wide / narrow:
+  // bf16 256 channels 14x14 30 / 23 (128), 90x90 37.4 / 34.0, 100x100 (a workgroup a tile) 38.2 / 42.2; 512 channels 25x42 41 / 34;
+  // 4 deformable groups, 256 channels 28x28 N=2 50 / 29 (64), 512 channels 25x42 76 / 50, N=2 79 / 70 (128) / 90 (64);
+  // fp32 256 channels 14x14 42 / 36, 28x28 48 / 43, 512 channels 25x42 (three a tile) 84 / 89.
+  if (!p->no_k_split) {
+    const long px_tiles = ((long)pl->n_chunk * g.Ho * g.Wo + kPT - 1) / kPT;
+    const bool f32 = p->dtype == MDCN_F32;
+    for (int ct : {64, 128}) {
+      const long tiles = px_tiles * ((g.cout_g + ct - 1) / ct) * g.G;
+      if (ct < pl->CT && (ct == 64 ? f32 || !uses_fused2(p, g, *pl) : !f32) && tiles * (f32 ? 4 : 2) <= num_cus()) {
+        pl->CT = ct;
+        break;
+      }
+    }
   }
   pl->n_ctiles = (g.cout_g + pl->CT - 1) / pl->CT;
   pl->xt_bytes = p->input_nhwc ? 0 : align_up((size_t)img * pl->n_chunk);
@@ -329,6 +368,8 @@ int make_plan(const mdcn_params *p, const Geom &g, Plan *pl) {
     }
   }
   if (p->path == MDCN_PATH_FUSED_WIDE && !wide_ok(p, g, *pl)) return MDCN_ERR_PATH;
+  Plan alt;
+  if (may_be_small && small_call(p, g, *pl, &alt)) *pl = alt;
   return MDCN_OK;
 }
 
@@ -337,7 +378,7 @@ int make_plan(const mdcn_params *p, const Geom &g, Plan *pl) {
 int make_pack_plan(const mdcn_pack_params *pp, const Geom &g, Plan *pl) {
   const mdcn_params *p = &pp->conv;
   if (p->input_nhwc) return MDCN_ERR_PATH;
-  const int rc = make_plan(p, g, pl);
+  const int rc = make_plan(p, g, pl, false);
   if (rc != MDCN_OK) return rc;
   if (pp->unmodulated) {
     pl->CO = 2 * g.DG * g.taps;
@@ -647,7 +688,7 @@ int run_typed(const mdcn_params *p, const Geom &g, const Plan &pl, hipStream_t s
         fa.om = dense_view((const E *)p->offset + (size_t)n0 * g.DG * 2 * g.taps * plane_out,
                            p->mask ? (const E *)p->mask + (size_t)n0 * g.DG * g.taps * plane_out : nullptr, g);
       }
-      fa.cut_max = pl.cut_bytes ? kCutMax : 0;
+      fa.cut_max = !pl.cut_bytes ? 0 : sizeof(E) == 4 ? kF32CutMax : uses_fused2(p, g, pl) ? kF2CutMax : kCutMax;
       fa.cut_part = cut_part;
       fa.cut_cnt = cut_cnt;
       fa.bias = p->bias;
@@ -737,7 +778,7 @@ int run(const mdcn_params *p, void *stream, float *ms, const mdcn_pack_params *p
   }
   // (the split-tile buffers come last and are optional: a workspace without them runs unsplit)
   // a call whose workspace does not hold the segment kernel's copies runs without that kernel, as it may
-  if (pl.seg && (p->workspace_bytes < pl.xt_bytes + pl.wp_bytes + pl.raw_bytes || !p->workspace ||
+  if (pl.seg && !pl.seg_small && (p->workspace_bytes < pl.xt_bytes + pl.wp_bytes + pl.raw_bytes || !p->workspace ||
                  ((uintptr_t)p->workspace % kAlign) != 0))
     drop_segments(&pl);
   const size_t need = pl.xt_bytes + pl.wp_bytes + pl.owp_bytes + pl.raw_bytes;
@@ -839,7 +880,7 @@ size_t mdcn_workspace_bytes(const mdcn_params *p) {
   if (check_params(p, &g, false) != MDCN_OK) return 0;
   Plan pl;
   if (make_plan(p, g, &pl) != MDCN_OK) return 0;
-  return pl.seg ? 0 : pl.xt_bytes + pl.wp_bytes + pl.cut_bytes;
+  return pl.seg && !pl.seg_small ? 0 : pl.xt_bytes + pl.wp_bytes + pl.cut_bytes;
 }
 
 size_t mdcn_workspace_wanted(const mdcn_params *p) {
@@ -862,7 +903,7 @@ int mdcn_forward_noalloc(const mdcn_params *p, void *hip_stream) {
   rc = make_plan(p, g, &pl);
   if (rc != MDCN_OK) return rc;
   mdcn_params q = *p;
-  if (pl.seg) {  // needs no scratch: the kernel, and the bits, of a mdcn_forward() with mdcn_workspace_bytes()
+  if (pl.seg && !pl.seg_small) {  // needs no scratch: the kernel, and the bits, of a mdcn_forward() with mdcn_workspace_bytes()
     q.workspace = nullptr;
     q.workspace_bytes = 0;
     return run(&q, hip_stream, nullptr);

@@ -54,7 +54,12 @@ constexpr int kProducerWaves = 4;                        // waves 4 .. 4 + kProd
 constexpr int kThreads = 256 + 64 * kProducerWaves;
 constexpr int kPxPerLane = 8 / kProducerWaves;           // pixels of the tile a producer lane serves
 constexpr int kTapGroups = kProducerWaves / 2;           // producer lanes per pixel in the table build
-constexpr int kCutMax = 4;         // parts a tile of the schedule's last round is cut into at most
+// Parts a tile of the schedule's last round is cut into at most.  The part that arrives last adds all of them up by
+// itself, 128 KiB each for a tile of 256 channels, so that more parts end by costing more than the steps they save.  (Whole call,
+// us.  bf16, eight-wave kernel, 512 channels 25x42: 4 parts 44.2, 6 41.2, 8 42.5, 12 45.9, and with 128-channel tiles 35.9, 33.6,
+// 33.2, 33.2.  fp32: 256 channels 14x14 4 parts 48, 8 42; 512 channels 25x42 92, 84, 16 parts of fewer steps 83.  Kernel
+// with specialised waves, 16 bits, 512 channels 25x42, 4 deformable groups: 4 parts 76, 8 80.)
+constexpr int kCutMax = 4, kF2CutMax = 6, kF32CutMax = 8;
 
 struct FusedArgs {
   Geom g;
