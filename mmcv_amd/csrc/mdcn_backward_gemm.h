@@ -25,7 +25,10 @@
 // and its gradients are zero and never written.
 #pragma once
 
+#include <type_traits>
+
 #include "mdcn_backward.h"
+#include "mdcn_fused_f32.h"
 
 namespace mdcn {
 
@@ -51,6 +54,89 @@ struct ColGradArgs {
   long total;      // workgroups with work: images of the pass x G x px_tiles x m_tiles
   uint32_t *dmax;  // bit pattern of the largest |d| stored so far (a float >= 0), or null
 };
+
+// A wave's products of one K step of either kernel: TILE / 64 x 2 blocks of 32 x 32 over 128 bytes of K, operand tiles
+// [row][8 chunks of 16 bytes, swizzled by the row number].
+//
+// fp32 runs on the bf16 matrix pipe: three bf16 planes per operand and six of their nine products, as in
+// fused_f32_kernel, whose error is that of fp32 arithmetic.  Operands are split behind the LDS reads (every wave for
+// itself: some 290 VALU instructions per 16 of K beside 48 MFMAs of 32 clocks, where the fp32 MFMAs were 64 of 64
+// clocks).  An infinity, or a number that bf16 rounds to one, leaves NaN in the planes and so in the sums: a workgroup that
+// finds any goes over its K range again with fp32 MFMAs (EXACT).
+// N=2 256 -> 256 50x84, us, fp32 / bf16 pipe: column gradient 151 / 93, weight gradient 107 / 70.  Errors against float64
+// (2-norm): grad_input 2.9e-7 / 2.5e-7, grad_weight 3.3e-7 / 3.0e-7.
+template <typename E, int TILE, bool EXACT>
+__device__ __forceinline__ void tile_products(f32x16 (&acc)[TILE / 64][2], const uint4 *A, const uint4 *B, int wm, int wn,
+                                              int frow, int fhalf) {
+  using TR = ElemTraits<E>;
+  constexpr int MB = TILE / 64;
+  // (the rows of a lane's fragments are multiples of 32 apart: one swizzle for all of them)
+  const uint4 *a0 = A + (wm * (TILE / 2) + frow) * 8, *b0 = B + (wn * 64 + frow) * 8;
+  auto load_a = [&](int mb, int ksub) { return a0[mb * 256 + ((ksub * 2 + fhalf) ^ (frow & 7))]; };
+  auto load_b = [&](int nb, int ksub) { return b0[nb * 256 + ((ksub * 2 + fhalf) ^ (frow & 7))]; };
+  if constexpr (sizeof(E) == 2 || EXACT) {
+#pragma unroll
+    for (int ksub = 0; ksub < 4; ++ksub) {
+      uint4 af[MB], bf[2];
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) af[mb] = load_a(mb, ksub);
+#pragma unroll
+      for (int nb = 0; nb < 2; ++nb) bf[nb] = load_b(nb, ksub);
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int nb = 0; nb < 2; ++nb) TR::mma(acc[mb][nb], af[mb], bf[nb]);
+    }
+  } else {
+    using TB = ElemTraits<bf16_t>;
+    // 8 values of K as three planes of an operand
+    auto split8 = [](const uint4 (&v)[2], uint4 (&p)[3]) {
+      uint2 lo[3], hi[3];
+      float r[4];
+      split3_finite({__uint_as_float(v[0].x), __uint_as_float(v[0].y), __uint_as_float(v[0].z), __uint_as_float(v[0].w)}, r, lo);
+      split3_finite({__uint_as_float(v[1].x), __uint_as_float(v[1].y), __uint_as_float(v[1].z), __uint_as_float(v[1].w)}, r, hi);
+#pragma unroll
+      for (int s = 0; s < 3; ++s) p[s] = make_uint4(lo[s].x, lo[s].y, hi[s].x, hi[s].y);
+    };
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {  // (any order of K will do: both operands have the same)
+      uint4 bp[2][3];
+#pragma unroll
+      for (int nb = 0; nb < 2; ++nb) split8({load_b(nb, half * 2), load_b(nb, half * 2 + 1)}, bp[nb]);
+      uint4 af[2] = {load_a(0, half * 2), load_a(0, half * 2 + 1)};
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) {
+        uint4 ap[3];
+        split8(af, ap);
+        if (mb + 1 < MB) af[0] = load_a(mb + 1, half * 2), af[1] = load_a(mb + 1, half * 2 + 1);
+        __builtin_amdgcn_sched_barrier(0);  // (or every block's planes are made ahead and spilled)
+        auto products = [&](int pa, int pb) {
+#pragma unroll
+          for (int nb = 0; nb < 2; ++nb) TB::mma(acc[mb][nb], ap[pa], bp[nb][pb]);
+        };
+        products(2, 0);  // smallest terms first
+        products(0, 2);
+        products(1, 1);
+        products(1, 0);
+        products(0, 1);
+        products(0, 0);
+      }
+    }
+  }
+}
+
+// Whether a sum is infinite or NaN.
+template <int MB>
+__device__ __forceinline__ bool not_finite(const f32x16 (&acc)[MB][2]) {
+  float t = 0.0f;
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) t = fmaf(acc[mb][nb][r], 0.0f, t);
+  return t != t;
+}
 
 // Workgroup = TILE rows of wT (one group) x TILE pixels of one image, reduction
 // over the group's output channels in slabs of 128 bytes; TILE / 32 waves as
@@ -110,42 +196,32 @@ __global__ __launch_bounds__(TILE * 2, TILE == 128 ? 2 : 1) void bwd_colgrad_ker
   };
 
   f32x16 acc[MB][2];
+  auto sweep = [&](auto how) {
+    constexpr bool exact = decltype(how)::value;
 #pragma unroll
-  for (int i = 0; i < MB; ++i)
+    for (int i = 0; i < MB; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
-  issue(0, 0);
-  for (int ks = 0; ks < a.kslabs; ++ks) {
-    const int buf = ks & 1;
-    if (ks + 1 < a.kslabs) {
-      issue(ks + 1, buf ^ 1);  // (its buffer was last read before the barrier that ended step ks - 1)
-      asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-    } else {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    }
-    __syncthreads();
-#pragma unroll
-    for (int ksub = 0; ksub < 4; ++ksub) {
-      uint4 af[MB], bf[2];
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb) {
-        const int row = wm * (TILE / 2) + mb * 32 + frow;
-        af[mb] = As[buf][row * 8 + ((ksub * 2 + fhalf) ^ (row & 7))];
+    issue(0, 0);
+    for (int ks = 0; ks < a.kslabs; ++ks) {
+      const int buf = ks & 1;
+      if (ks + 1 < a.kslabs) {
+        issue(ks + 1, buf ^ 1);  // (its buffer was last read before the barrier that ended step ks - 1)
+        asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+      } else {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       }
-#pragma unroll
-      for (int nb = 0; nb < 2; ++nb) {
-        const int row = wn * 64 + nb * 32 + frow;
-        bf[nb] = Bs[buf][row * 8 + ((ksub * 2 + fhalf) ^ (row & 7))];
-      }
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-        for (int nb = 0; nb < 2; ++nb) TR::mma(acc[mb][nb], af[mb], bf[nb]);
+      __syncthreads();
+      tile_products<E, TILE, exact>(acc, As[buf], Bs[buf], wm, wn, frow, fhalf);
+      __syncthreads();
     }
-    __syncthreads();
+  };
+  sweep(std::false_type());
+  if constexpr (sizeof(E) == 4) {
+    if (__syncthreads_or(not_finite(acc))) sweep(std::true_type());
   }
 
   // register r of lane l: A row (r/4)*8 + (l/32)*4 + r%4 of the block, B row l%32
@@ -717,7 +793,6 @@ struct WGradArgs {
 // not vary from run to run.
 template <typename E, int TILE>
 __global__ __launch_bounds__(TILE * 2, TILE == 128 ? 2 : 1) void bwd_wgrad_kernel(WGradArgs a) {
-  using TR = ElemTraits<E>;
   constexpr int ES = (int)sizeof(E);
   constexpr int PXC = 16 / ES;  // pixels per 16-byte chunk
   constexpr int MB = TILE / 64;
@@ -769,49 +844,39 @@ __global__ __launch_bounds__(TILE * 2, TILE == 128 ? 2 : 1) void bwd_wgrad_kerne
     }
   };
 
-  f32x16 acc[MB][2];
-#pragma unroll
-  for (int i = 0; i < MB; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-
   // this workgroup's contiguous share of the (image, K step) range
   const long work = (long)a.nb * a.ksteps;
   const long per = (work + a.splits - 1) / a.splits;
   const long w_begin = (long)split * per, w_end = min(work, w_begin + per);
-  if (w_begin < w_end) {
-    issue(w_begin, 0);
-    int buf = 0;
-    for (long wi = w_begin; wi < w_end; ++wi, buf ^= 1) {
-      if (wi + 1 < w_end) {
-        issue(wi + 1, buf ^ 1);
-        asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-      } else {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      }
-      __syncthreads();
+  f32x16 acc[MB][2];
+  auto sweep = [&](auto how) {
+    constexpr bool exact = decltype(how)::value;
 #pragma unroll
-      for (int ksub = 0; ksub < 4; ++ksub) {
-        uint4 af[MB], bf[2];
+    for (int i = 0; i < MB; ++i)
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb) {
-          const int row = wm * (TILE / 2) + mb * 32 + frow;
-          af[mb] = As[buf][row * 8 + ((ksub * 2 + fhalf) ^ (row & 7))];
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+
+    if (w_begin < w_end) {
+      issue(w_begin, 0);
+      int buf = 0;
+      for (long wi = w_begin; wi < w_end; ++wi, buf ^= 1) {
+        if (wi + 1 < w_end) {
+          issue(wi + 1, buf ^ 1);
+          asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+        } else {
+          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         }
-#pragma unroll
-        for (int nb = 0; nb < 2; ++nb) {
-          const int row = wn * 64 + nb * 32 + frow;
-          bf[nb] = Bs[buf][row * 8 + ((ksub * 2 + fhalf) ^ (row & 7))];
-        }
-#pragma unroll
-        for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-          for (int nb = 0; nb < 2; ++nb) TR::mma(acc[mb][nb], af[mb], bf[nb]);
+        __syncthreads();
+        tile_products<E, TILE, exact>(acc, As[buf], Bs[buf], wm, wn, frow, fhalf);
+        __syncthreads();
       }
-      __syncthreads();
     }
+  };
+  sweep(std::false_type());
+  if constexpr (sizeof(E) == 4) {
+    if (__syncthreads_or(not_finite(acc))) sweep(std::true_type());
   }
 
   // register r of lane l: A row (output channel) (r/4)*8 + (l/32)*4 + r%4 of the block, B row (column row) l%32

@@ -65,9 +65,10 @@ __device__ __forceinline__ void split3_not_rounded(float x, int half, uint32_t &
   l = (l & keep) | (lb << sh);
 }
 
-// Four floats as three bf16 planes of 8 bytes each.
-__device__ __forceinline__ void split3(const float (&x)[4], uint2 (&p)[3]) {
-  float r[4] = {x[0], x[1], x[2], x[3]};
+// Four floats, finite and below 2^128 (1 - 2^-9), as three bf16 planes of 8 bytes each; r: what each plane but the last left.
+__device__ __forceinline__ void split3_finite(const float (&x)[4], float (&r)[4], uint2 (&p)[3]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) r[i] = x[i];
 #pragma unroll
   for (int s = 0; s < 3; ++s) {
     uint32_t lo = ElemTraits<bf16_t>::pack2(r[0], r[1]), hi = ElemTraits<bf16_t>::pack2(r[2], r[3]);
@@ -80,6 +81,12 @@ __device__ __forceinline__ void split3(const float (&x)[4], uint2 (&p)[3]) {
       r[3] -= __uint_as_float(hi & 0xffff0000u);
     }
   }
+}
+
+// ... any four floats.
+__device__ __forceinline__ void split3(const float (&x)[4], uint2 (&p)[3]) {
+  float r[4];
+  split3_finite(x, r, p);
   // What is not finite, or rounds to infinity (from 2^128 (1 - 2^-9) on), has left NaN behind.
   if (__builtin_expect(__builtin_isunordered(r[0], r[1]) || __builtin_isunordered(r[2], r[3]), 0)) {
 #pragma unroll

@@ -59,3 +59,45 @@ def test_what_is_not_finite_stays_what_it_is():
     assert float((got[small] - ref[small]).norm() / ref[small].norm()) <= 1e-6
     large = ok & (ref.abs() >= 1e30)
     assert int(large.sum()) > 100 and float(((got[large] - ref[large]) / ref[large]).abs().max()) <= 1e-5
+
+
+def _backward_case(seed, n, cin, cout, h, w):
+    g = torch.Generator().manual_seed(seed)
+    off = torch.round(torch.randn(n, 18, h, w, generator=g) * 8) / 4 + 0.125   # exact, and never on a pixel
+    case = dict(input=torch.randn(n, cin, h, w, generator=g), offset=off,
+                mask=torch.round(torch.rand(n, 9, h, w, generator=g) * 255 + 1) / 256,
+                weight=torch.randn(cout, cin, 3, 3, generator=g) * 0.05, bias=None, stride=(1, 1), padding=(1, 1),
+                dilation=(1, 1), groups=1, deform_groups=1)
+    gy = torch.randn(n, cout, h, w, generator=g) * 10.0 ** (torch.rand(n, cout, h, w, generator=g) * 4 - 2)
+    return {k: v.cuda() if torch.is_tensor(v) else v for k, v in case.items()}, gy.cuda()
+
+
+@pytest.mark.parametrize('cin,cout', [(64, 64), (256, 200), (40, 256)], ids=['tile128', 'tile256', 'padded'])
+def test_gradients_are_fp32(cin, cout):
+    from common import capi_backward
+    dev, gy = _backward_case(cin, 2, cin, cout, 17, 21)
+    got = capi_backward(dev, gy, path=capi.PATH_FUSED)
+    ref = capi_backward({k: v.double() if torch.is_tensor(v) else v for k, v in dev.items()}, gy.double())
+    # grad_input, grad_offset, grad_mask: sums over cout and then over some 9 cin at most; grad_weight: over 714 pixels.
+    # Roundings of 2^-24 each, at random: sqrt(terms) of them.  grad_bias aside (float sums of grad_output).
+    for name, a, b in zip(('input', 'offset', 'mask', 'weight'), got, ref):
+        terms = 714 if name == 'weight' else cout + 9 * cin
+        assert float((a.double() - b).norm() / b.norm()) <= terms ** 0.5 * 2.0 ** -24, name
+
+
+@pytest.mark.parametrize('cin,cout', [(64, 64), (256, 256)], ids=['tile128', 'tile256'])
+def test_gradients_of_what_is_not_finite(cin, cout):
+    """An infinity, a NaN and the largest number in grad_output stay in the gradients they belong to."""
+    from common import capi_backward
+    dev, gy = _backward_case(cin + 1, 1, cin, cout, 16, 18)
+    big = torch.finfo(torch.float32).max
+    dev['weight'] *= 1e-3
+    gy[0, 3, 4, 5], gy[0, 9, 12, 7], gy[0, 11, 9, 9] = float('inf'), float('nan'), big
+    got = capi_backward(dev, gy, path=capi.PATH_FUSED)
+    ref = capi_backward(dev, gy, path=capi.PATH_DIRECT)
+    assert torch.equal(got[3].isnan(), ref[3].isnan()) and torch.equal(got[3].isinf(), ref[3].isinf())
+    for name, a, b in zip(('input', 'offset', 'mask', 'weight'), got, ref):
+        assert torch.equal(a.isfinite(), b.isfinite()), name
+        small = b.isfinite() & (b.abs() < 1e28)
+        assert 0 < int(small.sum()) < small.numel(), name
+        assert float((a[small] - b[small]).norm() / b[small].norm()) <= 1e-5, name
