@@ -262,8 +262,8 @@ void drop_segments(Plan *pl) {
 // Small calls of few terms, which the fused kernels cover too: there a tile's table, its first gathers and the sum
 // of its parts are most of the time, and a wavefront of the segment kernel has none of these.  Up to 18 iterations
 // (64 input channels of 3x3) and 64 output channels, until it has three waves per CU before they share K.  Whole
-// call, us, fused / segment kernel: fp32 64 -> 64 28x28 23.7 / 21.6, 56x56 26.9 / 22.9, 120x120 37.4 / 30.0, 150x150
-// 42.5 / 38.4, 200x200 64 / 64; 64 -> 256 56x56 37 / 44, 128 -> 64 32.1 / 34.8; bf16 64 -> 64 56x56 19.5 / 14.4, 150x150
+// call, us, fused / segment kernel: fp32 64 -> 64 28x28 24.1 / 18.4, 56x56 26.6 / 19.4, 120x120 37.4 / 29.6, 150x150
+// 43.6 / 43.0; 64 -> 256 56x56 37 / 44, 128 -> 64 32.1 / 34.8 (fp32 MFMAs); bf16 64 -> 64 56x56 19.5 / 14.4, 150x150
 // 26.2 / 21.5, 200x200 34.1 / 34.5.
 // Never with more scratch than the fused kernels ask for.
 bool small_call(const mdcn_params *p, const Geom &g, const Plan &fused, Plan *alt) {

@@ -30,7 +30,7 @@ struct SegPlan {
 struct SegArgs {
   Geom g;
   const void *xt;   // [N][chunks][H + 2][W + 2][16 bytes], chunks in order of the padded channels
-  const void *wp;   // [G][n_ctiles][iters][cq][nb][64 lanes][16 bytes]
+  const void *wp;   // [G][n_ctiles][iters][cq, split fp32: cq / 2 x 3 planes][nb][64 lanes][16 bytes]
   OffMaskView om;
   const void *bias;
   void *out;

@@ -19,21 +19,29 @@
 // Few pixels: `kshare` waves of the workgroup split the pairs of a pixel block
 // among them and add their accumulators up through LDS, in a fixed order.
 //
-// What bounds it: the vector-memory path of the CU, 64 bytes of corner data per
-// 16 bytes of S; with fp32 tensors the MFMAs (32x32x2) are close behind.  Measured against the
-// one-thread-per-output kernel that these shapes had before: N=2, 64 -> 64 channels, 8 deformable groups,
-// 180x320, fp32 23.9 ms -> 0.15 ms + 0.013 ms of pre-pass; N=4, 96 -> 72 channels, 2 deformable groups,
-// 37x53, bf16 1 733 us -> 15 + 5 us.
+// fp32 with two or more chunks a position: the products run on the bf16 matrix pipe, three exact planes per operand
+// and six of their nine products (mdcn_fused_f32.h); weights are split when they are packed, samples behind the blend.
+//
+// What bounds it: the vector-memory path of the CU (64 bytes of corner data per 16 bytes of S), the VALU (position,
+// blend, split) and the MFMAs take some 50 us each of the dg8 case below, and two to four waves a SIMD overlap them
+// only in part.  Measured against the one-thread-per-output kernel that these shapes had before: N=2, 64 -> 64 channels, 8 deformable
+// groups, 180x320, fp32 23.9 ms -> 193 us a call with fp32 MFMAs, 178 on the bf16 pipe (error against float64 4.3e-7 -> 1.8e-7);
+// N=1 64 -> 64 56x56 22.6 -> 19.2 us; N=4, 96 -> 72 channels, 2 deformable groups, 37x53, bf16 1 733 us -> 15 + 5 us.
 #include "mdcn_segment.h"
 
 #include <algorithm>
 
 #include "../../include/mdcn.h"
-#include "mdcn_fused.h"
+#include "mdcn_fused_f32.h"
 
 namespace mdcn {
 
 namespace {
+
+// fp32 on the bf16 matrix pipe, three planes per operand (mdcn_fused_f32.h): two chunks fill the K of one MFMA.
+constexpr bool seg_split(int es, int cq) { return es == 4 && cq >= 2; }
+// 16-byte weight fragments of one iteration and 32-channel block
+constexpr int seg_frags(int es, int cq) { return seg_split(es, cq) ? cq / 2 * 3 : cq; }
 
 // Weights to A-operand order and the input to chunk planes, one launch: the first
 // pack_blocks workgroups repack, the others copy 256 pixels of the bordered plane
@@ -45,7 +53,9 @@ __global__ __launch_bounds__(256) void seg_prepass_kernel(SegArgs a, const E *__
   const Geom &g = a.g;
   const SegPlan &s = a.s;
   if ((int)blockIdx.x < pack_blocks) {
-    const long total = (long)g.G * s.n_ctiles * s.iters * s.cq * s.nb * 64;
+    const bool split = seg_split((int)sizeof(E), s.cq);
+    const int qn = split ? s.cq / 2 : s.cq;     // fragments of an iteration, each of them three planes when split
+    const long total = (long)g.G * s.n_ctiles * s.iters * qn * s.nb * 64;
     const int grp_per_seg = s.cps / s.cq;
     for (long idx = (long)blockIdx.x * 256 + threadIdx.x; idx < total; idx += (long)pack_blocks * 256) {
       long r = idx;
@@ -53,8 +63,9 @@ __global__ __launch_bounds__(256) void seg_prepass_kernel(SegArgs a, const E *__
       r >>= 6;
       const int nb = (int)(r % s.nb);
       r /= s.nb;
-      const int q = (int)(r % s.cq);
-      r /= s.cq;
+      const long frag = r;  // (group, tile, iteration, fragment)
+      const int q = (int)(r % qn);
+      r /= qn;
       const int it = (int)(r % s.iters);
       r /= s.iters;
       const int ct = (int)(r % s.n_ctiles);
@@ -63,15 +74,28 @@ __global__ __launch_bounds__(256) void seg_prepass_kernel(SegArgs a, const E *__
       const int col = (ct * s.nb + nb) * 32 + (lane & 31);
       const int sg = p / g.taps, tap = p - sg * g.taps;
       const int sl = sg / grp_per_seg;                                   // segment of the group
-      const int c0 = ((sg - sl * grp_per_seg) * s.cq + q) * VC;           // first channel of the chunk in it
-      E v[VC];
-#pragma unroll
-      for (int i = 0; i < VC; ++i) {
+      // first channel of the fragment in it
+      const int c0 = ((sg - sl * grp_per_seg) * s.cq + (split ? 2 * q : q)) * VC;
+      auto at = [&](int i) {
         const bool ok = p < s.pairs && col < g.cout_g && c0 + i < s.seg;
         const E *src = w + ((long)(grp * g.cout_g + (ok ? col : 0)) * g.cin_g + (ok ? sl * s.seg + c0 + i : 0)) * g.taps +
                        (ok ? tap : 0);
-        v[i] = ok ? *src : from_f32<E>(0.0f);
+        return ok ? *src : from_f32<E>(0.0f);
+      };
+      if constexpr (sizeof(E) == 4) {
+        if (split) {
+          uint2 p0[3], p1[3];
+          split3({at(0), at(1), at(2), at(3)}, p0);
+          split3({at(4), at(5), at(6), at(7)}, p1);
+#pragma unroll
+          for (int k = 0; k < 3; ++k)
+            ((uint4 *)a.wp)[((frag * 3 + k) * s.nb + nb) * 64 + lane] = make_uint4(p0[k].x, p0[k].y, p1[k].x, p1[k].y);
+          continue;
+        }
       }
+      E v[VC];
+#pragma unroll
+      for (int i = 0; i < VC; ++i) v[i] = at(i);
       uint4 o;
       __builtin_memcpy(&o, v, 16);
       ((uint4 *)a.wp)[idx] = o;
@@ -103,10 +127,13 @@ __global__ __launch_bounds__(256) void seg_prepass_kernel(SegArgs a, const E *__
 }
 
 // Waves per SIMD the register budget is cut for.
-constexpr int seg_occupancy(int NB, int CQ) { return CQ * NB <= 4 && NB <= 2 ? 4 : (NB <= 4 && CQ * NB <= 8 ? 3 : 2); }
+constexpr int seg_occupancy(int ES, int NB, int CQ) {
+  if (seg_split(ES, CQ)) return CQ * NB <= 4 && CQ == 2 ? 3 : 2;
+  return CQ * NB <= 4 && NB <= 2 ? 4 : (NB <= 4 && CQ * NB <= 8 ? 3 : 2);
+}
 
 template <typename E, int NB, int CQ>
-__global__ __launch_bounds__(256, seg_occupancy(NB, CQ)) void segment_kernel(SegArgs a) {
+__global__ __launch_bounds__(256, seg_occupancy((int)sizeof(E), NB, CQ)) void segment_kernel(SegArgs a) {
   using TR = ElemTraits<E>;
   const Geom &g = a.g;
   const SegPlan &s = a.s;
@@ -188,11 +215,13 @@ __global__ __launch_bounds__(256, seg_occupancy(NB, CQ)) void segment_kernel(Seg
       o += a.plane_bytes;
     }
   };
-  const uint4 *wp = (const uint4 *)a.wp + (size_t)(grp * s.n_ctiles + ct) * s.iters * (CQ * NB * 64) + lane;
-  auto load_w = [&](int i, uint4 (&wf)[CQ][NB]) {
-    const uint4 *src = wp + (size_t)i * (CQ * NB * 64);
+  constexpr bool kSplit = seg_split((int)sizeof(E), CQ);
+  constexpr int FR = seg_frags((int)sizeof(E), CQ);
+  const uint4 *wp = (const uint4 *)a.wp + (size_t)(grp * s.n_ctiles + ct) * s.iters * (FR * NB * 64) + lane;
+  auto load_w = [&](int i, uint4 (&wf)[FR][NB]) {
+    const uint4 *src = wp + (size_t)i * (FR * NB * 64);
 #pragma unroll
-    for (int q = 0; q < CQ; ++q)
+    for (int q = 0; q < FR; ++q)
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb) wf[q][nb] = src[(q * NB + nb) * 64];
   };
@@ -207,7 +236,7 @@ __global__ __launch_bounds__(256, seg_occupancy(NB, CQ)) void segment_kernel(Seg
   if (i0 < i1) {
     Raw raw;
     Gather gv;
-    uint4 wf[CQ][NB];
+    uint4 wf[FR][NB];
     load_om(i0, raw);
     gather(raw, gv);
     load_w(i0, wf);
@@ -216,18 +245,42 @@ __global__ __launch_bounds__(256, seg_occupancy(NB, CQ)) void segment_kernel(Seg
       uint4 x[CQ];
 #pragma unroll
       for (int q = 0; q < CQ; ++q) x[q] = TR::blend(gv.v[q][0], gv.v[q][1], gv.v[q][2], gv.v[q][3], gv.w);
-      uint4 wc[CQ][NB];
+      uint4 wc[kSplit ? 1 : FR][NB];  // (split fp32 has no registers for both: its next fragments are fetched behind the products)
+      if constexpr (!kSplit) {
 #pragma unroll
-      for (int q = 0; q < CQ; ++q)
+        for (int q = 0; q < FR; ++q)
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) wc[q][nb] = wf[q][nb];
+          for (int nb = 0; nb < NB; ++nb) wc[q][nb] = wf[q][nb];
+      }
       // (the last iteration fetches its own data again: nobody reads it)
       gather(raw, gv);
       load_om(min(i + 2, i1 - 1), raw);
+      if constexpr (kSplit) {
 #pragma unroll
-      for (int q = 0; q < CQ; ++q)
+        for (int q = 0; q < CQ / 2; ++q) {
+          uint2 lo[3], hi[3];
+          const uint4 &u = x[2 * q], &v = x[2 * q + 1];
+          split3({__uint_as_float(u.x), __uint_as_float(u.y), __uint_as_float(u.z), __uint_as_float(u.w)}, lo);
+          split3({__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w)}, hi);
+          auto products = [&](int xp, int wpl) {
+            const uint4 xv = make_uint4(lo[xp].x, lo[xp].y, hi[xp].x, hi[xp].y);
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) TR::mma(acc[nb], wc[q][nb], x[q]);
+            for (int nb = 0; nb < NB; ++nb) ElemTraits<bf16_t>::mma(acc[nb], wf[3 * q + wpl][nb], xv);
+          };
+          products(2, 0);  // smallest terms first
+          products(0, 2);
+          products(1, 1);
+          products(1, 0);
+          products(0, 1);
+          products(0, 0);
+        }
+      } else {
+#pragma unroll
+        for (int q = 0; q < CQ; ++q)
+#pragma unroll
+          for (int nb = 0; nb < NB; ++nb) TR::mma(acc[nb], wc[q][nb], x[q]);
+      }
+      if constexpr (kSplit) __builtin_amdgcn_sched_barrier(0);
       load_w(min(i + 1, i1 - 1), wf);
     }
   }
@@ -279,8 +332,10 @@ hipError_t launch_nb(const SegArgs &a, hipStream_t st) {
   switch (a.s.nb) {
     case 1: return launch<E, 1, CQ>(a, st);
     case 2: return launch<E, 2, CQ>(a, st);
-    case 3: return launch<E, 3, CQ>(a, st);
     default: break;
+  }
+  if constexpr (!(seg_split((int)sizeof(E), CQ) && CQ == 4)) {
+    if (a.s.nb == 3) return launch<E, 3, CQ>(a, st);
   }
   if constexpr (CQ <= 2) {
     if (a.s.nb == 4) return launch<E, 4, CQ>(a, st);
@@ -331,7 +386,7 @@ bool seg_plan(const Geom &g, int es, int n_images, bool may_share, int cus, SegP
   double best = 0.0;
   s->cq = 0;
   for (int cq = 4; cq >= 1; cq /= 2) {
-    if (cq * s->nb > kSegFragsMax) continue;
+    if (cq * s->nb > kSegFragsMax || (es == 4 && cq == 4 && s->nb == 3)) continue;  // (18 fragments, split)
     const int groups = (cps0 + cq - 1) / cq;
     const double cost = groups * 1.5 + groups * cq;
     if (s->cq == 0 || cost < best) best = cost, s->cq = cq;
@@ -345,7 +400,7 @@ bool seg_plan(const Geom &g, int es, int n_images, bool may_share, int cus, SegP
   const uint64_t img = (uint64_t)g.G * s->nseg_g * s->cps * g.Hp * g.Wp * 16;
   if (img * (uint64_t)n_images > 0xF0000000ull) return false;
   s->xt_bytes = (size_t)(img * (uint64_t)n_images);
-  s->wp_bytes = (size_t)g.G * s->n_ctiles * s->iters * s->cq * s->nb * 1024;
+  s->wp_bytes = (size_t)g.G * s->n_ctiles * s->iters * seg_frags(es, s->cq) * s->nb * 1024;
   // Waves of a workgroup share a pixel block's K range while that leaves the chip's SIMDs short of two waves.
   const long waves = ((long)n_images * g.Ho * g.Wo + 31) / 32 * s->n_ctiles * g.G;
   s->kshare = 1;
