@@ -103,6 +103,44 @@ __device__ __forceinline__ void pack_weight_split(const Geom &g, const float *__
                                                   uint32_t *__restrict__ zero_ptr, int zero_n) {
   for (long i = first; i < zero_n; i += stride) zero_ptr[i] = 0u;
   const int nk = slabs * g.taps, blocks = CT / 32;
+  if (g.taps == 9 && (uintptr_t)w % 16 == 0) {  // 3x3: a lane's eight channels are 288 contiguous, aligned bytes
+    const long units = (long)g.G * n_ctiles * slabs * 2 * blocks * 64;
+    for (long idx = first; idx < units; idx += stride) {
+      long r = idx;
+      const int lane = (int)(r & 63);
+      r >>= 6;
+      const int blk = (int)(r % blocks);
+      r /= blocks;
+      const int half = (int)(r & 1);
+      r >>= 1;
+      const int slab = (int)(r % slabs);
+      r /= slabs;  // (group, tile)
+      const int ctile = (int)(r % n_ctiles), grp = (int)(r / n_ctiles);
+      const int col = ctile * CT + blk * 32 + (lane & 31);
+      const int c0 = slab * 32 + half * 16 + (lane >> 5) * 8;
+      float v[72];
+      const uint4 *src = (const uint4 *)(w + ((long)(grp * g.cout_g + min(col, g.cout_g - 1)) * g.cin_g + c0) * 9);
+#pragma unroll
+      for (int i = 0; i < 18; ++i) {
+        const uint4 q = src[i];
+        __builtin_memcpy(v + 4 * i, &q, 16);
+      }
+      if (col >= g.cout_g) {
+#pragma unroll
+        for (int i = 0; i < 72; ++i) v[i] = 0.0f;
+      }
+#pragma unroll
+      for (int tap = 0; tap < 9; ++tap) {
+        uint2 p0[3], p1[3];
+        split3({v[tap], v[9 + tap], v[18 + tap], v[27 + tap]}, p0);
+        split3({v[36 + tap], v[45 + tap], v[54 + tap], v[63 + tap]}, p1);
+        uint4 *dst = (uint4 *)wp + (((r * nk + slab * 9 + tap) * 2 + half) * 3 * blocks + blk) * 64 + lane;
+#pragma unroll
+        for (int s = 0; s < 3; ++s) dst[(long)s * blocks * 64] = make_uint4(p0[s].x, p0[s].y, p1[s].x, p1[s].y);
+      }
+    }
+    return;
+  }
   const long total = (long)g.G * n_ctiles * nk * 2 * blocks * 64;
   for (long idx = first; idx < total; idx += stride) {
     long r = idx;

@@ -69,3 +69,19 @@ def test_narrow_tiles_and_many_parts(kw, dtype):
     for _ in range(3):
         assert torch.equal(capi_forward(dev), y)
     assert rel_err(capi_forward(dev, unsplit=True).float().cpu().numpy(), ref) <= TOL[dtype]
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16, torch.float16], ids=['f32', 'bf16', 'f16'])
+@pytest.mark.parametrize('kw', [dict(N=1, Cin=128, Cout=72, H=9, W=11), dict(N=1, Cin=128, Cout=264, H=8, W=9),
+                                dict(N=1, Cin=256, Cout=70, H=7, W=9, groups=2)],
+                         ids=['tail', 'two_tiles', 'groups'])
+def test_weights_that_start_anywhere(kw, dtype):
+    """3x3 weights are repacked nine taps at a time where they start 16-byte aligned, one by one elsewhere."""
+    dev = cast_case(make_case(45, **kw), dtype, 'cuda')
+    y = capi_forward(dev, path=capi.PATH_FUSED)
+    flat = torch.empty(dev['weight'].numel() + 1, dtype=dtype, device='cuda')
+    flat[1:] = dev['weight'].flatten()
+    shifted = dict(dev, weight=flat[1:].view(dev['weight'].shape))
+    assert shifted['weight'].data_ptr() % 16 != 0 and dev['weight'].data_ptr() % 16 == 0
+    assert torch.equal(capi_forward(shifted, path=capi.PATH_FUSED), y)
+    assert rel_err(y.float().cpu().numpy(), oracle_forward(cast_case(make_case(45, **kw), dtype))) <= TOL[dtype]
