@@ -134,7 +134,8 @@ bool fused_ok(const mdcn_params *p, const Geom &g) {
 }
 
 // Length of the fp32 kernel's persistent schedule of `tiles` tiles of nk K steps in tile times, as UnitSchedule lays
-// it out: whole rounds, then the last round's tiles whole or cut into parts.
+// it out: whole rounds, then the last round's tiles whole or cut into parts.  (More than four parts count as four: with the sum of all of them they take no less.  N=1 256
+// channels 50x84, six parts of 256-channel tiles 84 us a call, three of 128-channel ones 69.)
 double schedule_rounds(long tiles, int nk, bool may_cut) {
   const int stride = std::max(1, num_cus() / 8);
   const long chunk = (tiles + 7) / 8;  // the fullest XCD
@@ -142,7 +143,7 @@ double schedule_rounds(long tiles, int nk, bool may_cut) {
   if (rest == 0) return (double)full;
   const int rounds = (nk + kGatherAhead - 1) / kGatherAhead;
   long parts = 1;
-  if (may_cut) parts = std::max<long>(1, std::min<long>(std::min<long>(stride / rest, kF32CutMax), rounds / (8 / kGatherAhead)));
+  if (may_cut) parts = std::max<long>(1, std::min<long>(std::min<long>(stride / rest, 4), rounds / (8 / kGatherAhead)));
   return (double)full + 1.0 / (double)parts;
 }
 

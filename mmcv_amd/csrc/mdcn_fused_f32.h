@@ -103,8 +103,11 @@ __device__ __forceinline__ void pack_weight_split(const Geom &g, const float *__
                                                   uint32_t *__restrict__ zero_ptr, int zero_n) {
   for (long i = first; i < zero_n; i += stride) zero_ptr[i] = 0u;
   const int nk = slabs * g.taps, blocks = CT / 32;
-  if (g.taps == 9 && (uintptr_t)w % 16 == 0) {  // 3x3: a lane's eight channels are 288 contiguous, aligned bytes
-    const long units = (long)g.G * n_ctiles * slabs * 2 * blocks * 64;
+  // 3x3: a lane's eight channels are 288 contiguous, aligned bytes, nine taps at a time.  From 512 -> 512 channels on (whole
+  // call, us, one by one / nine: N=1 512 channels 13x13 59.5 / 54.8): with fewer lanes to do it the nine splits of each are the
+  // longer chain (128 channels 28x28 29.4 / 31.2, 256 channels 28x28 42.9 / 44.9).
+  const long units = (long)g.G * n_ctiles * slabs * 2 * blocks * 64;
+  if (g.taps == 9 && (uintptr_t)w % 16 == 0 && units >= 32768) {
     for (long idx = first; idx < units; idx += stride) {
       long r = idx;
       const int lane = (int)(r & 63);
