@@ -676,7 +676,9 @@ __device__ __forceinline__ void scatter_tile(const BwdScatterArgs &a, const Scat
     }
     if constexpr (DATA) {
       __syncthreads();  // every add into the window has landed
-      // (padding channels only ever receive zeros, and zeros are not written)
+      // (Padding channels have no plane of their own: d is zero there, but NaN where grad_output is not finite, and what
+      // follows is another segment, the next image, or the end of the tensor.)
+      const int room = ps.room;
       float *gplane = a.gin32 + ((long)n * g.Cin + cs) * plane_in;
 #pragma unroll
       for (int j = 0; j < kSlots; ++j) {
@@ -692,8 +694,8 @@ __device__ __forceinline__ void scatter_tile(const BwdScatterArgs &a, const Scat
                 w64[cp * win_px] = 0;
                 const int lo = (int)(unsigned)(unsigned long long)e;
                 const int hi = (int)((e - (long long)lo) >> 32);
-                if (lo != 0) unsafeAtomicAdd(gi + (long)(2 * cp) * plane_in, (float)lo * fx_inv);
-                if (hi != 0) unsafeAtomicAdd(gi + (long)(2 * cp + 1) * plane_in, (float)hi * fx_inv);
+                if (lo != 0 && 2 * cp < room) unsafeAtomicAdd(gi + (long)(2 * cp) * plane_in, (float)lo * fx_inv);
+                if (hi != 0 && 2 * cp + 1 < room) unsafeAtomicAdd(gi + (long)(2 * cp + 1) * plane_in, (float)hi * fx_inv);
               }
             }
           } else {
@@ -702,7 +704,7 @@ __device__ __forceinline__ void scatter_tile(const BwdScatterArgs &a, const Scat
               const WT v = win[cc * win_px + q];
               if (v != (WT)0) {
                 win[cc * win_px + q] = (WT)0;
-                unsafeAtomicAdd(gi + (long)cc * plane_in, (float)v);
+                if (cc < room) unsafeAtomicAdd(gi + (long)cc * plane_in, (float)v);
               }
             }
           }

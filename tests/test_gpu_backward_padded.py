@@ -57,3 +57,19 @@ def test_padded_backward(name, kw, dtype):
         lib.mdcn_set_pass_limits(0, 0)
     for nm, r, o in zip(NAMES, ref, got):
         assert rel_err(o.float().cpu().numpy(), r) <= TOL[dtype], nm
+
+
+def test_padding_channels_have_no_gradient():
+    """An infinity of grad_output leaves NaN in the column gradient of the padding channels (zero weights times
+    infinity): what follows a segment's planes in grad_input -- here the other image's -- has none of it."""
+    print('padding, not finite', flush=True)
+    case = make_case(52, N=2, Cin=6, Cout=10, H=9, W=11, sigma=0.5)
+    gy = torch.randn(2, 10, 9, 11, generator=torch.Generator().manual_seed(4))
+    gy[0, 3, 4, 5] = float('inf')
+    dev, gyd = cast_case(case, torch.float32, 'cuda'), gy.cuda()
+    got, ref = capi_backward(dev, gyd), capi_backward(dev, gyd, path=capi.PATH_DIRECT)
+    assert not bool(ref[0][0].isfinite().all()) and bool(ref[0][1].isfinite().all())
+    for nm, a, b in zip(NAMES[:3], got, ref):
+        assert torch.equal(a.isfinite(), b.isfinite()), nm
+        ok = b.isfinite()
+        assert float((a[ok] - b[ok]).abs().max() / b[ok].abs().max()) <= TOL[torch.float32], nm
