@@ -634,7 +634,9 @@ __device__ __forceinline__ void scatter_tile(const BwdScatterArgs &a, const Scat
             } else {
 #pragma unroll
               for (int h = 0; h < 2; ++h) {
-                const float t = d[h] * m;
+                // (a lane with nothing for the window adds zeros to an entry that may be somebody's: also where its own
+                // d is infinite, which a weight of zero would make NaN)
+                const float t = to_win ? d[h] * m : 0.0f;
                 WT *wp = win + (2 * cp + h) * win_px + wbase;
                 atomicAdd(wp, (WT)(s00 * t));
                 atomicAdd(wp + 1, (WT)(s01 * t));

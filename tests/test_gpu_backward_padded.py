@@ -73,3 +73,22 @@ def test_padding_channels_have_no_gradient():
         assert torch.equal(a.isfinite(), b.isfinite()), nm
         ok = b.isfinite()
         assert float((a[ok] - b[ok]).abs().max() / b[ok].abs().max()) <= TOL[torch.float32], nm
+
+
+@pytest.mark.parametrize('cin', [64, 12], ids=['whole', 'padded'])
+def test_far_samples_of_what_is_not_finite(cin):
+    """Samples beyond the scatter kernel's window of a pixel whose grad_output is infinite: their gradient goes to the
+    corners they sample, and NaN to nobody else's."""
+    print('far, not finite', flush=True)
+    case = make_case(53, N=1, Cin=cin, Cout=16, H=32, W=96, sigma=0.5)
+    # one output pixel samples 40 columns to the right of itself: beyond the margin of either window
+    case['offset'][0, 1::2, 20, 20] += 40.0
+    gy = torch.randn(1, 16, 32, 96, generator=torch.Generator().manual_seed(5))
+    gy[0, 3, 20, 20] = float('inf')
+    dev, gyd = cast_case(case, torch.float32, 'cuda'), gy.cuda()
+    got, ref = capi_backward(dev, gyd), capi_backward(dev, gyd, path=capi.PATH_DIRECT)
+    assert not bool(ref[0].isfinite().all()) and bool(ref[0][..., :40].isfinite().all())
+    for nm, a, b in zip(NAMES[:3], got, ref):
+        assert torch.equal(a.isfinite(), b.isfinite()), nm
+        ok = b.isfinite()
+        assert float((a[ok] - b[ok]).abs().max() / b[ok].abs().max()) <= TOL[torch.float32], nm
