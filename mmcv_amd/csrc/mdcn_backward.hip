@@ -279,7 +279,7 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
   float *gin32 = staged ? gin_staging : (float *)bp->grad_input;
   float *bpart = (float *)take(pl.gb_bytes);
   uint32_t *dmax = (uint32_t *)take(pl.mx_bytes);
-  float *mmax = (float *)dmax + kAlign / 4;
+  uint32_t *mmax = dmax + kAlign / 4;
   uint32_t *far = dmax + 2 * kAlign / 4;
   unsigned char *xt = take(pl.xt_bytes), *gT = take(pl.gt_bytes), *wT = take(pl.wt_bytes);
   unsigned char *D = take(pl.d_bytes), *col = take(pl.col_bytes);

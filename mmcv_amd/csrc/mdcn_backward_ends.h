@@ -28,7 +28,7 @@ struct BwdPreArgs {
   long col_rows;           // rows of col whose padding is cleared
   int M_pad;
   uint32_t *dmax;          // cleared
-  float *mmax;             // one value per block of the mask job
+  uint32_t *mmax;          // one value per block of the mask job, the bit pattern of a float >= 0
   long n_mask;
   const void *off;
   long n_off, off_step;    // one offset in off_step is looked at
@@ -123,26 +123,30 @@ __global__ __launch_bounds__(256) void bwd_prepass_kernel(BwdPreArgs a) {
     return;
   }
   __shared__ float red[4];
-  if (b < a.end[kPreMask]) {  // largest |mask|, a share per block
+  if (b < a.end[kPreMask]) {  // largest |mask|, a share per block (as bits, so that infinity and NaN are the largest)
     const int nb = a.end[kPreMask] - a.end[kPreWeight], bi = b - a.end[kPreWeight];
     if (bi == 0 && tid == 0) *a.dmax = 0u;
     const E *x = (const E *)a.mask;
-    float mx = 0.0f;
+    uint32_t mx = 0u;
+    auto raise = [&](E v) { mx = max(mx, __float_as_uint(to_f32(v)) & 0x7fffffffu); };
     if (x) {
       const long nv = ((uintptr_t)x % 16) == 0 ? a.n_mask / EPV : 0;
       for (long v = (long)bi * 256 + tid; v < nv; v += (long)nb * 256) {
         const uint4 q = ((const uint4 *)x)[v];
         const E *e = (const E *)&q;
 #pragma unroll
-        for (int i = 0; i < EPV; ++i) mx = fmaxf(mx, fabsf(to_f32(e[i])));
+        for (int i = 0; i < EPV; ++i) raise(e[i]);
       }
-      for (long i = nv * EPV + (long)bi * 256 + tid; i < a.n_mask; i += (long)nb * 256) mx = fmaxf(mx, fabsf(to_f32(x[i])));
+      for (long i = nv * EPV + (long)bi * 256 + tid; i < a.n_mask; i += (long)nb * 256) raise(x[i]);
     }
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
-    if ((tid & 63) == 0) red[tid >> 6] = mx;
+    for (int o = 32; o > 0; o >>= 1) mx = max(mx, (uint32_t)__shfl_xor((int)mx, o));
+    if ((tid & 63) == 0) red[tid >> 6] = __uint_as_float(mx);
     __syncthreads();
-    if (tid == 0) a.mmax[bi] = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    if (tid == 0) {
+      for (int w = 0; w < 4; ++w) mx = max(mx, __float_as_uint(red[w]));
+      a.mmax[bi] = mx;
+    }
     return;
   }
   if (b < a.end[kPreFar]) {  // offsets that leave the scatter kernel's window, counted in a sample

@@ -52,7 +52,7 @@ struct ColGradArgs {
   int kslabs;      // cout_g / KC
   int n0;          // first image of the pass
   long total;      // workgroups with work: images of the pass x G x px_tiles x m_tiles
-  uint32_t *dmax;  // bit pattern of the largest |d| stored so far (a float >= 0), or null
+  uint32_t *dmax;  // bit pattern of the largest |d| stored so far (a float >= 0, infinite or NaN if one is), or null
 };
 
 // A wave's products of one K step of either kernel: TILE / 64 x 2 blocks of 32 x 32 over 128 bytes of K, operand tiles
@@ -227,19 +227,21 @@ __global__ __launch_bounds__(TILE * 2, TILE == 128 ? 2 : 1) void bwd_colgrad_ker
   // register r of lane l: A row (r/4)*8 + (l/32)*4 + r%4 of the block, B row l%32
   E *D = (E *)a.D;
   const int chunks = a.Cin / 16;
-  if (a.dmax) {  // (every accumulator counts: rows and pixels past the end repeat real ones or are zero)
-    float mx = 0.0f;
+  if (a.dmax) {  // (every accumulator counts: rows and pixels past the end repeat real ones, or are zero times real ones)
+    // Non-negative floats order like their bits, and infinity and NaN lie above all others.  The largest d is the one that is
+    // stored: in fp16 it may have become infinite.
+    uint32_t mx = 0u;
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
       for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, fabsf(acc[mb][nb][r]));
+        for (int r = 0; r < 16; ++r) mx = max(mx, __float_as_uint(acc[mb][nb][r]) & 0x7fffffffu);
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
-    // (non-negative floats order like their bits; the plain read first keeps all but the few
-    // waves that raise the maximum from queueing on one address)
-    if (lane == 0 && __float_as_uint(mx) > __builtin_nontemporal_load(a.dmax)) atomicMax(a.dmax, __float_as_uint(mx));
+    for (int o = 32; o > 0; o >>= 1) mx = max(mx, (uint32_t)__shfl_xor((int)mx, o));
+    mx = __float_as_uint(to_f32(from_f32<E>(__uint_as_float(mx)))) & 0x7fffffffu;
+    // (the plain read first keeps all but the few waves that raise the maximum from queueing on one address)
+    if (lane == 0 && mx > __builtin_nontemporal_load(a.dmax)) atomicMax(a.dmax, mx);
   }
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb) {
@@ -383,9 +385,9 @@ struct BwdScatterArgs {
   int parts;
   float *poff, *pmask;
   long off_total, mask_total;  // elements of grad_offset / grad_mask
-  // fixed-point window (16-bit tensors): largest |d|, and n_mmax values whose largest is that of |mask| (null: 1)
-  const uint32_t *dmax;
-  const float *mmax;
+  // fixed-point window (16-bit tensors): largest |d|, and n_mmax values whose largest is that of |mask| (null: 1),
+  // as bit patterns
+  const uint32_t *dmax, *mmax;
   int n_mmax;
 };
 
@@ -403,7 +405,8 @@ struct BwdScatterArgs {
 // odd channel's shifted up by 32 bits; the low half's borrows and carries into
 // the high half cancel when the entry is taken apart again (low = the entry's low
 // word as a signed number, high = (entry - low) >> 32), since neither sum leaves
-// 32 bits.
+// 32 bits.  Where d or the mask is not finite, or so small or large that no scale fits, nothing goes through the
+// window: every corner takes the way of those beyond it, an fp32 add to memory.
 // DATA: the gradient part (a.D, window, offset / mask sums).  COL: the kernel
 // stores the forward's columns (mask * bilinear sample, rounded to E as the
 // reference's columns tensor is) to a.col for the weight-gradient product.  At
@@ -418,18 +421,20 @@ __device__ __forceinline__ void scatter_tile(const BwdScatterArgs &a, const Scat
   static_assert(kScTH * kScTW == 256, "one thread per pixel of the tile");
   static_assert(kScTH * kScTW * kBwdTapsMax <= kScMaxAdds, "bound on the adds per window entry");
   float fx_scale = 1.0f, fx_inv = 1.0f;
+  bool fits = true;  // the window can be used
   if (kFixed && DATA) {
-    float mm = 1.0f;
+    uint32_t mb = 0x3f800000u;
     if (a.mmax) {
-      mm = (int)(threadIdx.x & 63) < a.n_mmax ? a.mmax[threadIdx.x & 63] : 0.0f;
+      mb = (int)(threadIdx.x & 63) < a.n_mmax ? a.mmax[threadIdx.x & 63] : 0u;
 #pragma unroll
-      for (int o = 32; o > 0; o >>= 1) mm = fmaxf(mm, __shfl_xor(mm, o));
+      for (int o = 32; o > 0; o >>= 1) mb = max(mb, (uint32_t)__shfl_xor((int)mb, o));
     }
-    const float bound = __uint_as_float(*a.dmax) * mm * (float)kScMaxAdds;
+    const float mm = __uint_as_float(mb), bound = __uint_as_float(*a.dmax) * mm * (float)kScMaxAdds;
     // largest power of two not above 2^30 / bound (any scale will do when everything is zero)
     const int e = (bound > 0.0f && bound < 3.0e38f) ? 29 - ilogbf(bound) : 0;
-    fx_scale = ldexpf(1.0f, max(-120, min(120, e)));
+    fx_scale = ldexpf(1.0f, min(120, e));
     fx_inv = 1.0f / fx_scale;
+    fits = bound < 3.0e38f && e <= 120 && mm * fx_scale < 3.0e38f;  // (false for NaN)
   }
   const Geom &g = a.g;
   const long plane_out = (long)g.Ho * g.Wo;
@@ -582,7 +587,7 @@ __device__ __forceinline__ void scatter_tile(const BwdScatterArgs &a, const Scat
           for (int i = 0; i < VecCh<E, CH>::NW; ++i) rd.raw[i] &= keep;
         }
         const int ry = y0 - wy0, rx = x0 - wx0;
-        const bool in_win = ry >= 0 && ry + 1 < wd.WH && rx >= 0 && rx + 1 < wd.WW;
+        const bool in_win = fits && ry >= 0 && ry + 1 < wd.WH && rx >= 0 && rx + 1 < wd.WW;
         const bool to_win = inside && in_win;
         // window is [channel][WH][WW]: neighbouring pixels, neighbouring banks; a lane with nothing
         // for the window adds its zeros at an entry of its own
@@ -684,7 +689,7 @@ __device__ __forceinline__ void scatter_tile(const BwdScatterArgs &a, const Scat
       float *gplane = a.gin32 + ((long)n * g.Cin + cs) * plane_in;
 #pragma unroll
       for (int j = 0; j < kSlots; ++j) {
-        if (flush_at[j] >= 0) {
+        if (fits && flush_at[j] >= 0) {  // (what is in a window that is not used is nobody's)
           const int q = tid + 256 * j;
           float *gi = gplane + flush_at[j];
           if constexpr (kFixed) {
