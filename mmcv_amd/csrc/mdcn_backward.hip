@@ -36,7 +36,7 @@ void make_bwd_plan(const mdcn_bwd_params *bp, const Geom &g, uint64_t pass_bytes
   pl->gw_bytes = (staged && bp->grad_weight) ? align_up((size_t)g.Cout * g.cin_g * g.taps * 4) : 0;
   pl->gb_bytes = (staged && bp->grad_bias) ? align_up((size_t)g.Cout * 4) : 0;
   pl->mx_bytes = 0;
-  pl->tiled = pl->gemm = pl->wgemm = false;
+  pl->tiled = pl->gemm = pl->wgemm = pl->fixed = false;
   pl->xt_bytes = pl->gt_bytes = pl->wt_bytes = pl->d_bytes = pl->col_bytes = pl->part_bytes = pl->wpart_bytes = 0;
   pl->w_tile = kCgTile;
   pl->w_splits = 1;
@@ -58,10 +58,17 @@ void make_bwd_plan(const mdcn_bwd_params *bp, const Geom &g, uint64_t pass_bytes
 
   // Matrix-core paths, for every channel count (padded in the copies) and any number of tiles: a call of 42
   // tiles (fp32, N=2, 256 channels, 50x84) takes 0.41 ms here and took 2.57 ms with a workgroup per tap, one
-  // whose channels fill nothing (bf16, N=4, 96 -> 72, 37x53) 0.12 ms instead of 0.90.  Channels per pass over the window: 16 / 8 of 32-bit fixed point (16-bit tensors),
-  // 8 / 4 doubles (fp32)
+  // whose channels fill nothing (bf16, N=4, 96 -> 72, 37x53) 0.12 ms instead of 0.90.
   const int KC = (int)(128 / es);
-  const int ch_big = es == 2 ? 16 : 8;
+  const long s_tiles = (long)g.N * g.DG * ((g.Ho + kScTH - 1) / kScTH) * ((g.Wo + kScTW - 1) / kScTW);
+  // 16-bit tensors hold d in 16 bits and sum grad_input in fixed point where d is what the call's time goes into: channels in
+  // whole 128-byte slabs and 64 or more tiles.  What is smaller keeps both in fp32 or better.  (A call for the weights
+  // alone has neither.)
+  const bool whole = g.Cin % KC == 0 && g.cout_g % KC == 0 && g.cin_g % 32 == 0 && g.ch_per_dg % 8 == 0;
+  pl->fixed = staged && (!bp->grad_input || (whole && (s_tiles >= 64 || forced)));
+  const size_t ds = pl->fixed ? es : 4;  // bytes of an element of d
+  // Channels per pass over the window: 16 / 8 of 32-bit fixed point, or 8 / 4 doubles
+  const int ch_big = pl->fixed ? 16 : 8;
   int u = g.cin_g, v = g.ch_per_dg;
   while (v) {
     const int t = u % v;
@@ -85,7 +92,7 @@ void make_bwd_plan(const mdcn_bwd_params *bp, const Geom &g, uint64_t pass_bytes
     }
   }
   pl->fR = window_margin(g, kScTH, kScTW, (long)kScWindowPx * (2 * ch_big / pl->sCH), &pl->fWH, &pl->fWW, kScFarMargin);
-  if (pl->fR <= pl->sR) pl->fWH = 0;
+  if (pl->fR <= pl->sR || pl->sCH * es < 16) pl->fWH = 0;  // (a pass reads 8 bytes of channels at least)
   ChanMap &im = pl->im, &om = pl->om;
   im.seg = seg;
   im.segp = padded(seg, pl->sCH);
@@ -95,9 +102,8 @@ void make_bwd_plan(const mdcn_bwd_params *bp, const Geom &g, uint64_t pass_bytes
   om.seg = om.cg = g.cout_g;
   om.nseg = 1;
   om.segp = om.cgp = padded(g.cout_g, KC);
-  const long s_tiles = (long)g.N * g.DG * ((g.Ho + kScTH - 1) / kScTH) * ((g.Wo + kScTW - 1) / kScTW);
   const int cin_p = g.G * im.cgp;
-  const size_t d_img = (size_t)g.taps * cin_p * plane_out * es;
+  const size_t d_img = (size_t)g.taps * cin_p * plane_out * ds;
   const bool mfma_ok = pl->sR >= 1 && d_img <= kBwdColGradCap && plane_out <= ((size_t)1 << 30) &&
                        (size_t)g.H * g.W <= ((size_t)1 << 30);  // (plane offsets held in 32 bits)
   if (mfma_ok) {
@@ -299,7 +305,7 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
   // channels a pass cost next to nothing (bf16, N=2 C=256 135x224, margins 5 and 11: sigma 1.0 0.77 ms with either,
   // 2.5 0.87 / 0.86, 4.0 1.63 / 0.94), half of 8 do: fp16, N=7 C=128 118x196 stride 2, margins 3 and 12: sigma
   // 2.0 0.56 / 0.59, 2.5 0.60 / 0.60, 4.0 0.94 / 0.65.
-  const uint32_t far_min = (uint32_t)(off_total / off_step / (pl.sCH * (int)sizeof(E) == 32 ? 32 : 5));
+  const uint32_t far_min = (uint32_t)(off_total / off_step / (pl.sCH * (pl.fixed ? 2 : 4) == 32 ? 32 : 5));
   auto up = [](long n, long per) { return (int)((n + per - 1) / per); };
   {
     BwdPreArgs a;
@@ -341,7 +347,7 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
         gemm ? up(n_in, kPreZeroPerBlock) : 0,
         wgemm && pl.P_pad > plane_out ? up(a.col_rows * (pl.P_pad - plane_out), kPrePadPerBlock) : 0,
         gemm ? up((long)g.G * pl.M_pad * pl.om.cgp, 256) : 0,
-        gemm && staged ? mask_blocks : 0,
+        gemm && pl.fixed ? mask_blocks : 0,
         gemm && pl.fWH ? far_blocks : 0,
         bp->grad_bias ? g.Cout * pl.bsplits : 0,
     };
@@ -370,14 +376,20 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
       ca.Cout = cout_p;
       ca.kslabs = pl.om.cgp / KC;
       ca.n0 = n0;
-      ca.dmax = staged ? dmax : nullptr;
+      ca.dmax = pl.fixed ? dmax : nullptr;
       ca.total = (long)nb * g.G * ca.px_tiles * ca.m_tiles;
-      if (pl.cg_tile == kCgTileBig)
-        hipLaunchKernelGGL((bwd_colgrad_kernel<E, kCgTileBig>), dim3((unsigned)((ca.total + 7) / 8 * 8)),
-                           dim3(2 * kCgTileBig), 0, st, ca);
+      auto launch = [&](auto dt) {
+        using DT = decltype(dt);
+        const dim3 grid((unsigned)((ca.total + 7) / 8 * 8));
+        if (pl.cg_tile == kCgTileBig)
+          hipLaunchKernelGGL((bwd_colgrad_kernel<E, DT, kCgTileBig>), grid, dim3(2 * kCgTileBig), 0, st, ca);
+        else
+          hipLaunchKernelGGL((bwd_colgrad_kernel<E, DT, kCgTile>), grid, dim3(2 * kCgTile), 0, st, ca);
+      };
+      if (pl.fixed)
+        launch(E());
       else
-        hipLaunchKernelGGL((bwd_colgrad_kernel<E, kCgTile>), dim3((unsigned)((ca.total + 7) / 8 * 8)),
-                           dim3(2 * kCgTile), 0, st, ca);
+        launch(0.0f);
       check();
     }
     BwdScatterArgs sa;
@@ -410,25 +422,31 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
     sa.n_mmax = mask_blocks;
     const long sblocks = (long)nb * g.DG * sa.tiles_y * sa.tiles_x;
     {
-      // 16-bit tensors: 32-bit fixed-point window (needs the maxima the data path computes;
-      // a columns-only call adds nothing to the window); fp32 tensors: doubles
-      constexpr bool k16 = sizeof(E) == 2;
-      using WT = typename std::conditional<k16, int32_t, double>::type;
-      constexpr int CHB = k16 ? 16 : 8;
+      // 32-bit fixed-point window (needs the maxima the data path computes; a columns-only call adds nothing to the
+      // window) or doubles
       const dim3 sgrid((unsigned)sblocks, (unsigned)sa.parts);
-      auto launch = [&](auto chv) {
+      auto launch = [&](auto wt, auto chv) {
+        using WT = decltype(wt);
         constexpr int CHS = decltype(chv)::value;
         if (gemm && wgemm)
           hipLaunchKernelGGL((bwd_scatter_kernel<E, CHS, WT, true, true>), sgrid, dim3(256), 0, st, sa);
         else if (gemm)
           hipLaunchKernelGGL((bwd_scatter_kernel<E, CHS, WT, true, false>), sgrid, dim3(256), 0, st, sa);
-        else
+        else if constexpr (sizeof(E) == 4 || sizeof(WT) == 4)  // (16-bit columns alone: always `fixed`)
           hipLaunchKernelGGL((bwd_scatter_kernel<E, CHS, WT, false, true>), sgrid, dim3(256), 0, st, sa);
       };
-      if (pl.sCH == CHB)
-        launch(std::integral_constant<int, CHB>());
-      else
-        launch(std::integral_constant<int, CHB / 2>());
+      if constexpr (sizeof(E) == 2) {
+        if (pl.fixed && pl.sCH == 16)
+          launch(int32_t(), std::integral_constant<int, 16>());
+        else if (pl.fixed)
+          launch(int32_t(), std::integral_constant<int, 8>());
+      }
+      if (!pl.fixed) {
+        if (pl.sCH == 8)
+          launch(double(), std::integral_constant<int, 8>());
+        else
+          launch(double(), std::integral_constant<int, 4>());
+      }
     }
     check();
     if (wgemm) {

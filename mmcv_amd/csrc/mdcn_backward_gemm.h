@@ -44,7 +44,7 @@ struct ColGradArgs {
   // (channel counts are those of the padded orders, see BwdPlan)
   const void *wT;  // [G][M_pad][cout_g]
   const void *gT;  // [N][Cout / KC][P][KC], KC = 128 bytes of channels
-  void *D;         // [images of the pass][Cin / 16][taps][P][16]
+  void *D;         // [images of the pass][Cin / 16][taps][P][16], of the kernel's DT
   int P;           // output pixels per image
   int px_tiles, m_tiles;
   int M, M_pad;    // taps * cin_g and its padded size
@@ -145,8 +145,8 @@ __device__ __forceinline__ bool not_finite(const f32x16 (&acc)[MB][2]) {
 // swizzled by the row number on the source side, so that fragment reads are
 // conflict free), double buffered.  A rows = (tap, channel), B rows = pixels:
 // a lane ends up with 4 x 4 consecutive channels of one pixel, which is what the
-// d layout wants (8- or 16-byte stores).
-template <typename E, int TILE>
+// d layout wants (8- or 16-byte stores).  DT: element of d, E or float.
+template <typename E, typename DT, int TILE>
 __global__ __launch_bounds__(TILE * 2, TILE == 128 ? 2 : 1) void bwd_colgrad_kernel(ColGradArgs a) {
   using TR = ElemTraits<E>;
   constexpr int ES = (int)sizeof(E);
@@ -225,7 +225,7 @@ __global__ __launch_bounds__(TILE * 2, TILE == 128 ? 2 : 1) void bwd_colgrad_ker
   }
 
   // register r of lane l: A row (r/4)*8 + (l/32)*4 + r%4 of the block, B row l%32
-  E *D = (E *)a.D;
+  DT *D = (DT *)a.D;
   const int chunks = a.Cin / 16;
   if (a.dmax) {  // (every accumulator counts: rows and pixels past the end repeat real ones, or are zero times real ones)
     // Non-negative floats order like their bits, and infinity and NaN lie above all others.  The largest d is the one that is
@@ -256,7 +256,7 @@ __global__ __launch_bounds__(TILE * 2, TILE == 128 ? 2 : 1) void bwd_colgrad_ker
       // The two halves of the wave exchange their 4-channel groups so that a lane holds 8 consecutive
       // channels: one 16-byte store per lane and 16 channels, 32 pixels x 32 bytes contiguous per instruction
       // (the lower half takes the first 8 channels of a 16-channel chunk, the upper half the second 8).
-      if constexpr (sizeof(E) == 2) {
+      if constexpr (sizeof(DT) == 2) {
 #pragma unroll
         for (int jp = 0; jp < 2; ++jp) {
           const f32x16 &c16 = acc[mb][nb];
@@ -266,16 +266,16 @@ __global__ __launch_bounds__(TILE * 2, TILE == 128 ? 2 : 1) void bwd_colgrad_ker
           const auto s0 = __builtin_amdgcn_permlane32_swap(a0, b0, false, false);
           const auto s1 = __builtin_amdgcn_permlane32_swap(a1, b1, false, false);
           const int c = cb + jp * 16 + fhalf * 8;
-          E *dst = D + ((((long)nl * chunks + (c >> 4)) * a.taps + tap) * a.P + px) * 16 + (c & 15);
+          DT *dst = D + ((((long)nl * chunks + (c >> 4)) * a.taps + tap) * a.P + px) * 16 + (c & 15);
           *(uint4 *)dst = make_uint4(s0[0], s1[0], s0[1], s1[1]);
         }
       } else {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const int c = cb + j * 8 + fhalf * 4;
-          E *dst = D + ((((long)nl * chunks + (c >> 4)) * a.taps + tap) * a.P + px) * 16 + (c & 15);
-          TR::store4((unsigned char *)dst, acc[mb][nb][4 * j], acc[mb][nb][4 * j + 1],
-                     acc[mb][nb][4 * j + 2], acc[mb][nb][4 * j + 3]);
+          DT *dst = D + ((((long)nl * chunks + (c >> 4)) * a.taps + tap) * a.P + px) * 16 + (c & 15);
+          *(float4 *)dst = make_float4(acc[mb][nb][4 * j], acc[mb][nb][4 * j + 1], acc[mb][nb][4 * j + 2],
+                                       acc[mb][nb][4 * j + 3]);
         }
       }
     }
@@ -328,10 +328,13 @@ struct VecCh {
     }
   }
   // acc + this's channels 2 i and 2 i + 1 times o's
-  __device__ __forceinline__ float dot_pair(const VecCh &o, int i, float acc) const {
-    if constexpr (sizeof(E) == 4) {
-      acc = fmaf(__uint_as_float(raw[2 * i]), __uint_as_float(o.raw[2 * i]), acc);
-      return fmaf(__uint_as_float(raw[2 * i + 1]), __uint_as_float(o.raw[2 * i + 1]), acc);
+  template <typename D>
+  __device__ __forceinline__ float dot_pair(const VecCh<D, CH> &o, int i, float acc) const {
+    if constexpr (sizeof(D) == 4) {
+      float lo, hi;
+      pair(i, lo, hi);
+      acc = fmaf(lo, __uint_as_float(o.raw[2 * i]), acc);
+      return fmaf(hi, __uint_as_float(o.raw[2 * i + 1]), acc);
     } else {
       return ElemTraits<E>::dot2(raw[i], o.raw[i], acc);
     }
@@ -393,8 +396,9 @@ struct BwdScatterArgs {
 
 // The window is not fp32: LDS single-precision atomic adds are slow on this
 // hardware (measured per wavefront instruction per CU: ds_add_f32 170 clocks,
-// ds_add_f64 26, ds_add_u32 11, whatever the addresses).  fp32 tensors use a
-// double-precision window (WT = double).  16-bit tensors use 32-bit fixed point
+// ds_add_f64 26, ds_add_u32 11, whatever the addresses).  fp32 tensors, and 16-bit
+// tensors of few or uneven channels or few tiles (BwdPlan::fixed), use a
+// double-precision window (WT = double) and an fp32 d.  Other 16-bit tensors have a 16-bit d and a window of 32-bit fixed point
 // (WT = int32_t): with B = max|d| * max|mask| bounding every contribution and at
 // most kScMaxAdds contributions per entry, the scale 2^k <= 2^30 / (B * kScMaxAdds)
 // cannot overflow, and one contribution is rounded to B * 2^-19 at worst -- two
@@ -418,6 +422,7 @@ __device__ __forceinline__ void scatter_tile(const BwdScatterArgs &a, const Scat
   static_assert(CH <= RC && RC % CH == 0, "a pass reads a record or a whole fraction of one");
   static_assert(CH % 2 == 0, "fixed-point window entries hold two channels");
   constexpr bool kFixed = sizeof(WT) == 4;
+  using DT = typename std::conditional<kFixed, E, float>::type;  // element of d
   static_assert(kScTH * kScTW == 256, "one thread per pixel of the tile");
   static_assert(kScTH * kScTW * kBwdTapsMax <= kScMaxAdds, "bound on the adds per window entry");
   float fx_scale = 1.0f, fx_inv = 1.0f;
@@ -520,7 +525,8 @@ __device__ __forceinline__ void scatter_tile(const BwdScatterArgs &a, const Scat
     int y0, x0;
     float ly, lx, m;
     bool inside;
-    VecCh<E, CH> r00, r01, r10, r11, rd;
+    VecCh<E, CH> r00, r01, r10, r11;
+    VecCh<DT, CH> rd;
   };
   auto fetch = [&](int c0, int tap, E e_dy, E e_dx, E e_m, Sample &s) {
     const int ti = tap / g.kw, tj = tap - ti * g.kw;
@@ -546,7 +552,7 @@ __device__ __forceinline__ void scatter_tile(const BwdScatterArgs &a, const Scat
     s.r10.load(xp + (long)g.Wp * RC);
     s.r11.load(xp + (long)(g.Wp + 1) * RC);
     if constexpr (DATA)
-      s.rd.load((const E *)a.D + (((long)nl * (a.cin_p / 16) + (c0 >> 4)) * g.taps + tap) * plane_out * 16 + pix * 16 +
+      s.rd.load((const DT *)a.D + (((long)nl * (a.cin_p / 16) + (c0 >> 4)) * g.taps + tap) * plane_out * 16 + pix * 16 +
                 (c0 & 15));
   };
   // A tap's loads are issued one tap ahead, in front of the previous tap's stores and atomics
@@ -580,11 +586,11 @@ __device__ __forceinline__ void scatter_tile(const BwdScatterArgs &a, const Scat
         const bool ok00 = y0 >= 0 && x0 >= 0, ok01 = y0 >= 0 && x1 <= g.W - 1;
         const bool ok10 = y1 <= g.H - 1 && x0 >= 0, ok11 = y1 <= g.H - 1 && x1 <= g.W - 1;
         const float w00 = hy * hx, w01 = hy * lx, w10 = ly * hx, w11 = ly * lx;
-        VecCh<E, CH> &rd = cur.rd;
+        VecCh<DT, CH> &rd = cur.rd;
         if constexpr (DATA) {
           const uint32_t keep = inside ? ~0u : 0u;  // (whatever d holds where nothing is sampled)
 #pragma unroll
-          for (int i = 0; i < VecCh<E, CH>::NW; ++i) rd.raw[i] &= keep;
+          for (int i = 0; i < VecCh<DT, CH>::NW; ++i) rd.raw[i] &= keep;
         }
         const int ry = y0 - wy0, rx = x0 - wx0;
         const bool in_win = fits && ry >= 0 && ry + 1 < wd.WH && rx >= 0 && rx + 1 < wd.WW;

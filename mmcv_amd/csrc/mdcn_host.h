@@ -31,6 +31,7 @@ struct BwdPlan {
   // matrix-core paths (bwd_colgrad_kernel + bwd_scatter_kernel, bwd_wgrad_kernel):
   bool gemm;       // data gradients
   bool wgemm;      // grad_weight from stored columns
+  bool fixed;      // column gradient in 16 bits and a fixed-point window (else fp32 and doubles)
   int sR, sWH, sWW;  // window of the scatter kernel
   int sCH;         // channels per pass over that window
   int fR, fWH, fWW;  // window with half as many channels a pass, for far offsets (fWH = 0: none)
@@ -48,7 +49,7 @@ struct BwdPlan {
   size_t gpad_bytes;     // grad_output with padded rows, when its own rows cannot be copied 16 bytes at a time
   size_t gb_bytes;  // sums of grad_bias
   int bsplits;      // ... shares of a channel's pixels (matrix-core paths)
-  size_t mx_bytes;  // the maxima that scale the fixed-point window (16-bit tensors)
+  size_t mx_bytes;  // the maxima that scale the fixed-point window, the counts of far offsets
   size_t total() const {
     return gin_bytes + gw_bytes + gb_bytes + mx_bytes + xt_bytes + gt_bytes + wt_bytes + d_bytes + col_bytes + part_bytes +
            wpart_bytes + gpad_bytes;

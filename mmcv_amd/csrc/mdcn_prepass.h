@@ -37,7 +37,7 @@ namespace mdcn {
 // time and whose neighbouring lanes read neighbouring pixels (the backward's scatter kernel): four pixels
 // share a cache line there, where the 128-byte records give every lane a line of its own.
 // MAPPED: the copy's channels are those of `cm`, cp of them (a multiple of RC elements for REC = 32, of KC for
-// REC = 128); padding channels are zero.
+// REC = 128), segments padded to a multiple of 4; padding channels are zero.
 template <typename E, bool BORDER, int REC = 128, bool MAPPED = false>
 __device__ __forceinline__ void relayout_vec_block(const Geom &g, const E *__restrict__ in, E *__restrict__ xt,
                                                    int n_pchunks, int b, const ChanMap &cm = ChanMap(), int cp = 0) {
@@ -71,8 +71,21 @@ __device__ __forceinline__ void relayout_vec_block(const Geom &g, const E *__res
   const int np = max(0, min(EPV, plane - p0));  // pixels of the run that exist
   int room = EPV;                               // channels of the thread's EPV that exist
   int c_src = slab * KC + cg * EPV;
-  if constexpr (MAPPED) c_src = c_src < cp ? chan_source(cm, c_src, room) : (room = 0);
-  if (p0 < plane && room > 0) {
+  // MAPPED: the last EPV - 4 of them may be another segment's (c_src4: what they would count from if it were one)
+  int room4 = 0, c_src4 = 0;
+  if constexpr (MAPPED) {
+    const int c = c_src;
+    c_src = c < cp ? chan_source(cm, c, room) : (room = 0);
+    if (EPV > 4 && cm.segp % EPV != 0) {  // (workgroup uniform)
+      c_src4 = c + 4 < cp ? chan_source(cm, c + 4, room4) - 4 : 0;
+      room = min(room, 4);
+      room4 = room4 > 0 ? room4 + 4 : 0;
+    } else {
+      room4 = room;
+      c_src4 = c_src;
+    }
+  }
+  if (p0 < plane && (room > 0 || room4 > 0)) {
     const E *src = in + ((long)n * g.Cin + c_src) * plane + p0;
     uint4 r[EPV];
     if (np == EPV && room >= EPV) {  // (16 bytes at the alignment of an element: one load instruction all the same)
@@ -83,7 +96,14 @@ __device__ __forceinline__ void relayout_vec_block(const Geom &g, const E *__res
       for (int j = 0; j < EPV; ++j) {
         E e[EPV];
 #pragma unroll
-        for (int i = 0; i < EPV; ++i) e[i] = i < np && j < room ? src[(long)j * plane + i] : from_f32<E>(0.0f);
+        for (int i = 0; i < EPV; ++i) e[i] = from_f32<E>(0.0f);
+        const bool second = MAPPED && j >= 4;
+        if (j < (second ? room4 : room)) {
+          const E *s = second ? in + ((long)n * g.Cin + c_src4) * plane + p0 : src;
+#pragma unroll
+          for (int i = 0; i < EPV; ++i)
+            if (i < np) e[i] = s[(long)j * plane + i];
+        }
         __builtin_memcpy(&r[j], e, 16);
       }
     }

@@ -92,3 +92,29 @@ def test_far_samples_of_what_is_not_finite(cin):
         assert torch.equal(a.isfinite(), b.isfinite()), nm
         ok = b.isfinite()
         assert float((a[ok] - b[ok]).abs().max() / b[ok].abs().max()) <= TOL[torch.float32], nm
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16], ids=['bf16', 'f16'])
+@pytest.mark.parametrize('name', ['few_tiles', 'seg4_dg8', 'seg20', 'seg48_dg2', 'gcd', 's2', 'far', 'far_s2', 'one_pixel'])
+def test_small_16bit_gradients_are_rounded_once(name, dtype):
+    """Calls of few tiles or uneven channels keep the column gradient and the sums of grad_input, grad_offset and
+    grad_mask in fp32: every element is the true one, rounded once -- also in an image whose gradients are small."""
+    print(f'case={name} dtype={dtype}', flush=True)
+    kw = dict(CASES).get(name, dict(N=2, Cin=128, Cout=64, H=14, W=30))
+    case = make_case(54, **kw)
+    # quarter pixels, never on one: exact positions, and no jump of the offsets' gradient
+    frac = torch.randint(1, 4, case['offset'].shape, generator=torch.Generator().manual_seed(1)) / 4
+    case['offset'] = torch.floor(case['offset']) + frac
+    gy = torch.randn(kw['N'], kw['Cout'], *case['offset'].shape[2:], generator=torch.Generator().manual_seed(6))
+    gy[0] *= 1e-3
+    dev, gyd = cast_case(case, dtype, 'cuda'), gy.to(dtype).cuda()
+    got = capi_backward(dev, gyd)
+    wide = {k: v.double() if torch.is_tensor(v) else v for k, v in dev.items()}
+    ref = capi_backward(wide, gyd.double())
+    half_ulp, tiny = (2.0 ** -8, 0.0) if dtype == torch.bfloat16 else (2.0 ** -11, 2.0 ** -25)
+    for nm, a, b in zip(NAMES[:3], got, ref):
+        for n in range(kw['N']):
+            # (sums of cout and then up to 9 cin fp32 products: 2^-24 each of terms no larger than the image's largest sum)
+            bound = b[n].abs() * half_ulp + tiny + (kw['Cout'] + 9 * kw['Cin']) * 2.0 ** -24 * b[n].abs().max()
+            worst = float(((a[n].double() - b[n]).abs() / bound).max())
+            assert worst <= 1.0, (nm, n, worst)
