@@ -79,8 +79,9 @@ void make_bwd_plan(const mdcn_bwd_params *bp, const Geom &g, uint64_t pass_bytes
   auto padded = [](int n, int to) { return (n + to - 1) / to * to; };
   pl->sCH = ch_big;
   pl->sR = window_margin(g, kScTH, kScTW, kScWindowPx, &pl->sWH, &pl->sWW);
-  // fewer channels at a time buy a wider window, and less padding where segments are short
-  const bool pads_less = 4 * padded(seg, ch_big) > 5 * padded(seg, ch_big / 2);
+  // fewer channels at a time buy a wider window, and less padding where segments are short (none in a fixed-point window,
+  // whose flush does not look where a segment ends)
+  const bool pads_less = pl->fixed && whole ? seg % ch_big != 0 : 4 * padded(seg, ch_big) > 5 * padded(seg, ch_big / 2);
   if (pl->sR < 2 || pads_less) {
     int wh, ww;
     const int r = window_margin(g, kScTH, kScTW, 2 * kScWindowPx, &wh, &ww);
