@@ -462,6 +462,8 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
       wa.nb = nb;
       wa.n0 = n0;
       wa.M = g.taps * pl.im.cgp;
+      wa.cgp = pl.im.cgp;
+      wa.rows = pl.im.nseg * pl.im.segp;
       wa.accumulate = n0 > 0;
       wa.cout_g = g.cout_g;
       wa.taps = g.taps;

@@ -796,6 +796,7 @@ struct WGradArgs {
   int ksteps;        // P_pad / (pixels per 128 bytes)
   int nb, n0;        // images of the pass, first image
   int M;             // taps * padded channels of a group
+  int cgp, rows;     // padded channels of a group, and how many of them have rows in col: its segments'
   int cout_g, taps, G, Cin, Cout;   // (Cin: padded)
   int co_tiles, m_tiles;
   int splits;        // workgroups sharing the (image, K step) range of one tile
@@ -813,7 +814,7 @@ struct WGradArgs {
 // 16 bytes again; the zero padding of col cancels them.  Rows past the group's
 // channels repeat its last row and are dropped at the end.  Each share of the K
 // range stores its partial tile (plain stores, rows of M contiguous);
-// wgrad_reduce_kernel adds the shares up in a fixed order, so grad_weight does
+// bwd_finish_kernel adds the shares up in a fixed order, so grad_weight does
 // not vary from run to run.
 template <typename E, int TILE>
 __global__ __launch_bounds__(TILE * 2, TILE == 128 ? 2 : 1) void bwd_wgrad_kernel(WGradArgs a) {
@@ -845,7 +846,11 @@ __global__ __launch_bounds__(TILE * 2, TILE == 128 ? 2 : 1) void bwd_wgrad_kerne
     const int row = (wave * 4 + c) * 8 + (lane >> 3);
     chunk[c] = (lane & 7) ^ (row & 7);
     const int co = min(ct * TILE + row, a.cout_g - 1);
-    const int m = min(mt * TILE + row, a.M - 1);
+    // (the rows of the channels that only fill up a group are never written: they would hold what was there before, NaN
+    // for instance, and an fp32 call then goes over its K range a second time)
+    int m = min(mt * TILE + row, a.M - 1);
+    const int tap = m / a.cgp;
+    m = min(m, tap * a.cgp + a.rows - 1);
     a_row[c] = ((long)grp * a.cout_g + co) * a.a_pitch;      // + n * Cout * a_pitch
     b_row[c] = ((long)grp * a.M + m) * a.P_pad;              // + nl * taps * Cin * P_pad
   }

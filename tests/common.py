@@ -216,7 +216,7 @@ def capi_pack_forward(case, own_conv=True, raw=None, want_raw=False, path=capi.P
     return out, raw_out
 
 
-def capi_backward(case, grad_output, want_bias=True, path=0, want_data=True, want_weight=True):
+def capi_backward(case, grad_output, want_bias=True, path=0, want_data=True, want_weight=True, ws_fill=None):
     """mdcn_backward through ctypes on device tensors of `case` (mask None:
     unmodulated); returns (grad_input, grad_offset, grad_mask or None, grad_weight,
     grad_bias or None)."""
@@ -248,6 +248,8 @@ def capi_backward(case, grad_output, want_bias=True, path=0, want_data=True, wan
         bp.grad_bias = g_b.data_ptr()
     ws_bytes = lib.mdcn_backward_workspace_bytes(ctypes.byref(bp))
     ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=x.device)
+    if ws_fill is not None:  # what the workspace holds before the call
+        ws.fill_(ws_fill)
     p.workspace = ws.data_ptr() if ws_bytes else None
     p.workspace_bytes = ws_bytes
     rc = lib.mdcn_backward(ctypes.byref(bp), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))

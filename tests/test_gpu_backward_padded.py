@@ -118,3 +118,16 @@ def test_small_16bit_gradients_are_rounded_once(name, dtype):
             bound = b[n].abs() * half_ulp + tiny + (kw['Cout'] + 9 * kw['Cin']) * 2.0 ** -24 * b[n].abs().max()
             worst = float(((a[n].double() - b[n]).abs() / bound).max())
             assert worst <= 1.0, (nm, n, worst)
+
+
+@pytest.mark.parametrize('cin,groups', [(40, 1), (24, 2), (6, 1)])
+def test_stale_workspace(cin, groups):
+    """Nothing depends on what the workspace held: not the results, and not the way they are computed either (fp32 sums
+    that meet a NaN are computed again with other roundings)."""
+    print(f'cin={cin} groups={groups}', flush=True)
+    dev = cast_case(make_case(55, N=2, Cin=cin, Cout=20, H=13, W=18, groups=groups), torch.float32, 'cuda')
+    gy = torch.randn(2, 20, 13, 18, generator=torch.Generator().manual_seed(8)).cuda()
+    zeros, nans = capi_backward(dev, gy, ws_fill=0), capi_backward(dev, gy, ws_fill=255)
+    assert torch.equal(zeros[3], nans[3]) and bool(nans[3].isfinite().all())
+    for a, b in zip(zeros[1:3], nans[1:3]):
+        assert torch.equal(a, b)
