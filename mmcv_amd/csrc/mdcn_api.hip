@@ -561,8 +561,9 @@ int run_typed(const mdcn_params *p, const Geom &g, const Plan &pl, hipStream_t s
         const long tile_px = 32 * (4 / pl.sp.kshare);
         sa.n_work = (sa.total_px + tile_px - 1) / tile_px * pl.sp.n_ctiles * g.G;
         tic();
-        if (seg_prepass(p->dtype, sa, (const E *)p->input + (size_t)n0 * g.Cin * g.H * g.W, n0 ? nullptr : p->weight,
-                        st) != hipSuccess)
+        sa.in = (const E *)p->input + (size_t)n0 * g.Cin * g.H * g.W;
+        sa.weight = p->weight;
+        if (seg_prepass(p->dtype, sa, n0 == 0, st) != hipSuccess)
           rc = MDCN_ERR_LAUNCH;
         toc(0);
         tic();
@@ -640,6 +641,10 @@ int run_typed(const mdcn_params *p, const Geom &g, const Plan &pl, hipStream_t s
       fa.g = gc;
       fa.xt = nhwc ? (const void *)in : (const void *)xt;
       fa.wp = wp;
+      fa.in = in;
+      fa.weight = p->weight;
+      fa.in_c = nhwc ? 1 : (long)g.H * g.W;
+      fa.in_px = nhwc ? g.Cin : 1;
       if (nhwc) {
         fa.px_bytes = (uint32_t)(g.Cin * es);
         fa.row_bytes = (uint32_t)g.W * fa.px_bytes;

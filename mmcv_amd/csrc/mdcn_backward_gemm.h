@@ -92,9 +92,8 @@ __device__ __forceinline__ void tile_products(f32x16 (&acc)[TILE / 64][2], const
     // 8 values of K as three planes of an operand
     auto split8 = [](const uint4 (&v)[2], uint4 (&p)[3]) {
       uint2 lo[3], hi[3];
-      float r[4];
-      split3_finite({__uint_as_float(v[0].x), __uint_as_float(v[0].y), __uint_as_float(v[0].z), __uint_as_float(v[0].w)}, r, lo);
-      split3_finite({__uint_as_float(v[1].x), __uint_as_float(v[1].y), __uint_as_float(v[1].z), __uint_as_float(v[1].w)}, r, hi);
+      split3({__uint_as_float(v[0].x), __uint_as_float(v[0].y), __uint_as_float(v[0].z), __uint_as_float(v[0].w)}, lo);
+      split3({__uint_as_float(v[1].x), __uint_as_float(v[1].y), __uint_as_float(v[1].z), __uint_as_float(v[1].w)}, hi);
 #pragma unroll
       for (int s = 0; s < 3; ++s) p[s] = make_uint4(lo[s].x, lo[s].y, hi[s].x, hi[s].y);
     };

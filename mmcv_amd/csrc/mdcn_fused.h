@@ -83,6 +83,11 @@ struct FusedArgs {
   int cut_max;
   void *cut_part;
   void *cut_cnt;
+  // fused_f32_kernel only: the call's own tensors, for outputs that are made again one by one (channels of `in` in_c
+  // elements apart, pixels in_px)
+  const void *in, *weight;
+  long in_c;
+  int in_px;
   // fused2_kernel only: first pixel of its tiles (a multiple of 256; the pixels in front of it belong to
   // fused3_kernel, which is launched beside it); n_ptiles counts the tiles from there on
   int px0;

@@ -28,6 +28,7 @@
 // two gather sets (209).
 #pragma once
 
+#include "mdcn_direct.h"
 #include "mdcn_fused.h"
 
 namespace mdcn {
@@ -45,28 +46,11 @@ constexpr size_t fused_f32_lds_bytes(int tmax) {
   return (size_t)kF32Tiles * kPT * 192 + (size_t)kPT * tmax * 20 + 16;
 }
 
-// Half `half` of the words h, m, l for an x whose first plane cannot be a rounded one.  Infinity and NaN go to
-// the last plane alone: of the products that are summed it meets the other operand's first plane only, which has that
-// operand's sign and is zero when it is, so that the result is what an fp32 product gives.  (In the first plane it would
-// meet the lower planes too, zeros and numbers of the other sign among them.)  Finite: a first plane that is cut off.
-__device__ __forceinline__ void split3_not_rounded(float x, int half, uint32_t &h, uint32_t &m, uint32_t &l) {
-  const uint32_t b = __float_as_uint(x);
-  uint32_t hb = 0u, mb = 0u, lb = (b >> 16) | ((b & 0x7fffffu) ? 0x40u : 0u);
-  if ((b & 0x7f800000u) != 0x7f800000u) {
-    hb = b >> 16;
-    const float r = x - __uint_as_float(b & 0xffff0000u);
-    mb = ElemTraits<bf16_t>::pack2(r, 0.0f) & 0xffffu;
-    lb = ElemTraits<bf16_t>::pack2(r - __uint_as_float(mb << 16), 0.0f) & 0xffffu;
-  }
-  const int sh = half * 16;
-  const uint32_t keep = 0xffff0000u >> sh;
-  h = (h & keep) | (hb << sh);
-  m = (m & keep) | (mb << sh);
-  l = (l & keep) | (lb << sh);
-}
-
-// Four floats, finite and below 2^128 (1 - 2^-9), as three bf16 planes of 8 bytes each; r: what each plane but the last left.
-__device__ __forceinline__ void split3_finite(const float (&x)[4], float (&r)[4], uint2 (&p)[3]) {
+// Four floats as three bf16 planes of 8 bytes each.  An infinity, or a number that bf16 rounds to one (from
+// 2^128 (1 - 2^-9) on), leaves NaN in the planes, and so in every sum that it is part of: sums that are not finite
+// are not used, but made again from the tensors themselves.
+__device__ __forceinline__ void split3(const float (&x)[4], uint2 (&p)[3]) {
+  float r[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) r[i] = x[i];
 #pragma unroll
@@ -80,18 +64,6 @@ __device__ __forceinline__ void split3_finite(const float (&x)[4], float (&r)[4]
       r[2] -= __uint_as_float(hi << 16);
       r[3] -= __uint_as_float(hi & 0xffff0000u);
     }
-  }
-}
-
-// ... any four floats.
-__device__ __forceinline__ void split3(const float (&x)[4], uint2 (&p)[3]) {
-  float r[4];
-  split3_finite(x, r, p);
-  // What is not finite, or rounds to infinity (from 2^128 (1 - 2^-9) on), has left NaN behind.
-  if (__builtin_expect(__builtin_isunordered(r[0], r[1]) || __builtin_isunordered(r[2], r[3]), 0)) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (r[i] != r[i]) split3_not_rounded(x[i], i & 1, i < 2 ? p[0].x : p[0].y, i < 2 ? p[1].x : p[1].y, i < 2 ? p[2].x : p[2].y);
   }
 }
 
@@ -173,6 +145,37 @@ __device__ __forceinline__ void pack_weight_split(const Geom &g, const float *__
   }
 }
 
+// The outputs of consumer wave `wave` in the first `units` units of its workgroup's schedule that are not finite, from the
+// call's own tensors.
+template <int CT, int WC, int MB, int NB>
+__device__ __forceinline__ void remake_not_finite(const FusedArgs &a, int units, int nk_tile_pad, int wave, int lane) {
+  const Geom &g = a.g;
+  const int plane_out = g.Ho * g.Wo;
+  UnitSchedule us;
+  us.init(a.n_ptiles * a.n_ctiles * g.G, nk_tile_pad, kF32Ahead, 8 / kF32Ahead, a.cut_max);
+#pragma unroll 1
+  for (int u = 0; u < units; ++u) {
+    int L = us.tile_of(u);
+    const int ctile = L % a.n_ctiles;
+    L /= a.n_ctiles;
+    const int grp = L % g.G, ptile = L / g.G;
+    const int c0 = ctile * CT + wave % WC * (MB * 32), p0 = ptile * kPT + wave / WC * (NB * 32) + lane;
+#pragma unroll 1
+    for (int i = 0; i < MB * 32 * (NB / 2); ++i) {
+      const int col = c0 + i / (NB / 2), p = p0 + i % (NB / 2) * 64;
+      if (col >= g.cout_g || p >= (int)a.total_px) continue;
+      const int n = p / plane_out, rem = p - n * plane_out;
+      const int co = grp * g.cout_g + col;
+      float *o = (float *)a.out + ((long)n * g.Cout + co) * plane_out + rem;
+      const float was = __hip_atomic_load(o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (was - was == 0.0f) continue;
+      const float v = direct_sum<float, false>(g, (const float *)a.in + (long)n * g.Cin * g.H * g.W, a.in_c, a.in_px, a.om,
+                                               (const float *)a.weight, n, co, rem / g.Wo, rem % g.Wo);
+      *o = v + (a.bias ? ((const float *)a.bias)[co] : 0.0f);
+    }
+  }
+}
+
 // MULTI_DG, UNBORDERED: as in fused_kernel.
 template <int CT, int TMAX, bool MULTI_DG, bool UNBORDERED>
 __global__ __launch_bounds__(kThreads, 2) void fused_f32_kernel(FusedArgs a) {
@@ -215,6 +218,8 @@ __global__ __launch_bounds__(kThreads, 2) void fused_f32_kernel(FusedArgs a) {
   UnitSchedule us;
   us.init(a.n_ptiles * a.n_ctiles * g.G, nk_tile_pad, kF32Ahead, 8 / kF32Ahead, a.cut_max);
 
+  bool bad = false;    // consumer waves: a sum of a stored tile was not finite
+  int units = us.T;    // ... how many of the units they have stored: all, or all but a part of a cut tile
   for (int u = 0; u < us.T; ++u) {
     const bool is_part = us.is_part(u);
     // K range of the unit: steps kb .. kb + nk - 1 of the tile, padded to nk_pad
@@ -627,8 +632,28 @@ __global__ __launch_bounds__(kThreads, 2) void fused_f32_kernel(FusedArgs a) {
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         }
       }
+      // (sums that are not finite, see split3: looked for in the accumulators, mended behind the last unit)
+      float t = 0.0f;
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) t = fmaf(acc[nb][mb][r], 0.0f, t);
+      if (!store_tile) units = u;
+      bad = bad || (store_tile && __any(t != t));
       MDCN_BARRIER_LDS();  // E1
     }
+  }
+
+  // ---- This wave's outputs that are not finite, made again one by one.  Lanes read back what the wave has stored, past the
+  // caches.  (The arguments are read again from where the launch put them: kept from the kernel's start for this, they
+  // would take the main loop's scalar registers, 3% of a call of N=8, 256 channels, 64x64.) ----
+  if (bad) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    auto kernarg = __builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(kernarg));
+    remake_not_finite<CT, WC, MB, NB>(*(const FusedArgs *)kernarg, units, nk_tile_pad, wave, lane);
   }
 }
 

@@ -34,6 +34,8 @@ struct SegArgs {
   OffMaskView om;
   const void *bias;
   void *out;
+  // the call's own tensors (a.g.N images of the input), for outputs that are made again one by one
+  const void *in, *weight;
   long total_px;
   long n_work;        // pixel tiles x n_ctiles x G
   uint32_t plane_bytes, row_bytes;
@@ -43,9 +45,9 @@ struct SegArgs {
 
 // Fills *s for images of *g on elements of es bytes; false when the shape is not covered.
 bool seg_plan(const Geom &g, int es, int n_images, bool may_share, int cus, SegPlan *s);
-// dtype: enum mdcn_dtype.  The pre-pass writes a.xt from the dense NCHW images `in` (a.g.N of them)
-// and, when `weight` is given, a.wp.
-hipError_t seg_prepass(int dtype, const SegArgs &a, const void *in, const void *weight, hipStream_t st);
+// dtype: enum mdcn_dtype.  The pre-pass writes a.xt from the dense NCHW images a.in (a.g.N of them)
+// and, when told to, a.wp from a.weight.
+hipError_t seg_prepass(int dtype, const SegArgs &a, bool pack, hipStream_t st);
 hipError_t seg_forward(int dtype, const SegArgs &a, hipStream_t st);
 
 }  // namespace mdcn

@@ -32,6 +32,7 @@
 #include <algorithm>
 
 #include "../../include/mdcn.h"
+#include "mdcn_direct.h"
 #include "mdcn_fused_f32.h"
 
 namespace mdcn {
@@ -289,7 +290,9 @@ __global__ __launch_bounds__(256, seg_occupancy((int)sizeof(E), NB, CQ)) void se
   E *out = (E *)a.out;
   const bool px_ok = p0 + pxl < a.total_px;
   E *dst = out + ((long)n * g.Cout + (long)grp * g.cout_g) * plane_out + rem;
+  float bad = 0.0f;   // NaN once a sum is not finite
   auto put = [&](int nb, int r, float v) {
+    if constexpr (kSplit) bad = fmaf(v, 0.0f, bad);
     const int col = (ct * NB + nb) * 32 + (r >> 2) * 8 + half * 4 + (r & 3);
     if (px_ok && col < g.cout_g) {
       if (a.bias) v += to_f32(((const E *)a.bias)[grp * g.cout_g + col]);
@@ -315,6 +318,27 @@ __global__ __launch_bounds__(256, seg_occupancy((int)sizeof(E), NB, CQ)) void se
         float v = 0.0f;
         for (int k = 0; k < s.kshare; ++k) v += red[((w0 + k) * 16 + r) * 64 + lane];
         put(nb, r, v);
+      }
+    }
+  }
+  if constexpr (kSplit) {
+    // sums that are not finite (split3): this lane's outputs that are not, one by one.  It reads back what it has
+    // stored, past the caches.
+    if (__any(bad != bad)) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      const int per = 16 / s.kshare;
+#pragma unroll 1
+      for (int i = 0; i < NB * per; ++i) {
+        const int nb = i / per, r = ks * per + i % per;
+        const int col = (ct * NB + nb) * 32 + (r >> 2) * 8 + half * 4 + (r & 3);
+        if (!px_ok || col >= g.cout_g) continue;
+        E *o = dst + (long)col * plane_out;
+        const float was = __hip_atomic_load(o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (was - was == 0.0f) continue;
+        const int co = grp * g.cout_g + col;
+        const float v = direct_sum<E, true>(g, (const E *)a.in + (long)n * g.Cin * g.H * g.W, (long)g.H * g.W, 1, a.om,
+                                            (const E *)a.weight, n, co, ho, wo);
+        *o = from_f32<E>(v + (a.bias ? to_f32(((const E *)a.bias)[co]) : 0.0f));
       }
     }
   }
@@ -353,13 +377,13 @@ hipError_t launch_e(const SegArgs &a, hipStream_t st) {
 }
 
 template <typename E>
-hipError_t prepass_e(const SegArgs &a, const void *in, const void *weight, hipStream_t st) {
+hipError_t prepass_e(const SegArgs &a, bool pack, hipStream_t st) {
   const int px_blocks = (a.g.Hp * a.g.Wp + 255) / 256;
   const long blocks = (long)a.g.N * a.g.G * a.s.nseg_g * a.s.cps * px_blocks;
   const long wtotal = (long)a.s.wp_bytes / 16;
-  const int pack_blocks = weight ? (int)std::max<long>(1, std::min<long>(wtotal / 256, 512)) : 0;
-  hipLaunchKernelGGL(seg_prepass_kernel<E>, dim3((unsigned)(blocks + pack_blocks)), dim3(256), 0, st, a, (const E *)in,
-                     (const E *)weight, pack_blocks, px_blocks);
+  const int pack_blocks = pack ? (int)std::max<long>(1, std::min<long>(wtotal / 256, 512)) : 0;
+  hipLaunchKernelGGL(seg_prepass_kernel<E>, dim3((unsigned)(blocks + pack_blocks)), dim3(256), 0, st, a, (const E *)a.in,
+                     (const E *)a.weight, pack_blocks, px_blocks);
   return hipGetLastError();
 }
 
@@ -408,11 +432,11 @@ bool seg_plan(const Geom &g, int es, int n_images, bool may_share, int cus, SegP
   return true;
 }
 
-hipError_t seg_prepass(int dtype, const SegArgs &a, const void *in, const void *weight, hipStream_t st) {
+hipError_t seg_prepass(int dtype, const SegArgs &a, bool pack, hipStream_t st) {
   switch (dtype) {
-    case MDCN_F32: return prepass_e<float>(a, in, weight, st);
-    case MDCN_F16: return prepass_e<f16_t>(a, in, weight, st);
-    default: return prepass_e<bf16_t>(a, in, weight, st);
+    case MDCN_F32: return prepass_e<float>(a, pack, st);
+    case MDCN_F16: return prepass_e<f16_t>(a, pack, st);
+    default: return prepass_e<bf16_t>(a, pack, st);
   }
 }
 

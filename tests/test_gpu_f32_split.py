@@ -101,3 +101,37 @@ def test_gradients_of_what_is_not_finite(cin, cout):
         small = b.isfinite() & (b.abs() < 1e28)
         assert 0 < int(small.sum()) < small.numel(), name
         assert float((a[small] - b[small]).norm() / b[small].norm()) <= 1e-5, name
+
+
+@pytest.mark.parametrize('shape', ['fused', 'fused_cut', 'nhwc', 'segment', 'segment_shared'])
+def test_infinity_times_infinity(shape):
+    """... is infinite, with the sign of the product, and so is a sum that only leaves fp32 at its end."""
+    print(f'case={shape}', flush=True)
+    g = torch.Generator().manual_seed(10)
+    n, c, cout, h, w = (1, 256, 64, 9, 10) if shape == 'fused_cut' else (2, 24, 40, 70, 80) if shape == 'segment' else \
+        (1, 24, 40, 12, 14) if shape == 'segment_shared' else (2, 64, 96, 12, 14)
+    x, wt = torch.rand(n, c, h, w, generator=g) + 0.1, torch.randn(cout, c, 3, 3, generator=g)
+    x[0, 3, 2, 2], x[0, 4, 5, 9] = float('inf'), -float('inf')
+    wt[5, 3], wt[6, 3], wt[7, 4] = float('inf'), -float('inf'), -float('inf')
+    wt[8, 5] = torch.finfo(torch.float32).max   # samples of this channel reach 1: products of up to fp32's largest, sums beyond
+    x[n - 1, 5] = 2.0
+    off = torch.rand(n, 18, h - 2, w - 2, generator=g) * 0.4 + 0.3
+    case = dict(input=x, offset=off, mask=torch.rand(n, 9, h - 2, w - 2, generator=g) * 0.5 + 0.4, weight=wt,
+                bias=None, stride=(1, 1), padding=(0, 0), dilation=(1, 1), groups=1, deform_groups=1)
+    dev = {k: v.cuda() if torch.is_tensor(v) else v for k, v in case.items()}
+    ref = capi_forward(dev, path=capi.PATH_DIRECT)
+    if shape.startswith('segment'):
+        from test_gpu_segment import segment_forward
+        got = segment_forward(dev)
+    else:
+        got = capi_forward(dict(dev, input_nhwc=shape == 'nhwc'), path=capi.PATH_FUSED)
+    assert int((ref[0, 5] == float('inf')).sum()) > 4 and int((ref[0, 6] == -float('inf')).sum()) > 4
+    assert int((ref[n - 1, 8] == float('inf')).sum()) > 4
+    assert torch.equal(got.isnan(), ref.isnan())
+    assert torch.equal(got == float('inf'), ref == float('inf')) and torch.equal(got == -float('inf'), ref == -float('inf'))
+    # what is finite: sums of up to 2304 products by fp32 adds on either side, sqrt(2304) * 2^-24 = 2.9e-6 each for random
+    # roundings; by channel, since those of the largest numbers are as coarse as these
+    for co in range(cout):
+        ok = ref[:, co].isfinite()
+        a, b = got[:, co][ok].double(), ref[:, co][ok].double()
+        assert float((a - b).norm()) <= 6e-6 * float(b.norm()), co
