@@ -61,8 +61,8 @@ struct ColGradArgs {
 // fp32 runs on the bf16 matrix pipe: three bf16 planes per operand and six of their nine products, as in
 // fused_f32_kernel, whose error is that of fp32 arithmetic.  Operands are split behind the LDS reads (every wave for
 // itself: some 290 VALU instructions per 16 of K beside 48 MFMAs of 32 clocks, where the fp32 MFMAs were 64 of 64
-// clocks).  An infinity, or a number that bf16 rounds to one, leaves NaN in the planes and so in the sums: a workgroup that
-// finds any goes over its K range again with fp32 MFMAs (EXACT).
+// clocks).  An infinity, or a number that the scale takes to one (kSplitScale), leaves NaN in the planes and so in the sums: a workgroup
+// that finds any goes over its K range again with fp32 MFMAs (EXACT).
 // N=2 256 -> 256 50x84, us, fp32 / bf16 pipe: column gradient 151 / 93, weight gradient 107 / 70.  Errors against float64
 // (2-norm): grad_input 2.9e-7 / 2.5e-7, grad_weight 3.3e-7 / 3.0e-7.
 template <typename E, int TILE, bool EXACT>
@@ -92,8 +92,9 @@ __device__ __forceinline__ void tile_products(f32x16 (&acc)[TILE / 64][2], const
     // 8 values of K as three planes of an operand
     auto split8 = [](const uint4 (&v)[2], uint4 (&p)[3]) {
       uint2 lo[3], hi[3];
-      split3({__uint_as_float(v[0].x), __uint_as_float(v[0].y), __uint_as_float(v[0].z), __uint_as_float(v[0].w)}, lo);
-      split3({__uint_as_float(v[1].x), __uint_as_float(v[1].y), __uint_as_float(v[1].z), __uint_as_float(v[1].w)}, hi);
+      auto scaled = [](uint32_t x) { return __uint_as_float(x) * kSplitScale; };
+      split3({scaled(v[0].x), scaled(v[0].y), scaled(v[0].z), scaled(v[0].w)}, lo);
+      split3({scaled(v[1].x), scaled(v[1].y), scaled(v[1].z), scaled(v[1].w)}, hi);
 #pragma unroll
       for (int s = 0; s < 3; ++s) p[s] = make_uint4(lo[s].x, lo[s].y, hi[s].x, hi[s].y);
     };
@@ -124,16 +125,19 @@ __device__ __forceinline__ void tile_products(f32x16 (&acc)[TILE / 64][2], const
   }
 }
 
-// Whether a sum is infinite or NaN.
+// Takes the scale of split operands out of the sums; whether one of them is infinite or NaN.
 template <int MB>
-__device__ __forceinline__ bool not_finite(const f32x16 (&acc)[MB][2]) {
+__device__ __forceinline__ bool unscale(f32x16 (&acc)[MB][2]) {
   float t = 0.0f;
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
     for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) t = fmaf(acc[mb][nb][r], 0.0f, t);
+      for (int r = 0; r < 16; ++r) {
+        acc[mb][nb][r] *= kSplitUnscale;
+        t = fmaf(acc[mb][nb][r], 0.0f, t);
+      }
   return t != t;
 }
 
@@ -220,7 +224,7 @@ __global__ __launch_bounds__(TILE * 2, TILE == 128 ? 2 : 1) void bwd_colgrad_ker
   };
   sweep(std::false_type());
   if constexpr (sizeof(E) == 4) {
-    if (__syncthreads_or(not_finite(acc))) sweep(std::true_type());
+    if (__syncthreads_or(unscale(acc))) sweep(std::true_type());
   }
 
   // register r of lane l: A row (r/4)*8 + (l/32)*4 + r%4 of the block, B row l%32
@@ -904,7 +908,7 @@ __global__ __launch_bounds__(TILE * 2, TILE == 128 ? 2 : 1) void bwd_wgrad_kerne
   };
   sweep(std::false_type());
   if constexpr (sizeof(E) == 4) {
-    if (__syncthreads_or(not_finite(acc))) sweep(std::true_type());
+    if (__syncthreads_or(unscale(acc))) sweep(std::true_type());
   }
 
   // register r of lane l: A row (output channel) (r/4)*8 + (l/32)*4 + r%4 of the block, B row (column row) l%32

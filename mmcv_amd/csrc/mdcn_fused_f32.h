@@ -34,6 +34,12 @@
 namespace mdcn {
 
 constexpr int kF32Planes = 3;
+// Both operands are multiplied by this before they are split, and the sums by its inverse squared: the third plane holds bits
+// down to 2^-23 of a number, and bf16, with the exponents of fp32, ends at 2^-126.  Unscaled, numbers below 2^-103 lose
+// some of their bits (2e-6 of a number of 2^-115, 2e-3 at 2^-125); scaled, the smallest normal number has
+// all of its 24.  In exchange numbers from 2^104 and sums from 2^80 on overflow, and are made again.
+constexpr float kSplitScale = 16777216.0f;
+constexpr float kSplitUnscale = 1.0f / (kSplitScale * kSplitScale);
 // K steps a gather is in flight: one register set, refilled behind its use, so that every load has a whole step
 // (some 3 000 clocks) to land.  (With two sets the compiler copies them into each other at the loop's
 // end and waits for all of their loads to do so.)
@@ -46,9 +52,9 @@ constexpr size_t fused_f32_lds_bytes(int tmax) {
   return (size_t)kF32Tiles * kPT * 192 + (size_t)kPT * tmax * 20 + 16;
 }
 
-// Four floats as three bf16 planes of 8 bytes each.  An infinity, or a number that bf16 rounds to one (from
-// 2^128 (1 - 2^-9) on), leaves NaN in the planes, and so in every sum that it is part of: sums that are not finite
-// are not used, but made again from the tensors themselves.
+// Four floats, scaled already, as three bf16 planes of 8 bytes each.  An infinity, or a number that bf16 rounds to one
+// (from 2^128 (1 - 2^-9) on), leaves NaN in the planes, and so in every sum that it is part of: sums that are not
+// finite are not used, but made again from the tensors themselves.
 __device__ __forceinline__ void split3(const float (&x)[4], uint2 (&p)[3]) {
   float r[4];
 #pragma unroll
@@ -105,6 +111,8 @@ __device__ __forceinline__ void pack_weight_split(const Geom &g, const float *__
         for (int i = 0; i < 72; ++i) v[i] = 0.0f;
       }
 #pragma unroll
+      for (int i = 0; i < 72; ++i) v[i] *= kSplitScale;
+#pragma unroll
       for (int tap = 0; tap < 9; ++tap) {
         uint2 p0[3], p1[3];
         split3({v[tap], v[9 + tap], v[18 + tap], v[27 + tap]}, p0);
@@ -135,7 +143,7 @@ __device__ __forceinline__ void pack_weight_split(const Geom &g, const float *__
     float v[8];
     const float *src = w + ((long)(grp * g.cout_g + min(col, g.cout_g - 1)) * g.cin_g + c0) * g.taps + tap;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = col < g.cout_g ? src[(long)i * g.taps] : 0.0f;
+    for (int i = 0; i < 8; ++i) v[i] = col < g.cout_g ? src[(long)i * g.taps] * kSplitScale : 0.0f;
     uint2 p0[3], p1[3];
     split3({v[0], v[1], v[2], v[3]}, p0);
     split3({v[4], v[5], v[6], v[7]}, p1);
@@ -280,7 +288,7 @@ __global__ __launch_bounds__(kThreads, 2) void fused_f32_kernel(FusedArgs a) {
             const int ti = tap / g.kw, tj = tap - ti * g.kw;
             TapSample sm =
                 make_tap_sample(tb_ho * g.sh - g.ph + ti * g.dh, tb_wo * g.sw - g.pw + tj * g.dw,
-                                to_f32(rdy[i]), to_f32(rdx[i]), mask_value<E>(rm[i], a.om.logit), g.H, g.W);
+                                to_f32(rdy[i]), to_f32(rdx[i]), mask_value<E>(rm[i], a.om.logit) * kSplitScale, g.H, g.W);
             // byte offset of the upper left corner, slab 0 of image tb_n
             uint32_t pix = (uint32_t)tb_n * a.img_bytes + corner_offset<UNBORDERED>(sm, g, a);
             uint32_t tw[4];
@@ -595,8 +603,10 @@ __global__ __launch_bounds__(kThreads, 2) void fused_f32_kernel(FusedArgs a) {
           for (int r4 = 0; r4 < 4; ++r4) {
             const int px = nb * 32 + r4 * 8 + fhalf * 4;
             const f32x16 &c = acc[np * 2 + nb][mb];
-            TR::store4(stage + frow * RB + px * ES, c[r4 * 4 + 0] + bv[mb], c[r4 * 4 + 1] + bv[mb],
-                       c[r4 * 4 + 2] + bv[mb], c[r4 * 4 + 3] + bv[mb]);
+            float v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = fmaf(c[r4 * 4 + e], kSplitUnscale, bv[mb]);
+            TR::store4(stage + frow * RB + px * ES, v[0], v[1], v[2], v[3]);
           }
         }
         // the same wave wrote and now reads: only its own LDS operations matter

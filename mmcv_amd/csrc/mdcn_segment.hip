@@ -85,9 +85,12 @@ __global__ __launch_bounds__(256) void seg_prepass_kernel(SegArgs a, const E *__
       };
       if constexpr (sizeof(E) == 4) {
         if (split) {
+          float v[8];
+#pragma unroll
+          for (int i = 0; i < 8; ++i) v[i] = at(i) * kSplitScale;
           uint2 p0[3], p1[3];
-          split3({at(0), at(1), at(2), at(3)}, p0);
-          split3({at(4), at(5), at(6), at(7)}, p1);
+          split3({v[0], v[1], v[2], v[3]}, p0);
+          split3({v[4], v[5], v[6], v[7]}, p1);
 #pragma unroll
           for (int k = 0; k < 3; ++k)
             ((uint4 *)a.wp)[((frag * 3 + k) * s.nb + nb) * 64 + lane] = make_uint4(p0[k].x, p0[k].y, p1[k].x, p1[k].y);
@@ -193,13 +196,14 @@ __global__ __launch_bounds__(256, seg_occupancy((int)sizeof(E), NB, CQ)) void se
     r.tij = p < s.pairs ? t.z : 0x7fff0000u;
     r.chunk = t.w;
   };
+  constexpr bool kSplit = seg_split((int)sizeof(E), CQ);
   struct Gather {
     uint4 v[CQ][4];
     uint4 w;
   };
   auto gather = [&](const Raw &r, Gather &v) {
     const TapSample sm = make_tap_sample(by + (int)(r.tij >> 16), bx + (int)(r.tij & 0xffffu), to_f32(r.dy), to_f32(r.dx),
-                                         mask_value<E>(r.m, a.om.logit), g.H, g.W);
+                                         mask_value<E>(r.m, a.om.logit) * (kSplit ? kSplitScale : 1.0f), g.H, g.W);
     // (a position outside reads border pixels: see corner_offset())
     const uint32_t pix = sm.inside ? (uint32_t)((sm.y0 + 1) * g.Wp + sm.x0 + 1) : (uint32_t)(g.Wp - 1);
     uint32_t o = img + r.chunk * a.plane_bytes + pix * 16u;
@@ -216,7 +220,6 @@ __global__ __launch_bounds__(256, seg_occupancy((int)sizeof(E), NB, CQ)) void se
       o += a.plane_bytes;
     }
   };
-  constexpr bool kSplit = seg_split((int)sizeof(E), CQ);
   constexpr int FR = seg_frags((int)sizeof(E), CQ);
   const uint4 *wp = (const uint4 *)a.wp + (size_t)(grp * s.n_ctiles + ct) * s.iters * (FR * NB * 64) + lane;
   auto load_w = [&](int i, uint4 (&wf)[FR][NB]) {
@@ -292,7 +295,10 @@ __global__ __launch_bounds__(256, seg_occupancy((int)sizeof(E), NB, CQ)) void se
   E *dst = out + ((long)n * g.Cout + (long)grp * g.cout_g) * plane_out + rem;
   float bad = 0.0f;   // NaN once a sum is not finite
   auto put = [&](int nb, int r, float v) {
-    if constexpr (kSplit) bad = fmaf(v, 0.0f, bad);
+    if constexpr (kSplit) {
+      bad = fmaf(v, 0.0f, bad);
+      v *= kSplitUnscale;
+    }
     const int col = (ct * NB + nb) * 32 + (r >> 2) * 8 + half * 4 + (r & 3);
     if (px_ok && col < g.cout_g) {
       if (a.bias) v += to_f32(((const E *)a.bias)[grp * g.cout_g + col]);

@@ -135,3 +135,52 @@ def test_infinity_times_infinity(shape):
         ok = ref[:, co].isfinite()
         a, b = got[:, co][ok].double(), ref[:, co][ok].double()
         assert float((a - b).norm()) <= 6e-6 * float(b.norm()), co
+
+
+TINY = [(2.0 ** -117, 1.0, 1.0), (1.0, 2.0 ** -117, 1.0), (2.0 ** 60, 2.0 ** -118, 1.0), (2.0 ** -30, 1.0, 2.0 ** -88)]
+
+
+@pytest.mark.parametrize('kernel', ['fused', 'segment'])
+@pytest.mark.parametrize('scale_x,scale_w,scale_m', TINY, ids=['x', 'w', 'w_large_x', 'mask'])
+def test_smallest_numbers_keep_their_bits(kernel, scale_x, scale_w, scale_m):
+    """Operands near the end of fp32's range: a number's lower bf16 planes lie below it."""
+    print(f'case={kernel} {scale_x} {scale_w} {scale_m}', flush=True)
+    g = torch.Generator().manual_seed(11)
+    n, cin, cout, h, w = 2, 64 if kernel == 'fused' else 40, 72, 13, 15
+    off = torch.round(torch.randn(n, 18, h, w, generator=g) * 8) / 4   # exact positions and corner weights
+    mask = torch.round(torch.rand(n, 9, h, w, generator=g) * 255 + 1) / 256 * scale_m
+    # (magnitudes of 1 to 2 times a factor: every operand stays a normal number, and the sums do)
+    sign = lambda *s: torch.randint(0, 2, s, generator=g) * 2.0 - 1.0
+    x = (1 + torch.rand(n, cin, h, w, generator=g)) * sign(n, cin, h, w) * scale_x
+    wt = (1 + torch.rand(cout, cin, 3, 3, generator=g)) * sign(cout, cin, 3, 3) * scale_w
+    case = dict(input=x, offset=off, mask=mask, weight=wt, bias=None, stride=(1, 1), padding=(1, 1),
+                dilation=(1, 1), groups=1, deform_groups=1)
+    dev = {k: v.cuda() if torch.is_tensor(v) else v for k, v in case.items()}
+    ref = capi_forward({k: v.double() if torch.is_tensor(v) else v for k, v in dev.items()})
+    if kernel == 'segment':
+        from test_gpu_segment import segment_forward
+        y = segment_forward(dev).double()
+    else:
+        y = capi_forward(dev, path=capi.PATH_FUSED).double()
+    # sums of up to 576 products: 1.8e-6 as above, and outputs of some 2^-114 at least, so that nothing is subnormal
+    assert float((y - ref).norm() / ref.norm()) <= 1.8e-6
+
+
+@pytest.mark.parametrize('scale_x,scale_w,scale_g', [(1.0, 1.0, 2.0 ** -119), (1.0, 2.0 ** -119, 1.0), (2.0 ** -119, 1.0, 1.0),
+                                                     (2.0 ** 40, 2.0 ** -119, 2.0 ** 40)], ids=['g', 'w', 'x', 'w_large_g'])
+def test_gradients_of_the_smallest_numbers(scale_x, scale_w, scale_g):
+    from common import capi_backward
+    print(f'case={scale_x} {scale_w} {scale_g}', flush=True)
+    dev, gy = _backward_case(12, 2, 64, 64, 11, 14)
+    sign = lambda t: torch.where(t < 0, -1.0, 1.0)
+    dev['input'] = sign(dev['input']) * (1 + dev['input'].abs().clamp(max=1)) * scale_x
+    dev['weight'] = sign(dev['weight']) * (1 + (20 * dev['weight']).abs().clamp(max=1)) * scale_w
+    gy = sign(gy) * (1 + gy.abs().clamp(max=1)) * scale_g
+    got = capi_backward(dev, gy, path=capi.PATH_FUSED)
+    ref = capi_backward({k: v.double() if torch.is_tensor(v) else v for k, v in dev.items()}, gy.double())
+    for name, a, b in zip(('input', 'offset', 'mask', 'weight'), got, ref):
+        # (a gradient below fp32's normal numbers has lost bits by itself)
+        if float(b.abs().max()) < 2.0 ** -120:
+            continue
+        terms = 308 if name == 'weight' else 64 + 9 * 64
+        assert float((a.double() - b).norm() / b.norm()) <= terms ** 0.5 * 2.0 ** -24, name
