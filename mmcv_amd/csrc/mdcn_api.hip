@@ -242,14 +242,14 @@ long wide_tiles_of_call(const mdcn_params *p, const Geom &g, const Plan &pl, lon
                     wide_tile_cost(pl.CT, g.sh == 1 && g.sw == 1));
 }
 
-// The segment kernel for a call the fused kernels do not take, in passes of n_chunk images.
-void plan_segments(const mdcn_params *p, const Geom &g, Plan *pl) {
+// The segment kernel for a call the fused kernels do not take, in passes of n_chunk images.  small: one that they do
+// take, whose 16-bit samples it rounds as they do.
+void plan_segments(const mdcn_params *p, const Geom &g, Plan *pl, bool small = false) {
   pl->seg = false;
   if (p->path == MDCN_PATH_DIRECT || p->dtype == MDCN_F64 || p->input_nhwc) return;
-  const int es = (int)elem_size(p->dtype);
-  if ((uint64_t)g.N * g.Ho * g.Wo > 0x7fffffffull || !seg_plan(g, es, 1, false, num_cus(), &pl->sp)) return;
+  if ((uint64_t)g.N * g.Ho * g.Wo > 0x7fffffffull || !seg_plan(g, p->dtype, small, 1, false, num_cus(), &pl->sp)) return;
   pl->n_chunk = (int)std::min<uint64_t>((uint64_t)g.N, std::max<uint64_t>(1, g_fwd_pass_bytes.load() / pl->sp.xt_bytes));
-  pl->seg = seg_plan(g, es, pl->n_chunk, !p->no_k_split, num_cus(), &pl->sp);
+  pl->seg = seg_plan(g, p->dtype, small, pl->n_chunk, !p->no_k_split, num_cus(), &pl->sp);
   pl->xt_bytes = align_up(pl->sp.xt_bytes);
   pl->wp_bytes = align_up(pl->sp.wp_bytes);
 }
@@ -271,7 +271,7 @@ bool small_call(const mdcn_params *p, const Geom &g, const Plan &fused, Plan *al
   if (p->path != MDCN_PATH_AUTO || p->input_nhwc || !fused.fused) return false;
   *alt = fused;
   alt->fused = false;
-  plan_segments(p, g, alt);
+  plan_segments(p, g, alt, true);
   if (!alt->seg || alt->n_chunk != g.N || alt->sp.iters > 18 || alt->sp.nb > 2) return false;
   const long waves = ((long)g.N * g.Ho * g.Wo + 31) / 32 * alt->sp.n_ctiles * g.G;
   if (waves > 3L * num_cus() || alt->xt_bytes + alt->wp_bytes > fused.xt_bytes + fused.wp_bytes) return false;

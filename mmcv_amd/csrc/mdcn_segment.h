@@ -9,8 +9,6 @@ namespace mdcn {
 
 constexpr int kSegPairsMax = 2048;   // (channel group, tap) pairs of one convolution group: 32 KB of LDS
 
-constexpr int kSegFragsMax = 12;     // weight fragments of one step a wave holds in registers
-
 // How the channels of a convolution group are laid out: in segments of `seg`
 // channels that belong to one deformable group, each padded to `cps` 16-byte
 // chunks, which are read cq at a time.
@@ -24,13 +22,14 @@ struct SegPlan {
   int nb;         // 32-channel blocks of output channels per tile
   int n_ctiles;   // tiles of output channels per group
   int kshare;     // waves of a workgroup that share a pixel block's K range: 1, 2 or 4
+  bool rounded;   // 16 bits: samples are rounded to the tensors' type, as the fused kernels do
   size_t xt_bytes, wp_bytes;
 };
 
 struct SegArgs {
   Geom g;
   const void *xt;   // [N][chunks][H + 2][W + 2][16 bytes], chunks in order of the padded channels
-  const void *wp;   // [G][n_ctiles][iters][cq, split fp32: cq / 2 x 3 planes][nb][64 lanes][16 bytes]
+  const void *wp;   // [G][n_ctiles][iters][fragments of 8 channels x bf16 planes, fp32 with cq = 1: 4 channels][nb][64 lanes][16 bytes]
   OffMaskView om;
   const void *bias;
   void *out;
@@ -43,9 +42,10 @@ struct SegArgs {
   SegPlan s;
 };
 
-// Fills *s for images of *g on elements of es bytes; false when the shape is not covered.
-bool seg_plan(const Geom &g, int es, int n_images, bool may_share, int cus, SegPlan *s);
-// dtype: enum mdcn_dtype.  The pre-pass writes a.xt from the dense NCHW images a.in (a.g.N of them)
+// Fills *s for images of *g of type dtype (enum mdcn_dtype); false when the shape is not covered.  rounded: see
+// SegPlan, for 64 output channels a tile at most.
+bool seg_plan(const Geom &g, int dtype, bool rounded, int n_images, bool may_share, int cus, SegPlan *s);
+// The pre-pass writes a.xt from the dense NCHW images a.in (a.g.N of them)
 // and, when told to, a.wp from a.weight.
 hipError_t seg_prepass(int dtype, const SegArgs &a, bool pack, hipStream_t st);
 hipError_t seg_forward(int dtype, const SegArgs &a, hipStream_t st);

@@ -9,7 +9,7 @@
 // 32 lanes take the even pairs of the pixels and the upper 32 the odd ones,
 // each lane reads its pixel's offsets and mask from the NCHW tensors (32 lanes =
 // 32 neighbouring pixels), gathers the four corners of cq chunks and blends them,
-// and what comes out is a B operand of the 32x32 MFMA as it stands (column =
+// and what comes out is a B operand of the 32x32 MFMA but for its rounding (column =
 // lane % 32, K half = lane / 32: K may be walked in any order as long as the
 // packed weights follow it).  No LDS tile, no barrier in the K loop; a position
 // is computed once per pair and used for cq chunks.  Neighbouring lanes sample
@@ -19,8 +19,12 @@
 // Few pixels: `kshare` waves of the workgroup split the pairs of a pixel block
 // among them and add their accumulators up through LDS, in a fixed order.
 //
-// fp32 with two or more chunks a position: the products run on the bf16 matrix pipe, three exact planes per operand
-// and six of their nine products (mdcn_fused_f32.h); weights are split when they are packed, samples behind the blend.
+// Samples are fp32 numbers whatever the tensors are, and the sums those of fp32 products: they run on the bf16 matrix
+// pipe, three exact planes per sample.  fp32 weights have three planes too and six of the nine products are summed
+// (mdcn_fused_f32.h), fp16 weights fit two (five of six), bf16 weights are one (all three).  Weights are split when they are
+// packed, samples behind the blend.  fp32 with one chunk a position (half a fragment) takes the fp32 MFMAs.
+// ROUND: small 16-bit calls of shapes that the fused kernels take round samples and corner weights to the type as these do,
+// and have nothing to split.
 //
 // What bounds it: the vector-memory path of the CU (64 bytes of corner data per 16 bytes of S), the VALU (position,
 // blend, split) and the MFMAs take some 50 us each of the dg8 case below, and two to four waves a SIMD overlap them
@@ -39,10 +43,20 @@ namespace mdcn {
 
 namespace {
 
-// fp32 on the bf16 matrix pipe, three planes per operand (mdcn_fused_f32.h): two chunks fill the K of one MFMA.
-constexpr bool seg_split(int es, int cq) { return es == 4 && cq >= 2; }
+// On the bf16 matrix pipe: eight channels, one or two chunks, are a lane's half of the K of one MFMA.
+constexpr bool seg_split(int es, int cq, bool rounded) { return !rounded && (es == 2 || cq >= 2); }
+// bf16 planes of a weight
+template <typename E>
+constexpr int kSegPlanes = 3;
+template <>
+constexpr int kSegPlanes<bf16_t> = 1;
+template <>
+constexpr int kSegPlanes<f16_t> = 2;
+int seg_planes(int dtype, bool rounded) {
+  return rounded ? 1 : dtype == MDCN_F32 ? kSegPlanes<float> : dtype == MDCN_F16 ? kSegPlanes<f16_t> : kSegPlanes<bf16_t>;
+}
 // 16-byte weight fragments of one iteration and 32-channel block
-constexpr int seg_frags(int es, int cq) { return seg_split(es, cq) ? cq / 2 * 3 : cq; }
+constexpr int seg_frags(int es, int planes, int cq) { return es == 2 ? cq * planes : cq >= 2 ? cq / 2 * planes : cq; }
 
 // Weights to A-operand order and the input to chunk planes, one launch: the first
 // pack_blocks workgroups repack, the others copy 256 pixels of the bordered plane
@@ -54,8 +68,9 @@ __global__ __launch_bounds__(256) void seg_prepass_kernel(SegArgs a, const E *__
   const Geom &g = a.g;
   const SegPlan &s = a.s;
   if ((int)blockIdx.x < pack_blocks) {
-    const bool split = seg_split((int)sizeof(E), s.cq);
-    const int qn = split ? s.cq / 2 : s.cq;     // fragments of an iteration, each of them three planes when split
+    const bool split = seg_split((int)sizeof(E), s.cq, s.rounded);
+    constexpr int CF = 8 / VC;                  // chunks of a fragment when split
+    const int qn = split ? s.cq / CF : s.cq;    // fragments of an iteration, when split as planes
     const long total = (long)g.G * s.n_ctiles * s.iters * qn * s.nb * 64;
     const int grp_per_seg = s.cps / s.cq;
     for (long idx = (long)blockIdx.x * 256 + threadIdx.x; idx < total; idx += (long)pack_blocks * 256) {
@@ -76,26 +91,25 @@ __global__ __launch_bounds__(256) void seg_prepass_kernel(SegArgs a, const E *__
       const int sg = p / g.taps, tap = p - sg * g.taps;
       const int sl = sg / grp_per_seg;                                   // segment of the group
       // first channel of the fragment in it
-      const int c0 = ((sg - sl * grp_per_seg) * s.cq + (split ? 2 * q : q)) * VC;
+      const int c0 = ((sg - sl * grp_per_seg) * s.cq + (split ? CF * q : q)) * VC;
       auto at = [&](int i) {
         const bool ok = p < s.pairs && col < g.cout_g && c0 + i < s.seg;
         const E *src = w + ((long)(grp * g.cout_g + (ok ? col : 0)) * g.cin_g + (ok ? sl * s.seg + c0 + i : 0)) * g.taps +
                        (ok ? tap : 0);
         return ok ? *src : from_f32<E>(0.0f);
       };
-      if constexpr (sizeof(E) == 4) {
-        if (split) {
-          float v[8];
+      if (split) {
+        float v[8];
 #pragma unroll
-          for (int i = 0; i < 8; ++i) v[i] = at(i) * kSplitScale;
-          uint2 p0[3], p1[3];
-          split3({v[0], v[1], v[2], v[3]}, p0);
-          split3({v[4], v[5], v[6], v[7]}, p1);
+        for (int i = 0; i < 8; ++i) v[i] = to_f32(at(i)) * kSplitScale;
+        uint2 p0[3], p1[3];
+        split3({v[0], v[1], v[2], v[3]}, p0);
+        split3({v[4], v[5], v[6], v[7]}, p1);
+        constexpr int NP = kSegPlanes<E>;  // (the planes that are left out are zero)
 #pragma unroll
-          for (int k = 0; k < 3; ++k)
-            ((uint4 *)a.wp)[((frag * 3 + k) * s.nb + nb) * 64 + lane] = make_uint4(p0[k].x, p0[k].y, p1[k].x, p1[k].y);
-          continue;
-        }
+        for (int k = 0; k < NP; ++k)
+          ((uint4 *)a.wp)[((frag * NP + k) * s.nb + nb) * 64 + lane] = make_uint4(p0[k].x, p0[k].y, p1[k].x, p1[k].y);
+        continue;
       }
       E v[VC];
 #pragma unroll
@@ -130,15 +144,41 @@ __global__ __launch_bounds__(256) void seg_prepass_kernel(SegArgs a, const E *__
              (size_t)q * 16) = o;
 }
 
+// Whether a wave has registers for the weight fragments of a step beside the corners and samples of cq chunks.
+constexpr bool seg_fits(int es, int planes, int nb, int cq) {
+  return seg_frags(es, planes, cq) * nb <= (cq == 4 ? 16 : 18) && cq * nb <= 12;
+}
+
 // Waves per SIMD the register budget is cut for.
-constexpr int seg_occupancy(int ES, int NB, int CQ) {
-  if (seg_split(ES, CQ)) return CQ * NB <= 4 && CQ == 2 ? 3 : 2;
+constexpr int seg_occupancy(int ES, int NB, int CQ, bool rounded) {
+  if (seg_split(ES, CQ, rounded)) return CQ * NB <= 4 && CQ == 2 ? 3 : 2;
   return CQ * NB <= 4 && NB <= 2 ? 4 : (NB <= 4 && CQ * NB <= 8 ? 3 : 2);
 }
 
-template <typename E, int NB, int CQ>
-__global__ __launch_bounds__(256, seg_occupancy((int)sizeof(E), NB, CQ)) void segment_kernel(SegArgs a) {
-  using TR = ElemTraits<E>;
+// 16 bytes of channels of one pixel from the same 16 bytes at its four corners, in fp32.
+template <typename E>
+__device__ __forceinline__ void blend(const uint4 (&v)[4], const uint32_t (&w)[4], float *o) {
+  constexpr int VC = 16 / (int)sizeof(E);
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const uint32_t d[4] = {v[q].x, v[q].y, v[q].z, v[q].w};
+    const float wq = __uint_as_float(w[q]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      float c[VC / 4];
+      if constexpr (VC == 4)
+        c[0] = __uint_as_float(d[j]);
+      else
+        ElemTraits<E>::unpack2(d[j], c[0], c[1]);
+#pragma unroll
+      for (int k = 0; k < VC / 4; ++k) o[VC / 4 * j + k] = q == 0 ? wq * c[k] : fmaf(wq, c[k], o[VC / 4 * j + k]);
+    }
+  }
+}
+
+template <typename E, int NB, int CQ, bool ROUND>
+__global__ __launch_bounds__(256, seg_occupancy((int)sizeof(E), NB, CQ, ROUND)) void segment_kernel(SegArgs a) {
+  constexpr int VC = 16 / (int)sizeof(E);
   const Geom &g = a.g;
   const SegPlan &s = a.s;
   extern __shared__ __align__(16) unsigned char smem[];
@@ -196,10 +236,10 @@ __global__ __launch_bounds__(256, seg_occupancy((int)sizeof(E), NB, CQ)) void se
     r.tij = p < s.pairs ? t.z : 0x7fff0000u;
     r.chunk = t.w;
   };
-  constexpr bool kSplit = seg_split((int)sizeof(E), CQ);
+  constexpr bool kSplit = seg_split((int)sizeof(E), CQ, ROUND);
   struct Gather {
     uint4 v[CQ][4];
-    uint4 w;
+    uint32_t w[4];
   };
   auto gather = [&](const Raw &r, Gather &v) {
     const TapSample sm = make_tap_sample(by + (int)(r.tij >> 16), bx + (int)(r.tij & 0xffffu), to_f32(r.dy), to_f32(r.dx),
@@ -207,9 +247,7 @@ __global__ __launch_bounds__(256, seg_occupancy((int)sizeof(E), NB, CQ)) void se
     // (a position outside reads border pixels: see corner_offset())
     const uint32_t pix = sm.inside ? (uint32_t)((sm.y0 + 1) * g.Wp + sm.x0 + 1) : (uint32_t)(g.Wp - 1);
     uint32_t o = img + r.chunk * a.plane_bytes + pix * 16u;
-    uint32_t tw[4];
-    TR::table_weights(sm, tw);
-    v.w = make_uint4(tw[0], tw[1], tw[2], tw[3]);
+    ElemTraits<typename std::conditional<ROUND, E, float>::type>::table_weights(sm, v.w);
 #pragma unroll
     for (int q = 0; q < CQ; ++q) {
       const unsigned char *top = xt + o, *bot = xt + (o + a.row_bytes);
@@ -220,7 +258,8 @@ __global__ __launch_bounds__(256, seg_occupancy((int)sizeof(E), NB, CQ)) void se
       o += a.plane_bytes;
     }
   };
-  constexpr int FR = seg_frags((int)sizeof(E), CQ);
+  constexpr int NP = ROUND ? 1 : kSegPlanes<E>;
+  constexpr int FR = seg_frags((int)sizeof(E), NP, CQ);
   const uint4 *wp = (const uint4 *)a.wp + (size_t)(grp * s.n_ctiles + ct) * s.iters * (FR * NB * 64) + lane;
   auto load_w = [&](int i, uint4 (&wf)[FR][NB]) {
     const uint4 *src = wp + (size_t)i * (FR * NB * 64);
@@ -246,10 +285,17 @@ __global__ __launch_bounds__(256, seg_occupancy((int)sizeof(E), NB, CQ)) void se
     load_w(i0, wf);
     load_om(min(i0 + 1, i1 - 1), raw);
     for (int i = i0; i < i1; ++i) {
-      uint4 x[CQ];
+      float x[ROUND ? 1 : CQ * VC];
+      uint4 xr[ROUND ? CQ : 1];
 #pragma unroll
-      for (int q = 0; q < CQ; ++q) x[q] = TR::blend(gv.v[q][0], gv.v[q][1], gv.v[q][2], gv.v[q][3], gv.w);
-      uint4 wc[kSplit ? 1 : FR][NB];  // (split fp32 has no registers for both: its next fragments are fetched behind the products)
+      for (int q = 0; q < CQ; ++q) {
+        if constexpr (ROUND)
+          xr[q] = ElemTraits<E>::blend(gv.v[q][0], gv.v[q][1], gv.v[q][2], gv.v[q][3],
+                                       make_uint4(gv.w[0], gv.w[1], gv.w[2], gv.w[3]));
+        else
+          blend<E>(gv.v[q], gv.w, x + q * VC);
+      }
+      uint4 wc[kSplit ? 1 : FR][NB];  // (split samples leave no registers for both: the next fragments are fetched behind the products)
       if constexpr (!kSplit) {
 #pragma unroll
         for (int q = 0; q < FR; ++q)
@@ -261,28 +307,32 @@ __global__ __launch_bounds__(256, seg_occupancy((int)sizeof(E), NB, CQ)) void se
       load_om(min(i + 2, i1 - 1), raw);
       if constexpr (kSplit) {
 #pragma unroll
-        for (int q = 0; q < CQ / 2; ++q) {
+        for (int q = 0; q < CQ * VC / 8; ++q) {
           uint2 lo[3], hi[3];
-          const uint4 &u = x[2 * q], &v = x[2 * q + 1];
-          split3({__uint_as_float(u.x), __uint_as_float(u.y), __uint_as_float(u.z), __uint_as_float(u.w)}, lo);
-          split3({__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w)}, hi);
+          const float *f = x + 8 * q;
+          split3({f[0], f[1], f[2], f[3]}, lo);
+          split3({f[4], f[5], f[6], f[7]}, hi);
           auto products = [&](int xp, int wpl) {
             const uint4 xv = make_uint4(lo[xp].x, lo[xp].y, hi[xp].x, hi[xp].y);
 #pragma unroll
-            for (int nb = 0; nb < NB; ++nb) ElemTraits<bf16_t>::mma(acc[nb], wf[3 * q + wpl][nb], xv);
+            for (int nb = 0; nb < NB; ++nb) ElemTraits<bf16_t>::mma(acc[nb], wf[NP * q + wpl][nb], xv);
           };
           products(2, 0);  // smallest terms first
-          products(0, 2);
-          products(1, 1);
+          if constexpr (NP > 2) products(0, 2);
+          if constexpr (NP > 1) products(1, 1);
           products(1, 0);
-          products(0, 1);
+          if constexpr (NP > 1) products(0, 1);
           products(0, 0);
         }
       } else {
 #pragma unroll
-        for (int q = 0; q < CQ; ++q)
+        for (int q = 0; q < CQ; ++q) {
+          if constexpr (!ROUND)
+            xr[0] = make_uint4(__float_as_uint(x[4 * q]), __float_as_uint(x[4 * q + 1]), __float_as_uint(x[4 * q + 2]),
+                               __float_as_uint(x[4 * q + 3]));
 #pragma unroll
-          for (int nb = 0; nb < NB; ++nb) TR::mma(acc[nb], wc[q][nb], x[q]);
+          for (int nb = 0; nb < NB; ++nb) ElemTraits<E>::mma(acc[nb], wc[q][nb], xr[ROUND ? q : 0]);
+        }
       }
       if constexpr (kSplit) __builtin_amdgcn_sched_barrier(0);
       load_w(min(i + 1, i1 - 1), wf);
@@ -339,7 +389,8 @@ __global__ __launch_bounds__(256, seg_occupancy((int)sizeof(E), NB, CQ)) void se
         const int col = (ct * NB + nb) * 32 + (r >> 2) * 8 + half * 4 + (r & 3);
         if (!px_ok || col >= g.cout_g) continue;
         E *o = dst + (long)col * plane_out;
-        const float was = __hip_atomic_load(o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        using U = typename std::conditional<sizeof(E) == 2, uint16_t, uint32_t>::type;
+        const float was = to_f32(__builtin_bit_cast(E, __hip_atomic_load((const U *)o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)));
         if (was - was == 0.0f) continue;
         const int co = grp * g.cout_g + col;
         const float v = direct_sum<E, true>(g, (const E *)a.in + (long)n * g.Cin * g.H * g.W, (long)g.H * g.W, 1, a.om,
@@ -350,25 +401,30 @@ __global__ __launch_bounds__(256, seg_occupancy((int)sizeof(E), NB, CQ)) void se
   }
 }
 
-template <typename E, int NB, int CQ>
+template <typename E, int NB, int CQ, bool ROUND = false>
 hipError_t launch(const SegArgs &a, hipStream_t st) {
   const size_t lds = (size_t)a.s.pairs * 16 + (a.s.kshare > 1 ? 4 * 16 * 64 * 4 : 0);
-  hipLaunchKernelGGL((segment_kernel<E, NB, CQ>), dim3((unsigned)((a.n_work + 7) / 8 * 8)), dim3(256), lds, st, a);
+  hipLaunchKernelGGL((segment_kernel<E, NB, CQ, ROUND>), dim3((unsigned)((a.n_work + 7) / 8 * 8)), dim3(256), lds, st, a);
   return hipGetLastError();
 }
 
 template <typename E, int CQ>
 hipError_t launch_nb(const SegArgs &a, hipStream_t st) {
+  if constexpr (sizeof(E) == 2) {
+    if (a.s.rounded) return a.s.nb == 1 ? launch<E, 1, CQ, true>(a, st) : a.s.nb == 2 ? launch<E, 2, CQ, true>(a, st) : hipErrorInvalidValue;
+  }
   switch (a.s.nb) {
     case 1: return launch<E, 1, CQ>(a, st);
     case 2: return launch<E, 2, CQ>(a, st);
     default: break;
   }
-  if constexpr (!(seg_split((int)sizeof(E), CQ) && CQ == 4)) {
+  if constexpr (seg_fits((int)sizeof(E), kSegPlanes<E>, 3, CQ)) {
     if (a.s.nb == 3) return launch<E, 3, CQ>(a, st);
   }
-  if constexpr (CQ <= 2) {
+  if constexpr (seg_fits((int)sizeof(E), kSegPlanes<E>, 4, CQ)) {
     if (a.s.nb == 4) return launch<E, 4, CQ>(a, st);
+  }
+  if constexpr (seg_fits((int)sizeof(E), kSegPlanes<E>, 6, CQ)) {
     if (a.s.nb == 6) return launch<E, 6, CQ>(a, st);
   }
   if constexpr (CQ == 1) {
@@ -395,8 +451,10 @@ hipError_t prepass_e(const SegArgs &a, bool pack, hipStream_t st) {
 
 }  // namespace
 
-bool seg_plan(const Geom &g, int es, int n_images, bool may_share, int cus, SegPlan *s) {
-  const int VC = 16 / es;
+bool seg_plan(const Geom &g, int dtype, bool rounded, int n_images, bool may_share, int cus, SegPlan *s) {
+  const int es = dtype == MDCN_F32 ? 4 : 2, VC = 16 / es;
+  s->rounded = rounded && es == 2;
+  const int planes = seg_planes(dtype, s->rounded);
   int u = g.cin_g, v = g.ch_per_dg;
   while (v) {
     const int t = u % v;
@@ -416,7 +474,7 @@ bool seg_plan(const Geom &g, int es, int n_images, bool may_share, int cus, SegP
   double best = 0.0;
   s->cq = 0;
   for (int cq = 4; cq >= 1; cq /= 2) {
-    if (cq * s->nb > kSegFragsMax || (es == 4 && cq == 4 && s->nb == 3)) continue;  // (18 fragments, split)
+    if (!seg_fits(es, planes, s->nb, cq)) continue;
     const int groups = (cps0 + cq - 1) / cq;
     const double cost = groups * 1.5 + groups * cq;
     if (s->cq == 0 || cost < best) best = cost, s->cq = cq;
@@ -430,7 +488,7 @@ bool seg_plan(const Geom &g, int es, int n_images, bool may_share, int cus, SegP
   const uint64_t img = (uint64_t)g.G * s->nseg_g * s->cps * g.Hp * g.Wp * 16;
   if (img * (uint64_t)n_images > 0xF0000000ull) return false;
   s->xt_bytes = (size_t)(img * (uint64_t)n_images);
-  s->wp_bytes = (size_t)g.G * s->n_ctiles * s->iters * seg_frags(es, s->cq) * s->nb * 1024;
+  s->wp_bytes = (size_t)g.G * s->n_ctiles * s->iters * seg_frags(es, planes, s->cq) * s->nb * 1024;
   // Waves of a workgroup share a pixel block's K range while that leaves the chip's SIMDs short of two waves.
   const long waves = ((long)n_images * g.Ho * g.Wo + 31) / 32 * s->n_ctiles * g.G;
   s->kshare = 1;

@@ -101,3 +101,36 @@ def test_segment_path_on_a_shape_of_the_fused_kernels():
     assert lib.mdcn_forward(ctypes.byref(p), None) == 0
     torch.cuda.synchronize()
     assert float((out.float() - ref).abs().max() / ref.abs().max()) <= TOL[torch.bfloat16]
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16], ids=['bf16', 'f16'])
+@pytest.mark.parametrize('name', ['seg1', 'seg3', 'seg8_dg8', 'seg24', 'seg40_groups', 'seg48', 'gcd', 'k5', 'cout150', 'cout250'])
+def test_16bit_results_are_rounded_once(name, dtype):
+    """Samples, products and sums of 16-bit tensors are those of fp32: every output is the true one, rounded once."""
+    print(f'case={name} dtype={dtype}', flush=True)
+    case = make_case(33, **CASES[name])
+    case['offset'] = torch.round(case['offset'] * 4) / 4   # exact positions and corner weights
+    dev = cast_case(case, dtype, 'cuda')
+    ref = capi_forward({k: v.double() if torch.is_tensor(v) else v for k, v in dev.items()})
+    y = segment_forward(dev).double()
+    half_ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    # an fp32 sum of (channel, tap) products of terms no larger than some 4 in all: 2^-24 each
+    terms = case['weight'][0].numel()
+    bound = ref.abs() * half_ulp + 2.0 ** -25 + terms * 2.0 ** -24 * 4
+    worst = float(((y - ref).abs() / bound).max())
+    assert worst <= 1.0, worst
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16], ids=['bf16', 'f16'])
+def test_16bit_infinities(dtype):
+    g = torch.Generator().manual_seed(12)
+    case = make_case(34, N=2, Cin=24, Cout=40, H=14, W=15, sigma=0.3, padding=0)
+    case['offset'] = torch.rand(case['offset'].shape, generator=g) * 0.4 + 0.3
+    case['input'][0, 3, 5, 5], case['input'][0, 4, 9, 9] = float('inf'), float('nan')
+    case['weight'][5, 3], case['weight'][6, 3], case['weight'][7, 9] = float('inf'), -float('inf'), float('nan')
+    dev = cast_case(case, dtype, 'cuda')
+    got, ref = segment_forward(dev), capi_forward(dev, path=capi.PATH_DIRECT)
+    assert torch.equal(got.isnan(), ref.isnan()) and torch.equal(got.isinf(), ref.isinf())
+    ok = ref.isfinite()
+    assert 0 < int(ok.sum()) < ok.numel()
+    assert float((got[ok] - ref[ok]).abs().max()) <= 2.0 ** (-7 if dtype == torch.bfloat16 else -10) * float(ref[ok].abs().max())
