@@ -154,7 +154,7 @@ int mdcn_fused_eligible(const mdcn_params *p);
 
 /* Which device kernels mdcn_forward() launches for the main stage of the call described by *p (shape,
  * dtype, path, no_k_split; of the pointers only `input` and `output` are looked at, for their alignment):
- * a static string such as "fused3_kernel", "fused3_kernel+fused2_kernel", "fused2_kernel", "fused_kernel",
+ * a static string such as "fused3_kernel", "fused3_kernel+fused2_kernel", "fused2_kernel", "fused_kernel", "fused_f32_kernel",
  * "segment_kernel" (given the scratch of mdcn_workspace_wanted()), "direct_kernel", "f64_forward_kernel"; "" for an invalid *p.  The first name is the kernel that does
  * most of the work.  For reports and tests (no counterpart in the reference). */
 const char *mdcn_forward_kernels(const mdcn_params *p);

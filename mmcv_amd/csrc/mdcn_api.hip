@@ -871,6 +871,7 @@ const char *mdcn_forward_kernels(const mdcn_params *p) {
   if (p->dtype == MDCN_F64) return "f64_forward_kernel";
   if (pl.seg) return "segment_kernel";
   if (!pl.fused) return "direct_kernel";
+  if (p->dtype == MDCN_F32) return "fused_f32_kernel";
   if (!uses_fused2(p, g, pl)) return "fused_kernel";
   const size_t es = elem_size(p->dtype);
   const long plane_out = (long)g.Ho * g.Wo;

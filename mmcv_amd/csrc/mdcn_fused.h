@@ -1,4 +1,4 @@
-// Fused DCNv2 forward for gfx950: implicit GEMM  out[pixel, cout] = S[pixel, k] * W[k, cout]
+// Fused DCNv2 forward for gfx950, 16-bit tensors (fp32: mdcn_fused_f32.h): implicit GEMM  out[pixel, cout] = S[pixel, k] * W[k, cout]
 // where S (the "columns" of the reference's two-pass design,
 // mmcv/ops/csrc/pytorch/modulated_deform_conv.cpp:101-124) is produced on the
 // fly -- offset/mask-modulated bilinear samples computed by wavefronts and
@@ -7,8 +7,8 @@
 // Work split.  A persistent workgroup of 8 wavefronts owns, one after another,
 // tiles of PT = 128 consecutive output pixels (flattened n*Ho*Wo + ho*Wo + wo)
 // x CT output channels of one group.  K runs over (slab of KC channels) x
-// (tap), slab outer, tap inner.  A slab is 128 bytes of channels (64 bf16/fp16,
-// 32 fp32), and the input copy is stored slab-major
+// (tap), slab outer, tap inner.  A slab is 128 bytes of channels (64 bf16/fp16),
+// and the input copy is stored slab-major
 // ([N][Cin/KC][H+2][W+2][KC]): one bilinear corner of one slab is exactly one
 // aligned 128-byte cache line, so every byte a gather pulls from L2 is used.
 //
@@ -19,18 +19,18 @@
 //     bilinear weights (positions and weights in fp32).  Per K step, each lane
 //     gathers for two pixels 2 x 16 bytes of channels at each of the four corners
 //     (16 x global_load_dwordx4, issued kGatherAhead steps ahead, held in
-//     registers), blends them (16-bit types: horizontal corners paired with
-//     v_perm_b32, one v_dot2 per two products; fp32: FMA) and writes 4 x 16
+//     registers), blends them (bf16: horizontal corners paired with
+//     v_perm_b32, one v_dot2 per two products; fp16: packed FMA) and writes 4 x 16
 //     bytes of the sample tile.
 //   waves 0..3  CONSUMERS.  2 x 2 over the tile (64 pixels x CT/2 channels
 //     each): read sample and weight fragments from LDS, run MFMA
-//     (32x32x16 bf16/f16, 32x32x2 fp32) into fp32 accumulators; at the end of
+//     (32x32x16 bf16/f16) into fp32 accumulators; at the end of
 //     the tile add the bias, round once, transpose through LDS and store
 //     16 bytes per lane along W of the NCHW output.  They also issue the
 //     direct-to-LDS copy of the weight tile kWeightAhead steps ahead.
 // One workgroup barrier per K step keeps the two roles in step; the sample
 // tile is double buffered, the weight tiles sit in a ring of kWeightSlots.
-// Where the epilogue's staging fits one ring slot (16-bit types, CT = 256) the
+// Where the epilogue's staging fits one ring slot (CT = 256) the
 // producers start the next tile (table, gathers, first sample tile) while the
 // consumers store the current one.
 //
@@ -297,8 +297,8 @@ template <typename E>
 constexpr int stage_row_bytes() {
   return 64 * (int)sizeof(E) + 16;
 }
-static_assert(2 * 32 * (64 * 4 + 16) <= 2 * kPT * kRowB, "two staging areas fit the sample tiles");
-static_assert(2 * 32 * (64 * 4 + 16) <= kWeightSlots * 64 * kRowB,
+static_assert(2 * 32 * stage_row_bytes<bf16_t>() <= 2 * kPT * kRowB, "two staging areas fit the sample tiles");
+static_assert(2 * 32 * stage_row_bytes<bf16_t>() <= kWeightSlots * 64 * kRowB,
               "two staging areas fit the smallest weight ring");
 
 // LDS of one workgroup: two sample tiles, the ring of weight tiles, the
@@ -435,6 +435,7 @@ __device__ __forceinline__ int tile_chunk(int r, int c) { return r * kRowChunks 
 // (clamp_to_image), which keeps the reference's per-corner rule.
 template <typename E, int CT, int TMAX, bool MULTI_DG, bool UNBORDERED>
 __global__ __launch_bounds__(kThreads, 2) void fused_kernel(FusedArgs a) {
+  static_assert(sizeof(E) == 2, "fp32 tensors: fused_f32_kernel");
   using TR = ElemTraits<E>;
   constexpr int PT = kPT;
   constexpr int KC = TR::KC;
@@ -498,10 +499,6 @@ __global__ __launch_bounds__(kThreads, 2) void fused_kernel(FusedArgs a) {
 
     if (producer) {
       // =================== PRODUCER ===================
-      // fp32 tiles of <= 128 channels: the consumers' MFMAs are short of work there and the step
-      // waits for the producers, so the arbiter is told to prefer them (cfg 3: 0.527 -> 0.486 ms).
-      // With 256-channel fp32 tiles the same setting costs 1-3 %, with 16-bit tensors it is a wash.
-      if constexpr (sizeof(E) == 4 && CT <= 128) __builtin_amdgcn_s_setprio(2);
       const int ptid = tid - 256;
       const int q = ptid & 3;          // this lane handles 16-byte chunks q and q + 4 of a row
       const int pxl = ptid >> 2;       // ... of pixels pxl and pxl + 64 of the tile

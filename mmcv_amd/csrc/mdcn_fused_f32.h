@@ -1,4 +1,4 @@
-// fp32 forward: the implicit GEMM of mdcn_fused.h with its products on the bf16
+// fp32 forward: the implicit GEMM of mdcn_fused.h, its products on the bf16
 // matrix pipe.
 //
 // The fp32 MFMA (32x32x2) runs at a sixteenth of the bf16 rate, and an fp32 tile
@@ -6,11 +6,11 @@
 // h = bf16(x), m = bf16(x - h), l = x - h - m, 8 mantissa bits each (both differences
 // are exact).  A product of two such sums has nine terms, each exact in fp32; the
 // kernel accumulates six of them in fp32 -- hh, hm, mh, mm, hl, lh -- and leaves
-// out ml, lm and ll, which together are at most 2^-25 of the product (|m| <= 2^-9 |x|,
-// |l| <= 2^-18 |x|): less than the 2^-24 an fp32 multiplication rounds by.  Six bf16 MFMAs of
-// K = 16 take 192 clocks where eight fp32 ones take 512.  Results are those of
-// fp32 arithmetic: against float64, with positions that fp32 holds exactly, the relative
-// error (2-norm) is 3.7e-7 for 2 304 terms and 5.1e-7 for 4 608; with fp32 MFMAs it was 4.3e-7 and 5.9e-7.
+// out ml, lm and ll.  |m| <= 2^-8 |x| and |l| <= 2^-17 |x|, so that these are at most
+// (2^-24 + 2^-34) of the product together, as much as an fp32 multiplication may round by.  What
+// a sum of many terms loses it loses for the most part where it is added up, and a bf16 MFMA adds sixteen terms at a time, an
+// fp32 one two.  Against float64, with positions that fp32 holds exactly, the relative error (2-norm) is 3.7e-7 for 2 304 terms and 5.1e-7 for 4 608; with fp32 MFMAs it was 4.3e-7 and 5.9e-7.  Six bf16
+// MFMAs of K = 16 take 192 clocks where eight fp32 ones take 512.
 //
 // Roles, tables, schedule, cut tiles and epilogue are those of fused_kernel.  What
 // differs: a K step (32 channels of a tap) is two half steps of 16 channels; sample and

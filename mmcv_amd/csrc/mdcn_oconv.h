@@ -15,7 +15,7 @@ namespace mdcn {
 struct OconvArgs {
   Geom g;
   const void *xt;     // zero-bordered slab-major input copy
-  const void *owp;    // packed conv_offset weights, see pack_offset_weight_kernel
+  const void *owp;    // packed conv_offset weights, see pack_offset_chunks
   const void *obias;  // (CO) or null
   void *raw;          // [N * Ho * Wo][CO_pad]
   long total_px;      // N * Ho * Wo
