@@ -302,10 +302,11 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
   const long off_step = std::max<long>(1, (off_total >> 16) | 1);
   const int far_blocks = (int)std::max<long>(1, std::min<long>(off_total / off_step / 1024, 64));
 
-  // Share of offset components beyond the margin from which the far window is the better one.  Half of 16 (fp32: 8)
+  // Share of offset components beyond the margin from which the far window is the better one.  Half of 16 (doubles: 8)
   // channels a pass cost next to nothing (bf16, N=2 C=256 135x224, margins 5 and 11: sigma 1.0 0.77 ms with either,
   // 2.5 0.87 / 0.86, 4.0 1.63 / 0.94), half of 8 do: fp16, N=7 C=128 118x196 stride 2, margins 3 and 12: sigma
-  // 2.0 0.56 / 0.59, 2.5 0.60 / 0.60, 4.0 0.94 / 0.65.
+  // 2.0 0.56 / 0.59, 2.5 0.60 / 0.60, 4.0 0.94 / 0.65.  bf16 in doubles, whole training call in us, N=4 96 -> 72 channels
+  // 37x53: sigma 1.0 131 / 132, 2.5 135 / 130, 4.0 154 / 132; N=2 C=128 60x80: 2.0 147 / 153, 3.0 158 / 153, 4.0 195 / 157.
   const uint32_t far_min = (uint32_t)(off_total / off_step / (pl.sCH * (pl.fixed ? 2 : 4) == 32 ? 32 : 5));
   auto up = [](long n, long per) { return (int)((n + per - 1) / per); };
   {

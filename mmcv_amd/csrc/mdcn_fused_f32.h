@@ -20,9 +20,10 @@
 // the weights; the consumer waves lie along the channels, so that each weight fragment has one
 // reader, which loads it from L2 into registers.
 //
-// What bounds it: a K step of a 128 x 256 tile is 3 072 clocks of MFMAs per SIMD, and the producers' floating-point
-// VALU work (the blend and the split, some 150 instructions a step) does not run beside the MFMAs of
-// the other wave of its SIMD but adds to them, 1 300 clocks.  Measured, main kernel, N=8 256 -> 256 64x64: 325 us
+// What bounds it (N=8 256 -> 256 64x64, counters): the MFMA pipe, busy in 41 % of the cycles -- a K step of a 128 x 256
+// tile is 3 072 clocks of MFMAs per SIMD and takes 7 500; a large product of the library reaches 43 % of the pipe's peak.  The other
+// VALU instructions (the blend and the split for the most part) are 12 % of the cycles, the address unit of the vector-memory path is
+// busy in 30 %, and waves wait in a quarter of theirs.  Measured, main kernel, N=8 256 -> 256 64x64: 325 us
 // with fp32 MFMAs, 213 us (MFMAs alone: 116); N=2 50x84, 128-channel tiles: 144 -> 108 us.  Tried and
 // not faster: weights through LDS (213), fp32 tiles' producers at a higher or lower wave priority (209 - 224),
 // two gather sets (209).

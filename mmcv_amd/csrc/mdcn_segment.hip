@@ -26,11 +26,12 @@
 // ROUND: small 16-bit calls of shapes that the fused kernels take round samples and corner weights to the type as these do,
 // and have nothing to split.
 //
-// What bounds it: the vector-memory path of the CU (64 bytes of corner data per 16 bytes of S), the VALU (position,
-// blend, split) and the MFMAs take some 50 us each of the dg8 case below, and two to four waves a SIMD overlap them
-// only in part.  Measured against the one-thread-per-output kernel that these shapes had before: N=2, 64 -> 64 channels, 8 deformable
-// groups, 180x320, fp32 23.9 ms -> 193 us a call with fp32 MFMAs, 178 on the bf16 pipe (error against float64 4.3e-7 -> 1.8e-7);
-// N=1 64 -> 64 56x56 22.6 -> 19.2 us; N=4, 96 -> 72 channels, 2 deformable groups, 37x53, bf16 1 733 us -> 15 + 5 us.
+// What bounds it: the vector-memory path of the CU (64 bytes of corner data per 16 bytes of S): its address unit is busy in
+// 76 % of the cycles of the dg8 case below; VALU (position, blend, split) 26 %, MFMAs 16 % (counters).  Measured against the
+// one-thread-per-output kernel that these shapes had before: N=2, 64 -> 64 channels, 8 deformable
+// groups, 180x320, fp32 23.9 ms -> 193 us a call with fp32 MFMAs, 173 on the bf16 pipe (error against float64 4.3e-7 -> 1.8e-7);
+// N=1 64 -> 64 56x56 22.6 -> 19.1 us; N=4, 96 -> 72 channels, 2 deformable groups, 37x53, bf16 1 733 us -> 21, fp16 21
+// (19 and 18 with samples rounded to 16 bits; the dg8 case in bf16 80 and 77, in fp16 88 and 76).
 #include "mdcn_segment.h"
 
 #include <algorithm>
