@@ -22,7 +22,7 @@
 // the input's channels (those of one group and one deformable group) to whole
 // passes of the scatter kernel, a group's to a multiple of 32, the output
 // channels of a group to 128 bytes.  Padding is zero in every copy, so it adds nothing
-// and its gradients are zero and never written.
+// and its gradients -- zero, or NaN where grad_output is not finite -- are never written.
 #pragma once
 
 #include <type_traits>
