@@ -35,7 +35,8 @@ def _run(cmd, cwd=None):
     subprocess.check_call(cmd, cwd=cwd)
 
 
-SOURCES = ['mdcn_api.hip', 'mdcn_backward.hip', 'mdcn_oconv.hip', 'mdcn_segment.hip']
+SOURCES = ['mdcn_api.hip', 'mdcn_backward.hip', 'mdcn_backward_bf16.hip', 'mdcn_backward_f16.hip', 'mdcn_oconv.hip',
+           'mdcn_segment.hip']
 
 
 def build_hip(extra=(), check=True):

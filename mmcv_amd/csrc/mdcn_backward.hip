@@ -4,6 +4,7 @@
 
 #include "mdcn_backward.h"
 #include "mdcn_backward_ends.h"
+#include "mdcn_backward_fused.h"
 #include "mdcn_backward_gemm.h"
 #include "mdcn_f64.h"
 #include "mdcn_fused.h"
@@ -36,7 +37,8 @@ void make_bwd_plan(const mdcn_bwd_params *bp, const Geom &g, uint64_t pass_bytes
   pl->gw_bytes = (staged && bp->grad_weight) ? align_up((size_t)g.Cout * g.cin_g * g.taps * 4) : 0;
   pl->gb_bytes = (staged && bp->grad_bias) ? align_up((size_t)g.Cout * 4) : 0;
   pl->mx_bytes = 0;
-  pl->tiled = pl->gemm = pl->wgemm = pl->fixed = false;
+  pl->tiled = pl->gemm = pl->wgemm = pl->fused = false;
+  pl->n_wnorm = pl->tw_log = 0;
   pl->xt_bytes = pl->gt_bytes = pl->wt_bytes = pl->d_bytes = pl->col_bytes = pl->part_bytes = pl->wpart_bytes = 0;
   pl->w_tile = kCgTile;
   pl->w_splits = 1;
@@ -44,6 +46,7 @@ void make_bwd_plan(const mdcn_bwd_params *bp, const Geom &g, uint64_t pass_bytes
   pl->bsplits = 0;
   pl->im = pl->om = ChanMap{1, 1, 1, 1, 1};
   pl->parts = 1;
+  pl->sched = FusedSchedule{0, 1};
   pl->n_chunk = g.N;
   pl->M_pad = 0;
   pl->cg_tile = kCgTile;
@@ -61,14 +64,13 @@ void make_bwd_plan(const mdcn_bwd_params *bp, const Geom &g, uint64_t pass_bytes
   // whose channels fill nothing (bf16, N=4, 96 -> 72, 37x53) 0.12 ms instead of 0.90.
   const int KC = (int)(128 / es);
   const long s_tiles = (long)g.N * g.DG * ((g.Ho + kScTH - 1) / kScTH) * ((g.Wo + kScTW - 1) / kScTW);
-  // 16-bit tensors hold d in 16 bits and sum grad_input in fixed point where d is what the call's time goes into: channels in
-  // whole 128-byte slabs and 64 or more tiles.  What is smaller keeps both in fp32 or better.  (A call for the weights
-  // alone has neither.)
+  // 16-bit tensors whose channels come in whole 128-byte slabs, and 64 or more tiles of them: the data side in one kernel,
+  // d in registers and grad_input summed in fixed point.  What is smaller or uneven, and fp32, goes through memory with
+  // an fp32 d and sums in doubles.
   const bool whole = g.Cin % KC == 0 && g.cout_g % KC == 0 && g.cin_g % 32 == 0 && g.ch_per_dg % 8 == 0;
-  pl->fixed = staged && (!bp->grad_input || (whole && (s_tiles >= 64 || forced)));
-  const size_t ds = pl->fixed ? es : 4;  // bytes of an element of d
-  // Channels per pass over the window: 16 / 8 of 32-bit fixed point, or 8 / 4 doubles
-  const int ch_big = pl->fixed ? 16 : 8;
+  pl->fused = staged && bp->grad_input && whole && (s_tiles >= 64 || forced) && (g.kh - 1) * g.dh < 255 && (g.kw - 1) * g.dw < 255 && s_tiles < (1L << 28);
+  const bool columns_only = staged && !bp->grad_input;
+  const size_t ds = pl->fused || columns_only ? es : 4;  // bytes of an element of d, or of the columns
   int u = g.cin_g, v = g.ch_per_dg;
   while (v) {
     const int t = u % v;
@@ -77,23 +79,40 @@ void make_bwd_plan(const mdcn_bwd_params *bp, const Geom &g, uint64_t pass_bytes
   }
   const int seg = u;
   auto padded = [](int n, int to) { return (n + to - 1) / to * to; };
-  pl->sCH = ch_big;
-  pl->sR = window_margin(g, kScTH, kScTW, kScWindowPx, &pl->sWH, &pl->sWW);
-  // fewer channels at a time buy a wider window, and less padding where segments are short (none in a fixed-point window,
-  // whose flush does not look where a segment ends)
-  const bool pads_less = pl->fixed && whole ? seg % ch_big != 0 : 4 * padded(seg, ch_big) > 5 * padded(seg, ch_big / 2);
-  if (pl->sR < 2 || pads_less) {
-    int wh, ww;
-    const int r = window_margin(g, kScTH, kScTW, 2 * kScWindowPx, &wh, &ww);
-    if (r > pl->sR || pads_less) {
-      pl->sCH = ch_big / 2;
-      pl->sR = r;
-      pl->sWH = wh;
-      pl->sWW = ww;
+  // Channels per pass over the window, and its margins: fewer channels at a time buy a wider window.  A second, wider one
+  // is for calls whose offsets leave the first.
+  if (pl->fused) {
+    // the tile shape that fewer tiles cover the plane with
+    const long n32 = (long)((g.Ho + 7) / 8) * ((g.Wo + 31) / 32), n16 = (long)((g.Ho + 15) / 16) * ((g.Wo + 15) / 16);
+    pl->tw_log = n16 < n32 ? 4 : 5;
+    const int TW = 1 << pl->tw_log, TH = 256 / TW;
+    pl->sCH = 16;
+    pl->sR = seg % 16 == 0 ? window_margin(g, TH, TW, bf_window_px(16), &pl->sWH, &pl->sWW) : -1;
+    if (pl->sR < 2) {
+      pl->sCH = 8;
+      pl->sR = window_margin(g, TH, TW, bf_window_px(8), &pl->sWH, &pl->sWW);
     }
+    pl->fR = window_margin(g, TH, TW, bf_window_px(8), &pl->fWH, &pl->fWW, kScFarMargin);
+    if (pl->fR <= pl->sR) pl->fWH = 0;
+  } else {
+    const int ch_big = columns_only ? 16 : 8;  // doubles: 8 or 4
+    pl->sCH = ch_big;
+    pl->sR = window_margin(g, kScTH, kScTW, kScWindowPx, &pl->sWH, &pl->sWW);
+    // (half the channels also mean less padding where segments are short)
+    const bool pads_less = 4 * padded(seg, ch_big) > 5 * padded(seg, ch_big / 2);
+    if (pl->sR < 2 || pads_less) {
+      int wh, ww;
+      const int r = window_margin(g, kScTH, kScTW, 2 * kScWindowPx, &wh, &ww);
+      if (r > pl->sR || pads_less) {
+        pl->sCH = ch_big / 2;
+        pl->sR = r;
+        pl->sWH = wh;
+        pl->sWW = ww;
+      }
+    }
+    pl->fR = window_margin(g, kScTH, kScTW, (long)kScWindowPx * (2 * ch_big / pl->sCH), &pl->fWH, &pl->fWW, kScFarMargin);
+    if (pl->fR <= pl->sR || pl->sCH * es < 16) pl->fWH = 0;  // (a pass reads 8 bytes of channels at least)
   }
-  pl->fR = window_margin(g, kScTH, kScTW, (long)kScWindowPx * (2 * ch_big / pl->sCH), &pl->fWH, &pl->fWW, kScFarMargin);
-  if (pl->fR <= pl->sR || pl->sCH * es < 16) pl->fWH = 0;  // (a pass reads 8 bytes of channels at least)
   ChanMap &im = pl->im, &om = pl->om;
   im.seg = seg;
   im.segp = padded(seg, pl->sCH);
@@ -107,6 +126,7 @@ void make_bwd_plan(const mdcn_bwd_params *bp, const Geom &g, uint64_t pass_bytes
   const size_t d_img = (size_t)g.taps * cin_p * plane_out * ds;
   const bool mfma_ok = pl->sR >= 1 && d_img <= kBwdColGradCap && plane_out <= ((size_t)1 << 30) &&
                        (size_t)g.H * g.W <= ((size_t)1 << 30);  // (plane offsets held in 32 bits)
+  pl->fused = pl->fused && mfma_ok;
   if (mfma_ok) {
     pl->gemm = bp->grad_input != nullptr;
     pl->wgemm = bp->grad_weight != nullptr;
@@ -117,7 +137,13 @@ void make_bwd_plan(const mdcn_bwd_params *bp, const Geom &g, uint64_t pass_bytes
     pl->gw_bytes = 0;
     // Workgroups per tile: enough for eight rounds or so of the chip's 2 x CUs slots
     const int passes = g.ch_per_dg / seg * (im.segp / pl->sCH);
-    while (pl->parts < 8 && s_tiles * pl->parts < 4096 && 2 * pl->parts <= passes) pl->parts *= 2;
+    if (pl->fused) {
+      pl->sched.passes = passes;
+      pl->sched.tiles = pl->n_chunk * g.DG * ((g.Ho + (256 >> pl->tw_log) - 1) / (256 >> pl->tw_log)) *
+                        ((g.Wo + (1 << pl->tw_log) - 1) >> pl->tw_log);
+    } else {
+      while (pl->parts < 8 && s_tiles * pl->parts < 4096 && 2 * pl->parts <= passes) pl->parts *= 2;
+    }
     pl->bsplits = 1;
     if (bp->grad_bias) {
       const long runs = (long)g.N * (((long)plane_out + kBiasRun - 1) / kBiasRun);
@@ -127,12 +153,16 @@ void make_bwd_plan(const mdcn_bwd_params *bp, const Geom &g, uint64_t pass_bytes
   }
   if (pl->gemm) {
     pl->cg_tile = (g.taps * im.cgp >= kCgTileBig && plane_out >= (size_t)kCgTileBig) ? kCgTileBig : kCgTile;
-    pl->M_pad = padded(g.taps * im.cgp, pl->cg_tile);
+    pl->M_pad = pl->fused ? g.taps * im.cgp : padded(g.taps * im.cgp, pl->cg_tile);
     pl->gt_bytes = align_up((size_t)g.N * g.G * om.cgp * plane_out * es);
     pl->wt_bytes = align_up((size_t)g.G * pl->M_pad * om.cgp * es);
-    pl->d_bytes = align_up(d_img * pl->n_chunk);
-    pl->mx_bytes = 3 * kAlign;
-    if (pl->parts > 1) pl->part_bytes = align_up((size_t)pl->parts * g.N * g.DG * 3 * g.taps * plane_out * 4);
+    pl->d_bytes = pl->fused ? 0 : align_up(d_img * pl->n_chunk);
+    pl->n_wnorm = pl->fused ? g.G * ((g.cin_g * g.taps + 63) / 64) : 0;
+    pl->mx_bytes = kAlign + align_up((size_t)pl->n_wnorm * 4);
+    if (pl->fused)
+      pl->part_bytes = align_up((size_t)((g.N + pl->n_chunk - 1) / pl->n_chunk) * FusedSchedule::kGroups * 3 * g.taps * 256 * 4);
+    else if (pl->parts > 1)
+      pl->part_bytes = align_up((size_t)pl->parts * g.N * g.DG * 3 * g.taps * plane_out * 4);
   }
   if (pl->wgemm) {
     const long kpx = 128 / (long)es;  // pixels per K step
@@ -285,9 +315,8 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
   float *gin_staging = (float *)take(pl.gin_bytes);
   float *gin32 = staged ? gin_staging : (float *)bp->grad_input;
   float *bpart = (float *)take(pl.gb_bytes);
-  uint32_t *dmax = (uint32_t *)take(pl.mx_bytes);
-  uint32_t *mmax = dmax + kAlign / 4;
-  uint32_t *far = dmax + 2 * kAlign / 4;
+  uint32_t *far = (uint32_t *)take(pl.mx_bytes);
+  uint32_t *wnorm = far + kAlign / 4;
   unsigned char *xt = take(pl.xt_bytes), *gT = take(pl.gt_bytes), *wT = take(pl.wt_bytes);
   unsigned char *D = take(pl.d_bytes), *col = take(pl.col_bytes);
   const long off_total = (long)g.N * g.DG * 2 * g.taps * plane_out, mask_total = off_total / 2;
@@ -296,7 +325,6 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
   float *wpart = (float *)take(pl.wpart_bytes);
   unsigned char *gpad = take(pl.gpad_bytes);
   const long n_in = (long)g.N * g.Cin * g.H * g.W;
-  const int mask_blocks = (int)std::max<long>(1, std::min<long>(mask_total / (256 * EPV), 64));
 
   // a sample of the offsets, 64 Ki of them at most, decides which window the scatter kernel uses
   const long off_step = std::max<long>(1, (off_total >> 16) | 1);
@@ -307,7 +335,7 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
   // 2.5 0.87 / 0.86, 4.0 1.63 / 0.94), half of 8 do: fp16, N=7 C=128 118x196 stride 2, margins 3 and 12: sigma
   // 2.0 0.56 / 0.59, 2.5 0.60 / 0.60, 4.0 0.94 / 0.65.  bf16 in doubles, whole training call in us, N=4 96 -> 72 channels
   // 37x53: sigma 1.0 131 / 132, 2.5 135 / 130, 4.0 154 / 132; N=2 C=128 60x80: 2.0 147 / 153, 3.0 158 / 153, 4.0 195 / 157.
-  const uint32_t far_min = (uint32_t)(off_total / off_step / (pl.sCH * (pl.fixed ? 2 : 4) == 32 ? 32 : 5));
+  const uint32_t far_min = (uint32_t)(off_total / off_step / (pl.fused || pl.sCH == 8 ? 32 : 5));
   auto up = [](long n, long per) { return (int)((n + per - 1) / per); };
   {
     BwdPreArgs a;
@@ -319,7 +347,6 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
     a.in = p->input;
     a.gout = bp->grad_output;
     a.w = p->weight;
-    a.mask = p->mask;
     a.xt = xt;
     a.gT = gT;
     a.wT = wT;
@@ -332,9 +359,7 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
     a.P_pad = pl.P_pad;
     a.col_rows = (long)pl.n_chunk * g.taps * cin_p;
     a.M_pad = pl.M_pad;
-    a.dmax = dmax;
-    a.mmax = mmax;
-    a.n_mask = mask_total;
+    a.wnorm = wnorm;
     a.off = p->offset;
     a.n_off = off_total;
     a.off_step = off_step;
@@ -349,7 +374,7 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
         gemm ? up(n_in, kPreZeroPerBlock) : 0,
         wgemm && pl.P_pad > plane_out ? up(a.col_rows * (pl.P_pad - plane_out), kPrePadPerBlock) : 0,
         gemm ? up((long)g.G * pl.M_pad * pl.om.cgp, 256) : 0,
-        gemm && pl.fixed ? mask_blocks : 0,
+        pl.n_wnorm,
         gemm && pl.fWH ? far_blocks : 0,
         bp->grad_bias ? g.Cout * pl.bsplits : 0,
     };
@@ -360,11 +385,11 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
   }
   for (int n0 = 0; n0 < g.N; n0 += pl.n_chunk) {
     const int nb = std::min(pl.n_chunk, g.N - n0);
-    if (gemm) {
+    if (gemm && !pl.fused) {
       ColGradArgs ca;
       ca.wT = wT;
       ca.gT = gT;
-      ca.D = D;
+      ca.D = (float *)D;
       ca.P = (int)plane_out;
       ca.px_tiles = (int)((plane_out + pl.cg_tile - 1) / pl.cg_tile);
       ca.m_tiles = pl.M_pad / pl.cg_tile;
@@ -378,22 +403,45 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
       ca.Cout = cout_p;
       ca.kslabs = pl.om.cgp / KC;
       ca.n0 = n0;
-      ca.dmax = pl.fixed ? dmax : nullptr;
       ca.total = (long)nb * g.G * ca.px_tiles * ca.m_tiles;
-      auto launch = [&](auto dt) {
-        using DT = decltype(dt);
-        const dim3 grid((unsigned)((ca.total + 7) / 8 * 8));
-        if (pl.cg_tile == kCgTileBig)
-          hipLaunchKernelGGL((bwd_colgrad_kernel<E, DT, kCgTileBig>), grid, dim3(2 * kCgTileBig), 0, st, ca);
-        else
-          hipLaunchKernelGGL((bwd_colgrad_kernel<E, DT, kCgTile>), grid, dim3(2 * kCgTile), 0, st, ca);
-      };
-      if (pl.fixed)
-        launch(E());
+      const dim3 grid((unsigned)((ca.total + 7) / 8 * 8));
+      if (pl.cg_tile == kCgTileBig)
+        hipLaunchKernelGGL((bwd_colgrad_kernel<E, kCgTileBig>), grid, dim3(2 * kCgTileBig), 0, st, ca);
       else
-        launch(0.0f);
+        hipLaunchKernelGGL((bwd_colgrad_kernel<E, kCgTile>), grid, dim3(2 * kCgTile), 0, st, ca);
       check();
     }
+    if (pl.fused) {
+      if constexpr (staged) {
+        BwdFusedArgs fa;
+        fa.g = g;
+        fa.xt = xt;
+        fa.gT = gT;
+        fa.wT = wT;
+        fa.om = om;
+        fa.gin32 = gin32;
+        fa.goff = bp->grad_offset;
+        fa.gmask = bp->grad_mask;
+        fa.col = wgemm ? col : nullptr;
+        fa.P_pad = pl.P_pad;
+        fa.tw_log = pl.tw_log;
+        fa.tiles_x = (g.Wo + (1 << pl.tw_log) - 1) >> pl.tw_log;
+        fa.tiles_y = (g.Ho + (256 >> pl.tw_log) - 1) / (256 >> pl.tw_log);
+        fa.win = ScatterWindow{pl.sR, pl.sWH, pl.sWW};
+        fa.win_far = ScatterWindow{pl.fR, pl.fWH, pl.fWW};
+        fa.far = far;
+        fa.n_far = far_blocks;
+        fa.far_min = far_min;
+        fa.n0 = n0;
+        fa.sched = pl.sched;
+        fa.sched.tiles = pl.sched.tiles / pl.n_chunk * nb;
+        fa.part = poff + (long)(n0 / pl.n_chunk) * FusedSchedule::kGroups * 3 * g.taps * 256;
+        fa.wnorm = wnorm;
+        fa.n_wnorm = pl.n_wnorm;
+        launch_fused<E>(fa, pl.sCH, st);
+        check();
+      }
+    } else {
     BwdScatterArgs sa;
     sa.g = g;
     sa.xt = xt;
@@ -419,38 +467,27 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
     sa.pmask = pmask;
     sa.off_total = off_total;
     sa.mask_total = mask_total;
-    sa.dmax = dmax;
-    sa.mmax = p->mask ? mmax : nullptr;
-    sa.n_mmax = mask_blocks;
     const long sblocks = (long)nb * g.DG * sa.tiles_y * sa.tiles_x;
-    {
-      // 32-bit fixed-point window (needs the maxima the data path computes; a columns-only call adds nothing to the
-      // window) or doubles
-      const dim3 sgrid((unsigned)sblocks, (unsigned)sa.parts);
-      auto launch = [&](auto wt, auto chv) {
-        using WT = decltype(wt);
-        constexpr int CHS = decltype(chv)::value;
-        if (gemm && wgemm)
-          hipLaunchKernelGGL((bwd_scatter_kernel<E, CHS, WT, true, true>), sgrid, dim3(256), 0, st, sa);
-        else if (gemm)
-          hipLaunchKernelGGL((bwd_scatter_kernel<E, CHS, WT, true, false>), sgrid, dim3(256), 0, st, sa);
-        else if constexpr (sizeof(E) == 4 || sizeof(WT) == 4)  // (16-bit columns alone: always `fixed`)
-          hipLaunchKernelGGL((bwd_scatter_kernel<E, CHS, WT, false, true>), sgrid, dim3(256), 0, st, sa);
-      };
-      if constexpr (sizeof(E) == 2) {
-        if (pl.fixed && pl.sCH == 16)
-          launch(int32_t(), std::integral_constant<int, 16>());
-        else if (pl.fixed)
-          launch(int32_t(), std::integral_constant<int, 8>());
-      }
-      if (!pl.fixed) {
-        if (pl.sCH == 8)
-          launch(double(), std::integral_constant<int, 8>());
+    const dim3 sgrid((unsigned)sblocks, (unsigned)sa.parts);
+    auto launch = [&](auto chv) {
+      constexpr int CHS = decltype(chv)::value;
+      if (!gemm) {
+        if constexpr (staged || CHS <= 8) hipLaunchKernelGGL((bwd_scatter_kernel<E, CHS, false, true>), sgrid, dim3(256), 0, st, sa);
+      } else if constexpr (CHS <= 8) {
+        if (wgemm)
+          hipLaunchKernelGGL((bwd_scatter_kernel<E, CHS, true, true>), sgrid, dim3(256), 0, st, sa);
         else
-          launch(double(), std::integral_constant<int, 4>());
+          hipLaunchKernelGGL((bwd_scatter_kernel<E, CHS, true, false>), sgrid, dim3(256), 0, st, sa);
       }
-    }
+    };
+    if (pl.sCH == 16)
+      launch(std::integral_constant<int, 16>());
+    else if (pl.sCH == 8)
+      launch(std::integral_constant<int, 8>());
+    else
+      launch(std::integral_constant<int, 4>());
     check();
+    }
     if (wgemm) {
       WGradArgs wa;
       wa.gout = pl.gpad_bytes ? (const void *)gpad : bp->grad_output;
@@ -507,9 +544,22 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
     a.bpart = bpart;
     a.gb = bp->grad_bias;
     a.bsplits = pl.bsplits;
+    a.fpart = poff;
+    a.tw_log = pl.tw_log;
+    a.n_chunk = pl.n_chunk;
+    a.chunks = pl.fused ? (g.N + pl.n_chunk - 1) / pl.n_chunk : 0;
+    a.sched = a.sched_last = pl.sched;
+    a.sched_last.tiles = pl.sched.tiles / pl.n_chunk * (g.N - (a.chunks - 1) * pl.n_chunk);
+    auto cut_tiles = [](const FusedSchedule &sc) {
+      int n = 0;
+      for (int x = 0; x < FusedSchedule::kXcds; ++x) n += sc.shares(x) > 1 ? sc.rest(x) : 0;
+      return n;
+    };
+    a.cut = cut_tiles(a.sched);
+    a.cut_last = cut_tiles(a.sched_last);
     const int jobs[kFinJobs] = {
         gemm && staged ? up(n_in, 1024) : 0,
-        gemm && pl.parts > 1 ? up(off_total, 1024) : 0,
+        pl.fused ? ((a.chunks - 1) * a.cut + a.cut_last) * 3 * g.taps : gemm && pl.parts > 1 ? up(off_total, 1024) : 0,
         gemm && pl.parts > 1 && bp->grad_mask ? up(mask_total, 1024) : 0,
         wgemm ? g.Cout * up(pl.im.cgp, kFinWeightCh) : 0,
         bp->grad_bias ? up(g.Cout, 256) : 0,

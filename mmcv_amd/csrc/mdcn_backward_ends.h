@@ -6,20 +6,20 @@
 // each some four microseconds on the device and as much on the host.
 #pragma once
 
-#include "mdcn_backward_gemm.h"
+#include "mdcn_backward_fused.h"
 #include "mdcn_prepass.h"
 
 namespace mdcn {
 
 constexpr int kPreJobs = 9;
-enum { kPreX, kPreG, kPreRows, kPreZero, kPreColPad, kPreWeight, kPreMask, kPreFar, kPreBias };
+enum { kPreX, kPreG, kPreRows, kPreZero, kPreColPad, kPreWeight, kPreNorm, kPreFar, kPreBias };
 
 struct BwdPreArgs {
   Geom g;
   ChanMap im, om;          // padded orders of the input and output channels
   int cin_p, cout_p;
   int end[kPreJobs];       // job j has the blocks from end[j - 1] on
-  const void *in, *gout, *w, *mask;
+  const void *in, *gout, *w;
   void *xt, *gT, *wT, *gpad, *col;
   float *gin32;
   long n_in;               // elements of gin32
@@ -27,9 +27,7 @@ struct BwdPreArgs {
   long P_pad;
   long col_rows;           // rows of col whose padding is cleared
   int M_pad;
-  uint32_t *dmax;          // cleared
-  uint32_t *mmax;          // one value per block of the mask job, the bit pattern of a float >= 0
-  long n_mask;
+  uint32_t *wnorm;         // bound on the norm of 64 rows of the weight matrix, one per block of the job
   const void *off;
   long n_off, off_step;    // one offset in off_step is looked at
   float far_from;          // ... and counted when it is larger than this
@@ -93,12 +91,13 @@ __global__ __launch_bounds__(256) void bwd_prepass_kernel(BwdPreArgs a) {
     }
     return;
   }
-  if (b < a.end[kPreColPad]) {  // padding columns [P, P_pad) of the rows of the columns matrix
-    const int padn = (int)(a.P_pad - plane);
+  if (b < a.end[kPreColPad]) {  // padding pixels [P, P_pad) of the columns matrix: of its rows, or of runs of 16 of them
+    constexpr int RUN = sizeof(E) == 2 ? 16 : 1;
+    const int padn = (int)(a.P_pad - plane) * RUN;
     const long i0 = (long)(b - a.end[kPreZero]) * kPrePadPerBlock;
     for (int k = 0; k < kPrePadPerBlock / 256; ++k) {
       const long i = i0 + k * 256 + tid, r = i / padn;
-      if (r < a.col_rows) ((E *)a.col)[r * a.P_pad + plane + (i - r * padn)] = from_f32<E>(0.0f);
+      if (r < a.col_rows / RUN) ((E *)a.col)[(r * a.P_pad + plane) * RUN + (i - r * padn)] = from_f32<E>(0.0f);
     }
     return;
   }
@@ -123,34 +122,40 @@ __global__ __launch_bounds__(256) void bwd_prepass_kernel(BwdPreArgs a) {
     return;
   }
   __shared__ float red[4];
-  if (b < a.end[kPreMask]) {  // largest |mask|, a share per block (as bits, so that infinity and NaN are the largest)
-    const int nb = a.end[kPreMask] - a.end[kPreWeight], bi = b - a.end[kPreWeight];
-    if (bi == 0 && tid == 0) *a.dmax = 0u;
-    const E *x = (const E *)a.mask;
+  if (b < a.end[kPreNorm]) {  // bound on the norms over the output channels of a group of 64 (channel, tap)
+    __shared__ float sq[256];
+    __shared__ uint32_t big[256];
+    const int L = g.cin_g * g.taps, runs = (L + 63) / 64;
+    const int bi = b - a.end[kPreWeight], grp = bi / runs;
+    const int q = (bi - grp * runs) * 64 + (tid & 63);
+    float ss = 0.0f;
     uint32_t mx = 0u;
-    auto raise = [&](E v) { mx = max(mx, __float_as_uint(to_f32(v)) & 0x7fffffffu); };
-    if (x) {
-      const long nv = ((uintptr_t)x % 16) == 0 ? a.n_mask / EPV : 0;
-      for (long v = (long)bi * 256 + tid; v < nv; v += (long)nb * 256) {
-        const uint4 q = ((const uint4 *)x)[v];
-        const E *e = (const E *)&q;
-#pragma unroll
-        for (int i = 0; i < EPV; ++i) raise(e[i]);
+    if (q < L) {
+      const E *src = (const E *)a.w + (long)grp * g.cout_g * L + q;
+#pragma unroll 8
+      for (int co = tid >> 6; co < g.cout_g; co += 4) {
+        const float v = to_f32(src[(long)co * L]);
+        ss = fmaf(v, v, ss);
+        mx = max(mx, __float_as_uint(v) & 0x7fffffffu);
       }
-      for (long i = nv * EPV + (long)bi * 256 + tid; i < a.n_mask; i += (long)nb * 256) raise(x[i]);
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) mx = max(mx, (uint32_t)__shfl_xor((int)mx, o));
-    if ((tid & 63) == 0) red[tid >> 6] = __uint_as_float(mx);
+    sq[tid] = ss;
+    big[tid] = mx;
     __syncthreads();
-    if (tid == 0) {
-      for (int w = 0; w < 4; ++w) mx = max(mx, __float_as_uint(red[w]));
-      a.mmax[bi] = mx;
+    if (tid < 64) {
+      for (int w = 1; w < 4; ++w) {
+        ss += sq[w * 64 + tid];
+        mx = max(mx, big[w * 64 + tid]);
+      }
+      uint32_t nb = norm_bound(ss, mx, g.cout_g);
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) nb = max(nb, (uint32_t)__shfl_xor((int)nb, o));
+      if (tid == 0) a.wnorm[bi] = nb;
     }
     return;
   }
   if (b < a.end[kPreFar]) {  // offsets that leave the scatter kernel's window, counted in a sample
-    const int nb = a.end[kPreFar] - a.end[kPreMask], bi = b - a.end[kPreMask];
+    const int nb = a.end[kPreFar] - a.end[kPreNorm], bi = b - a.end[kPreNorm];
     float cnt = 0.0f;  // (64 Ki samples at most: exact)
     for (long i = ((long)bi * 256 + tid) * a.off_step; i < a.n_off; i += (long)nb * 256 * a.off_step)
       cnt += fabsf(to_f32(((const E *)a.off)[i])) > a.far_from ? 1.0f : 0.0f;
@@ -203,6 +208,10 @@ struct BwdFinArgs {
   void *goff, *gmask;
   long off_total, mask_total;
   int parts;
+  // fused: cut tiles of each pass of images, `cut` of the first and cut_last of the last
+  FusedSchedule sched, sched_last;
+  const float *fpart;   // [pass][workgroup][3 taps][256]
+  int tw_log, n_chunk, chunks, cut, cut_last;
   const float *wpart;   // [splits][G][cout_g][taps * im.cgp]
   void *gw;
   int splits;
@@ -243,6 +252,12 @@ __global__ __launch_bounds__(256) void bwd_finish_kernel(BwdFinArgs a) {
   const int b = (int)blockIdx.x;
   if (b < a.end[kFinInput]) {
     sum_parts_block<E>(a.gin32, (E *)a.gin, a.n_in, 1, b);
+    return;
+  }
+  if (b < a.end[kFinOffset] && a.chunks > 0) {
+    const int bi = b - a.end[kFinInput], per = a.cut * 3 * g.taps, c = per ? min(bi / per, a.chunks - 1) : a.chunks - 1;
+    fused_sums_block<E>(g, c == a.chunks - 1 ? a.sched_last : a.sched, a.tw_log, c * a.n_chunk,
+                        a.fpart + (long)c * FusedSchedule::kGroups * 3 * g.taps * 256, (E *)a.goff, (E *)a.gmask, bi - c * per);
     return;
   }
   if (b < a.end[kFinOffset]) {

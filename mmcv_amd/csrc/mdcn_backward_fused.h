@@ -1,0 +1,679 @@
+// Backward, data side, of 16-bit tensors in one kernel: the column gradient
+// d[pixel, (tap, c)] = sum_co grad_output[co, pixel] * weight[co, c, tap] comes
+// out of the matrix cores into registers and is used there -- for the offset and
+// mask gradients, for grad_input through a window in LDS, beside the sampling of
+// the forward's columns for the weight gradient (the reference's first GEMM and
+// its three element-wise kernels, mmcv/ops/csrc/pytorch/modulated_deform_conv.cpp:199-206,
+// cpu/modulated_deform_conv.cpp:34-107,170-320).  d never exists in memory and is
+// never rounded to 16 bits.
+#pragma once
+
+#include "mdcn_backward_gemm.h"
+
+namespace mdcn {
+
+constexpr int kBfThreads = 512, kBfWaves = kBfThreads / 64;
+constexpr int kBfItems = (kBwdTapsMax + 1) / 2;     // pairs of taps
+constexpr int kBfK = 128;                           // of K at a time
+// Blocks of products of a pass of CH channels, bytes of LDS of a stage of weights (32 rows a block, kBfK of K; two stages are
+// held) and pixels of the window beside them.
+constexpr int bf_blocks(int ch) { return (kBfItems * ch + 15) / 16; }
+constexpr int bf_stage_bytes(int ch) { return bf_blocks(ch) * 32 * kBfK * 2; }
+constexpr int kBfLdsBytes = 163072;
+constexpr int bf_window_px(int ch) { return (kBfLdsBytes - 2 * bf_stage_bytes(ch)) / (4 * ch); }
+constexpr float kRoundMagic = 12582912.0f;          // 1.5 * 2^23: adding it leaves an integer in the mantissa
+constexpr uint32_t kRoundBits = 0x4B400000u;        // ... on top of these bits
+
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+
+struct BwdFusedArgs {
+  Geom g;
+  const void *xt;   // zero-bordered input copy in 32-byte records [N][Cin / 16][H + 2][W + 2][16]
+  const void *gT;   // grad_output, pixel major [N][Cout / 64][P][64]
+  const void *wT;   // [G][taps * cin_g][cout_g], row tap * cin_g + channel
+  OffMaskView om;   // (dense tensors: logit is kMaskPlain or kMaskNone)
+  float *gin32;
+  void *goff;
+  void *gmask;      // null when unmodulated
+  void *col;        // columns of the pass [image][Cin / 16][taps][P_pad][16], or null
+  long P_pad;
+  int tw_log;       // a tile of 256 pixels is 1 << tw_log wide (16 or 32)
+  int tiles_x, tiles_y;
+  ScatterWindow win, win_far;   // (win_far.WH = 0: none)
+  const uint32_t *far;          // counts of sampled offsets beyond win's margin; above far_min in all, win_far is used
+  int n_far;
+  uint32_t far_min;
+  int n0;           // first image of the pass
+  FusedSchedule sched;
+  float *part;      // [workgroup][3 taps][256]: sums of the offset (y and x of a tap) and mask gradients of a share of a tile
+  const uint32_t *wnorm;   // bounds on the norm of a row of wT, as bits; n_wnorm of them
+  int n_wnorm;
+};
+
+// An upper bound of the 2-norm of k numbers whose squares add up to `ss` and whose largest has the bits `mx`; infinite or
+// NaN if one of them is.  (Squares outside of fp32's range: the largest times the root of their number.)
+__device__ __forceinline__ uint32_t norm_bound(float ss, uint32_t mx, int k) {
+  const float m = __uint_as_float(mx);
+  const bool plain = m > 1e-15f && m < 1e15f;
+  return __float_as_uint(1.0005f * (plain ? sqrtf(ss) : m * sqrtf((float)k)));
+}
+
+// One tile of 256 output pixels (tile b), channels [c_first, c_last) of its deformable group; part: where the sums of a share go,
+// or null.  Eight wavefronts, 32 pixels each.  Per pass of CH channels:
+//
+// Products: blocks of 32 rows of weights -- two taps of 16 channels, or four of 8 -- times the wavefront's 32 pixels, K in chunks
+// of 128.  The weights of a pass go to LDS for all wavefronts (two chunks; copied during the scatter of the pass before), rows in
+// an order that gives a lane consecutive channels of one (pixel, tap) of the result.  grad_output comes in registers, 16
+// bytes a lane and 16 of K, each chunk loaded into the registers of the one before.
+// Scatter: a lane takes its pixel's taps of one parity, 8 channels at a time, their corners loaded two such units ahead.
+// Every wait in it is for loads that are due: whatever the compiler keeps in scratch or fetches from the argument block
+// again there makes it wait for all loads, or all LDS adds, under way (the kernel took 2.1 ms in the shape below with either,
+// 1.35 without).  Hence the asm statements without text below: they hold a sum where it is, and a value in its register.
+// Window: 32-bit fixed point in LDS.  Its scale comes from bounds this workgroup takes itself -- |d| is at most the norm of
+// the pixel's grad_output times that of a row of weights -- so that no sum of contributions leaves 2^30 and no
+// contribution 2^21.  What is added to an entry is the bit pattern of fmaf(weight, d, 1.5 * 2^23), for two channels at
+// once: every tap of every pixel adds to four entries, the same ones for all channels, so the number of adds an entry has
+// seen is known from a count made once per tile, and what the patterns hold beside the integers is subtracted when the entry is
+// read.  (Two instructions per channel and corner, where taking it off each contribution was six per two.)  Where grad_output,
+// weights or mask are not finite, or so small or large that no scale fits, nothing goes through the window.
+// Samples beyond the window are added to memory one at a time, a lane for every channel and corner.
+//
+// bf16, N=16, 256 -> 256 channels, 100x152: 1.35 ms for what took 0.52 (column gradient to memory) + 1.50 (scatter kernel reading
+// it); a pass takes a CU 43 thousand clocks: 22 scatter (VALU busy in 17, LDS adds 18), 7 products (MFMA 5), 7 flush, the rest
+// waits at the three barriers.
+template <typename E, int CH, bool DEEP>
+__device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterWindow &wd, int b, int c_first, int c_last, float *part, uint4 *lds,
+                                           float *red) {
+  using TR = ElemTraits<E>;
+  constexpr int NP = CH / 2;
+  constexpr int PLANE = bf_window_px(CH);
+  constexpr int PER = 16 / CH;                        // items per block of products
+  constexpr int U = CH / 8;                           // units of 8 channels an item has
+  constexpr int LA = 2 / U;                           // items between a unit and the loads for it
+  constexpr int kBlocks = bf_blocks(CH);
+  constexpr int kStage = bf_stage_bytes(CH);
+  constexpr int kSlots = (PLANE + kBfThreads - 1) / kBfThreads;
+  uint4 *wst = lds;
+  unsigned long long *win = (unsigned long long *)(lds + 2 * kStage / 16);
+  const Geom &g = a.g;
+  const long plane_out = (long)g.Ho * g.Wo, plane_in = (long)g.H * g.W, slab_px = (long)g.Hp * g.Wp;
+  int tid = threadIdx.x, lane = tid & 63, frow = lane & 31, half = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tx = b % a.tiles_x;
+  b /= a.tiles_x;
+  const int ty = b % a.tiles_y;
+  b /= a.tiles_y;
+  const int dgi = b % g.DG, nl = b / g.DG;
+  const int n = a.n0 + nl;
+  const int TW = 1 << a.tw_log, TH = 256 >> a.tw_log;
+  const int ho = ty * TH + ((wave * 32 + frow) >> a.tw_log), wo = tx * TW + (frow & (TW - 1));
+  const bool valid = ho < g.Ho && wo < g.Wo;
+  const long pix = (long)min(ho, g.Ho - 1) * g.Wo + min(wo, g.Wo - 1);   // (lanes past the image: any pixel of it)
+  const int wy0 = ty * TH * g.sh - g.ph - wd.R, wx0 = tx * TW * g.sw - g.pw - wd.R;
+  int WW = wd.WW, WH = wd.WH;
+  asm volatile("" : "+s"(WW), "+s"(WH));   // (kept: fetched again for every use, each wait for one would be for all LDS adds)
+  const int win_px = WH * WW;
+  const uint32_t inv_ww = (1u << 22) / (uint32_t)WW + 1u;   // k / WW = k * inv_ww >> 22 for every pixel k of a window
+
+  // This lane's taps 2 i + half: offsets, mask and place in the kernel
+  uint32_t t_off[kBfItems], t_m[kBfItems];   // dy | dx << 16; mask | row << 16 | column << 24, a row of 255: no such tap
+  {
+    const E *off = (const E *)a.om.off + (long)n * a.om.off_n + pix * a.om.off_px + (long)(dgi * 2 * g.taps) * a.om.off_ch;
+    const E *msk = (const E *)a.om.msk + (long)n * a.om.msk_n + pix * a.om.msk_px + (long)(dgi * g.taps) * a.om.msk_ch;
+    int row = 0, col = 0;
+    auto tap_at = [&](int tap) {   // (one after the other)
+      const uint32_t at = tap < g.taps ? (uint32_t)(row * g.dh) | (uint32_t)(col * g.dw) << 8 : 255u;
+      if (++col == g.kw) {
+        col = 0;
+        ++row;
+      }
+      return at;
+    };
+#pragma unroll
+    for (int i = 0; i < kBfItems; ++i) {
+      const int tap = 2 * i + half, tc = min(tap, g.taps - 1);
+      const uint32_t at0 = tap_at(2 * i), at1 = tap_at(2 * i + 1);
+      t_off[i] = (uint32_t)__builtin_bit_cast(uint16_t, off[(long)(2 * tc) * a.om.off_ch]) |
+                 (uint32_t)__builtin_bit_cast(uint16_t, off[(long)(2 * tc + 1) * a.om.off_ch]) << 16;
+      t_m[i] = (uint32_t)__builtin_bit_cast(uint16_t, msk[(long)tc * a.om.msk_ch]) | (half ? at1 : at0) << 16;
+    }
+  }
+  float *lone = red + 3 * kBfWaves + wave * 16;   // of this wavefront
+  const int items = (g.taps + 1) / 2, blocks = (items + PER - 1) / PER;
+
+  // (1: unmodulated)
+  auto mask_of = [&](int i) { return a.om.logit == kMaskNone ? 1.0f : to_f32(__builtin_bit_cast(E, (uint16_t)t_m[i])); };
+  auto has_tap = [&](int i) { return ((t_m[i] >> 16) & 255u) != 255u; };
+  int base_y = ho * g.sh - g.ph, base_x = wo * g.sw - g.pw;
+  struct Place {
+    int y0, x0;
+    float ly, lx;
+    bool inside;
+  };
+  auto place = [&](int i) {
+    Place p;
+    float dy, dx;
+    TR::unpack2(t_off[i], dy, dx);
+    const int row = (int)(t_m[i] >> 16) & 255;
+    const float py = (float)(base_y + row) + dy;
+    const float px = (float)(base_x + (int)(t_m[i] >> 24)) + dx;
+    p.inside = valid && row != 255 && py > -1.0f && px > -1.0f && py < (float)g.H && px < (float)g.W;
+    const float fy = floorf(py), fx = floorf(px);
+    p.y0 = p.inside ? (int)fy : -1;
+    p.x0 = p.inside ? (int)fx : -1;
+    p.ly = p.inside ? py - fy : 0.0f;
+    p.lx = p.inside ? px - fx : 0.0f;
+    return p;
+  };
+
+  // Passes of CH channels each.  (The copies hold the tensors' own channels; a pass lies in one group.)
+  const int c_begin = dgi * g.ch_per_dg + c_first, c_end = dgi * g.ch_per_dg + c_last;
+  auto group_of = [&](int c0) { return g.G == 1 ? 0 : c0 / g.cin_g; };
+
+  // Copies of a stage of weights: 32 rows a block, 128 (or what is left: 64) of K, pieces of 16 bytes swizzled by the row.  Chunk kh of K goes to buffer
+  // kh % 2.
+  const int nkh = (g.cout_g + kBfK - 1) / kBfK;
+  const uint32_t lds_w = (uint32_t)(uintptr_t)(lptr_t)wst + (uint32_t)wave * 1024u;
+  auto issue = [&](int c0, int kh) {
+    const int sh = g.cout_g - kh * kBfK >= kBfK ? 4 : 3;
+    const int grp = group_of(c0);
+    const unsigned char *base = (const unsigned char *)a.wT +
+                                (((long)grp * g.taps * g.cin_g + (c0 - grp * g.cin_g)) * g.cout_g + kh * kBfK) * 2;
+    const int copies = blocks << (sh - 1);   // of 1 KiB
+    const uint32_t lds = (uint32_t)__builtin_amdgcn_readfirstlane((int)(lds_w + (uint32_t)(kh & 1) * (uint32_t)kStage));
+#pragma unroll
+    for (int c = 0; c < 8 * kBlocks / kBfWaves; ++c) {
+      if (wave + kBfWaves * c < copies) {
+        const uint32_t u = (uint32_t)((wave + kBfWaves * c) * 64 + lane);
+        const uint32_t row = u >> sh, s = u - (row << sh);
+        const int blk = (int)(row >> 5), r8 = (int)(row >> 3) & 3, hh = (int)(row >> 2) & 1, r4 = (int)row & 3;
+        // result register 4 * r8 + r4 of the lanes of half hh
+        const int tap = min(PER * 2 * blk + (PER == 2 ? 2 * (r8 >> 1) : 0) + hh, g.taps - 1);
+        const int ch = 4 * (PER == 2 ? r8 & 1 : r8) + r4;
+        copy16_global_to_lds(base + (uint32_t)((tap * g.cin_g + ch) * g.cout_g) * 2u + ((s ^ (row & 7u)) * 16u),
+                             lds + (uint32_t)c * (kBfWaves * 1024u));
+      }
+    }
+  };
+  // This lane's grad_output of chunk kh of K, the products' second operand: j-th 16 of it (j < 4, or < 8 where the chunk is whole)
+  const unsigned char *gpx = (const unsigned char *)a.gT + ((long)n * (g.Cout / 64) * plane_out + pix) * 128 + half * 16;
+  auto whole_chunk = [&](int kh) { return g.cout_g - kh * kBfK >= kBfK; };
+  auto g_at = [&](int grp, int kh, int j) {
+    return *(const uint4 *)(gpx + ((long)(grp * (g.cout_g / 64) + kh * 2 + j / 4) * plane_out) * 128 + j % 4 * 32);
+  };
+  uint4 gf[8];
+  auto load_g = [&](int grp, int kh) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) gf[j] = g_at(grp, kh, j);
+    if (whole_chunk(kh)) {
+#pragma unroll
+      for (int j = 4; j < 8; ++j) gf[j] = g_at(grp, kh, j);
+    }
+  };
+  // the first two stages of a pass
+  auto issue_first = [&](int c0) {
+    issue(c0, 0);
+    if (nkh > 1) issue(c0, 1);
+  };
+  issue_first(c_begin);
+
+  // Bounds and scale.  (The barrier also ends the tile before: nobody is at the window any more.)
+  __syncthreads();
+  const int grp0 = group_of(c_begin), grp1 = group_of(c_end - 1);
+  bool fits;
+  float scale, inv_scale;
+  {
+    uint32_t norm = 0u;
+    for (int grp = grp0; grp <= grp1; ++grp) {
+      float ss = 0.0f;
+      u16x2 big = {0, 0};   // largest magnitudes, as bits
+#pragma unroll 1
+      for (int k = 0; k < g.cout_g / 64; ++k) {
+        uint4 v[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = g_at(grp, k / 2, k % 2 * 4 + j);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const uint32_t w[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            ss = TR::dot2(w[q], w[q], ss);
+            const u16x2 m = __builtin_bit_cast(u16x2, w[q] & 0x7fff7fffu);
+            big = __builtin_elementwise_max(big, m);
+          }
+        }
+      }
+      uint32_t mx = __float_as_uint(to_f32(__builtin_bit_cast(E, max(big.x, big.y))));
+      ss += __shfl_xor(ss, 32);
+      mx = max(mx, (uint32_t)__shfl_xor((int)mx, 32));
+      norm = max(norm, norm_bound(ss, mx, g.cout_g));
+    }
+    load_g(grp0, 0);
+    float msum = 0.0f;
+    uint32_t mmax = 0u;
+#pragma unroll
+    for (int i = 0; i < kBfItems; ++i) {
+      const float m = has_tap(i) ? fabsf(mask_of(i)) : 0.0f;
+      msum += m;
+      mmax = max(mmax, __float_as_uint(m));
+    }
+    msum += __shfl_xor(msum, 32);
+    mmax = max(mmax, (uint32_t)__shfl_xor((int)mmax, 32));
+    float all = valid ? __uint_as_float(norm) * msum : 0.0f;
+    uint32_t one = __float_as_uint(valid ? __uint_as_float(norm) * __uint_as_float(mmax) : 0.0f);
+    mmax = valid ? mmax : 0u;
+#pragma unroll
+    for (int o = 16; o > 0; o >>= 1) {
+      all += __shfl_xor(all, o);
+      one = max(one, (uint32_t)__shfl_xor((int)one, o));
+      mmax = max(mmax, (uint32_t)__shfl_xor((int)mmax, o));
+    }
+    uint32_t wn = 0u;
+    for (int i = lane; i < a.n_wnorm; i += 64) wn = max(wn, a.wnorm[i]);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) wn = max(wn, (uint32_t)__shfl_xor((int)wn, o));
+    if (lane == 0) {
+      red[wave * 3] = all;
+      red[wave * 3 + 1] = __uint_as_float(one);
+      red[wave * 3 + 2] = __uint_as_float(mmax);
+    }
+    // (the counts of adds go where the window will be)
+    for (int i = tid; i < win_px; i += kBfThreads) ((uint32_t *)win)[i] = 0u;
+    __syncthreads();
+    all = 0.0f;
+    one = mmax = 0u;
+#pragma unroll
+    for (int w = 0; w < kBfWaves; ++w) {
+      all += red[w * 3];
+      one = max(one, __float_as_uint(red[w * 3 + 1]));
+      mmax = max(mmax, __float_as_uint(red[w * 3 + 2]));
+    }
+    all *= __uint_as_float(wn);
+    const float top = __uint_as_float(one) * __uint_as_float(wn);
+    const int e = (all > 0.0f && all < 3.0e38f) ? min(29 - ilogbf(all), top > 0.0f ? 20 - ilogbf(top) : 120) : 0;
+    scale = __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint(ldexpf(1.0f, min(120, e)))));
+    inv_scale = 1.0f / scale;
+    fits = __builtin_amdgcn_readfirstlane(all < 3.0e38f && e <= 120 && __uint_as_float(mmax) * scale < 3.0e38f) != 0;  // (false for NaN)
+  }
+  // (a window that cannot be used has no rows: every sample is beyond it)
+  const int win_h = fits ? WH : 0;
+  auto window_at = [&](const Place &p, bool &in_win) {
+    const int ry = p.y0 - wy0, rx = p.x0 - wx0;
+    in_win = ry >= 0 && ry + 1 < win_h && rx >= 0 && rx + 1 < WW;
+    // a lane with nothing for the window adds its zeros at an entry of its own
+    return p.inside && in_win ? ry * WW + rx : lane;
+  };
+  // How many adds the window pixels that this thread flushes (tid, tid + 512, ...) see in a pass, 16 bits each
+  uint32_t adds[(kSlots + 1) / 2];
+  {
+#pragma unroll
+    for (int i = 0; i < kBfItems; ++i) {
+      if (i < items) {
+        bool in_win;
+        uint32_t *c = (uint32_t *)win + window_at(place(i), in_win);
+        atomicAdd(c, 1u);
+        atomicAdd(c + 1, 1u);
+        atomicAdd(c + WW, 1u);
+        atomicAdd(c + WW + 1, 1u);
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kSlots; ++j) {
+      const int q = tid + kBfThreads * j;
+      const uint32_t c = q < win_px ? ((const uint32_t *)win)[q] : 0u;
+      adds[j / 2] = j % 2 ? adds[j / 2] | c << 16 : c;
+    }
+    __syncthreads();
+    for (int i = tid; i < PLANE * NP / 2; i += kBfThreads) ((uint4 *)win)[i] = make_uint4(0u, 0u, 0u, 0u);
+  }
+
+  // Corners of 8 channels of an item, loaded one unit of work ahead: first channel c0 of the pass, half h of its channels
+  struct Corners {
+    VecCh<E, 8> r00, r01, r10, r11;
+  };
+  auto fetch = [&](int c0, const Place &p, int h, Corners &s) {
+    // corners outside the image read the copy's zero border
+    const E *xp = (const E *)a.xt + (((long)n * (g.Cin / 16) + c0 / 16) * slab_px) * 16 + (c0 % 16) + h * 8 +
+                  ((long)(p.y0 + 1) * g.Wp + (p.x0 + 1)) * 16;
+    s.r00.load(xp);
+    s.r01.load(xp + 16);
+    s.r10.load(xp + (long)g.Wp * 16);
+    s.r11.load(xp + (long)(g.Wp + 1) * 16);
+  };
+
+  float acc_m[kBfItems], acc_y[kBfItems], acc_x[kBfItems];
+#pragma unroll
+  for (int i = 0; i < kBfItems; ++i) acc_m[i] = acc_y[i] = acc_x[i] = 0.0f;
+
+  // every copy of a stage has landed, and every wavefront is past whatever it did before
+  auto settle = [&]() {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+  };
+  f32x16 d[kBlocks];
+  // Products of chunk kh of K; the next chunk's grad_output is loaded into the registers of what has been used.
+  auto products = [&](int grp, int kh) {
+    const bool more = kh + 1 < nkh;
+    const int pitch = whole_chunk(kh) ? 16 : 8;
+    const uint4 *w0 = wst + (kh & 1) * (kStage / 16) + frow * pitch;
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      if (s == 0 || whole_chunk(kh)) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const uint4 *wj = w0 + 8 * s + ((2 * j + half) ^ (frow & 7));
+          uint4 f[kBlocks];
+#pragma unroll
+          for (int blk = 0; blk < kBlocks; ++blk) f[blk] = wj[blk * 32 * pitch];
+#pragma unroll
+          for (int blk = 0; blk < kBlocks; ++blk) TR::mma(d[blk], f[blk], gf[4 * s + j]);
+        }
+        // fragments are read three products ahead of theirs
+        __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
+#pragma unroll
+        for (int j = 0; j < 4 * kBlocks - 3; ++j) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x008, 3, 0);
+        if (more && (s == 0 || whole_chunk(kh + 1))) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) gf[4 * s + j] = g_at(grp, kh + 1, 4 * s + j);
+        }
+      }
+    }
+  };
+  // All of a pass's products; the first two stages are in LDS.
+  auto products_of = [&](int c0) {
+    const int grp = group_of(c0);
+#pragma unroll
+    for (int blk = 0; blk < kBlocks; ++blk)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) d[blk][r] = 0.0f;
+    products(grp, 0);
+    if (nkh > 1) products(grp, 1);
+    if constexpr (DEEP) {
+      for (int kh = 2; kh < nkh; kh += 2) {
+        __syncthreads();   // nobody reads the stages any more
+        issue(c0, kh);
+        if (kh + 1 < nkh) issue(c0, kh + 1);
+        settle();
+        products(grp, kh);
+        if (kh + 1 < nkh) products(grp, kh + 1);
+      }
+    }
+    // (No load is under way here.  The compiler, which follows each branch above by itself, is told so, or it waits for
+    // whatever is under way at the next use of these registers.)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) asm volatile("" : "+v"(gf[j].x), "+v"(gf[j].y), "+v"(gf[j].z), "+v"(gf[j].w));
+  };
+  // Adds what the window holds of the CH channels from cf on to grad_input, and clears it.
+  auto flush = [&](int cf) {
+    float *gplane = a.gin32 + ((long)n * g.Cin + cf) * plane_in;
+#pragma unroll
+    for (int j = 0; j < kSlots; ++j) {
+      const uint32_t seen = j % 2 ? adds[j / 2] >> 16 : adds[j / 2] & 0xffffu;
+      if (seen != 0u) {
+        const int k = tid + kBfThreads * j, r = (int)(((uint32_t)k * inv_ww) >> 22);
+        const int y = wy0 + r, x = wx0 + k - r * WW;
+        unsigned long long *e = win + k;
+        unsigned long long v[NP];
+#pragma unroll
+        for (int cp = 0; cp < NP; ++cp) v[cp] = e[cp * PLANE];
+#pragma unroll
+        for (int cp = 0; cp < NP; ++cp) e[cp * PLANE] = 0ull;
+        if (fits && y >= 0 && y < g.H && x >= 0 && x < g.W) {
+          const unsigned long long bias = (unsigned long long)seen * kRoundBits;
+          float *gi = gplane + (y * g.W + x);
+#pragma unroll
+          for (int cp = 0; cp < NP; ++cp, gi += 2 * plane_in) {
+            const long long s = (long long)(v[cp] - (bias + (bias << 32)));
+            const int lo = (int)(uint32_t)s, hi = (int)((s - (long long)lo) >> 32);
+            unsafeAtomicAdd(gi, (float)lo * inv_scale);
+            unsafeAtomicAdd(gi + plane_in, (float)hi * inv_scale);
+          }
+        }
+      }
+    }
+  };
+  settle();
+  for (int c0 = c_begin; c0 < c_end; c0 += CH) {
+    // (Opaque to the optimiser: it would otherwise move what follows from these in every pass -- positions, addresses of
+    // all stages -- out of this loop, and spill it.)
+#pragma unroll
+    for (int i = 0; i < kBfItems; ++i) asm volatile("" : "+v"(t_off[i]), "+v"(t_m[i]));
+#pragma unroll
+    for (int j = 0; j < (kSlots + 1) / 2; ++j) asm volatile("" : "+v"(adds[j]));
+    asm volatile("" : "+v"(lane), "+v"(frow), "+v"(half), "+v"(tid), "+v"(base_y), "+v"(base_x));
+    products_of(c0);
+    Place p[LA + 1];
+#pragma unroll
+    for (int i = 0; i < LA; ++i) p[i] = place(i);
+    Corners q[3];
+    fetch(c0, p[0], 0, q[0]);
+    fetch(c0, p[LA - 1], U - 1, q[1]);
+    if (c0 > c_begin) flush(c0 - CH);   // (behind these loads: a wavefront's loads wait for every add in front of them)
+    __syncthreads();   // the window is zero and the stages are free
+    if (c0 + CH < c_end) issue_first(c0 + CH);
+    __builtin_amdgcn_sched_barrier(0);
+    E *cbase = (E *)a.col + ((((long)nl * (g.Cin / 16) + c0 / 16) * g.taps + half) * a.P_pad + pix) * 16 + c0 % 16;
+#pragma unroll
+    for (int i = 0; i < kBfItems; ++i) {
+      if (i < items) {
+        Place &next = p[(i + LA) % (LA + 1)];
+        const Place c = p[i % (LA + 1)];
+        if (i + LA < kBfItems) next = place(i + LA);
+        const float ly = c.ly, lx = c.lx, hy = 1.0f - ly, hx = 1.0f - lx;
+        const float mk = mask_of(i);
+        const float m = c.inside ? mk : 0.0f;
+        const int y0 = c.y0, x0 = c.x0, y1 = y0 + 1, x1 = x0 + 1;
+        const bool ok00 = y0 >= 0 && x0 >= 0, ok01 = y0 >= 0 && x1 <= g.W - 1;
+        const bool ok10 = y1 <= g.H - 1 && x0 >= 0, ok11 = y1 <= g.H - 1 && x1 <= g.W - 1;
+        const float w00 = hy * hx, w01 = hy * lx, w10 = ly * hx, w11 = ly * lx;
+        bool in_win;
+        const int wbase = window_at(c, in_win);
+        const bool to_win = c.inside && in_win;
+        const float s00 = (to_win && ok00) ? w00 : 0.0f, s01 = (to_win && ok01) ? w01 : 0.0f;
+        const float s10 = (to_win && ok10) ? w10 : 0.0f, s11 = (to_win && ok11) ? w11 : 0.0f;
+        const float mts = m * scale;
+        const float v00 = m * w00, v01 = m * w01, v10 = m * w10, v11 = m * w11;
+        float S00 = 0.0f, S01 = 0.0f, S10 = 0.0f, S11 = 0.0f;
+        if (!fits) {  // (then d may be anything where nothing is sampled; otherwise it is finite and meets zeros there)
+#pragma unroll
+          for (int k = 0; k < CH; ++k)
+            d[i / PER][(i % PER) * CH + k] = c.inside ? d[i / PER][(i % PER) * CH + k] : 0.0f;
+        }
+#pragma unroll
+        for (int h = 0; h < U; ++h) {
+          const Corners &cur = q[(i * U + h) % 3];
+          if (i + LA < kBfItems) fetch(c0, next, h, q[(i * U + h + 2) % 3]);
+          unsigned long long *wp0 = win + h * 4 * PLANE + wbase, *wp1 = wp0 + WW;
+          uint32_t cv[4];
+#pragma unroll
+          for (int cp = 0; cp < 4; ++cp) {
+            const float d0 = d[i / PER][(i % PER) * CH + h * 8 + 2 * cp], d1 = d[i / PER][(i % PER) * CH + h * 8 + 2 * cp + 1];
+            float q00[2], q01[2], q10[2], q11[2];
+            cur.r00.pair(cp, q00[0], q00[1]);
+            cur.r01.pair(cp, q01[0], q01[1]);
+            cur.r10.pair(cp, q10[0], q10[1]);
+            cur.r11.pair(cp, q11[0], q11[1]);
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+              const float dd = e ? d1 : d0;
+              S00 = fmaf(dd, q00[e], S00);
+              S01 = fmaf(dd, q01[e], S01);
+              S10 = fmaf(dd, q10[e], S10);
+              S11 = fmaf(dd, q11[e], S11);
+            }
+            auto column = [&](int e) { return fmaf(v00, q00[e], fmaf(v01, q01[e], fmaf(v10, q10[e], v11 * q11[e]))); };
+            cv[cp] = TR::pack2(column(0), column(1));
+            // (Here and now: the optimiser would move these sums behind the branches below and keep all corners until then.)
+            asm volatile("" : "+v"(cv[cp]), "+v"(S00), "+v"(S01), "+v"(S10), "+v"(S11));
+            const float tl = d0 * mts, th = d1 * mts;
+            auto entry = [&](float w) {
+              return (unsigned long long)__float_as_uint(fmaf(w, tl, kRoundMagic)) |
+                     (unsigned long long)__float_as_uint(fmaf(w, th, kRoundMagic)) << 32;
+            };
+            atomicAdd(wp0 + cp * PLANE, entry(s00));
+            atomicAdd(wp0 + cp * PLANE + 1, entry(s01));
+            atomicAdd(wp1 + cp * PLANE, entry(s10));
+            atomicAdd(wp1 + cp * PLANE + 1, entry(s11));
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          if (a.col && valid && has_tap(i))
+            *(uint4 *)(cbase + (long)(2 * i) * a.P_pad * 16 + h * 8) = make_uint4(cv[0], cv[1], cv[2], cv[3]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        acc_m[i] += w00 * S00 + w01 * S01 + w10 * S10 + w11 * S11;
+        acc_y[i] += m * (hx * (S10 - S00) + lx * (S11 - S01));
+        acc_x[i] += m * (hy * (S01 - S00) + ly * (S11 - S10));
+        // Samples beyond the window go to memory directly, one at a time: a lane for every channel and corner.
+        for (unsigned long long rest = __ballot(c.inside && !in_win); rest != 0ull; rest &= rest - 1ull) {
+          const int l = __ffsll((long long)rest) - 1;
+          if (lane == l) {
+#pragma unroll
+            for (int k = 0; k < CH; ++k) lone[k] = d[i / PER][(i % PER) * CH + k] * m;
+          }
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+          const int fy = __builtin_amdgcn_readlane(c.y0, l), fx = __builtin_amdgcn_readlane(c.x0, l);
+          const float gy = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(c.ly), l));
+          const float gx = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(c.lx), l));
+          const int k = lane % CH, corner = lane / CH;
+          const int yy = fy + (corner >> 1), xx = fx + (corner & 1);
+          const float w = ((corner & 2) ? gy : 1.0f - gy) * ((corner & 1) ? gx : 1.0f - gx);
+          const float t = lone[k];
+          if (corner < 4 && yy >= 0 && yy < g.H && xx >= 0 && xx < g.W)
+            unsafeAtomicAdd(a.gin32 + ((long)n * g.Cin + c0 + k) * plane_in + ((long)yy * g.W + xx), w * t);
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    load_g(group_of(min(c0 + CH, c_end - 1)), 0);
+    // Every add into the window has landed behind this barrier, and so have the copies of the next pass's weights: since them
+    // a wavefront has issued loads of corners for two items or more (8 each) and some of grad_output, or waits for everything.
+    if (items > 2)
+      asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+  }
+  flush(c_end - CH);
+  if (part) {
+    const int px = wave * 32 + frow;
+#pragma unroll
+    for (int i = 0; i < kBfItems; ++i) {
+      const int tap = 2 * i + half;
+      if (tap < g.taps) {
+        part[(2 * tap) * 256 + px] = acc_y[i];
+        part[(2 * tap + 1) * 256 + px] = acc_x[i];
+        part[(2 * g.taps + tap) * 256 + px] = acc_m[i];
+      }
+    }
+  } else if (valid) {
+    const long ob = ((long)n * g.DG + dgi) * 2 * g.taps, mb = ob / 2;
+    E *goff = (E *)a.goff, *gmask = (E *)a.gmask;
+#pragma unroll
+    for (int i = 0; i < kBfItems; ++i) {
+      const int tap = 2 * i + half;
+      if (tap < g.taps) {
+        goff[(ob + 2 * tap) * plane_out + pix] = from_f32<E>(acc_y[i]);
+        goff[(ob + 2 * tap + 1) * plane_out + pix] = from_f32<E>(acc_x[i]);
+        if (gmask) gmask[(mb + tap) * plane_out + pix] = from_f32<E>(acc_m[i]);
+      }
+    }
+  }
+}
+
+// CH channels a pass over the window; CHF when many offsets lie beyond its margin (decided on the device, from a sample of the
+// offsets that the pre-pass has looked at).
+template <typename E, int CH, int CHF, bool DEEP>
+__global__ __launch_bounds__(kBfThreads, 2) void bwd_fused_kernel(BwdFusedArgs a) {
+  __shared__ uint4 lds[kBfLdsBytes / 16];
+  __shared__ float red[(3 + 16) * kBfWaves];
+  bool far = false;
+  if (a.win_far.WH > 0) {
+    uint32_t n = (int)(threadIdx.x & 63) < a.n_far ? a.far[threadIdx.x & 63] : 0u;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o);
+    far = __builtin_amdgcn_readfirstlane((int)n) > (int)a.far_min;
+  }
+  const FusedSchedule &sc = a.sched;
+  const int xcd = blockIdx.x % FusedSchedule::kXcds, j = blockIdx.x / FusedSchedule::kXcds;
+  const int rounds = sc.count(xcd) / FusedSchedule::kPerXcd, rest = sc.rest(xcd);
+  for (int r = 0; r <= rounds; ++r) {
+    int tile = sc.first(xcd) + r * FusedSchedule::kPerXcd + j;
+    int first = 0, last = sc.passes;
+    float *part = nullptr;
+    if (r == rounds) {
+      const int shares = sc.shares(xcd), k = j / shares, share = j - k * shares;
+      if (k >= rest) break;
+      tile += k - j;
+      first = sc.passes * share / shares;
+      last = sc.passes * (share + 1) / shares;
+      if (shares > 1) part = a.part + (long)(xcd * FusedSchedule::kPerXcd + j) * 3 * a.g.taps * 256;
+    }
+    if constexpr (CHF == CH) {
+      fused_tile<E, CH, DEEP>(a, far ? a.win_far : a.win, tile, first * CH, last * CH, part, lds, red);
+    } else {
+      if (far)
+        fused_tile<E, CHF, DEEP>(a, a.win_far, tile, first * CH, last * CH, part, lds, red);
+      else
+        fused_tile<E, CH, DEEP>(a, a.win, tile, first * CH, last * CH, part, lds, red);
+    }
+  }
+}
+
+// Adds up the shares of cut tile `b / (3 taps)` (counted over the XCDs' last rounds), row b % (3 taps) of its sums: one thread a pixel.
+template <typename E>
+__device__ __forceinline__ void fused_sums_block(const Geom &g, const FusedSchedule &sc, int tw_log, int n0, const float *part, E *goff,
+                                                 E *gmask, int b) {
+  const int rows = 3 * g.taps, row = b % rows;
+  int k = b / rows, xcd = 0;
+  while (xcd < FusedSchedule::kXcds - 1 && (sc.shares(xcd) < 2 || k >= sc.rest(xcd))) {
+    if (sc.shares(xcd) > 1) k -= sc.rest(xcd);
+    ++xcd;
+  }
+  const int shares = sc.shares(xcd);
+  const float *p = part + ((long)(xcd * FusedSchedule::kPerXcd + k * shares) * rows + row) * 256 + threadIdx.x;
+  float s = p[0];
+  for (int i = 1; i < shares; ++i) s += p[(long)i * rows * 256];
+  int t = sc.first(xcd) + sc.count(xcd) - sc.rest(xcd) + k;
+  const int TW = 1 << tw_log, TH = 256 >> tw_log, tiles_x = (g.Wo + TW - 1) / TW, tiles_y = (g.Ho + TH - 1) / TH;
+  const int tx = t % tiles_x;
+  t /= tiles_x;
+  const int ty = t % tiles_y;
+  t /= tiles_y;
+  const int ho = ty * TH + ((int)threadIdx.x >> tw_log), wo = tx * TW + ((int)threadIdx.x & (TW - 1));
+  if (ho >= g.Ho || wo >= g.Wo) return;
+  const long nd = (long)n0 * g.DG + t, plane = (long)g.Ho * g.Wo, pix = (long)ho * g.Wo + wo;   // (t: image of the pass, deformable group)
+  if (row < 2 * g.taps)
+    goff[(nd * 2 * g.taps + row) * plane + pix] = from_f32<E>(s);
+  else if (gmask)
+    gmask[(nd * g.taps + row - 2 * g.taps) * plane + pix] = from_f32<E>(s);
+}
+
+// Launches the kernel with ch (16 or 8) channels a pass.  (Defined in a source per element type.)
+template <typename E>
+void launch_fused(const BwdFusedArgs &a, int ch, hipStream_t st);
+template <>
+void launch_fused<bf16_t>(const BwdFusedArgs &a, int ch, hipStream_t st);
+template <>
+void launch_fused<f16_t>(const BwdFusedArgs &a, int ch, hipStream_t st);
+
+template <typename E>
+void launch_fused_impl(const BwdFusedArgs &a, int ch, hipStream_t st) {
+  const dim3 grid(FusedSchedule::kGroups);
+  const bool deep = a.g.cout_g > 2 * kBfK;
+  if (ch == 16 && !deep)
+    hipLaunchKernelGGL((bwd_fused_kernel<E, 16, 8, false>), grid, dim3(kBfThreads), 0, st, a);
+  else if (ch == 16)
+    hipLaunchKernelGGL((bwd_fused_kernel<E, 16, 8, true>), grid, dim3(kBfThreads), 0, st, a);
+  else if (!deep)
+    hipLaunchKernelGGL((bwd_fused_kernel<E, 8, 8, false>), grid, dim3(kBfThreads), 0, st, a);
+  else
+    hipLaunchKernelGGL((bwd_fused_kernel<E, 8, 8, true>), grid, dim3(kBfThreads), 0, st, a);
+}
+
+}  // namespace mdcn

@@ -1,4 +1,5 @@
-// Backward, data side, for channel counts that fill MFMA tiles: the column
+// Backward on the matrix cores, for fp32 tensors and for 16-bit calls of few tiles or uneven channels (the others have
+// bwd_fused_kernel for the data side, and bwd_wgrad_kernel here): the column
 // gradient  d[pixel, (tap, c)] = sum_co grad_output[co, pixel] * weight[co, c, tap]
 // (the reference's first GEMM, mmcv/ops/csrc/pytorch/modulated_deform_conv.cpp:199-206)
 // is a plain matrix product, so it runs on the matrix cores
@@ -6,8 +7,8 @@
 // layout made for that kernel: d[image][16-channel chunk][tap][pixel][16].  The
 // scatter kernel (bwd_scatter_kernel) then is the reference's three element-wise
 // kernels in one pass (cpu/modulated_deform_conv.cpp:34-107,170-320): a thread
-// owns an output pixel, reads 4 to 16 channels of d and of the four corners (from
-// the zero-bordered pixel-major input copy, 16 or 32 contiguous bytes per corner,
+// owns an output pixel, reads 4 or 8 channels of d and of the four corners (from
+// the zero-bordered pixel-major input copy, 8 to 32 contiguous bytes per corner,
 // one tap ahead of their use), forms its share of grad_offset / grad_mask from
 // the four sums of d times a corner's values, and adds the grad_input
 // contributions into an LDS window around its 8 x 32 pixel tile, which is flushed
@@ -44,7 +45,7 @@ struct ColGradArgs {
   // (channel counts are those of the padded orders, see BwdPlan)
   const void *wT;  // [G][M_pad][cout_g]
   const void *gT;  // [N][Cout / KC][P][KC], KC = 128 bytes of channels
-  void *D;         // [images of the pass][Cin / 16][taps][P][16], of the kernel's DT
+  float *D;        // [images of the pass][Cin / 16][taps][P][16]
   int P;           // output pixels per image
   int px_tiles, m_tiles;
   int M, M_pad;    // taps * cin_g and its padded size
@@ -52,7 +53,6 @@ struct ColGradArgs {
   int kslabs;      // cout_g / KC
   int n0;          // first image of the pass
   long total;      // workgroups with work: images of the pass x G x px_tiles x m_tiles
-  uint32_t *dmax;  // bit pattern of the largest |d| stored so far (a float >= 0, infinite or NaN if one is), or null
 };
 
 // A wave's products of one K step of either kernel: TILE / 64 x 2 blocks of 32 x 32 over 128 bytes of K, operand tiles
@@ -148,8 +148,8 @@ __device__ __forceinline__ bool unscale(f32x16 (&acc)[MB][2]) {
 // swizzled by the row number on the source side, so that fragment reads are
 // conflict free), double buffered.  A rows = (tap, channel), B rows = pixels:
 // a lane ends up with 4 x 4 consecutive channels of one pixel, which is what the
-// d layout wants (8- or 16-byte stores).  DT: element of d, E or float.
-template <typename E, typename DT, int TILE>
+// d layout wants (16-byte stores).
+template <typename E, int TILE>
 __global__ __launch_bounds__(TILE * 2, TILE == 128 ? 2 : 1) void bwd_colgrad_kernel(ColGradArgs a) {
   using TR = ElemTraits<E>;
   constexpr int ES = (int)sizeof(E);
@@ -228,32 +228,7 @@ __global__ __launch_bounds__(TILE * 2, TILE == 128 ? 2 : 1) void bwd_colgrad_ker
   }
 
   // register r of lane l: A row (r/4)*8 + (l/32)*4 + r%4 of the block, B row l%32
-  DT *D = (DT *)a.D;
   const int chunks = a.Cin / 16;
-  if (a.dmax) {  // (every accumulator counts: rows and pixels past the end repeat real ones, or are zero times real ones)
-    // Floats of one sign order like their bits, and infinity and NaN lie above all others: the positive ones are the
-    // largest as signed numbers, the negative ones as unsigned numbers.  (Two v_max3 per two elements; clearing
-    // the sign first takes three, 1% of a call of N=16, 256 channels, 100x152.)
-    int pos = 0;
-    uint32_t neg = 0u;
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-      for (int nb = 0; nb < 2; ++nb)
-#pragma unroll
-        for (int r = 0; r < 16; r += 2) {
-          const uint32_t u = __float_as_uint(acc[mb][nb][r]), v = __float_as_uint(acc[mb][nb][r + 1]);
-          pos = max(max(pos, (int)u), (int)v);
-          neg = max(max(neg, u), v);
-        }
-    uint32_t mx = max((uint32_t)pos, neg & 0x7fffffffu);
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) mx = max(mx, (uint32_t)__shfl_xor((int)mx, o));
-    // the largest d is the one that is stored: in fp16 it may have become infinite
-    mx = __float_as_uint(to_f32(from_f32<E>(__uint_as_float(mx)))) & 0x7fffffffu;
-    // (the plain read first keeps all but the few waves that raise the maximum from queueing on one address)
-    if (lane == 0 && mx > __builtin_nontemporal_load(a.dmax)) atomicMax(a.dmax, mx);
-  }
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb) {
     const int m0 = mt * TILE + wm * (TILE / 2) + mb * 32;  // a block = one tap, 32 consecutive channels
@@ -264,30 +239,12 @@ __global__ __launch_bounds__(TILE * 2, TILE == 128 ? 2 : 1) void bwd_colgrad_ker
     for (int nb = 0; nb < 2; ++nb) {
       const int px = pt * TILE + wn * 64 + nb * 32 + frow;
       if (px >= a.P) continue;
-      // The two halves of the wave exchange their 4-channel groups so that a lane holds 8 consecutive
-      // channels: one 16-byte store per lane and 16 channels, 32 pixels x 32 bytes contiguous per instruction
-      // (the lower half takes the first 8 channels of a 16-channel chunk, the upper half the second 8).
-      if constexpr (sizeof(DT) == 2) {
 #pragma unroll
-        for (int jp = 0; jp < 2; ++jp) {
-          const f32x16 &c16 = acc[mb][nb];
-          const int ja = 2 * jp, jb = 2 * jp + 1;
-          const uint32_t a0 = TR::pack2(c16[4 * ja], c16[4 * ja + 1]), a1 = TR::pack2(c16[4 * ja + 2], c16[4 * ja + 3]);
-          const uint32_t b0 = TR::pack2(c16[4 * jb], c16[4 * jb + 1]), b1 = TR::pack2(c16[4 * jb + 2], c16[4 * jb + 3]);
-          const auto s0 = __builtin_amdgcn_permlane32_swap(a0, b0, false, false);
-          const auto s1 = __builtin_amdgcn_permlane32_swap(a1, b1, false, false);
-          const int c = cb + jp * 16 + fhalf * 8;
-          DT *dst = D + ((((long)nl * chunks + (c >> 4)) * a.taps + tap) * a.P + px) * 16 + (c & 15);
-          *(uint4 *)dst = make_uint4(s0[0], s1[0], s0[1], s1[1]);
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int c = cb + j * 8 + fhalf * 4;
-          DT *dst = D + ((((long)nl * chunks + (c >> 4)) * a.taps + tap) * a.P + px) * 16 + (c & 15);
-          *(float4 *)dst = make_float4(acc[mb][nb][4 * j], acc[mb][nb][4 * j + 1], acc[mb][nb][4 * j + 2],
-                                       acc[mb][nb][4 * j + 3]);
-        }
+      for (int j = 0; j < 4; ++j) {
+        const int c = cb + j * 8 + fhalf * 4;
+        float *dst = a.D + ((((long)nl * chunks + (c >> 4)) * a.taps + tap) * a.P + px) * 16 + (c & 15);
+        *(float4 *)dst = make_float4(acc[mb][nb][4 * j], acc[mb][nb][4 * j + 1], acc[mb][nb][4 * j + 2],
+                                     acc[mb][nb][4 * j + 3]);
       }
     }
   }
@@ -295,18 +252,12 @@ __global__ __launch_bounds__(TILE * 2, TILE == 128 ? 2 : 1) void bwd_colgrad_ker
 
 // Bytes of the scatter kernel's window (two workgroups per CU).  It holds CH
 // channels of a WH x WW pixel neighbourhood of the tile; kScWindowPx pixels fit
-// with the larger channel count of a type (16-bit tensors: 16 channels of 32-bit
-// fixed point; fp32 tensors: 8 channels of doubles), twice as many -- stride 2,
-// dilation -- with the smaller one.  (A 48 KB window with 8 channels and three
+// with 8 channels of doubles, twice as many -- stride 2, dilation -- with 4.  (A 48 KB window with 8 channels and three
 // workgroups per CU was slower: the passes over the window double.)
 constexpr int kScWindowBytes = 60 * 1024;
 constexpr int kScWindowPx = kScWindowBytes / 64;
 // Largest margin of the window for far offsets.
 constexpr int kScFarMargin = 12;
-// Contributions one window entry can receive at most: every (pixel, tap) of the
-// tile touches an entry at most once per channel.
-constexpr int kScMaxAdds = 256 * 9;
-
 // CH consecutive channels (8 to 32 bytes) as floats.
 template <typename E, int CH>
 struct VecCh {
@@ -380,7 +331,7 @@ struct BwdScatterArgs {
   float *gin32;
   void *goff;
   void *gmask;     // null when unmodulated
-  void *col;       // columns of the pass [image][group][tap][padded channel of the group][P_pad], or null
+  void *col;       // columns of the pass (WGradArgs::col), or null
   ChanMap im;      // padded order of the input channels
   int cin_p;       // ... how many there are
   long P_pad;      // row pitch of col in elements
@@ -399,59 +350,22 @@ struct BwdScatterArgs {
   int parts;
   float *poff, *pmask;
   long off_total, mask_total;  // elements of grad_offset / grad_mask
-  // fixed-point window (16-bit tensors): largest |d|, and n_mmax values whose largest is that of |mask| (null: 1),
-  // as bit patterns
-  const uint32_t *dmax, *mmax;
-  int n_mmax;
 };
 
 // The window is not fp32: LDS single-precision atomic adds are slow on this
 // hardware (measured per wavefront instruction per CU: ds_add_f32 170 clocks,
-// ds_add_f64 26, ds_add_u32 11, whatever the addresses).  fp32 tensors, and 16-bit
-// tensors of few or uneven channels or few tiles (BwdPlan::fixed), use a
-// double-precision window (WT = double) and an fp32 d.  Other 16-bit tensors have a 16-bit d and a window of 32-bit fixed point
-// (WT = int32_t): with B = max|d| * max|mask| bounding every contribution and at
-// most kScMaxAdds contributions per entry, the scale 2^k <= 2^30 / (B * kScMaxAdds)
-// cannot overflow, and one contribution is rounded to B * 2^-19 at worst -- two
-// thousand times finer than the bf16/fp16 rounding of the result.  Integer sums
-// are exact, so the window part of grad_input does not depend on the order of
-// the adds.  Two channels share one 64-bit entry (ds_add_u64 costs 14 clocks
-// where two ds_add_u32 cost 22): the even channel's value sign-extended plus the
-// odd channel's shifted up by 32 bits; the low half's borrows and carries into
-// the high half cancel when the entry is taken apart again (low = the entry's low
-// word as a signed number, high = (entry - low) >> 32), since neither sum leaves
-// 32 bits.  Where d or the mask is not finite, or so small or large that no scale fits, nothing goes through the
-// window: every corner takes the way of those beyond it, an fp32 add to memory.
+// ds_add_f64 26, ds_add_u64 14, ds_add_u32 11, whatever the addresses), so it holds doubles.  16-bit
+// tensors that fill the tiles have bwd_fused_kernel, whose window is fixed point.
 // DATA: the gradient part (a.D, window, offset / mask sums).  COL: the kernel
 // stores the forward's columns (mask * bilinear sample, rounded to E as the
 // reference's columns tensor is) to a.col for the weight-gradient product.  At
 // least one of the two.
-template <typename E, int CH, typename WT, bool DATA, bool COL>
-__device__ __forceinline__ void scatter_tile(const BwdScatterArgs &a, const ScatterWindow &wd, WT *win) {
+template <typename E, int CH, bool DATA, bool COL>
+__device__ __forceinline__ void scatter_tile(const BwdScatterArgs &a, const ScatterWindow &wd, double *win) {
   constexpr int RC = 32 / (int)sizeof(E);   // channels per record of the input copy
   static_assert(DATA || COL, "nothing to do");
   static_assert(CH <= RC && RC % CH == 0, "a pass reads a record or a whole fraction of one");
-  static_assert(CH % 2 == 0, "fixed-point window entries hold two channels");
-  constexpr bool kFixed = sizeof(WT) == 4;
-  using DT = typename std::conditional<kFixed, E, float>::type;  // element of d
   static_assert(kScTH * kScTW == 256, "one thread per pixel of the tile");
-  static_assert(kScTH * kScTW * kBwdTapsMax <= kScMaxAdds, "bound on the adds per window entry");
-  float fx_scale = 1.0f, fx_inv = 1.0f;
-  bool fits = true;  // the window can be used
-  if (kFixed && DATA) {
-    uint32_t mb = 0x3f800000u;
-    if (a.mmax) {
-      mb = (int)(threadIdx.x & 63) < a.n_mmax ? a.mmax[threadIdx.x & 63] : 0u;
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) mb = max(mb, (uint32_t)__shfl_xor((int)mb, o));
-    }
-    const float mm = __uint_as_float(mb), bound = __uint_as_float(*a.dmax) * mm * (float)kScMaxAdds;
-    // largest power of two not above 2^30 / bound (any scale will do when everything is zero)
-    const int e = (bound > 0.0f && bound < 3.0e38f) ? 29 - ilogbf(bound) : 0;
-    fx_scale = ldexpf(1.0f, min(120, e));
-    fx_inv = 1.0f / fx_scale;
-    fits = bound < 3.0e38f && e <= 120 && mm * fx_scale < 3.0e38f;  // (false for NaN)
-  }
   const Geom &g = a.g;
   const long plane_out = (long)g.Ho * g.Wo;
   const long plane_in = (long)g.H * g.W;
@@ -470,7 +384,6 @@ __device__ __forceinline__ void scatter_tile(const BwdScatterArgs &a, const Scat
   const long pix = valid ? (long)ho * g.Wo + wo : 0;
   const int wy0 = ty * kScTH * g.sh - g.ph - wd.R, wx0 = tx * kScTW * g.sw - g.pw - wd.R;
   const int win_px = wd.WH * wd.WW;
-  const int win_h = fits ? wd.WH : 0;  // (a window that cannot be used has no rows: every sample is beyond it)
 
   const E *off = (const E *)a.om.off + (long)n * a.om.off_n + pix * a.om.off_px +
                  (long)(dgi * 2 * g.taps) * a.om.off_ch;
@@ -513,15 +426,14 @@ __device__ __forceinline__ void scatter_tile(const BwdScatterArgs &a, const Scat
 
   // Window pixels this thread flushes (tid, tid + 256, ...) as offsets into an image plane, the same
   // in every pass; -1 for one outside the image or past the window (it only ever receives zeros).
-  constexpr int NE = kFixed ? CH / 2 : CH;  // window entries per pixel
-  constexpr int kSlots = DATA ? (kScWindowBytes / (NE * 8) + 255) / 256 : 1;
+  constexpr int kSlots = DATA ? (kScWindowBytes / (CH * 8) + 255) / 256 : 1;
   int flush_at[kSlots];
   if constexpr (DATA) {
 #pragma unroll
     for (int j = 0; j < kSlots; ++j) {
       const int q = tid + 256 * j;
       const int y = wy0 + q / wd.WW, x = wx0 + q % wd.WW;
-      flush_at[j] = (fits && q < win_px && y >= 0 && y < g.H && x >= 0 && x < g.W) ? y * g.W + x : -1;
+      flush_at[j] = (q < win_px && y >= 0 && y < g.H && x >= 0 && x < g.W) ? y * g.W + x : -1;
     }
     // (the flush leaves the window zeroed for the next pass)
     for (int i = tid; i < kScWindowBytes / 16; i += 256) ((uint4 *)win)[i] = make_uint4(0u, 0u, 0u, 0u);
@@ -538,7 +450,7 @@ __device__ __forceinline__ void scatter_tile(const BwdScatterArgs &a, const Scat
     float ly, lx, m;
     bool inside;
     VecCh<E, CH> r00, r01, r10, r11;
-    VecCh<DT, CH> rd;
+    VecCh<float, CH> rd;
   };
   auto fetch = [&](int c0, int tap, E e_dy, E e_dx, E e_m, Sample &s) {
     const int ti = tap / g.kw, tj = tap - ti * g.kw;
@@ -564,7 +476,7 @@ __device__ __forceinline__ void scatter_tile(const BwdScatterArgs &a, const Scat
     s.r10.load(xp + (long)g.Wp * RC);
     s.r11.load(xp + (long)(g.Wp + 1) * RC);
     if constexpr (DATA)
-      s.rd.load((const DT *)a.D + (((long)nl * (a.cin_p / 16) + (c0 >> 4)) * g.taps + tap) * plane_out * 16 + pix * 16 +
+      s.rd.load((const float *)a.D + (((long)nl * (a.cin_p / 16) + (c0 >> 4)) * g.taps + tap) * plane_out * 16 + pix * 16 +
                 (c0 & 15));
   };
   // A tap's loads are issued one tap ahead, in front of the previous tap's stores and atomics
@@ -577,9 +489,16 @@ __device__ __forceinline__ void scatter_tile(const BwdScatterArgs &a, const Scat
   for (int pi = ps_begin; pi < ps_end; ++pi) {
     if constexpr (DATA) __syncthreads();  // the window is zero: first fill or the previous pass's flush
     const int c0 = ps.c0, cs = ps.cs;
-    // row of the columns matrix of channel c0 at tap 0 (a chunk stays inside one group)
-    E *cbase = (E *)a.col +
-               (((long)nl * a.cin_p + (long)ps.grp * a.im.cgp) * g.taps + (c0 - ps.grp * a.im.cgp)) * a.P_pad + pix;
+    // this pixel's columns of channel c0 at tap 0, and the way to the next tap (a pass stays inside one group)
+    E *cbase;
+    long ctap;
+    if constexpr (sizeof(E) == 2) {
+      cbase = (E *)a.col + (((long)nl * (a.cin_p / 16) + c0 / 16) * g.taps * a.P_pad + pix) * 16 + c0 % 16;
+      ctap = a.P_pad * 16;
+    } else {
+      cbase = (E *)a.col + (((long)nl * a.cin_p + (long)ps.grp * a.im.cgp) * g.taps + (c0 - ps.grp * a.im.cgp)) * a.P_pad + pix;
+      ctap = (long)a.im.cgp * a.P_pad;
+    }
     const Pass nps = pass_at(min(pi + 1, ps_end - 1));  // (the last pass fetches its own first tap again: unused)
     const int c_next = nps.c0;
 #pragma unroll
@@ -598,21 +517,20 @@ __device__ __forceinline__ void scatter_tile(const BwdScatterArgs &a, const Scat
         const bool ok00 = y0 >= 0 && x0 >= 0, ok01 = y0 >= 0 && x1 <= g.W - 1;
         const bool ok10 = y1 <= g.H - 1 && x0 >= 0, ok11 = y1 <= g.H - 1 && x1 <= g.W - 1;
         const float w00 = hy * hx, w01 = hy * lx, w10 = ly * hx, w11 = ly * lx;
-        VecCh<DT, CH> &rd = cur.rd;
+        VecCh<float, CH> &rd = cur.rd;
         if constexpr (DATA) {
           const uint32_t keep = inside ? ~0u : 0u;  // (whatever d holds where nothing is sampled)
 #pragma unroll
-          for (int i = 0; i < VecCh<DT, CH>::NW; ++i) rd.raw[i] &= keep;
+          for (int i = 0; i < VecCh<float, CH>::NW; ++i) rd.raw[i] &= keep;
         }
         const int ry = y0 - wy0, rx = x0 - wx0;
-        const bool in_win = ry >= 0 && ry + 1 < win_h && rx >= 0 && rx + 1 < wd.WW;
+        const bool in_win = ry >= 0 && ry + 1 < wd.WH && rx >= 0 && rx + 1 < wd.WW;
         const bool to_win = inside && in_win;
         // window is [channel][WH][WW]: neighbouring pixels, neighbouring banks; a lane with nothing
         // for the window adds its zeros at an entry of its own
         const int wbase = to_win ? ry * wd.WW + rx : (tid & 63);
         const float s00 = (to_win && ok00) ? w00 : 0.0f, s01 = (to_win && ok01) ? w01 : 0.0f;
         const float s10 = (to_win && ok10) ? w10 : 0.0f, s11 = (to_win && ok11) ? w11 : 0.0f;
-        const float mts = m * fx_scale;
         // sums over the pass's channels of d times each corner's value: the offset and mask
         // gradients are combinations of these four
         float S00 = 0.0f, S01 = 0.0f, S10 = 0.0f, S11 = 0.0f;
@@ -639,41 +557,28 @@ __device__ __forceinline__ void scatter_tile(const BwdScatterArgs &a, const Scat
           if constexpr (DATA) {
             float d[2];
             rd.pair(cp, d[0], d[1]);
-            if constexpr (kFixed) {
-              // round(w * ts) to nearest even in one multiply-add: the sum's mantissa holds the
-              // integer (|w * ts| < 2^19 by the choice of the scale).  An entry is the even
-              // channel's value sign-extended plus the odd one's shifted up 32 bits.
-              const float tl = d[0] * mts, th = d[1] * mts;
-              auto entry = [](float w, float tl, float th) {
-                const int lo = __float_as_int(fmaf(w, tl, 12582912.0f)) - 0x4B400000;
-                const uint32_t hi = (uint32_t)__float_as_int(fmaf(w, th, 12582912.0f)) - 0x4B400000u + (uint32_t)(lo >> 31);
-                return (unsigned long long)(uint32_t)lo | ((unsigned long long)hi << 32);
-              };
-              unsigned long long *wp = (unsigned long long *)win + cp * win_px + wbase;
-              atomicAdd(wp, entry(s00, tl, th));
-              atomicAdd(wp + 1, entry(s01, tl, th));
-              atomicAdd(wp + wd.WW, entry(s10, tl, th));
-              atomicAdd(wp + wd.WW + 1, entry(s11, tl, th));
-            } else {
 #pragma unroll
-              for (int h = 0; h < 2; ++h) {
-                // (a lane with nothing for the window adds zeros to an entry that may be somebody's: also where its own
-                // d is infinite, which a weight of zero would make NaN)
-                const float t = to_win ? d[h] * m : 0.0f;
-                WT *wp = win + (2 * cp + h) * win_px + wbase;
-                atomicAdd(wp, (WT)(s00 * t));
-                atomicAdd(wp + 1, (WT)(s01 * t));
-                atomicAdd(wp + wd.WW, (WT)(s10 * t));
-                atomicAdd(wp + wd.WW + 1, (WT)(s11 * t));
-              }
+            for (int h = 0; h < 2; ++h) {
+              // (a lane with nothing for the window adds zeros to an entry that may be somebody's: also where its own
+              // d is infinite, which a weight of zero would make NaN)
+              const float t = to_win ? d[h] * m : 0.0f;
+              double *wp = win + (2 * cp + h) * win_px + wbase;
+              atomicAdd(wp, (double)(s00 * t));
+              atomicAdd(wp + 1, (double)(s01 * t));
+              atomicAdd(wp + wd.WW, (double)(s10 * t));
+              atomicAdd(wp + wd.WW + 1, (double)(s11 * t));
             }
           }
         }
         if constexpr (COL) {
           if (valid) {
-            E *crow = cbase + (long)tap * a.im.cgp * a.P_pad;
+            E *crow = cbase + tap * ctap;
+            if constexpr (sizeof(E) == 2) {
+              __builtin_memcpy(__builtin_assume_aligned(crow, CH >= 8 ? 16 : 8), cv, sizeof(cv));
+            } else {
 #pragma unroll
-            for (int cc = 0; cc < CH; ++cc) crow[(long)cc * a.P_pad] = cv[cc];
+              for (int cc = 0; cc < CH; ++cc) crow[(long)cc * a.P_pad] = cv[cc];
+            }
           }
         }
         if constexpr (DATA) {
@@ -707,30 +612,15 @@ __device__ __forceinline__ void scatter_tile(const BwdScatterArgs &a, const Scat
       float *gplane = a.gin32 + ((long)n * g.Cin + cs) * plane_in;
 #pragma unroll
       for (int j = 0; j < kSlots; ++j) {
-        if (flush_at[j] >= 0) {  // (what is in a window that is not used is nobody's)
+        if (flush_at[j] >= 0) {
           const int q = tid + 256 * j;
           float *gi = gplane + flush_at[j];
-          if constexpr (kFixed) {
-            long long *w64 = (long long *)win + q;
 #pragma unroll
-            for (int cp = 0; cp < NE; ++cp) {
-              const long long e = w64[cp * win_px];
-              if (e != 0) {
-                w64[cp * win_px] = 0;
-                const int lo = (int)(unsigned)(unsigned long long)e;
-                const int hi = (int)((e - (long long)lo) >> 32);
-                if (lo != 0) unsafeAtomicAdd(gi + (long)(2 * cp) * plane_in, (float)lo * fx_inv);
-                if (hi != 0) unsafeAtomicAdd(gi + (long)(2 * cp + 1) * plane_in, (float)hi * fx_inv);
-              }
-            }
-          } else {
-#pragma unroll
-            for (int cc = 0; cc < NE; ++cc) {
-              const WT v = win[cc * win_px + q];
-              if (v != (WT)0) {
-                win[cc * win_px + q] = (WT)0;
-                if (cc < room) unsafeAtomicAdd(gi + (long)cc * plane_in, (float)v);
-              }
+          for (int cc = 0; cc < CH; ++cc) {
+            const double v = win[cc * win_px + q];
+            if (v != 0.0) {
+              win[cc * win_px + q] = 0.0;
+              if (cc < room) unsafeAtomicAdd(gi + (long)cc * plane_in, (float)v);
             }
           }
         }
@@ -771,27 +661,29 @@ __device__ __forceinline__ void scatter_tile(const BwdScatterArgs &a, const Scat
 // Few offsets beyond the margin of the wide pass's window: CH channels a pass.  Many: half as many channels over a
 // window twice as large, since a corner outside the window costs CH global atomics.  (Which of the two is
 // decided on the device, from a sample of the offsets that the pre-pass has looked at.)
-template <typename E, int CH, typename WT, bool DATA, bool COL>
+template <typename E, int CH, bool DATA, bool COL>
 __global__ __launch_bounds__(256, 2) void bwd_scatter_kernel(BwdScatterArgs a) {
-  __shared__ __align__(16) WT win[DATA ? kScWindowBytes / sizeof(WT) : 4];
+  __shared__ __align__(16) double win[DATA ? kScWindowBytes / 8 : 4];
   if constexpr (DATA && CH * (int)sizeof(E) >= 16) {
     if (a.win_far.WH > 0) {
       uint32_t n = (int)(threadIdx.x & 63) < a.n_far ? a.far[threadIdx.x & 63] : 0u;
 #pragma unroll
       for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o);
       if (__builtin_amdgcn_readfirstlane((int)n) > (int)a.far_min) {
-        scatter_tile<E, CH / 2, WT, DATA, COL>(a, a.win_far, win);
+        scatter_tile<E, CH / 2, DATA, COL>(a, a.win_far, win);
         return;
       }
     }
   }
-  scatter_tile<E, CH, WT, DATA, COL>(a, a.win, win);
+  scatter_tile<E, CH, DATA, COL>(a, a.win, win);
 }
 
 struct WGradArgs {
   const void *gout;  // [N][Cout][a_pitch]: grad_output in place (a_pitch = P) or its padded copy (P_pad)
   long a_pitch;
-  const void *col;   // [images of the pass][G][taps][padded channels of a group][P_pad]
+  // Columns: 16-bit tensors [images of the pass][padded channel / 16][taps][P_pad][16], stored 32 bytes a pixel and tap; fp32
+  // [images of the pass][G][taps][padded channels of a group][P_pad]
+  const void *col;
   float *part;       // partial sums [split][G][cout_g][M], every element written
   int accumulate;    // 0: the first pass writes them; 1: a later one adds to them
   int P;
@@ -806,16 +698,51 @@ struct WGradArgs {
   long total;        // workgroups with work: G x co_tiles x m_tiles x splits
 };
 
+// A wave's products of one K step with the second operand pixel major: B holds TILE / 16 runs of 64 pixels x 16 columns
+// (32 bytes a pixel).  An LDS read that transposes gives a lane four consecutive pixels of one column: 16 lanes
+// together read four pixels' 128 bytes.
+template <typename E, int TILE>
+__device__ __forceinline__ void tile_products_tr(f32x16 (&acc)[TILE / 64][2], const uint4 *A, const uint4 *B, int wm, int wn,
+                                                 int lane) {
+  using TR = ElemTraits<E>;
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) s16x4 *lds4_t;
+  constexpr int MB = TILE / 64;
+  const int frow = lane & 31, fhalf = lane >> 5;
+  const uint4 *a0 = A + (wm * (TILE / 2) + frow) * 8;
+  // run of this lane's column, the pixel whose 8 bytes it reads
+  const unsigned char *b0 = (const unsigned char *)B + (wn * 4 + ((lane >> 4) & 1)) * 2048 +
+                            (fhalf * 8 + ((lane & 15) >> 2)) * 32 + (lane & 3) * 8;
+#pragma unroll
+  for (int ksub = 0; ksub < 4; ++ksub) {
+    uint4 af[MB], bf[2];
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) af[mb] = a0[mb * 256 + ((ksub * 2 + fhalf) ^ (frow & 7))];
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb) {
+      const unsigned char *b = b0 + nb * 4096 + ksub * 512;
+      const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4_t)(lptr_t)(void *)b);
+      const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4_t)(lptr_t)(void *)(b + 128));
+      const uint2 l2 = __builtin_bit_cast(uint2, lo), h2 = __builtin_bit_cast(uint2, hi);
+      bf[nb] = make_uint4(l2.x, l2.y, h2.x, h2.y);
+    }
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int nb = 0; nb < 2; ++nb) TR::mma(acc[mb][nb], af[mb], bf[nb]);
+  }
+}
+
 // grad_weight[co, (c, tap)] += sum over the pass's images and pixels of
 // grad_output[co, pixel] * col[(tap, c), pixel]: a plain product with the pixels
 // as reduction dimension (the reference's second GEMM,
-// mmcv/ops/csrc/pytorch/modulated_deform_conv.cpp:227-237).  Workgroup = 128
-// output channels x 128 column rows of one group over a share of the (image,
+// mmcv/ops/csrc/pytorch/modulated_deform_conv.cpp:227-237).  Workgroup = TILE
+// output channels x TILE columns of one group over a share of the (image,
 // 128-byte pixel run) steps; both operand tiles go to LDS with direct copies as
 // in bwd_colgrad_kernel (grad_output is read in place: its rows are pixel
-// contiguous).  Runs of pixels past the end of an image read the row's last
-// 16 bytes again; the zero padding of col cancels them.  Rows past the group's
-// channels repeat its last row and are dropped at the end.  Each share of the K
+// contiguous; columns of 16-bit tensors are pixel major and transposed on the way out of LDS).  Runs of pixels past the end
+// of an image read the row's last 16 bytes again; the zero padding of col cancels them.  Rows past the group's
+// channels repeat its last ones and are dropped at the end.  Each share of the K
 // range stores its partial tile (plain stores, rows of M contiguous);
 // bwd_finish_kernel adds the shares up in a fixed order, so grad_weight does
 // not vary from run to run.
@@ -849,13 +776,23 @@ __global__ __launch_bounds__(TILE * 2, TILE == 128 ? 2 : 1) void bwd_wgrad_kerne
     const int row = (wave * 4 + c) * 8 + (lane >> 3);
     chunk[c] = (lane & 7) ^ (row & 7);
     const int co = min(ct * TILE + row, a.cout_g - 1);
-    // (the rows of the channels that only fill up a group are never written: they would hold what was there before, NaN
-    // for instance, and an fp32 call then goes over its K range a second time)
-    int m = min(mt * TILE + row, a.M - 1);
-    const int tap = m / a.cgp;
-    m = min(m, tap * a.cgp + a.rows - 1);
     a_row[c] = ((long)grp * a.cout_g + co) * a.a_pitch;      // + n * Cout * a_pitch
-    b_row[c] = ((long)grp * a.M + m) * a.P_pad;              // + nl * taps * Cin * P_pad
+    // (+ nl * taps * Cin * P_pad)
+    if constexpr (sizeof(E) == 2) {
+      // one KiB = 32 pixels of a run of 16 columns.  (Columns that only fill up a group may hold anything: each is an
+      // accumulator column of its own, which is not looked at.)
+      const int blk = wave * 4 + c;
+      const int m = min(mt * TILE + (blk >> 1) * 16, a.M - 16);
+      const int tap = m / a.cgp;
+      b_row[c] = (((long)((grp * a.cgp + m - tap * a.cgp) / 16) * a.taps + tap) * a.P_pad + (blk & 1) * 32) * 16 + lane * 8;
+    } else {
+      // (the rows of the channels that only fill up a group are never written: they would hold what was there before, NaN
+      // for instance, and the call then goes over its K range a second time)
+      int m = min(mt * TILE + row, a.M - 1);
+      const int tap = m / a.cgp;
+      m = min(m, tap * a.cgp + a.rows - 1);
+      b_row[c] = ((long)grp * a.M + m) * a.P_pad + chunk[c] * PXC;
+    }
   }
   const uint32_t lds_a = (uint32_t)(uintptr_t)(lptr_t)(&As[0][0]) +
                          (uint32_t)__builtin_amdgcn_readfirstlane(wave) * 4096u;
@@ -872,7 +809,7 @@ __global__ __launch_bounds__(TILE * 2, TILE == 128 ? 2 : 1) void bwd_wgrad_kerne
     for (int c = 0; c < 4; ++c) {
       const int px = p0 + chunk[c] * PXC;
       copy16_global_to_lds(ga + a_row[c] + min(px, last_chunk_px), lds_a + (uint32_t)buf * kBuf + (uint32_t)c * 1024u);
-      copy16_global_to_lds(cb + b_row[c] + px, lds_b + (uint32_t)buf * kBuf + (uint32_t)c * 1024u);
+      copy16_global_to_lds(cb + b_row[c] + (sizeof(E) == 2 ? (long)p0 * 16 : p0), lds_b + (uint32_t)buf * kBuf + (uint32_t)c * 1024u);
     }
   };
 
@@ -901,7 +838,10 @@ __global__ __launch_bounds__(TILE * 2, TILE == 128 ? 2 : 1) void bwd_wgrad_kerne
           asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         }
         __syncthreads();
-        tile_products<E, TILE, exact>(acc, As[buf], Bs[buf], wm, wn, frow, fhalf);
+        if constexpr (sizeof(E) == 2)
+          tile_products_tr<E, TILE>(acc, As[buf], Bs[buf], wm, wn, lane);
+        else
+          tile_products<E, TILE, exact>(acc, As[buf], Bs[buf], wm, wn, frow, fhalf);
         __syncthreads();
       }
     }

@@ -160,4 +160,24 @@ __device__ __forceinline__ float mask_value(E raw, int logit) {
   return m;
 }
 
+// bwd_fused_kernel: which tiles, and which of their passes, a workgroup takes.  The tiles are dealt out to the XCDs in contiguous runs, and within
+// an XCD round by round, so that its 32 workgroups -- one a CU -- are at neighbouring tiles and at the same channels at a time:
+// their adds to grad_input meet in the XCD's L2, and so do the rows of the input and the weights they read.  The tiles of
+// a last round that is not full are cut into as many shares of passes as there are workgroups for.
+struct FusedSchedule {
+  static constexpr int kXcds = 8, kPerXcd = 32, kGroups = kXcds * kPerXcd;
+  int tiles, passes;   // (passes of a tile)
+  __host__ __device__ int chunk() const { return (tiles + kXcds - 1) / kXcds; }
+  __host__ __device__ int first(int xcd) const { return xcd * chunk(); }
+  __host__ __device__ int count(int xcd) const {
+    const int c = tiles - first(xcd);
+    return c < 0 ? 0 : c < chunk() ? c : chunk();
+  }
+  __host__ __device__ int rest(int xcd) const { return count(xcd) % kPerXcd; }
+  __host__ __device__ int shares(int xcd) const {   // of a tile of the last round
+    const int r = rest(xcd), s = r ? kPerXcd / r : 1;
+    return s < passes ? s : passes;
+  }
+};
+
 }  // namespace mdcn

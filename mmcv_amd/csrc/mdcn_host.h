@@ -31,10 +31,12 @@ struct BwdPlan {
   // matrix-core paths (bwd_colgrad_kernel + bwd_scatter_kernel, bwd_wgrad_kernel):
   bool gemm;       // data gradients
   bool wgemm;      // grad_weight from stored columns
-  bool fixed;      // column gradient in 16 bits and a fixed-point window (else fp32 and doubles)
+  bool fused;      // ... by bwd_fused_kernel, column gradient in registers (else fp32 in memory, a window of doubles)
   int sR, sWH, sWW;  // window of the scatter kernel
   int sCH;         // channels per pass over that window
-  int fR, fWH, fWW;  // window with half as many channels a pass, for far offsets (fWH = 0: none)
+  int fR, fWH, fWW;  // window for far offsets (fWH = 0: none), with half as many channels a pass, or 8
+  int tw_log;      // fused: log2 of the width of a tile of 256 pixels
+  int n_wnorm;     // bounds on the rows of the weight matrix (fused)
   int n_chunk;     // images per pass
   int cg_tile;     // tile of the column-gradient product (kCgTile or kCgTileBig)
   // Padded channel orders of its copies: segments of the input's channels to whole passes of sCH, a group's to
@@ -43,13 +45,14 @@ struct BwdPlan {
   int M_pad;       // rows of the transposed weight matrix per group
   long P_pad;      // row pitch of the columns matrix
   int parts;       // workgroups of the scatter kernel per tile (shares of the channels)
+  FusedSchedule sched;  // fused: of a whole pass of images
   size_t xt_bytes, gt_bytes, wt_bytes, d_bytes, col_bytes, part_bytes;
   int w_tile, w_splits;  // weight-gradient product: tile, shares of the K range
   size_t wpart_bytes;    // ... and their partial sums
   size_t gpad_bytes;     // grad_output with padded rows, when its own rows cannot be copied 16 bytes at a time
   size_t gb_bytes;  // sums of grad_bias
   int bsplits;      // ... shares of a channel's pixels (matrix-core paths)
-  size_t mx_bytes;  // the maxima that scale the fixed-point window, the counts of far offsets
+  size_t mx_bytes;  // the counts of far offsets, the bounds on the rows of the weight matrix
   size_t total() const {
     return gin_bytes + gw_bytes + gb_bytes + mx_bytes + xt_bytes + gt_bytes + wt_bytes + d_bytes + col_bytes + part_bytes +
            wpart_bytes + gpad_bytes;

@@ -1,0 +1,81 @@
+"""The 16-bit backward in one kernel (bwd_fused_kernel) where it can go wrong: edges of its tiles, chunks of output channels
+that are not full, eight channels a pass, odd numbers of taps, cut tiles beside whole rounds of them, offsets beyond either
+window; all gradients against the same call in double precision."""
+import pytest
+import torch
+
+from mmcv_amd import capi
+from common import capi_backward, cast_case, make_case
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    ('one_tile', dict(N=1, Cin=64, Cout=64, H=16, W=16)),
+    ('edges_w32', dict(N=2, Cin=64, Cout=128, H=7, W=65)),
+    ('edges_w16', dict(N=1, Cin=128, Cout=64, H=17, W=33)),
+    ('k192', dict(N=1, Cin=64, Cout=192, H=15, W=18)),
+    ('k320', dict(N=1, Cin=64, Cout=320, H=9, W=31)),
+    ('k512', dict(N=1, Cin=128, Cout=512, H=13, W=21)),
+    ('k640_8ch', dict(N=1, Cin=64, Cout=640, H=11, W=20, deform_groups=8)),
+    ('8ch', dict(N=1, Cin=192, Cout=64, H=18, W=17, deform_groups=8)),
+    ('groups', dict(N=2, Cin=128, Cout=256, H=12, W=34, groups=2, deform_groups=2)),
+    ('group_in_dg', dict(N=1, Cin=128, Cout=128, H=12, W=20, groups=2)),
+    ('k1x1', dict(N=1, Cin=64, Cout=64, H=20, W=20, k=(1, 1), padding=0)),
+    ('k1x3', dict(N=1, Cin=64, Cout=64, H=9, W=40, k=(1, 3), padding=(0, 1))),
+    ('k2x2', dict(N=1, Cin=64, Cout=64, H=19, W=23, k=(2, 2))),
+    ('s2', dict(N=2, Cin=64, Cout=64, H=37, W=69, stride=2)),
+    ('dil3', dict(N=1, Cin=64, Cout=64, H=24, W=26, dilation=3, padding=3)),
+    ('far', dict(N=1, Cin=64, Cout=64, H=40, W=45, sigma=6.0)),
+    ('far_s2', dict(N=1, Cin=128, Cout=64, H=60, W=75, stride=2, sigma=9.0)),
+    ('past_far', dict(N=1, Cin=64, Cout=64, H=50, W=55, sigma=20.0)),
+    ('rounds', dict(N=2, Cin=64, Cout=64, H=190, W=194, sigma=1.5)),   # 36 or 37 tiles per XCD: a round, and cut ones
+]
+NAMES = ('grad_input', 'grad_offset', 'grad_mask', 'grad_weight', 'grad_bias')
+#: Unit roundoff: the largest relative error of one rounding.  Over many values its root mean square is 0.42 of that (an error
+#: uniform within a last place, values spread over their binade), and two independent ones -- the columns are rounded before they
+#: are summed -- add up to 0.6; 0.5 and 0.7 leave room for what else there is, and not for another rounding.  grad_bias has too few
+#: values for a mean.
+U = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}
+SHARE = dict(grad_input=0.5, grad_offset=0.5, grad_mask=0.5, grad_weight=0.7, grad_bias=1.0)
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16], ids=['bf16', 'f16'])
+@pytest.mark.parametrize('name,kw', CASES, ids=[c[0] for c in CASES])
+def test_fused_backward(name, kw, dtype):
+    print(f'case={name} dtype={dtype}', flush=True)
+    dev = cast_case(make_case(71, **kw), dtype, 'cuda')
+    Ho, Wo = dev['offset'].shape[2:]
+    gy = torch.randn(kw['N'], kw['Cout'], Ho, Wo, generator=torch.Generator().manual_seed(4)).to(dtype).cuda()
+    for modulated in (True, False):
+        case = dict(dev) if modulated else dict(dev, mask=None)
+        ref = capi_backward({k: v.double() if torch.is_tensor(v) else v for k, v in case.items()}, gy.double())
+        for want in (dict(), dict(want_weight=False)):
+            got = capi_backward(case, gy, path=capi.PATH_FUSED, **want)
+            for nm, r, o in zip(NAMES, ref, got):
+                if o is None or (nm == 'grad_weight' and not want.get('want_weight', True)):
+                    continue
+                err = float((o.double() - r).norm() / r.norm())
+                assert err <= U[dtype] * SHARE[nm], (nm, modulated, want, err)
+    # the shares of a tile are added up in a fixed order, and integers in any: two runs differ by the order of the adds to memory
+    # alone, which is grad_input's
+    again = capi_backward(dev, gy, path=capi.PATH_FUSED)
+    first = capi_backward(dev, gy, path=capi.PATH_FUSED)
+    for nm, a, b in zip(NAMES[1:], again[1:], first[1:]):
+        assert torch.equal(a, b), nm
+
+
+def test_passes_of_images():
+    """Cut tiles of several passes of images, the last one of another size, have places of their own for their shares."""
+    kw = dict(N=5, Cin=64, Cout=64, H=33, W=47)
+    dev = cast_case(make_case(72, **kw), torch.bfloat16, 'cuda')
+    gy = torch.randn(5, 64, 33, 47, generator=torch.Generator().manual_seed(5)).bfloat16().cuda()
+    whole = capi_backward(dev, gy, path=capi.PATH_FUSED)
+    lib = capi.load()
+    lib.mdcn_set_pass_limits(0, 2 * 9 * 64 * 33 * 47 * 2)   # two images' columns
+    try:
+        parts = capi_backward(dev, gy, path=capi.PATH_FUSED)
+    finally:
+        lib.mdcn_set_pass_limits(0, 0)
+    # the offsets' sums are cut at other channels: fp32 sums in another order, which round to a neighbour now and then
+    for nm, a, b in zip(NAMES, whole, parts):
+        assert float((a.double() - b.double()).norm() / a.double().norm()) <= 0.1 * U[torch.bfloat16], nm
