@@ -357,6 +357,7 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
     a.x_chunks = up((long)g.H * g.W, 32 * EPV);
     a.g_chunks = up(plane_out, 32 * EPV);
     a.P_pad = pl.P_pad;
+    a.run = pl.sCH;
     a.col_rows = (long)pl.n_chunk * g.taps * cin_p;
     a.M_pad = pl.M_pad;
     a.wnorm = wnorm;
@@ -451,6 +452,7 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
     sa.goff = bp->grad_offset;
     sa.gmask = bp->grad_mask;
     sa.col = wgemm ? col : nullptr;
+    sa.run = pl.sCH;
     sa.P_pad = pl.P_pad;
     sa.tiles_x = (g.Wo + kScTW - 1) / kScTW;
     sa.tiles_y = (g.Ho + kScTH - 1) / kScTH;
@@ -514,12 +516,22 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
       const long tiles = (long)g.G * wa.co_tiles * wa.m_tiles;
       wa.splits = pl.w_splits;
       wa.total = tiles * wa.splits;
-      if (wtile == kCgTileBig)
-        hipLaunchKernelGGL((bwd_wgrad_kernel<E, kCgTileBig>), dim3((unsigned)((wa.total + 7) / 8 * 8)),
-                           dim3(2 * kCgTileBig), 0, st, wa);
-      else
-        hipLaunchKernelGGL((bwd_wgrad_kernel<E, kCgTile>), dim3((unsigned)((wa.total + 7) / 8 * 8)),
-                           dim3(2 * kCgTile), 0, st, wa);
+      auto launch_w = [&](auto runv) {
+        constexpr int RUN = decltype(runv)::value;
+        const dim3 wgrid((unsigned)((wa.total + 7) / 8 * 8));
+        if (wtile == kCgTileBig)
+          hipLaunchKernelGGL((bwd_wgrad_kernel<E, kCgTileBig, RUN>), wgrid, dim3(2 * kCgTileBig), 0, st, wa);
+        else
+          hipLaunchKernelGGL((bwd_wgrad_kernel<E, kCgTile, RUN>), wgrid, dim3(2 * kCgTile), 0, st, wa);
+      };
+      if (!staged || pl.sCH == 16)
+        launch_w(std::integral_constant<int, 16>());
+      else if constexpr (staged) {
+        if (pl.sCH == 8)
+          launch_w(std::integral_constant<int, 8>());
+        else
+          launch_w(std::integral_constant<int, 4>());
+      }
       check();
     }
   }

@@ -26,6 +26,7 @@ struct BwdPreArgs {
   int x_chunks, g_chunks;  // pixel chunks of the re-layouts
   long P_pad;
   long col_rows;           // rows of col whose padding is cleared
+  int run;                 // WGradArgs::run
   int M_pad;
   uint32_t *wnorm;         // bound on the norm of 64 rows of the weight matrix, one per block of the job
   const void *off;
@@ -91,13 +92,13 @@ __global__ __launch_bounds__(256) void bwd_prepass_kernel(BwdPreArgs a) {
     }
     return;
   }
-  if (b < a.end[kPreColPad]) {  // padding pixels [P, P_pad) of the columns matrix: of its rows, or of runs of 16 of them
-    constexpr int RUN = sizeof(E) == 2 ? 16 : 1;
-    const int padn = (int)(a.P_pad - plane) * RUN;
+  if (b < a.end[kPreColPad]) {  // padding pixels [P, P_pad) of the columns matrix: of its rows, or of runs of them
+    const int run = sizeof(E) == 2 ? a.run : 1;
+    const int padn = (int)(a.P_pad - plane) * run;
     const long i0 = (long)(b - a.end[kPreZero]) * kPrePadPerBlock;
     for (int k = 0; k < kPrePadPerBlock / 256; ++k) {
       const long i = i0 + k * 256 + tid, r = i / padn;
-      if (r < a.col_rows / RUN) ((E *)a.col)[(r * a.P_pad + plane) * RUN + (i - r * padn)] = from_f32<E>(0.0f);
+      if (r < a.col_rows / run) ((E *)a.col)[(r * a.P_pad + plane) * run + (i - r * padn)] = from_f32<E>(0.0f);
     }
     return;
   }

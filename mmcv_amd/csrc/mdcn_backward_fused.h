@@ -35,7 +35,7 @@ struct BwdFusedArgs {
   float *gin32;
   void *goff;
   void *gmask;      // null when unmodulated
-  void *col;        // columns of the pass [image][Cin / 16][taps][P_pad][16], or null
+  void *col;        // columns of the pass [image][Cin / CH][taps][P_pad][CH], or null: CH the kernel's
   long P_pad;
   int tw_log;       // a tile of 256 pixels is 1 << tw_log wide (16 or 32)
   int tiles_x, tiles_y;
@@ -81,7 +81,7 @@ __device__ __forceinline__ uint32_t norm_bound(float ss, uint32_t mx, int k) {
 // bf16, N=16, 256 -> 256 channels, 100x152: 1.35 ms for what took 0.52 (column gradient to memory) + 1.50 (scatter kernel reading
 // it); a pass takes a CU 43 thousand clocks: 22 scatter (VALU busy in 17, LDS adds 18), 7 products (MFMA 5), 7 flush, the rest
 // waits at the three barriers.
-template <typename E, int CH, bool DEEP>
+template <typename E, int CH, int RUN, bool DEEP>
 __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterWindow &wd, int b, int c_first, int c_last, float *part, uint4 *lds,
                                            float *red) {
   using TR = ElemTraits<E>;
@@ -457,7 +457,7 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
     __syncthreads();   // the window is zero and the stages are free
     if (c0 + CH < c_end) issue_first(c0 + CH);
     __builtin_amdgcn_sched_barrier(0);
-    E *cbase = (E *)a.col + ((((long)nl * (g.Cin / 16) + c0 / 16) * g.taps + half) * a.P_pad + pix) * 16 + c0 % 16;
+    E *cbase = (E *)a.col + ((((long)nl * (g.Cin / RUN) + c0 / RUN) * g.taps + half) * a.P_pad + pix) * RUN + c0 % RUN;
 #pragma unroll
     for (int i = 0; i < kBfItems; ++i) {
       if (i < items) {
@@ -522,7 +522,7 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
             __builtin_amdgcn_sched_barrier(0);
           }
           if (a.col && valid && has_tap(i))
-            *(uint4 *)(cbase + (long)(2 * i) * a.P_pad * 16 + h * 8) = make_uint4(cv[0], cv[1], cv[2], cv[3]);
+            *(uint4 *)(cbase + (long)(2 * i) * a.P_pad * RUN + h * 8) = make_uint4(cv[0], cv[1], cv[2], cv[3]);
           __builtin_amdgcn_sched_barrier(0);
         }
         acc_m[i] += w00 * S00 + w01 * S01 + w10 * S10 + w11 * S11;
@@ -615,12 +615,12 @@ __global__ __launch_bounds__(kBfThreads, 2) void bwd_fused_kernel(BwdFusedArgs a
       if (shares > 1) part = a.part + (long)(xcd * FusedSchedule::kPerXcd + j) * 3 * a.g.taps * 256;
     }
     if constexpr (CHF == CH) {
-      fused_tile<E, CH, DEEP>(a, far ? a.win_far : a.win, tile, first * CH, last * CH, part, lds, red);
+      fused_tile<E, CH, CH, DEEP>(a, far ? a.win_far : a.win, tile, first * CH, last * CH, part, lds, red);
     } else {
       if (far)
-        fused_tile<E, CHF, DEEP>(a, a.win_far, tile, first * CH, last * CH, part, lds, red);
+        fused_tile<E, CHF, CH, DEEP>(a, a.win_far, tile, first * CH, last * CH, part, lds, red);
       else
-        fused_tile<E, CH, DEEP>(a, a.win, tile, first * CH, last * CH, part, lds, red);
+        fused_tile<E, CH, CH, DEEP>(a, a.win, tile, first * CH, last * CH, part, lds, red);
     }
   }
 }

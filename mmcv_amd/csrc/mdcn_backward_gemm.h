@@ -332,6 +332,7 @@ struct BwdScatterArgs {
   void *goff;
   void *gmask;     // null when unmodulated
   void *col;       // columns of the pass (WGradArgs::col), or null
+  int run;
   ChanMap im;      // padded order of the input channels
   int cin_p;       // ... how many there are
   long P_pad;      // row pitch of col in elements
@@ -361,7 +362,7 @@ struct BwdScatterArgs {
 // reference's columns tensor is) to a.col for the weight-gradient product.  At
 // least one of the two.
 template <typename E, int CH, bool DATA, bool COL>
-__device__ __forceinline__ void scatter_tile(const BwdScatterArgs &a, const ScatterWindow &wd, double *win) {
+__device__ __forceinline__ void scatter_tile(const BwdScatterArgs &a, const ScatterWindow &wd, double *win, float *lone) {
   constexpr int RC = 32 / (int)sizeof(E);   // channels per record of the input copy
   static_assert(DATA || COL, "nothing to do");
   static_assert(CH <= RC && RC % CH == 0, "a pass reads a record or a whole fraction of one");
@@ -482,9 +483,11 @@ __device__ __forceinline__ void scatter_tile(const BwdScatterArgs &a, const Scat
   // A tap's loads are issued one tap ahead, in front of the previous tap's stores and atomics
   // (a wait for loads also waits for every older store, and the compiler cannot move a load
   // above a store that might alias it); the last tap of a pass fetches the first of the next.
-  Sample cur;
+  // Two samples take turns: copying the next one over the current one would wait for its loads at the end of every tap
+  // (backward of fp32, N=2, 256 channels, 50x84: 329 against 322 us; N=8, 128 channels, 60x80, stride 2: 196 / 187).
+  Sample smp[2];
   Pass ps = pass_at(ps_begin);
-  fetch(ps.c0, 0, t_dy[0], t_dx[0], t_m[0], cur);
+  fetch(ps.c0, 0, t_dy[0], t_dx[0], t_m[0], smp[0]);
 
   for (int pi = ps_begin; pi < ps_end; ++pi) {
     if constexpr (DATA) __syncthreads();  // the window is zero: first fill or the previous pass's flush
@@ -493,8 +496,8 @@ __device__ __forceinline__ void scatter_tile(const BwdScatterArgs &a, const Scat
     E *cbase;
     long ctap;
     if constexpr (sizeof(E) == 2) {
-      cbase = (E *)a.col + (((long)nl * (a.cin_p / 16) + c0 / 16) * g.taps * a.P_pad + pix) * 16 + c0 % 16;
-      ctap = a.P_pad * 16;
+      cbase = (E *)a.col + (((long)nl * (a.cin_p / a.run) + c0 / a.run) * g.taps * a.P_pad + pix) * a.run + c0 % a.run;
+      ctap = a.P_pad * a.run;
     } else {
       cbase = (E *)a.col + (((long)nl * a.cin_p + (long)ps.grp * a.im.cgp) * g.taps + (c0 - ps.grp * a.im.cgp)) * a.P_pad + pix;
       ctap = (long)a.im.cgp * a.P_pad;
@@ -504,13 +507,14 @@ __device__ __forceinline__ void scatter_tile(const BwdScatterArgs &a, const Scat
 #pragma unroll
     for (int tap = 0; tap < kBwdTapsMax; ++tap) {
       if (tap < g.taps) {
-        Sample nxt;
+        Sample &cur = smp[tap & 1], &nxt = smp[(tap + 1) & 1];
         {
           const bool more = tap + 1 < g.taps;  // workgroup uniform
           const int tn = tap + 1 < kBwdTapsMax ? tap + 1 : 0;  // (a constant once the loop is unrolled)
           fetch(more ? c0 : c_next, more ? tn : 0, more ? t_dy[tn] : t_dy[0], more ? t_dx[tn] : t_dx[0],
                 more ? t_m[tn] : t_m[0], nxt);
         }
+        __builtin_amdgcn_sched_barrier(0);   // (these loads first, then the wait for the current sample's)
         const bool inside = cur.inside;
         const int y0 = cur.y0, x0 = cur.x0, y1 = y0 + 1, x1 = x0 + 1;
         const float ly = cur.ly, lx = cur.lx, hy = 1.0f - ly, hx = 1.0f - lx, m = cur.m;
@@ -585,23 +589,28 @@ __device__ __forceinline__ void scatter_tile(const BwdScatterArgs &a, const Scat
           acc_m[tap] += w00 * S00 + w01 * S01 + w10 * S10 + w11 * S11;
           acc_y[tap] += m * (hx * (S10 - S00) + lx * (S11 - S01));
           acc_x[tap] += m * (hy * (S01 - S00) + ly * (S11 - S10));
-          if (inside && !in_win) {  // rare: corners beyond the window go to memory directly
-            const long o00 = (long)y0 * g.W + x0, o01 = o00 + 1, o10 = o00 + g.W, o11 = o10 + 1;
-            float d[CH];
-            rd.unpack(d);
+          // Samples beyond the window go to memory directly, one at a time: a lane for every channel and corner.
+          for (unsigned long long rest = __ballot(inside && !in_win); rest != 0ull; rest &= rest - 1ull) {
+            const int l = __ffsll((long long)rest) - 1, lane = tid & 63;
+            if (lane == l) {
+              float d[CH];
+              rd.unpack(d);
 #pragma unroll
-            for (int cc = 0; cc < CH; ++cc) {
-              if (cc >= ps.room) break;
-              const float t = d[cc] * m;
-              float *gi = a.gin32 + ((long)n * g.Cin + cs + cc) * plane_in;
-              if (ok00) unsafeAtomicAdd(gi + o00, w00 * t);
-              if (ok01) unsafeAtomicAdd(gi + o01, w01 * t);
-              if (ok10) unsafeAtomicAdd(gi + o10, w10 * t);
-              if (ok11) unsafeAtomicAdd(gi + o11, w11 * t);
+              for (int cc = 0; cc < CH; ++cc) lone[cc] = d[cc] * m;
             }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            const int fy = __builtin_amdgcn_readlane(y0, l), fx = __builtin_amdgcn_readlane(x0, l);
+            const float gy = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(ly), l));
+            const float gx = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(lx), l));
+            const int k = lane % CH, corner = lane / CH;
+            const int yy = fy + (corner >> 1), xx = fx + (corner & 1);
+            const float w = ((corner & 2) ? gy : 1.0f - gy) * ((corner & 1) ? gx : 1.0f - gx);
+            const float t = lone[k];
+            if (corner < 4 && k < ps.room && yy >= 0 && yy < g.H && xx >= 0 && xx < g.W)
+              unsafeAtomicAdd(a.gin32 + ((long)n * g.Cin + cs + k) * plane_in + ((long)yy * g.W + xx), w * t);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
           }
         }
-        cur = nxt;
       }
     }
     if constexpr (DATA) {
@@ -626,6 +635,7 @@ __device__ __forceinline__ void scatter_tile(const BwdScatterArgs &a, const Scat
         }
       }
     }
+    if (g.taps & 1) smp[0] = smp[1];   // (the next pass's first)
     ps = nps;
   }
   if constexpr (DATA) {
@@ -664,25 +674,28 @@ __device__ __forceinline__ void scatter_tile(const BwdScatterArgs &a, const Scat
 template <typename E, int CH, bool DATA, bool COL>
 __global__ __launch_bounds__(256, 2) void bwd_scatter_kernel(BwdScatterArgs a) {
   __shared__ __align__(16) double win[DATA ? kScWindowBytes / 8 : 4];
+  __shared__ float lone[4 * CH];   // CH of each wavefront
+  float *mine = lone + (threadIdx.x >> 6) * CH;
   if constexpr (DATA && CH * (int)sizeof(E) >= 16) {
     if (a.win_far.WH > 0) {
       uint32_t n = (int)(threadIdx.x & 63) < a.n_far ? a.far[threadIdx.x & 63] : 0u;
 #pragma unroll
       for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o);
       if (__builtin_amdgcn_readfirstlane((int)n) > (int)a.far_min) {
-        scatter_tile<E, CH / 2, DATA, COL>(a, a.win_far, win);
+        scatter_tile<E, CH / 2, DATA, COL>(a, a.win_far, win, mine);
         return;
       }
     }
   }
-  scatter_tile<E, CH, DATA, COL>(a, a.win, win);
+  scatter_tile<E, CH, DATA, COL>(a, a.win, win, mine);
 }
 
 struct WGradArgs {
   const void *gout;  // [N][Cout][a_pitch]: grad_output in place (a_pitch = P) or its padded copy (P_pad)
   long a_pitch;
-  // Columns: 16-bit tensors [images of the pass][padded channel / 16][taps][P_pad][16], stored 32 bytes a pixel and tap; fp32
-  // [images of the pass][G][taps][padded channels of a group][P_pad]
+  // Columns: 16-bit tensors [images of the pass][padded channel / run][taps][P_pad][run], run = 16, 8 or 4 channels, those that
+  // are stored together (runs of 16 half filled by each of two passes: 173 -> 184 us for the backward of bf16 N=2, 32 channels,
+  // 150x200, 4 deformable groups); fp32 [images of the pass][G][taps][padded channels of a group][P_pad]
   const void *col;
   float *part;       // partial sums [split][G][cout_g][M], every element written
   int accumulate;    // 0: the first pass writes them; 1: a later one adds to them
@@ -698,10 +711,10 @@ struct WGradArgs {
   long total;        // workgroups with work: G x co_tiles x m_tiles x splits
 };
 
-// A wave's products of one K step with the second operand pixel major: B holds TILE / 16 runs of 64 pixels x 16 columns
-// (32 bytes a pixel).  An LDS read that transposes gives a lane four consecutive pixels of one column: 16 lanes
-// together read four pixels' 128 bytes.
-template <typename E, int TILE>
+// A wave's products of one K step with the second operand pixel major: B holds, for every 16 columns, 16 / run runs of 64 pixels x
+// run columns.  An LDS read that transposes gives a lane four consecutive pixels of one column: 16 lanes
+// read 8 bytes each, four pixels of every four columns.
+template <typename E, int TILE, int RUN>
 __device__ __forceinline__ void tile_products_tr(f32x16 (&acc)[TILE / 64][2], const uint4 *A, const uint4 *B, int wm, int wn,
                                                  int lane) {
   using TR = ElemTraits<E>;
@@ -710,9 +723,11 @@ __device__ __forceinline__ void tile_products_tr(f32x16 (&acc)[TILE / 64][2], co
   constexpr int MB = TILE / 64;
   const int frow = lane & 31, fhalf = lane >> 5;
   const uint4 *a0 = A + (wm * (TILE / 2) + frow) * 8;
-  // run of this lane's column, the pixel whose 8 bytes it reads
-  const unsigned char *b0 = (const unsigned char *)B + (wn * 4 + ((lane >> 4) & 1)) * 2048 +
-                            (fhalf * 8 + ((lane & 15) >> 2)) * 32 + (lane & 3) * 8;
+  // the four columns and the pixel whose 8 bytes this lane reads
+  constexpr int per = RUN / 4, pitch = RUN * 2;
+  const int quad = lane & 3;
+  const unsigned char *b0 = (const unsigned char *)B + (wn * 4 + ((lane >> 4) & 1)) * 2048 + quad / per * (64 * pitch) +
+                            (fhalf * 8 + ((lane & 15) >> 2)) * pitch + quad % per * 8;
 #pragma unroll
   for (int ksub = 0; ksub < 4; ++ksub) {
     uint4 af[MB], bf[2];
@@ -720,9 +735,9 @@ __device__ __forceinline__ void tile_products_tr(f32x16 (&acc)[TILE / 64][2], co
     for (int mb = 0; mb < MB; ++mb) af[mb] = a0[mb * 256 + ((ksub * 2 + fhalf) ^ (frow & 7))];
 #pragma unroll
     for (int nb = 0; nb < 2; ++nb) {
-      const unsigned char *b = b0 + nb * 4096 + ksub * 512;
+      const unsigned char *b = b0 + nb * 4096 + ksub * 16 * pitch;
       const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4_t)(lptr_t)(void *)b);
-      const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4_t)(lptr_t)(void *)(b + 128));
+      const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4_t)(lptr_t)(void *)(b + 4 * pitch));
       const uint2 l2 = __builtin_bit_cast(uint2, lo), h2 = __builtin_bit_cast(uint2, hi);
       bf[nb] = make_uint4(l2.x, l2.y, h2.x, h2.y);
     }
@@ -746,7 +761,8 @@ __device__ __forceinline__ void tile_products_tr(f32x16 (&acc)[TILE / 64][2], co
 // range stores its partial tile (plain stores, rows of M contiguous);
 // bwd_finish_kernel adds the shares up in a fixed order, so grad_weight does
 // not vary from run to run.
-template <typename E, int TILE>
+// RUN: run of 16-bit columns.
+template <typename E, int TILE, int RUN>
 __global__ __launch_bounds__(TILE * 2, TILE == 128 ? 2 : 1) void bwd_wgrad_kernel(WGradArgs a) {
   constexpr int ES = (int)sizeof(E);
   constexpr int PXC = 16 / ES;  // pixels per 16-byte chunk
@@ -779,12 +795,14 @@ __global__ __launch_bounds__(TILE * 2, TILE == 128 ? 2 : 1) void bwd_wgrad_kerne
     a_row[c] = ((long)grp * a.cout_g + co) * a.a_pitch;      // + n * Cout * a_pitch
     // (+ nl * taps * Cin * P_pad)
     if constexpr (sizeof(E) == 2) {
-      // one KiB = 32 pixels of a run of 16 columns.  (Columns that only fill up a group may hold anything: each is an
-      // accumulator column of its own, which is not looked at.)
+      // This lane's 16 bytes of the 2 KiB of 16 columns.  (Columns that only fill up a group may hold anything: each is
+      // an accumulator column of its own, which is not looked at.)
       const int blk = wave * 4 + c;
       const int m = min(mt * TILE + (blk >> 1) * 16, a.M - 16);
       const int tap = m / a.cgp;
-      b_row[c] = (((long)((grp * a.cgp + m - tap * a.cgp) / 16) * a.taps + tap) * a.P_pad + (blk & 1) * 32) * 16 + lane * 8;
+      const int at = (blk & 1) * 512 + lane * 8;   // element of the 64 pixels x 16 columns
+      const int sub = at / (64 * RUN), px = (at - sub * 64 * RUN) / RUN;
+      b_row[c] = (((long)((grp * a.cgp + m - tap * a.cgp) / RUN + sub) * a.taps + tap) * a.P_pad + px) * RUN + at % RUN;
     } else {
       // (the rows of the channels that only fill up a group are never written: they would hold what was there before, NaN
       // for instance, and the call then goes over its K range a second time)
@@ -809,7 +827,7 @@ __global__ __launch_bounds__(TILE * 2, TILE == 128 ? 2 : 1) void bwd_wgrad_kerne
     for (int c = 0; c < 4; ++c) {
       const int px = p0 + chunk[c] * PXC;
       copy16_global_to_lds(ga + a_row[c] + min(px, last_chunk_px), lds_a + (uint32_t)buf * kBuf + (uint32_t)c * 1024u);
-      copy16_global_to_lds(cb + b_row[c] + (sizeof(E) == 2 ? (long)p0 * 16 : p0), lds_b + (uint32_t)buf * kBuf + (uint32_t)c * 1024u);
+      copy16_global_to_lds(cb + b_row[c] + (sizeof(E) == 2 ? (long)p0 * RUN : p0), lds_b + (uint32_t)buf * kBuf + (uint32_t)c * 1024u);
     }
   };
 
@@ -839,7 +857,7 @@ __global__ __launch_bounds__(TILE * 2, TILE == 128 ? 2 : 1) void bwd_wgrad_kerne
         }
         __syncthreads();
         if constexpr (sizeof(E) == 2)
-          tile_products_tr<E, TILE>(acc, As[buf], Bs[buf], wm, wn, lane);
+          tile_products_tr<E, TILE, RUN>(acc, As[buf], Bs[buf], wm, wn, lane);
         else
           tile_products<E, TILE, exact>(acc, As[buf], Bs[buf], wm, wn, frow, fhalf);
         __syncthreads();
