@@ -293,6 +293,39 @@ size_t mdcn_backward_workspace_bytes(const mdcn_bwd_params *p);
 /* Enqueue the backward on `hip_stream`.  Returns an mdcn_status. */
 int mdcn_backward(const mdcn_bwd_params *p, void *hip_stream);
 
+/*
+ * ModulatedDeformConv2dPack and DeformConv2dPack in training
+ * (mmcv/ops/modulated_deform_conv.py:327-335, mmcv/ops/deform_conv.py:405-409): what
+ * lies around the deformable convolution.
+ *
+ * mdcn_pack_split(): `offset` and `mask`, dense as mdcn_params describes them, from
+ * p->raw: the conv_offset output, dense, the logits taken through the sigmoid and rounded.
+ *
+ * mdcn_pack_trains(): 1 when mdcn_pack_backward() covers the shape in *p, else 0 (no pointer is
+ * looked at): channels in whole 128 bytes, the halo of a tile of conv_offset's pixels
+ * fits LDS.
+ */
+int mdcn_pack_split(const mdcn_pack_params *p, void *offset, void *mask, void *hip_stream);
+int mdcn_pack_trains(const mdcn_pack_params *p);
+
+/* bwd: as for mdcn_backward() with the forward's offset and mask; grad_input,
+ * grad_offset and grad_mask are set.  On return grad_input holds the whole gradient of
+ * the input -- what reaches it through the offsets and the mask is added when
+ * through_input is 1 --, grad_offset and grad_mask what mdcn_backward() leaves there.
+ * grad_offset_weight, grad_offset_bias: conv_offset's, or NULL; sums in fp32, in a fixed
+ * order, rounded once. */
+typedef struct mdcn_pack_bwd_params {
+  mdcn_bwd_params bwd;
+  const void *offset_weight;
+  void *grad_offset_weight;
+  void *grad_offset_bias;
+  int32_t unmodulated;
+  int32_t through_input;
+} mdcn_pack_bwd_params;
+
+size_t mdcn_pack_backward_workspace_bytes(const mdcn_pack_bwd_params *p);
+int mdcn_pack_backward(const mdcn_pack_bwd_params *p, void *hip_stream);
+
 #ifdef __cplusplus
 }
 #endif

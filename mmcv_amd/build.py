@@ -36,7 +36,7 @@ def _run(cmd, cwd=None):
 
 
 SOURCES = ['mdcn_api.hip', 'mdcn_backward.hip', 'mdcn_backward_bf16.hip', 'mdcn_backward_f16.hip', 'mdcn_oconv.hip',
-           'mdcn_segment.hip']
+           'mdcn_oconv_backward.hip', 'mdcn_segment.hip']
 
 
 def build_hip(extra=(), check=True):

@@ -19,7 +19,8 @@ EXPORTS = ('mdcn_abi_version', 'mdcn_set_pass_limits', 'mdcn_status_string', 'md
            'mdcn_fused_eligible', 'mdcn_forward_kernels', 'mdcn_workspace_bytes', 'mdcn_workspace_wanted',
            'mdcn_forward', 'mdcn_forward_noalloc',
            'mdcn_forward_timed', 'mdcn_pack_workspace_bytes', 'mdcn_pack_forward',
-           'mdcn_pack_forward_timed', 'mdcn_backward_workspace_bytes', 'mdcn_backward')
+           'mdcn_pack_forward_timed', 'mdcn_backward_workspace_bytes', 'mdcn_backward',
+           'mdcn_pack_trains', 'mdcn_pack_split', 'mdcn_pack_backward_workspace_bytes', 'mdcn_pack_backward')
 
 
 class MdcnParams(ctypes.Structure):
@@ -42,6 +43,12 @@ class MdcnBwdParams(ctypes.Structure):
     _fields_ = [('conv', MdcnParams)] + [(n, ctypes.c_void_p) for n in
                                          ('grad_output', 'grad_input', 'grad_offset', 'grad_mask',
                                           'grad_weight', 'grad_bias')]
+
+
+class MdcnPackBwdParams(ctypes.Structure):
+    _fields_ = [('bwd', MdcnBwdParams), ('offset_weight', ctypes.c_void_p),
+                ('grad_offset_weight', ctypes.c_void_p), ('grad_offset_bias', ctypes.c_void_p),
+                ('unmodulated', ctypes.c_int32), ('through_input', ctypes.c_int32)]
 
 
 _lib = None
@@ -90,6 +97,15 @@ def load():
         lib.mdcn_backward_workspace_bytes.argtypes = [BP]
         lib.mdcn_backward.restype = ctypes.c_int
         lib.mdcn_backward.argtypes = [BP, ctypes.c_void_p]
+        lib.mdcn_pack_trains.restype = ctypes.c_int
+        lib.mdcn_pack_trains.argtypes = [PP]
+        lib.mdcn_pack_split.restype = ctypes.c_int
+        lib.mdcn_pack_split.argtypes = [PP, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p]
+        PB = ctypes.POINTER(MdcnPackBwdParams)
+        lib.mdcn_pack_backward_workspace_bytes.restype = ctypes.c_size_t
+        lib.mdcn_pack_backward_workspace_bytes.argtypes = [PB]
+        lib.mdcn_pack_backward.restype = ctypes.c_int
+        lib.mdcn_pack_backward.argtypes = [PB, ctypes.c_void_p]
         _lib = lib
     return _lib
 

@@ -7,6 +7,8 @@
 // There is no CPU implementation here on purpose: a call with CPU tensors
 // raises, the way the reference's device registry does for a device nobody
 // registered (mmcv/ops/csrc/common/pytorch_device_registry.hpp:120-126).
+#include <ATen/TensorSubclassLikeUtils.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/functions/basic_ops.h>
@@ -384,13 +386,19 @@ void deform_conv_forward(Tensor input, Tensor weight, Tensor offset, Tensor outp
   TORCH_CHECK(rc == MDCN_OK, op, ": ", mdcn_status_string(rc));
 }
 
-// Shared by the three backward ops: checks, contiguity, workspace and the call.
+// What the Pack layers' backward adds to the convolution's: gradients through conv_offset.  Undefined: not wanted.
+struct PackHead {
+  Tensor weight, grad_weight, grad_bias;
+  bool through_input;
+};
+
+// Shared by the backward ops: checks, contiguity, workspace and the call.
 // Tensors with zero elements stand for "not wanted".
 void run_backward(const char *op, const Tensor &input, const Tensor &weight, const Tensor &offset,
                   const Tensor &mask, const Tensor &grad_output, Tensor grad_input,
                   Tensor grad_offset, Tensor grad_mask, Tensor grad_weight, Tensor grad_bias,
                   int kernel_h, int kernel_w, int stride_h, int stride_w, int pad_h, int pad_w,
-                  int dilation_h, int dilation_w, int group, int deformable_group) {
+                  int dilation_h, int dilation_w, int group, int deformable_group, const PackHead *head = nullptr) {
   TORCH_CHECK(input.dim() == 4 && weight.dim() == 4 && offset.dim() == 4 && grad_output.dim() == 4, op,
               " expects 4-D input, weight, offset and grad_output");
   const at::Device dev = input.device();
@@ -472,13 +480,25 @@ void run_backward(const char *op, const Tensor &input, const Tensor &weight, con
   bp.grad_mask = ptr(grad_mask);
   bp.grad_weight = ptr(grad_weight);
   bp.grad_bias = ptr(grad_bias);
-  const size_t ws = mdcn_backward_workspace_bytes(&bp);
+  mdcn_pack_bwd_params pb{};
+  if (head) {
+    keep.push_back(head->weight.contiguous());
+    pb.offset_weight = keep.back().data_ptr();
+    pb.grad_offset_weight = head->grad_weight.defined() ? head->grad_weight.data_ptr() : nullptr;
+    pb.grad_offset_bias = head->grad_bias.defined() ? head->grad_bias.data_ptr() : nullptr;
+    pb.unmodulated = modulated ? 0 : 1;
+    pb.through_input = head->through_input ? 1 : 0;
+    pb.bwd = bp;
+  }
+  const size_t ws = head ? mdcn_pack_backward_workspace_bytes(&pb) : mdcn_backward_workspace_bytes(&bp);
   if (ws > 0) {
     keep.push_back(at::empty({(int64_t)ws}, input.options().dtype(at::kByte)));
     p.workspace = keep.back().data_ptr();
     p.workspace_bytes = ws;
+    pb.bwd = bp;
   }
-  rc = mdcn_backward(&bp, (void *)c10::hip::getCurrentHIPStream().stream());
+  void *stream = (void *)c10::hip::getCurrentHIPStream().stream();
+  rc = head ? mdcn_pack_backward(&pb, stream) : mdcn_backward(&bp, stream);
   TORCH_CHECK(rc == MDCN_OK, op, ": ", mdcn_status_string(rc));
 }
 
@@ -586,6 +606,20 @@ Tensor layer_forward(const Tensor &input, const Tensor &offset, const Tensor &ma
   return output;
 }
 
+// what torch.autograd.function.once_differentiable does
+void refuse_second(torch::autograd::variable_list &out) {
+  torch::autograd::variable_list defined;
+  for (auto &t : out)
+    if (t.defined()) defined.push_back(t.detach().set_requires_grad(true));
+  const int64_t n = (int64_t)defined.size();
+  auto err = std::make_shared<torch::autograd::DelayedError>(
+      "trying to differentiate twice a function that was marked with @once_differentiable", n);
+  defined = (*err)(std::move(defined));
+  size_t i = 0;
+  for (auto &t : out)
+    if (t.defined()) t = defined[i++];
+}
+
 struct LayerFunction : public torch::autograd::Function<LayerFunction> {
   static Tensor forward(torch::autograd::AutogradContext *ctx, const Tensor &input_, const Tensor &offset,
                         const c10::optional<Tensor> &mask_, const Tensor &weight_, const c10::optional<Tensor> &bias_,
@@ -629,18 +663,7 @@ struct LayerFunction : public torch::autograd::Function<LayerFunction> {
                      or_none(mask), grads[0], or_none(out[0]), or_none(out[1]), or_none(out[2]), or_none(out[3]),
                      or_none(out[4]), q.kh, q.kw, q.sh, q.sw, q.ph, q.pw, q.dh, q.dw, q.groups, q.dgroups);
     }
-    if (twice) {  // what torch.autograd.function.once_differentiable does
-      torch::autograd::variable_list defined;
-      for (auto &t : out)
-        if (t.defined()) defined.push_back(t.detach().set_requires_grad(true));
-      const int64_t n = (int64_t)defined.size();
-      auto err = std::make_shared<torch::autograd::DelayedError>(
-          "trying to differentiate twice a function that was marked with @once_differentiable", n);
-      defined = (*err)(std::move(defined));
-      size_t i = 0;
-      for (auto &t : out)
-        if (t.defined()) t = defined[i++];
-    }
+    if (twice) refuse_second(out);
     return out;
   }
 };
@@ -676,6 +699,123 @@ Tensor pack_call(const Tensor &x_, const Tensor &offset_weight, const c10::optio
                                      with_bias ? like(*bias_, offset_weight) : none, output, q.kh, q.kw, sh, sw, ph, pw,
                                      dh, dw, groups, dgroups, with_bias, false, unmodulated);
   return output;
+}
+
+// ... and with them: conv_offset, split, sigmoid and the convolution as one node, whose forward has conv_offset from torch -- its
+// last bits decide between which pixels a sample lies and so what the gradients are -- and whose backward is the library's.
+struct PackFunction : public torch::autograd::Function<PackFunction> {
+  static Tensor forward(torch::autograd::AutogradContext *ctx, const Tensor &x, const Tensor &offset_weight,
+                        const c10::optional<Tensor> &offset_bias, const Tensor &weight, const c10::optional<Tensor> &bias,
+                        std::vector<int64_t> geo, bool unmodulated) {
+    const LayerGeo q(weight, geo);
+    const Tensor raw = at::conv2d(x, offset_weight, offset_bias, {q.sh, q.sw}, {q.ph, q.pw}, {q.dh, q.dw}).contiguous();
+    Tensor offset = raw, mask;
+    if (!unmodulated) {
+      const int64_t n = q.dgroups * q.kh * q.kw;
+      offset = at::empty({x.size(0), 2 * n, raw.size(2), raw.size(3)}, raw.options());
+      mask = at::empty({x.size(0), n, raw.size(2), raw.size(3)}, raw.options());
+      c10::DeviceGuard guard(x.device());
+      mdcn_pack_params pp = pack_params(x, weight, q, unmodulated);
+      pp.raw = raw.data_ptr();
+      const int rc = mdcn_pack_split(&pp, offset.data_ptr(), mask.data_ptr(), (void *)c10::hip::getCurrentHIPStream().stream());
+      TORCH_CHECK(rc == MDCN_OK, "modulated_deform_conv_pack_forward: ", mdcn_status_string(rc));
+    }
+    Tensor output = layer_forward(x, offset, mask, weight, bias.has_value() ? *bias : Tensor(), q);
+    ctx->save_for_backward({x, offset_weight, offset, mask, weight});
+    geo.push_back(offset_bias.has_value() ? 1 : 0);
+    geo.push_back(bias.has_value() ? 1 : 0);
+    ctx->saved_data["geo"] = geo;
+    return output;
+  }
+
+  static mdcn_pack_params pack_params(const Tensor &x, const Tensor &weight, const LayerGeo &q, bool unmodulated) {
+    mdcn_pack_params pp{};
+    mdcn_params &p = pp.conv;
+    p.dtype = mdcn_dtype_of(x);
+    p.path = g_path.load();
+    p.no_k_split = g_no_k_split.load();
+    p.N = (int)x.size(0); p.Cin = (int)x.size(1); p.H = (int)x.size(2); p.W = (int)x.size(3);
+    p.Cout = (int)weight.size(0); p.kh = (int)q.kh; p.kw = (int)q.kw;
+    p.sh = (int)q.sh; p.sw = (int)q.sw; p.ph = (int)q.ph; p.pw = (int)q.pw; p.dh = (int)q.dh; p.dw = (int)q.dw;
+    p.groups = (int)q.groups; p.dgroups = (int)q.dgroups;
+    pp.unmodulated = unmodulated ? 1 : 0;
+    return pp;
+  }
+
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx,
+                                                 torch::autograd::variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    const Tensor &x = saved[0], &ow = saved[1], &offset = saved[2], &mask = saved[3], &weight = saved[4];
+    const std::vector<int64_t> geo = ctx->saved_data["geo"].toIntVector();
+    const LayerGeo q(weight, geo);
+    const bool with_ob = geo[geo.size() - 2] != 0, with_b = geo.back() != 0;
+    // (needs_input_grad counts the tensors that were given)
+    const size_t iw = with_ob ? 3 : 2;
+    const bool want_x = ctx->needs_input_grad(0), want_ow = ctx->needs_input_grad(1);
+    const bool want_ob = with_ob && ctx->needs_input_grad(2);
+    const bool want_w = ctx->needs_input_grad(iw), want_b = with_b && ctx->needs_input_grad(iw + 1);
+    const bool twice = at::GradMode::is_enabled() && grads[0].requires_grad();
+    torch::autograd::variable_list out(7);
+    {
+      at::AutoGradMode no_grad(false);
+      const Tensor none = at::empty({0}, x.options());
+      auto fresh = [&](const Tensor &t) { return at::empty_like(t, t.options(), at::MemoryFormat::Contiguous); };
+      auto or_none = [&](const Tensor &t) { return t.defined() ? t : none; };
+      PackHead head;
+      Tensor gx, goff, gmask;
+      const bool through = want_x || want_ow || want_ob;
+      if (through) {
+        head.weight = ow;
+        head.through_input = want_x;
+        gx = fresh(x);
+        goff = fresh(offset);
+        if (mask.defined()) gmask = fresh(mask);
+        if (want_x) out[0] = gx;
+        if (want_ow) out[1] = head.grad_weight = fresh(ow);
+        if (want_ob) out[2] = head.grad_bias = at::empty({ow.size(0)}, ow.options());
+      }
+      if (want_w) out[3] = fresh(weight);
+      if (want_b) out[4] = at::empty({weight.size(0)}, weight.options());
+      if (through || want_w || want_b)
+        run_backward(mask.defined() ? "modulated_deform_conv_backward" : "deform_conv_backward", x, weight, offset,
+                     or_none(mask), grads[0].contiguous(), or_none(gx), or_none(goff), or_none(gmask), or_none(out[3]),
+                     or_none(out[4]), q.kh, q.kw, q.sh, q.sw, q.ph, q.pw, q.dh, q.dw, q.groups, q.dgroups,
+                     through ? &head : nullptr);
+    }
+    if (twice) refuse_second(out);
+    return out;
+  }
+};
+
+// The Pack's forward with gradients, or nothing for a call that is not covered: what the library refuses, parameters of
+// several types or shapes that do not fit (the layer's own sequence has the errors), tangents, tensors
+// and modes that want to see torch's operations.
+c10::optional<Tensor> pack_train_call(const Tensor &x, const Tensor &ow, const c10::optional<Tensor> &ob, const Tensor &weight,
+                                      const c10::optional<Tensor> &bias, int64_t sh, int64_t sw, int64_t ph, int64_t pw,
+                                      int64_t dh, int64_t dw, int64_t groups, int64_t dgroups, int64_t step, bool unmodulated) {
+  if (c10::impl::dispatch_mode_enabled()) return c10::nullopt;
+  const Tensor b = bias.has_value() ? *bias : Tensor(), o = ob.has_value() ? *ob : Tensor();
+  for (const Tensor *t : {&x, &ow, &o, &weight, &b}) {
+    if (!t->defined()) continue;
+    if (!t->is_cuda() || t->device() != x.device() || t->scalar_type() != x.scalar_type() || at::isTensorSubclassLike(*t) ||
+        t->_fw_grad(0).defined() || t->is_conj() || t->is_neg())
+      return c10::nullopt;
+  }
+  const auto type = x.scalar_type();
+  if ((type != at::kFloat && type != at::kHalf && type != at::kBFloat16) || x.dim() != 4 || weight.dim() != 4 || ow.dim() != 4 ||
+      x.size(0) == 0 || groups <= 0 || dgroups <= 0)
+    return c10::nullopt;
+  const int64_t kh = weight.size(2), kw = weight.size(3), co = (unmodulated ? 2 : 3) * dgroups * kh * kw;
+  if (ow.size(0) != co || ow.size(1) != x.size(1) || ow.size(2) != kh || ow.size(3) != kw ||
+      weight.size(1) * groups != x.size(1) || (o.defined() && o.numel() != co) || (b.defined() && b.numel() != weight.size(0)))
+    return c10::nullopt;
+  const std::vector<int64_t> geo = {sh, sw, ph, pw, dh, dw, groups, dgroups, step};
+  const mdcn_pack_params pp = PackFunction::pack_params(x, weight, LayerGeo(weight, geo), unmodulated);
+  {
+    c10::DeviceGuard guard(x.device());
+    if (!mdcn_pack_trains(&pp)) return c10::nullopt;
+  }
+  return PackFunction::apply(x, ow, ob, weight, bias, geo, unmodulated);
 }
 
 }  // namespace
@@ -736,6 +876,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("pack_call", &pack_call,
         "pack_call(x, offset_weight, offset_bias | None, weight, bias | None, sh, sw, ph, pw, dh, dw, groups, "
         "deform_groups, unmodulated): the Pack layers' forward, no autograd");
+  m.def("pack_train_call", &pack_train_call,
+        "pack_train_call(x, offset_weight, offset_bias | None, weight, bias | None, sh, sw, ph, pw, dh, dw, groups, "
+        "deform_groups, im2col_step, unmodulated): the Pack layers' forward with autograd; None where the library does not cover the call");
   m.def("set_path", [](int path) {
           TORCH_CHECK(path >= MDCN_PATH_AUTO && path <= MDCN_PATH_SEGMENT,
                       "path must be 0 (auto), 1 (fused), 2 (direct), 3 (fused, specialised-wave kernel only), "

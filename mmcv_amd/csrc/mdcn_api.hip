@@ -19,6 +19,7 @@
 #include "mdcn_fused3.h"
 #include "mdcn_fused_f32.h"
 #include "mdcn_oconv.h"
+#include "mdcn_oconv_backward.h"
 #include "mdcn_host.h"
 #include "mdcn_prepass.h"
 #include "mdcn_segment.h"
@@ -800,6 +801,21 @@ int run(const mdcn_params *p, void *stream, float *ms, const mdcn_pack_params *p
   }
 }
 
+template <typename E>
+int split_raw(const mdcn_pack_params *pp, const Geom &g, E *offset, E *mask, hipStream_t st) {
+  const long plane = (long)g.Ho * g.Wo * g.DG * g.taps, total = 3 * plane * g.N, per = 256 * (16 / (long)sizeof(E));
+  hipLaunchKernelGGL(raw_split_kernel<E>, dim3((unsigned)((total + per - 1) / per)), dim3(256), 0, st, (const E *)pp->raw, offset,
+                     mask, 2 * plane, plane, total);
+  return hipGetLastError() == hipSuccess ? MDCN_OK : MDCN_ERR_LAUNCH;
+}
+
+// Workspace: the convolution's, then conv_offset's, which reads the copy of the input the former leaves.
+bool plan_pack_backward(const mdcn_pack_bwd_params *pb, const Geom &g, BwdPlan *pl, OconvBwdPlan *ol) {
+  make_bwd_plan(&pb->bwd, g, g_bwd_pass_bytes.load(), pl);
+  return oconv_bwd_plan(g, pb->bwd.conv.dtype, pb->unmodulated != 0, pb->through_input != 0,
+                        pb->grad_offset_weight || pb->grad_offset_bias, !pl->plain_copy(), num_cus(), ol);
+}
+
 int check_bwd(const mdcn_bwd_params *bp, Geom *g, bool need_ptrs) {
   if (!bp) return MDCN_ERR_NULL;
   const mdcn_params *p = &bp->conv;
@@ -961,6 +977,65 @@ int mdcn_backward(const mdcn_bwd_params *bp, void *hip_stream) {
   if (need > 0 && (!p->workspace || p->workspace_bytes < need || ((uintptr_t)p->workspace % kAlign) != 0))
     return MDCN_ERR_WORKSPACE;
   return run_backward(bp, g, pl, (hipStream_t)hip_stream);
+}
+
+int mdcn_pack_trains(const mdcn_pack_params *pp) {
+  Geom g;
+  if (!pp || check_params(&pp->conv, &g, false) != MDCN_OK || pp->conv.input_nhwc) return 0;
+  OconvBwdPlan ol;
+  return oconv_bwd_plan(g, pp->conv.dtype, pp->unmodulated != 0, true, true, false, num_cus(), &ol) ? 1 : 0;
+}
+
+int mdcn_pack_split(const mdcn_pack_params *pp, void *offset, void *mask, void *hip_stream) {
+  if (!pp || !pp->raw || !offset || !mask) return MDCN_ERR_NULL;
+  Geom g;
+  const int rc = check_params(&pp->conv, &g, false);
+  if (rc != MDCN_OK) return rc;
+  hipStream_t st = (hipStream_t)hip_stream;
+  switch (pp->conv.dtype) {
+    case MDCN_F32: return split_raw<float>(pp, g, (float *)offset, (float *)mask, st);
+    case MDCN_F16: return split_raw<f16_t>(pp, g, (f16_t *)offset, (f16_t *)mask, st);
+    case MDCN_BF16: return split_raw<bf16_t>(pp, g, (bf16_t *)offset, (bf16_t *)mask, st);
+    default: return MDCN_ERR_DTYPE;
+  }
+}
+
+size_t mdcn_pack_backward_workspace_bytes(const mdcn_pack_bwd_params *pb) {
+  Geom g;
+  if (!pb || check_bwd(&pb->bwd, &g, false) != MDCN_OK) return 0;
+  BwdPlan pl;
+  OconvBwdPlan ol;
+  return plan_pack_backward(pb, g, &pl, &ol) ? pl.total() + ol.total() : 0;
+}
+
+int mdcn_pack_backward(const mdcn_pack_bwd_params *pb, void *hip_stream) {
+  if (!pb) return MDCN_ERR_NULL;
+  Geom g;
+  int rc = check_bwd(&pb->bwd, &g, true);
+  if (rc != MDCN_OK) return rc;
+  const mdcn_params *p = &pb->bwd.conv;
+  if (!pb->offset_weight || !pb->bwd.grad_input || (!pb->unmodulated) != (p->mask != nullptr)) return MDCN_ERR_NULL;
+  BwdPlan pl;
+  OconvBwdPlan ol;
+  if (!plan_pack_backward(pb, g, &pl, &ol)) return MDCN_ERR_PATH;
+  const size_t need = pl.total() + ol.total();
+  if (need > 0 && (!p->workspace || p->workspace_bytes < need || ((uintptr_t)p->workspace % kAlign) != 0))
+    return MDCN_ERR_WORKSPACE;
+  rc = run_backward(&pb->bwd, g, pl, (hipStream_t)hip_stream);
+  if (rc != MDCN_OK || (!ol.data && !ol.weight)) return rc;
+  unsigned char *ws = (unsigned char *)p->workspace;
+  OconvBwdArgs a{};
+  a.g = g;
+  a.x = p->input;
+  a.ow = pb->offset_weight;
+  a.goff = pb->bwd.grad_offset;
+  a.gmask = pb->bwd.grad_mask;
+  a.mask = p->mask;
+  a.gin = pb->bwd.grad_input;
+  a.gw = pb->grad_offset_weight;
+  a.gb = pb->grad_offset_bias;
+  a.xt = pl.plain_copy() ? ws + pl.xt_at() : nullptr;
+  return oconv_backward(p->dtype, ol, a, ws + pl.total(), (hipStream_t)hip_stream) == hipSuccess ? MDCN_OK : MDCN_ERR_LAUNCH;
 }
 
 int mdcn_pack_forward_timed(const mdcn_pack_params *pp, void *hip_stream, float ms[5]) {

@@ -53,6 +53,9 @@ struct BwdPlan {
   size_t gb_bytes;  // sums of grad_bias
   int bsplits;      // ... shares of a channel's pixels (matrix-core paths)
   size_t mx_bytes;  // the counts of far offsets, the bounds on the rows of the weight matrix
+  // where the matrix-core paths have their copy of the input, and whether its channels are the input's own
+  size_t xt_at() const { return gin_bytes + gb_bytes + mx_bytes; }
+  bool plain_copy() const { return (gemm || wgemm) && im.segp == im.seg && im.cgp == im.cg; }
   size_t total() const {
     return gin_bytes + gw_bytes + gb_bytes + mx_bytes + xt_bytes + gt_bytes + wt_bytes + d_bytes + col_bytes + part_bytes +
            wpart_bytes + gpad_bytes;

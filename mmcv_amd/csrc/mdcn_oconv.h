@@ -119,4 +119,35 @@ __global__ __launch_bounds__(256) void raw_to_nchw_kernel(const E *__restrict__ 
   }
 }
 
+// raw, dense (N, n_off + n_msk channels), by images: the first run_off elements of an image are offsets, copied, the
+// other run_msk mask logits.  A thread has 16 bytes of raw.
+template <typename E>
+__global__ __launch_bounds__(256) void raw_split_kernel(const E *__restrict__ raw, E *__restrict__ off, E *__restrict__ msk,
+                                                        long run_off, long run_msk, long total) {
+  constexpr int EPV = 16 / (int)sizeof(E);
+  const long i0 = ((long)blockIdx.x * 256 + threadIdx.x) * EPV;
+  if (i0 >= total) return;
+  const long run = run_off + run_msk, n = i0 / run, r0 = i0 - n * run;
+  E *o = off + n * run_off, *m = msk + n * run_msk - run_off;
+  if (i0 + EPV <= total && (r0 + EPV <= run_off || (r0 >= run_off && r0 + EPV <= run))) {
+    E v[EPV];
+    __builtin_memcpy(v, raw + i0, 16);
+    if (r0 < run_off) {
+      __builtin_memcpy(o + r0, v, 16);
+    } else {
+#pragma unroll
+      for (int k = 0; k < EPV; ++k) v[k] = from_f32<E>(mask_value<E>(v[k], kMaskLogit));
+      __builtin_memcpy(m + r0, v, 16);
+    }
+    return;
+  }
+  for (int k = 0; k < EPV && i0 + k < total; ++k) {
+    const long nk = (i0 + k) / run, r = i0 + k - nk * run;
+    if (r < run_off)
+      off[nk * run_off + r] = raw[i0 + k];
+    else
+      msk[nk * run_msk + r - run_off] = from_f32<E>(mask_value<E>(raw[i0 + k], kMaskLogit));
+  }
+}
+
 }  // namespace mdcn

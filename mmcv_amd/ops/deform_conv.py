@@ -21,12 +21,13 @@ from torch.nn.modules.utils import _pair, _single
 
 from ..utils import ext_loader
 from .modulated_deform_conv import (_conv_output_size, _in_one_call,
+                                    _offset_conv_in_library,
                                     _renamed_kwargs)
 from .registry import MODELS
 
 ext_module = ext_loader.load_ext('_ext', [
     'deform_conv_forward', 'deform_conv_backward_input',
-    'deform_conv_backward_parameters', 'layer_call', 'pack_call'
+    'deform_conv_backward_parameters', 'layer_call', 'pack_call', 'pack_train_call'
 ])
 
 
@@ -265,6 +266,13 @@ class DeformConv2dPack(DeformConv2d):
             return deform_conv2d_pack(x, self.conv_offset, self.weight, self.stride,
                                       self.padding, self.dilation, self.groups,
                                       self.deform_groups)
+        if needs_grad and _offset_conv_in_library(x, self) and self.im2col_step > 0 \
+                and x.size(0) % max(min(self.im2col_step, x.size(0)), 1) == 0:
+            y = ext_module.pack_train_call(x, self.conv_offset.weight, self.conv_offset.bias, self.weight, None,
+                                           *_pair(self.stride), *_pair(self.padding), *_pair(self.dilation), self.groups,
+                                           self.deform_groups, min(self.im2col_step, x.size(0)), True)
+            if y is not None:
+                return y
         offset = self.conv_offset(x)
         return deform_conv2d(x, offset, self.weight, self.stride, self.padding,
                              self.dilation, self.groups, self.deform_groups,
