@@ -4,9 +4,9 @@
 // and of conv_offset.bias.  Four launches: oconv_bwd_prep_kernel, oconv_dgrad_kernel,
 // oconv_wgrad_kernel, oconv_bwd_finish_kernel.  In us, 27 channels of conv_offset, 3x3, and before them the fifteen
 // launches of torch's convolution, sigmoid, cat, chunk, their backward and the sum of the two gradients of the input:
-//   bf16 N=16 256 channels 100x152: 25 + 121 + 95 + 6; a training call 3030 instead of 3474
-//   bf16 N=2 256 channels 50x84: 6 + 13 + 10 + 6; 363 instead of 440
-//   fp32 N=2 256 channels 50x84: 6 + 28 + 35 + 5; 570 instead of 600
+//   bf16 N=16 256 channels 100x152: 25 + 111 + 93 + 6; a training call 3010 instead of 3474
+//   bf16 N=2 256 channels 50x84: 6 + 10 + 10 + 6; 358 instead of 440
+//   fp32 N=2 256 channels 50x84: 6 + 26 + 31 + 5; 560 instead of 600
 #pragma once
 
 #include "mdcn_common.h"
@@ -22,7 +22,7 @@ constexpr int kOwTaps = 9, kOwWaves = 3;              // taps of a workgroup of 
 struct OconvBwdPlan {
   int CO, cob;            // conv_offset channels, blocks of 32 of them
   int Wp;                 // row pitch of the channel-major gradient: whole runs of 32 pixels
-  int d_th, gh, gw, d_lds;   // data kernel: input rows per tile, rows and columns of its gradient halo, LDS bytes of that
+  int d_th, d_waves, d_cper, gh, gw, d_lds;   // data kernel: input rows per wave, waves, blocks of 32 channels, rows and columns of its gradient halo, LDS bytes of that
   int w_th, lw, plane_chunks, w_lds;  // weight kernel: output rows per tile, columns of its input halo, its planes in LDS
   int tgroups, splits;    // ... groups of kOwTaps taps, shares of its tiles
   bool data, weight;
@@ -53,8 +53,9 @@ struct OconvBwdArgs {
   int g_blocks, segs;     // pre-pass: blocks of the gradients, runs of 64 pixels per row
   uint32_t lw_inv;        // 2^20 / lw, rounded up
   int plane_chunks;
+  long d_work;            // tiles times blocks of channels of the data kernel
   int tgroups, splits, tiles;
-  int waves;              // data kernel: blocks of 32 input channels per workgroup
+  int waves, c_per, c_groups;  // data kernel: waves, blocks of 32 input channels per workgroup, workgroups per tile
 };
 
 hipError_t oconv_backward(int dtype, const OconvBwdPlan &pl, OconvBwdArgs a, unsigned char *ws, hipStream_t st);

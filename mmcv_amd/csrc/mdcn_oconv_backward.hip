@@ -89,14 +89,16 @@ __global__ __launch_bounds__(256) void oconv_bwd_prep_kernel(OconvBwdArgs a) {
 
 __device__ __forceinline__ int floor_div(int v, int d) { return v >= 0 ? v / d : -((-v + d - 1) / d); }
 
-// grad_input += conv_transpose(gradient, weight).  Workgroup = TH rows x 32 columns of the input and 32 input channels per
-// wave; the gradient pixels that the tile meets go to LDS pixel major (a block of 32 output channels at a
-// time), each wave multiplies weights (rows: input channels) with them (columns: pixels) tap by tap, so that
-// a tap is another LDS address, and a weight fragment serves TH products.  With a stride only some taps meet a pixel:
-// rows are skipped, lanes whose column a tap does not meet read a column of zeros.  The sum is added to
-// grad_input, which the deformable convolution's backward has written, and rounded once.  What bounds it: 16-bit types the
-// loads and stores of grad_input, two bytes a lane (its bytes alone, read and written, would take half of the time); fp32
-// the matrix units and how evenly the tiles fall on the CUs.
+// grad_input += conv_transpose(gradient, weight).  Workgroup = TH rows per wave x 32 columns of the input, and c_per blocks
+// of 32 input channels one after the other.  The gradient pixels that the tile meets go to LDS pixel major (a block of 32 output
+// channels at a time), each wave multiplies weights (rows: input channels) with them (columns: pixels) tap by tap, so that a
+// tap is another LDS address, and a weight fragment serves TH products of each wave -- the waves read it at about the
+// same time, three of them from L1.  With a stride only some taps meet a pixel: rows are skipped, lanes whose column a tap
+// does not meet read a column of zeros.  The sum is added to grad_input, which the deformable convolution's backward has
+// written, and rounded once.  What bounds it: 16-bit types the way to grad_input and back (its 249 MB would take 53 of the 111 us
+// of the first call in the header), fp32 the matrix units, whose rounds of waves are not full.  A wave with four rows and channels of
+// its own, every wave with its own weights from L2 then: 121 us, 13 and 30 us instead of 10 and 22 for N=2 and 8, 50x84.
+// Two pixels a lane on the way to grad_input, traded between neighbours, took longer (137 us).
 template <typename E, int TH, bool UNIT, int LDS_BYTES>
 __global__ __launch_bounds__(256, 2) void oconv_dgrad_kernel(OconvBwdArgs a) {
   using TR = ElemTraits<E>;
@@ -109,14 +111,16 @@ __global__ __launch_bounds__(256, 2) void oconv_dgrad_kernel(OconvBwdArgs a) {
   const int tid = threadIdx.x, nthr = a.waves * 64;
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int frow = lane & 31, fhalf = lane >> 5;
-  int b = (int)blockIdx.x;
-  const int cblocks = g.Cin / 32 / a.waves;
-  const int cblk = (b % cblocks) * a.waves + wave;
-  b /= cblocks;
-  const int tx = b % a.tiles_x;
+  // (neighbouring tiles share cache lines of grad_input and rows of their halo: an XCD has a run of them)
+  long b = xcd_work_index(a.d_work);
+  if (b < 0) return;
+  const int tx = (int)(b % a.tiles_x);
   b /= a.tiles_x;
-  const int y0 = b % a.tiles_y * TH, n = b / a.tiles_y, x0 = tx * 32;
-  const int ho0 = floor_div(y0 + g.ph - (g.kh - 1) * g.dh, g.sh);
+  const int yt = (int)(b % a.tiles_y) * TH * a.waves, x0 = tx * 32;
+  b /= a.tiles_y;
+  const int n = (int)(b / a.c_groups), c_first = (int)(b % a.c_groups) * a.c_per, c_end = min(c_first + a.c_per, g.Cin / 32);
+  const int y0 = yt + wave * TH;  // this wave's rows
+  const int ho0 = floor_div(yt + g.ph - (g.kh - 1) * g.dh, g.sh);
   const int wo0 = floor_div(x0 + g.pw - (g.kw - 1) * g.dw, g.sw);
   const int pitch = (a.gw_cols + 1) * RB;  // a column of zeros behind the last one
   unsigned char *L = (unsigned char *)lds;
@@ -126,94 +130,119 @@ __global__ __launch_bounds__(256, 2) void oconv_dgrad_kernel(OconvBwdArgs a) {
     coltab[i] = (w * g.sw == v ? w - wo0 : a.gw_cols) * RB;
   }
 
-  // (fp32: two sums of half the products each, whose roundings add up to less than those of one)
-  constexpr int NS = sizeof(E) == 4 ? 2 : 1;
-  f32x16 acc[TH][NS];
-#pragma unroll
-  for (int th = 0; th < TH; ++th)
-#pragma unroll
-    for (int s = 0; s < NS; ++s)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[th][s][r] = 0.0f;
-
-  const uint4 *wsrc = (const uint4 *)a.owf + (long)cblk * a.cob * g.taps * KQ * 64 + lane;
-  const int t_all = a.cob * g.taps;
+  const int t_end = c_end * a.cob * g.taps;
   uint4 wf[AHEAD][KQ];
   auto load_weights = [&](int t, uint4 (&w)[KQ]) {
-    const uint4 *src = wsrc + (long)min(t, t_all - 1) * (KQ * 64);  // (past the end: never used)
+    const uint4 *src = (const uint4 *)a.owf + (long)min(t, t_end - 1) * (KQ * 64) + lane;  // (past the end: never used)
 #pragma unroll
     for (int q = 0; q < KQ; ++q) w[q] = src[q * 64];
   };
 #pragma unroll
-  for (int i = 0; i < AHEAD; ++i) load_weights(i, wf[i]);
+  for (int i = 0; i < AHEAD; ++i) load_weights(c_first * a.cob * g.taps + i, wf[i]);
 
-  constexpr int CPP = 2 * KQ;  // 16-byte chunks of a record
-  for (int cb = 0; cb < a.cob; ++cb) {
-    __syncthreads();
-    const int cols = a.gw_cols + 1, items = a.gh * cols * CPP;
-    for (int i = tid; i < items; i += nthr) {
-      const int q = i % CPP, px = i / CPP, r = px / cols, c = px - r * cols;
-      const int ho = ho0 + r, wo = wo0 + c;
-      uint4 v = make_uint4(0u, 0u, 0u, 0u);
-      if (c < a.gw_cols && ho >= 0 && ho < g.Ho && wo >= 0 && wo < g.Wo)
-        v = ((const uint4 *)a.gpm)[((((long)n * g.Ho + ho) * g.Wo + wo) * a.cob + cb) * CPP + q];
-      *(uint4 *)(L + (long)px * RB + q * 16) = v;
-    }
-    __syncthreads();
-    int ti = 0, tj = 0;
-    for (int g0 = 0; g0 < g.taps; g0 += AHEAD) {
-      const int next = cb * g.taps + min(g0 + AHEAD, g.taps);
+  for (int cblk = c_first; cblk < c_end; ++cblk) {
+    // (fp32: two sums of half the products each, whose roundings add up to less than those of one)
+    constexpr int NS = sizeof(E) == 4 ? 2 : 1;
+    f32x16 acc[TH][NS];
 #pragma unroll
-      for (int i = 0; i < AHEAD; ++i) {
-        if (g0 + i < g.taps) {
-          const int col = coltab[tj * 32 + frow] + fhalf * 16;
-          int row[TH];
+    for (int th = 0; th < TH; ++th)
 #pragma unroll
-          for (int th = 0; th < TH; ++th) {
-            const int v = y0 + th + g.ph - ti * g.dh;
-            if constexpr (UNIT) {
-              row[th] = v - ho0;
-            } else {
-              const int h = floor_div(v, g.sh);
-              row[th] = h * g.sh == v ? h - ho0 : -1;
-            }
-          }
+      for (int s = 0; s < NS; ++s)
 #pragma unroll
-          for (int q = 0; q < KQ; ++q) {
-            // (read ahead of the branches: behind one, each product would wait for its own read)
-            uint4 gf[TH];
+        for (int r = 0; r < 16; ++r) acc[th][s][r] = 0.0f;
+
+    // What the sums are added to, on its way while they are formed.  Register r of lane l: input channel (r / 4) * 8 + (l / 32) * 4 +
+    // r % 4, column l % 32
+    const int x = x0 + frow;
+    const long plane_in = (long)g.H * g.W;
+    E *out = (E *)a.gin + ((long)n * g.Cin + cblk * 32 + fhalf * 4) * plane_in + (long)y0 * g.W + x;
+    auto at = [&](int th, int r) { return out + ((r >> 2) * 8 + (r & 3)) * plane_in + (long)th * g.W; };
+    E old[TH][16];
+    if (x < g.W) {
 #pragma unroll
-            for (int th = 0; th < TH; ++th) gf[th] = *(const uint4 *)(L + (UNIT ? row[th] : max(row[th], 0)) * pitch + col + q * 32);
+      for (int th = 0; th < TH; ++th) {
+        if (y0 + th >= g.H) break;
 #pragma unroll
-            for (int th = 0; th < TH; ++th)
-              if (UNIT || row[th] >= 0) TR::mma(acc[th][q % NS], wf[i][q], gf[th]);
-          }
-          if (++tj == g.kw) tj = 0, ++ti;
-        }
-        load_weights(next + i, wf[i]);
+        for (int r = 0; r < 16; ++r) old[th][r] = *at(th, r);
       }
     }
-  }
 
-  // register r of lane l: input channel (r / 4) * 8 + (l / 32) * 4 + r % 4, column l % 32
-  const int x = x0 + frow;
-  const long plane_in = (long)g.H * g.W;
-  E *out = (E *)a.gin + ((long)n * g.Cin + cblk * 32 + fhalf * 4) * plane_in + (long)y0 * g.W + x;
-  if (x < g.W) {
-    // (a row's values are on their way while the one before is stored)
-    E v[2][16];
-    auto load = [&](int th) {
+    constexpr int CPP = 2 * KQ;  // 16-byte chunks of a record
+    for (int cb = 0; cb < a.cob; ++cb) {
+      if (a.cob > 1 || cblk == c_first) {
+        __syncthreads();
+        const int cols = a.gw_cols + 1, items = a.gh * cols * CPP;
+        for (int i = tid; i < items; i += nthr) {
+          const int q = i % CPP, px = i / CPP, r = px / cols, c = px - r * cols;
+          const int ho = ho0 + r, wo = wo0 + c;
+          uint4 v = make_uint4(0u, 0u, 0u, 0u);
+          if (c < a.gw_cols && ho >= 0 && ho < g.Ho && wo >= 0 && wo < g.Wo)
+            v = ((const uint4 *)a.gpm)[((((long)n * g.Ho + ho) * g.Wo + wo) * a.cob + cb) * CPP + q];
+          *(uint4 *)(L + (long)px * RB + q * 16) = v;
+        }
+        __syncthreads();
+      }
+      const int t_base = (cblk * a.cob + cb) * g.taps;
+      // Operands are read a step ahead -- a step is 16 bytes of a tap -- and kept there: the compiler would put each read in front
+      // of its product, which then waits for it
+      auto rows_of = [&](int ti, int (&row)[TH]) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) v[th & 1][r] = out[((r >> 2) * 8 + (r & 3)) * plane_in + (long)th * g.W];
-    };
-    load(0);
+        for (int th = 0; th < TH; ++th) {
+          const int v = y0 + th + g.ph - ti * g.dh;
+          if constexpr (UNIT) {
+            row[th] = v - ho0;
+          } else {
+            const int h = floor_div(v, g.sh);
+            row[th] = h * g.sh == v ? h - ho0 : -1;
+          }
+        }
+      };
+      auto read = [&](const int (&row)[TH], int col, int q, uint4 (&gf)[TH]) {
 #pragma unroll
-    for (int th = 0; th < TH; ++th) {
-      if (y0 + th >= g.H) break;
-      if (th + 1 < TH && y0 + th + 1 < g.H) load(th + 1);
+        for (int th = 0; th < TH; ++th) gf[th] = *(const uint4 *)(L + (UNIT ? row[th] : max(row[th], 0)) * pitch + col + fhalf * 16 + q * 32);
+      };
+      int ti = 0, tj = 0, row[TH], row_next[TH];
+      int col = coltab[frow];
+      uint4 gf[2][TH];
+      rows_of(0, row);
+      read(row, col, 0, gf[0]);
+      for (int g0 = 0; g0 < g.taps; g0 += AHEAD) {
+        const int next = t_base + min(g0 + AHEAD, g.taps);
 #pragma unroll
-      for (int r = 0; r < 16; ++r)
-        out[((r >> 2) * 8 + (r & 3)) * plane_in + (long)th * g.W] = from_f32<E>(to_f32(v[th & 1][r]) + (NS == 2 ? acc[th][0][r] + acc[th][NS - 1][r] : acc[th][0][r]));
+        for (int i = 0; i < AHEAD; ++i) {
+          if (g0 + i < g.taps) {
+            if (g0 + i + 1 < g.taps && ++tj == g.kw) tj = 0, ++ti;
+            const int col_next = coltab[tj * 32 + frow];
+            rows_of(ti, row_next);
+#pragma unroll
+            for (int q = 0; q < KQ; ++q) {
+              if (q + 1 < KQ)
+                read(row, col, q + 1, gf[(q + 1) & 1]);
+              else
+                read(row_next, col_next, 0, gf[0]);
+              __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+              for (int th = 0; th < TH; ++th)
+                if (UNIT || row[th] >= 0) TR::mma(acc[th][q % NS], wf[i][q], gf[q & 1][th]);
+              __builtin_amdgcn_sched_barrier(0);
+            }
+            col = col_next;
+#pragma unroll
+            for (int th = 0; th < TH; ++th) row[th] = row_next[th];
+          }
+          load_weights(next + i, wf[i]);
+        }
+      }
+    }
+
+    if (x < g.W) {
+#pragma unroll
+      for (int th = 0; th < TH; ++th) {
+        if (y0 + th >= g.H) break;
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          *at(th, r) = from_f32<E>(to_f32(old[th][r]) + (NS == 2 ? acc[th][0][r] + acc[th][NS - 1][r] : acc[th][0][r]));
+      }
     }
   }
 }
@@ -230,8 +259,9 @@ typedef __attribute__((address_space(3))) s16x4_t *lds_s16x4_t;
 // them with LDS reads that transpose.  The gradients' copy is channel major, 16 bytes a lane (their chunks swizzled
 // against the rows).  A wave has taps of its own and all pixels, so that its sums are its own too; those of the shares meet in the
 // finishing launch.  Columns past the end of a row read its last pixel's input: their gradients are zero.
-// What bounds it: LDS reads (16-bit types: four of 16 bytes for three products) and the copies' latency; fp32 the matrix units.  Input
-// staged from NCHW by way of registers, transposed with VALU work, took 200 us where this takes 95.
+// What bounds it: the copies' latency between two barriers, LDS reads (16-bit types: four of 16 bytes for three products); fp32 the
+// matrix units.  Input staged from NCHW by way of registers, transposed with VALU work, took 200 us where this takes 93; reads
+// left in front of their products 36 instead of 31 (fp32, N=2, 256 channels, 50x84); six waves, two to three taps, 41.
 template <typename E, int LDS_BYTES>
 __global__ __launch_bounds__(64 * kOwWaves) void oconv_wgrad_kernel(OconvBwdArgs a, int TH) {
   using TR = ElemTraits<E>;
@@ -243,8 +273,12 @@ __global__ __launch_bounds__(64 * kOwWaves) void oconv_wgrad_kernel(OconvBwdArgs
   const int tid = threadIdx.x, waves = blockDim.x >> 6;
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int frow = lane & 31, fhalf = lane >> 5;
-  int b = (int)blockIdx.x;
+  // (an XCD has a run of the shares with all their channels: neighbouring tiles share rows of the input, the blocks of
+  // channels of a share its gradients)
   const int cblocks = g.Cin / 32;
+  const long work = xcd_work_index((long)a.splits * a.tgroups * a.cob * cblocks);
+  if (work < 0) return;
+  int b = (int)work;
   const int ci0 = b % cblocks * 32;
   b /= cblocks;
   const int cb = b % a.cob;
@@ -325,40 +359,54 @@ __global__ __launch_bounds__(64 * kOwWaves) void oconv_wgrad_kernel(OconvBwdArgs
         else
           colad[ks][k] = min(ks * 16 + (k >> 2) * 8 + fhalf * 4 + (k & 3), last) * g.sw * 32 + (frow >> 3) * PC * 16 + (frow & 7) * 4;
       }
+    // Operands are read a step ahead -- a step is a pair of 16 bytes of pixels -- and kept there: the compiler would put each read in
+    // front of its product, which then waits for it
+    auto read = [&](int row, int step, uint4 &gv, uint4 (&xv)[NT]) {
+      const int ks = step / NG, s = step % NG, c = (ks * 16) / EPV + 2 * s + fhalf;
+      gv = *(const uint4 *)(G + row * (32 * CHK * 16) + (c ^ (sizeof(E) == 2 ? (frow >> 2) & 3 : frow & 7)) * 16);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const unsigned char *p = X + (row * row_bytes + tapoff[t]);
+        if constexpr (sizeof(E) == 2) {
+          const s16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t)(lptr_t)(void *)(p + colad[ks][0]));
+          const s16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t)(lptr_t)(void *)(p + colad[ks][1]));
+          const uint2 l2 = __builtin_bit_cast(uint2, lo), h2 = __builtin_bit_cast(uint2, hi);
+          xv[t] = make_uint4(l2.x, l2.y, h2.x, h2.y);
+        } else {
+          xv[t] = make_uint4(*(const uint32_t *)(p + colad[ks][(4 * s) % NA]), *(const uint32_t *)(p + colad[ks][(4 * s + 1) % NA]),
+                             *(const uint32_t *)(p + colad[ks][(4 * s + 2) % NA]), *(const uint32_t *)(p + colad[ks][(4 * s + 3) % NA]));
+        }
+      }
+    };
     float tsum = 0.0f;
+    uint4 gv[2], xv[2][NT];
+    read(0, 0, gv[0], xv[0]);
     for (int row = 0; row < rows; ++row) {
-      const unsigned char *base = X + row * row_bytes;
+      // (nor sums of these and the row's and the tap's offsets for each of them, carried over the rows)
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-        for (int s = 0; s < NG; ++s) {
-          const int c = (ks * 16) / EPV + 2 * s + fhalf;
-          const uint4 gv = *(const uint4 *)(G + row * (32 * CHK * 16) + (c ^ (sizeof(E) == 2 ? (frow >> 2) & 3 : frow & 7)) * 16);
-          uint4 xv[NT];
+        for (int k = 0; k < NA; ++k) asm volatile("" : "+v"(colad[ks][k]));
 #pragma unroll
-          for (int t = 0; t < NT; ++t) {
-            const unsigned char *p = base + tapoff[t];
-            if constexpr (sizeof(E) == 2) {
-              const s16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t)(lptr_t)(void *)(p + colad[ks][0]));
-              const s16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t)(lptr_t)(void *)(p + colad[ks][1]));
-              const uint2 l2 = __builtin_bit_cast(uint2, lo), h2 = __builtin_bit_cast(uint2, hi);
-              xv[t] = make_uint4(l2.x, l2.y, h2.x, h2.y);
-            } else {
-              xv[t] = make_uint4(*(const uint32_t *)(p + colad[ks][(4 * s) % NA]), *(const uint32_t *)(p + colad[ks][(4 * s + 1) % NA]),
-                                 *(const uint32_t *)(p + colad[ks][(4 * s + 2) % NA]), *(const uint32_t *)(p + colad[ks][(4 * s + 3) % NA]));
-            }
-          }
+      for (int step = 0; step < 2 * NG; ++step) {
+        const int cur = step & 1;
+        if (step + 1 < 2 * NG)
+          read(row, step + 1, gv[cur ^ 1], xv[cur ^ 1]);
+        else
+          read(min(row + 1, rows - 1), 0, gv[cur ^ 1], xv[cur ^ 1]);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-          for (int t = 0; t < NT; ++t) TR::mma(acc[t], gv, xv[t]);
-          if (sums) {
-            E e[EPV];
-            __builtin_memcpy(e, &gv, 16);
-            float v = 0.0f;
+        for (int t = 0; t < NT; ++t) TR::mma(acc[t], gv[cur], xv[cur][t]);
+        if (sums) {
+          E e[EPV];
+          __builtin_memcpy(e, &gv[cur], 16);
+          float v = 0.0f;
 #pragma unroll
-            for (int k = 0; k < EPV; k += 4) v += (to_f32(e[k]) + to_f32(e[k + 1])) + (to_f32(e[k + 2]) + to_f32(e[k + 3]));
-            tsum += v;
-          }
+          for (int k = 0; k < EPV; k += 4) v += (to_f32(e[k]) + to_f32(e[k + 1])) + (to_f32(e[k + 2]) + to_f32(e[k + 3]));
+          tsum += v;
         }
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
     bsum += tsum;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -431,31 +479,32 @@ hipError_t run(const OconvBwdPlan &pl, OconvBwdArgs a, hipStream_t st) {
   hipLaunchKernelGGL(oconv_bwd_prep_kernel<E>, dim3((unsigned)(a.g_blocks + (frags + 255) / 256)), dim3(256), 0, st, a);
   if (pl.data) {
     OconvBwdArgs d = a;
-    d.waves = 4;
-    while (g.Cin / 32 % d.waves) --d.waves;
+    d.waves = pl.d_waves;
     d.gh = pl.gh;
     d.gw_cols = pl.gw;
-    d.tiles_y = (g.H + pl.d_th - 1) / pl.d_th;
+    d.c_per = pl.d_cper;
+    d.c_groups = (g.Cin / 32 + d.c_per - 1) / d.c_per;
+    const int rows = pl.d_th * d.waves;
+    d.tiles_y = (g.H + rows - 1) / rows;
     d.tiles_x = (g.W + 31) / 32;
-    const dim3 grid((unsigned)((long)g.N * d.tiles_y * d.tiles_x * (g.Cin / 32 / d.waves))), block(d.waves * 64);
-    auto launch = [&](auto th) {
-      constexpr int TH = decltype(th)::value;
-      const bool small = pl.d_lds <= kOdLdsSmall;
-      if (g.sh == 1 && small)
-        hipLaunchKernelGGL((oconv_dgrad_kernel<E, TH, true, kOdLdsSmall>), grid, block, 0, st, d);
-      else if (g.sh == 1)
-        hipLaunchKernelGGL((oconv_dgrad_kernel<E, TH, true, kOdLds>), grid, block, 0, st, d);
-      else if (small)
-        hipLaunchKernelGGL((oconv_dgrad_kernel<E, TH, false, kOdLdsSmall>), grid, block, 0, st, d);
-      else
-        hipLaunchKernelGGL((oconv_dgrad_kernel<E, TH, false, kOdLds>), grid, block, 0, st, d);
+    d.d_work = (long)g.N * d.tiles_y * d.tiles_x * d.c_groups;
+    const dim3 grid((unsigned)((d.d_work + 7) / 8 * 8)), block(d.waves * 64);
+    auto launch = [&](auto th, auto unit, auto bytes) {
+      constexpr int TH = decltype(th)::value, LDS = decltype(bytes)::value;
+      hipLaunchKernelGGL((oconv_dgrad_kernel<E, TH, decltype(unit)::value, LDS>), grid, block, 0, st, d);
     };
-    if (pl.d_th == 4)
-      launch(std::integral_constant<int, 4>());
-    else if (pl.d_th == 2)
-      launch(std::integral_constant<int, 2>());
+    auto launch_th = [&](auto th) {
+      using Small = std::integral_constant<int, kOdLdsSmall>;
+      using Big = std::integral_constant<int, kOdLds>;
+      if (g.sh == 1)
+        pl.d_lds <= kOdLdsSmall ? launch(th, std::true_type(), Small()) : launch(th, std::true_type(), Big());
+      else
+        pl.d_lds <= kOdLdsSmall ? launch(th, std::false_type(), Small()) : launch(th, std::false_type(), Big());
+    };
+    if (pl.d_th == 2)
+      launch_th(std::integral_constant<int, 2>());
     else
-      launch(std::integral_constant<int, 1>());
+      launch_th(std::integral_constant<int, 1>());
   }
   if (pl.weight) {
     a.tiles_y = (g.Ho + pl.w_th - 1) / pl.w_th;
@@ -472,7 +521,7 @@ hipError_t run(const OconvBwdPlan &pl, OconvBwdArgs a, hipStream_t st) {
       hipLaunchKernelGGL((relayout_vec_kernel<E, true, 32>), dim3((unsigned)((long)g.N * (g.Cin / (8 * EPV)) * n_pchunks)), dim3(256), 0,
                          st, g, (const E *)a.x, (E *)a.own_xt, n_pchunks);
     }
-    const dim3 grid((unsigned)((long)pl.splits * pl.tgroups * a.cob * (g.Cin / 32)));
+    const dim3 grid((unsigned)(((long)pl.splits * pl.tgroups * a.cob * (g.Cin / 32) + 7) / 8 * 8));
     const dim3 block(64 * std::min(kOwWaves, (g.taps + kOwTaps / kOwWaves - 1) / (kOwTaps / kOwWaves)));
     if (pl.w_lds <= kOwLds3)
       hipLaunchKernelGGL((oconv_wgrad_kernel<E, kOwLds3>), grid, block, 0, st, a, pl.w_th);
@@ -500,23 +549,24 @@ bool oconv_bwd_plan(const Geom &g, int dtype, bool unmodulated, bool data, bool 
   const long limit = 1L << 30;  // blocks of a launch, pixels of a plane
   if ((long)g.H * g.W > limit || (long)g.N * g.Ho * ((pl->Wp + 63) / 64) > limit) return false;
 
-  // data: the rows a workgroup with which the fullest CU has the least to do (a row's worth for its halo and its
-  // weights on top)
+  // data: four waves, fewer where their rows' halo does not fit; as many rows a wave (fp32: one) and blocks of channels a
+  // workgroup as leave four and eight workgroups per CU
   const int rb = 32 * es + 16;
   auto halo = [](long n, long k, long d, long s) { return (n - 1 + (k - 1) * d) / s + (s > 1 ? 2 : 1); };
   const long gw = halo(32, g.kw, g.dw, g.sw);
-  auto d_lds = [&](int th) { return halo(th, g.kh, g.dh, g.sh) * (gw + 1) * rb; };
-  int waves = 4;
-  while (g.Cin / 32 % waves) --waves;
-  auto d_groups = [&](int th) { return (long)g.N * ((g.H + th - 1) / th) * ((g.W + 31) / 32) * (g.Cin / 32 / waves); };
-  auto d_cost = [&](int th) { return (double)((d_groups(th) * waves + 4L * cus - 1) / (4L * cus)) * (th + 0.25); };
-  pl->d_th = 0;
-  for (int th : {4, 2, 1})
-    if (d_lds(th) <= kOdLds && (pl->d_th == 0 || d_cost(th) < d_cost(pl->d_th))) pl->d_th = th;
-  if (pl->d_th == 0 || d_groups(pl->d_th) > limit) return false;
-  pl->d_lds = (int)d_lds(pl->d_th);
+  auto d_lds = [&](long rows) { return halo(rows, g.kh, g.dh, g.sh) * (gw + 1) * rb; };
+  pl->d_waves = 4;
+  while (pl->d_waves > 1 && d_lds(pl->d_waves) > kOdLds) --pl->d_waves;
+  const int waves = pl->d_waves, cblocks = g.Cin / 32;
+  auto d_tiles = [&](int th) { return (long)g.N * ((g.H + th * waves - 1) / (th * waves)) * ((g.W + 31) / 32); };
+  pl->d_th = es == 2 ? 2 : g.sh == 1 ? 1 : 2;  // (of two rows at a stride one meets fewer taps)
+  while (pl->d_th > 1 && (d_lds(pl->d_th * waves) > kOdLds || d_tiles(pl->d_th) * cblocks < 4L * cus)) pl->d_th /= 2;
+  pl->d_cper = 1;
+  while (pl->cob == 1 && pl->d_cper * 2 <= cblocks && d_tiles(pl->d_th) * (cblocks / (pl->d_cper * 2)) >= 8L * cus) pl->d_cper *= 2;
+  if (d_lds(pl->d_th * waves) > kOdLds || d_tiles(pl->d_th) * cblocks > limit) return false;
+  pl->d_lds = (int)d_lds(pl->d_th * waves);
   pl->gw = (int)gw;
-  pl->gh = (int)halo(pl->d_th, g.kh, g.dh, g.sh);
+  pl->gh = (int)halo(pl->d_th * waves, g.kh, g.dh, g.sh);
 
   // weight: the same for the rows of its tiles, whose LDS says how many workgroups share a CU
   const long lw = 31L * g.sw + (long)(g.kw - 1) * g.dw + 1;
