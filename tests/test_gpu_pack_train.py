@@ -140,6 +140,50 @@ def test_gradients_that_are_asked_for():
             assert float((g - want[n]).abs().max()) <= 1e-5 * float(want[n].abs().max()), (take, n)
 
 
+@pytest.mark.parametrize('form', ['channels_last', 'weights_channels_last', 'slice', 'transposed', 'gradient_expanded',
+                                  'gradient_transposed', 'unaligned', 'saved_on_cpu', 'no_offset_bias', 'other_stream'])
+def test_forms(monkeypatch, form):
+    """Orders and strides of what a call is given, against the layer's own sequence of operations."""
+    import contextlib
+    from mmcv_amd.ops import ModulatedDeformConv2dPack
+    monkeypatch.setattr(torch.backends.cudnn, 'deterministic', True)
+    layer, x = _layer(ModulatedDeformConv2dPack, (2, 64, 48, 11, 13, 3, 1, 1, 1, 1), torch.float32)
+    go = torch.randn(2, 48, 11, 13, device='cuda')
+    if form == 'channels_last':
+        x = x.to(memory_format=torch.channels_last)
+    elif form == 'weights_channels_last':
+        layer = layer.to(memory_format=torch.channels_last)
+    elif form == 'slice':
+        x = torch.randn(2, 70, 14, 13, device='cuda')[:, 3:67, 2:13]
+    elif form == 'transposed':
+        x = x.transpose(2, 3).contiguous().transpose(2, 3)
+    elif form == 'gradient_expanded':
+        go = torch.randn(1, 48, 1, 1, device='cuda').expand(2, 48, 11, 13)
+    elif form == 'gradient_transposed':
+        go = go.transpose(2, 3).contiguous().transpose(2, 3)
+    elif form == 'unaligned':
+        x = torch.randn(x.numel() + 1, device='cuda')[1:].view(x.shape)
+    elif form == 'no_offset_bias':
+        layer.conv_offset.bias = None
+    assert form != 'slice' or not x.is_contiguous()
+    got = []
+    for fuse in ('none', 'full'):
+        layer.fuse = fuse
+        stream = torch.cuda.Stream() if form == 'other_stream' else torch.cuda.current_stream()
+        stream.wait_stream(torch.cuda.current_stream())
+        hooks = torch.autograd.graph.save_on_cpu() if form == 'saved_on_cpu' else contextlib.nullcontext()
+        with torch.cuda.stream(stream), hooks:
+            x1 = x.detach().requires_grad_(True)
+            y = layer(x1)
+            names = [x1] + list(layer.parameters())
+            grads = torch.autograd.grad(y, names, go)
+        torch.cuda.synchronize()
+        got.append((y.detach(),) + grads)
+    assert torch.equal(got[0][0], got[1][0])
+    for a, b in zip(*got):  # (sums in fp32 of up to 1 728 terms, in other orders)
+        assert a.shape == b.shape and float((a - b).abs().max()) <= 1e-5 * float(a.abs().max())
+
+
 def test_second_derivative_raises():
     from mmcv_amd.ops import ModulatedDeformConv2dPack
     layer, x = _layer(ModulatedDeformConv2dPack, SHAPES[0], torch.float32)
