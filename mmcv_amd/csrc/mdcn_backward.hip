@@ -368,16 +368,24 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
     a.far = far;
     a.bpart = bpart;
     a.bsplits = pl.bsplits;
+    // The bias sums read grad_output a second time.  At the end of the launch they find it in the last-level cache (256 MB) unless
+    // what the jobs between move -- its re-layout, the zeros of grad_input -- is more than that holds; right behind the re-layout
+    // they find its end.  Whole launch in us at the end / behind the re-layout: bf16, 256 channels 100x152, N=8 (249 MB
+    // between) 76 / 79, N=9 (280) 87.6 / 85.9, N=10 (311) 98 / 95, N=16 (498) 175 / 163; 128 channels 200x200, N=16 (655) 230 / 194; fp32,
+    // 256 channels 100x152, N=6 (280) 88 / 91, N=8 (374) 128 / 124; N=2 50x84 14.4 / 16.7.
+    const bool early = 2.0 * g.N * g.Cout * plane_out * sizeof(E) + 4.0 * n_in > 300e6;
+    const int bias_blocks = bp->grad_bias ? g.Cout * pl.bsplits : 0;
     const int jobs[kPreJobs] = {
         g.N * up(cin_p, KC) * a.x_chunks,
         gemm ? g.N * (cout_p / KC) * a.g_chunks : 0,
+        early ? bias_blocks : 0,
         pl.gpad_bytes ? up((long)g.N * g.Cout * (pl.P_pad / EPV), 256) : 0,
         gemm ? up(n_in, kPreZeroPerBlock) : 0,
         wgemm && pl.P_pad > plane_out ? up(a.col_rows * (pl.P_pad - plane_out), kPrePadPerBlock) : 0,
         gemm ? up((long)g.G * pl.M_pad * pl.om.cgp, 256) : 0,
         pl.n_wnorm,
         gemm && pl.fWH ? far_blocks : 0,
-        bp->grad_bias ? g.Cout * pl.bsplits : 0,
+        early ? 0 : bias_blocks,
     };
     int total = 0;
     for (int j = 0; j < kPreJobs; ++j) a.end[j] = total += jobs[j];

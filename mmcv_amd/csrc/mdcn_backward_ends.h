@@ -11,8 +11,8 @@
 
 namespace mdcn {
 
-constexpr int kPreJobs = 9;
-enum { kPreX, kPreG, kPreRows, kPreZero, kPreColPad, kPreWeight, kPreNorm, kPreFar, kPreBias };
+constexpr int kPreJobs = 10;
+enum { kPreX, kPreG, kPreBiasEarly, kPreRows, kPreZero, kPreColPad, kPreWeight, kPreNorm, kPreFar, kPreBias };
 
 struct BwdPreArgs {
   Geom g;
@@ -59,9 +59,38 @@ __global__ __launch_bounds__(256) void bwd_prepass_kernel(BwdPreArgs a) {
     relayout_vec_block<E, false, 128, true>(gg, (const E *)a.gout, (E *)a.gT, a.g_chunks, b - a.end[kPreX], a.om, a.cout_p);
     return;
   }
+  __shared__ float red[4];
+  if (b >= a.end[kPreFar] || (b >= a.end[kPreG] && b < a.end[kPreBiasEarly])) {
+    // sums of grad_output over the pixels, a share of an output channel's runs per block (in one of two places of the launch)
+    const int bi = b - (b >= a.end[kPreFar] ? a.end[kPreFar] : a.end[kPreG]);
+    const int co = bi / a.bsplits, split = bi - co * a.bsplits;
+    const int runs = (int)((plane + kBiasRun - 1) / kBiasRun);
+    float s = 0.0f;
+    for (int w = split; w < g.N * runs; w += a.bsplits) {
+      const int n = w / runs, p0 = (w - n * runs) * kBiasRun;
+      const int len = (int)min((long)kBiasRun, plane - p0);
+      const E *src = (const E *)a.gout + ((long)n * g.Cout + co) * plane + p0;
+      const int nv = len / EPV;
+#pragma unroll 4
+      for (int v = tid; v < nv; v += 256) {
+        uint4 q;
+        __builtin_memcpy(&q, src + (long)v * EPV, 16);
+        const E *e = (const E *)&q;
+#pragma unroll
+        for (int i = 0; i < EPV; ++i) s += to_f32(e[i]);
+      }
+      for (int i = nv * EPV + tid; i < len; i += 256) s += to_f32(src[i]);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+    if ((tid & 63) == 0) red[tid >> 6] = s;
+    __syncthreads();
+    if (tid == 0) a.bpart[(long)co * a.bsplits + split] = (red[0] + red[1]) + (red[2] + red[3]);
+    return;
+  }
   if (b < a.end[kPreRows]) {  // grad_output with rows that start 16-byte aligned, zeros behind the image
     const long per_row = a.P_pad / EPV;
-    const long i = (long)(b - a.end[kPreG]) * 256 + tid;
+    const long i = (long)(b - a.end[kPreBiasEarly]) * 256 + tid;
     const long r = i / per_row;
     const int p = (int)(i - r * per_row) * EPV;
     if (r >= (long)g.N * g.Cout) return;
@@ -122,7 +151,6 @@ __global__ __launch_bounds__(256) void bwd_prepass_kernel(BwdPreArgs a) {
     ((E *)a.wT)[idx] = v;
     return;
   }
-  __shared__ float red[4];
   if (b < a.end[kPreNorm]) {  // bound on the norms over the output channels of a group of 64 (channel, tap)
     __shared__ float sq[256];
     __shared__ uint32_t big[256];
@@ -155,7 +183,7 @@ __global__ __launch_bounds__(256) void bwd_prepass_kernel(BwdPreArgs a) {
     }
     return;
   }
-  if (b < a.end[kPreFar]) {  // offsets that leave the scatter kernel's window, counted in a sample
+  {  // offsets that leave the scatter kernel's window, counted in a sample
     const int nb = a.end[kPreFar] - a.end[kPreNorm], bi = b - a.end[kPreNorm];
     float cnt = 0.0f;  // (64 Ki samples at most: exact)
     for (long i = ((long)bi * 256 + tid) * a.off_step; i < a.n_off; i += (long)nb * 256 * a.off_step)
@@ -166,32 +194,6 @@ __global__ __launch_bounds__(256) void bwd_prepass_kernel(BwdPreArgs a) {
     __syncthreads();
     if (tid == 0) a.far[bi] = (uint32_t)((red[0] + red[1]) + (red[2] + red[3]));
     return;
-  }
-  {  // sums of grad_output over the pixels, a share of an output channel's runs per block
-    const int bi = b - a.end[kPreFar];
-    const int co = bi / a.bsplits, split = bi - co * a.bsplits;
-    const int runs = (int)((plane + kBiasRun - 1) / kBiasRun);
-    float s = 0.0f;
-    for (int w = split; w < g.N * runs; w += a.bsplits) {
-      const int n = w / runs, p0 = (w - n * runs) * kBiasRun;
-      const int len = (int)min((long)kBiasRun, plane - p0);
-      const E *src = (const E *)a.gout + ((long)n * g.Cout + co) * plane + p0;
-      const int nv = len / EPV;
-#pragma unroll 4
-      for (int v = tid; v < nv; v += 256) {
-        uint4 q;
-        __builtin_memcpy(&q, src + (long)v * EPV, 16);
-        const E *e = (const E *)&q;
-#pragma unroll
-        for (int i = 0; i < EPV; ++i) s += to_f32(e[i]);
-      }
-      for (int i = nv * EPV + tid; i < len; i += 256) s += to_f32(src[i]);
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-    if ((tid & 63) == 0) red[tid >> 6] = s;
-    __syncthreads();
-    if (tid == 0) a.bpart[(long)co * a.bsplits + split] = (red[0] + red[1]) + (red[2] + red[3]);
   }
 }
 
