@@ -38,7 +38,7 @@ void make_bwd_plan(const mdcn_bwd_params *bp, const Geom &g, uint64_t pass_bytes
   pl->gb_bytes = (staged && bp->grad_bias) ? align_up((size_t)g.Cout * 4) : 0;
   pl->mx_bytes = 0;
   pl->tiled = pl->gemm = pl->wgemm = pl->fused = false;
-  pl->n_wnorm = pl->tw_log = 0;
+  pl->tw_log = 0;
   pl->xt_bytes = pl->gt_bytes = pl->wt_bytes = pl->d_bytes = pl->col_bytes = pl->part_bytes = pl->wpart_bytes = 0;
   pl->w_tile = kCgTile;
   pl->w_splits = 1;
@@ -157,8 +157,7 @@ void make_bwd_plan(const mdcn_bwd_params *bp, const Geom &g, uint64_t pass_bytes
     pl->gt_bytes = align_up((size_t)g.N * g.G * om.cgp * plane_out * es);
     pl->wt_bytes = align_up((size_t)g.G * pl->M_pad * om.cgp * es);
     pl->d_bytes = pl->fused ? 0 : align_up(d_img * pl->n_chunk);
-    pl->n_wnorm = pl->fused ? g.G * ((g.cin_g * g.taps + 63) / 64) : 0;
-    pl->mx_bytes = kAlign + align_up((size_t)pl->n_wnorm * 4);
+    pl->mx_bytes = kAlign;
     if (pl->fused)
       pl->part_bytes = align_up((size_t)((g.N + pl->n_chunk - 1) / pl->n_chunk) * FusedSchedule::kGroups * 3 * g.taps * 256 * 4);
     else if (pl->parts > 1)
@@ -316,7 +315,6 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
   float *gin32 = staged ? gin_staging : (float *)bp->grad_input;
   float *bpart = (float *)take(pl.gb_bytes);
   uint32_t *far = (uint32_t *)take(pl.mx_bytes);
-  uint32_t *wnorm = far + kAlign / 4;
   unsigned char *xt = take(pl.xt_bytes), *gT = take(pl.gt_bytes), *wT = take(pl.wt_bytes);
   unsigned char *D = take(pl.d_bytes), *col = take(pl.col_bytes);
   const long off_total = (long)g.N * g.DG * 2 * g.taps * plane_out, mask_total = off_total / 2;
@@ -360,7 +358,6 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
     a.run = pl.sCH;
     a.col_rows = (long)pl.n_chunk * g.taps * cin_p;
     a.M_pad = pl.M_pad;
-    a.wnorm = wnorm;
     a.off = p->offset;
     a.n_off = off_total;
     a.off_step = off_step;
@@ -383,7 +380,6 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
         gemm ? up(n_in, kPreZeroPerBlock) : 0,
         wgemm && pl.P_pad > plane_out ? up(a.col_rows * (pl.P_pad - plane_out), kPrePadPerBlock) : 0,
         gemm ? up((long)g.G * pl.M_pad * pl.om.cgp, 256) : 0,
-        pl.n_wnorm,
         gemm && pl.fWH ? far_blocks : 0,
         early ? 0 : bias_blocks,
     };
@@ -445,8 +441,6 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
         fa.sched = pl.sched;
         fa.sched.tiles = pl.sched.tiles / pl.n_chunk * nb;
         fa.part = poff + (long)(n0 / pl.n_chunk) * FusedSchedule::kGroups * 3 * g.taps * 256;
-        fa.wnorm = wnorm;
-        fa.n_wnorm = pl.n_wnorm;
         launch_fused<E>(fa, pl.sCH, st);
         check();
       }

@@ -11,8 +11,8 @@
 
 namespace mdcn {
 
-constexpr int kPreJobs = 10;
-enum { kPreX, kPreG, kPreBiasEarly, kPreRows, kPreZero, kPreColPad, kPreWeight, kPreNorm, kPreFar, kPreBias };
+constexpr int kPreJobs = 9;
+enum { kPreX, kPreG, kPreBiasEarly, kPreRows, kPreZero, kPreColPad, kPreWeight, kPreFar, kPreBias };
 
 struct BwdPreArgs {
   Geom g;
@@ -28,7 +28,6 @@ struct BwdPreArgs {
   long col_rows;           // rows of col whose padding is cleared
   int run;                 // WGradArgs::run
   int M_pad;
-  uint32_t *wnorm;         // bound on the norm of 64 rows of the weight matrix, one per block of the job
   const void *off;
   long n_off, off_step;    // one offset in off_step is looked at
   float far_from;          // ... and counted when it is larger than this
@@ -151,40 +150,8 @@ __global__ __launch_bounds__(256) void bwd_prepass_kernel(BwdPreArgs a) {
     ((E *)a.wT)[idx] = v;
     return;
   }
-  if (b < a.end[kPreNorm]) {  // bound on the norms over the output channels of a group of 64 (channel, tap)
-    __shared__ float sq[256];
-    __shared__ uint32_t big[256];
-    const int L = g.cin_g * g.taps, runs = (L + 63) / 64;
-    const int bi = b - a.end[kPreWeight], grp = bi / runs;
-    const int q = (bi - grp * runs) * 64 + (tid & 63);
-    float ss = 0.0f;
-    uint32_t mx = 0u;
-    if (q < L) {
-      const E *src = (const E *)a.w + (long)grp * g.cout_g * L + q;
-#pragma unroll 8
-      for (int co = tid >> 6; co < g.cout_g; co += 4) {
-        const float v = to_f32(src[(long)co * L]);
-        ss = fmaf(v, v, ss);
-        mx = max(mx, __float_as_uint(v) & 0x7fffffffu);
-      }
-    }
-    sq[tid] = ss;
-    big[tid] = mx;
-    __syncthreads();
-    if (tid < 64) {
-      for (int w = 1; w < 4; ++w) {
-        ss += sq[w * 64 + tid];
-        mx = max(mx, big[w * 64 + tid]);
-      }
-      uint32_t nb = norm_bound(ss, mx, g.cout_g);
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) nb = max(nb, (uint32_t)__shfl_xor((int)nb, o));
-      if (tid == 0) a.wnorm[bi] = nb;
-    }
-    return;
-  }
   {  // offsets that leave the scatter kernel's window, counted in a sample
-    const int nb = a.end[kPreFar] - a.end[kPreNorm], bi = b - a.end[kPreNorm];
+    const int nb = a.end[kPreFar] - a.end[kPreWeight], bi = b - a.end[kPreWeight];
     float cnt = 0.0f;  // (64 Ki samples at most: exact)
     for (long i = ((long)bi * 256 + tid) * a.off_step; i < a.n_off; i += (long)nb * 256 * a.off_step)
       cnt += fabsf(to_f32(((const E *)a.off)[i])) > a.far_from ? 1.0f : 0.0f;

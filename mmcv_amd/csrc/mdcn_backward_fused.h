@@ -24,8 +24,6 @@ constexpr int bf_window_px(int ch) { return (kBfLdsBytes - 2 * bf_stage_bytes(ch
 constexpr float kRoundMagic = 12582912.0f;          // 1.5 * 2^23: adding it leaves an integer in the mantissa
 constexpr uint32_t kRoundBits = 0x4B400000u;        // ... on top of these bits
 
-typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
-
 struct BwdFusedArgs {
   Geom g;
   const void *xt;   // zero-bordered input copy in 32-byte records [N][Cin / 16][H + 2][W + 2][16]
@@ -46,16 +44,17 @@ struct BwdFusedArgs {
   int n0;           // first image of the pass
   FusedSchedule sched;
   float *part;      // [workgroup][3 taps][256]: sums of the offset (y and x of a tap) and mask gradients of a share of a tile
-  const uint32_t *wnorm;   // bounds on the norm of a row of wT, as bits; n_wnorm of them
-  int n_wnorm;
 };
 
-// An upper bound of the 2-norm of k numbers whose squares add up to `ss` and whose largest has the bits `mx`; infinite or
-// NaN if one of them is.  (Squares outside of fp32's range: the largest times the root of their number.)
-__device__ __forceinline__ uint32_t norm_bound(float ss, uint32_t mx, int k) {
-  const float m = __uint_as_float(mx);
-  const bool plain = m > 1e-15f && m < 1e15f;
-  return __float_as_uint(1.0005f * (plain ? sqrtf(ss) : m * sqrtf((float)k)));
+// The largest value of a wavefront's lanes.
+__device__ __forceinline__ uint32_t wave_max(uint32_t v) {
+  // (within rows of 16 lanes, rotated by 8, 4, 2 and 1)
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x128, 0xf, 0xf, false));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x124, 0xf, 0xf, false));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x122, 0xf, 0xf, false));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x121, 0xf, 0xf, false));
+  return max(max((uint32_t)__builtin_amdgcn_readlane((int)v, 0), (uint32_t)__builtin_amdgcn_readlane((int)v, 16)),
+             max((uint32_t)__builtin_amdgcn_readlane((int)v, 32), (uint32_t)__builtin_amdgcn_readlane((int)v, 48)));
 }
 
 // One tile of 256 output pixels (tile b), channels [c_first, c_last) of its deformable group; part: where the sums of a share go,
@@ -69,13 +68,18 @@ __device__ __forceinline__ uint32_t norm_bound(float ss, uint32_t mx, int k) {
 // Every wait in it is for loads that are due: whatever the compiler keeps in scratch or fetches from the argument block
 // again there makes it wait for all loads, or all LDS adds, under way (the kernel took 2.1 ms in the shape below with either,
 // 1.35 without).  Hence the asm statements without text below: they hold a sum where it is, and a value in its register.
-// Window: 32-bit fixed point in LDS.  Its scale comes from bounds this workgroup takes itself -- |d| is at most the norm of
-// the pixel's grad_output times that of a row of weights -- so that no sum of contributions leaves 2^30 and no
-// contribution 2^21.  What is added to an entry is the bit pattern of fmaf(weight, d, 1.5 * 2^23), for two channels at
+// Window: 32-bit fixed point in LDS.  Its scale is the pass's own: from the largest |d| of its products over the tile, the largest
+// mask value and the number of adds the busiest entry sees, so that no contribution leaves 2^21 and no sum of them 2^30.  The
+// first decides where no entry sees more than 512, and the quantum is then 2^-20 or 2^-21 of the largest contribution there could
+// be.  (Bounds of |d| from norms of grad_output and weights instead: training calls of N=16 256 channels 100x152 in bf16 2 319
+// us where this takes 2 329, of N=8 512 channels 25x42 in fp16 371 / 363.  But such a scale goes by gradients that the weights do not
+// carry on: fp16, 256 output channels, one of them without weights and with 300 times the gradient: error of grad_input
+// 8.6e-4 of its norm, where its one rounding is 2.1e-4 and this stays at that.)
+// What is added to an entry is the bit pattern of fmaf(weight, d, 1.5 * 2^23), for two channels at
 // once: every tap of every pixel adds to four entries, the same ones for all channels, so the number of adds an entry has
 // seen is known from a count made once per tile, and what the patterns hold beside the integers is subtracted when the entry is
-// read.  (Two instructions per channel and corner, where taking it off each contribution was six per two.)  Where grad_output,
-// weights or mask are not finite, or so small or large that no scale fits, nothing goes through the window.
+// read.  (Two instructions per channel and corner, where taking it off each contribution was six per two.)  In a pass where d or
+// the mask is not finite, or so small or large that no scale fits, nothing goes through the window.
 // Samples beyond the window are added to memory one at a time, a lane for every channel and corner.
 //
 // bf16, N=16, 256 -> 256 channels, 100x152: 1.35 ms for what took 0.52 (column gradient to memory) + 1.50 (scatter kernel reading
@@ -138,7 +142,7 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
       t_m[i] = (uint32_t)__builtin_bit_cast(uint16_t, msk[(long)tc * a.om.msk_ch]) | (half ? at1 : at0) << 16;
     }
   }
-  float *lone = red + 3 * kBfWaves + wave * 16;   // of this wavefront
+  float *lone = red + 4 * kBfWaves + wave * 16;   // of this wavefront
   const int items = (g.taps + 1) / 2, blocks = (items + PER - 1) / PER;
 
   // (1: unmodulated)
@@ -217,94 +221,39 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
   };
   issue_first(c_begin);
 
-  // Bounds and scale.  (The barrier also ends the tile before: nobody is at the window any more.)
+  // (The barrier ends the tile before: nobody is at the window any more.)
   __syncthreads();
-  const int grp0 = group_of(c_begin), grp1 = group_of(c_end - 1);
-  bool fits;
-  float scale, inv_scale;
+  load_g(group_of(c_begin), 0);
+  // (the counts of adds go where the window will be)
+  for (int i = tid; i < win_px; i += kBfThreads) ((uint32_t *)win)[i] = 0u;
+  // Largest mask value, and the sum of all of the tile's
   {
-    uint32_t norm = 0u;
-    for (int grp = grp0; grp <= grp1; ++grp) {
-      float ss = 0.0f;
-      u16x2 big = {0, 0};   // largest magnitudes, as bits
-#pragma unroll 1
-      for (int k = 0; k < g.cout_g / 64; ++k) {
-        uint4 v[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = g_at(grp, k / 2, k % 2 * 4 + j);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const uint32_t w[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            ss = TR::dot2(w[q], w[q], ss);
-            const u16x2 m = __builtin_bit_cast(u16x2, w[q] & 0x7fff7fffu);
-            big = __builtin_elementwise_max(big, m);
-          }
-        }
-      }
-      uint32_t mx = __float_as_uint(to_f32(__builtin_bit_cast(E, max(big.x, big.y))));
-      ss += __shfl_xor(ss, 32);
-      mx = max(mx, (uint32_t)__shfl_xor((int)mx, 32));
-      norm = max(norm, norm_bound(ss, mx, g.cout_g));
-    }
-    load_g(grp0, 0);
-    float msum = 0.0f;
-    uint32_t mmax = 0u;
+    float sum = 0.0f;
+    uint32_t top = 0u;
 #pragma unroll
     for (int i = 0; i < kBfItems; ++i) {
-      const float m = has_tap(i) ? fabsf(mask_of(i)) : 0.0f;
-      msum += m;
-      mmax = max(mmax, __float_as_uint(m));
+      const float m = valid && has_tap(i) ? fabsf(mask_of(i)) : 0.0f;
+      sum += m;
+      top = max(top, __float_as_uint(m));
     }
-    msum += __shfl_xor(msum, 32);
-    mmax = max(mmax, (uint32_t)__shfl_xor((int)mmax, 32));
-    float all = valid ? __uint_as_float(norm) * msum : 0.0f;
-    uint32_t one = __float_as_uint(valid ? __uint_as_float(norm) * __uint_as_float(mmax) : 0.0f);
-    mmax = valid ? mmax : 0u;
 #pragma unroll
-    for (int o = 16; o > 0; o >>= 1) {
-      all += __shfl_xor(all, o);
-      one = max(one, (uint32_t)__shfl_xor((int)one, o));
-      mmax = max(mmax, (uint32_t)__shfl_xor((int)mmax, o));
-    }
-    uint32_t wn = 0u;
-    for (int i = lane; i < a.n_wnorm; i += 64) wn = max(wn, a.wnorm[i]);
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) wn = max(wn, (uint32_t)__shfl_xor((int)wn, o));
+    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
+    top = wave_max(top);
     if (lane == 0) {
-      red[wave * 3] = all;
-      red[wave * 3 + 1] = __uint_as_float(one);
-      red[wave * 3 + 2] = __uint_as_float(mmax);
+      red[wave] = __uint_as_float(top);
+      red[kBfWaves + wave] = sum;
     }
-    // (the counts of adds go where the window will be)
-    for (int i = tid; i < win_px; i += kBfThreads) ((uint32_t *)win)[i] = 0u;
-    __syncthreads();
-    all = 0.0f;
-    one = mmax = 0u;
-#pragma unroll
-    for (int w = 0; w < kBfWaves; ++w) {
-      all += red[w * 3];
-      one = max(one, __float_as_uint(red[w * 3 + 1]));
-      mmax = max(mmax, __float_as_uint(red[w * 3 + 2]));
-    }
-    all *= __uint_as_float(wn);
-    const float top = __uint_as_float(one) * __uint_as_float(wn);
-    const int e = (all > 0.0f && all < 3.0e38f) ? min(29 - ilogbf(all), top > 0.0f ? 20 - ilogbf(top) : 120) : 0;
-    scale = __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint(ldexpf(1.0f, min(120, e)))));
-    inv_scale = 1.0f / scale;
-    fits = __builtin_amdgcn_readfirstlane(all < 3.0e38f && e <= 120 && __uint_as_float(mmax) * scale < 3.0e38f) != 0;  // (false for NaN)
   }
-  // (a window that cannot be used has no rows: every sample is beyond it)
-  const int win_h = fits ? WH : 0;
+  __syncthreads();
   auto window_at = [&](const Place &p, bool &in_win) {
     const int ry = p.y0 - wy0, rx = p.x0 - wx0;
-    in_win = ry >= 0 && ry + 1 < win_h && rx >= 0 && rx + 1 < WW;
+    in_win = ry >= 0 && ry + 1 < WH && rx >= 0 && rx + 1 < WW;
     // a lane with nothing for the window adds its zeros at an entry of its own
     return p.inside && in_win ? ry * WW + rx : lane;
   };
   // How many adds the window pixels that this thread flushes (tid, tid + 512, ...) see in a pass, 16 bits each
   uint32_t adds[(kSlots + 1) / 2];
+  float mask_top, mask_sum;   // bounds on the mask value of a contribution, and on the sum of those of an entry
   {
 #pragma unroll
     for (int i = 0; i < kBfItems; ++i) {
@@ -318,16 +267,34 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
       }
     }
     __syncthreads();
+    uint32_t most = 0u;
 #pragma unroll
     for (int j = 0; j < kSlots; ++j) {
       const int q = tid + kBfThreads * j;
       const uint32_t c = q < win_px ? ((const uint32_t *)win)[q] : 0u;
       adds[j / 2] = j % 2 ? adds[j / 2] | c << 16 : c;
+      most = max(most, c);
     }
+    most = wave_max(most);
+    if (lane == 0) red[2 * kBfWaves + wave] = __uint_as_float(most);
     __syncthreads();
+    uint32_t top = 0u;
+    mask_sum = 0.0f;
+    most = 0u;
+#pragma unroll
+    for (int w = 0; w < kBfWaves; ++w) {
+      top = max(top, __float_as_uint(red[w]));
+      mask_sum += red[kBfWaves + w];
+      most = max(most, __float_as_uint(red[2 * kBfWaves + w]));
+    }
+    mask_top = __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)top));
+    mask_sum = fminf(mask_sum, (float)most * mask_top);   // (NaN only if both are: a mask that is NaN makes both so)
+    mask_sum = __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint(mask_sum)));
     for (int i = tid; i < PLANE * NP / 2; i += kBfThreads) ((uint4 *)win)[i] = make_uint4(0u, 0u, 0u, 0u);
   }
-
+  // The scale of the pass in the window, and whether there is one
+  bool fits = false;
+  float scale = 1.0f, inv_scale = 1.0f;
   // Corners of 8 channels of an item, loaded one unit of work ahead: first channel c0 of the pass, half h of its channels
   struct Corners {
     VecCh<E, 8> r00, r01, r10, r11;
@@ -408,6 +375,35 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
 #pragma unroll
     for (int j = 0; j < 8; ++j) asm volatile("" : "+v"(gf[j].x), "+v"(gf[j].y), "+v"(gf[j].z), "+v"(gf[j].w));
   };
+  // Leaves the largest |d| of this wavefront, as bits (NaN above all), where the others find it behind a barrier.
+  auto put_largest = [&]() {
+    int pos = 0;         // bits as signed numbers: the largest of the positive ones
+    uint32_t neg = 0u;   // as unsigned ones: the largest magnitude of the negative ones, if there are any
+#pragma unroll
+    for (int blk = 0; blk < kBlocks; ++blk) {
+      if (blk < blocks) {   // (the others hold products of nothing)
+#pragma unroll
+        for (int r = 0; r < 16; r += 2) {
+          const int v0 = (int)__float_as_uint(d[blk][r]), v1 = (int)__float_as_uint(d[blk][r + 1]);
+          pos = max(max(v0, v1), pos);
+          neg = max(max((uint32_t)v0, (uint32_t)v1), neg);
+        }
+      }
+    }
+    const uint32_t largest = wave_max(max((uint32_t)pos, neg & 0x7fffffffu));
+    if (lane == 0) red[3 * kBfWaves + wave] = __uint_as_float(largest);
+  };
+  auto take_scale = [&]() {
+    uint32_t bits = 0u;
+#pragma unroll
+    for (int w = 0; w < kBfWaves; ++w) bits = max(bits, __float_as_uint(red[3 * kBfWaves + w]));
+    const float dmax = __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)bits));
+    const float all = dmax * mask_sum, one = dmax * mask_top;   // bounds of a sum and of a contribution
+    const int e = (all > 0.0f && all < 3.0e38f) ? min(29 - ilogbf(all), one > 0.0f ? 20 - ilogbf(one) : 120) : 0;
+    scale = __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint(ldexpf(1.0f, min(120, e)))));
+    inv_scale = 1.0f / scale;
+    fits = __builtin_amdgcn_readfirstlane(all < 3.0e38f && e <= 120 && mask_top * scale < 3.0e38f) != 0;  // (false for NaN)
+  };
   // Adds what the window holds of the CH channels from cf on to grad_input, and clears it.
   auto flush = [&](int cf) {
     float *gplane = a.gin32 + ((long)n * g.Cin + cf) * plane_in;
@@ -447,6 +443,7 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
     for (int j = 0; j < (kSlots + 1) / 2; ++j) asm volatile("" : "+v"(adds[j]));
     asm volatile("" : "+v"(lane), "+v"(frow), "+v"(half), "+v"(tid), "+v"(base_y), "+v"(base_x));
     products_of(c0);
+    put_largest();
     Place p[LA + 1];
 #pragma unroll
     for (int i = 0; i < LA; ++i) p[i] = place(i);
@@ -456,6 +453,7 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
     if (c0 > c_begin) flush(c0 - CH);   // (behind these loads: a wavefront's loads wait for every add in front of them)
     __syncthreads();   // the window is zero and the stages are free
     if (c0 + CH < c_end) issue_first(c0 + CH);
+    take_scale();
     __builtin_amdgcn_sched_barrier(0);
     E *cbase = (E *)a.col + ((((long)nl * (g.Cin / RUN) + c0 / RUN) * g.taps + half) * a.P_pad + pix) * RUN + c0 % RUN;
 #pragma unroll
@@ -473,12 +471,14 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
         const float w00 = hy * hx, w01 = hy * lx, w10 = ly * hx, w11 = ly * lx;
         bool in_win;
         const int wbase = window_at(c, in_win);
+        in_win = in_win && fits;
         const bool to_win = c.inside && in_win;
         const float s00 = (to_win && ok00) ? w00 : 0.0f, s01 = (to_win && ok01) ? w01 : 0.0f;
         const float s10 = (to_win && ok10) ? w10 : 0.0f, s11 = (to_win && ok11) ? w11 : 0.0f;
         const float mts = m * scale;
         const float v00 = m * w00, v01 = m * w01, v10 = m * w10, v11 = m * w11;
         float S00 = 0.0f, S01 = 0.0f, S10 = 0.0f, S11 = 0.0f;
+        // (What a pass without a scale adds to the window is dropped by the flush.)
         if (!fits) {  // (then d may be anything where nothing is sampled; otherwise it is finite and meets zeros there)
 #pragma unroll
           for (int k = 0; k < CH; ++k)
@@ -591,7 +591,7 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
 template <typename E, int CH, int CHF, bool DEEP>
 __global__ __launch_bounds__(kBfThreads, 2) void bwd_fused_kernel(BwdFusedArgs a) {
   __shared__ uint4 lds[kBfLdsBytes / 16];
-  __shared__ float red[(3 + 16) * kBfWaves];
+  __shared__ float red[(4 + 16) * kBfWaves];
   bool far = false;
   if (a.win_far.WH > 0) {
     uint32_t n = (int)(threadIdx.x & 63) < a.n_far ? a.far[threadIdx.x & 63] : 0u;

@@ -36,7 +36,6 @@ struct BwdPlan {
   int sCH;         // channels per pass over that window
   int fR, fWH, fWW;  // window for far offsets (fWH = 0: none), with half as many channels a pass, or 8
   int tw_log;      // fused: log2 of the width of a tile of 256 pixels
-  int n_wnorm;     // bounds on the rows of the weight matrix (fused)
   int n_chunk;     // images per pass
   int cg_tile;     // tile of the column-gradient product (kCgTile or kCgTileBig)
   // Padded channel orders of its copies: segments of the input's channels to whole passes of sCH, a group's to
@@ -52,7 +51,7 @@ struct BwdPlan {
   size_t gpad_bytes;     // grad_output with padded rows, when its own rows cannot be copied 16 bytes at a time
   size_t gb_bytes;  // sums of grad_bias
   int bsplits;      // ... shares of a channel's pixels (matrix-core paths)
-  size_t mx_bytes;  // the counts of far offsets, the bounds on the rows of the weight matrix
+  size_t mx_bytes;  // the counts of far offsets
   // where the matrix-core paths have their copy of the input, and whether its channels are the input's own
   size_t xt_at() const { return gin_bytes + gb_bytes + mx_bytes; }
   bool plain_copy() const { return (gemm || wgemm) && im.segp == im.seg && im.cgp == im.cg; }

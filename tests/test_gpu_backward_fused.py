@@ -64,6 +64,45 @@ def test_fused_backward(name, kw, dtype):
         assert torch.equal(a, b), nm
 
 
+# Output channels whose weights and gradients differ in magnitude: (how many, weight's factor, gradient's factor).  A filter that
+# has died in front of a normalisation layer has weights of zero and a gradient hundreds of times the others'.
+UNEVEN = [
+    ('one_dead_100', 1, 0.0, 100.0),
+    ('one_dead_300', 1, 0.0, 300.0),
+    ('four_dead_300', 4, 0.0, 300.0),
+    ('one_small', 1, 2.0 ** -9, 300.0),
+    ('one_large', 1, 300.0, 2.0 ** -9),
+    ('most_dead', 250, 0.0, 300.0),
+    ('powers', 256, 1.0, 1.0),   # each channel's weights by a power of two, its gradient by the inverse
+]
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16], ids=['bf16', 'f16'])
+@pytest.mark.parametrize('name,count,fw,fg', UNEVEN, ids=[c[0] for c in UNEVEN])
+def test_uneven_channels(name, count, fw, fg, dtype):
+    """The window's quantum goes by the column gradient itself: grad_input stays within its one rounding whatever
+    the parts of grad_output that the weights do not carry into it are."""
+    print(f'case={name} dtype={dtype}', flush=True)
+    case = make_case(73, N=1, Cin=64, Cout=256, H=33, W=40)
+    gy = torch.randn(1, 256, 33, 40, generator=torch.Generator().manual_seed(6))
+    case['weight'][:count] *= fw
+    gy[:, :count] *= fg
+    if name == 'powers':
+        by = 2.0 ** torch.randint(-6, 7, (count, 1, 1, 1), generator=torch.Generator().manual_seed(7))
+        case['weight'] *= by
+        gy /= by.transpose(0, 1)
+    dev, gy = cast_case(case, dtype, 'cuda'), gy.to(dtype).cuda()
+    for modulated in (True, False):
+        call = dict(dev) if modulated else dict(dev, mask=None)
+        ref = capi_backward({k: v.double() if torch.is_tensor(v) else v for k, v in call.items()}, gy.double())
+        got = capi_backward(call, gy, path=capi.PATH_FUSED)
+        for nm, r, o in zip(NAMES, ref, got):
+            if o is not None:
+                err = float((o.double() - r).norm() / r.norm())
+                print(nm, modulated, err, flush=True)
+                assert err <= U[dtype] * SHARE[nm], (nm, modulated, err)
+
+
 def test_passes_of_images():
     """Cut tiles of several passes of images, the last one of another size, have places of their own for their shares."""
     kw = dict(N=5, Cin=64, Cout=64, H=33, W=47)
