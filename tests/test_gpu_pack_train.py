@@ -218,11 +218,48 @@ def test_calls_that_keep_the_module():
     layer(x).sum().backward()
     assert all(p.grad is not None for p in layer.conv_offset.parameters())
     layer, x = fresh()
+    inner = layer.conv_offset._conv_forward
+    layer.conv_offset._conv_forward = lambda *a: (seen.append('inner'), inner(*a))[1]
+    layer(x)
+    assert seen.pop() == 'inner'
+    layer, x = fresh()
     with torch.autocast('cuda', dtype=torch.bfloat16):
         assert layer(x).dtype == torch.bfloat16
     layer, x = fresh()
     with torch.autograd.forward_ad.dual_level(), pytest.raises(NotImplementedError):
         layer(torch.autograd.forward_ad.make_dual(x, torch.ones_like(x)))
+
+
+@pytest.mark.parametrize('modulated', [True, False], ids=['dcnv2', 'dcnv1'])
+def test_function_modes(monkeypatch, modulated):
+    """A function mode sees the operations of a training call; the one that places new tensors does not ask for them."""
+    from mmcv_amd.ops import DeformConv2dPack, ModulatedDeformConv2dPack
+    import mmcv_amd.ops.deform_conv as dc
+    import mmcv_amd.ops.modulated_deform_conv as mdc
+    seen = []
+
+    class Watch(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(getattr(func, '__name__', str(func)))
+            return func(*args, **(kwargs or {}))
+
+    layer, x = _layer(ModulatedDeformConv2dPack if modulated else DeformConv2dPack, SHAPES[0], torch.float32)
+    x.requires_grad_(True)
+    with Watch():
+        layer(x)
+    assert {'conv2d', 'chunk', 'cat', 'sigmoid'} <= set(seen) if modulated else 'conv2d' in seen
+    module, calls = mdc if modulated else dc, []
+    ext = module.ext_module
+
+    class Spy:
+        def __getattr__(self, name):
+            calls.append(name)
+            return getattr(ext, name)
+
+    monkeypatch.setattr(module, 'ext_module', Spy())
+    with torch.device('cuda'):
+        layer(x)
+    assert calls == ['pack_train_call']
 
 
 def test_captured_step():
