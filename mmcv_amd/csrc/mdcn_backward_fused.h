@@ -65,9 +65,10 @@ __device__ __forceinline__ uint32_t wave_max(uint32_t v) {
 // an order that gives a lane consecutive channels of one (pixel, tap) of the result.  grad_output comes in registers, 16
 // bytes a lane and 16 of K, each chunk loaded into the registers of the one before.
 // Scatter: a lane takes its pixel's taps of one parity, 8 channels at a time, their corners loaded two such units ahead.
-// Every wait in it is for loads that are due: whatever the compiler keeps in scratch or fetches from the argument block
-// again there makes it wait for all loads, or all LDS adds, under way (the kernel took 2.1 ms in the shape below with either,
+// Every wait among its items is for loads that are due: whatever the compiler keeps in scratch or fetches from the argument
+// block again there makes it wait for all loads, or all LDS adds, under way (the kernel took 2.1 ms in the shape below with either,
 // 1.35 without).  Hence the asm statements without text below: they hold a sum where it is, and a value in its register.
+// (Not so around the products: the half chunk is a branch, at whose end the compiler waits for grad_output's loads.)
 // Window: 32-bit fixed point in LDS.  Its scale is the pass's own: from the largest |d| of its products over the tile, the largest
 // mask value and the number of adds the busiest entry sees, so that no contribution leaves 2^21 and no sum of them 2^30.  The
 // first decides where no entry sees more than 512, and the quantum is then 2^-20 or 2^-21 of the largest contribution there could
@@ -315,7 +316,7 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
 
   // every copy of a stage has landed, and every wavefront is past whatever it did before
   auto settle = [&]() {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(0) ; lds-copies" ::: "memory");
     __syncthreads();
   };
   f32x16 d[kBlocks];
@@ -551,13 +552,11 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
       }
     }
     load_g(group_of(min(c0 + CH, c_end - 1)), 0);
-    // Every add into the window has landed behind this barrier, and so have the copies of the next pass's weights: since them
-    // a wavefront has issued loads of corners for two items or more (8 each) and some of grad_output, or waits for everything.
-    if (items > 2)
-      asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
-    else
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
+    // Every add into the window has landed behind this barrier, and so have the copies of the next pass's weights.  (What is
+    // waited for beside them are the loads just above, which the products are about to use, and the last stores of columns.  A count
+    // of the loads issued since the copies instead would have nothing to spare: 16 with 8 channels a pass, 5 taps and 64 output
+    // channels; and with 128 or more the compiler waits for these loads anyway.)
+    settle();
   }
   flush(c_end - CH);
   if (part) {
@@ -592,6 +591,7 @@ template <typename E, int CH, int CHF, bool DEEP>
 __global__ __launch_bounds__(kBfThreads, 2) void bwd_fused_kernel(BwdFusedArgs a) {
   __shared__ uint4 lds[kBfLdsBytes / 16];
   __shared__ float red[(4 + 16) * kBfWaves];
+  asm volatile("; mdcn-counted-waits");
   bool far = false;
   if (a.win_far.WH > 0) {
     uint32_t n = (int)(threadIdx.x & 63) < a.n_far ? a.far[threadIdx.x & 63] : 0u;

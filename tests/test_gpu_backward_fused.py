@@ -118,3 +118,33 @@ def test_passes_of_images():
     # the offsets' sums are cut at other channels: fp32 sums in another order, which round to a neighbour now and then
     for nm, a, b in zip(NAMES, whole, parts):
         assert float((a.double() - b.double()).norm() / a.double().norm()) <= 0.1 * U[torch.bfloat16], nm
+
+
+# 5 to 8 taps: as few loads behind the copies of the next pass's weights as there are where items are skipped.
+FEW_TAPS = [
+    ('k1x5', dict(k=(1, 5), padding=(0, 2))),
+    ('k2x3', dict(k=(2, 3), padding=1)),
+    ('k1x7', dict(k=(1, 7), padding=(0, 3))),
+    ('k2x4', dict(k=(2, 4), padding=1)),
+]
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16], ids=['bf16', 'f16'])
+@pytest.mark.parametrize('ch', [16, 8])
+@pytest.mark.parametrize('cout', [64, 128])
+@pytest.mark.parametrize('name,kw', FEW_TAPS, ids=[c[0] for c in FEW_TAPS])
+def test_five_to_eight_taps(name, kw, cout, ch, dtype):
+    """Many passes of few taps, 16 and 8 channels a pass, with columns and without."""
+    print(f'case={name} cout={cout} ch={ch} dtype={dtype}', flush=True)
+    # (segments of 24 channels make passes of 8)
+    shape = dict(N=1, Cin=128 if ch == 16 else 192, Cout=cout, H=21, W=37, deform_groups=1 if ch == 16 else 8)
+    dev = cast_case(make_case(74, **shape, **kw), dtype, 'cuda')
+    gy = torch.randn(1, cout, *dev['offset'].shape[2:], generator=torch.Generator().manual_seed(8)).to(dtype).cuda()
+    ref = capi_backward({k: v.double() if torch.is_tensor(v) else v for k, v in dev.items()}, gy.double())
+    for want in (dict(), dict(want_weight=False)):
+        got = capi_backward(dev, gy, path=capi.PATH_FUSED, **want)
+        for nm, r, o in zip(NAMES, ref, got):
+            if o is None or (nm == 'grad_weight' and not want.get('want_weight', True)):
+                continue
+            err = float((o.double() - r).norm() / r.norm())
+            assert err <= U[dtype] * SHARE[nm], (nm, want, err)

@@ -485,6 +485,26 @@ def test_built_library_passes_the_assembly_scans():
     assert len(asm_check.wait_count_findings(shifted)) >= 1
 
 
+def test_fused_backward_waits_for_its_copies():
+    """The 16-bit backward in one kernel copies weights to LDS directly for the pass after the one it is at.  Its waits for
+    these are part of the third scan, and none of them counts loads behind the copies: how many there are
+    depends on taps and channels."""
+    import os
+    import re
+    import pytest
+    from mmcv_amd import asm_check, build
+    path = os.path.join(build.LIBDIR, 'libmdcn_hip.s')
+    if not os.path.exists(path) or os.path.getmtime(path) + 5 < os.path.getmtime(build.HIP_LIB):
+        pytest.skip('no device assembly beside the built library (mmcv_amd/lib/libmdcn_hip.s)')
+    text = open(path).read()
+    kernels = [k for k in asm_check._kernels(text) if 'bwd_fused_kernel' in k[0]]
+    assert len(kernels) >= 8
+    for name, ins, _ in kernels:
+        assert any(t == 'counted-waits' for _, t, _, _ in ins), name
+        waits = [(t, c) for _, t, c, in_asm in ins if in_asm and t.startswith('s_waitcnt')]
+        assert waits and all(re.fullmatch(r's_waitcnt vmcnt\(0\)', t) and 'lds-copies' in c for t, c in waits), (name, waits)
+
+
 def test_bench_refuses_more_than_one_gpu():
     """bench.py measures one GPU: --gpus above 1 ends with a message and exit status 2 before anything
     touches a device."""
