@@ -81,7 +81,8 @@ __device__ __forceinline__ uint32_t wave_max(uint32_t v) {
 // seen is known from a count made once per tile, and what the patterns hold beside the integers is subtracted when the entry is
 // read.  (Two instructions per channel and corner, where taking it off each contribution was six per two.)  In a pass where d or
 // the mask is not finite, or so small or large that no scale fits, nothing goes through the window.
-// Samples beyond the window are added to memory one at a time, a lane for every channel and corner.
+// Samples beyond the window are added to memory one at a time, a lane for every channel and corner.  (Backward of fp16 N=8 256
+// channels 50x84: 0.42 ms, with one infinity in grad_output -- no window in 1 tile's passes -- 2.1; where every lane added its own samples 7.3.)
 //
 // bf16, N=16, 256 -> 256 channels, 100x152: 1.35 ms for what took 0.52 (column gradient to memory) + 1.50 (scatter kernel reading
 // it); a pass takes a CU 43 thousand clocks: 22 scatter (VALU busy in 17, LDS adds 18), 7 products (MFMA 5), 7 flush, the rest

@@ -258,6 +258,14 @@ constexpr int kScWindowBytes = 60 * 1024;
 constexpr int kScWindowPx = kScWindowBytes / 64;
 // Largest margin of the window for far offsets.
 constexpr int kScFarMargin = 12;
+// Samples beyond the window that a wavefront adds at a time, and the floats each has in LDS: position and channels.
+template <int CH>
+constexpr int kLoneAtOnce = CH >= 16 ? 1 : 16 / CH;
+template <int CH>
+constexpr int kLoneStride = (CH + 4 + 3) / 4 * 4;
+template <int CH>
+constexpr int kLoneFloats = kLoneAtOnce<CH> * kLoneStride<CH>;
+
 // CH consecutive channels (8 to 32 bytes) as floats.
 template <typename E, int CH>
 struct VecCh {
@@ -589,26 +597,34 @@ __device__ __forceinline__ void scatter_tile(const BwdScatterArgs &a, const Scat
           acc_m[tap] += w00 * S00 + w01 * S01 + w10 * S10 + w11 * S11;
           acc_y[tap] += m * (hx * (S10 - S00) + lx * (S11 - S01));
           acc_x[tap] += m * (hy * (S01 - S00) + ly * (S11 - S10));
-          // Samples beyond the window go to memory directly, one at a time: a lane for every channel and corner.
-          for (unsigned long long rest = __ballot(inside && !in_win); rest != 0ull; rest &= rest - 1ull) {
-            const int l = __ffsll((long long)rest) - 1, lane = tid & 63;
-            if (lane == l) {
-              float d[CH];
-              rd.unpack(d);
+          // Samples beyond the window go to memory directly, a lane for every channel and corner of kLoneAtOnce<CH> samples at a
+          // time: what a lane takes part in comes through LDS, position first, then the channels.  Backward in us, every lane its own
+          // sample with 4 CH atomics / one sample at a time / this: bf16 N=2 C=128 60x80 stride 2 (4 channels a pass, margin 3)
+          // sigma 3 116 / 128 / 112, 5 125 / 159 / 122, 10 210 / 214 / 150; bf16 N=2 C=256 50x84 (8 channels, margin 5) sigma 6
+          // 277 / 256 / 248, 20 1 049 / 716 / 659.
+          constexpr int S = kLoneAtOnce<CH>, LS = kLoneStride<CH>;
+          const unsigned long long beyond = __ballot(inside && !in_win);
+          if (beyond != 0ull) {
+            const int lane = tid & 63, total = __popcll(beyond), mine = lane / (4 * CH);
+            const int rank = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(beyond >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)beyond, 0u));
+            const int k = lane % CH, corner = lane / CH % 4;
+            for (int done = 0; done < total; done += S) {
+              if (inside && !in_win && rank >= done && rank < done + S) {
+                float *q = lone + (rank - done) * LS, d[CH];
+                *(float4 *)q = make_float4(__int_as_float(y0), __int_as_float(x0), ly, lx);
+                rd.unpack(d);
 #pragma unroll
-              for (int cc = 0; cc < CH; ++cc) lone[cc] = d[cc] * m;
+                for (int cc = 0; cc < CH; ++cc) q[4 + cc] = d[cc] * m;
+              }
+              __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+              const float4 at = *(const float4 *)(lone + mine * LS);
+              const float t = lone[mine * LS + 4 + k];
+              const int yy = __float_as_int(at.x) + (corner >> 1), xx = __float_as_int(at.y) + (corner & 1);
+              const float w = ((corner & 2) ? at.z : 1.0f - at.z) * ((corner & 1) ? at.w : 1.0f - at.w);
+              if (done + mine < total && k < ps.room && yy >= 0 && yy < g.H && xx >= 0 && xx < g.W)
+                unsafeAtomicAdd(a.gin32 + ((long)n * g.Cin + cs + k) * plane_in + ((long)yy * g.W + xx), w * t);
+              __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             }
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            const int fy = __builtin_amdgcn_readlane(y0, l), fx = __builtin_amdgcn_readlane(x0, l);
-            const float gy = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(ly), l));
-            const float gx = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(lx), l));
-            const int k = lane % CH, corner = lane / CH;
-            const int yy = fy + (corner >> 1), xx = fx + (corner & 1);
-            const float w = ((corner & 2) ? gy : 1.0f - gy) * ((corner & 1) ? gx : 1.0f - gx);
-            const float t = lone[k];
-            if (corner < 4 && k < ps.room && yy >= 0 && yy < g.H && xx >= 0 && xx < g.W)
-              unsafeAtomicAdd(a.gin32 + ((long)n * g.Cin + cs + k) * plane_in + ((long)yy * g.W + xx), w * t);
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
           }
         }
       }
@@ -674,8 +690,9 @@ __device__ __forceinline__ void scatter_tile(const BwdScatterArgs &a, const Scat
 template <typename E, int CH, bool DATA, bool COL>
 __global__ __launch_bounds__(256, 2) void bwd_scatter_kernel(BwdScatterArgs a) {
   __shared__ __align__(16) double win[DATA ? kScWindowBytes / 8 : 4];
-  __shared__ float lone[4 * CH];   // CH of each wavefront
-  float *mine = lone + (threadIdx.x >> 6) * CH;
+  constexpr int kLone = kLoneFloats<CH> > kLoneFloats<CH / 2> ? kLoneFloats<CH> : kLoneFloats<CH / 2>;
+  __shared__ __align__(16) float lone[4 * kLone];   // of each wavefront
+  float *mine = lone + (threadIdx.x >> 6) * kLone;
   if constexpr (DATA && CH * (int)sizeof(E) >= 16) {
     if (a.win_far.WH > 0) {
       uint32_t n = (int)(threadIdx.x & 63) < a.n_far ? a.far[threadIdx.x & 63] : 0u;

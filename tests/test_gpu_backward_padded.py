@@ -131,3 +131,34 @@ def test_stale_workspace(cin, groups):
     assert torch.equal(zeros[3], nans[3]) and bool(nans[3].isfinite().all())
     for a, b in zip(zeros[1:3], nans[1:3]):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize('count', [1, 2, 3, 5, 8, 9, 17, 63, 64])
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16], ids=['f32', 'bf16'])
+@pytest.mark.parametrize('name,kw', [
+    ('8ch', dict(Cin=64)),
+    ('8ch_padded', dict(Cin=20)),
+    ('4ch', dict(Cin=64, stride=2)),
+    ('4ch_padded', dict(Cin=6, deform_groups=1)),
+], ids=['8ch', '8ch_padded', '4ch', '4ch_padded'])
+def test_samples_beyond_the_window(name, kw, dtype, count):
+    """`count` of the 64 pixels of every second wavefront's two rows sample 40 columns away, beyond either window: groups of samples
+    that go to memory together, full and not, and many enough of them that the window for far offsets is used."""
+    print(f'case={name} dtype={dtype} count={count}', flush=True)
+    s = kw.get('stride', 1)
+    case = make_case(55, N=1, Cout=24, H=15 * s + 1, W=95 * s + 1, sigma=0.0, **{k: v for k, v in kw.items()})
+    off = case['offset']
+    off += 0.25
+    px = torch.randperm(64, generator=torch.Generator().manual_seed(count))[:count]
+    for y0 in range(0, off.shape[2] - 1, 4):
+        off[0, 1::2, y0 + px // 32, px % 32] += 40.0
+    gy = torch.randn(1, 24, *off.shape[2:], generator=torch.Generator().manual_seed(7))
+    dev, gyd = cast_case(case, dtype, 'cuda'), gy.to(dtype).cuda()
+    ref = capi_backward({k: v.double() if torch.is_tensor(v) else v for k, v in dev.items()}, gyd.double())
+    got = capi_backward(dev, gyd)
+    # 16 bits: one rounding, of root mean square 0.42 of the unit roundoff; fp32: products of 24 terms and sums of some tens of them,
+    # each rounded, 2^-24 sqrt(100)
+    limit = 10 * 2.0 ** -24 if dtype == torch.float32 else 0.5 * 2.0 ** -8
+    for nm, r, o in zip(NAMES[:3], ref, got):
+        err = float((o.double() - r).norm() / r.norm())
+        assert err <= limit, (nm, err)
