@@ -262,6 +262,26 @@ def test_function_modes(monkeypatch, modulated):
     assert calls == ['pack_train_call']
 
 
+@pytest.mark.parametrize('which', ['weight', 'bias'])
+@pytest.mark.parametrize('modulated', [True, False], ids=['dcnv2', 'dcnv1'])
+def test_parameter_subclasses(modulated, which):
+    """A subclass of Parameter sees the convolution it is a parameter of."""
+    from mmcv_amd.ops import DeformConv2dPack, ModulatedDeformConv2dPack
+    seen = []
+
+    class Watched(nn.Parameter):
+        @classmethod
+        def __torch_function__(cls, func, types, args=(), kwargs=None):
+            seen.append(getattr(func, '__name__', str(func)))
+            with torch._C.DisableTorchFunctionSubclass():
+                return func(*args, **(kwargs or {}))
+
+    layer, x = _layer(ModulatedDeformConv2dPack if modulated else DeformConv2dPack, SHAPES[0], torch.float32)
+    setattr(layer.conv_offset, which, Watched(getattr(layer.conv_offset, which).detach()))
+    layer(x.requires_grad_(True)).sum().backward()
+    assert 'conv2d' in seen
+
+
 def test_captured_step():
     """A training step in a graph, replayed on new input."""
     from mmcv_amd.ops import ModulatedDeformConv2dPack
