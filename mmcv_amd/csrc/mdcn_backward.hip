@@ -124,7 +124,8 @@ void make_bwd_plan(const mdcn_bwd_params *bp, const Geom &g, uint64_t pass_bytes
   om.segp = om.cgp = padded(g.cout_g, KC);
   const int cin_p = g.G * im.cgp;
   const size_t d_img = (size_t)g.taps * cin_p * plane_out * ds;
-  const bool mfma_ok = pl->sR >= 1 && d_img <= kBwdColGradCap && plane_out <= ((size_t)1 << 30) &&
+  // (the limit goes by the columns; an fp32 d beside 16-bit ones has twice their bytes)
+  const bool mfma_ok = pl->sR >= 1 && d_img / ds * es <= kBwdColGradCap && plane_out <= ((size_t)1 << 30) &&
                        (size_t)g.H * g.W <= ((size_t)1 << 30);  // (plane offsets held in 32 bits)
   pl->fused = pl->fused && mfma_ok;
   if (mfma_ok) {

@@ -8,7 +8,7 @@ namespace mdcn {
 
 constexpr size_t kAlign = 256;
 // Column gradient (and columns) held in memory per pass of the backward's matrix-core paths.
-constexpr uint64_t kBwdColGradCap = (uint64_t)3 << 29;  // 1.5 GiB each
+constexpr uint64_t kBwdColGradCap = (uint64_t)3 << 29;  // 1.5 GiB each (of one image: an fp32 d beside 16-bit columns 3)
 inline size_t align_up(size_t v) { return (v + kAlign - 1) / kAlign * kAlign; }
 
 inline size_t elem_size(int dtype) { return dtype == MDCN_F64 ? 8 : dtype == MDCN_F32 ? 4 : 2; }

@@ -162,3 +162,21 @@ def test_samples_beyond_the_window(name, kw, dtype, count):
     for nm, r, o in zip(NAMES[:3], ref, got):
         err = float((o.double() - r).norm() / r.norm())
         assert err <= limit, (nm, err)
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16], ids=['bf16', 'f16'])
+def test_large_plane_of_uneven_channels(dtype):
+    """An image whose fp32 column gradient is larger than its columns may be (1.5 GiB) has the matrix cores all the same."""
+    print(f'large plane dtype={dtype}', flush=True)
+    case = make_case(56, N=1, Cin=96, Cout=16, H=720, W=1280)
+    frac = torch.randint(1, 4, case['offset'].shape, generator=torch.Generator().manual_seed(1)) / 4
+    case['offset'] = torch.floor(case['offset']) + frac   # quarter pixels: exact positions in either type
+    gy = torch.randn(1, 16, 720, 1280, generator=torch.Generator().manual_seed(9))
+    dev, gyd = cast_case(case, dtype, 'cuda'), gy.to(dtype).cuda()
+    got = capi_backward(dev, gyd)
+    ref = capi_backward({k: v.double() if torch.is_tensor(v) else v for k, v in dev.items()}, gyd.double())
+    u = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    # root mean square of one rounding: 0.42 of the unit roundoff; of two -- grad_weight's columns are rounded -- 0.6
+    for nm, r, o, share in zip(NAMES, ref, got, (0.5, 0.5, 0.5, 0.7, 1.0)):
+        err = float((o.double() - r).norm() / r.norm())
+        assert err <= share * u, (nm, err)

@@ -485,6 +485,28 @@ def test_built_library_passes_the_assembly_scans():
     assert len(asm_check.wait_count_findings(shifted)) >= 1
 
 
+def test_backward_workspace_of_large_planes():
+    """Up to 1.5 GiB of columns for an image the backward runs on the matrix cores and asks for their workspace, whether 16-bit
+    channels are whole (column gradient in registers) or not (in memory, in fp32); beyond that it takes the general kernels."""
+    import ctypes
+    from mmcv_amd import capi
+    lib = capi.load()
+
+    def wanted(cin, h, w):
+        bp = capi.MdcnBwdParams()
+        bp.conv = capi.make_params(capi.MDCN_BF16, 1, cin, h, w, cin, 3, 3, (1, 1), (1, 1), (1, 1), 1, 1)
+        for f in ('grad_output', 'grad_input', 'grad_offset', 'grad_mask', 'grad_weight', 'grad_bias'):
+            setattr(bp, f, 256)   # (nothing is read)
+        return lib.mdcn_backward_workspace_bytes(ctypes.byref(bp))
+
+    for cin, h, w in ((64, 720, 1280), (96, 720, 1280), (100, 600, 900), (96, 400, 600)):
+        columns = 9 * cin * h * w * 2
+        assert columns < 3 << 29
+        assert wanted(cin, h, w) > columns * (1 if cin == 64 else 3), (cin, h, w)
+    for cin, h, w in ((128, 720, 1280), (96, 900, 1280)):
+        assert wanted(cin, h, w) < 9 * cin * h * w * 2, (cin, h, w)
+
+
 def test_fused_backward_waits_for_its_copies():
     """The 16-bit backward in one kernel copies weights to LDS directly for the pass after the one it is at.  Its waits for
     these are part of the third scan, and none of them counts loads behind the copies: how many there are
