@@ -299,7 +299,8 @@ int mdcn_backward(const mdcn_bwd_params *p, void *hip_stream);
  * lies around the deformable convolution.
  *
  * mdcn_pack_split(): `offset` and `mask`, dense as mdcn_params describes them, from
- * p->raw: the conv_offset output, dense, the logits taken through the sigmoid and rounded.
+ * p->raw: the conv_offset output, dense, the logits taken through the sigmoid and rounded.  An unmodulated
+ * layer's raw is its offsets and has no logits: MDCN_ERR_PATH.
  *
  * mdcn_pack_trains(): 1 when mdcn_pack_backward() covers the shape in *p, else 0 (no pointer is
  * looked at): channels in whole 128 bytes, the halo of a tile of conv_offset's pixels

@@ -988,6 +988,7 @@ int mdcn_pack_trains(const mdcn_pack_params *pp) {
 
 int mdcn_pack_split(const mdcn_pack_params *pp, void *offset, void *mask, void *hip_stream) {
   if (!pp || !pp->raw || !offset || !mask) return MDCN_ERR_NULL;
+  if (pp->unmodulated) return MDCN_ERR_PATH;  // (all of raw is offsets: there is nothing to split)
   Geom g;
   const int rc = check_params(&pp->conv, &g, false);
   if (rc != MDCN_OK) return rc;

@@ -102,6 +102,20 @@ def test_forward_rejects_bad_calls_before_touching_the_device():
     assert lib.mdcn_forward_timed(ctypes.byref(p), None, None) == -1
 
 
+def test_pack_split_wants_mask_logits():
+    """conv_offset's output of a layer without modulation has no mask logits, so splitting it would read past its end."""
+    lib = capi.load()
+    buf = ctypes.create_string_buffer(64)
+    addr = ctypes.addressof(buf)
+    for dtype in (capi.MDCN_F32, capi.MDCN_F16, capi.MDCN_BF16):
+        pp = capi.MdcnPackParams()
+        pp.conv = capi.make_params(dtype, 1, 32, 8, 8, 4, 3, 3, (1, 1), (1, 1))
+        pp.raw, pp.unmodulated = addr, 1
+        assert lib.mdcn_pack_split(ctypes.byref(pp), addr, addr, None) == -5
+        pp.unmodulated = 0
+        assert lib.mdcn_pack_split(ctypes.byref(pp), addr, None, None) == -1
+
+
 # ---- Python op layer ----------------------------------------------------------
 
 def test_ext_module_exports():
