@@ -67,6 +67,9 @@ void make_bwd_plan(const mdcn_bwd_params *bp, const Geom &g, uint64_t pass_bytes
   // 16-bit tensors whose channels come in whole 128-byte slabs, and 64 or more tiles of them: the data side in one kernel,
   // d in registers and grad_input summed in fixed point.  What is smaller or uneven, and fp32, goes through memory with
   // an fp32 d and sums in doubles.
+  // (The 64 comes from a kernel before this one, which lost to the other path below it.  This one does not: bf16 backward in us, this
+  // kernel / the other path: N=1 64 channels 25x42, 8 tiles, 50 / 60; N=1 512 25x42, 8, 103 / 233; N=2 256 50x84, 42, 147 / 219; N=3 512
+  // 40x60 stride 2, 4 deformable groups, 36, 142 / 180; above it N=4 256 50x84, 84, 234 / 353; N=1 64 100x152, 65, 84 / 100.)
   const bool whole = g.Cin % KC == 0 && g.cout_g % KC == 0 && g.cin_g % 32 == 0 && g.ch_per_dg % 8 == 0;
   pl->fused = staged && bp->grad_input && whole && (s_tiles >= 64 || forced) && (g.kh - 1) * g.dh < 255 && (g.kw - 1) * g.dw < 255 && s_tiles < (1L << 28);
   const bool columns_only = staged && !bp->grad_input;
@@ -329,12 +332,20 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
   const long off_step = std::max<long>(1, (off_total >> 16) | 1);
   const int far_blocks = (int)std::max<long>(1, std::min<long>(off_total / off_step / 1024, 64));
 
-  // Share of offset components beyond the margin from which the far window is the better one.  Half of 16 (doubles: 8)
-  // channels a pass cost next to nothing (bf16, N=2 C=256 135x224, margins 5 and 11: sigma 1.0 0.77 ms with either,
-  // 2.5 0.87 / 0.86, 4.0 1.63 / 0.94), half of 8 do: fp16, N=7 C=128 118x196 stride 2, margins 3 and 12: sigma
-  // 2.0 0.56 / 0.59, 2.5 0.60 / 0.60, 4.0 0.94 / 0.65.  bf16 in doubles, whole training call in us, N=4 96 -> 72 channels
-  // 37x53: sigma 1.0 131 / 132, 2.5 135 / 130, 4.0 154 / 132; N=2 C=128 60x80: 2.0 147 / 153, 3.0 158 / 153, 4.0 195 / 157.
-  const uint32_t far_min = (uint32_t)(off_total / off_step / (pl.fused || pl.sCH == 8 ? 32 : 5));
+  // Share of offset components beyond the margin from which the far window is taken: its passes of fewer channels against
+  // the samples beyond the other one.  Backward in us, near / far window, by the offsets' sigma:
+  // - bwd_fused_kernel, 16 channels a pass or 8.  A pass's products take as long for half the channels, so the line goes by their
+  //   K.  bf16, margins 7 and 12: N=8 256 channels 50x84 3.5 433 / 558, 4.0 462 / 563, 4.5 514 / 565, 5.0 608 / 570; N=2 256 135x224 3.5
+  //   622 / 679, 4.0 702 / 695, 4.5 819 / 714; margins 8 and 12: N=16 512 25x42 4.0 554 / 730, 6.0 600 / 731.  (Shares: 0.045 for 3.5
+  //   and a margin of 7, 0.080 for 4.0, 0.119 for 4.5.)  N=8 64 96x160 3.0 278 / 288, 3.5 302 / 296, 4.0 336 / 306; N=8 128 60x60 3.5
+  //   172 / 176, 4.0 184 / 179.
+  // - ... 8 or 8, over another window: fp16 N=7 128 118x196 stride 2, margins 8 and 12: 3.0 351 / 353, 4.0 379 / 368, 6.0 480 / 425.
+  // - Doubles, 8 or 4, margins 5 and 11: fp32 N=2 256 50x84 2.0 321 / 331, 3.0 328 / 332, 4.0 351 / 338, 6.0 539 / 366; bf16 N=2 128 60x80 3.0
+  //   121 / 124, 4.0 131 / 126, 6.0 240 / 138; N=4 96 -> 72 37x53 2.0 116 / 105, 4.0 118 / 103.
+  // - ... 4 or 2, margins 3 and 12: fp32 N=4 128 60x80 stride 2 2.0 131 / 164, 4.0 147 / 173, 6.0 178 / 181.  (The line is from when every
+  //   sample beyond the window cost more.)
+  const int far_share = pl.fused && pl.sCH == 16 && g.cout_g > kBfK ? 11 : pl.fused || pl.sCH == 8 ? 32 : 5;
+  const uint32_t far_min = (uint32_t)(off_total / off_step / far_share);
   auto up = [](long n, long per) { return (int)((n + per - 1) / per); };
   {
     BwdPreArgs a;

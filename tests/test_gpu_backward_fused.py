@@ -28,6 +28,9 @@ CASES = [
     ('far', dict(N=1, Cin=64, Cout=64, H=40, W=45, sigma=6.0)),
     ('far_s2', dict(N=1, Cin=128, Cout=64, H=60, W=75, stride=2, sigma=9.0)),
     ('past_far', dict(N=1, Cin=64, Cout=64, H=50, W=55, sigma=20.0)),
+    # (more than 128 output channels: up to a share of 1/11 beyond the margin of 7 or 8 the first window is used)
+    ('k256_first_window', dict(N=1, Cin=64, Cout=256, H=40, W=45, sigma=4.0)),
+    ('k256_far', dict(N=1, Cin=64, Cout=256, H=40, W=45, sigma=5.5)),
     ('rounds', dict(N=2, Cin=64, Cout=64, H=190, W=194, sigma=1.5)),   # 36 or 37 tiles per XCD: a round, and cut ones
 ]
 NAMES = ('grad_input', 'grad_offset', 'grad_mask', 'grad_weight', 'grad_bias')
