@@ -302,9 +302,10 @@ int mdcn_backward(const mdcn_bwd_params *p, void *hip_stream);
  * p->raw: the conv_offset output, dense, the logits taken through the sigmoid and rounded.  An unmodulated
  * layer's raw is its offsets and has no logits: MDCN_ERR_PATH.
  *
- * mdcn_pack_trains(): 1 when mdcn_pack_backward() covers the shape in *p, else 0 (no pointer is
- * looked at): channels in whole 128 bytes, the halo of a tile of conv_offset's pixels
- * fits LDS.
+ * mdcn_pack_trains(): 1 when a layer should leave conv_offset's backward to mdcn_pack_backward(), else 0 (no
+ * pointer is looked at).  Covered are channels in whole 128 bytes where the halo of a tile of conv_offset's
+ * pixels fits LDS; of these, calls that a plain convolution's backward is faster for -- mostly fp32 with more than 32
+ * channels of conv_offset, kernels of many taps -- answer 0, and mdcn_pack_backward() takes them all the same.
  */
 int mdcn_pack_split(const mdcn_pack_params *p, void *offset, void *mask, void *hip_stream);
 int mdcn_pack_trains(const mdcn_pack_params *p);

@@ -983,7 +983,8 @@ int mdcn_pack_trains(const mdcn_pack_params *pp) {
   Geom g;
   if (!pp || check_params(&pp->conv, &g, false) != MDCN_OK || pp->conv.input_nhwc) return 0;
   OconvBwdPlan ol;
-  return oconv_bwd_plan(g, pp->conv.dtype, pp->unmodulated != 0, true, true, false, num_cus(), &ol) ? 1 : 0;
+  return oconv_bwd_plan(g, pp->conv.dtype, pp->unmodulated != 0, true, true, false, num_cus(), &ol) &&
+         oconv_bwd_pays(g, pp->conv.dtype, pp->unmodulated != 0);
 }
 
 int mdcn_pack_split(const mdcn_pack_params *pp, void *offset, void *mask, void *hip_stream) {

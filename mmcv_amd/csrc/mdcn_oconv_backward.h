@@ -35,6 +35,10 @@ struct OconvBwdPlan {
 bool oconv_bwd_plan(const Geom &g, int dtype, bool unmodulated, bool data, bool weight, bool own_copy, int cus,
                     OconvBwdPlan *pl);
 
+// Whether a training call of the layers is not slower for it than with torch's convolution backward (for shapes that
+// oconv_bwd_plan covers).
+bool oconv_bwd_pays(const Geom &g, int dtype, bool unmodulated);
+
 struct OconvBwdArgs {
   Geom g;
   int CO, cob, Wp;

@@ -607,6 +607,26 @@ bool oconv_bwd_plan(const Geom &g, int dtype, bool unmodulated, bool data, bool 
   return true;
 }
 
+// Training calls in us, torch's convolution backward and the operations around it / this one.  What it saves is launches and passes
+// over memory, some 50 us of device time and more on the host; what it costs is that both kernels go over padded blocks of 32
+// channels of conv_offset, and tap by tap, one after another.
+// fp32, whose products are six of bf16 each, at a stride and dilation of 1 (elsewhere torch's own take long) and beyond one block,
+// by the work of tiles of 4 x 32 pixels.  Calls with mask: N=4 256 channels 50x84, 2 deformable groups (92 M) 951 / 953, 4 groups (184 M)
+// 1 101 / 1 131; N=8 256 25x42, 4 (132 M) 751 / 800; N=8 128 25x42, 4 (66 M) 408 / 406.  Of a long chain of taps and blocks, or without mask:
+// N=1 64 30x40, 8 groups (8.2 M) 255 / 241, N=1 256 13x21, 8 (8.3 M) 276 / 314, N=2 64 30x40, 8 (16 M) 238 / 255; 5x5 taps 374 / 416 (9.8 M), 7x7 586 / 741;
+// without mask N=1 128 25x42, 4 (6.1 M) 240 / 209, N=2 256 13x21, 4 (7.1 M) 257 / 269, N=8 256 25x42, 2 (66 M) 612 / 640.
+// (One block: without mask, N=8 256 25x42, 586 / 595 at worst, with it 611 / 603; N=2 256 50x84 566 / 559 and 595 / 565.)
+// 16 bits: only chains as long as those of 7x7 taps where workgroups are few, N=1 64 30x40 (32) 627 / 650 and 606 / 624 without mask; N=4
+// (128) 1 902 / 1 800.
+bool oconv_bwd_pays(const Geom &g, int dtype, bool unmodulated) {
+  const int cob = ((unmodulated ? 2 : 3) * g.DG * g.taps + 31) / 32, chain = cob * g.taps;
+  if (dtype != MDCN_F32)
+    return chain <= 150 || (long)g.N * ((g.H + 3) / 4) * ((g.W + 31) / 32) * (g.Cin / 32) >= 100;
+  if (cob == 1 || g.sh != 1 || g.sw != 1 || g.dh != 1 || g.dw != 1) return true;
+  const double work = (double)g.N * ((g.Ho + 3) / 4 * 4) * ((g.Wo + 31) / 32 * 32) * g.Cin * chain;
+  return work <= (!unmodulated && chain <= 40 ? 100e6 : 6.2e6);
+}
+
 hipError_t oconv_backward(int dtype, const OconvBwdPlan &pl, OconvBwdArgs a, unsigned char *ws, hipStream_t st) {
   auto take = [&](size_t bytes) {
     unsigned char *q = ws;

@@ -116,6 +116,29 @@ def test_pack_split_wants_mask_logits():
         assert lib.mdcn_pack_split(ctypes.byref(pp), addr, None, None) == -1
 
 
+def test_pack_trains_where_it_pays():
+    """Calls that are faster with torch's convolution backward are left to it: fp32 with several blocks of conv_offset's
+    channels and much work, or many taps; 16 bits with many taps and few workgroups."""
+    lib = capi.load()
+
+    def trains(dtype, n, c, h, w, k=3, dg=1, stride=1, unmodulated=0):
+        pp = capi.MdcnPackParams()
+        pp.conv = capi.make_params(dtype, n, c, h, w, c, k, k, (stride,) * 2, (k // 2,) * 2, (1, 1), 1, dg)
+        pp.unmodulated = unmodulated
+        return lib.mdcn_pack_trains(ctypes.byref(pp))
+
+    f32, bf16 = capi.MDCN_F32, capi.MDCN_BF16
+    # slower inside the library: 1 216 -> 1 337 us, 638 -> 697, 369 -> 388, 586 -> 741, 362 -> 508, 998 -> 1 074, 376 -> 417, 627 -> 650
+    for call in ((f32, 16, 256, 25, 42, 3, 4), (f32, 8, 256, 25, 42, 3, 4, 1, 1), (f32, 1, 64, 100, 152, 3, 8), (f32, 1, 64, 30, 40, 7),
+                 (f32, 1, 64, 15, 20, 7), (f32, 16, 256, 25, 42, 3, 2, 1, 1), (f32, 8, 128, 25, 42, 3, 8, 1, 1), (bf16, 1, 64, 30, 40, 7)):
+        assert trains(*call) == 0, call
+    # as fast or faster: one block of channels whatever the size, small calls, strides, 16 bits
+    for call in ((f32, 2, 256, 50, 84), (f32, 8, 512, 25, 42, 3, 1, 1, 1), (f32, 16, 256, 100, 152), (f32, 1, 128, 25, 42, 3, 4, 1, 1), (f32, 4, 128, 50, 84, 3, 2),
+                 (f32, 1, 64, 15, 20, 3, 8), (f32, 2, 128, 50, 84, 3, 4, 2), (f32, 8, 128, 64, 96, 3, 2, 2, 1), (bf16, 16, 256, 25, 42, 3, 4), (bf16, 8, 128, 25, 42, 3, 16),
+                 (bf16, 1, 64, 30, 40, 5), (bf16, 4, 64, 30, 40, 7)):
+        assert trains(*call) == 1, call
+
+
 # ---- Python op layer ----------------------------------------------------------
 
 def test_ext_module_exports():
