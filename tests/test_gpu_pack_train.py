@@ -262,6 +262,30 @@ def test_function_modes(monkeypatch, modulated):
     assert calls == ['pack_train_call']
 
 
+@pytest.mark.parametrize('dtype,channels', [(torch.float32, 48), (torch.bfloat16, 96), (torch.float64, 64)], ids=['f32', 'bf16', 'f64'])
+@pytest.mark.parametrize('modulated', [True, False], ids=['dcnv2', 'dcnv1'])
+def test_uneven_channels_do_not_ask(monkeypatch, modulated, dtype, channels):
+    """Channels that conv_offset's backward in the library does not cover go to the sequence of operations without a call into it.
+    (Double precision is asked for and refused.)"""
+    from mmcv_amd.ops import DeformConv2dPack, ModulatedDeformConv2dPack
+    import mmcv_amd.ops.deform_conv as dc
+    import mmcv_amd.ops.modulated_deform_conv as mdc
+    module, calls = mdc if modulated else dc, []
+    ext = module.ext_module
+
+    class Spy:
+        def __getattr__(self, name):
+            calls.append(name)
+            return getattr(ext, name)
+
+    shape = (1, channels, 32, 9, 17, 3, 1, 1, 1, 1)
+    layer, x = _layer(ModulatedDeformConv2dPack if modulated else DeformConv2dPack, shape, dtype)
+    monkeypatch.setattr(module, 'ext_module', Spy())
+    y, _, grads = _step(layer, x)
+    assert ('pack_train_call' in calls) == (dtype == torch.float64)
+    assert y.shape == (1, 32, 9, 17) and all(bool(g.isfinite().all()) for g in grads)
+
+
 @pytest.mark.parametrize('which', ['weight', 'bias'])
 @pytest.mark.parametrize('modulated', [True, False], ids=['dcnv2', 'dcnv1'])
 def test_parameter_subclasses(modulated, which):
