@@ -84,7 +84,7 @@ __device__ __forceinline__ uint32_t wave_max(uint32_t v) {
 // Samples beyond the window are added to memory one at a time, a lane for every channel and corner.  (Backward of fp16 N=8 256
 // channels 50x84: 0.42 ms, with one infinity in grad_output -- no window in 1 tile's passes -- 2.1; where every lane added its own samples 7.3.)
 //
-// bf16, N=16, 256 -> 256 channels, 100x152: 1.35 ms for what took 0.52 (column gradient to memory) + 1.50 (scatter kernel reading
+// bf16, N=16, 256 -> 256 channels, 100x152: 1.36 ms (1.35 with the scale from norms) for what took 0.52 (column gradient to memory) + 1.50 (scatter kernel reading
 // it); a pass takes a CU 43 thousand clocks: 22 scatter (VALU busy in 17, LDS adds 18), 7 products (MFMA 5), 7 flush, the rest
 // waits at the three barriers.
 template <typename E, int CH, int RUN, bool DEEP>

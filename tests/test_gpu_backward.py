@@ -243,7 +243,7 @@ def test_full_size_all_five_gradients_against_oracle():
 
 def test_fixed_point_window_with_wide_dynamic_range():
     """16-bit tensors sum grad_input in a 32-bit fixed-point window scaled by the largest column
-    gradient of the call.  With grad_output spanning six decades, the gradient as a whole stays
+    gradient of a tile and pass.  With grad_output spanning six decades, the gradient as a whole stays
     within tolerance of the oracle (error against the largest element), and the region whose
     contributions are a million times smaller than the largest carries an absolute error of at most
     a few window quanta, i.e. far below the 16-bit rounding of the large elements -- but not a
