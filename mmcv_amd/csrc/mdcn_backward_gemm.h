@@ -728,6 +728,15 @@ struct WGradArgs {
   long total;        // workgroups with work: G x co_tiles x m_tiles x splits
 };
 
+// Where an element of run `run` of a block of 16 columns lies among the 64 x RUN of that run: at its index with these bits
+// toggled.  A transposing read takes four pixels of all of a block's runs at once, whole multiples of 512 bytes apart: on the
+// same banks, unless each run has its fours of pixels in another order.  (Weight gradient in us, in order / so: bf16 N=12 64 channels
+// 16x25 stride 2, runs of 4, 14.0 / 11.7; N=4 96 -> 72 37x53, runs of 8, 14.6 / 14.1.)
+template <int RUN>
+__device__ __forceinline__ int tr_swizzle(int run) {
+  return run * (4 * RUN);
+}
+
 // A wave's products of one K step with the second operand pixel major: B holds, for every 16 columns, 16 / run runs of 64 pixels x
 // run columns.  An LDS read that transposes gives a lane four consecutive pixels of one column: 16 lanes
 // read 8 bytes each, four pixels of every four columns.
@@ -740,11 +749,11 @@ __device__ __forceinline__ void tile_products_tr(f32x16 (&acc)[TILE / 64][2], co
   constexpr int MB = TILE / 64;
   const int frow = lane & 31, fhalf = lane >> 5;
   const uint4 *a0 = A + (wm * (TILE / 2) + frow) * 8;
-  // the four columns and the pixel whose 8 bytes this lane reads
+  // the four columns and the pixel whose 8 bytes this lane reads; four pixels of a run lie where tr_swizzle has put them
   constexpr int per = RUN / 4, pitch = RUN * 2;
-  const int quad = lane & 3;
-  const unsigned char *b0 = (const unsigned char *)B + (wn * 4 + ((lane >> 4) & 1)) * 2048 + quad / per * (64 * pitch) +
-                            (fhalf * 8 + ((lane & 15) >> 2)) * pitch + quad % per * 8;
+  const int quad = lane & 3, run = quad / per, px = fhalf * 8 + ((lane & 15) >> 2), sw = 2 * tr_swizzle<RUN>(run);
+  const unsigned char *b0 = (const unsigned char *)B + (wn * 4 + ((lane >> 4) & 1)) * 2048 + run * (64 * pitch) + quad % per * 8;
+  const unsigned char *b_lo = b0 + ((px * pitch) ^ sw), *b_hi = b0 + (((px + 4) * pitch) ^ sw);
 #pragma unroll
   for (int ksub = 0; ksub < 4; ++ksub) {
     uint4 af[MB], bf[2];
@@ -752,9 +761,9 @@ __device__ __forceinline__ void tile_products_tr(f32x16 (&acc)[TILE / 64][2], co
     for (int mb = 0; mb < MB; ++mb) af[mb] = a0[mb * 256 + ((ksub * 2 + fhalf) ^ (frow & 7))];
 #pragma unroll
     for (int nb = 0; nb < 2; ++nb) {
-      const unsigned char *b = b0 + nb * 4096 + ksub * 16 * pitch;
-      const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4_t)(lptr_t)(void *)b);
-      const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4_t)(lptr_t)(void *)(b + 4 * pitch));
+      const int at = nb * 4096 + ksub * 16 * pitch;
+      const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4_t)(lptr_t)(void *)(b_lo + at));
+      const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4_t)(lptr_t)(void *)(b_hi + at));
       const uint2 l2 = __builtin_bit_cast(uint2, lo), h2 = __builtin_bit_cast(uint2, hi);
       bf[nb] = make_uint4(l2.x, l2.y, h2.x, h2.y);
     }
@@ -818,8 +827,8 @@ __global__ __launch_bounds__(TILE * 2, TILE == 128 ? 2 : 1) void bwd_wgrad_kerne
       const int m = min(mt * TILE + (blk >> 1) * 16, a.M - 16);
       const int tap = m / a.cgp;
       const int at = (blk & 1) * 512 + lane * 8;   // element of the 64 pixels x 16 columns
-      const int sub = at / (64 * RUN), px = (at - sub * 64 * RUN) / RUN;
-      b_row[c] = (((long)((grp * a.cgp + m - tap * a.cgp) / RUN + sub) * a.taps + tap) * a.P_pad + px) * RUN + at % RUN;
+      const int sub = at / (64 * RUN), in = (at - sub * 64 * RUN) ^ tr_swizzle<RUN>(sub);   // (whole fours of pixels trade places)
+      b_row[c] = ((long)((grp * a.cgp + m - tap * a.cgp) / RUN + sub) * a.taps + tap) * a.P_pad * RUN + in;
     } else {
       // (the rows of the channels that only fill up a group are never written: they would hold what was there before, NaN
       // for instance, and the call then goes over its K range a second time)
