@@ -27,6 +27,30 @@ int window_margin(const Geom &g, int th, int tw, long max_px, int *WH, int *WW, 
   return R;
 }
 
+// Workgroups that share a tile's passes over the window in bwd_scatter_kernel.  Two fit a CU but take nearly twice as long
+// there -- LDS adds and VALU are busy with either --, so what counts is the longest share times the workgroups that a CU gets; a share
+// costs some 0.4 of a pass beside its passes (offsets and mask, first loads, its sums for bwd_finish_kernel to add).  A power of two up to
+// eight, until the launch fills the chip eight times over, is where it starts from and what calls of many tiles stay with: there any number is within 2 %.
+// Whole training calls in us, parts as powers of two / as this has them: bf16 N=4 96 -> 72 channels 37x53, 2 deformable groups (80
+// tiles, 6 passes each) 4 129 / 6 110 (3: 115); fp32 N=2 256 50x84 (42, 32) 8 438 / 12 407 (6: 436, 16: 423, 32: 411); N=1 256 50x84 (21, 32)
+// 8 266 / 12 249; N=1 512 25x42 (8, 64) 8 390 / 32 294 (12: 354, 16: 321, 64: 308); N=2 128 60x80 stride 2 (16, 32) 8 159 / 16 138; N=4 512
+// 25x42 (32, 64) 8 667 / 16 646; bf16 N=2 200 -> 160 40x60 (20, 25) 8 168 / 25 134.
+int scatter_parts(long tiles, int passes) {
+  constexpr int kCus = 256, kMost = 32;
+  auto cost = [&](int parts) {
+    const long wgs = tiles * parts, longest = (passes + parts - 1) / parts;
+    if (wgs <= kCus) return (double)longest + 0.4;
+    if (wgs <= 2 * kCus) return 1.7 * ((double)longest + 0.4);
+    return 0.85 * (double)wgs / kCus * ((double)passes / parts + 0.4) + 0.3 * (double)longest;
+  };
+  int best = 1;
+  while (best < 8 && tiles * best < 4096 && 2 * best <= passes) best *= 2;
+  double least = 0.9 * cost(best);   // (what changes for less than a tenth may as well be noise)
+  for (int parts = best + 1; parts <= kMost && parts <= passes && tiles * parts <= 4 * kCus; ++parts)
+    if (cost(parts) <= least) least = cost(best = parts);
+  return best;
+}
+
 }  // namespace
 
 void make_bwd_plan(const mdcn_bwd_params *bp, const Geom &g, uint64_t pass_bytes, BwdPlan *pl) {
@@ -139,14 +163,13 @@ void make_bwd_plan(const mdcn_bwd_params *bp, const Geom &g, uint64_t pass_bytes
     pl->n_chunk = (int)std::min<uint64_t>((uint64_t)g.N, std::max<uint64_t>(1, pass_bytes / d_img));
     pl->xt_bytes = align_up((size_t)g.N * cin_p * g.Hp * g.Wp * es);
     pl->gw_bytes = 0;
-    // Workgroups per tile: enough for eight rounds or so of the chip's 2 x CUs slots
     const int passes = g.ch_per_dg / seg * (im.segp / pl->sCH);
     if (pl->fused) {
       pl->sched.passes = passes;
       pl->sched.tiles = pl->n_chunk * g.DG * ((g.Ho + (256 >> pl->tw_log) - 1) / (256 >> pl->tw_log)) *
                         ((g.Wo + (1 << pl->tw_log) - 1) >> pl->tw_log);
     } else {
-      while (pl->parts < 8 && s_tiles * pl->parts < 4096 && 2 * pl->parts <= passes) pl->parts *= 2;
+      pl->parts = scatter_parts(s_tiles, passes);
     }
     pl->bsplits = 1;
     if (bp->grad_bias) {

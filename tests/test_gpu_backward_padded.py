@@ -59,6 +59,21 @@ def test_padded_backward(name, kw, dtype):
         assert rel_err(o.float().cpu().numpy(), r) <= TOL[dtype], nm
 
 
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16], ids=['f32', 'bf16'])
+@pytest.mark.parametrize('cin,dg,h', [(24, 1, 9), (40, 1, 9), (96, 2, 9), (200, 1, 17), (504, 1, 5), (520, 1, 9)])
+def test_shares_of_passes(cin, dg, h, dtype):
+    """A tile's 3, 5, 6, 25, 63 and 65 passes over the window among as many workgroups, or 32 of them: every pass is somebody's."""
+    print(f'cin={cin} dg={dg} h={h} dtype={dtype}', flush=True)
+    case = cast_case(make_case(55, N=1, Cin=cin, Cout=36, H=h, W=37, deform_groups=dg), dtype)
+    gy = torch.randn(1, 36, h, 37, generator=torch.Generator().manual_seed(7)).to(dtype)
+    geo = dict(stride=1, padding=1, dilation=1, groups=1, deform_groups=dg)
+    ref = oracle.backward(*[case[k].float().numpy() for k in ('input', 'offset', 'mask', 'weight')],
+                          gy.float().numpy(), True, **geo)
+    for nm, r, o in zip(NAMES, ref, capi_backward(cast_case(case, dtype, 'cuda'), gy.cuda())):
+        err = rel_err(o.float().cpu().numpy(), r)
+        assert err <= TOL[dtype], (nm, err)
+
+
 def test_padding_channels_have_no_gradient():
     """An infinity of grad_output leaves NaN in the column gradient of the padding channels (zero weights times
     infinity): what follows a segment's planes in grad_input -- here the other image's -- has none of it."""
