@@ -69,10 +69,12 @@ __device__ __forceinline__ uint32_t wave_max(uint32_t v) {
 // block again there makes it wait for all loads, or all LDS adds, under way (the kernel took 2.1 ms in the shape below with either,
 // 1.35 without).  Hence the asm statements without text below: they hold a sum where it is, and a value in its register.
 // (Not so around the products: the half chunk is a branch, at whose end the compiler waits for grad_output's loads.)
-// Window: 32-bit fixed point in LDS.  Its scale is the pass's own: from the largest |d| of its products over the tile, the largest
-// mask value and the number of adds the busiest entry sees, so that no contribution leaves 2^21 and no sum of them 2^30.  The
+// Window: 32-bit fixed point in LDS.  Its scale is the pass's own: from the largest |d * mask| of a sample of the tile and
+// the number of adds the busiest entry sees, so that no contribution leaves 2^21 and no sum of them 2^30.  The
 // first decides where no entry sees more than 512, and the quantum is then 2^-20 or 2^-21 of the largest contribution there could
-// be.  (Bounds of |d| from norms of grad_output and weights instead: training calls of N=16 256 channels 100x152 in bf16 2 319
+// be.  (The largest |d| times the largest mask, wherever each of them is, is five instructions a tap less and no faster, and loses bits to a
+// large gradient under a small mask: fp16, one pixel of a mask of 0 and 1 000 times the gradient: error of grad_input 3.3e-3 of its
+// norm where this has 2.1e-4, its one rounding.)  (Bounds of |d| from norms of grad_output and weights instead: training calls of N=16 256 channels 100x152 in bf16 2 319
 // us where this takes 2 329, of N=8 512 channels 25x42 in fp16 371 / 363.  But such a scale goes by gradients that the weights do not
 // carry on: fp16, 256 output channels, one of them without weights and with 300 times the gradient: error of grad_input
 // 8.6e-4 of its norm, where its one rounding is 2.1e-4 and this stays at that.)
@@ -144,11 +146,11 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
       t_m[i] = (uint32_t)__builtin_bit_cast(uint16_t, msk[(long)tc * a.om.msk_ch]) | (half ? at1 : at0) << 16;
     }
   }
-  float *lone = red + 4 * kBfWaves + wave * 16;   // of this wavefront
+  float *lone = red + 3 * kBfWaves + wave * 16;   // of this wavefront
   const int items = (g.taps + 1) / 2, blocks = (items + PER - 1) / PER;
 
-  // (1: unmodulated)
-  auto mask_of = [&](int i) { return a.om.logit == kMaskNone ? 1.0f : to_f32(__builtin_bit_cast(E, (uint16_t)t_m[i])); };
+  // (zero where nothing is sampled, once the tile has begun)
+  auto mask_of = [&](int i) { return to_f32(__builtin_bit_cast(E, (uint16_t)t_m[i])); };
   auto has_tap = [&](int i) { return ((t_m[i] >> 16) & 255u) != 255u; };
   int base_y = ho * g.sh - g.ph, base_x = wo * g.sw - g.pw;
   struct Place {
@@ -228,23 +230,18 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
   load_g(group_of(c_begin), 0);
   // (the counts of adds go where the window will be)
   for (int i = tid; i < win_px; i += kBfThreads) ((uint32_t *)win)[i] = 0u;
-  // Largest mask value, and the sum of all of the tile's
+  // A mask of zero where nothing is sampled, and the tile's largest
   {
-    float sum = 0.0f;
     uint32_t top = 0u;
 #pragma unroll
     for (int i = 0; i < kBfItems; ++i) {
-      const float m = valid && has_tap(i) ? fabsf(mask_of(i)) : 0.0f;
-      sum += m;
-      top = max(top, __float_as_uint(m));
+      const uint32_t one = (uint32_t)__builtin_bit_cast(uint16_t, from_f32<E>(1.0f));
+      const uint32_t m = a.om.logit == kMaskNone ? one : t_m[i] & 0xffffu;   // (1: unmodulated)
+      t_m[i] = (t_m[i] & 0xffff0000u) | (place(i).inside ? m : 0u);
+      top = max(top, __float_as_uint(fabsf(mask_of(i))));
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
     top = wave_max(top);
-    if (lane == 0) {
-      red[wave] = __uint_as_float(top);
-      red[kBfWaves + wave] = sum;
-    }
+    if (lane == 0) red[wave] = __uint_as_float(top);
   }
   __syncthreads();
   auto window_at = [&](const Place &p, bool &in_win) {
@@ -255,7 +252,7 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
   };
   // How many adds the window pixels that this thread flushes (tid, tid + 512, ...) see in a pass, 16 bits each
   uint32_t adds[(kSlots + 1) / 2];
-  float mask_top, mask_sum;   // bounds on the mask value of a contribution, and on the sum of those of an entry
+  float mask_top, adds_top;   // the largest mask value, and the largest number of adds
   {
 #pragma unroll
     for (int i = 0; i < kBfItems; ++i) {
@@ -278,20 +275,17 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
       most = max(most, c);
     }
     most = wave_max(most);
-    if (lane == 0) red[2 * kBfWaves + wave] = __uint_as_float(most);
+    if (lane == 0) red[kBfWaves + wave] = __uint_as_float(most);
     __syncthreads();
     uint32_t top = 0u;
-    mask_sum = 0.0f;
     most = 0u;
 #pragma unroll
     for (int w = 0; w < kBfWaves; ++w) {
       top = max(top, __float_as_uint(red[w]));
-      mask_sum += red[kBfWaves + w];
-      most = max(most, __float_as_uint(red[2 * kBfWaves + w]));
+      most = max(most, __float_as_uint(red[kBfWaves + w]));
     }
     mask_top = __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)top));
-    mask_sum = fminf(mask_sum, (float)most * mask_top);   // (NaN only if both are: a mask that is NaN makes both so)
-    mask_sum = __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint(mask_sum)));
+    adds_top = __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint((float)most)));
     for (int i = tid; i < PLANE * NP / 2; i += kBfThreads) ((uint4 *)win)[i] = make_uint4(0u, 0u, 0u, 0u);
   }
   // The scale of the pass in the window, and whether there is one
@@ -377,31 +371,35 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
 #pragma unroll
     for (int j = 0; j < 8; ++j) asm volatile("" : "+v"(gf[j].x), "+v"(gf[j].y), "+v"(gf[j].z), "+v"(gf[j].w));
   };
-  // Leaves the largest |d| of this wavefront, as bits (NaN above all), where the others find it behind a barrier.
+  // Leaves the largest |d * mask| of this wavefront, as bits (NaN above all), where the others find it behind a barrier.
   auto put_largest = [&]() {
-    int pos = 0;         // bits as signed numbers: the largest of the positive ones
-    uint32_t neg = 0u;   // as unsigned ones: the largest magnitude of the negative ones, if there are any
+    uint32_t largest = 0u;
 #pragma unroll
-    for (int blk = 0; blk < kBlocks; ++blk) {
-      if (blk < blocks) {   // (the others hold products of nothing)
+    for (int i = 0; i < kBfItems; ++i) {
+      if (i < items) {
+        int pos = 0;         // bits as signed numbers: the largest of the positive ones
+        uint32_t neg = 0u;   // as unsigned ones: the largest magnitude of the negative ones, if there are any
 #pragma unroll
-        for (int r = 0; r < 16; r += 2) {
-          const int v0 = (int)__float_as_uint(d[blk][r]), v1 = (int)__float_as_uint(d[blk][r + 1]);
+        for (int k = 0; k < CH; k += 2) {
+          const int v0 = (int)__float_as_uint(d[i / PER][(i % PER) * CH + k]), v1 = (int)__float_as_uint(d[i / PER][(i % PER) * CH + k + 1]);
           pos = max(max(v0, v1), pos);
           neg = max(max((uint32_t)v0, (uint32_t)v1), neg);
         }
+        // (what is not finite makes this NaN where the mask is zero)
+        const float c = __uint_as_float(max((uint32_t)pos, neg & 0x7fffffffu)) * mask_of(i);
+        largest = max(largest, __float_as_uint(c) & 0x7fffffffu);
       }
     }
-    const uint32_t largest = wave_max(max((uint32_t)pos, neg & 0x7fffffffu));
-    if (lane == 0) red[3 * kBfWaves + wave] = __uint_as_float(largest);
+    largest = wave_max(largest);
+    if (lane == 0) red[2 * kBfWaves + wave] = __uint_as_float(largest);
   };
   auto take_scale = [&]() {
     uint32_t bits = 0u;
 #pragma unroll
-    for (int w = 0; w < kBfWaves; ++w) bits = max(bits, __float_as_uint(red[3 * kBfWaves + w]));
-    const float dmax = __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)bits));
-    const float all = dmax * mask_sum, one = dmax * mask_top;   // bounds of a sum and of a contribution
-    const int e = (all > 0.0f && all < 3.0e38f) ? min(29 - ilogbf(all), one > 0.0f ? 20 - ilogbf(one) : 120) : 0;
+    for (int w = 0; w < kBfWaves; ++w) bits = max(bits, __float_as_uint(red[2 * kBfWaves + w]));
+    const float one = __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)bits));
+    const float all = one * adds_top;   // bounds of a contribution and of a sum
+    const int e = (all > 0.0f && all < 3.0e38f) ? min(29 - ilogbf(all), 20 - ilogbf(one)) : 0;
     scale = __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint(ldexpf(1.0f, min(120, e)))));
     inv_scale = 1.0f / scale;
     fits = __builtin_amdgcn_readfirstlane(all < 3.0e38f && e <= 120 && mask_top * scale < 3.0e38f) != 0;  // (false for NaN)
@@ -465,8 +463,7 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
         const Place c = p[i % (LA + 1)];
         if (i + LA < kBfItems) next = place(i + LA);
         const float ly = c.ly, lx = c.lx, hy = 1.0f - ly, hx = 1.0f - lx;
-        const float mk = mask_of(i);
-        const float m = c.inside ? mk : 0.0f;
+        const float m = mask_of(i);
         const int y0 = c.y0, x0 = c.x0, y1 = y0 + 1, x1 = x0 + 1;
         const bool ok00 = y0 >= 0 && x0 >= 0, ok01 = y0 >= 0 && x1 <= g.W - 1;
         const bool ok10 = y1 <= g.H - 1 && x0 >= 0, ok11 = y1 <= g.H - 1 && x1 <= g.W - 1;
@@ -591,7 +588,7 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
 template <typename E, int CH, int CHF, bool DEEP>
 __global__ __launch_bounds__(kBfThreads, 2) void bwd_fused_kernel(BwdFusedArgs a) {
   __shared__ uint4 lds[kBfLdsBytes / 16];
-  __shared__ float red[(4 + 16) * kBfWaves];
+  __shared__ float red[(3 + 16) * kBfWaves];
   asm volatile("; mdcn-counted-waits");
   bool far = false;
   if (a.win_far.WH > 0) {

@@ -106,6 +106,31 @@ def test_uneven_channels(name, count, fw, fg, dtype):
                 assert err <= U[dtype] * SHARE[nm], (nm, modulated, err)
 
 
+# Pixels whose gradients are large where their mask is next to nothing: (how many, gradient's factor, mask there).
+CLOSED = [('one_1e3_zero', 1, 1e3, 0.0), ('one_8e3_2^-10', 1, 8e3, 2.0 ** -10), ('row_300_zero', 40, 300.0, 0.0),
+          ('one_1e2_negative', 1, 1e2, -2.0 ** -9)]
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16], ids=['bf16', 'f16'])
+@pytest.mark.parametrize('name,count,fg,mask', CLOSED, ids=[c[0] for c in CLOSED])
+def test_closed_gates(name, count, fg, mask, dtype):
+    """The window's quantum goes by what is added to it, the column gradient times the mask of the same sample: a large gradient
+    under a small mask, or where nothing is sampled, takes no bits from the tile's other pixels."""
+    print(f'case={name} dtype={dtype}', flush=True)
+    case = make_case(75, N=1, Cin=64, Cout=128, H=33, W=40)
+    gy = torch.randn(1, 128, 33, 40, generator=torch.Generator().manual_seed(9))
+    gy[:, :, 20, :count] *= fg
+    case['mask'][:, :, 20, :count] = mask
+    gy[:, :, 9, 7] *= fg   # (all of its samples beyond the image)
+    case['offset'][:, :, 9, 7] = 1e4
+    dev, gy = cast_case(case, dtype, 'cuda'), gy.to(dtype).cuda()
+    ref = capi_backward({k: v.double() if torch.is_tensor(v) else v for k, v in dev.items()}, gy.double())[0]
+    got = capi_backward(dev, gy, path=capi.PATH_FUSED)[0].double()
+    err = float((got - ref).norm() / ref.norm())
+    print(err, flush=True)
+    assert err <= U[dtype] * SHARE['grad_input'], err
+
+
 def test_passes_of_images():
     """Cut tiles of several passes of images, the last one of another size, have places of their own for their shares."""
     kw = dict(N=5, Cin=64, Cout=64, H=33, W=47)
