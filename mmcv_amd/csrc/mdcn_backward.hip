@@ -93,7 +93,8 @@ void make_bwd_plan(const mdcn_bwd_params *bp, const Geom &g, uint64_t pass_bytes
   // (bf16 backward in us, this kernel / the other path: N=1 64 channels 25x42, 8 tiles, 50 / 60; N=1 512 25x42, 8, 103 / 233; N=2 256 50x84, 42,
   // 147 / 219; N=3 512 40x60 stride 2, 4 deformable groups, 36, 142 / 180; N=4 256 50x84, 84, 234 / 353; N=1 64 100x152, 65, 84 / 100.)
   const bool whole = g.Cin % KC == 0 && g.cout_g % KC == 0 && g.cin_g % 32 == 0 && g.ch_per_dg % 8 == 0;
-  pl->fused = staged && bp->grad_input && whole && (g.kh - 1) * g.dh < 255 && (g.kw - 1) * g.dw < 255 && s_tiles < (1L << 28);
+  pl->fused = staged && bp->grad_input && whole && (g.kh - 1) * g.dh < 255 && (g.kw - 1) * g.dw < 255 && s_tiles < (1L << 28) &&
+              (long)g.Ho * g.Wo < kBfPlaneMax && (long)g.Hp * g.Wp < kBfPlaneMax;
   const bool columns_only = staged && !bp->grad_input;
   const size_t ds = pl->fused || columns_only ? es : 4;  // bytes of an element of d, or of the columns
   int u = g.cin_g, v = g.ch_per_dg;
@@ -391,6 +392,7 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
     a.run = pl.sCH;
     a.col_rows = (long)pl.n_chunk * g.taps * cin_p;
     a.M_pad = pl.M_pad;
+    a.wt_run = pl.fused ? kBfK : 0;
     a.off = p->offset;
     a.n_off = off_total;
     a.off_step = off_step;

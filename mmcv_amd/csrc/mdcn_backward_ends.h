@@ -28,6 +28,7 @@ struct BwdPreArgs {
   long col_rows;           // rows of col whose padding is cleared
   int run;                 // WGradArgs::run
   int M_pad;
+  int wt_run;              // wT in runs of this many output channels (see there), or 0
   const void *off;
   long n_off, off_step;    // one offset in off_step is looked at
   float far_from;          // ... and counted when it is larger than this
@@ -132,7 +133,9 @@ __global__ __launch_bounds__(256) void bwd_prepass_kernel(BwdPreArgs a) {
   }
   if (b < a.end[kPreWeight]) {
     // weight[Cout][cin_g][taps] -> wT[G][M_pad][om.cgp], row m = tap * im.cgp + padded channel, zero where
-    // either channel is padding and in the rows up to M_pad
+    // either channel is padding and in the rows up to M_pad.  With wt_run it is [G][run][M_pad][wt_run], the last run what is left: what
+    // bwd_fused_kernel copies at a time is one piece of memory for a tap (256 bytes of rows 1 KB apart, as with
+    // 512 output channels, are in one of four channels of the L2).
     const long total = (long)g.G * a.M_pad * a.om.cgp;
     const long idx = (long)(b - a.end[kPreColPad]) * 256 + tid;
     if (idx >= total) return;
@@ -147,7 +150,12 @@ __global__ __launch_bounds__(256) void bwd_prepass_kernel(BwdPreArgs a) {
     E v = from_f32<E>(0.0f);
     if (tap < g.taps && room > 0 && co < g.cout_g)
       v = ((const E *)a.w)[((long)(grp * g.cout_g + co) * g.cin_g + c) * g.taps + tap];
-    ((E *)a.wT)[idx] = v;
+    long at = idx;
+    if (a.wt_run) {
+      const int run = co / a.wt_run, len = min(a.wt_run, a.om.cgp - run * a.wt_run);
+      at = (long)grp * a.M_pad * a.om.cgp + (long)run * a.wt_run * a.M_pad + (long)m * len + (co - run * a.wt_run);
+    }
+    ((E *)a.wT)[at] = v;
     return;
   }
   {  // offsets that leave the scatter kernel's window, counted in a sample

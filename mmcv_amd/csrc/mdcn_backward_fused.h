@@ -21,6 +21,7 @@ constexpr int bf_blocks(int ch) { return (kBfItems * ch + 15) / 16; }
 constexpr int bf_stage_bytes(int ch) { return bf_blocks(ch) * 32 * kBfK * 2; }
 constexpr int kBfLdsBytes = 163072;
 constexpr int bf_window_px(int ch) { return (kBfLdsBytes - 2 * bf_stage_bytes(ch)) / (4 * ch); }
+constexpr long kBfPlaneMax = 1L << 24;              // pixels of a plane, its zero border included
 constexpr float kRoundMagic = 12582912.0f;          // 1.5 * 2^23: adding it leaves an integer in the mantissa
 constexpr uint32_t kRoundBits = 0x4B400000u;        // ... on top of these bits
 
@@ -28,7 +29,7 @@ struct BwdFusedArgs {
   Geom g;
   const void *xt;   // zero-bordered input copy in 32-byte records [N][Cin / 16][H + 2][W + 2][16]
   const void *gT;   // grad_output, pixel major [N][Cout / 64][P][64]
-  const void *wT;   // [G][taps * cin_g][cout_g], row tap * cin_g + channel
+  const void *wT;   // [G][chunk of kBfK output channels][taps * cin_g][of the chunk], row tap * cin_g + channel
   OffMaskView om;   // (dense tensors: logit is kMaskPlain or kMaskNone)
   float *gin32;
   void *goff;
@@ -63,16 +64,18 @@ __device__ __forceinline__ uint32_t wave_max(uint32_t v) {
 // Products: blocks of 32 rows of weights -- two taps of 16 channels, or four of 8 -- times the wavefront's 32 pixels, K in chunks
 // of 128.  The weights of a pass go to LDS for all wavefronts (two chunks; copied during the scatter of the pass before), rows in
 // an order that gives a lane consecutive channels of one (pixel, tap) of the result.  grad_output comes in registers, 16
-// bytes a lane and 16 of K, each chunk loaded into the registers of the one before.
+// bytes a lane and 16 of K, each half chunk loaded into the registers of the one before it, a pass's first during the last tap of the
+// scatter before it.  These loads take 2 to 5 thousand clocks (a round's tiles have more grad_output than an L2 holds), so no
+// branch and no wait for something else lies between them and their products.  More than 256 output channels: a chunk's copies are
+// on their way during the products of the one before.
 // Scatter: a lane takes its pixel's taps of one parity, 8 channels at a time, their corners loaded two such units ahead.
 // Every wait among its items is for loads that are due: whatever the compiler keeps in scratch or fetches from the argument
 // block again there makes it wait for all loads, or all LDS adds, under way (the kernel took 2.1 ms in the shape below with either,
 // 1.35 without).  Hence the asm statements without text below: they hold a sum where it is, and a value in its register.
-// (Not so around the products: the half chunk is a branch, at whose end the compiler waits for grad_output's loads.)
 // Window: 32-bit fixed point in LDS.  Its scale is the pass's own: from the largest |d * mask| of a sample of the tile and
 // the number of adds the busiest entry sees, so that no contribution leaves 2^21 and no sum of them 2^30.  The
 // first decides where no entry sees more than 512, and the quantum is then 2^-20 or 2^-21 of the largest contribution there could
-// be.  (The largest |d| times the largest mask, wherever each of them is, is five instructions a tap less and no faster, and loses bits to a
+// be.  (The largest |d| times the largest mask, wherever each of them is, is an instruction a tap less, and loses bits to a
 // large gradient under a small mask: fp16, one pixel of a mask of 0 and 1 000 times the gradient: error of grad_input 3.3e-3 of its
 // norm where this has 2.1e-4, its one rounding.)  (Bounds of |d| from norms of grad_output and weights instead: training calls of N=16 256 channels 100x152 in bf16 2 319
 // us where this takes 2 329, of N=8 512 channels 25x42 in fp16 371 / 363.  But such a scale goes by gradients that the weights do not
@@ -86,9 +89,11 @@ __device__ __forceinline__ uint32_t wave_max(uint32_t v) {
 // Samples beyond the window are added to memory one at a time, a lane for every channel and corner.  (Backward of fp16 N=8 256
 // channels 50x84: 0.42 ms, with one infinity in grad_output -- no window in 1 tile's passes -- 2.1; where every lane added its own samples 7.3.)
 //
-// bf16, N=16, 256 -> 256 channels, 100x152: 1.36 ms (1.35 with the scale from norms) for what took 0.52 (column gradient to memory) + 1.50 (scatter kernel reading
-// it); a pass takes a CU 43 thousand clocks: 22 scatter (VALU busy in 17, LDS adds 18), 7 products (MFMA 5), 7 flush, the rest
-// waits at the three barriers.
+// bf16, N=16, 256 -> 256 channels, 100x152: 1.29 ms for what took 0.52 (column gradient to memory) + 1.50 (scatter kernel reading
+// it); a pass takes a CU 40 thousand clocks: 25 scatter (VALU busy in 16, LDS adds 18), 6 products (MFMA 5), 7 flush, the rest
+// waits at the barriers.  fp16 without modulation, N=8, 512 -> 512 channels, 25x42: 0.17 ms.  (Whole training calls, us: 2 224 and
+// 348; 2 361 and 372 with grad_output loaded within branches and behind the scatter, the argument block kept as it was loaded,
+// 64-bit addresses in each lane and the largest of a pass found with integers, two instructions a value.)
 template <typename E, int CH, int RUN, bool DEEP>
 __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterWindow &wd, int b, int c_first, int c_last, float *part, uint4 *lds,
                                            float *red) {
@@ -103,9 +108,22 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
   constexpr int kSlots = (PLANE + kBfThreads - 1) / kBfThreads;
   uint4 *wst = lds;
   unsigned long long *win = (unsigned long long *)(lds + 2 * kStage / 16);
-  const Geom &g = a.g;
+  // What a pass reads of the argument block, a scalar each: as parts of its sixteen-register loads they would be put away and fetched
+  // back sixteen at a time (366 of the scatter's 2 679 VALU instructions).
+  Geom g = a.g;
+  auto apart = [](const void *p) {
+    auto q = (const __attribute__((address_space(1))) unsigned char *)p;   // (or nothing would say that it is global memory)
+    asm volatile("" : "+s"(q));
+    return (const unsigned char *)q;
+  };
+  const unsigned char *wt = apart(a.wT), *gt = apart(a.gT), *xt = apart(a.xt);
+  unsigned char *cols = (unsigned char *)apart(a.col);
+  float *gin = (float *)apart(a.gin32);
+  uint32_t col_px = (uint32_t)a.P_pad;
+  asm volatile("" : "+s"(g.H), "+s"(g.W), "+s"(g.Wp), "+s"(g.Cin), "+s"(g.cin_g), "+s"(g.cout_g), "+s"(g.taps), "+s"(g.G), "+s"(col_px));
   const long plane_out = (long)g.Ho * g.Wo, plane_in = (long)g.H * g.W, slab_px = (long)g.Hp * g.Wp;
   int tid = threadIdx.x, lane = tid & 63, frow = lane & 31, half = lane >> 5;
+  asm volatile("" : "+v"(lane), "+v"(frow), "+v"(half), "+v"(tid));   // (or addresses of all copies are kept over the tiles, in scratch)
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int tx = b % a.tiles_x;
   b /= a.tiles_x;
@@ -116,7 +134,9 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
   const int TW = 1 << a.tw_log, TH = 256 >> a.tw_log;
   const int ho = ty * TH + ((wave * 32 + frow) >> a.tw_log), wo = tx * TW + (frow & (TW - 1));
   const bool valid = ho < g.Ho && wo < g.Wo;
-  const long pix = (long)min(ho, g.Ho - 1) * g.Wo + min(wo, g.Wo - 1);   // (lanes past the image: any pixel of it)
+  // (lanes past the image: any pixel of it.  Addresses are a scalar base and a lane's 32 bits wherever a pass needs them: planes have
+  // fewer than kBfPlaneMax pixels.)
+  const uint32_t pix = (uint32_t)(min(ho, g.Ho - 1) * g.Wo + min(wo, g.Wo - 1));
   const int wy0 = ty * TH * g.sh - g.ph - wd.R, wx0 = tx * TW * g.sw - g.pw - wd.R;
   int WW = wd.WW, WH = wd.WH;
   asm volatile("" : "+s"(WW), "+s"(WH));   // (kept: fetched again for every use, each wait for one would be for all LDS adds)
@@ -125,27 +145,6 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
 
   // This lane's taps 2 i + half: offsets, mask and place in the kernel
   uint32_t t_off[kBfItems], t_m[kBfItems];   // dy | dx << 16; mask | row << 16 | column << 24, a row of 255: no such tap
-  {
-    const E *off = (const E *)a.om.off + (long)n * a.om.off_n + pix * a.om.off_px + (long)(dgi * 2 * g.taps) * a.om.off_ch;
-    const E *msk = (const E *)a.om.msk + (long)n * a.om.msk_n + pix * a.om.msk_px + (long)(dgi * g.taps) * a.om.msk_ch;
-    int row = 0, col = 0;
-    auto tap_at = [&](int tap) {   // (one after the other)
-      const uint32_t at = tap < g.taps ? (uint32_t)(row * g.dh) | (uint32_t)(col * g.dw) << 8 : 255u;
-      if (++col == g.kw) {
-        col = 0;
-        ++row;
-      }
-      return at;
-    };
-#pragma unroll
-    for (int i = 0; i < kBfItems; ++i) {
-      const int tap = 2 * i + half, tc = min(tap, g.taps - 1);
-      const uint32_t at0 = tap_at(2 * i), at1 = tap_at(2 * i + 1);
-      t_off[i] = (uint32_t)__builtin_bit_cast(uint16_t, off[(long)(2 * tc) * a.om.off_ch]) |
-                 (uint32_t)__builtin_bit_cast(uint16_t, off[(long)(2 * tc + 1) * a.om.off_ch]) << 16;
-      t_m[i] = (uint32_t)__builtin_bit_cast(uint16_t, msk[(long)tc * a.om.msk_ch]) | (half ? at1 : at0) << 16;
-    }
-  }
   float *lone = red + 3 * kBfWaves + wave * 16;   // of this wavefront
   const int items = (g.taps + 1) / 2, blocks = (items + PER - 1) / PER;
 
@@ -182,41 +181,38 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
   // kh % 2.
   const int nkh = (g.cout_g + kBfK - 1) / kBfK;
   const uint32_t lds_w = (uint32_t)(uintptr_t)(lptr_t)wst + (uint32_t)wave * 1024u;
+  const uint32_t rows_g = (uint32_t)(g.taps * g.cin_g);
   auto issue = [&](int c0, int kh) {
     const int sh = g.cout_g - kh * kBfK >= kBfK ? 4 : 3;
     const int grp = group_of(c0);
-    const unsigned char *base = (const unsigned char *)a.wT +
-                                (((long)grp * g.taps * g.cin_g + (c0 - grp * g.cin_g)) * g.cout_g + kh * kBfK) * 2;
+    const uint32_t row_bytes = 16u << sh;
+    const unsigned char *base = wt + ((long)grp * g.cout_g + kh * kBfK) * rows_g * 2 + (long)(c0 - grp * g.cin_g) * row_bytes;
     const int copies = blocks << (sh - 1);   // of 1 KiB
+    // Copies are 32 or 64 rows apart, so all of a lane's are the same row of their blocks: result register 4 * r8 + r4 of the lanes of half hh
+    const uint32_t row0 = (uint32_t)(wave * 64 + lane) >> sh, s = (uint32_t)lane & ((1u << sh) - 1u);
+    const uint32_t r8 = (row0 >> 3) & 3u, hh = (row0 >> 2) & 1u, r4 = row0 & 3u;
+    const uint32_t ch = 4 * (PER == 2 ? r8 & 1 : r8) + r4, at = ch * row_bytes + ((s ^ (row0 & 7u)) * 16u);
+    const uint32_t tap0 = PER * 2 * (row0 >> 5) + (PER == 2 ? 2 * (r8 >> 1) : 0) + hh, tap_bytes = (uint32_t)g.cin_g * row_bytes;
     const uint32_t lds = (uint32_t)__builtin_amdgcn_readfirstlane((int)(lds_w + (uint32_t)(kh & 1) * (uint32_t)kStage));
 #pragma unroll
     for (int c = 0; c < 8 * kBlocks / kBfWaves; ++c) {
       if (wave + kBfWaves * c < copies) {
-        const uint32_t u = (uint32_t)((wave + kBfWaves * c) * 64 + lane);
-        const uint32_t row = u >> sh, s = u - (row << sh);
-        const int blk = (int)(row >> 5), r8 = (int)(row >> 3) & 3, hh = (int)(row >> 2) & 1, r4 = (int)row & 3;
-        // result register 4 * r8 + r4 of the lanes of half hh
-        const int tap = min(PER * 2 * blk + (PER == 2 ? 2 * (r8 >> 1) : 0) + hh, g.taps - 1);
-        const int ch = 4 * (PER == 2 ? r8 & 1 : r8) + r4;
-        copy16_global_to_lds(base + (uint32_t)((tap * g.cin_g + ch) * g.cout_g) * 2u + ((s ^ (row & 7u)) * 16u),
-                             lds + (uint32_t)c * (kBfWaves * 1024u));
+        const uint32_t tap = min(tap0 + (uint32_t)(PER * 2 * c) * (sh == 4 ? 1u : 2u), (uint32_t)g.taps - 1u);
+        copy16_global_to_lds(base + (tap * tap_bytes + at), lds + (uint32_t)c * (kBfWaves * 1024u));
       }
     }
   };
   // This lane's grad_output of chunk kh of K, the products' second operand: j-th 16 of it (j < 4, or < 8 where the chunk is whole)
-  const unsigned char *gpx = (const unsigned char *)a.gT + ((long)n * (g.Cout / 64) * plane_out + pix) * 128 + half * 16;
+  const unsigned char *gbase = gt + (long)n * (g.Cout / 64) * plane_out * 128;
   auto whole_chunk = [&](int kh) { return g.cout_g - kh * kBfK >= kBfK; };
-  auto g_at = [&](int grp, int kh, int j) {
-    return *(const uint4 *)(gpx + ((long)(grp * (g.cout_g / 64) + kh * 2 + j / 4) * plane_out) * 128 + j % 4 * 32);
-  };
   uint4 gf[8];
-  auto load_g = [&](int grp, int kh) {
+  // (the second half of a half chunk is the first once more: read, and not used)
+  auto load_g_half = [&](int grp, int kh, int s) {
+    const unsigned char *p = gbase + ((long)(grp * (g.cout_g / 64) + kh * 2 + (whole_chunk(kh) ? s : 0)) * plane_out) * 128;
+    uint32_t at = pix * 128u + (uint32_t)half * 16u;
+    asm volatile("" : "+v"(at));
 #pragma unroll
-    for (int j = 0; j < 4; ++j) gf[j] = g_at(grp, kh, j);
-    if (whole_chunk(kh)) {
-#pragma unroll
-      for (int j = 4; j < 8; ++j) gf[j] = g_at(grp, kh, j);
-    }
+    for (int j = 0; j < 4; ++j) gf[4 * s + j] = *(const uint4 *)(p + j * 32 + at);
   };
   // the first two stages of a pass
   auto issue_first = [&](int c0) {
@@ -224,10 +220,32 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
     if (nkh > 1) issue(c0, 1);
   };
   issue_first(c_begin);
+  {
+    const E *off = (const E *)a.om.off + (long)n * a.om.off_n + (long)pix * a.om.off_px + (long)(dgi * 2 * g.taps) * a.om.off_ch;
+    const E *msk = (const E *)a.om.msk + (long)n * a.om.msk_n + (long)pix * a.om.msk_px + (long)(dgi * g.taps) * a.om.msk_ch;
+    int row = 0, col = 0;
+    auto tap_at = [&](int tap) {   // (one after the other)
+      const uint32_t at = tap < g.taps ? (uint32_t)(row * g.dh) | (uint32_t)(col * g.dw) << 8 : 255u;
+      if (++col == g.kw) {
+        col = 0;
+        ++row;
+      }
+      return at;
+    };
+#pragma unroll
+    for (int i = 0; i < kBfItems; ++i) {
+      const int tap = 2 * i + half, tc = min(tap, g.taps - 1);
+      const uint32_t at0 = tap_at(2 * i), at1 = tap_at(2 * i + 1);
+      t_off[i] = (uint32_t)__builtin_bit_cast(uint16_t, off[(long)(2 * tc) * a.om.off_ch]) |
+                 (uint32_t)__builtin_bit_cast(uint16_t, off[(long)(2 * tc + 1) * a.om.off_ch]) << 16;
+      t_m[i] = (uint32_t)__builtin_bit_cast(uint16_t, msk[(long)tc * a.om.msk_ch]) | (half ? at1 : at0) << 16;
+    }
+  }
 
   // (The barrier ends the tile before: nobody is at the window any more.)
   __syncthreads();
-  load_g(group_of(c_begin), 0);
+  load_g_half(group_of(c_begin), 0, 0);
+  load_g_half(group_of(c_begin), 0, 1);
   // (the counts of adds go where the window will be)
   for (int i = tid; i < win_px; i += kBfThreads) ((uint32_t *)win)[i] = 0u;
   // A mask of zero where nothing is sampled, and the tile's largest
@@ -238,6 +256,7 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
       const uint32_t one = (uint32_t)__builtin_bit_cast(uint16_t, from_f32<E>(1.0f));
       const uint32_t m = a.om.logit == kMaskNone ? one : t_m[i] & 0xffffu;   // (1: unmodulated)
       t_m[i] = (t_m[i] & 0xffff0000u) | (place(i).inside ? m : 0u);
+      asm volatile("" : "+v"(t_off[i]), "+v"(t_m[i]));   // (here and now, or the halves they are made of are kept)
       top = max(top, __float_as_uint(fabsf(mask_of(i))));
     }
     top = wave_max(top);
@@ -297,12 +316,13 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
   };
   auto fetch = [&](int c0, const Place &p, int h, Corners &s) {
     // corners outside the image read the copy's zero border
-    const E *xp = (const E *)a.xt + (((long)n * (g.Cin / 16) + c0 / 16) * slab_px) * 16 + (c0 % 16) + h * 8 +
-                  ((long)(p.y0 + 1) * g.Wp + (p.x0 + 1)) * 16;
-    s.r00.load(xp);
-    s.r01.load(xp + 16);
-    s.r10.load(xp + (long)g.Wp * 16);
-    s.r11.load(xp + (long)(g.Wp + 1) * 16);
+    const unsigned char *xp = xt + (((long)n * (g.Cin / 16) + c0 / 16) * slab_px) * 32 + (c0 % 16) * 2 + h * 16;
+    uint32_t top = (uint32_t)((p.y0 + 1) * g.Wp + (p.x0 + 1)) * 32u, bot = top + (uint32_t)g.Wp * 32u;
+    asm volatile("" : "+v"(top), "+v"(bot));   // (these beside a scalar base, and no sums of the two)
+    s.r00.load((const E *)(xp + top));
+    s.r01.load((const E *)(xp + 32 + top));
+    s.r10.load((const E *)(xp + bot));
+    s.r11.load((const E *)(xp + 32 + bot));
   };
 
   float acc_m[kBfItems], acc_y[kBfItems], acc_x[kBfItems];
@@ -315,37 +335,26 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
     __syncthreads();
   };
   f32x16 d[kBlocks];
-  // Products of chunk kh of K; the next chunk's grad_output is loaded into the registers of what has been used.
-  auto products = [&](int grp, int kh) {
-    const bool more = kh + 1 < nkh;
-    const int pitch = whole_chunk(kh) ? 16 : 8;
+  // Products of half s of chunk kh of K.
+  auto products_half = [&](int kh, int s, int pitch) {
     const uint4 *w0 = wst + (kh & 1) * (kStage / 16) + frow * pitch;
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      if (s == 0 || whole_chunk(kh)) {
+    for (int j = 0; j < 4; ++j) {
+      const uint4 *wj = w0 + 8 * s + ((2 * j + half) ^ (frow & 7));
+      uint4 f[kBlocks];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const uint4 *wj = w0 + 8 * s + ((2 * j + half) ^ (frow & 7));
-          uint4 f[kBlocks];
+      for (int blk = 0; blk < kBlocks; ++blk) f[blk] = wj[blk * 32 * pitch];
 #pragma unroll
-          for (int blk = 0; blk < kBlocks; ++blk) f[blk] = wj[blk * 32 * pitch];
-#pragma unroll
-          for (int blk = 0; blk < kBlocks; ++blk) TR::mma(d[blk], f[blk], gf[4 * s + j]);
-        }
-        // fragments are read three products ahead of theirs
-        __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
-#pragma unroll
-        for (int j = 0; j < 4 * kBlocks - 3; ++j) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        }
-        __builtin_amdgcn_sched_group_barrier(0x008, 3, 0);
-        if (more && (s == 0 || whole_chunk(kh + 1))) {
-#pragma unroll
-          for (int j = 0; j < 4; ++j) gf[4 * s + j] = g_at(grp, kh + 1, 4 * s + j);
-        }
-      }
+      for (int blk = 0; blk < kBlocks; ++blk) TR::mma(d[blk], f[blk], gf[4 * s + j]);
     }
+    // fragments are read three products ahead of theirs
+    __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
+#pragma unroll
+    for (int j = 0; j < 4 * kBlocks - 3; ++j) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, 3, 0);
   };
   // All of a pass's products; the first two stages are in LDS.
   auto products_of = [&](int c0) {
@@ -354,17 +363,32 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
     for (int blk = 0; blk < kBlocks; ++blk)
 #pragma unroll
       for (int r = 0; r < 16; ++r) d[blk][r] = 0.0f;
-    products(grp, 0);
-    if (nkh > 1) products(grp, 1);
+    // A chunk's grad_output goes into the registers of what has been used.  (No branch between a load and its product: the
+    // waits are for the half chunk that is due, with the next one under way.)
+    auto chunk_and_load = [&](int kh, auto between) {
+      products_half(kh, 0, 16);
+      load_g_half(grp, kh + 1, 0);
+      products_half(kh, 1, 16);
+      between();
+      load_g_half(grp, kh + 1, 1);
+    };
+    auto last_chunk = [&](int kh) {
+      products_half(kh, 0, whole_chunk(kh) ? 16 : 8);
+      if (whole_chunk(kh)) products_half(kh, 1, 16);
+    };
     if constexpr (DEEP) {
-      for (int kh = 2; kh < nkh; kh += 2) {
-        __syncthreads();   // nobody reads the stages any more
-        issue(c0, kh);
-        if (kh + 1 < nkh) issue(c0, kh + 1);
-        settle();
-        products(grp, kh);
-        if (kh + 1 < nkh) products(grp, kh + 1);
+      chunk_and_load(0, [] { __syncthreads(); });   // (nobody reads the first stage any more)
+      issue(c0, 2);
+      for (int kh = 1; kh + 1 < nkh; ++kh) {
+        chunk_and_load(kh, settle);   // (every wavefront is past this stage, and the next one has landed)
+        if (kh + 2 < nkh) issue(c0, kh + 2);
       }
+      last_chunk(nkh - 1);
+    } else if (nkh > 1) {
+      chunk_and_load(0, [] {});
+      last_chunk(1);
+    } else {
+      last_chunk(0);
     }
     // (No load is under way here.  The compiler, which follows each branch above by itself, is told so, or it waits for
     // whatever is under way at the next use of these registers.)
@@ -373,25 +397,18 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
   };
   // Leaves the largest |d * mask| of this wavefront, as bits (NaN above all), where the others find it behind a barrier.
   auto put_largest = [&]() {
-    uint32_t largest = 0u;
+    float largest = 0.0f;
 #pragma unroll
     for (int i = 0; i < kBfItems; ++i) {
-      if (i < items) {
-        int pos = 0;         // bits as signed numbers: the largest of the positive ones
-        uint32_t neg = 0u;   // as unsigned ones: the largest magnitude of the negative ones, if there are any
+      float c = 0.0f;
 #pragma unroll
-        for (int k = 0; k < CH; k += 2) {
-          const int v0 = (int)__float_as_uint(d[i / PER][(i % PER) * CH + k]), v1 = (int)__float_as_uint(d[i / PER][(i % PER) * CH + k + 1]);
-          pos = max(max(v0, v1), pos);
-          neg = max(max((uint32_t)v0, (uint32_t)v1), neg);
-        }
-        // (what is not finite makes this NaN where the mask is zero)
-        const float c = __uint_as_float(max((uint32_t)pos, neg & 0x7fffffffu)) * mask_of(i);
-        largest = max(largest, __float_as_uint(c) & 0x7fffffffu);
-      }
+      for (int k = 0; k < CH; ++k) c = __builtin_elementwise_maximum(c, fabsf(d[i / PER][(i % PER) * CH + k]));
+      // (what is not finite makes this NaN where the mask is zero)
+      c *= mask_of(i);
+      largest = __builtin_elementwise_maximum(largest, i < items ? fabsf(c) : 0.0f);
     }
-    largest = wave_max(largest);
-    if (lane == 0) red[2 * kBfWaves + wave] = __uint_as_float(largest);
+    const uint32_t bits = wave_max(__float_as_uint(largest) & 0x7fffffffu);
+    if (lane == 0) red[2 * kBfWaves + wave] = __uint_as_float(bits);
   };
   auto take_scale = [&]() {
     uint32_t bits = 0u;
@@ -406,7 +423,7 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
   };
   // Adds what the window holds of the CH channels from cf on to grad_input, and clears it.
   auto flush = [&](int cf) {
-    float *gplane = a.gin32 + ((long)n * g.Cin + cf) * plane_in;
+    float *gplane = gin + ((long)n * g.Cin + cf) * plane_in;
 #pragma unroll
     for (int j = 0; j < kSlots; ++j) {
       const uint32_t seen = j % 2 ? adds[j / 2] >> 16 : adds[j / 2] & 0xffffu;
@@ -421,13 +438,19 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
         for (int cp = 0; cp < NP; ++cp) e[cp * PLANE] = 0ull;
         if (fits && y >= 0 && y < g.H && x >= 0 && x < g.W) {
           const unsigned long long bias = (unsigned long long)seen * kRoundBits;
-          float *gi = gplane + (y * g.W + x);
+          uint32_t at = (uint32_t)(y * g.W + x) * 4u;
+          long step = plane_in;
+          asm volatile("" : "+s"(step));   // (or its multiples are kept, and put away)
+          auto into = [&](int c) {
+            asm volatile("" : "+v"(at));   // (a plane's address stays a scalar, and this beside it)
+            return (float *)((unsigned char *)(gplane + c * step) + at);
+          };
 #pragma unroll
-          for (int cp = 0; cp < NP; ++cp, gi += 2 * plane_in) {
+          for (int cp = 0; cp < NP; ++cp) {
             const long long s = (long long)(v[cp] - (bias + (bias << 32)));
             const int lo = (int)(uint32_t)s, hi = (int)((s - (long long)lo) >> 32);
-            unsafeAtomicAdd(gi, (float)lo * inv_scale);
-            unsafeAtomicAdd(gi + plane_in, (float)hi * inv_scale);
+            unsafeAtomicAdd(into(2 * cp), (float)lo * inv_scale);
+            unsafeAtomicAdd(into(2 * cp + 1), (float)hi * inv_scale);
           }
         }
       }
@@ -454,10 +477,19 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
     __syncthreads();   // the window is zero and the stages are free
     if (c0 + CH < c_end) issue_first(c0 + CH);
     take_scale();
+    const int grp_next = group_of(min(c0 + CH, c_end - 1));
     __builtin_amdgcn_sched_barrier(0);
-    E *cbase = (E *)a.col + ((((long)nl * (g.Cin / RUN) + c0 / RUN) * g.taps + half) * a.P_pad + pix) * RUN + c0 % RUN;
+    unsigned char *cbase = cols + (((long)nl * (g.Cin / RUN) + c0 / RUN) * g.taps * col_px * RUN + c0 % RUN) * 2;
+    uint32_t cat = ((uint32_t)half * col_px + pix) * (RUN * 2u);
 #pragma unroll
     for (int i = 0; i < kBfItems; ++i) {
+      // The next pass's grad_output, where the products were that are through.  (Not within the branch: the registers
+      // would be kept for the way round it.)
+      if (i == kBfItems - 3 + U) {
+        load_g_half(grp_next, 0, 0);
+        load_g_half(grp_next, 0, 1);
+        __builtin_amdgcn_sched_barrier(0);
+      }
       if (i < items) {
         Place &next = p[(i + LA) % (LA + 1)];
         const Place c = p[i % (LA + 1)];
@@ -520,8 +552,9 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
             atomicAdd(wp1 + cp * PLANE + 1, entry(s11));
             __builtin_amdgcn_sched_barrier(0);
           }
-          if (a.col && valid && has_tap(i))
-            *(uint4 *)(cbase + (long)(2 * i) * a.P_pad * RUN + h * 8) = make_uint4(cv[0], cv[1], cv[2], cv[3]);
+          asm volatile("" : "+v"(cat));
+          if (cols && valid && has_tap(i))
+            *(uint4 *)(cbase + (long)(2 * i) * col_px * (RUN * 2) + h * 16 + cat) = make_uint4(cv[0], cv[1], cv[2], cv[3]);
           __builtin_amdgcn_sched_barrier(0);
         }
         acc_m[i] += w00 * S00 + w01 * S01 + w10 * S10 + w11 * S11;
@@ -543,17 +576,16 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
           const float w = ((corner & 2) ? gy : 1.0f - gy) * ((corner & 1) ? gx : 1.0f - gx);
           const float t = lone[k];
           if (corner < 4 && yy >= 0 && yy < g.H && xx >= 0 && xx < g.W)
-            unsafeAtomicAdd(a.gin32 + ((long)n * g.Cin + c0 + k) * plane_in + ((long)yy * g.W + xx), w * t);
+            unsafeAtomicAdd(gin + ((long)n * g.Cin + c0 + k) * plane_in + ((long)yy * g.W + xx), w * t);
           __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         }
         __builtin_amdgcn_sched_barrier(0);
       }
     }
-    load_g(group_of(min(c0 + CH, c_end - 1)), 0);
     // Every add into the window has landed behind this barrier, and so have the copies of the next pass's weights.  (What is
-    // waited for beside them are the loads just above, which the products are about to use, and the last stores of columns.  A count
+    // waited for beside them are the loads of grad_output, which the products are about to use, and the last stores of columns.  A count
     // of the loads issued since the copies instead would have nothing to spare: 16 with 8 channels a pass, 5 taps and 64 output
-    // channels; and with 128 or more the compiler waits for these loads anyway.)
+    // channels.)
     settle();
   }
   flush(c_end - CH);

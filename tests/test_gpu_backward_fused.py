@@ -15,6 +15,7 @@ CASES = [
     ('edges_w16', dict(N=1, Cin=128, Cout=64, H=17, W=33)),
     ('k192', dict(N=1, Cin=64, Cout=192, H=15, W=18)),
     ('k320', dict(N=1, Cin=64, Cout=320, H=9, W=31)),
+    ('k448', dict(N=1, Cin=64, Cout=448, H=10, W=37)),
     ('k512', dict(N=1, Cin=128, Cout=512, H=13, W=21)),
     ('k640_8ch', dict(N=1, Cin=64, Cout=640, H=11, W=20, deform_groups=8)),
     ('8ch', dict(N=1, Cin=192, Cout=64, H=18, W=17, deform_groups=8)),

@@ -564,6 +564,24 @@ def test_fused_backward_waits_for_its_copies():
         assert waits and all(re.fullmatch(r's_waitcnt vmcnt\(0\)', t) and 'lds-copies' in c for t, c in waits), (name, waits)
 
 
+def test_backward_workspace_of_planes_past_32_bits():
+    """The 16-bit backward in one kernel addresses a plane's pixels with 32 bits: an input plane of 2^24 pixels, border included, or more
+    goes through memory, with an fp32 column gradient in the workspace."""
+    import ctypes
+    from mmcv_amd import capi
+    lib = capi.load()
+
+    def wanted(side):
+        bp = capi.MdcnBwdParams()
+        bp.conv = capi.make_params(capi.MDCN_BF16, 1, 64, side, side, 64, 1, 1, (2, 2), (0, 0), (1, 1), 1, 1)
+        for f in ('grad_output', 'grad_input', 'grad_offset', 'grad_mask', 'grad_weight', 'grad_bias'):
+            setattr(bp, f, 256)   # (nothing is read)
+        return lib.mdcn_backward_workspace_bytes(ctypes.byref(bp))
+
+    columns = 64 * 2047 * 2047 * 2
+    assert wanted(4093) - wanted(4091) < columns // 10 and wanted(4094) - wanted(4093) > 2 * columns
+
+
 def test_bench_refuses_more_than_one_gpu():
     """bench.py measures one GPU: --gpus above 1 ends with a message and exit status 2 before anything
     touches a device."""
