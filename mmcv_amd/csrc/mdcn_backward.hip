@@ -178,7 +178,14 @@ void make_bwd_plan(const mdcn_bwd_params *bp, const Geom &g, uint64_t pass_bytes
     }
   }
   if (pl->gemm) {
-    pl->cg_tile = (g.taps * im.cgp >= kCgTileBig && plane_out >= (size_t)kCgTileBig) ? kCgTileBig : kCgTile;
+    // Tiles of 256 for 16-bit calls that have more than two and a half rounds of them.  Otherwise of 128, two workgroups a CU: the
+    // last round is fuller, one's products cover the other's barriers, and what fp32 splits behind its LDS reads costs it no more.
+    // Training calls in us, 256 / 128: fp32 N=2 256 channels 50x84 (306 tiles of 256) 404 / 380; N=1 512 25x42 (90) 284 / 260; N=8 512 13x21
+    // 424 / 380; N=2 256 100x152 (1 080) 1 058 / 1 029; N=8 256 64x64 (1 152) 1 045 / 1 031; bf16 N=4 96 -> 72 37x53 (128) 113 / 110; N=4
+    // 240 60x60 (540) 336 / 331; N=8 104 -> 96 100x100 (1 280) 713 / 720; N=8 312 -> 300 90x100 (3 168) 2 092 / 2 133.
+    const long big_tiles = (long)pl->n_chunk * g.G * (((long)plane_out + kCgTileBig - 1) / kCgTileBig) *
+                           ((g.taps * im.cgp + kCgTileBig - 1) / kCgTileBig);
+    pl->cg_tile = (es == 2 && g.taps * im.cgp >= kCgTileBig && plane_out >= (size_t)kCgTileBig && big_tiles > 640) ? kCgTileBig : kCgTile;
     pl->M_pad = pl->fused ? g.taps * im.cgp : padded(g.taps * im.cgp, pl->cg_tile);
     pl->gt_bytes = align_up((size_t)g.N * g.G * om.cgp * plane_out * es);
     pl->wt_bytes = align_up((size_t)g.G * pl->M_pad * om.cgp * es);
@@ -194,11 +201,18 @@ void make_bwd_plan(const mdcn_bwd_params *bp, const Geom &g, uint64_t pass_bytes
     pl->P_pad = ((long)plane_out + kpx - 1) / kpx * kpx;
     pl->col_bytes = align_up((size_t)pl->n_chunk * g.taps * cin_p * pl->P_pad * es);
     const int M = g.taps * im.cgp;
-    pl->w_tile = (g.cout_g >= 192 && M >= kCgTileBig) ? kCgTileBig : kCgTile;
+    const long work = (long)pl->n_chunk * (pl->P_pad / kpx);
+    // Tiles of 256 where a workgroup's share is long enough: K steps of it were the chip filled evenly.  Shorter ones are mostly
+    // their first copies and the partial sums, of which two workgroups of 128 a CU do one beside the other's products.
+    // Training calls in us, 256 / 128: fp32 steps of 4.7 (N=1 256 channels 50x84) 245 / 234, 9.3 (N=2) 385 / 380, 10.1 (N=8 512 13x21) 380 / 383,
+    // 16.7 (N=1 256 100x152) 587 / 589, 23.7 (N=3 256 72x100) 835 / 842; bf16 and fp16 steps of 0.4 (N=1 512 13x13) 108 / 101, 2.4 (N=1 512
+    // 25x42) 132 / 121, 4.6 (N=2 256 50x84) 174 / 166, 9.3 (N=4) 272 / 260, 19.1 (N=8 512 25x42) 351 / 345, 22.8 (N=8 256 72x72) 508 / 507,
+    // 25.1 (N=3 256 100x152) 525 / 537, 28.7 (N=12 512 25x42) 482 / 473, 33.5 (N=4 256 100x152) 637 / 653, 66.9 (N=8) 1 203 / 1 246.
+    const long big_steps = work * g.G * ((g.cout_g + kCgTileBig - 1) / kCgTileBig) * ((M + kCgTileBig - 1) / kCgTileBig);
+    pl->w_tile = (g.cout_g >= 192 && M >= kCgTileBig && big_steps > 256L * (es == 4 ? 10 : 20)) ? kCgTileBig : kCgTile;
     const long tiles = (long)g.G * ((g.cout_g + pl->w_tile - 1) / pl->w_tile) * ((M + pl->w_tile - 1) / pl->w_tile);
     // one round of workgroups (256-tiles: one per CU, 128-tiles: two), shares of at least 8 K steps
     const long slots = pl->w_tile == kCgTileBig ? 256 : 512;
-    const long work = (long)pl->n_chunk * (pl->P_pad / kpx);
     pl->w_splits = (int)std::max<long>(1, std::min<long>(std::min<long>(work / 8, 64), slots / tiles));
     pl->wpart_bytes = align_up((size_t)pl->w_splits * g.Cout * M * 4);
     // grad_output rows go to LDS 16 bytes at a time: in place when they start aligned
@@ -445,9 +459,12 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
       ca.n0 = n0;
       ca.total = (long)nb * g.G * ca.px_tiles * ca.m_tiles;
       const dim3 grid((unsigned)((ca.total + 7) / 8 * 8));
-      if (pl.cg_tile == kCgTileBig)
-        hipLaunchKernelGGL((bwd_colgrad_kernel<E, kCgTileBig>), grid, dim3(2 * kCgTileBig), 0, st, ca);
-      else
+      bool big = false;
+      if constexpr (sizeof(E) == 2) {
+        big = pl.cg_tile == kCgTileBig;
+        if (big) hipLaunchKernelGGL((bwd_colgrad_kernel<E, kCgTileBig>), grid, dim3(2 * kCgTileBig), 0, st, ca);
+      }
+      if (!big)
         hipLaunchKernelGGL((bwd_colgrad_kernel<E, kCgTile>), grid, dim3(2 * kCgTile), 0, st, ca);
       check();
     }

@@ -195,3 +195,18 @@ def test_large_plane_of_uneven_channels(dtype):
     for nm, r, o, share in zip(NAMES, ref, got, (0.5, 0.5, 0.5, 0.7, 1.0)):
         err = float((o.double() - r).norm() / r.norm())
         assert err <= share * u, (nm, err)
+
+
+@pytest.mark.parametrize('dtype,n,h,w', [(torch.float32, 1, 100, 103), (torch.bfloat16, 4, 92, 100), (torch.float16, 2, 90, 100)],
+                         ids=['f32', 'bf16', 'f16'])
+def test_large_products(dtype, n, h, w):
+    """Just above the sizes from which the products run in tiles of 256 (2 898 and 5 184 K steps for the weight gradient of fp32 and
+    bf16, 648 tiles of the fp16 column gradient), channels uneven.  fp32 sums of up to 10 300 products: 1e-5 of the norm; 16 bits: one
+    rounding of the result and one of the columns."""
+    print(f'dtype={dtype} n={n}', flush=True)
+    dev = cast_case(make_case(57, N=n, Cin=232, Cout=200, H=h, W=w), dtype, 'cuda')
+    gy = torch.randn(n, 200, h, w, generator=torch.Generator().manual_seed(9)).to(dtype).cuda()
+    ref = capi_backward({k: v.double() if torch.is_tensor(v) else v for k, v in dev.items()}, gy.double())
+    for nm, r, o in zip(NAMES, ref, capi_backward(dev, gy)):
+        err = float((o.double() - r).norm() / r.norm())
+        assert err <= {torch.float32: 1e-5, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype], (nm, err)
