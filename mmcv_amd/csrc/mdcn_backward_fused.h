@@ -214,6 +214,10 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
 #pragma unroll
     for (int j = 0; j < 4; ++j) gf[4 * s + j] = *(const uint4 *)(p + j * 32 + at);
   };
+  // Whether a pass's first chunk has its second half loaded.  Passes of 8 channels leave it out with 64 output channels (N=4 64
+  // channels, 8 deformable groups, 120x160: 302 -> 286 us); with 16 the branch costs 44 reloads of spilled registers, and more than it saves
+  // (N=4 256 channels 50x84: 260 -> 269).
+  auto first_second = [&]() { return CH == 16 || whole_chunk(0); };
   // the first two stages of a pass
   auto issue_first = [&](int c0) {
     issue(c0, 0);
@@ -245,7 +249,7 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
   // (The barrier ends the tile before: nobody is at the window any more.)
   __syncthreads();
   load_g_half(group_of(c_begin), 0, 0);
-  load_g_half(group_of(c_begin), 0, 1);
+  if (first_second()) load_g_half(group_of(c_begin), 0, 1);
   // (the counts of adds go where the window will be)
   for (int i = tid; i < win_px; i += kBfThreads) ((uint32_t *)win)[i] = 0u;
   // A mask of zero where nothing is sampled, and the tile's largest
@@ -487,7 +491,7 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
       // would be kept for the way round it.)
       if (i == kBfItems - 3 + U) {
         load_g_half(grp_next, 0, 0);
-        load_g_half(grp_next, 0, 1);
+        if (first_second()) load_g_half(grp_next, 0, 1);
         __builtin_amdgcn_sched_barrier(0);
       }
       if (i < items) {
