@@ -72,12 +72,13 @@ __device__ __forceinline__ uint32_t wave_max(uint32_t v) {
 // Every wait among its items is for loads that are due: whatever the compiler keeps in scratch or fetches from the argument
 // block again there makes it wait for all loads, or all LDS adds, under way (the kernel took 2.1 ms in the shape below with either,
 // 1.35 without).  Hence the asm statements without text below: they hold a sum where it is, and a value in its register.
-// Window: 32-bit fixed point in LDS.  Its scale is the pass's own: from the largest |d * mask| of a sample of the tile and
-// the number of adds the busiest entry sees, so that no contribution leaves 2^21 and no sum of them 2^30.  The
+// Window: 32-bit fixed point in LDS.  Its scale is the pass's own: from the largest |d| of its products over the tile, the largest
+// mask value and the number of adds the busiest entry sees, so that no contribution leaves 2^21 and no sum of them 2^30.  The
 // first decides where no entry sees more than 512, and the quantum is then 2^-20 or 2^-21 of the largest contribution there could
-// be.  (The largest |d| times the largest mask, wherever each of them is, is an instruction a tap less, and loses bits to a
-// large gradient under a small mask: fp16, one pixel of a mask of 0 and 1 000 times the gradient: error of grad_input 3.3e-3 of its
-// norm where this has 2.1e-4, its one rounding.)  (Bounds of |d| from norms of grad_output and weights instead: training calls of N=16 256 channels 100x152 in bf16 2 319
+// be.  Where the largest |d * mask| of a sample gives three bits or more, the scale is from that instead: else one large gradient
+// under a small mask takes bits from its whole tile (fp16, one pixel of a mask of 0 and 1 000 times the gradient: error of grad_input
+// 3.3e-3 of its norm, so 2.1e-4, its one rounding).  Below three bits (inputs whose large gradients and open masks meet somewhere in a
+// tile) results stay those of the first scale, bit for bit.  The second costs N=16 256 channels 100x152 in bf16 0.6 % (2 247 -> 2 261 us).  (Bounds of |d| from norms of grad_output and weights instead: training calls of N=16 256 channels 100x152 in bf16 2 319
 // us where this takes 2 329, of N=8 512 channels 25x42 in fp16 371 / 363.  But such a scale goes by gradients that the weights do not
 // carry on: fp16, 256 output channels, one of them without weights and with 300 times the gradient: error of grad_input
 // 8.6e-4 of its norm, where its one rounding is 2.1e-4 and this stays at that.)
@@ -145,7 +146,7 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
 
   // This lane's taps 2 i + half: offsets, mask and place in the kernel
   uint32_t t_off[kBfItems], t_m[kBfItems];   // dy | dx << 16; mask | row << 16 | column << 24, a row of 255: no such tap
-  float *lone = red + 3 * kBfWaves + wave * 16;   // of this wavefront
+  float *lone = red + 5 * kBfWaves + wave * 16;   // of this wavefront
   const int items = (g.taps + 1) / 2, blocks = (items + PER - 1) / PER;
 
   // (zero where nothing is sampled, once the tile has begun)
@@ -252,19 +253,26 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
   if (first_second()) load_g_half(group_of(c_begin), 0, 1);
   // (the counts of adds go where the window will be)
   for (int i = tid; i < win_px; i += kBfThreads) ((uint32_t *)win)[i] = 0u;
-  // A mask of zero where nothing is sampled, and the tile's largest
+  // Largest mask value and the sum of all of the tile's; then a mask of zero where nothing is sampled
   {
-    uint32_t top = 0u;
+    float top = 0.0f, sum = 0.0f;
 #pragma unroll
     for (int i = 0; i < kBfItems; ++i) {
       const uint32_t one = (uint32_t)__builtin_bit_cast(uint16_t, from_f32<E>(1.0f));
       const uint32_t m = a.om.logit == kMaskNone ? one : t_m[i] & 0xffffu;   // (1: unmodulated)
+      const float v = valid && has_tap(i) ? fabsf(to_f32(__builtin_bit_cast(E, (uint16_t)m))) : 0.0f;
+      top = fmaxf(top, v);   // (NaN is left out: where it is sampled, the largest |d * mask| has it)
+      sum += v;
       t_m[i] = (t_m[i] & 0xffff0000u) | (place(i).inside ? m : 0u);
       asm volatile("" : "+v"(t_off[i]), "+v"(t_m[i]));   // (here and now, or the halves they are made of are kept)
-      top = max(top, __float_as_uint(fabsf(mask_of(i))));
     }
-    top = wave_max(top);
-    if (lane == 0) red[wave] = __uint_as_float(top);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
+    const uint32_t bits = wave_max(__float_as_uint(top));
+    if (lane == 0) {
+      red[wave] = __uint_as_float(bits);
+      red[kBfWaves + wave] = sum;
+    }
   }
   __syncthreads();
   auto window_at = [&](const Place &p, bool &in_win) {
@@ -275,7 +283,9 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
   };
   // How many adds the window pixels that this thread flushes (tid, tid + 512, ...) see in a pass, 16 bits each
   uint32_t adds[(kSlots + 1) / 2];
-  float mask_top, adds_top;   // the largest mask value, and the largest number of adds
+  // Largest mask value, a bound on the sum of those of an entry, largest number of adds.  (In LDS: as scalars of the whole tile they cost
+  // registers that are then short elsewhere.)
+  float *tops = red + (5 + 16) * kBfWaves;
   {
 #pragma unroll
     for (int i = 0; i < kBfItems; ++i) {
@@ -298,17 +308,21 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
       most = max(most, c);
     }
     most = wave_max(most);
-    if (lane == 0) red[kBfWaves + wave] = __uint_as_float(most);
+    if (lane == 0) red[2 * kBfWaves + wave] = __uint_as_float(most);
     __syncthreads();
-    uint32_t top = 0u;
+    float top = 0.0f, sum = 0.0f;
     most = 0u;
 #pragma unroll
     for (int w = 0; w < kBfWaves; ++w) {
-      top = max(top, __float_as_uint(red[w]));
-      most = max(most, __float_as_uint(red[kBfWaves + w]));
+      top = fmaxf(top, red[w]);
+      sum += red[kBfWaves + w];
+      most = max(most, __float_as_uint(red[2 * kBfWaves + w]));
     }
-    mask_top = __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)top));
-    adds_top = __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint((float)most)));
+    if (tid == 0) {
+      tops[0] = top;
+      tops[1] = fminf(sum, (float)most * top);
+      tops[2] = (float)most;
+    }
     for (int i = tid; i < PLANE * NP / 2; i += kBfThreads) ((uint4 *)win)[i] = make_uint4(0u, 0u, 0u, 0u);
   }
   // The scale of the pass in the window, and whether there is one
@@ -399,28 +413,43 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
 #pragma unroll
     for (int j = 0; j < 8; ++j) asm volatile("" : "+v"(gf[j].x), "+v"(gf[j].y), "+v"(gf[j].z), "+v"(gf[j].w));
   };
-  // Leaves the largest |d * mask| of this wavefront, as bits (NaN above all), where the others find it behind a barrier.
+  // Leaves the largest |d| and the largest |d * mask| of this wavefront, as bits (NaN above all), where the others find them behind a
+  // barrier.
   auto put_largest = [&]() {
-    float largest = 0.0f;
+    float largest_d = 0.0f, largest = 0.0f;
 #pragma unroll
     for (int i = 0; i < kBfItems; ++i) {
       float c = 0.0f;
 #pragma unroll
       for (int k = 0; k < CH; ++k) c = __builtin_elementwise_maximum(c, fabsf(d[i / PER][(i % PER) * CH + k]));
+      largest_d = __builtin_elementwise_maximum(largest_d, i < items ? c : 0.0f);
       // (what is not finite makes this NaN where the mask is zero)
       c *= mask_of(i);
       largest = __builtin_elementwise_maximum(largest, i < items ? fabsf(c) : 0.0f);
     }
+    const uint32_t bits_d = wave_max(__float_as_uint(largest_d) & 0x7fffffffu);
     const uint32_t bits = wave_max(__float_as_uint(largest) & 0x7fffffffu);
-    if (lane == 0) red[2 * kBfWaves + wave] = __uint_as_float(bits);
+    if (lane == 0) {
+      red[3 * kBfWaves + wave] = __uint_as_float(bits_d);
+      red[4 * kBfWaves + wave] = __uint_as_float(bits);
+    }
   };
   auto take_scale = [&]() {
-    uint32_t bits = 0u;
-#pragma unroll
-    for (int w = 0; w < kBfWaves; ++w) bits = max(bits, __float_as_uint(red[2 * kBfWaves + w]));
-    const float one = __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)bits));
-    const float all = one * adds_top;   // bounds of a contribution and of a sum
-    const int e = (all > 0.0f && all < 3.0e38f) ? min(29 - ilogbf(all), 20 - ilogbf(one)) : 0;
+    // (the waves' eight words of either, a lane each, and the largest of eight lanes: sixteen reads at once are registers too many here)
+    uint32_t bits = __float_as_uint(red[3 * kBfWaves + (lane & 15)]);
+    bits = max(bits, (uint32_t)__builtin_amdgcn_mov_dpp((int)bits, 0xB1, 0xf, 0xf, true));    // of two
+    bits = max(bits, (uint32_t)__builtin_amdgcn_mov_dpp((int)bits, 0x4E, 0xf, 0xf, true));    // of four
+    bits = max(bits, (uint32_t)__builtin_amdgcn_mov_dpp((int)bits, 0x141, 0xf, 0xf, true));   // of eight
+    const float dmax = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)bits, 0));
+    const float one = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)bits, 8));
+    // exponent of a scale, from a bound of a sum and one of a contribution
+    auto exponent = [](float all, float one) {
+      return (all > 0.0f && all < 3.0e38f) ? min(29 - ilogbf(all), one > 0.0f ? 20 - ilogbf(one) : 120) : 0;
+    };
+    const float mask_top = tops[0];
+    const float apart = dmax * tops[1], all = one * tops[2];
+    const int e_apart = exponent(apart, dmax * mask_top), e_one = exponent(all, one);
+    const int e = !(apart < 3.0e38f) || e_one >= e_apart + 3 ? e_one : e_apart;
     scale = __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint(ldexpf(1.0f, min(120, e)))));
     inv_scale = 1.0f / scale;
     fits = __builtin_amdgcn_readfirstlane(all < 3.0e38f && e <= 120 && mask_top * scale < 3.0e38f) != 0;  // (false for NaN)
@@ -624,7 +653,7 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
 template <typename E, int CH, int CHF, bool DEEP>
 __global__ __launch_bounds__(kBfThreads, 2) void bwd_fused_kernel(BwdFusedArgs a) {
   __shared__ uint4 lds[kBfLdsBytes / 16];
-  __shared__ float red[(3 + 16) * kBfWaves];
+  __shared__ float red[(5 + 16) * kBfWaves + 3];
   asm volatile("; mdcn-counted-waits");
   bool far = false;
   if (a.win_far.WH > 0) {

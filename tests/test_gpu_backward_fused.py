@@ -132,6 +132,26 @@ def test_closed_gates(name, count, fg, mask, dtype):
     assert err <= U[dtype] * SHARE['grad_input'], err
 
 
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16], ids=['bf16', 'f16'])
+@pytest.mark.parametrize('mask,e', [(0.25, 20), (2.0 ** -4, 24)], ids=['within_3_bits', 'beyond'])
+def test_quantum(mask, e, dtype):
+    """The window's quantum, bit for bit: 2^-20 of the largest |d| times the largest mask, wherever each of them is, and of the largest
+    product of the two only where that gives three bits or more."""
+    print(f'mask={mask} dtype={dtype}', flush=True)
+    # 1x1 kernel, weights of one, integer positions: the column gradient is grad_output, a pixel has one contribution
+    case = make_case(77, N=1, Cin=64, Cout=64, H=16, W=16, k=(1, 1), padding=0)
+    case['weight'] = torch.eye(64).reshape(64, 64, 1, 1)
+    case['offset'].zero_()
+    case['mask'].fill_(0.25)
+    case['mask'][0, 0, 5, 6], case['mask'][0, 0, 11, 3] = 1.0, mask
+    gy = torch.randn(1, 64, 16, 16, generator=torch.Generator().manual_seed(11)) * 2.0 ** -14
+    gy[0, ::8, 11, 3] = 1.0   # (in every pass's channels)
+    dev, gy = cast_case(case, dtype, 'cuda'), gy.to(dtype).cuda()
+    got = capi_backward(dev, gy, path=capi.PATH_FUSED)[0]
+    ref = torch.round(gy.double() * dev['mask'].double() * 2.0 ** e) * 2.0 ** -e
+    assert torch.equal(got, ref.to(dtype)), float((got.double() - ref).abs().max() * 2.0 ** e)
+
+
 def test_passes_of_images():
     """Cut tiles of several passes of images, the last one of another size, have places of their own for their shares."""
     kw = dict(N=5, Cin=64, Cout=64, H=33, W=47)
