@@ -168,7 +168,9 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
     p.inside = valid && row != 255 && py > -1.0f && px > -1.0f && py < (float)g.H && px < (float)g.W;
     const float fy = floorf(py), fx = floorf(px);
     p.y0 = p.inside ? (int)fy : -1;
-    p.x0 = p.inside ? (int)fx : -1;
+    // (nothing sampled: the right border of the row above the image, whose next pixel is the left one of the image's first: four
+    // zeros.  At -1 the last corner would be the image's first pixel, and d times it an infinity where neither is.)
+    p.x0 = p.inside ? (int)fx : g.W;
     p.ly = p.inside ? py - fy : 0.0f;
     p.lx = p.inside ? px - fx : 0.0f;
     return p;

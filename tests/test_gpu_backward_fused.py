@@ -152,6 +152,25 @@ def test_quantum(mask, e, dtype):
     assert torch.equal(got, ref.to(dtype)), float((got.double() - ref).abs().max() * 2.0 ** e)
 
 
+@pytest.mark.parametrize('groups', [1, 8], ids=['16ch', '8ch'])
+def test_large_gradients_where_nothing_is_sampled(groups):
+    """A sample beyond the image has gradients of zero, whatever the column gradient there times a corner of the image is."""
+    print(f'groups={groups}', flush=True)
+    case = make_case(76, N=1, Cin=64, Cout=64, H=33, W=40, deform_groups=groups)
+    gy = torch.randn(1, 64, 33, 40, generator=torch.Generator().manual_seed(10))
+    gy[:, :, 9, 7] *= 1e37
+    case['offset'][:, :, 9, 7] = 1e4
+    case['input'][:, :, :2, :2] *= 1e3
+    dev, gy = cast_case(case, torch.bfloat16, 'cuda'), gy.bfloat16().cuda()
+    ref = capi_backward({k: v.double() if torch.is_tensor(v) else v for k, v in dev.items()}, gy.double())
+    got = capi_backward(dev, gy, path=capi.PATH_FUSED)
+    for nm, r, o in zip(NAMES[:4], ref, got):   # (grad_bias: a sum of gradients up to 1e38)
+        assert bool(o.isfinite().all()), nm
+        err = float((o.double() - r).norm() / r.norm())
+        assert err <= U[torch.bfloat16] * SHARE[nm], (nm, err)
+    assert not bool(got[1][:, :, 9, 7].any()) and not bool(got[2][:, :, 9, 7].any())
+
+
 def test_passes_of_images():
     """Cut tiles of several passes of images, the last one of another size, have places of their own for their shares."""
     kw = dict(N=5, Cin=64, Cout=64, H=33, W=47)
