@@ -449,8 +449,8 @@ __device__ __forceinline__ void scatter_tile(const BwdScatterArgs &a, const Scat
   }
 
   // One tap's sampling position and what was loaded there.  No branch around a tap's body: a
-  // position outside the sampling range (or a lane past the image) samples the border's corner
-  // pixel with weights, mask and d of zero, so it stores a column of zeros and adds zeros.
+  // position outside the sampling range (or a lane past the image) samples four pixels of the
+  // border with weights, mask and d of zero, so it stores a column of zeros and adds zeros.
   // Per-corner conditions become weights of zero too: a wavefront pays for an LDS atomic
   // whether or not a lane sits it out, and a branch per corner and channel was most of the
   // instructions this kernel issued.
@@ -473,7 +473,7 @@ __device__ __forceinline__ void scatter_tile(const BwdScatterArgs &a, const Scat
     s.inside = valid && (py > -1.0f) && (px > -1.0f) && (py < (float)g.H) && (px < (float)g.W);
     const float fy = floorf(py), fx = floorf(px);
     s.y0 = s.inside ? (int)fy : -1;
-    s.x0 = s.inside ? (int)fx : -1;
+    s.x0 = s.inside ? (int)fx : g.W;   // (nothing sampled: four zeros, the right border's above the image and the pixel behind each)
     s.ly = s.inside ? py - fy : 0.0f;
     s.lx = s.inside ? px - fx : 0.0f;
     s.m = s.inside ? mask_value<E>(e_m, a.om.logit) : 0.0f;

@@ -171,6 +171,24 @@ def test_large_gradients_where_nothing_is_sampled(groups):
     assert not bool(got[1][:, :, 9, 7].any()) and not bool(got[2][:, :, 9, 7].any())
 
 
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16, torch.float16], ids=['f32', 'bf16', 'f16'])
+@pytest.mark.parametrize('cin,path', [(64, capi.PATH_FUSED), (40, capi.PATH_AUTO)], ids=['whole', 'uneven'])
+def test_corner_pixel_that_nobody_samples(cin, path, dtype):
+    """An infinity in the image's first pixel, and samples beyond the image, but none of that pixel: no gradient has it."""
+    print(f'cin={cin} dtype={dtype}', flush=True)
+    case = make_case(78, N=2, Cin=cin, Cout=64, H=17, W=40)
+    case['offset'] = 3.0 + torch.randint(1, 4, case['offset'].shape, generator=torch.Generator().manual_seed(12)) / 4
+    case['offset'][:, :, 9, 7] = 1e4
+    gy = torch.randn(2, 64, 17, 40, generator=torch.Generator().manual_seed(13))
+    dev, gy = cast_case(case, dtype, 'cuda'), gy.to(dtype).cuda()
+    bad = dict(dev, input=dev['input'].clone())
+    bad['input'][:, :, 0, 0] = float('inf')
+    for want in (dict(), dict(want_data=False)):
+        ref, got = capi_backward(dev, gy, path=path, **want), capi_backward(bad, gy, path=path, **want)
+        for nm, a, b in zip(NAMES[1:], got[1:], ref[1:]):   # (grad_input is summed in no order, and the image has no part in it)
+            assert torch.equal(a, b), (nm, want)
+
+
 def test_passes_of_images():
     """Cut tiles of several passes of images, the last one of another size, have places of their own for their shares."""
     kw = dict(N=5, Cin=64, Cout=64, H=33, W=47)
