@@ -88,13 +88,18 @@ void make_bwd_plan(const mdcn_bwd_params *bp, const Geom &g, uint64_t pass_bytes
   // whose channels fill nothing (bf16, N=4, 96 -> 72, 37x53) 0.12 ms instead of 0.90.
   const int KC = (int)(128 / es);
   const long s_tiles = (long)g.N * g.DG * ((g.Ho + kScTH - 1) / kScTH) * ((g.Wo + kScTW - 1) / kScTW);
-  // 16-bit tensors whose channels come in whole 128-byte slabs: the data side in one kernel, d in registers and grad_input summed in
-  // fixed point that leaves it its one rounding.  What is uneven, and fp32, goes through memory with an fp32 d and sums in doubles.
-  // (bf16 backward in us, this kernel / the other path: N=1 64 channels 25x42, 8 tiles, 50 / 60; N=1 512 25x42, 8, 103 / 233; N=2 256 50x84, 42,
-  // 147 / 219; N=3 512 40x60 stride 2, 4 deformable groups, 36, 142 / 180; N=4 256 50x84, 84, 234 / 353; N=1 64 100x152, 65, 84 / 100.)
+  // 16-bit tensors whose channels come in whole 128-byte slabs, and 64 or more tiles of them: the data side in one kernel,
+  // d in registers and grad_input summed in fixed point.  What is smaller or uneven, and fp32, goes through memory with
+  // an fp32 d and sums in doubles.
+  // (The 64 is a line of precision, not of speed: small calls have had sums in doubles since before this kernel, and fixed point takes
+  // bits from gradients beside much larger ones of the same tile -- error of the others by themselves, beside one
+  // pixel of 1e3 / 1e5 times their gradient: fp16 2.2e-3 / 0.18 of their norm, bf16 3.1e-3 / 0.20, where sums in doubles leave one
+  // rounding, 2.1e-4 and 1.7e-3.  Whole training calls in us, this
+  // kernel / the other path: bf16 N=1 512 channels 25x42, 8 tiles, 130 / 163; fp16 N=2 256 50x84, 42, 178 / 226; bf16 N=4 512 25x42, 32, 239 /
+  // 316; N=3 512 40x60 stride 2, 4 deformable groups, 36, 192 / 220; N=1 128 56x56, 14, 82 to 111 / 94.)
   const bool whole = g.Cin % KC == 0 && g.cout_g % KC == 0 && g.cin_g % 32 == 0 && g.ch_per_dg % 8 == 0;
-  pl->fused = staged && bp->grad_input && whole && (g.kh - 1) * g.dh < 255 && (g.kw - 1) * g.dw < 255 && s_tiles < (1L << 28) &&
-              (long)g.Ho * g.Wo < kBfPlaneMax && (long)g.Hp * g.Wp < kBfPlaneMax;
+  pl->fused = staged && bp->grad_input && whole && (s_tiles >= 64 || forced) && (g.kh - 1) * g.dh < 255 && (g.kw - 1) * g.dw < 255 &&
+              s_tiles < (1L << 28) && (long)g.Ho * g.Wo < kBfPlaneMax && (long)g.Hp * g.Wp < kBfPlaneMax;
   const bool columns_only = staged && !bp->grad_input;
   const size_t ds = pl->fused || columns_only ? es : 4;  // bytes of an element of d, or of the columns
   int u = g.cin_g, v = g.ch_per_dg;

@@ -1,4 +1,4 @@
-// Backward on the matrix cores, for fp32 tensors and for 16-bit calls of uneven channels (the others have
+// Backward on the matrix cores, for fp32 tensors and for 16-bit calls of few tiles or uneven channels (the others have
 // bwd_fused_kernel for the data side, and bwd_wgrad_kernel here): the column
 // gradient  d[pixel, (tap, c)] = sum_co grad_output[co, pixel] * weight[co, c, tap]
 // (the reference's first GEMM, mmcv/ops/csrc/pytorch/modulated_deform_conv.cpp:199-206)

@@ -135,6 +135,35 @@ def test_small_16bit_gradients_are_rounded_once(name, dtype):
             assert worst <= 1.0, (nm, n, worst)
 
 
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16], ids=['bf16', 'f16'])
+@pytest.mark.parametrize('name', ['few_tiles', 'one_tile', 'seg20', 's2'])
+def test_small_16bit_gradients_beside_a_large_one(name, dtype):
+    """... and in a tile of which one pixel, its mask open, has 1e5 times the gradient of the others: what that pixel does not reach
+    keeps the bits it has by itself."""
+    print(f'case={name} dtype={dtype}', flush=True)
+    kw = dict(CASES + [('few_tiles', dict(N=2, Cin=128, Cout=64, H=14, W=30)), ('one_tile', dict(N=1, Cin=64, Cout=128, H=8, W=17))])[name]
+    case = make_case(58, **kw)
+    frac = torch.randint(1, 4, case['offset'].shape, generator=torch.Generator().manual_seed(1)) / 4
+    case['offset'] = torch.floor(case['offset']) + frac
+    gy = torch.randn(kw['N'], kw['Cout'], *case['offset'].shape[2:], generator=torch.Generator().manual_seed(6)) / 64
+    case['mask'][0, :, 4, 4] = 1.0
+    even = gy.clone()
+    even[0, :, 4, 4] = 0.0
+    gy[0, :, 4, 4] *= 1e5
+    dev, gyd = cast_case(case, dtype, 'cuda'), gy.to(dtype).cuda()
+    got = capi_backward(dev, gyd)[0].double()
+    wide = {k: v.double() if torch.is_tensor(v) else v for k, v in dev.items()}
+    ref, alone = (capi_backward(wide, v.to(dtype).double().cuda())[0] for v in (gy, even))
+    far = ref == alone   # elements that the pixel does not reach
+    assert far.sum() > far.numel() // 2
+    half_ulp, tiny = (2.0 ** -8, 0.0) if dtype == torch.bfloat16 else (2.0 ** -11, 2.0 ** -25)
+    # (sums of cout fp32 products: 2^-24 each of terms no larger than the largest of these sums)
+    bound = ref.abs() * half_ulp + tiny + (kw['Cout'] + 9 * kw['Cin']) * 2.0 ** -24 * ref[far].abs().max()
+    worst = float(((got - ref).abs() / bound)[far].max())
+    print(worst, flush=True)
+    assert worst <= 1.0, worst
+
+
 @pytest.mark.parametrize('cin,groups', [(40, 1), (24, 2), (6, 1)])
 def test_stale_workspace(cin, groups):
     """Nothing depends on what the workspace held: not the results, and not the way they are computed either (fp32 sums
