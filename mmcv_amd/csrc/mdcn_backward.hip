@@ -183,14 +183,20 @@ void make_bwd_plan(const mdcn_bwd_params *bp, const Geom &g, uint64_t pass_bytes
     }
   }
   if (pl->gemm) {
-    // Tiles of 256 for 16-bit calls that have more than two and a half rounds of them.  Otherwise of 128, two workgroups a CU: the
-    // last round is fuller, one's products cover the other's barriers, and what fp32 splits behind its LDS reads costs it no more.
+    // Tiles of 256 for 16-bit calls that have more than two and a half rounds of them, and for fp32 calls of three rounds whose
+    // rounds are full: what they are filled with, in tiles of 128, is 7 in 8 (16 K steps or more) to 15 in 16 (8) or more.  Otherwise of 128, two workgroups
+    // a CU: the last round is fuller, one's products cover the other's barriers, and what fp32 splits behind its LDS reads costs it no more.
     // Training calls in us, 256 / 128: fp32 N=2 256 channels 50x84 (306 tiles of 256) 404 / 380; N=1 512 25x42 (90) 284 / 260; N=8 512 13x21
-    // 424 / 380; N=2 256 100x152 (1 080) 1 058 / 1 029; N=8 256 64x64 (1 152) 1 045 / 1 031; bf16 N=4 96 -> 72 37x53 (128) 113 / 110; N=4
-    // 240 60x60 (540) 336 / 331; N=8 104 -> 96 100x100 (1 280) 713 / 720; N=8 312 -> 300 90x100 (3 168) 2 092 / 2 133.
-    const long big_tiles = (long)pl->n_chunk * g.G * (((long)plane_out + kCgTileBig - 1) / kCgTileBig) *
-                           ((g.taps * im.cgp + kCgTileBig - 1) / kCgTileBig);
-    pl->cg_tile = (es == 2 && g.taps * im.cgp >= kCgTileBig && plane_out >= (size_t)kCgTileBig && big_tiles > 640) ? kCgTileBig : kCgTile;
+    // 424 / 380; 256 channels, 8 K steps: filled to 0.87 (N=12 50x84) 1 790 / 1 765, 0.90 (N=8 64x64) 1 077 / 1 060, 0.93 (N=16 50x84) 2 300 / 2 283,
+    // 0.93 (N=4 100x152) 2 028 / 2 011, 0.97 (N=6 100x152) 2 922 / 2 994, 1 (N=16 64x64) 2 014 / 2 020; 512 channels, 16: 0.75 (N=8 32x32) 915 / 891,
+    // 0.90 (N=16 32x32) 1 614 / 1 626, 0.90 (N=4 64x64) 1 630 / 1 647, 0.93 (N=8 50x84) 3 487 / 3 566, 0.95 (N=6 48x48) 1 596 / 1 625; bf16 N=4 96 -> 72
+    // 37x53 (128 tiles) 113 / 110; N=4 240 60x60 (540) 336 / 331; N=8 104 -> 96 100x100 (1 280) 713 / 720; N=8 312 -> 300 90x100 (3 168) 2 092 / 2 133.
+    auto tiles_of = [&](long tile) {
+      return (long)pl->n_chunk * g.G * (((long)plane_out + tile - 1) / tile) * ((g.taps * im.cgp + tile - 1) / tile);
+    };
+    const long big_tiles = tiles_of(kCgTileBig), rounds = (big_tiles + 255) / 256, k_steps = om.cgp * (long)es / 128;
+    const bool full = big_tiles >= 768 && tiles_of(kCgTile) * 128 >= rounds * 4 * 256 * (128 - std::min<long>(16, k_steps));
+    pl->cg_tile = (g.taps * im.cgp >= kCgTileBig && plane_out >= (size_t)kCgTileBig && (es == 2 ? big_tiles > 640 : full)) ? kCgTileBig : kCgTile;
     pl->M_pad = pl->fused ? g.taps * im.cgp : padded(g.taps * im.cgp, pl->cg_tile);
     pl->gt_bytes = align_up((size_t)g.N * g.G * om.cgp * plane_out * es);
     pl->wt_bytes = align_up((size_t)g.G * pl->M_pad * om.cgp * es);
@@ -464,12 +470,9 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
       ca.n0 = n0;
       ca.total = (long)nb * g.G * ca.px_tiles * ca.m_tiles;
       const dim3 grid((unsigned)((ca.total + 7) / 8 * 8));
-      bool big = false;
-      if constexpr (sizeof(E) == 2) {
-        big = pl.cg_tile == kCgTileBig;
-        if (big) hipLaunchKernelGGL((bwd_colgrad_kernel<E, kCgTileBig>), grid, dim3(2 * kCgTileBig), 0, st, ca);
-      }
-      if (!big)
+      if (pl.cg_tile == kCgTileBig)
+        hipLaunchKernelGGL((bwd_colgrad_kernel<E, kCgTileBig>), grid, dim3(2 * kCgTileBig), 0, st, ca);
+      else
         hipLaunchKernelGGL((bwd_colgrad_kernel<E, kCgTile>), grid, dim3(2 * kCgTile), 0, st, ca);
       check();
     }

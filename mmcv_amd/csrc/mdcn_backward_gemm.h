@@ -34,10 +34,11 @@
 namespace mdcn {
 
 // Rows of either operand per workgroup tile of the two products: 256 (8
-// wavefronts, each 128 x 64) where both operands have that many rows, else 128
-// (4 wavefronts, each 64 x 64).  Per K step a 256-tile moves 64 KB for 2 048 MFMA
+// wavefronts, each 128 x 64, a workgroup a CU) or 128 (4 wavefronts, each 64 x 64,
+// two).  Per K step a 256-tile moves 64 KB for 2 048 MFMA
 // clocks, a 128-tile 32 KB for 512: with two K steps in flight the small tile is
-// bound by the latency of its copies, the large one is not.
+// bound by the latency of its copies, the large one is not.  Which of them a call has goes
+// by how full its rounds and how long its shares are (make_bwd_plan, with both sides measured).
 constexpr int kCgTile = 128;
 constexpr int kCgTileBig = 256;
 

@@ -103,6 +103,43 @@ def test_gradients_of_what_is_not_finite(cin, cout):
         assert float((a[small] - b[small]).norm() / b[small].norm()) <= 1e-5, name
 
 
+# Calls that run in tiles of 256: the column gradient of 9 x 113 and 8 x 96 tiles (three and four full rounds of the chip), the weight
+# gradient of 6 144 K steps (2 560 and more) with an uneven last tile of rows (9 x 224 = 7.875 x 256).
+LARGE = [(113, 256, 32), (96, 224, 256)]
+
+
+@pytest.mark.parametrize('n,cin,cout', LARGE, ids=['column', 'column_weight'])
+def test_gradients_in_tiles_of_256(n, cin, cout):
+    from common import capi_backward
+    print(f'n={n}', flush=True)
+    dev, gy = _backward_case(cin + 2, n, cin, cout, 16, 16)
+    got = capi_backward(dev, gy, path=capi.PATH_FUSED)
+    ref = capi_backward({k: v.double() if torch.is_tensor(v) else v for k, v in dev.items()}, gy.double())
+    for name, a, b in zip(('input', 'offset', 'mask', 'weight'), got, ref):   # (bounds: above)
+        terms = 256 * n if name == 'weight' else cout + 9 * cin
+        assert float((a.double() - b).norm() / b.norm()) <= terms ** 0.5 * 2.0 ** -24, name
+
+
+@pytest.mark.parametrize('n,cin,cout', LARGE, ids=['column', 'column_weight'])
+def test_tiles_of_256_of_what_is_not_finite(n, cin, cout):
+    """A workgroup whose sums are not finite makes its tile again: in the first tile, in the uneven last one, and nowhere else."""
+    from common import capi_backward
+    print(f'n={n}', flush=True)
+    dev, gy = _backward_case(cin + 3, n, cin, cout, 16, 16)
+    big = torch.finfo(torch.float32).max
+    dev['weight'] *= 1e-3
+    dev['input'][3, cin - 1, 6, 6] = float('inf')
+    gy[0, 3, 4, 5], gy[n - 1, 9, 12, 7], gy[n // 2, 11, 9, 9] = float('inf'), float('nan'), big
+    got = capi_backward(dev, gy, path=capi.PATH_FUSED)
+    ref = capi_backward(dev, gy, path=capi.PATH_DIRECT)
+    assert torch.equal(got[3].isnan(), ref[3].isnan()) and torch.equal(got[3].isinf(), ref[3].isinf())
+    for name, a, b in zip(('input', 'offset', 'mask', 'weight'), got, ref):
+        assert torch.equal(a.isfinite(), b.isfinite()), name
+        small = b.isfinite() & (b.abs() < 1e28)
+        assert 0 < int(small.sum()) < small.numel(), name
+        assert float((a[small] - b[small]).norm() / b[small].norm()) <= 1e-5, name
+
+
 @pytest.mark.parametrize('shape', ['fused', 'fused_cut', 'nhwc', 'segment', 'segment_shared'])
 def test_infinity_times_infinity(shape):
     """... is infinite, with the sign of the product, and so is a sum that only leaves fp32 at its end."""
