@@ -183,20 +183,19 @@ void make_bwd_plan(const mdcn_bwd_params *bp, const Geom &g, uint64_t pass_bytes
     }
   }
   if (pl->gemm) {
-    // Tiles of 256 for 16-bit calls that have more than two and a half rounds of them, and for fp32 calls of three rounds whose
-    // rounds are full: what they are filled with, in tiles of 128, is 7 in 8 (16 K steps or more) to 15 in 16 (8) or more.  Otherwise of 128, two workgroups
-    // a CU: the last round is fuller, one's products cover the other's barriers, and what fp32 splits behind its LDS reads costs it no more.
+    // Tiles of 256 for calls that have more than two and a half rounds of them, in fp32 if the rounds are full: what they are filled
+    // with, in tiles of 128, is 7 in 8 or more with 16 K steps and more, 15 in 16 with 8, 1 - steps / 128.  Otherwise of 128, two workgroups a CU: the last round is fuller, one's products cover the other's barriers, and what fp32 splits behind its LDS reads costs it no more.
     // Training calls in us, 256 / 128: fp32 N=2 256 channels 50x84 (306 tiles of 256) 404 / 380; N=1 512 25x42 (90) 284 / 260; N=8 512 13x21
     // 424 / 380; 256 channels, 8 K steps: filled to 0.87 (N=12 50x84) 1 790 / 1 765, 0.90 (N=8 64x64) 1 077 / 1 060, 0.93 (N=16 50x84) 2 300 / 2 283,
     // 0.93 (N=4 100x152) 2 028 / 2 011, 0.97 (N=6 100x152) 2 922 / 2 994, 1 (N=16 64x64) 2 014 / 2 020; 512 channels, 16: 0.75 (N=8 32x32) 915 / 891,
-    // 0.90 (N=16 32x32) 1 614 / 1 626, 0.90 (N=4 64x64) 1 630 / 1 647, 0.93 (N=8 50x84) 3 487 / 3 566, 0.95 (N=6 48x48) 1 596 / 1 625; bf16 N=4 96 -> 72
+    // 0.90 (N=16 32x32) 1 614 / 1 626, 0.94 (N=10 32x32, 720 tiles) 1 093 / 1 120, 0.90 (N=4 64x64) 1 630 / 1 647, 0.93 (N=8 50x84) 3 487 / 3 566, 0.95 (N=6 48x48) 1 596 / 1 625; bf16 N=4 96 -> 72
     // 37x53 (128 tiles) 113 / 110; N=4 240 60x60 (540) 336 / 331; N=8 104 -> 96 100x100 (1 280) 713 / 720; N=8 312 -> 300 90x100 (3 168) 2 092 / 2 133.
     auto tiles_of = [&](long tile) {
       return (long)pl->n_chunk * g.G * (((long)plane_out + tile - 1) / tile) * ((g.taps * im.cgp + tile - 1) / tile);
     };
     const long big_tiles = tiles_of(kCgTileBig), rounds = (big_tiles + 255) / 256, k_steps = om.cgp * (long)es / 128;
-    const bool full = big_tiles >= 768 && tiles_of(kCgTile) * 128 >= rounds * 4 * 256 * (128 - std::min<long>(16, k_steps));
-    pl->cg_tile = (g.taps * im.cgp >= kCgTileBig && plane_out >= (size_t)kCgTileBig && (es == 2 ? big_tiles > 640 : full)) ? kCgTileBig : kCgTile;
+    const bool full = tiles_of(kCgTile) * 128 >= rounds * 4 * 256 * (128 - std::min<long>(16, k_steps));
+    pl->cg_tile = (g.taps * im.cgp >= kCgTileBig && plane_out >= (size_t)kCgTileBig && big_tiles > 640 && (es == 2 || full)) ? kCgTileBig : kCgTile;
     pl->M_pad = pl->fused ? g.taps * im.cgp : padded(g.taps * im.cgp, pl->cg_tile);
     pl->gt_bytes = align_up((size_t)g.N * g.G * om.cgp * plane_out * es);
     pl->wt_bytes = align_up((size_t)g.G * pl->M_pad * om.cgp * es);

@@ -103,7 +103,7 @@ def test_gradients_of_what_is_not_finite(cin, cout):
         assert float((a[small] - b[small]).norm() / b[small].norm()) <= 1e-5, name
 
 
-# Calls that run in tiles of 256: the column gradient of 9 x 113 and 8 x 96 tiles (three and four full rounds of the chip), the weight
+# Calls that run in tiles of 256: the column gradient of 9 x 113 and 8 x 96 tiles (four and three rounds of the chip, full), the weight
 # gradient of 6 144 K steps (2 560 and more) with an uneven last tile of rows (9 x 224 = 7.875 x 256).
 LARGE = [(113, 256, 32), (96, 224, 256)]
 
