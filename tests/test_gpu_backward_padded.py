@@ -239,3 +239,15 @@ def test_large_products(dtype, n, h, w):
     for nm, r, o in zip(NAMES, ref, capi_backward(dev, gy)):
         err = float((o.double() - r).norm() / r.norm())
         assert err <= {torch.float32: 1e-5, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype], (nm, err)
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16], ids=['bf16', 'f16'])
+def test_large_products_of_uneven_rows(dtype):
+    """The same with rows of the products that fill the last tile of 256 to seven eighths (9 x 224): 5 760 K steps and 1 440 tiles."""
+    print(f'dtype={dtype}', flush=True)
+    dev = cast_case(make_case(59, N=5, Cin=224, Cout=200, H=92, W=100), dtype, 'cuda')
+    gy = torch.randn(5, 200, 92, 100, generator=torch.Generator().manual_seed(10)).to(dtype).cuda()
+    ref = capi_backward({k: v.double() if torch.is_tensor(v) else v for k, v in dev.items()}, gy.double())
+    for nm, r, o in zip(NAMES, ref, capi_backward(dev, gy)):
+        err = float((o.double() - r).norm() / r.norm())
+        assert err <= {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype], (nm, err)

@@ -72,7 +72,7 @@ def _backward_case(seed, n, cin, cout, h, w):
     return {k: v.cuda() if torch.is_tensor(v) else v for k, v in case.items()}, gy.cuda()
 
 
-@pytest.mark.parametrize('cin,cout', [(64, 64), (256, 200), (40, 256)], ids=['tile128', 'tile256', 'padded'])
+@pytest.mark.parametrize('cin,cout', [(64, 64), (256, 200), (40, 256)], ids=['narrow', 'wide', 'padded'])
 def test_gradients_are_fp32(cin, cout):
     from common import capi_backward
     dev, gy = _backward_case(cin, 2, cin, cout, 17, 21)
@@ -85,7 +85,7 @@ def test_gradients_are_fp32(cin, cout):
         assert float((a.double() - b).norm() / b.norm()) <= terms ** 0.5 * 2.0 ** -24, name
 
 
-@pytest.mark.parametrize('cin,cout', [(64, 64), (256, 256)], ids=['tile128', 'tile256'])
+@pytest.mark.parametrize('cin,cout', [(64, 64), (256, 256)], ids=['narrow', 'wide'])
 def test_gradients_of_what_is_not_finite(cin, cout):
     """An infinity, a NaN and the largest number in grad_output stay in the gradients they belong to."""
     from common import capi_backward
