@@ -78,9 +78,9 @@ __device__ __forceinline__ uint32_t wave_max(uint32_t v) {
 // be.  Where the largest |d * mask| of a sample gives three bits or more, the scale is from that instead: else one large gradient
 // under a small mask takes bits from its whole tile (fp16, one pixel of a mask of 0 and 1 000 times the gradient: error of grad_input
 // 3.3e-3 of its norm, so 2.1e-4, its one rounding).  Below three bits (inputs whose large gradients and open masks meet somewhere in a
-// tile) results stay those of the first scale, bit for bit.  The second costs N=16 256 channels 100x152 in bf16 0.6 % (2 247 -> 2 261 us).  (Bounds of |d| from norms of grad_output and weights instead: training calls of N=16 256 channels 100x152 in bf16 2 319
-// us where this takes 2 329, of N=8 512 channels 25x42 in fp16 371 / 363.  But such a scale goes by gradients that the weights do not
-// carry on: fp16, 256 output channels, one of them without weights and with 300 times the gradient: error of grad_input
+// tile) results stay those of the first scale, bit for bit.  The second costs training calls of N=16 256 channels 100x152 in bf16 0.3 %
+// (2 377 -> 2 383 us).  (Bounds of |d| from norms of grad_output and weights instead: 0.4 % less there, 2 % more for N=8 512 channels 25x42 in
+// fp16.  But such a scale goes by gradients that the weights do not carry on: fp16, 256 output channels, one of them without weights and with 300 times the gradient: error of grad_input
 // 8.6e-4 of its norm, where its one rounding is 2.1e-4 and this stays at that.)
 // What is added to an entry is the bit pattern of fmaf(weight, d, 1.5 * 2^23), for two channels at
 // once: every tap of every pixel adds to four entries, the same ones for all channels, so the number of adds an entry has
@@ -437,7 +437,8 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
     }
   };
   auto take_scale = [&]() {
-    // (the waves' eight words of either, a lane each, and the largest of eight lanes: sixteen reads at once are registers too many here)
+    // (the waves' eight words of either, a lane each, and the largest of eight lanes: sixteen reads at once are more registers than there
+    // are here)
     uint32_t bits = __float_as_uint(red[3 * kBfWaves + (lane & 15)]);
     bits = max(bits, (uint32_t)__builtin_amdgcn_mov_dpp((int)bits, 0xB1, 0xf, 0xf, true));    // of two
     bits = max(bits, (uint32_t)__builtin_amdgcn_mov_dpp((int)bits, 0x4E, 0xf, 0xf, true));    // of four
@@ -445,8 +446,9 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
     const float dmax = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)bits, 0));
     const float one = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)bits, 8));
     // exponent of a scale, from a bound of a sum and one of a contribution
-    auto exponent = [](float all, float one) {
-      return (all > 0.0f && all < 3.0e38f) ? min(29 - ilogbf(all), one > 0.0f ? 20 - ilogbf(one) : 120) : 0;
+    auto exponent = [](float all, float one) {   // (positive and finite where it counts: frexp's exponent is ilogb's + 1)
+      const int e = min(30 - __builtin_amdgcn_frexp_expf(all), one > 0.0f ? 21 - __builtin_amdgcn_frexp_expf(one) : 120);
+      return (all > 0.0f && all < 3.0e38f) ? e : 0;
     };
     const float mask_top = tops[0];
     const float apart = dmax * tops[1], all = one * tops[2];
