@@ -184,12 +184,16 @@ void make_bwd_plan(const mdcn_bwd_params *bp, const Geom &g, uint64_t pass_bytes
   }
   if (pl->gemm) {
     // Tiles of 256 for calls that have more than two and a half rounds of them, in fp32 if the rounds are full: what they are filled
-    // with, in tiles of 128, is 7 in 8 or more with 16 K steps and more, 15 in 16 with 8, 1 - steps / 128.  Otherwise of 128, two workgroups a CU: the last round is fuller, one's products cover the other's barriers, and what fp32 splits behind its LDS reads costs it no more.
-    // Training calls in us, 256 / 128: fp32 N=2 256 channels 50x84 (306 tiles of 256) 404 / 380; N=1 512 25x42 (90) 284 / 260; N=8 512 13x21
-    // 424 / 380; 256 channels, 8 K steps: filled to 0.87 (N=12 50x84) 1 790 / 1 765, 0.90 (N=8 64x64) 1 077 / 1 060, 0.93 (N=16 50x84) 2 300 / 2 283,
-    // 0.93 (N=4 100x152) 2 028 / 2 011, 0.97 (N=6 100x152) 2 922 / 2 994, 1 (N=16 64x64) 2 014 / 2 020; 512 channels, 16: 0.75 (N=8 32x32) 915 / 891,
-    // 0.90 (N=16 32x32) 1 614 / 1 626, 0.94 (N=10 32x32, 720 tiles) 1 093 / 1 120, 0.90 (N=4 64x64) 1 630 / 1 647, 0.93 (N=8 50x84) 3 487 / 3 566, 0.95 (N=6 48x48) 1 596 / 1 625; bf16 N=4 96 -> 72
-    // 37x53 (128 tiles) 113 / 110; N=4 240 60x60 (540) 336 / 331; N=8 104 -> 96 100x100 (1 280) 713 / 720; N=8 312 -> 300 90x100 (3 168) 2 092 / 2 133.
+    // with, in tiles of 128, is 7 in 8 or more with 16 K steps and more, 15 in 16 with 8, 1 - steps / 128.  Otherwise of 128, two
+    // workgroups a CU: the last round is fuller, one's products cover the other's barriers, and what fp32 splits behind its LDS reads costs
+    // it no more.  Training calls in us, 256 / 128:
+    // fp32 of few tiles of 256: N=2 256 channels 50x84 (306) 404 / 380; N=1 512 25x42 (90) 284 / 260; N=8 512 13x21 424 / 380;
+    // fp32 256 channels, 8 K steps, by how full: 0.87 (N=12 50x84) 1 790 / 1 765, 0.90 (N=8 64x64) 1 077 / 1 060, 0.93 (N=16 50x84) 2 300 /
+    // 2 283, 0.93 (N=4 100x152) 2 028 / 2 011, 0.97 (N=6 100x152) 2 922 / 2 994, 1 (N=16 64x64) 2 014 / 2 020;
+    // fp32 512 channels, 16: 0.75 (N=8 32x32) 915 / 891, 0.90 (N=16 32x32) 1 614 / 1 626, 0.94 (N=10 32x32, 720 tiles) 1 093 / 1 120, 0.90 (N=4
+    // 64x64) 1 630 / 1 647, 0.93 (N=8 50x84) 3 487 / 3 566, 0.95 (N=6 48x48) 1 596 / 1 625;
+    // 16 bits: N=4 96 -> 72 37x53 (128 tiles) 113 / 110; N=4 240 60x60 (540) 336 / 331; N=8 104 -> 96 100x100 (1 280) 713 / 720; N=8 312 -> 300
+    // 90x100 (3 168) 2 092 / 2 133.
     auto tiles_of = [&](long tile) {
       return (long)pl->n_chunk * g.G * (((long)plane_out + tile - 1) / tile) * ((g.taps * im.cgp + tile - 1) / tile);
     };
@@ -218,6 +222,7 @@ void make_bwd_plan(const mdcn_bwd_params *bp, const Geom &g, uint64_t pass_bytes
     // 16.7 (N=1 256 100x152) 587 / 589, 23.7 (N=3 256 72x100) 835 / 842; bf16 and fp16 steps of 0.4 (N=1 512 13x13) 108 / 101, 2.4 (N=1 512
     // 25x42) 132 / 121, 4.6 (N=2 256 50x84) 174 / 166, 9.3 (N=4) 272 / 260, 19.1 (N=8 512 25x42) 351 / 345, 22.8 (N=8 256 72x72) 508 / 507,
     // 25.1 (N=3 256 100x152) 525 / 537, 28.7 (N=12 512 25x42) 482 / 473, 33.5 (N=4 256 100x152) 637 / 653, 66.9 (N=8) 1 203 / 1 246.
+    // (28.7 goes the other way, why is not known; fp32 is even from 9 to 24.)
     const long big_steps = work * g.G * ((g.cout_g + kCgTileBig - 1) / kCgTileBig) * ((M + kCgTileBig - 1) / kCgTileBig);
     pl->w_tile = (g.cout_g >= 192 && M >= kCgTileBig && big_steps > 256L * (es == 4 ? 10 : 20)) ? kCgTileBig : kCgTile;
     const long tiles = (long)g.G * ((g.cout_g + pl->w_tile - 1) / pl->w_tile) * ((M + pl->w_tile - 1) / pl->w_tile);

@@ -92,9 +92,11 @@ __device__ __forceinline__ uint32_t wave_max(uint32_t v) {
 //
 // bf16, N=16, 256 -> 256 channels, 100x152: 1.29 ms for what took 0.52 (column gradient to memory) + 1.50 (scatter kernel reading
 // it); a pass takes a CU 40 thousand clocks: 25 scatter (VALU busy in 16, LDS adds 18), 6 products (MFMA 5), 7 flush, the rest
-// waits at the barriers.  fp16 without modulation, N=8, 512 -> 512 channels, 25x42: 0.17 ms.  (Whole training calls, us: 2 224 and
-// 348; 2 361 and 372 with grad_output loaded within branches and behind the scatter, the argument block kept as it was loaded,
-// 64-bit addresses in each lane and the largest of a pass found with integers, two instructions a value.)
+// waits at the barriers.  fp16 without modulation, N=8, 512 -> 512 channels, 25x42: 0.17 ms.  (Whole training calls with
+// grad_output loaded within branches and behind the scatter, the argument block kept as it was loaded, 64-bit addresses in each lane and the
+// largest of a pass found with integers, two instructions a value, took 0.4 to 4 % longer, by the card: on four of them, before / now, us,
+// 2 333 / 2 246, 2 349 / 2 261, 2 335 / 2 277, 2 414 / 2 386, and 397 / 364, 363 / 344.)
+// No scratch but with more than 256 output channels and 16 of the input's a pass: 20 (bf16) and 8 bytes (fp16), read at a tile's start.
 template <typename E, int CH, int RUN, bool DEEP>
 __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterWindow &wd, int b, int c_first, int c_last, float *part, uint4 *lds,
                                            float *red) {
@@ -217,9 +219,10 @@ __device__ __forceinline__ void fused_tile(const BwdFusedArgs &a, const ScatterW
 #pragma unroll
     for (int j = 0; j < 4; ++j) gf[4 * s + j] = *(const uint4 *)(p + j * 32 + at);
   };
-  // Whether a pass's first chunk has its second half loaded.  Passes of 8 channels leave it out with 64 output channels (N=4 64
-  // channels, 8 deformable groups, 120x160: 302 -> 286 us); with 16 the branch costs 44 reloads of spilled registers, and more than it saves
-  // (N=4 256 channels 50x84: 260 -> 269).
+  // Whether a pass's first chunk has its second half loaded.  Passes of 8 channels leave it out with 64 output channels (bf16 training calls,
+  // loaded / left out, us: N=4 64 channels, 8 deformable groups, 120x160 304 / 296, N=8 96x128 356 / 345).  The branch costs those of 128 output
+  // channels that take it and load all the same (N=4 128, 16 deformable groups, 120x160 610 / 620, 90x150 469 / 479); with 16 channels a pass
+  // it would be 44 reloads of spilled registers, more than it saves (N=4 256 channels 50x84: 260 / 269).
   auto first_second = [&]() { return CH == 16 || whole_chunk(0); };
   // the first two stages of a pass
   auto issue_first = [&](int c0) {

@@ -353,8 +353,8 @@ struct BwdScatterArgs {
   uint32_t far_min;
   int n0;          // first image of the pass
   // A deformable group's channels are shared among `parts` workgroups per tile
-  // (blockIdx.y), so that the launch has several times more workgroups than the
-  // chip has room for and its last round is short; with parts > 1 each writes its
+  // (blockIdx.y): up to 8 of them where that makes the last of many rounds short, up
+  // to 32 where tiles are few (scatter_parts); with parts > 1 each writes its
   // share of the offset / mask sums as floats to poff / pmask ([part][layout of
   // grad_offset / grad_mask]), which bwd_finish_kernel adds up.
   int parts;
