@@ -162,12 +162,16 @@ const char *mdcn_forward_kernels(const mdcn_params *p);
 /* Bytes of device scratch mdcn_forward() asks for (of the pointer fields only
  * `input` is looked at, see mdcn_fused_eligible()).  The fused path keeps a
  * zero-bordered channels-last copy of the input and the repacked weights there;
- * the direct path and MDCN_F64 need none.  Where the schedule of a launch ends in a
- * round that fills at most half of an XCD's workgroups (see no_k_split), the figure
- * ends with an optional region (one 128 x 256 fp32 tile and a counter per workgroup,
- * 32 MiB on a 256-CU device) through which the workgroups that would otherwise idle
- * share the K range of that round's tiles: a workspace that is smaller by that region
- * is accepted too and only runs that last round unshared.  Returns 0 for an invalid *p
+ * the direct path and MDCN_F64 need none.  The figure ends with up to two optional
+ * regions.  First, for fp32 calls that are made of fp16 pairs, their exponents and the
+ * sampling positions (2 bytes per input pixel and 32 channels, 4 bytes per group and
+ * 20 per deformable group and tap of an output pixel).  Second, where the schedule of
+ * a launch ends in a round that fills at most half of an XCD's workgroups (see
+ * no_k_split), one 128 x 256 fp32 tile and a counter per workgroup (32 MiB on a
+ * 256-CU device) through which the workgroups that would otherwise idle share the K
+ * range of that round's tiles.  A workspace that is smaller by the second or by both
+ * is accepted too: it runs that last round unshared, and makes fp32 products of
+ * bf16 triples, which is slower.  Returns 0 for an invalid *p
  * (mdcn_forward then reports the error). */
 size_t mdcn_workspace_bytes(const mdcn_params *p);
 
@@ -192,8 +196,8 @@ int mdcn_forward(const mdcn_params *p, void *hip_stream);
  * to a buffer of MDCN_NOALLOC_SCRATCH_BYTES that is part of the library's
  * device image (each device the library runs on holds one until the process
  * ends).  Calls whose mdcn_workspace_bytes() exceeds that size return
- * MDCN_ERR_SCRATCH_LIMIT and enqueue nothing (the optional region at the end
- * of the workspace is used when it fits as well and left out otherwise).  The call allocates and frees
+ * MDCN_ERR_SCRATCH_LIMIT and enqueue nothing (the optional regions at the end
+ * of the workspace are used when they fit as well and left out otherwise).  The call allocates and frees
  * nothing, on the host or on the device -- from the second call on a device on: the
  * first one asks the runtime for the buffer's address and the device's CU count, so
  * make one call outside a graph capture before capturing.  All calls on one device share the

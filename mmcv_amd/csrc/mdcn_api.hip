@@ -9,6 +9,7 @@
 #include <atomic>
 #include <cstdio>
 #include <mutex>
+#include <numeric>
 #include <type_traits>
 
 #include "mdcn_common.h"
@@ -21,6 +22,7 @@
 #include "mdcn_oconv.h"
 #include "mdcn_oconv_backward.h"
 #include "mdcn_host.h"
+#include "mdcn_pairs.h"
 #include "mdcn_prepass.h"
 #include "mdcn_segment.h"
 
@@ -154,6 +156,9 @@ struct Plan {
   int n_chunk;       // images per launch of the fused path
   size_t xt_bytes;   // channels-last copy of one chunk
   size_t wp_bytes;   // packed weights
+  // fp32 as fp16 pairs (may be left out: bf16 triples): magnitudes of the input's pixels, exponents of weights and of samples
+  size_t max_bytes, wexp_bytes, rexp_bytes, tpix_bytes;   // (four weights to an offset)
+  size_t pair_bytes() const { return max_bytes + wexp_bytes + rexp_bytes + 5 * tpix_bytes; }
   size_t cut_bytes;  // eight-wave kernel: buffers and counters of the tiles it cuts along K (may be left out)
   int cut_wgs;     // ... one buffer and one counter per workgroup of its grid
   bool seg;          // segment kernel: the shapes the fused kernels do not cover
@@ -277,9 +282,22 @@ bool small_call(const mdcn_params *p, const Geom &g, const Plan &fused, Plan *al
   const long waves = ((long)g.N * g.Ho * g.Wo + 31) / 32 * alt->sp.n_ctiles * g.G;
   if (waves > 3L * num_cus() || alt->xt_bytes + alt->wp_bytes > fused.xt_bytes + fused.wp_bytes) return false;
   alt->seg_small = true;
+  alt->max_bytes = alt->wexp_bytes = alt->rexp_bytes = alt->tpix_bytes = 0;
   alt->cut_bytes = 0;
   alt->cut_wgs = 0;
   return true;
+}
+
+// Products of fp16 pairs or of bf16 triples (mdcn_fused_f32.h): pairs cost a launch in front of the main kernel's, 4 to 5 us, and
+// save so much a K step of 256 channels that any schedule makes up for it, less with 128 and little with 64, whose steps the
+// gathers bound.  Whole call, us, triples / pairs.  256 channels a tile: 256 channels 50x84 N=2 (24 steps a workgroup) 94.9 / 69.3, 512 channels
+// 25x42 N=4 162.7 / 118.1; 128: 128 channels 64x64 N=2 (9) 36.7 / 35.8, 256 channels 50x84 (24) 55.5 / 50.5; 64: 256 channels 28x28
+// (8) 31.1 / 34.3, 64 channels 200x200 (22) 51.5 / 54.9, N=8 (176) 256 / 254.
+bool pairs_pay(const mdcn_params *p, const Geom &g, const Plan &pl) {
+  const int nk = pl.slabs * g.taps;
+  const long px_tiles = ((long)pl.n_chunk * g.Ho * g.Wo + kPT - 1) / kPT;
+  const double steps = schedule_rounds(px_tiles * pl.n_ctiles * g.G, nk, !p->no_k_split) * nk;
+  return steps >= (pl.CT == 256 ? 4 : pl.CT == 128 ? 9 : 140);
 }
 
 int make_plan(const mdcn_params *p, const Geom &g, Plan *pl, bool may_be_small = true) {
@@ -289,7 +307,7 @@ int make_plan(const mdcn_params *p, const Geom &g, Plan *pl, bool may_be_small =
   pl->fused = ok && p->path != MDCN_PATH_DIRECT && p->path != MDCN_PATH_SEGMENT;
   pl->seg = pl->seg_small = false;
   pl->CT = pl->KC = pl->n_ctiles = pl->slabs = pl->n_chunk = 0;
-  pl->xt_bytes = pl->wp_bytes = pl->owp_bytes = pl->raw_bytes = pl->cut_bytes = 0;
+  pl->xt_bytes = pl->wp_bytes = pl->owp_bytes = pl->raw_bytes = pl->cut_bytes = pl->max_bytes = pl->wexp_bytes = pl->rexp_bytes = pl->tpix_bytes = 0;
   pl->cut_wgs = 0;
   pl->CO = 3 * g.DG * g.taps;
   pl->CO_pad = (pl->CO + 31) / 32 * 32;
@@ -337,6 +355,12 @@ int make_plan(const mdcn_params *p, const Geom &g, Plan *pl, bool may_be_small =
   pl->xt_bytes = p->input_nhwc ? 0 : align_up((size_t)img * pl->n_chunk);
   // (fp32: three bf16 planes, 6 bytes an element)
   pl->wp_bytes = align_up((size_t)g.G * pl->n_ctiles * pl->slabs * g.taps * pl->CT * pl->KC * (es == 4 ? 6 : es));
+  if (p->dtype == MDCN_F32 && !p->input_nhwc && pairs_pay(p, g, *pl)) {
+    pl->max_bytes = align_up((size_t)pl->n_chunk * g.H * g.W * (g.Cin / pl->KC) * 2);
+    pl->wexp_bytes = align_up((size_t)g.G * pl->n_ctiles * pl->CT * 4);
+    pl->rexp_bytes = align_up((size_t)g.G * pl->n_chunk * g.Ho * g.Wo * 4);
+    pl->tpix_bytes = align_up((size_t)g.DG * g.taps * pl->n_chunk * g.Ho * g.Wo * 4);
+  }
   // Tiles of the 128-pixel kernels' last round are cut along K where workgroups would otherwise idle: one
   // 128 x 256 fp32 tile and a counter per workgroup of the persistent grid -- asked for only when a launch
   // of this call has such a round (the 256-pixel kernel never cuts; what it leaves to the 128-pixel one may)
@@ -394,7 +418,7 @@ int make_pack_plan(const mdcn_pack_params *pp, const Geom &g, Plan *pl) {
       if (pl->CO_pad > 128) {  // accumulator blocks of the conv_offset kernel
         if (forced_fused(p->path)) return MDCN_ERR_PATH;
         pl->fused = false;
-        pl->xt_bytes = pl->wp_bytes = pl->cut_bytes = 0;
+        pl->xt_bytes = pl->wp_bytes = pl->cut_bytes = pl->max_bytes = pl->wexp_bytes = pl->rexp_bytes = pl->tpix_bytes = 0;
         pl->cut_wgs = 0;
         plan_segments(p, g, pl);
       } else {
@@ -417,9 +441,11 @@ hipError_t launch_fused_ct(const FusedArgs &fa, bool unbordered, hipStream_t st)
   const dim3 grid(per_xcd * 8), block(kThreads);
   if constexpr (sizeof(E) == 4) {
     if (unbordered)
-      hipLaunchKernelGGL((fused_f32_kernel<CT, TMAX, MULTI_DG, true>), grid, block, 0, st, fa);
+      hipLaunchKernelGGL((fused_f32_kernel<CT, TMAX, MULTI_DG, true, 3>), grid, block, 0, st, fa);
+    else if (fa.row_exp)
+      hipLaunchKernelGGL((fused_f32_kernel<CT, TMAX, MULTI_DG, false, 2>), grid, block, 0, st, fa);
     else
-      hipLaunchKernelGGL((fused_f32_kernel<CT, TMAX, MULTI_DG, false>), grid, block, 0, st, fa);
+      hipLaunchKernelGGL((fused_f32_kernel<CT, TMAX, MULTI_DG, false, 3>), grid, block, 0, st, fa);
   } else {
     if (unbordered)
       hipLaunchKernelGGL((fused_kernel<E, CT, TMAX, MULTI_DG, true>), grid, block, 0, st, fa);
@@ -589,7 +615,22 @@ int run_typed(const mdcn_params *p, const Geom &g, const Plan &pl, hipStream_t s
     E *raw_pm = (E *)(ws + pl.xt_bytes + pl.wp_bytes + pl.owp_bytes);
     const bool own_oconv = px && px->offset_weight;
     const int cof = pl.CO_pad / 32;
-    float *cut_part = (float *)(ws + pl.xt_bytes + pl.wp_bytes + pl.owp_bytes + pl.raw_bytes);
+    unsigned char *opt = ws + pl.xt_bytes + pl.wp_bytes + pl.owp_bytes + pl.raw_bytes;
+    const bool pairs = pl.max_bytes != 0;
+    PairArgs pa{};
+    pa.w = (const float *)p->weight;
+    pa.wp = wp;
+    pa.row_max = (uint16_t *)opt;
+    pa.wexp = (int *)(opt + pl.max_bytes);
+    pa.row_exp = (int *)(opt + pl.max_bytes + pl.wexp_bytes);
+    pa.tab_pix = (uint32_t *)((unsigned char *)pa.row_exp + pl.rexp_bytes);
+    pa.tab_w = (float4 *)((unsigned char *)pa.tab_pix + pl.tpix_bytes);
+    pa.unit = std::max(1, std::gcd(g.cin_g, g.ch_per_dg) / pl.KC);
+    pa.CT = pl.CT;
+    pa.n_ctiles = pl.n_ctiles;
+    pa.slabs = pl.slabs;
+    pa.slabs_total = g.Cin / pl.KC;
+    float *cut_part = (float *)(opt + pl.pair_bytes());
     uint32_t *cut_cnt = (uint32_t *)((unsigned char *)cut_part + align_up((size_t)pl.cut_wgs * kPT * kF2CT * 4));
     if (!pl.cut_bytes) cut_part = nullptr, cut_cnt = nullptr;
 
@@ -620,13 +661,24 @@ int run_typed(const mdcn_params *p, const Geom &g, const Plan &pl, hipStream_t s
         const int n_pchunks = (gc.H * gc.W + 32 * EPV - 1) / (32 * EPV);
         const long blocks = (long)gc.N * (gc.Cin / pl.KC) * n_pchunks;
         tic();
-        if (!packed) {
-          const int pack_blocks = (int)std::max<long>(1, std::min<long>(wtotal / (256 * 8), 512));
-          OffsetPack op = {nullptr, nullptr, 0, 1, 0, 0};
-          if (own_oconv) {
-            const long chunks = (long)(g.Cin / pl.KC) * g.taps * 4 * cof * 64;
-            op = OffsetPack{px->offset_weight, owp, pl.CO, cof, chunks, (int)std::min<long>((chunks + 255) / 256, 512)};
+        OffsetPack op = {nullptr, nullptr, 0, 1, 0, 0};
+        if (!packed && own_oconv) {
+          const long chunks = (long)(g.Cin / pl.KC) * g.taps * 4 * cof * 64;
+          op = OffsetPack{px->offset_weight, owp, pl.CO, cof, chunks, (int)std::min<long>((chunks + 255) / 256, 512)};
+        }
+        if constexpr (sizeof(E) == 4) {
+          if (pairs) {
+            pa.g = gc;
+            pa.zero_ptr = cut_cnt;
+            pa.zero_n = packed ? 0 : pl.cut_wgs;
+            const int wmax_blocks = packed ? 0 : pair_col_groups(g, pl.n_ctiles, pl.CT);
+            hipLaunchKernelGGL(pair_relayout_kernel, dim3((unsigned)(blocks + wmax_blocks + op.blocks)), dim3(256), 0, st, pa,
+                               in, xt, n_pchunks, wmax_blocks, op);
           }
+        }
+        if (pairs) {
+        } else if (!packed) {
+          const int pack_blocks = (int)std::max<long>(1, std::min<long>(wtotal / (256 * 8), 512));
           hipLaunchKernelGGL(prepass_kernel<E>, dim3((unsigned)(blocks + pack_blocks + op.blocks)), dim3(256), 0, st, gc,
                              in, xt, n_pchunks, g, (const E *)p->weight, wp, pl.CT, pl.KC, pl.n_ctiles, pl.slabs, wtotal,
                              pack_blocks, cut_cnt, pl.cut_wgs, op);
@@ -643,6 +695,10 @@ int run_typed(const mdcn_params *p, const Geom &g, const Plan &pl, hipStream_t s
       fa.xt = nhwc ? (const void *)in : (const void *)xt;
       fa.wp = wp;
       fa.in = in;
+      fa.row_exp = pairs ? pa.row_exp : nullptr;
+      fa.wexp = pa.wexp;
+      fa.tab_pix = pa.tab_pix;
+      fa.tab_w = pa.tab_w;
       fa.weight = p->weight;
       fa.in_c = nhwc ? 1 : (long)g.H * g.W;
       fa.in_px = nhwc ? g.Cin : 1;
@@ -708,6 +764,21 @@ int run_typed(const mdcn_params *p, const Geom &g, const Plan &pl, hipStream_t s
       fa.plane_px = g.Hp * g.Wp;
       fa.out_vec_ok = (plane_out % (long)(16 / es) == 0) && (((uintptr_t)fa.out % 16) == 0);
       fa.px0 = 0;
+      if constexpr (sizeof(E) == 4) {
+        if (pairs && rc == MDCN_OK) {
+          tic();
+          pa.g = gc;
+          pa.om = fa.om;
+          pa.img_bytes = fa.img_bytes;
+          pa.row_bytes = fa.row_bytes;
+          const int pack_blocks = packed ? 0 : pair_col_groups(g, pl.n_ctiles, pl.CT) * pl.slabs;
+          const int sample_blocks = g.G * (int)((fa.total_px + 63) / 64);
+          hipLaunchKernelGGL(pair_exponent_kernel, dim3((unsigned)(sample_blocks + pack_blocks)), dim3(256), 0, st, pa, sample_blocks);
+          packed = true;
+          if (hipGetLastError() != hipSuccess) rc = MDCN_ERR_LAUNCH;
+          toc(0);
+        }
+      }
       tic();
       const bool eight_wave = uses_fused2(p, g, pl);
       bool rest = true;
@@ -792,7 +863,8 @@ int run(const mdcn_params *p, void *stream, float *ms, const mdcn_pack_params *p
   if (need > 0 && (!p->workspace || p->workspace_bytes < need ||
                    ((uintptr_t)p->workspace % kAlign) != 0))
     return MDCN_ERR_WORKSPACE;
-  if (p->workspace_bytes < need + pl.cut_bytes) pl.cut_bytes = 0, pl.cut_wgs = 0;
+  if (p->workspace_bytes < need + pl.pair_bytes()) pl.max_bytes = pl.wexp_bytes = pl.rexp_bytes = pl.tpix_bytes = 0;
+  if (p->workspace_bytes < need + pl.pair_bytes() + pl.cut_bytes) pl.cut_bytes = 0, pl.cut_wgs = 0;
   hipStream_t st = (hipStream_t)stream;
   switch (p->dtype) {
     case MDCN_F32: return run_typed<float>(p, g, pl, st, ms, px);
@@ -903,7 +975,7 @@ size_t mdcn_workspace_bytes(const mdcn_params *p) {
   if (check_params(p, &g, false) != MDCN_OK) return 0;
   Plan pl;
   if (make_plan(p, g, &pl) != MDCN_OK) return 0;
-  return pl.seg && !pl.seg_small ? 0 : pl.xt_bytes + pl.wp_bytes + pl.cut_bytes;
+  return pl.seg && !pl.seg_small ? 0 : pl.xt_bytes + pl.wp_bytes + pl.pair_bytes() + pl.cut_bytes;
 }
 
 size_t mdcn_workspace_wanted(const mdcn_params *p) {
@@ -911,7 +983,7 @@ size_t mdcn_workspace_wanted(const mdcn_params *p) {
   if (check_params(p, &g, false) != MDCN_OK) return 0;
   Plan pl;
   if (make_plan(p, g, &pl) != MDCN_OK) return 0;
-  return pl.xt_bytes + pl.wp_bytes + pl.cut_bytes;
+  return pl.xt_bytes + pl.wp_bytes + pl.pair_bytes() + pl.cut_bytes;
 }
 
 int mdcn_forward(const mdcn_params *p, void *hip_stream) {
@@ -950,7 +1022,7 @@ size_t mdcn_pack_workspace_bytes(const mdcn_pack_params *pp) {
   if (!pp || check_params(&pp->conv, &g, false) != MDCN_OK) return 0;
   Plan pl;
   if (make_pack_plan(pp, g, &pl) != MDCN_OK) return 0;
-  return pl.xt_bytes + pl.wp_bytes + pl.owp_bytes + pl.raw_bytes + pl.cut_bytes;
+  return pl.xt_bytes + pl.wp_bytes + pl.owp_bytes + pl.raw_bytes + pl.pair_bytes() + pl.cut_bytes;
 }
 
 int mdcn_pack_forward(const mdcn_pack_params *pp, void *hip_stream) {

@@ -88,6 +88,11 @@ struct FusedArgs {
   const void *in, *weight;
   long in_c;
   int in_px;
+  // ... with fp16 pairs (else null): the exponents of the rows of samples, [group][pixel of the launch], and of the output
+  // channels' weights, [group][n_ctiles * CT]
+  const int *row_exp, *wexp;
+  const uint32_t *tab_pix;  // ... and what their tables hold, [deformable group, tap][pixel of the launch]
+  const float4 *tab_w;
   // fused2_kernel only: first pixel of its tiles (a multiple of 256; the pixels in front of it belong to
   // fused3_kernel, which is launched beside it); n_ptiles counts the tiles from there on
   int px0;

@@ -1,16 +1,23 @@
-// fp32 forward: the implicit GEMM of mdcn_fused.h, its products on the bf16
+// fp32 forward: the implicit GEMM of mdcn_fused.h, its products on the 16-bit
 // matrix pipe.
 //
-// The fp32 MFMA (32x32x2) runs at a sixteenth of the bf16 rate, and an fp32 tile
-// was bound by it.  An fp32 number is the sum of three bf16 numbers exactly:
-// h = bf16(x), m = bf16(x - h), l = x - h - m, 8 mantissa bits each (both differences
-// are exact).  A product of two such sums has nine terms, each exact in fp32; the
-// kernel accumulates six of them in fp32 -- hh, hm, mh, mm, hl, lh -- and leaves
-// out ml, lm and ll.  |m| <= 2^-8 |x| and |l| <= 2^-17 |x|, so that these are at most
-// (2^-24 + 2^-34) of the product together, as much as an fp32 multiplication may round by.  What
-// a sum of many terms loses it loses for the most part where it is added up, and a bf16 MFMA adds sixteen terms at a time, an
-// fp32 one two.  Against float64, with positions that fp32 holds exactly, the relative error (2-norm) is 3.7e-7 for 2 304 terms and 5.1e-7 for 4 608; with fp32 MFMAs it was 4.3e-7 and 5.9e-7.  Six bf16
-// MFMAs of K = 16 take 192 clocks where eight fp32 ones take 512.
+// The fp32 MFMA (32x32x2) runs at a sixteenth of the 16-bit rate, and an fp32 tile
+// was bound by it.  Two ways to make an fp32 product of 16-bit ones:
+//
+// Pairs (PLANES = 2).  h = fp16(x), l = fp16(x - h): what is left of x is at most 2^-23 |x|, half of that for most.  Three products,
+// hl, lh and hh, are summed in fp32; ll, at most 2^-22 of the product and a ninth of it on average, is left out.  fp16 has
+// few exponents, so rows are scaled by powers of two: an output channel's weights by the largest of them, an output pixel's samples by the
+// largest there can be, from the magnitudes of the input pixels its corners lie on (mdcn_pairs.h); sums are scaled back at the end.  A number
+// keeps its 22 bits down to 2^-17 of the largest of its row, below that what lies above 2^-40 of it.
+// Triples (PLANES = 3), for calls that pairs do not pay for (pairs_pay), channels-last input, and workspaces without room for the exponents.
+// An fp32 number is the sum of three bf16 numbers exactly: h = bf16(x), m = bf16(x - h), l = x - h - m, 8 mantissa bits each
+// (both differences are exact).  Six of nine products are summed -- hh, hm, mh, mm, hl, lh; |m| <= 2^-8 |x| and |l| <= 2^-17 |x|, so that ml, lm
+// and ll are at most (2^-24 + 2^-34) of the product together, as much as an fp32 multiplication may round by.
+//
+// What a sum of many terms loses it loses for the most part where it is added up: an MFMA adds sixteen terms at a time, and pairs have half as many of
+// them.  Against float64, with positions that fp32 holds exactly, the relative error (2-norm) is 2.8e-7 (pairs) and 3.6e-7 (triples)
+// for 2 304 terms, 3.2e-7 and 4.2e-7 for 4 608; with fp32 MFMAs it was 4.3e-7 and 5.9e-7.  Channels whose magnitudes span six decades, the
+// weights the same the other way round: 7.0e-7 / 3.6e-7.  For K = 16 six bf16 MFMAs take 192 clocks, three fp16 ones 96, eight fp32 ones 512.
 //
 // Roles, tables, schedule, cut tiles and epilogue are those of fused_kernel.  What
 // differs: a K step (32 channels of a tap) is two half steps of 16 channels; sample and
@@ -20,14 +27,15 @@
 // the weights; the consumer waves lie along the channels, so that each weight fragment has one
 // reader, which loads it from L2 into registers.
 //
-// What bounds it (N=8 256 -> 256 64x64, counters): the MFMA pipe, busy in 41 % of the cycles -- a K step of a 128 x 256
-// tile is 3 072 clocks of MFMAs per SIMD and takes 7 500; a large product of the library reaches 43 % of the pipe's peak.  The other
-// VALU instructions (the blend and the split for the most part) are 12 % of the cycles, the address unit of the vector-memory path is
-// busy in 30 %, and waves wait in a quarter of theirs.  Measured, main kernel, N=8 256 -> 256 64x64: 325 us
-// with fp32 MFMAs, 213 us (MFMAs alone: 116); N=2 50x84, 128-channel tiles: 144 -> 108 us.  Tried and
-// not faster: weights through LDS (213), fp32 tiles' producers at a higher or lower wave priority (209 - 224),
-// two gather sets (209).
+// What bounds it (N=8 256 -> 256 64x64, pairs, clocks in the kernel): a K step of a 128 x 256 tile takes 2 650 at the 1.8 GHz that the card runs it at.
+// The consumers' half is 2 050 of them, 1 536 MFMAs; the producers' 2 480, and the barrier waits for them: 150 VALU instructions, which make no progress while
+// MFMAs are issued on their SIMD, between gathers.  Main kernel, us: 325 with fp32 MFMAs, 213 triples, 131 pairs (MFMAs alone: 58); whole call
+// 230 -> 148.  N=2 50x84, whole call: 103 -> 69.  Without weights' loads, gathers, MFMAs (each alone, at 146): 132, 120, 128.
+// Tried and not faster: weights through LDS, producers at a higher or lower wave priority (triples), weights' loads a half step
+// earlier (pairs, 152 against 149).
 #pragma once
+
+#include <type_traits>
 
 #include "mdcn_direct.h"
 #include "mdcn_fused.h"
@@ -35,20 +43,25 @@
 namespace mdcn {
 
 constexpr int kF32Planes = 3;
+// ... or two fp16 planes (see the head of the file): fp16 pairs are scaled row by row so that the largest number there can be
+// in a row of either operand lies in [2^14, 2^15).
+constexpr int kPairTop = 14;
 // Both operands are multiplied by this before they are split, and the sums by its inverse squared: the third plane holds bits
 // down to 2^-23 of a number, and bf16, with the exponents of fp32, ends at 2^-126.  Unscaled, numbers below 2^-103 lose
 // some of their bits (2e-6 of a number of 2^-115, 2e-3 at 2^-125); scaled, the smallest normal number has
 // all of its 24.  In exchange numbers from 2^104 and sums from 2^80 on overflow, and are made again.
 constexpr float kSplitScale = 16777216.0f;
 constexpr float kSplitUnscale = 1.0f / (kSplitScale * kSplitScale);
-// K steps a gather is in flight: one register set, refilled behind its use, so that every load has a whole step
+// K steps a gather is in flight, bf16 triples: one register set, refilled behind its use, so that every load has a whole step
 // (some 3 000 clocks) to land.  (With two sets the compiler copies them into each other at the loop's
 // end and waits for all of their loads to do so.)
 constexpr int kF32Ahead = 1;
+// ... fp16 pairs, whose steps are shorter: two sets, taken in turn by a loop of two steps.
+constexpr int kPairAhead = 2;
 // Sample tiles: one being read, one ready, so that the consumers fetch their first fragments of a step ahead of the
 // barrier that ends the one before, and one being written.
 constexpr int kF32Tiles = 3;
-// LDS of one workgroup: sample tiles, table.
+// LDS of one workgroup (three planes; of two it is less): sample tiles, table.
 constexpr size_t fused_f32_lds_bytes(int tmax) {
   return (size_t)kF32Tiles * kPT * 192 + (size_t)kPT * tmax * 20 + 16;
 }
@@ -72,6 +85,37 @@ __device__ __forceinline__ void split3(const float (&x)[4], uint2 (&p)[3]) {
       r[3] -= __uint_as_float(hi & 0xffff0000u);
     }
   }
+}
+
+// Four floats, scaled already, as an fp16 number and the fp16 number nearest to what that leaves.  An infinity, and what is beyond
+// fp16, leaves NaN or an infinity.
+__device__ __forceinline__ void split2(const float (&x)[4], uint2 (&p)[2]) {
+  f16x2 h[2], l[2];
+  float minus = -1.0f;
+  asm("" : "+s"(minus));     // (... and makes two instructions of the mixed multiply-add below)
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    uint32_t hw = __builtin_bit_cast(uint32_t, f16x2{(f16_t)x[2 * i], (f16_t)x[2 * i + 1]});
+    asm("" : "+v"(hw));  // (or the compiler converts each number a second time)
+    h[i] = __builtin_bit_cast(f16x2, hw);
+    l[i] = f16x2{(f16_t)fmaf((float)h[i].x, minus, x[2 * i]), (f16_t)fmaf((float)h[i].y, minus, x[2 * i + 1])};
+  }
+  p[0] = make_uint2(__builtin_bit_cast(uint32_t, h[0]), __builtin_bit_cast(uint32_t, h[1]));
+  p[1] = make_uint2(__builtin_bit_cast(uint32_t, l[0]), __builtin_bit_cast(uint32_t, l[1]));
+}
+
+// The power of two that takes `top`, the largest magnitude of a row, to [2^kPairTop, 2^(kPairTop + 1)); 0 for a row of zeros and
+// for one that is not finite.
+__device__ __forceinline__ int pair_exponent(float top) {
+  const int e = (int)(__float_as_uint(top) >> 23) & 0xff;
+  return top == 0.0f || e == 0xff ? 0 : kPairTop + 127 - e;   // (a subnormal number: as if it were normal)
+}
+
+// ... of a row of samples, whose corner weights take it: `most` is the largest magnitude of a mask value, and no product
+// of the two overflows.  -113 .. 127.
+__device__ __forceinline__ int sample_exponent(float top, float most) {
+  const int em = (int)(__float_as_uint(most) >> 23) & 0xff;
+  return min(pair_exponent(top), min(127, 126 + 127 - em));
 }
 
 // weight[Cout][Cin/G][kh][kw] -> wp[G][n_ctiles][nk][2 half steps][3 planes][CT / 32][64 lanes][8 bf16]: A
@@ -156,12 +200,12 @@ __device__ __forceinline__ void pack_weight_split(const Geom &g, const float *__
 
 // The outputs of consumer wave `wave` in the first `units` units of its workgroup's schedule that are not finite, from the
 // call's own tensors.
-template <int CT, int WC, int MB, int NB>
+template <int CT, int WC, int MB, int NB, int AHEAD>
 __device__ __forceinline__ void remake_not_finite(const FusedArgs &a, int units, int nk_tile_pad, int wave, int lane) {
   const Geom &g = a.g;
   const int plane_out = g.Ho * g.Wo;
   UnitSchedule us;
-  us.init(a.n_ptiles * a.n_ctiles * g.G, nk_tile_pad, kF32Ahead, 8 / kF32Ahead, a.cut_max);
+  us.init(a.n_ptiles * a.n_ctiles * g.G, nk_tile_pad, AHEAD, 8 / AHEAD, a.cut_max);
 #pragma unroll 1
   for (int u = 0; u < units; ++u) {
     int L = us.tile_of(u);
@@ -185,12 +229,14 @@ __device__ __forceinline__ void remake_not_finite(const FusedArgs &a, int units,
   }
 }
 
-// MULTI_DG, UNBORDERED: as in fused_kernel.
-template <int CT, int TMAX, bool MULTI_DG, bool UNBORDERED>
+// MULTI_DG, UNBORDERED: as in fused_kernel.  PLANES: bf16 triples or fp16 pairs.
+template <int CT, int TMAX, bool MULTI_DG, bool UNBORDERED, int PLANES>
 __global__ __launch_bounds__(kThreads, 2) void fused_f32_kernel(FusedArgs a) {
   using E = float;
   using TR = ElemTraits<E>;
-  using TB = ElemTraits<bf16_t>;
+  constexpr bool kPairs = PLANES == 2;
+  constexpr int AHEAD = kPairs ? kPairAhead : kF32Ahead;
+  using TB = ElemTraits<std::conditional_t<kPairs, f16_t, bf16_t>>;
   constexpr int PT = kPT;
   constexpr int KC = TR::KC;
   constexpr int ES = (int)sizeof(E);
@@ -199,18 +245,19 @@ __global__ __launch_bounds__(kThreads, 2) void fused_f32_kernel(FusedArgs a) {
   constexpr int WC = CT / 32 < 4 ? CT / 32 : 4;
   constexpr int MB = CT / 32 / WC;
   constexpr int NB = WC;   // (4 / (4 / WC))
-  constexpr int WBLK = kF32Planes * CT / 32;    // 1 KiB fragments of a half-step weight tile
+  constexpr int WBLK = PLANES * CT / 32;    // 1 KiB fragments of a half-step weight tile
   constexpr int TPT = (TMAX + kTapGroups - 1) / kTapGroups;  // table entries per producer lane
-  constexpr int XFRAG = kF32Planes * (PT / 32) * 64;      // 16-byte pieces of a half step of a sample tile
+  constexpr int XFRAG = PLANES * (PT / 32) * 64;      // 16-byte pieces of a half step of a sample tile
   __shared__ uint4 Xs[kF32Tiles][2 * XFRAG];              // sample tiles
   __shared__ uint32_t tpix[PT * TMAX];                    // (pixel, tap) table, [tap][PT]: corner byte offset
   __shared__ uint4 tws[PT * TMAX];                        // ... and the four weights
   __shared__ uint32_t part_arrived;                       // parts of a cut tile that were there before this one
+  __shared__ __align__(16) int row_exp[kPairs ? PT : 4];  // pairs: exponents of the tile's pixels
 
   const Geom &g = a.g;
   const int taps = g.taps;
   const int nk_tile = a.slabs * taps;
-  const int nk_tile_pad = (nk_tile + kF32Ahead - 1) / kF32Ahead * kF32Ahead;
+  const int nk_tile_pad = (nk_tile + AHEAD - 1) / AHEAD * AHEAD;
   const int plane_out = g.Ho * g.Wo;
   const int total_px = (int)a.total_px;
   const int spd = g.ch_per_dg / KC;  // slabs per deformable group
@@ -225,7 +272,7 @@ __global__ __launch_bounds__(kThreads, 2) void fused_f32_kernel(FusedArgs a) {
   // neighbouring tiles share stay in its L2.  Tiles of the run's last round are
   // cut along K (UnitSchedule): parts of at least 8 steps.
   UnitSchedule us;
-  us.init(a.n_ptiles * a.n_ctiles * g.G, nk_tile_pad, kF32Ahead, 8 / kF32Ahead, a.cut_max);
+  us.init(a.n_ptiles * a.n_ctiles * g.G, nk_tile_pad, AHEAD, 8 / AHEAD, a.cut_max);
 
   bool bad = false;    // consumer waves: a sum of a stored tile was not finite
   int units = us.T;    // ... how many of the units they have stored: all, or all but a part of a cut tile
@@ -267,7 +314,36 @@ __global__ __launch_bounds__(kThreads, 2) void fused_f32_kernel(FusedArgs a) {
         tb_ho = tb_rem / g.Wo;
         tb_wo = tb_rem - tb_ho * g.Wo;
       }
+      // what takes the lane's pixel to fp16's range (a row of a padded pixel holds zeros)
+      float scale = kSplitScale;
+      if constexpr (kPairs) {
+        const int e = a.row_exp[(long)grp * total_px + min(tb_p, total_px - 1)];
+        scale = __uint_as_float((uint32_t)(e + 127) << 23);
+        if (ptid < PT) row_exp[tb_pl] = e;
+      }
       auto build_table = [&](int dgi) {
+        if constexpr (kPairs) {   // made by pair_exponent_kernel; scaled here
+          const long at = (long)(dgi * taps) * total_px + min(tb_p, total_px - 1);
+          uint32_t pix[TPT];
+          float4 w[TPT];
+#pragma unroll
+          for (int i = 0; i < TPT; ++i) {
+            const long e = at + (long)min((ptid >> 7) + kTapGroups * i, taps - 1) * total_px;
+            pix[i] = a.tab_pix[e];
+            w[i] = a.tab_w[e];
+          }
+          const float s = tb_valid ? scale : 0.0f;
+#pragma unroll
+          for (int i = 0; i < TPT; ++i) {
+            const int tap = (ptid >> 7) + kTapGroups * i;
+            if (tap < taps) {
+              tpix[tap * PT + tb_pl] = pix[i];
+              tws[tap * PT + tb_pl] = make_uint4(__float_as_uint(w[i].x * s), __float_as_uint(w[i].y * s), __float_as_uint(w[i].z * s),
+                                                 __float_as_uint(w[i].w * s));
+            }
+          }
+          return;
+        }
         // (an invalid pixel reads the entries of pixel 0 of image 0 and stores zeros)
         const E *off = (const E *)a.om.off + (long)tb_n * a.om.off_n + (long)tb_rem * a.om.off_px +
                        (long)(dgi * 2 * taps) * a.om.off_ch;
@@ -289,7 +365,7 @@ __global__ __launch_bounds__(kThreads, 2) void fused_f32_kernel(FusedArgs a) {
             const int ti = tap / g.kw, tj = tap - ti * g.kw;
             TapSample sm =
                 make_tap_sample(tb_ho * g.sh - g.ph + ti * g.dh, tb_wo * g.sw - g.pw + tj * g.dw,
-                                to_f32(rdy[i]), to_f32(rdx[i]), mask_value<E>(rm[i], a.om.logit) * kSplitScale, g.H, g.W);
+                                to_f32(rdy[i]), to_f32(rdx[i]), mask_value<E>(rm[i], a.om.logit) * scale, g.H, g.W);
             // byte offset of the upper left corner, slab 0 of image tb_n
             uint32_t pix = (uint32_t)tb_n * a.img_bytes + corner_offset<UNBORDERED>(sm, g, a);
             uint32_t tw[4];
@@ -304,11 +380,10 @@ __global__ __launch_bounds__(kThreads, 2) void fused_f32_kernel(FusedArgs a) {
         }
       };
 
-      // -- gather state: kF32Ahead register sets, set m % kF32Ahead holds step m;
+      // -- gather state: AHEAD register sets, set m % AHEAD holds step m;
       //    [pixel][corner][half of the lane's 32 bytes]
-      uint4 gv[kF32Ahead][kPxPerLane][4][2];
-      uint4 gw[kF32Ahead][kPxPerLane];
-
+      uint4 gv[AHEAD][kPxPerLane][4][2];
+      uint4 gw[AHEAD][kPxPerLane];
       // Gather of the cursor's step (rebuilding the table first when the step
       // opens a new deformable group), then move the cursor on.
       auto issue_gather = [&](uint4 (&v)[kPxPerLane][4][2], uint4 (&w)[kPxPerLane]) {
@@ -375,11 +450,13 @@ __global__ __launch_bounds__(kThreads, 2) void fused_f32_kernel(FusedArgs a) {
             v[h][3][half] = *(const uint4 *)(bot + pxb);
             __builtin_amdgcn_sched_barrier(0);
             // channels 4 q .. 4 q + 3 of half step `half`: 8 bytes of the fragments of lane half q >> 1
-            uint2 pl[3];
-            split3({__uint_as_float(s.x), __uint_as_float(s.y), __uint_as_float(s.z), __uint_as_float(s.w)}, pl);
+            uint2 pl[PLANES];
+            const float sv[4] = {__uint_as_float(s.x), __uint_as_float(s.y), __uint_as_float(s.z), __uint_as_float(s.w)};
+            if constexpr (kPairs) split2(sv, pl);
+            else split3(sv, pl);
             uint2 *dst = (uint2 *)&Xs[buf][half * XFRAG + (row >> 5) * 64 + (q >> 1) * 32 + (row & 31)] + (q & 1);
 #pragma unroll
-            for (int p = 0; p < kF32Planes; ++p) dst[p * (PT / 32) * 64 * 2] = pl[p];
+            for (int p = 0; p < PLANES; ++p) dst[p * (PT / 32) * 64 * 2] = pl[p];
           }
           w[h] = wn[h];
         }
@@ -390,17 +467,20 @@ __global__ __launch_bounds__(kThreads, 2) void fused_f32_kernel(FusedArgs a) {
       MDCN_BARRIER_LDS();  // B0: table visible
 
 #pragma unroll
-      for (int j = 0; j < kF32Ahead; ++j) issue_gather(gv[j], gw[j]);
+      for (int j = 0; j < AHEAD; ++j) issue_gather(gv[j], gw[j]);
       commit_and_refill(0, gv[0], gw[0]);
-      commit_and_refill(1, gv[0], gw[0]);
+      commit_and_refill(1, gv[AHEAD - 1], gw[AHEAD - 1]);
       MDCN_BARRIER_LDS();  // B1: X[0], X[1] visible
 
       // (steps past nk repeat the last one and nobody reads what they produce)
       int wt = 2;
-      for (int ks = 0; ks < nk; ++ks) {
-        commit_and_refill(wt, gv[0], gw[0]);
-        wt = wt == kF32Tiles - 1 ? 0 : wt + 1;
-        MDCN_BARRIER_LDS();  // end of step ks: X[ks+2] visible
+      for (int ks = 0; ks < nk_pad; ks += AHEAD) {
+#pragma unroll
+        for (int j = 0; j < AHEAD; ++j) {
+          commit_and_refill(wt, gv[j], gw[j]);
+          wt = wt == kF32Tiles - 1 ? 0 : wt + 1;
+          MDCN_BARRIER_LDS();  // end of step ks + j: X[ks+j+2] visible
+        }
       }
       // The gathers issued past the last step are never read.  Retire them with a
       // wait the compiler can see: it tracks these loads' destination registers,
@@ -428,6 +508,10 @@ __global__ __launch_bounds__(kThreads, 2) void fused_f32_kernel(FusedArgs a) {
 
       const int frow = lane & 31;
       const int fhalf = lane >> 5;
+      int wexp[MB];   // pairs: exponents of this lane's output channels
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
+        wexp[mb] = kPairs ? ((const int *)a.wexp)[(grp * a.n_ctiles + ctile) * CT + (wave_c * MB + mb) * 32 + frow] : 0;
       // bias of this lane's output channels, fetched now so that the epilogue
       // never waits on a load (a wait there would also wait for its own stores)
       float bv[MB];
@@ -451,31 +535,31 @@ __global__ __launch_bounds__(kThreads, 2) void fused_f32_kernel(FusedArgs a) {
       const uint4 *wp_tile = (const uint4 *)a.wp +
                              ((size_t)(grp * a.n_ctiles + ctile) * nk_tile + kb) * (size_t)(2 * WBLK * 64) +
                              wave_c * MB * 64 + lane;
-      uint4 wf[2][kF32Planes][MB];
-      auto load_weights = [&](int hs, uint4 (&w)[kF32Planes][MB]) {
+      uint4 wf[2][PLANES][MB];
+      auto load_weights = [&](int hs, uint4 (&w)[PLANES][MB]) {
         const uint4 *src = wp_tile + (size_t)min(hs, 2 * nk - 1) * (WBLK * 64);  // (past the end: never used)
 #pragma unroll
-        for (int p = 0; p < kF32Planes; ++p)
+        for (int p = 0; p < PLANES; ++p)
 #pragma unroll
           for (int mb = 0; mb < MB; ++mb) w[p][mb] = src[(p * (CT / 32) + mb) * 64];
       };
       load_weights(0, wf[0]);
       MDCN_BARRIER_LDS();  // B0
 #pragma unroll
-      for (int v = 0; v < kF32Ahead + 2; ++v) mirror_issue();
+      for (int v = 0; v < AHEAD + 2; ++v) mirror_issue();
       MDCN_BARRIER_LDS();  // B1
 
       // Sample fragments [plane][pixel block], each plane fetched while the products of the one before run -- the
       // first ones of a step during the last products of the step before.
       constexpr bool kEarlyX = CT <= 128;  // two planes that early, where the registers allow
-      uint4 xf[kF32Planes][NB];
+      uint4 xf[PLANES][NB];
       auto load_x = [&](int tile, int half, int p) {
         const uint4 *X = Xs[tile] + half * XFRAG + wave_p * (NB * 64) + lane;
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) xf[p][nb] = X[p * (PT / 32) * 64 + nb * 64];
       };
-      load_x(0, 0, 2);
-      if constexpr (kEarlyX) load_x(0, 0, 1);
+      load_x(0, 0, PLANES - 1);
+      if constexpr (kEarlyX && !kPairs) load_x(0, 0, 1);
       int rt = 0;
       for (int ks = 0; ks < nk; ++ks) {
         const int nt = rt == kF32Tiles - 1 ? 0 : rt + 1;
@@ -490,16 +574,18 @@ __global__ __launch_bounds__(kThreads, 2) void fused_f32_kernel(FusedArgs a) {
           };
           // (the order is kept: the scheduler, left to itself, reads each fragment right in front of its first use)
           load_weights(2 * ks + half + 1, wf[half ^ 1]);
-          if constexpr (!kEarlyX) load_x(rt, half, 1);
+          if constexpr (!kEarlyX && !kPairs) load_x(rt, half, 1);
           load_x(rt, half, 0);
           __builtin_amdgcn_sched_barrier(0);
-          products(2, 0);  // smallest terms first
-          products(1, 1);
+          if constexpr (!kPairs) {
+            products(2, 0);  // smallest terms first
+            products(1, 1);
+          }
           products(1, 0);
-          load_x(half ? nt : rt, half ^ 1, 2);
-          if constexpr (kEarlyX) load_x(half ? nt : rt, half ^ 1, 1);
+          load_x(half ? nt : rt, half ^ 1, PLANES - 1);
+          if constexpr (kEarlyX && !kPairs) load_x(half ? nt : rt, half ^ 1, 1);
           __builtin_amdgcn_sched_barrier(0);
-          products(0, 2);
+          if constexpr (!kPairs) products(0, 2);
           products(0, 1);
           products(0, 0);
         }
@@ -507,6 +593,7 @@ __global__ __launch_bounds__(kThreads, 2) void fused_f32_kernel(FusedArgs a) {
         mirror_issue();
         MDCN_BARRIER_LDS();  // end of step ks
       }
+      for (int ks = nk; ks < nk_pad; ++ks) MDCN_BARRIER_LDS();
       MDCN_BARRIER_LDS();  // E0: the sample tiles become staging
 
       // ---- a part of a tile: the parts meet in memory.  Every part stores its
@@ -604,9 +691,16 @@ __global__ __launch_bounds__(kThreads, 2) void fused_f32_kernel(FusedArgs a) {
           for (int r4 = 0; r4 < 4; ++r4) {
             const int px = nb * 32 + r4 * 8 + fhalf * 4;
             const f32x16 &c = acc[np * 2 + nb][mb];
+            int pexp[4] = {0, 0, 0, 0};
+            if constexpr (kPairs) {
+              const int4 pe = *(const int4 *)&row_exp[(wave_p * NB + np * 2) * 32 + px];
+              pexp[0] = pe.x, pexp[1] = pe.y, pexp[2] = pe.z, pexp[3] = pe.w;
+            }
             float v[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = fmaf(c[r4 * 4 + e], kSplitUnscale, bv[mb]);
+            for (int e = 0; e < 4; ++e)
+              v[e] = kPairs ? __builtin_amdgcn_ldexpf(c[r4 * 4 + e], -(pexp[e] + wexp[mb])) + bv[mb]
+                            : fmaf(c[r4 * 4 + e], kSplitUnscale, bv[mb]);
             TR::store4(stage + frow * RB + px * ES, v[0], v[1], v[2], v[3]);
           }
         }
@@ -667,7 +761,7 @@ __global__ __launch_bounds__(kThreads, 2) void fused_f32_kernel(FusedArgs a) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     auto kernarg = __builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(kernarg));
-    remake_not_finite<CT, WC, MB, NB>(*(const FusedArgs *)kernarg, units, nk_tile_pad, wave, lane);
+    remake_not_finite<CT, WC, MB, NB, AHEAD>(*(const FusedArgs *)kernarg, units, nk_tile_pad, wave, lane);
   }
 }
 

@@ -36,11 +36,14 @@ namespace mdcn {
 // of channels, i.e. each 128-byte slab as four planes -- for a reader that takes 32 bytes of a pixel at a
 // time and whose neighbouring lanes read neighbouring pixels (the backward's scatter kernel): four pixels
 // share a cache line there, where the 128-byte records give every lane a line of its own.
+// row_max (fp32, whole slabs; or null): also the largest magnitude of each pixel's channels of the slab, the upper 16 bits of a float rounded up,
+// [N][Cin/KC / max_unit][H*W][max_unit] (an infinity for what is not finite).
 // MAPPED: the copy's channels are those of `cm`, cp of them (a multiple of RC elements for REC = 32, of KC for
 // REC = 128), segments padded to a multiple of 4; padding channels are zero.
 template <typename E, bool BORDER, int REC = 128, bool MAPPED = false>
 __device__ __forceinline__ void relayout_vec_block(const Geom &g, const E *__restrict__ in, E *__restrict__ xt,
-                                                   int n_pchunks, int b, const ChanMap &cm = ChanMap(), int cp = 0) {
+                                                   int n_pchunks, int b, const ChanMap &cm = ChanMap(), int cp = 0,
+                                                   uint16_t *__restrict__ row_max = nullptr, int max_unit = 1) {
   static_assert(REC == 128 || REC == 32, "whole slabs or quarters of them");
   constexpr int EPV = 16 / (int)sizeof(E);
   constexpr int KC = 128 / (int)sizeof(E);
@@ -126,6 +129,24 @@ __device__ __forceinline__ void relayout_vec_block(const Geom &g, const E *__res
       for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int i = 0; i < 4; ++i) ow[i * 4 + j] = rw[j * 4 + i];
+    }
+  }
+  if constexpr (sizeof(E) == 4 && BORDER && REC == 128 && !MAPPED) {
+    if (row_max) {
+      uint32_t top[EPV];
+#pragma unroll
+      for (int i = 0; i < EPV; ++i) {
+        int t = (int)max(max(o[i].x & 0x7fffffffu, o[i].y & 0x7fffffffu), max(o[i].z & 0x7fffffffu, o[i].w & 0x7fffffffu));
+        // over the eight lanes that hold the pixel: lane ^ 1, lane ^ 2, the other four
+        t = max(t, __builtin_amdgcn_update_dpp(t, t, 0xB1, 0xf, 0xf, false));
+        t = max(t, __builtin_amdgcn_update_dpp(t, t, 0x4E, 0xf, 0xf, false));
+        t = max(t, __builtin_amdgcn_update_dpp(t, t, 0x141, 0xf, 0xf, false));
+        top[i] = (uint32_t)t;
+      }
+      if (cg < np) {   // the lane of pixel cg
+        const uint32_t t = cg == 0 ? top[0] : cg == 1 ? top[1] : cg == 2 ? top[2] : top[3];
+        row_max[(((long)n * (slabs_total / max_unit) + slab / max_unit) * plane + p0 + cg) * max_unit + slab % max_unit] = (uint16_t)((min(t, 0x7f800000u) + 0xffffu) >> 16);
+      }
     }
   }
   if constexpr (REC == 128) {
