@@ -136,18 +136,25 @@ bool fused_ok(const mdcn_params *p, const Geom &g) {
   return true;
 }
 
-// Length of the fp32 kernel's persistent schedule of `tiles` tiles of nk K steps in tile times, as UnitSchedule lays
-// it out: whole rounds, then the last round's tiles whole or cut into parts.  (More than four parts count as four: with the sum of all of them they take no less.  N=1 256
+// Length of the fp32 kernel's persistent schedule of `tiles` tiles of nk K steps in tile times, as PartSchedule lays
+// it out: whole rounds, then the last round's tiles whole, in equal parts or (*even) in even shares, whichever is shorter with what it costs that
+// parts meet.  (More than four parts count as four: with the sum of all of them they take no less.  N=1 256
 // channels 50x84, six parts of 256-channel tiles 84 us a call, three of 128-channel ones 69.)
-double schedule_rounds(long tiles, int nk, bool may_cut) {
+// kEvenCost: steps that even shares cost beyond equal parts' or a whole tile's: a second unit, and twice the parts through memory.
+constexpr double kEvenCost = 14.0;
+double schedule_rounds(long tiles, int nk, bool may_cut, bool *even = nullptr) {
   const int stride = std::max(1, num_cus() / 8);
+  if (even) *even = false;
   const long chunk = (tiles + 7) / 8;  // the fullest XCD
   const long full = chunk / stride, rest = chunk % stride;
   if (rest == 0) return (double)full;
-  const int rounds = (nk + kGatherAhead - 1) / kGatherAhead;
-  long parts = 1;
-  if (may_cut) parts = std::max<long>(1, std::min<long>(std::min<long>(stride / rest, 4), rounds / (8 / kGatherAhead)));
-  return (double)full + 1.0 / (double)parts;
+  const int rounds = (nk + kGatherAhead - 1) / kGatherAhead, min_rounds = 8 / kGatherAhead;
+  if (!may_cut) return (double)full + 1.0;
+  const long parts = std::max<long>(1, std::min<long>(std::min<long>(stride / rest, 4), rounds / min_rounds));
+  const double equal = 1.0 / (double)parts, shares = (double)rest / stride + kEvenCost / nk;
+  if (shares >= equal || rest * rounds < 3L * min_rounds * stride) return (double)full + equal;
+  if (even) *even = true;
+  return (double)full + shares;
 }
 
 struct Plan {
@@ -160,7 +167,8 @@ struct Plan {
   size_t max_bytes, wexp_bytes, rexp_bytes, tpix_bytes;   // (four weights to an offset)
   size_t pair_bytes() const { return max_bytes + wexp_bytes + rexp_bytes + 5 * tpix_bytes; }
   size_t cut_bytes;  // eight-wave kernel: buffers and counters of the tiles it cuts along K (may be left out)
-  int cut_wgs;     // ... one buffer and one counter per workgroup of its grid
+  int cut_wgs;     // ... one buffer (cut_even: two) and one counter per workgroup of its grid
+  bool cut_even;   // fp32: even shares of the last round
   bool seg;          // segment kernel: the shapes the fused kernels do not cover
   bool seg_small;    // ... or small calls of those they do
   SegPlan sp;
@@ -170,6 +178,8 @@ struct Plan {
   size_t owp_bytes;  // packed conv_offset weights (fused path, conv_offset run here)
   size_t raw_bytes;  // conv_offset output kept in the workspace
 };
+
+size_t part_buffers(const Plan &pl) { return align_up((size_t)pl.cut_wgs * (pl.cut_even ? 2 : 1) * kPT * kF2CT * 4); }
 
 // What a pack-level call adds to the plain one.
 struct PackExtra {
@@ -309,6 +319,7 @@ int make_plan(const mdcn_params *p, const Geom &g, Plan *pl, bool may_be_small =
   pl->CT = pl->KC = pl->n_ctiles = pl->slabs = pl->n_chunk = 0;
   pl->xt_bytes = pl->wp_bytes = pl->owp_bytes = pl->raw_bytes = pl->cut_bytes = pl->max_bytes = pl->wexp_bytes = pl->rexp_bytes = pl->tpix_bytes = 0;
   pl->cut_wgs = 0;
+  pl->cut_even = false;
   pl->CO = 3 * g.DG * g.taps;
   pl->CO_pad = (pl->CO + 31) / 32 * 32;
   pl->mask_kind = kMaskLogit;
@@ -323,14 +334,15 @@ int make_plan(const mdcn_params *p, const Geom &g, Plan *pl, bool may_be_small =
   const uint64_t img = (uint64_t)g.Hp * g.Wp * g.Cin * es;
   pl->n_chunk = (int)std::min<uint64_t>((uint64_t)g.N, std::max<uint64_t>(1, g_fwd_pass_bytes.load() / img));
   if (p->dtype == MDCN_F32 && pl->CT == 256) {
-    // an fp32 tile's time goes with its width: a 128-channel tile takes 0.56 of a 256-channel one (N=8, 256
-    // channels, 64x64: 240 us as 512 tiles of 128 channels, 213 us as 256 of 256), so what counts is how
-    // evenly the tiles fill the workgroups
+    // What counts is how evenly the tiles fill the workgroups, and a tile's time, which goes with its width: a K step of 128 channels takes
+    // 0.72 of one of 256 (1 910 and 2 650 clocks); where all tiles are cut what parts cost each other goes with the width too (N=1 256
+    // channels 50x84: 33 tiles of 256 channels in six parts 61.2 us a call, 66 of 128 in three 50.5).
     const long px_tiles = ((long)pl->n_chunk * g.Ho * g.Wo + kPT - 1) / kPT;
     const int nk = pl->slabs * g.taps;
     auto cost = [&](int ct) {
       const long tiles = px_tiles * ((g.cout_g + ct - 1) / ct) * g.G;
-      return schedule_rounds(tiles, nk, !p->no_k_split) * (ct == 256 ? 1.0 : 0.56);
+      const double rounds = schedule_rounds(tiles, nk, !p->no_k_split);
+      return rounds * (ct == 256 ? 1.0 : rounds < 1.0 ? 0.56 : 0.72);
     };
     if (cost(128) < 0.95 * cost(256)) pl->CT = 128;
   }
@@ -388,9 +400,14 @@ int make_plan(const mdcn_params *p, const Geom &g, Plan *pl, bool may_be_small =
       }
       cuts = may_cut((px + kPT - 1) / kPT * pl->n_ctiles * g.G);
     }
+    if (p->dtype == MDCN_F32) {   // (by the first pass's schedule, which all have but the last)
+      const long tiles = ((long)pl->n_chunk * plane_out + kPT - 1) / kPT * pl->n_ctiles * g.G;
+      (void)schedule_rounds(tiles, pl->slabs * g.taps, true, &pl->cut_even);
+      cuts = cuts || pl->cut_even;
+    }
     if (cuts) {
       pl->cut_wgs = num_cus() / 8 * 8;
-      pl->cut_bytes = align_up((size_t)pl->cut_wgs * kPT * kF2CT * 4) + align_up((size_t)pl->cut_wgs * 4);
+      pl->cut_bytes = part_buffers(*pl) + align_up((size_t)pl->cut_wgs * 4);
     }
   }
   if (p->path == MDCN_PATH_FUSED_WIDE && !wide_ok(p, g, *pl)) return MDCN_ERR_PATH;
@@ -631,7 +648,7 @@ int run_typed(const mdcn_params *p, const Geom &g, const Plan &pl, hipStream_t s
     pa.slabs = pl.slabs;
     pa.slabs_total = g.Cin / pl.KC;
     float *cut_part = (float *)(opt + pl.pair_bytes());
-    uint32_t *cut_cnt = (uint32_t *)((unsigned char *)cut_part + align_up((size_t)pl.cut_wgs * kPT * kF2CT * 4));
+    uint32_t *cut_cnt = (uint32_t *)((unsigned char *)cut_part + part_buffers(pl));
     if (!pl.cut_bytes) cut_part = nullptr, cut_cnt = nullptr;
 
     // weights: once per call -- inside the launch that re-lays the first batch chunk; on their own when
@@ -752,6 +769,7 @@ int run_typed(const mdcn_params *p, const Geom &g, const Plan &pl, hipStream_t s
                            p->mask ? (const E *)p->mask + (size_t)n0 * g.DG * g.taps * plane_out : nullptr, g);
       }
       fa.cut_max = !pl.cut_bytes ? 0 : sizeof(E) == 4 ? kF32CutMax : uses_fused2(p, g, pl) ? kF2CutMax : kCutMax;
+      fa.cut_even = pl.cut_even;
       fa.cut_part = cut_part;
       fa.cut_cnt = cut_cnt;
       fa.bias = p->bias;

@@ -81,6 +81,7 @@ struct FusedArgs {
   // cut_max parts (0 or 1: never) that meet in cut_part, gridDim.x buffers of kPT x 256 floats,
   // counted in cut_cnt, gridDim.x words that are zero when the kernel starts
   int cut_max;
+  int cut_even;   // fused_f32_kernel only: the last round's tiles end to end, an even share for each workgroup (PartSchedule)
   void *cut_part;
   void *cut_cnt;
   // fused_f32_kernel only: the call's own tensors, for outputs that are made again one by one (channels of `in` in_c

@@ -66,6 +66,88 @@ constexpr size_t fused_f32_lds_bytes(int tmax) {
   return (size_t)kF32Tiles * kPT * 192 + (size_t)kPT * tmax * 20 + 16;
 }
 
+// Units of one workgroup: as UnitSchedule's, tiles round robin within the XCD's run and then the last round's tiles in parts.  These
+// `rest` tiles lie end to end, rest * rounds rounds of K steps, and workgroup w of the XCD's `stride` has those from pos(w) to
+// pos(w + 1): an equal part of one tile (`parts` workgroups each, some may have nothing), or, `even`, the same number of rounds for
+// everybody, wherever tiles begin; a workgroup then has parts of up to two tiles, and a tile up to three.  Parts of less than min_rounds
+// are not made.  host: the same arithmetic for the plan.
+struct PartSchedule {
+  int xcd, wg, stride, tile0, full, rest, rounds, round, min_rounds, parts, per_wg;
+  int begin, end;   // this workgroup's rounds of the last round
+  bool even;
+
+  __host__ __device__ __forceinline__ void init(int xcd_, int wg_, int stride_, int total_tiles, int nk_pad, int round_, int min_rounds_,
+                                                int cut_max, bool even_) {
+    xcd = xcd_, wg = wg_, stride = stride_, round = round_, min_rounds = min_rounds_;
+    per_wg = even_ ? 2 : 1;
+    const int chunk = (total_tiles + 7) >> 3;
+    tile0 = xcd * chunk;
+    const int left = total_tiles - tile0, count = left < 0 ? 0 : left < chunk ? left : chunk;
+    full = count / stride;
+    rest = count - full * stride;
+    rounds = nk_pad / round;
+    even = even_ && rest * rounds >= 3 * min_rounds * stride;   // (no share may vanish between two tiles)
+    parts = 1;
+    if (even) {
+      begin = pos(wg), end = pos(wg + 1);
+      return;
+    }
+    if (cut_max > 1 && rest > 0) {
+      parts = stride / rest < cut_max ? stride / rest : cut_max;
+      parts = parts < rounds / min_rounds ? parts : rounds / min_rounds;
+      parts = parts > 1 ? parts : 1;
+    }
+    const int t = wg / parts, i = wg - t * parts;
+    begin = t * rounds + i * rounds / parts, end = t * rounds + (i + 1) * rounds / parts;
+    if (t >= rest) end = begin;
+  }
+  __host__ __device__ __forceinline__ int pos(int w) const {   // even shares
+    const int x = w * rest * rounds / stride, r = x % rounds;
+    return r < min_rounds ? x - r : rounds - r < min_rounds ? x - r + rounds : x;
+  }
+  __host__ __device__ __forceinline__ int units() const {
+    if (begin == end) return full;
+    return full + (even && (end - 1) / rounds > begin / rounds ? 2 : 1);
+  }
+  struct Unit {
+    int tile, kb, pad;          // K steps kb .. kb + pad - 1 of a tile
+    bool is_part;
+    int slot;                   // of its tile among the last round's
+    int first, n, idx;          // first workgroup with a part of the tile, number of parts, which one this is
+    bool first_behind;          // the first part is its workgroup's second
+  };
+  __host__ __device__ __forceinline__ Unit unit(int u) const {
+    Unit r;
+    r.tile = tile0 + wg + u * stride;
+    r.kb = 0, r.pad = rounds * round;
+    r.is_part = false;
+    r.slot = r.first = r.idx = 0, r.n = 1;
+    r.first_behind = false;
+    if (u < full) return r;
+    if (!even) {
+      r.slot = wg / parts;
+      r.first = r.slot * parts, r.n = parts, r.idx = wg - r.first;
+    } else {
+      r.slot = begin / rounds + u - full;
+      int f = wg, l = wg;
+      while (f > 0 && pos(f) > r.slot * rounds) --f;
+      while (l + 1 < stride && pos(l + 1) < (r.slot + 1) * rounds) ++l;
+      r.first = f, r.n = l - f + 1, r.idx = wg - f;
+      r.first_behind = pos(f) < r.slot * rounds;
+    }
+    const int t0 = r.slot * rounds, lo = begin > t0 ? begin : t0, hi = end < t0 + rounds ? end : t0 + rounds;
+    r.tile = tile0 + full * stride + r.slot;
+    r.kb = (lo - t0) * round, r.pad = (hi - lo) * round;
+    r.is_part = hi - lo < rounds;
+    return r;
+  }
+  // buffer of part i of a unit's tile (one for each workgroup; even: two), and the counter of the tile
+  __host__ __device__ __forceinline__ int buffer(const Unit &r, int i) const {
+    return (xcd * stride + r.first + i) * per_wg + (i == 0 && r.first_behind ? 1 : 0);
+  }
+  __host__ __device__ __forceinline__ int counter(const Unit &r) const { return xcd * stride + r.slot; }
+};
+
 // Four floats, scaled already, as three bf16 planes of 8 bytes each.  An infinity, or a number that bf16 rounds to one
 // (from 2^128 (1 - 2^-9) on), leaves NaN in the planes, and so in every sum that it is part of: sums that are not
 // finite are not used, but made again from the tensors themselves.
@@ -198,17 +280,19 @@ __device__ __forceinline__ void pack_weight_split(const Geom &g, const float *__
   }
 }
 
-// The outputs of consumer wave `wave` in the first `units` units of its workgroup's schedule that are not finite, from the
-// call's own tensors.
+// The outputs of consumer wave `wave` in the units of its workgroup's schedule that are not finite, from the call's own tensors; units of the last round
+// whose bit is set in `skip` were stored by others.
 template <int CT, int WC, int MB, int NB, int AHEAD>
-__device__ __forceinline__ void remake_not_finite(const FusedArgs &a, int units, int nk_tile_pad, int wave, int lane) {
+__device__ __forceinline__ void remake_not_finite(const FusedArgs &a, uint32_t skip, int nk_tile_pad, int wave, int lane) {
   const Geom &g = a.g;
   const int plane_out = g.Ho * g.Wo;
-  UnitSchedule us;
-  us.init(a.n_ptiles * a.n_ctiles * g.G, nk_tile_pad, AHEAD, 8 / AHEAD, a.cut_max);
+  PartSchedule us;
+  us.init((int)(blockIdx.x & 7), (int)(blockIdx.x >> 3), (int)(gridDim.x >> 3), a.n_ptiles * a.n_ctiles * g.G, nk_tile_pad, AHEAD, 8 / AHEAD,
+          a.cut_max, a.cut_even != 0);
 #pragma unroll 1
-  for (int u = 0; u < units; ++u) {
-    int L = us.tile_of(u);
+  for (int u = 0; u < us.units(); ++u) {
+    if (u >= us.full && (skip >> (u - us.full) & 1)) continue;
+    int L = us.unit(u).tile;
     const int ctile = L % a.n_ctiles;
     L /= a.n_ctiles;
     const int grp = L % g.G, ptile = L / g.G;
@@ -270,19 +354,21 @@ __global__ __launch_bounds__(kThreads, 2) void fused_f32_kernel(FusedArgs a) {
   // XCD-aware persistent schedule: consecutive workgroup ids sit on different
   // XCDs; each XCD walks one contiguous run of tiles so that the halo rows
   // neighbouring tiles share stay in its L2.  Tiles of the run's last round are
-  // cut along K (UnitSchedule): parts of at least 8 steps.
-  UnitSchedule us;
-  us.init(a.n_ptiles * a.n_ctiles * g.G, nk_tile_pad, AHEAD, 8 / AHEAD, a.cut_max);
+  // cut along K (PartSchedule): parts of at least 8 steps.
+  PartSchedule us;
+  us.init((int)(blockIdx.x & 7), (int)(blockIdx.x >> 3), (int)(gridDim.x >> 3), a.n_ptiles * a.n_ctiles * g.G, nk_tile_pad, AHEAD, 8 / AHEAD,
+          a.cut_max, a.cut_even != 0);
 
   bool bad = false;    // consumer waves: a sum of a stored tile was not finite
-  int units = us.T;    // ... how many of the units they have stored: all, or all but a part of a cut tile
-  for (int u = 0; u < us.T; ++u) {
-    const bool is_part = us.is_part(u);
+  uint32_t skip = 0;   // ... units of the last round that they have not stored: parts of cut tiles
+  const int units = us.units();
+  for (int u = 0; u < units; ++u) {
+    const PartSchedule::Unit un = us.unit(u);
+    const bool is_part = un.is_part;
     // K range of the unit: steps kb .. kb + nk - 1 of the tile, padded to nk_pad
-    const int kb = is_part ? us.part_kb : 0;
-    const int nk_pad = is_part ? us.part_pad : nk_tile_pad;
+    const int kb = un.kb, nk_pad = un.pad;
     const int nk = min(nk_tile - kb, nk_pad);
-    int L = us.tile_of(u);
+    int L = un.tile;
     const int ctile = L % a.n_ctiles;
     L /= a.n_ctiles;
     const int grp = L % g.G;
@@ -603,16 +689,15 @@ __global__ __launch_bounds__(kThreads, 2) void fused_f32_kernel(FusedArgs a) {
       // the sum does not depend on who was last -- and goes on to the epilogue; the
       // others are done.  Nobody waits for anybody; the last part leaves the counter
       // at zero for the next launch.  Stores and loads are device coherent (sc1):
-      // they go past the caches private to a CU or an XCD.  A part is a workgroup's
-      // last unit, and the producers take part in the two barriers.
+      // they go past the caches private to a CU or an XCD.  The producers take part in the
+      // two barriers.
       bool store_tile = true;
       if (is_part) {
         constexpr int NQ = NB * MB * 4;           // 16-byte quads of accumulators per lane
         constexpr int CQ = 8;                     // quads read back at a time (NQ is a multiple of 8)
-        const int tslot = us.counter_slot();
-        const unsigned char *pbase =
-            (const unsigned char *)a.cut_part + (size_t)us.buffer_slot0() * (size_t)(PT * 256 * 4);
-        const unsigned char *mine = uniform_ptr(pbase + (size_t)us.part_idx * (size_t)(PT * 256 * 4));
+        const int tslot = us.counter(un);
+        auto part_of = [&](int i) { return (const unsigned char *)a.cut_part + (size_t)us.buffer(un, i) * (size_t)(PT * 256 * 4); };
+        const unsigned char *mine = uniform_ptr(part_of(un.idx));
         // quad j of the 256 consumer lanes is one 4 KiB run.  (The offset is opaque to the optimiser,
         // which would otherwise form the addresses below ahead of the unit loop and keep them live.)
         uint32_t voff = (uint32_t)tid * 16u;
@@ -637,12 +722,11 @@ __global__ __launch_bounds__(kThreads, 2) void fused_f32_kernel(FusedArgs a) {
           part_arrived = __hip_atomic_fetch_add((uint32_t *)a.cut_cnt + tslot, 1u, __ATOMIC_RELAXED,
                                                 __HIP_MEMORY_SCOPE_AGENT);
         MDCN_BARRIER_LDS();
-        store_tile = part_arrived == (uint32_t)(us.parts - 1);
+        store_tile = part_arrived == (uint32_t)(un.n - 1);
         if (store_tile) {
-          const bool two = us.parts == 2;
-          const unsigned char *src0 = two ? pbase + (size_t)(1 - us.part_idx) * (size_t)(PT * 256 * 4) : pbase;
-          for (int i = two ? 1 : 0; i < us.parts; ++i) {
-            const unsigned char *src = uniform_ptr(src0);
+          const bool two = un.n == 2;
+          for (int i = two ? 1 : 0; i < un.n; ++i) {
+            const unsigned char *src = uniform_ptr(part_of(two ? 1 - un.idx : i));
 #pragma unroll
             for (int q0 = 0; q0 < NQ; q0 += CQ) {
               f32x4 tmp[CQ];
@@ -662,7 +746,6 @@ __global__ __launch_bounds__(kThreads, 2) void fused_f32_kernel(FusedArgs a) {
                       i == 0 ? tmp[j][e] : acc[blk / MB][blk % MB][4 * qd + e] + tmp[j][e];
               }
             }
-            src0 += PT * 256 * 4;
           }
           if (tid == 0)
             __hip_atomic_store((uint32_t *)a.cut_cnt + tslot, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -748,7 +831,7 @@ __global__ __launch_bounds__(kThreads, 2) void fused_f32_kernel(FusedArgs a) {
         for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
           for (int r = 0; r < 16; ++r) t = fmaf(acc[nb][mb][r], 0.0f, t);
-      if (!store_tile) units = u;
+      if (!store_tile) skip |= 1u << (u - us.full);
       bad = bad || (store_tile && __any(t != t));
       MDCN_BARRIER_LDS();  // E1
     }
@@ -761,7 +844,7 @@ __global__ __launch_bounds__(kThreads, 2) void fused_f32_kernel(FusedArgs a) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     auto kernarg = __builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(kernarg));
-    remake_not_finite<CT, WC, MB, NB, AHEAD>(*(const FusedArgs *)kernarg, units, nk_tile_pad, wave, lane);
+    remake_not_finite<CT, WC, MB, NB, AHEAD>(*(const FusedArgs *)kernarg, skip, nk_tile_pad, wave, lane);
   }
 }
 
