@@ -180,6 +180,7 @@ struct Plan {
 };
 
 size_t part_buffers(const Plan &pl) { return align_up((size_t)pl.cut_wgs * (pl.cut_even ? 2 : 1) * kPT * kF2CT * 4); }
+size_t cut_region(const Plan &pl) { return part_buffers(pl) + align_up((size_t)pl.cut_wgs * 4); }
 
 // What a pack-level call adds to the plain one.
 struct PackExtra {
@@ -407,7 +408,7 @@ int make_plan(const mdcn_params *p, const Geom &g, Plan *pl, bool may_be_small =
     }
     if (cuts) {
       pl->cut_wgs = num_cus() / 8 * 8;
-      pl->cut_bytes = part_buffers(*pl) + align_up((size_t)pl->cut_wgs * 4);
+      pl->cut_bytes = cut_region(*pl);
     }
   }
   if (p->path == MDCN_PATH_FUSED_WIDE && !wide_ok(p, g, *pl)) return MDCN_ERR_PATH;
@@ -882,6 +883,10 @@ int run(const mdcn_params *p, void *stream, float *ms, const mdcn_pack_params *p
                    ((uintptr_t)p->workspace % kAlign) != 0))
     return MDCN_ERR_WORKSPACE;
   if (p->workspace_bytes < need + pl.pair_bytes()) pl.max_bytes = pl.wexp_bytes = pl.rexp_bytes = pl.tpix_bytes = 0;
+  if (pl.cut_even && p->workspace_bytes < need + pl.pair_bytes() + pl.cut_bytes) {  // equal parts have half of the buffers
+    pl.cut_even = false;
+    pl.cut_bytes = cut_region(pl);
+  }
   if (p->workspace_bytes < need + pl.pair_bytes() + pl.cut_bytes) pl.cut_bytes = 0, pl.cut_wgs = 0;
   hipStream_t st = (hipStream_t)stream;
   switch (p->dtype) {
