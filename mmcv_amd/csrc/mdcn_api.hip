@@ -904,7 +904,7 @@ int split_raw(const mdcn_pack_params *pp, const Geom &g, E *offset, E *mask, hip
   return hipGetLastError() == hipSuccess ? MDCN_OK : MDCN_ERR_LAUNCH;
 }
 
-// Workspace: the convolution's, then conv_offset's, which reads the copy of the input the former leaves.
+// Workspace: the convolution's, then conv_offset's, which reads the copy of the input the former leaves, then (optional) the maxima.
 bool plan_pack_backward(const mdcn_pack_bwd_params *pb, const Geom &g, BwdPlan *pl, OconvBwdPlan *ol) {
   make_bwd_plan(&pb->bwd, g, g_bwd_pass_bytes.load(), pl);
   return oconv_bwd_plan(g, pb->bwd.conv.dtype, pb->unmodulated != 0, pb->through_input != 0,
@@ -1058,7 +1058,7 @@ size_t mdcn_backward_workspace_bytes(const mdcn_bwd_params *bp) {
   if (check_bwd(bp, &g, false) != MDCN_OK) return 0;
   BwdPlan pl;
   make_bwd_plan(bp, g, g_bwd_pass_bytes.load(), &pl);
-  return pl.total();
+  return pl.total() + pl.max_bytes();
 }
 
 int mdcn_backward(const mdcn_bwd_params *bp, void *hip_stream) {
@@ -1071,6 +1071,7 @@ int mdcn_backward(const mdcn_bwd_params *bp, void *hip_stream) {
   const mdcn_params *p = &bp->conv;
   if (need > 0 && (!p->workspace || p->workspace_bytes < need || ((uintptr_t)p->workspace % kAlign) != 0))
     return MDCN_ERR_WORKSPACE;
+  if (pl.max_bytes() && p->workspace_bytes >= need + pl.max_bytes()) pl.max_at = need;
   return run_backward(bp, g, pl, (hipStream_t)hip_stream);
 }
 
@@ -1102,7 +1103,7 @@ size_t mdcn_pack_backward_workspace_bytes(const mdcn_pack_bwd_params *pb) {
   if (!pb || check_bwd(&pb->bwd, &g, false) != MDCN_OK) return 0;
   BwdPlan pl;
   OconvBwdPlan ol;
-  return plan_pack_backward(pb, g, &pl, &ol) ? pl.total() + ol.total() : 0;
+  return plan_pack_backward(pb, g, &pl, &ol) ? pl.total() + ol.total() + pl.max_bytes() : 0;
 }
 
 int mdcn_pack_backward(const mdcn_pack_bwd_params *pb, void *hip_stream) {
@@ -1118,6 +1119,7 @@ int mdcn_pack_backward(const mdcn_pack_bwd_params *pb, void *hip_stream) {
   const size_t need = pl.total() + ol.total();
   if (need > 0 && (!p->workspace || p->workspace_bytes < need || ((uintptr_t)p->workspace % kAlign) != 0))
     return MDCN_ERR_WORKSPACE;
+  if (pl.max_bytes() && p->workspace_bytes >= need + pl.max_bytes()) pl.max_at = need;
   rc = run_backward(&pb->bwd, g, pl, (hipStream_t)hip_stream);
   if (rc != MDCN_OK || (!ol.data && !ol.weight)) return rc;
   unsigned char *ws = (unsigned char *)p->workspace;

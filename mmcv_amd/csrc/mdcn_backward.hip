@@ -67,6 +67,7 @@ void make_bwd_plan(const mdcn_bwd_params *bp, const Geom &g, uint64_t pass_bytes
   pl->w_tile = kCgTile;
   pl->w_splits = 1;
   pl->gpad_bytes = 0;
+  pl->gmax_bytes = pl->wmax_bytes = pl->max_at = 0;
   pl->bsplits = 0;
   pl->im = pl->om = ChanMap{1, 1, 1, 1, 1};
   pl->parts = 1;
@@ -205,6 +206,12 @@ void make_bwd_plan(const mdcn_bwd_params *bp, const Geom &g, uint64_t pass_bytes
     pl->wt_bytes = align_up((size_t)g.G * pl->M_pad * om.cgp * es);
     pl->d_bytes = pl->fused ? 0 : align_up(d_img * pl->n_chunk);
     pl->mx_bytes = kAlign;
+    // fp32: the column gradient as fp16 pairs (tile_products), with sums of up to 64 products as bf16 triples: their error is as large (grad_input against
+    // float64, triples / pairs: 64 output channels 1.23e-7 / 1.26e-7, 72 1.43e-7 / 1.37e-7, 256 2.49e-7 / 1.99e-7, 512 3.57e-7 / 2.66e-7).
+    if (es == 4 && om.cgp > 64) {
+      pl->gmax_bytes = align_up((size_t)g.N * g.G * (om.cgp / KC) * plane_out * 2);
+      pl->wmax_bytes = align_up((size_t)g.G * pl->M_pad * (om.cgp / KC) * 2);
+    }
     if (pl->fused)
       pl->part_bytes = align_up((size_t)((g.N + pl->n_chunk - 1) / pl->n_chunk) * FusedSchedule::kGroups * 3 * g.taps * 256 * 4);
     else if (pl->parts > 1)
@@ -377,6 +384,8 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
   float *pmask = poff + (long)pl.parts * off_total;
   float *wpart = (float *)take(pl.wpart_bytes);
   unsigned char *gpad = take(pl.gpad_bytes);
+  uint16_t *gmax = pl.max_at ? (uint16_t *)((unsigned char *)p->workspace + pl.max_at) : nullptr;
+  uint16_t *wmax = pl.max_at ? (uint16_t *)((unsigned char *)p->workspace + pl.max_at + pl.gmax_bytes) : nullptr;
   const long n_in = (long)g.N * g.Cin * g.H * g.W;
 
   // a sample of the offsets, 64 Ki of them at most, decides which window the scatter kernel uses
@@ -411,6 +420,8 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
     a.xt = xt;
     a.gT = gT;
     a.wT = wT;
+    a.gmax = gmax;
+    a.wmax = wmax;
     a.gpad = gpad;
     a.col = col;
     a.gin32 = gin32;
@@ -458,6 +469,8 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
       ColGradArgs ca;
       ca.wT = wT;
       ca.gT = gT;
+      ca.gmax = gmax;
+      ca.wmax = wmax;
       ca.D = (float *)D;
       ca.P = (int)plane_out;
       ca.px_tiles = (int)((plane_out + pl.cg_tile - 1) / pl.cg_tile);
@@ -474,10 +487,18 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
       ca.n0 = n0;
       ca.total = (long)nb * g.G * ca.px_tiles * ca.m_tiles;
       const dim3 grid((unsigned)((ca.total + 7) / 8 * 8));
-      if (pl.cg_tile == kCgTileBig)
-        hipLaunchKernelGGL((bwd_colgrad_kernel<E, kCgTileBig>), grid, dim3(2 * kCgTileBig), 0, st, ca);
-      else
-        hipLaunchKernelGGL((bwd_colgrad_kernel<E, kCgTile>), grid, dim3(2 * kCgTile), 0, st, ca);
+      auto launch = [&](auto pairs) {
+        if (pl.cg_tile == kCgTileBig)
+          hipLaunchKernelGGL((bwd_colgrad_kernel<E, kCgTileBig, decltype(pairs)::value>), grid, dim3(2 * kCgTileBig), 0, st, ca);
+        else
+          hipLaunchKernelGGL((bwd_colgrad_kernel<E, kCgTile, decltype(pairs)::value>), grid, dim3(2 * kCgTile), 0, st, ca);
+      };
+      if constexpr (sizeof(E) == 4) {
+        if (gmax) launch(std::true_type());
+        else launch(std::false_type());
+      } else {
+        launch(std::false_type());
+      }
       check();
     }
     if (pl.fused) {

@@ -21,6 +21,7 @@ struct BwdPreArgs {
   int end[kPreJobs];       // job j has the blocks from end[j - 1] on
   const void *in, *gout, *w;
   void *xt, *gT, *wT, *gpad, *col;
+  uint16_t *gmax, *wmax;   // fp32, or null: see ColGradArgs
   float *gin32;
   long n_in;               // elements of gin32
   int x_chunks, g_chunks;  // pixel chunks of the re-layouts
@@ -56,7 +57,7 @@ __global__ __launch_bounds__(256) void bwd_prepass_kernel(BwdPreArgs a) {
     gg.Cin = g.Cout;
     gg.H = g.Ho;
     gg.W = g.Wo;
-    relayout_vec_block<E, false, 128, true>(gg, (const E *)a.gout, (E *)a.gT, a.g_chunks, b - a.end[kPreX], a.om, a.cout_p);
+    relayout_vec_block<E, false, 128, true>(gg, (const E *)a.gout, (E *)a.gT, a.g_chunks, b - a.end[kPreX], a.om, a.cout_p, a.gmax);
     return;
   }
   __shared__ float red[4];
@@ -150,6 +151,14 @@ __global__ __launch_bounds__(256) void bwd_prepass_kernel(BwdPreArgs a) {
     E v = from_f32<E>(0.0f);
     if (tap < g.taps && room > 0 && co < g.cout_g)
       v = ((const E *)a.w)[((long)(grp * g.cout_g + co) * g.cin_g + c) * g.taps + tap];
+    if constexpr (sizeof(E) == 4) {
+      if (a.wmax) {   // (32 neighbouring lanes have 32 output channels of a row)
+        int top = (int)(__float_as_uint(v) & 0x7fffffffu);
+#pragma unroll
+        for (int s = 16; s; s >>= 1) top = max(top, __shfl_xor(top, s));
+        if ((tid & 31) == 0) a.wmax[idx >> 5] = (uint16_t)((min((uint32_t)top, 0x7f800000u) + 0xffffu) >> 16);
+      }
+    }
     long at = idx;
     if (a.wt_run) {
       const int run = co / a.wt_run, len = min(a.wt_run, a.om.cgp - run * a.wt_run);

@@ -46,6 +46,9 @@ struct ColGradArgs {
   // (channel counts are those of the padded orders, see BwdPlan)
   const void *wT;  // [G][M_pad][cout_g]
   const void *gT;  // [N][Cout / KC][P][KC], KC = 128 bytes of channels
+  // fp32 as fp16 pairs: the largest magnitude of each 128 bytes of either, as relayout_vec_block's row_max
+  const uint16_t *wmax;  // [G][M_pad][cout_g / KC]
+  const uint16_t *gmax;  // [N][Cout / KC][P]
   float *D;        // [images of the pass][Cin / 16][taps][P][16]
   int P;           // output pixels per image
   int px_tiles, m_tiles;
@@ -59,23 +62,27 @@ struct ColGradArgs {
 // A wave's products of one K step of either kernel: TILE / 64 x 2 blocks of 32 x 32 over 128 bytes of K, operand tiles
 // [row][8 chunks of 16 bytes, swizzled by the row number].
 //
-// fp32 runs on the bf16 matrix pipe: three bf16 planes per operand and six of their nine products, as in
-// fused_f32_kernel, whose error is that of fp32 arithmetic.  Operands are split behind the LDS reads (every wave for
-// itself: some 290 VALU instructions per 16 of K beside 48 MFMAs of 32 clocks, where the fp32 MFMAs were 64 of 64
-// clocks).  An infinity, or a number that the scale takes to one (kSplitScale), leaves NaN in the planes and so in the sums: a workgroup
-// that finds any goes over its K range again with fp32 MFMAs (EXACT).
-// N=2 256 -> 256 50x84, us, fp32 / bf16 pipe: column gradient 151 / 93, weight gradient 107 / 70.  Errors against float64
-// (2-norm): grad_input 2.9e-7 / 2.5e-7, grad_weight 3.3e-7 / 3.0e-7.
-template <typename E, int TILE, bool EXACT>
+// fp32 runs on the 16-bit matrix pipe, as in fused_f32_kernel, with an error that is that of fp32 arithmetic: of bf16 triples (six of the nine products
+// of three planes; the weight gradient, whose rows have no exponents at hand) or of fp16 pairs (three products of two planes; the column
+// gradient of more than 64 output channels).  Pairs are scaled row by row: a pixel's channels of grad_output and a weight row's output
+// channels by the largest of them, which the pre-pass writes beside its copies.  Operands are split behind the LDS reads, every wave for itself: beside
+// 48 bf16 MFMAs of 32 clocks per 16 of K, or 24 fp16 ones, some 290 VALU instructions, which is what pairs are bound by.  An infinity, or a number that the
+// scale takes to one (kSplitScale), leaves NaN in the planes and so in the sums: a workgroup
+// that finds any goes over its K range again with fp32 MFMAs (PLANES = 0).
+// Column gradient in us, triples / pairs: N=2 256 -> 256 50x84 78 / 57 (fp32 MFMAs 151), N=8 64x64 279 / 202, N=4 512 64x64 484 / 338 (tiles of 256), N=4 128 60x80
+// 54 / 45.  Weight gradient, N=2 256 50x84, fp32 MFMAs / triples: 107 / 70.  Errors against float64 (2-norm) there: grad_input
+// 2.9e-7 with fp32 MFMAs, 2.5e-7, 2.0e-7 pairs; grad_weight 3.3e-7 / 3.0e-7.
+// PLANES: 3, 2 (fp16 pairs, rows scaled by the powers of two ea and eb of the lane's), 0 (products of E itself).
+template <typename E, int TILE, int PLANES>
 __device__ __forceinline__ void tile_products(f32x16 (&acc)[TILE / 64][2], const uint4 *A, const uint4 *B, int wm, int wn,
-                                              int frow, int fhalf) {
+                                              int frow, int fhalf, const int (&ea)[TILE / 64], const int (&eb)[2]) {
   using TR = ElemTraits<E>;
   constexpr int MB = TILE / 64;
   // (the rows of a lane's fragments are multiples of 32 apart: one swizzle for all of them)
   const uint4 *a0 = A + (wm * (TILE / 2) + frow) * 8, *b0 = B + (wn * 64 + frow) * 8;
   auto load_a = [&](int mb, int ksub) { return a0[mb * 256 + ((ksub * 2 + fhalf) ^ (frow & 7))]; };
   auto load_b = [&](int nb, int ksub) { return b0[nb * 256 + ((ksub * 2 + fhalf) ^ (frow & 7))]; };
-  if constexpr (sizeof(E) == 2 || EXACT) {
+  if constexpr (sizeof(E) == 2 || PLANES == 0) {
 #pragma unroll
     for (int ksub = 0; ksub < 4; ++ksub) {
       uint4 af[MB], bf[2];
@@ -89,35 +96,46 @@ __device__ __forceinline__ void tile_products(f32x16 (&acc)[TILE / 64][2], const
         for (int nb = 0; nb < 2; ++nb) TR::mma(acc[mb][nb], af[mb], bf[nb]);
     }
   } else {
-    using TB = ElemTraits<bf16_t>;
-    // 8 values of K as three planes of an operand
-    auto split8 = [](const uint4 (&v)[2], uint4 (&p)[3]) {
-      uint2 lo[3], hi[3];
-      auto scaled = [](uint32_t x) { return __uint_as_float(x) * kSplitScale; };
-      split3({scaled(v[0].x), scaled(v[0].y), scaled(v[0].z), scaled(v[0].w)}, lo);
-      split3({scaled(v[1].x), scaled(v[1].y), scaled(v[1].z), scaled(v[1].w)}, hi);
+    using TB = ElemTraits<std::conditional_t<PLANES == 2, f16_t, bf16_t>>;
+    // 8 values of K as the planes of an operand
+    auto split8 = [](const uint4 (&v)[2], uint4 (&p)[PLANES], int e) {
+      uint2 lo[PLANES], hi[PLANES];
+      auto scaled = [&](uint32_t x) {
+        return PLANES == 2 ? __builtin_amdgcn_ldexpf(__uint_as_float(x), e) : __uint_as_float(x) * kSplitScale;
+      };
+      const float s0[4] = {scaled(v[0].x), scaled(v[0].y), scaled(v[0].z), scaled(v[0].w)};
+      const float s1[4] = {scaled(v[1].x), scaled(v[1].y), scaled(v[1].z), scaled(v[1].w)};
+      if constexpr (PLANES == 2) {
+        split2(s0, lo);
+        split2(s1, hi);
+      } else {
+        split3(s0, lo);
+        split3(s1, hi);
+      }
 #pragma unroll
-      for (int s = 0; s < 3; ++s) p[s] = make_uint4(lo[s].x, lo[s].y, hi[s].x, hi[s].y);
+      for (int s = 0; s < PLANES; ++s) p[s] = make_uint4(lo[s].x, lo[s].y, hi[s].x, hi[s].y);
     };
 #pragma unroll
     for (int half = 0; half < 2; ++half) {  // (any order of K will do: both operands have the same)
-      uint4 bp[2][3];
+      uint4 bp[2][PLANES];
 #pragma unroll
-      for (int nb = 0; nb < 2; ++nb) split8({load_b(nb, half * 2), load_b(nb, half * 2 + 1)}, bp[nb]);
+      for (int nb = 0; nb < 2; ++nb) split8({load_b(nb, half * 2), load_b(nb, half * 2 + 1)}, bp[nb], eb[nb]);
       uint4 af[2] = {load_a(0, half * 2), load_a(0, half * 2 + 1)};
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb) {
-        uint4 ap[3];
-        split8(af, ap);
+        uint4 ap[PLANES];
+        split8(af, ap, ea[mb]);
         if (mb + 1 < MB) af[0] = load_a(mb + 1, half * 2), af[1] = load_a(mb + 1, half * 2 + 1);
         __builtin_amdgcn_sched_barrier(0);  // (or every block's planes are made ahead and spilled)
         auto products = [&](int pa, int pb) {
 #pragma unroll
           for (int nb = 0; nb < 2; ++nb) TB::mma(acc[mb][nb], ap[pa], bp[nb][pb]);
         };
-        products(2, 0);  // smallest terms first
-        products(0, 2);
-        products(1, 1);
+        if constexpr (PLANES == 3) {
+          products(2, 0);  // smallest terms first
+          products(0, 2);
+          products(1, 1);
+        }
         products(1, 0);
         products(0, 1);
         products(0, 0);
@@ -150,7 +168,8 @@ __device__ __forceinline__ bool unscale(f32x16 (&acc)[MB][2]) {
 // conflict free), double buffered.  A rows = (tap, channel), B rows = pixels:
 // a lane ends up with 4 x 4 consecutive channels of one pixel, which is what the
 // d layout wants (16-byte stores).
-template <typename E, int TILE>
+// PAIRS: fp32 as fp16 pairs (see tile_products).
+template <typename E, int TILE, bool PAIRS>
 __global__ __launch_bounds__(TILE * 2, TILE == 128 ? 2 : 1) void bwd_colgrad_kernel(ColGradArgs a) {
   using TR = ElemTraits<E>;
   constexpr int ES = (int)sizeof(E);
@@ -199,9 +218,30 @@ __global__ __launch_bounds__(TILE * 2, TILE == 128 ? 2 : 1) void bwd_colgrad_ker
     }
   };
 
+  // pairs: exponents of the tile's rows of A, then of B
+  __shared__ __align__(16) int exps[PAIRS ? 2 * TILE : 4];
+  int ea[MB] = {}, eb[2] = {};
+  issue(0, 0);
+  if constexpr (PAIRS) {
+    const int row = tid & (TILE - 1);
+    const bool is_b = tid >= TILE;   // (wave uniform)
+    const uint16_t *src = is_b ? a.gmax + ((long)n * (a.Cout / KC) + (long)grp * a.kslabs) * a.P + min(pt * TILE + row, a.P - 1)
+                               : a.wmax + ((long)grp * a.M_pad + (long)mt * TILE + row) * a.kslabs;
+    const long step = is_b ? a.P : 1;
+    uint32_t top = 0;
+#pragma unroll 8
+    for (int s = 0; s < a.kslabs; ++s) top = max(top, (uint32_t)src[s * step]);
+    exps[tid] = pair_exponent(__uint_as_float(top << 16));
+    __syncthreads();
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) ea[mb] = exps[wm * (TILE / 2) + mb * 32 + frow];
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb) eb[nb] = exps[TILE + wn * 64 + nb * 32 + frow];
+  }
+
   f32x16 acc[MB][2];
-  auto sweep = [&](auto how) {
-    constexpr bool exact = decltype(how)::value;
+  auto sweep = [&](auto planes) {
+    constexpr int PLANES = decltype(planes)::value;
 #pragma unroll
     for (int i = 0; i < MB; ++i)
 #pragma unroll
@@ -209,7 +249,6 @@ __global__ __launch_bounds__(TILE * 2, TILE == 128 ? 2 : 1) void bwd_colgrad_ker
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
-    issue(0, 0);
     for (int ks = 0; ks < a.kslabs; ++ks) {
       const int buf = ks & 1;
       if (ks + 1 < a.kslabs) {
@@ -219,13 +258,38 @@ __global__ __launch_bounds__(TILE * 2, TILE == 128 ? 2 : 1) void bwd_colgrad_ker
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       }
       __syncthreads();
-      tile_products<E, TILE, exact>(acc, As[buf], Bs[buf], wm, wn, frow, fhalf);
+      tile_products<E, TILE, PLANES>(acc, As[buf], Bs[buf], wm, wn, frow, fhalf, ea, eb);
       __syncthreads();
     }
   };
-  sweep(std::false_type());
+  sweep(std::integral_constant<int, PAIRS ? 2 : 3>());
   if constexpr (sizeof(E) == 4) {
-    if (__syncthreads_or(unscale(acc))) sweep(std::true_type());
+    bool bad;
+    if constexpr (PAIRS) {
+      float t = 0.0f;
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int4 e4 = *(const int4 *)&exps[wm * (TILE / 2) + mb * 32 + j * 8 + fhalf * 4];
+          const int e[4] = {e4.x, e4.y, e4.z, e4.w};
+#pragma unroll
+          for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const float c = __builtin_amdgcn_ldexpf(acc[mb][nb][j * 4 + i], -(e[i] + eb[nb]));
+              acc[mb][nb][j * 4 + i] = c;
+              t = fmaf(c, 0.0f, t);
+            }
+        }
+      bad = t != t;
+    } else {
+      bad = unscale(acc);
+    }
+    if (__syncthreads_or(bad)) {
+      issue(0, 0);
+      sweep(std::integral_constant<int, 0>());
+    }
   }
 
   // register r of lane l: A row (r/4)*8 + (l/32)*4 + r%4 of the block, B row l%32
@@ -863,8 +927,9 @@ __global__ __launch_bounds__(TILE * 2, TILE == 128 ? 2 : 1) void bwd_wgrad_kerne
   const long per = (work + a.splits - 1) / a.splits;
   const long w_begin = (long)split * per, w_end = min(work, w_begin + per);
   f32x16 acc[MB][2];
-  auto sweep = [&](auto how) {
-    constexpr bool exact = decltype(how)::value;
+  const int unused[MB] = {}, unused2[2] = {};
+  auto sweep = [&](auto planes) {
+    constexpr int PLANES = decltype(planes)::value;
 #pragma unroll
     for (int i = 0; i < MB; ++i)
 #pragma unroll
@@ -886,14 +951,14 @@ __global__ __launch_bounds__(TILE * 2, TILE == 128 ? 2 : 1) void bwd_wgrad_kerne
         if constexpr (sizeof(E) == 2)
           tile_products_tr<E, TILE, RUN>(acc, As[buf], Bs[buf], wm, wn, lane);
         else
-          tile_products<E, TILE, exact>(acc, As[buf], Bs[buf], wm, wn, frow, fhalf);
+          tile_products<E, TILE, PLANES>(acc, As[buf], Bs[buf], wm, wn, frow, fhalf, unused, unused2);
         __syncthreads();
       }
     }
   };
-  sweep(std::false_type());
+  sweep(std::integral_constant<int, 3>());
   if constexpr (sizeof(E) == 4) {
-    if (__syncthreads_or(unscale(acc))) sweep(std::true_type());
+    if (__syncthreads_or(unscale(acc))) sweep(std::integral_constant<int, 0>());
   }
 
   // register r of lane l: A row (output channel) (r/4)*8 + (l/32)*4 + r%4 of the block, B row (column row) l%32

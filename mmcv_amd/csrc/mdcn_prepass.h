@@ -131,7 +131,7 @@ __device__ __forceinline__ void relayout_vec_block(const Geom &g, const E *__res
         for (int i = 0; i < 4; ++i) ow[i * 4 + j] = rw[j * 4 + i];
     }
   }
-  if constexpr (sizeof(E) == 4 && BORDER && REC == 128 && !MAPPED) {
+  if constexpr (sizeof(E) == 4 && REC == 128 && BORDER != MAPPED) {
     if (row_max) {
       uint32_t top[EPV];
 #pragma unroll
