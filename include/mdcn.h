@@ -289,9 +289,9 @@ typedef struct mdcn_bwd_params {
  * tensors and, for shapes whose column gradient runs on the matrix cores,
  * pixel-major copies of input and grad_output, the transposed weights and the
  * column gradient of up to 1.5 GiB of images at a time; may be 0.
- * For fp32 the figure ends with a region that may be left out: magnitudes for a
+ * For fp32 and more than 64 output channels a group the figure ends with a region that may be left out: magnitudes for a
  * column gradient made of fp16 pairs (2 bytes per output pixel and 32 channels of
- * grad_output, and per row of weights); without it it is made of bf16 triples, which is slower.
+ * grad_output, 4 per row of weights); without it it is made of bf16 triples, which is slower.
  * conv.path: MDCN_PATH_AUTO picks by shape and size; MDCN_PATH_FUSED asks for
  * the tiled kernels whatever the problem size (MDCN_ERR_PATH if the shape rules
  * them out); MDCN_PATH_DIRECT keeps the one-workgroup-per-tap kernel. */

@@ -67,7 +67,7 @@ void make_bwd_plan(const mdcn_bwd_params *bp, const Geom &g, uint64_t pass_bytes
   pl->w_tile = kCgTile;
   pl->w_splits = 1;
   pl->gpad_bytes = 0;
-  pl->gmax_bytes = pl->wmax_bytes = pl->max_at = 0;
+  pl->gmax_bytes = pl->wexp_bytes = pl->max_at = 0;
   pl->bsplits = 0;
   pl->im = pl->om = ChanMap{1, 1, 1, 1, 1};
   pl->parts = 1;
@@ -193,6 +193,8 @@ void make_bwd_plan(const mdcn_bwd_params *bp, const Geom &g, uint64_t pass_bytes
     // 2 283, 0.93 (N=4 100x152) 2 028 / 2 011, 0.97 (N=6 100x152) 2 922 / 2 994, 1 (N=16 64x64) 2 014 / 2 020;
     // fp32 512 channels, 16: 0.75 (N=8 32x32) 915 / 891, 0.90 (N=16 32x32) 1 614 / 1 626, 0.94 (N=10 32x32, 720 tiles) 1 093 / 1 120, 0.90 (N=4
     // 64x64) 1 630 / 1 647, 0.93 (N=8 50x84) 3 487 / 3 566, 0.95 (N=6 48x48) 1 596 / 1 625;
+    // (triples; with pairs, of all calls of more than 128 tiles of 256, by this rule: N=8 256 64x64 872 / 863, N=8 512 32x32 709 / 695, N=3 512 25x42 479 / 450, N=4 256 50x84 605 / 594,
+    // N=16 128 100x152 2 721 / 2 751.)
     // 16 bits: N=4 96 -> 72 37x53 (128 tiles) 113 / 110; N=4 240 60x60 (540) 336 / 331; N=8 104 -> 96 100x100 (1 280) 713 / 720; N=8 312 -> 300
     // 90x100 (3 168) 2 092 / 2 133.
     auto tiles_of = [&](long tile) {
@@ -210,7 +212,7 @@ void make_bwd_plan(const mdcn_bwd_params *bp, const Geom &g, uint64_t pass_bytes
     // float64, triples / pairs: 64 output channels 1.23e-7 / 1.26e-7, 72 1.43e-7 / 1.37e-7, 256 2.49e-7 / 1.99e-7, 512 3.57e-7 / 2.66e-7).
     if (es == 4 && om.cgp > 64) {
       pl->gmax_bytes = align_up((size_t)g.N * g.G * (om.cgp / KC) * plane_out * 2);
-      pl->wmax_bytes = align_up((size_t)g.G * pl->M_pad * (om.cgp / KC) * 2);
+      pl->wexp_bytes = align_up((size_t)g.G * pl->M_pad * 4);
     }
     if (pl->fused)
       pl->part_bytes = align_up((size_t)((g.N + pl->n_chunk - 1) / pl->n_chunk) * FusedSchedule::kGroups * 3 * g.taps * 256 * 4);
@@ -385,7 +387,7 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
   float *wpart = (float *)take(pl.wpart_bytes);
   unsigned char *gpad = take(pl.gpad_bytes);
   uint16_t *gmax = pl.max_at ? (uint16_t *)((unsigned char *)p->workspace + pl.max_at) : nullptr;
-  uint16_t *wmax = pl.max_at ? (uint16_t *)((unsigned char *)p->workspace + pl.max_at + pl.gmax_bytes) : nullptr;
+  int *wexp = pl.max_at ? (int *)((unsigned char *)p->workspace + pl.max_at + pl.gmax_bytes) : nullptr;
   const long n_in = (long)g.N * g.Cin * g.H * g.W;
 
   // a sample of the offsets, 64 Ki of them at most, decides which window the scatter kernel uses
@@ -421,7 +423,7 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
     a.gT = gT;
     a.wT = wT;
     a.gmax = gmax;
-    a.wmax = wmax;
+    a.wexp = wexp;
     a.gpad = gpad;
     a.col = col;
     a.gin32 = gin32;
@@ -454,7 +456,7 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
         pl.gpad_bytes ? up((long)g.N * g.Cout * (pl.P_pad / EPV), 256) : 0,
         gemm ? up(n_in, kPreZeroPerBlock) : 0,
         wgemm && pl.P_pad > plane_out ? up(a.col_rows * (pl.P_pad - plane_out), kPrePadPerBlock) : 0,
-        gemm ? up((long)g.G * pl.M_pad * pl.om.cgp, 256) : 0,
+        gemm ? wexp ? up((long)g.G * pl.M_pad, kPrePairRows) : up((long)g.G * pl.M_pad * pl.om.cgp, 256) : 0,
         gemm && pl.fWH ? far_blocks : 0,
         early ? 0 : bias_blocks,
     };
@@ -470,7 +472,7 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
       ca.wT = wT;
       ca.gT = gT;
       ca.gmax = gmax;
-      ca.wmax = wmax;
+      ca.wexp = wexp;
       ca.D = (float *)D;
       ca.P = (int)plane_out;
       ca.px_tiles = (int)((plane_out + pl.cg_tile - 1) / pl.cg_tile);

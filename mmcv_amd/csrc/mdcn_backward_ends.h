@@ -21,7 +21,8 @@ struct BwdPreArgs {
   int end[kPreJobs];       // job j has the blocks from end[j - 1] on
   const void *in, *gout, *w;
   void *xt, *gT, *wT, *gpad, *col;
-  uint16_t *gmax, *wmax;   // fp32, or null: see ColGradArgs
+  uint16_t *gmax;          // fp32 as fp16 pairs, or null: see ColGradArgs
+  int *wexp;
   float *gin32;
   long n_in;               // elements of gin32
   int x_chunks, g_chunks;  // pixel chunks of the re-layouts
@@ -38,8 +39,68 @@ struct BwdPreArgs {
   int bsplits;
 };
 
+constexpr int kPrePairRows = 8;              // rows of wT a block writes as fp16 pairs
 constexpr int kPreZeroPerBlock = 256 * 32;   // floats a block of the zero job clears
 constexpr int kPrePadPerBlock = 256 * 8;     // elements a block of the col-pad job clears
+
+// fp32 as fp16 pairs: rows of wT scaled by a power of two that goes by the largest finite number of each, and split.  The 32 values of a slab are four
+// times eight, which a lane of the product takes at a time: the first halves of eight in one 16-byte piece, the second ones in the piece two behind
+// it.  32 lanes a row, eight output channels each.
+__device__ __forceinline__ void pack_weight_row_pairs(const BwdPreArgs &a, int b) {
+  const Geom &g = a.g;
+  const int lane = threadIdx.x & 31;
+  const long row = (long)b * kPrePairRows + ((int)threadIdx.x >> 5);
+  if (row >= (long)g.G * a.M_pad) return;
+  const int grp = (int)(row / a.M_pad), m = (int)(row - (long)grp * a.M_pad);
+  const int tap = m / a.im.cgp;
+  int room;
+  const int c = chan_source(a.im, m - tap * a.im.cgp, room);  // (of the first group: channel within a group)
+  const bool there = tap < g.taps && room > 0;
+  const long pitch = (long)g.cin_g * g.taps;
+  const float *src = (const float *)a.w + (long)grp * g.cout_g * pitch + (long)c * g.taps + tap;
+  const int eights = a.om.cgp / 8;
+  // values j of eight number o: of pieces q and q + 2 of their slab
+  auto load = [&](int o, float (&v)[8]) {
+    const int q = (o >> 1 & 1) * 4 + (o & 1), co0 = (o >> 2) * 32 + q * 4;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int co = co0 + (j & 3) + (j >> 2) * 8;
+      v[j] = there && o < eights && co < g.cout_g ? src[co * pitch] : 0.0f;
+    }
+  };
+  float first[8], v[8];
+  uint32_t top = 0u;
+  auto largest = [&](const float (&x)[8]) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const uint32_t t = __float_as_uint(x[j]) & 0x7fffffffu;
+      top = max(top, t < 0x7f800000u ? t : 0u);
+    }
+  };
+  load(lane, first);
+  largest(first);
+  for (int o = lane + 32; o < eights; o += 32) {
+    load(o, v);
+    largest(v);
+  }
+#pragma unroll
+  for (int s = 16; s; s >>= 1) top = max(top, (uint32_t)__shfl_xor((int)top, s));
+  const int e = pair_exponent(__uint_as_float(top));
+  if (lane == 0) a.wexp[row] = e;
+  uint4 *dst = (uint4 *)a.wT + row * (a.om.cgp / 4);
+  for (int o = lane; o < eights; o += 32) {
+    if (o != lane) load(o, v);
+    float x[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] = __builtin_amdgcn_ldexpf(o == lane ? first[j] : v[j], e);
+    uint2 lo[2], hi[2];
+    split2({x[0], x[1], x[2], x[3]}, lo);
+    split2({x[4], x[5], x[6], x[7]}, hi);
+    uint4 *d = dst + (o >> 2) * 8 + (o >> 1 & 1) * 4 + (o & 1);
+    d[0] = make_uint4(lo[0].x, lo[0].y, hi[0].x, hi[0].y);
+    d[2] = make_uint4(lo[1].x, lo[1].y, hi[1].x, hi[1].y);
+  }
+}
 
 template <typename E>
 __global__ __launch_bounds__(256) void bwd_prepass_kernel(BwdPreArgs a) {
@@ -137,6 +198,12 @@ __global__ __launch_bounds__(256) void bwd_prepass_kernel(BwdPreArgs a) {
     // either channel is padding and in the rows up to M_pad.  With wt_run it is [G][run][M_pad][wt_run], the last run what is left: what
     // bwd_fused_kernel copies at a time is one piece of memory for a tap (256 bytes of rows 1 KB apart, as with
     // 512 output channels, are in one of four channels of the L2).
+    if constexpr (sizeof(E) == 4) {
+      if (a.wexp) {
+        pack_weight_row_pairs(a, b - a.end[kPreColPad]);
+        return;
+      }
+    }
     const long total = (long)g.G * a.M_pad * a.om.cgp;
     const long idx = (long)(b - a.end[kPreColPad]) * 256 + tid;
     if (idx >= total) return;
@@ -151,14 +218,6 @@ __global__ __launch_bounds__(256) void bwd_prepass_kernel(BwdPreArgs a) {
     E v = from_f32<E>(0.0f);
     if (tap < g.taps && room > 0 && co < g.cout_g)
       v = ((const E *)a.w)[((long)(grp * g.cout_g + co) * g.cin_g + c) * g.taps + tap];
-    if constexpr (sizeof(E) == 4) {
-      if (a.wmax) {   // (32 neighbouring lanes have 32 output channels of a row)
-        int top = (int)(__float_as_uint(v) & 0x7fffffffu);
-#pragma unroll
-        for (int s = 16; s; s >>= 1) top = max(top, __shfl_xor(top, s));
-        if ((tid & 31) == 0) a.wmax[idx >> 5] = (uint16_t)((min((uint32_t)top, 0x7f800000u) + 0xffffu) >> 16);
-      }
-    }
     long at = idx;
     if (a.wt_run) {
       const int run = co / a.wt_run, len = min(a.wt_run, a.om.cgp - run * a.wt_run);

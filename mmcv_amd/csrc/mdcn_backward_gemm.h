@@ -46,9 +46,9 @@ struct ColGradArgs {
   // (channel counts are those of the padded orders, see BwdPlan)
   const void *wT;  // [G][M_pad][cout_g]
   const void *gT;  // [N][Cout / KC][P][KC], KC = 128 bytes of channels
-  // fp32 as fp16 pairs: the largest magnitude of each 128 bytes of either, as relayout_vec_block's row_max
-  const uint16_t *wmax;  // [G][M_pad][cout_g / KC]
-  const uint16_t *gmax;  // [N][Cout / KC][P]
+  // fp32 as fp16 pairs: wT holds them already (pack_weight_row_pairs), with these exponents of its rows, [G][M_pad]; and the largest
+  const int *wexp;
+  const uint16_t *gmax;  // magnitude of each 128 bytes of gT, as relayout_vec_block's row_max, [N][Cout / KC][P]
   float *D;        // [images of the pass][Cin / 16][taps][P][16]
   int P;           // output pixels per image
   int px_tiles, m_tiles;
@@ -65,15 +65,18 @@ struct ColGradArgs {
 // fp32 runs on the 16-bit matrix pipe, as in fused_f32_kernel, with an error that is that of fp32 arithmetic: of bf16 triples (six of the nine products
 // of three planes; the weight gradient, whose rows have no exponents at hand) or of fp16 pairs (three products of two planes; the column
 // gradient of more than 64 output channels).  Pairs are scaled row by row: a pixel's channels of grad_output and a weight row's output
-// channels by the largest of them, which the pre-pass writes beside its copies.  Operands are split behind the LDS reads, every wave for itself: beside
-// 48 bf16 MFMAs of 32 clocks per 16 of K, or 24 fp16 ones, some 290 VALU instructions, which is what pairs are bound by.  An infinity, or a number that the
+// channels by the largest of them.  The weights are split by the pre-pass, a row at a time; for grad_output it writes the largest of each 128 bytes
+// beside its copy.  What is not split before is split behind the LDS reads, every wave for itself: some 290 VALU instructions per 16 of K for triples,
+// beside 48 MFMAs of 32 clocks, a third of that for pairs in tiles of 256, half in tiles of 128, beside 24.  An infinity, or a number that the
 // scale takes to one (kSplitScale), leaves NaN in the planes and so in the sums: a workgroup
 // that finds any goes over its K range again with fp32 MFMAs (PLANES = 0).
-// Column gradient in us, triples / pairs: N=2 256 -> 256 50x84 78 / 57 (fp32 MFMAs 151), N=8 64x64 279 / 202, N=4 512 64x64 484 / 338 (tiles of 256), N=4 128 60x80
-// 54 / 45.  Weight gradient, N=2 256 50x84, fp32 MFMAs / triples: 107 / 70.  Errors against float64 (2-norm) there: grad_input
+// Column gradient in us, triples / pairs split behind the reads / weights split before: N=8 256 -> 256 64x64 279 / 202 / 188, N=4 512 64x64 484 / 338 / 300 (tiles of
+// 256), N=4 128 60x80 54 / 45 / 43; whole training calls, pairs, weights split behind the reads / before: N=1 512 25x42 235 / 223, N=8 512 13x21 332 / 317, N=4 512 64x64 1 308 / 1 275.
+// Weight gradient, N=2 256 50x84, fp32 MFMAs / triples: 107 / 70.  Errors against float64 (2-norm) there: grad_input
 // 2.9e-7 with fp32 MFMAs, 2.5e-7, 2.0e-7 pairs; grad_weight 3.3e-7 / 3.0e-7.
 // PLANES: 3, 2 (fp16 pairs, rows scaled by the powers of two ea and eb of the lane's), 0 (products of E itself).
-template <typename E, int TILE, int PLANES>
+// SPLIT_A: A holds fp16 pairs (pack_weight_row_pairs).
+template <typename E, int TILE, int PLANES, bool SPLIT_A = false>
 __device__ __forceinline__ void tile_products(f32x16 (&acc)[TILE / 64][2], const uint4 *A, const uint4 *B, int wm, int wn,
                                               int frow, int fhalf, const int (&ea)[TILE / 64], const int (&eb)[2]) {
   using TR = ElemTraits<E>;
@@ -87,7 +90,26 @@ __device__ __forceinline__ void tile_products(f32x16 (&acc)[TILE / 64][2], const
     for (int ksub = 0; ksub < 4; ++ksub) {
       uint4 af[MB], bf[2];
 #pragma unroll
-      for (int mb = 0; mb < MB; ++mb) af[mb] = load_a(mb, ksub);
+      for (int mb = 0; mb < MB; ++mb) {
+        if constexpr (SPLIT_A) {
+          const uint4 h4 = load_a(mb, ksub & 2), l4 = load_a(mb, ksub | 1);
+          const uint32_t hw[2] = {ksub & 1 ? h4.z : h4.x, ksub & 1 ? h4.w : h4.y}, lw[2] = {ksub & 1 ? l4.z : l4.x, ksub & 1 ? l4.w : l4.y};
+          uint32_t x[4];
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            const f16x2 h = __builtin_bit_cast(f16x2, hw[i]), l = __builtin_bit_cast(f16x2, lw[i]);
+            // (what is left of an infinity is NaN)
+            auto whole = [&](f16_t hi, f16_t lo) {
+              const float f = (float)hi;
+              return __float_as_uint(fabsf(f) <= 65504.0f ? __builtin_amdgcn_ldexpf(f + (float)lo, -ea[mb]) : f);
+            };
+            x[2 * i] = whole(h.x, l.x), x[2 * i + 1] = whole(h.y, l.y);
+          }
+          af[mb] = make_uint4(x[0], x[1], x[2], x[3]);
+        } else {
+          af[mb] = load_a(mb, ksub);
+        }
+      }
 #pragma unroll
       for (int nb = 0; nb < 2; ++nb) bf[nb] = load_b(nb, ksub);
 #pragma unroll
@@ -124,7 +146,8 @@ __device__ __forceinline__ void tile_products(f32x16 (&acc)[TILE / 64][2], const
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb) {
         uint4 ap[PLANES];
-        split8(af, ap, ea[mb]);
+        if constexpr (SPLIT_A) ap[0] = af[0], ap[1] = af[1];
+        else split8(af, ap, ea[mb]);
         if (mb + 1 < MB) af[0] = load_a(mb + 1, half * 2), af[1] = load_a(mb + 1, half * 2 + 1);
         __builtin_amdgcn_sched_barrier(0);  // (or every block's planes are made ahead and spilled)
         auto products = [&](int pa, int pb) {
@@ -224,14 +247,15 @@ __global__ __launch_bounds__(TILE * 2, TILE == 128 ? 2 : 1) void bwd_colgrad_ker
   issue(0, 0);
   if constexpr (PAIRS) {
     const int row = tid & (TILE - 1);
-    const bool is_b = tid >= TILE;   // (wave uniform)
-    const uint16_t *src = is_b ? a.gmax + ((long)n * (a.Cout / KC) + (long)grp * a.kslabs) * a.P + min(pt * TILE + row, a.P - 1)
-                               : a.wmax + ((long)grp * a.M_pad + (long)mt * TILE + row) * a.kslabs;
-    const long step = is_b ? a.P : 1;
-    uint32_t top = 0;
+    if (tid < TILE) {
+      exps[tid] = a.wexp[(long)grp * a.M_pad + (long)mt * TILE + row];
+    } else {
+      const uint16_t *src = a.gmax + ((long)n * (a.Cout / KC) + (long)grp * a.kslabs) * a.P + min(pt * TILE + row, a.P - 1);
+      uint32_t top = 0;
 #pragma unroll 8
-    for (int s = 0; s < a.kslabs; ++s) top = max(top, (uint32_t)src[s * step]);
-    exps[tid] = pair_exponent(__uint_as_float(top << 16));
+      for (int s = 0; s < a.kslabs; ++s) top = max(top, (uint32_t)src[(long)s * a.P]);
+      exps[tid] = pair_exponent(__uint_as_float(top << 16));
+    }
     __syncthreads();
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) ea[mb] = exps[wm * (TILE / 2) + mb * 32 + frow];
@@ -258,7 +282,7 @@ __global__ __launch_bounds__(TILE * 2, TILE == 128 ? 2 : 1) void bwd_colgrad_ker
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       }
       __syncthreads();
-      tile_products<E, TILE, PLANES>(acc, As[buf], Bs[buf], wm, wn, frow, fhalf, ea, eb);
+      tile_products<E, TILE, PLANES, PAIRS>(acc, As[buf], Bs[buf], wm, wn, frow, fhalf, ea, eb);
       __syncthreads();
     }
   };

@@ -62,10 +62,8 @@ def test_error_is_that_of_fp32(shape):
     assert by_pixel <= 2 * ((K + C) ** 0.5 + 4) * 2.0 ** -24 * (16 if few < 10 else 8), by_pixel
 
 
-def test_without_room_for_magnitudes():
-    """A workspace that ends in front of them gives the same call as bf16 triples, a smaller one is refused."""
-    dev, go = _case(8, 2, 64, 128, 33, 37)
-    y = capi_backward(dev, go, path=capi.PATH_FUSED)[0]
+def _as_triples(dev, go):
+    """The gradients of input, offset and mask with a workspace that ends in front of the magnitudes."""
     lib = capi.load()
     bp = capi.MdcnBwdParams()
     bp.conv = capi.make_params(capi.MDCN_F32, 2, 64, 33, 37, 128, 3, 3, (1, 1), (1, 1), (1, 1), 1, 1)
@@ -76,13 +74,36 @@ def test_without_room_for_magnitudes():
     bp.grad_output = go.data_ptr()
     bp.grad_input, bp.grad_offset, bp.grad_mask = (t.data_ptr() for t in out)
     up = lambda v: (v + 255) // 256 * 256
-    need = lib.mdcn_backward_workspace_bytes(ctypes.byref(bp)) - up(2 * 4 * 33 * 37 * 2) - up(640 * 4 * 2)
+    need = lib.mdcn_backward_workspace_bytes(ctypes.byref(bp)) - up(2 * 4 * 33 * 37 * 2) - up(640 * 4)
     ws = torch.empty(need, dtype=torch.uint8, device='cuda')
     p.workspace, p.workspace_bytes = ws.data_ptr(), need
     stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
     assert lib.mdcn_backward(ctypes.byref(bp), stream) == 0
     torch.cuda.synchronize()
-    assert not torch.equal(out[0], y)
-    assert float((out[0] - y).norm() / y.norm()) <= 2 * (128 ** 0.5 + 4) * 2.0 ** -24
     p.workspace_bytes = need - 256
     assert lib.mdcn_backward(ctypes.byref(bp), stream) == -4
+    return out
+
+
+def test_without_room_for_magnitudes():
+    """Such a workspace gives the same call as bf16 triples, a smaller one is refused."""
+    dev, go = _case(8, 2, 64, 128, 33, 37)
+    y = capi_backward(dev, go, path=capi.PATH_FUSED)[0]
+    gin = _as_triples(dev, go)[0]
+    assert not torch.equal(gin, y)
+    assert float((gin - y).norm() / y.norm()) <= 2 * (128 ** 0.5 + 4) * 2.0 ** -24
+
+
+@pytest.mark.parametrize('where', ['weight', 'grad_output'])
+@pytest.mark.parametrize('value', [float('inf'), float('nan'), 3e38])
+def test_not_finite(where, value):
+    """One number that fp16 pairs cannot hold, or whose row overflows: what is finite, and its value, as with bf16 triples."""
+    print(f'case={where} {value}', flush=True)
+    dev, go = _case(9, 2, 64, 128, 33, 37)
+    dev['weight'][:, 7] *= 1e6   # a row whose other numbers fp16 does not hold unscaled
+    (dev['weight'] if where == 'weight' else go)[1, 7, 1, 1] = value
+    for y, ref in zip(capi_backward(dev, go, path=capi.PATH_FUSED)[:3], _as_triples(dev, go)):
+        assert torch.equal(y.isnan(), ref.isnan()) and torch.equal(y.isinf(), ref.isinf())
+        ok = ref.isfinite()
+        d, r = (y - ref)[ok].double(), ref[ok].double()
+        assert float(d.norm() / r.norm()) <= 4 * (128 ** 0.5 + 4) * 2.0 ** -24
