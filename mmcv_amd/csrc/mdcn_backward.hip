@@ -67,7 +67,7 @@ void make_bwd_plan(const mdcn_bwd_params *bp, const Geom &g, uint64_t pass_bytes
   pl->w_tile = kCgTile;
   pl->w_splits = 1;
   pl->gpad_bytes = 0;
-  pl->gmax_bytes = pl->wexp_bytes = pl->max_at = 0;
+  pl->gmax_bytes = pl->wexp_bytes = pl->wpair_bytes = pl->max_at = 0;
   pl->bsplits = 0;
   pl->im = pl->om = ChanMap{1, 1, 1, 1, 1};
   pl->parts = 1;
@@ -213,6 +213,7 @@ void make_bwd_plan(const mdcn_bwd_params *bp, const Geom &g, uint64_t pass_bytes
     if (es == 4 && om.cgp > 64) {
       pl->gmax_bytes = align_up((size_t)g.N * g.G * (om.cgp / KC) * plane_out * 2);
       pl->wexp_bytes = align_up((size_t)g.G * pl->M_pad * 4);
+      pl->wpair_bytes = pl->wt_bytes;
     }
     if (pl->fused)
       pl->part_bytes = align_up((size_t)((g.N + pl->n_chunk - 1) / pl->n_chunk) * FusedSchedule::kGroups * 3 * g.taps * 256 * 4);
@@ -388,6 +389,7 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
   unsigned char *gpad = take(pl.gpad_bytes);
   uint16_t *gmax = pl.max_at ? (uint16_t *)((unsigned char *)p->workspace + pl.max_at) : nullptr;
   int *wexp = pl.max_at ? (int *)((unsigned char *)p->workspace + pl.max_at + pl.gmax_bytes) : nullptr;
+  void *wpair = (unsigned char *)wexp + pl.wexp_bytes;
   const long n_in = (long)g.N * g.Cin * g.H * g.W;
 
   // a sample of the offsets, 64 Ki of them at most, decides which window the scatter kernel uses
@@ -424,6 +426,7 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
     a.wT = wT;
     a.gmax = gmax;
     a.wexp = wexp;
+    a.wpair = wpair;
     a.gpad = gpad;
     a.col = col;
     a.gin32 = gin32;
@@ -456,7 +459,7 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
         pl.gpad_bytes ? up((long)g.N * g.Cout * (pl.P_pad / EPV), 256) : 0,
         gemm ? up(n_in, kPreZeroPerBlock) : 0,
         wgemm && pl.P_pad > plane_out ? up(a.col_rows * (pl.P_pad - plane_out), kPrePadPerBlock) : 0,
-        gemm ? wexp ? up((long)g.G * pl.M_pad, kPrePairRows) : up((long)g.G * pl.M_pad * pl.om.cgp, 256) : 0,
+        gemm ? up((long)g.G * pl.M_pad * pl.om.cgp, 256) + (wexp ? up((long)g.G * pl.M_pad, kPrePairRows) : 0) : 0,
         gemm && pl.fWH ? far_blocks : 0,
         early ? 0 : bias_blocks,
     };
@@ -473,6 +476,7 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
       ca.gT = gT;
       ca.gmax = gmax;
       ca.wexp = wexp;
+      ca.wpair = wpair;
       ca.D = (float *)D;
       ca.P = (int)plane_out;
       ca.px_tiles = (int)((plane_out + pl.cg_tile - 1) / pl.cg_tile);

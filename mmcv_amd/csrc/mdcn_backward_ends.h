@@ -23,6 +23,7 @@ struct BwdPreArgs {
   void *xt, *gT, *wT, *gpad, *col;
   uint16_t *gmax;          // fp32 as fp16 pairs, or null: see ColGradArgs
   int *wexp;
+  void *wpair;
   float *gin32;
   long n_in;               // elements of gin32
   int x_chunks, g_chunks;  // pixel chunks of the re-layouts
@@ -43,7 +44,7 @@ constexpr int kPrePairRows = 8;              // rows of wT a block writes as fp1
 constexpr int kPreZeroPerBlock = 256 * 32;   // floats a block of the zero job clears
 constexpr int kPrePadPerBlock = 256 * 8;     // elements a block of the col-pad job clears
 
-// fp32 as fp16 pairs: rows of wT scaled by a power of two that goes by the largest finite number of each, and split.  The 32 values of a slab are four
+// fp32 as fp16 pairs: wpair is wT, its rows scaled by a power of two that goes by the largest finite number of each, and split.  The 32 values of a slab are four
 // times eight, which a lane of the product takes at a time: the first halves of eight in one 16-byte piece, the second ones in the piece two behind
 // it.  32 lanes a row, eight output channels each.
 __device__ __forceinline__ void pack_weight_row_pairs(const BwdPreArgs &a, int b) {
@@ -87,7 +88,7 @@ __device__ __forceinline__ void pack_weight_row_pairs(const BwdPreArgs &a, int b
   for (int s = 16; s; s >>= 1) top = max(top, (uint32_t)__shfl_xor((int)top, s));
   const int e = pair_exponent(__uint_as_float(top));
   if (lane == 0) a.wexp[row] = e;
-  uint4 *dst = (uint4 *)a.wT + row * (a.om.cgp / 4);
+  uint4 *dst = (uint4 *)a.wpair + row * (a.om.cgp / 4);
   for (int o = lane; o < eights; o += 32) {
     if (o != lane) load(o, v);
     float x[8];
@@ -198,13 +199,14 @@ __global__ __launch_bounds__(256) void bwd_prepass_kernel(BwdPreArgs a) {
     // either channel is padding and in the rows up to M_pad.  With wt_run it is [G][run][M_pad][wt_run], the last run what is left: what
     // bwd_fused_kernel copies at a time is one piece of memory for a tap (256 bytes of rows 1 KB apart, as with
     // 512 output channels, are in one of four channels of the L2).
+    const long total = (long)g.G * a.M_pad * a.om.cgp;
     if constexpr (sizeof(E) == 4) {
-      if (a.wexp) {
-        pack_weight_row_pairs(a, b - a.end[kPreColPad]);
+      const int pairs_from = a.end[kPreColPad] + (int)((total + 255) / 256);
+      if (a.wexp && b >= pairs_from) {
+        pack_weight_row_pairs(a, b - pairs_from);
         return;
       }
     }
-    const long total = (long)g.G * a.M_pad * a.om.cgp;
     const long idx = (long)(b - a.end[kPreColPad]) * 256 + tid;
     if (idx >= total) return;
     long r = idx;

@@ -46,7 +46,8 @@ struct ColGradArgs {
   // (channel counts are those of the padded orders, see BwdPlan)
   const void *wT;  // [G][M_pad][cout_g]
   const void *gT;  // [N][Cout / KC][P][KC], KC = 128 bytes of channels
-  // fp32 as fp16 pairs: wT holds them already (pack_weight_row_pairs), with these exponents of its rows, [G][M_pad]; and the largest
+  // fp32 as fp16 pairs: those of wT (pack_weight_row_pairs), exponents of its rows, [G][M_pad], and the largest
+  const void *wpair;
   const int *wexp;
   const uint16_t *gmax;  // magnitude of each 128 bytes of gT, as relayout_vec_block's row_max, [N][Cout / KC][P]
   float *D;        // [images of the pass][Cin / 16][taps][P][16]
@@ -65,7 +66,7 @@ struct ColGradArgs {
 // fp32 runs on the 16-bit matrix pipe, as in fused_f32_kernel, with an error that is that of fp32 arithmetic: of bf16 triples (six of the nine products
 // of three planes; the weight gradient, whose rows have no exponents at hand) or of fp16 pairs (three products of two planes; the column
 // gradient of more than 64 output channels).  Pairs are scaled row by row: a pixel's channels of grad_output and a weight row's output
-// channels by the largest of them.  The weights are split by the pre-pass, a row at a time; for grad_output it writes the largest of each 128 bytes
+// channels by the largest of them.  The weights are split by the pre-pass, a row at a time, beside wT, which the fp32 sweep reads; for grad_output it writes the largest of each 128 bytes
 // beside its copy.  What is not split before is split behind the LDS reads, every wave for itself: some 290 VALU instructions per 16 of K for triples,
 // beside 48 MFMAs of 32 clocks, a third of that for pairs in tiles of 256, half in tiles of 128, beside 24.  An infinity, or a number that the
 // scale takes to one (kSplitScale), leaves NaN in the planes and so in the sums: a workgroup
@@ -90,26 +91,7 @@ __device__ __forceinline__ void tile_products(f32x16 (&acc)[TILE / 64][2], const
     for (int ksub = 0; ksub < 4; ++ksub) {
       uint4 af[MB], bf[2];
 #pragma unroll
-      for (int mb = 0; mb < MB; ++mb) {
-        if constexpr (SPLIT_A) {
-          const uint4 h4 = load_a(mb, ksub & 2), l4 = load_a(mb, ksub | 1);
-          const uint32_t hw[2] = {ksub & 1 ? h4.z : h4.x, ksub & 1 ? h4.w : h4.y}, lw[2] = {ksub & 1 ? l4.z : l4.x, ksub & 1 ? l4.w : l4.y};
-          uint32_t x[4];
-#pragma unroll
-          for (int i = 0; i < 2; ++i) {
-            const f16x2 h = __builtin_bit_cast(f16x2, hw[i]), l = __builtin_bit_cast(f16x2, lw[i]);
-            // (what is left of an infinity is NaN)
-            auto whole = [&](f16_t hi, f16_t lo) {
-              const float f = (float)hi;
-              return __float_as_uint(fabsf(f) <= 65504.0f ? __builtin_amdgcn_ldexpf(f + (float)lo, -ea[mb]) : f);
-            };
-            x[2 * i] = whole(h.x, l.x), x[2 * i + 1] = whole(h.y, l.y);
-          }
-          af[mb] = make_uint4(x[0], x[1], x[2], x[3]);
-        } else {
-          af[mb] = load_a(mb, ksub);
-        }
-      }
+      for (int mb = 0; mb < MB; ++mb) af[mb] = load_a(mb, ksub);
 #pragma unroll
       for (int nb = 0; nb < 2; ++nb) bf[nb] = load_b(nb, ksub);
 #pragma unroll
@@ -221,7 +203,7 @@ __global__ __launch_bounds__(TILE * 2, TILE == 128 ? 2 : 1) void bwd_colgrad_ker
   for (int c = 0; c < 4; ++c) {
     const int row = (wave * 4 + c) * 8 + (lane >> 3);
     const int ch = (lane & 7) ^ (row & 7);
-    a_src[c] = (const unsigned char *)a.wT +
+    a_src[c] = (const unsigned char *)(PAIRS ? a.wpair : a.wT) +
                ((long)grp * a.M_pad + (long)mt * TILE + row) * a.cout_g * ES + ch * 16;
     // rows past the image repeat its last pixel; they are never stored
     const int px = min(pt * TILE + row, a.P - 1);
@@ -282,7 +264,7 @@ __global__ __launch_bounds__(TILE * 2, TILE == 128 ? 2 : 1) void bwd_colgrad_ker
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       }
       __syncthreads();
-      tile_products<E, TILE, PLANES, PAIRS>(acc, As[buf], Bs[buf], wm, wn, frow, fhalf, ea, eb);
+      tile_products<E, TILE, PLANES, PAIRS && PLANES == 2>(acc, As[buf], Bs[buf], wm, wn, frow, fhalf, ea, eb);
       __syncthreads();
     }
   };
@@ -311,6 +293,11 @@ __global__ __launch_bounds__(TILE * 2, TILE == 128 ? 2 : 1) void bwd_colgrad_ker
       bad = unscale(acc);
     }
     if (__syncthreads_or(bad)) {
+      if constexpr (PAIRS) {
+        const long to_whole = (const unsigned char *)a.wT - (const unsigned char *)a.wpair;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) a_src[c] += to_whole;
+      }
       issue(0, 0);
       sweep(std::integral_constant<int, 0>());
     }

@@ -55,10 +55,10 @@ struct BwdPlan {
   // where the matrix-core paths have their copy of the input, and whether its channels are the input's own
   size_t xt_at() const { return gin_bytes + gb_bytes + mx_bytes; }
   bool plain_copy() const { return (gemm || wgemm) && im.segp == im.seg && im.cgp == im.cg; }
-  // fp32 column gradient of fp16 pairs: magnitudes of grad_output's pixels and exponents of the weights' rows, at max_at of the workspace (0: not
+  // fp32 column gradient of fp16 pairs: magnitudes of grad_output's pixels, exponents of the weights' rows and these as pairs, at max_at of the workspace (0: not
   // there, bf16 triples)
-  size_t gmax_bytes, wexp_bytes, max_at;
-  size_t max_bytes() const { return gmax_bytes + wexp_bytes; }
+  size_t gmax_bytes, wexp_bytes, wpair_bytes, max_at;
+  size_t max_bytes() const { return gmax_bytes + wexp_bytes + wpair_bytes; }
   size_t total() const {
     return gin_bytes + gw_bytes + gb_bytes + mx_bytes + xt_bytes + gt_bytes + wt_bytes + d_bytes + col_bytes + part_bytes +
            wpart_bytes + gpad_bytes;

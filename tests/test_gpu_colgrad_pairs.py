@@ -74,7 +74,7 @@ def _as_triples(dev, go):
     bp.grad_output = go.data_ptr()
     bp.grad_input, bp.grad_offset, bp.grad_mask = (t.data_ptr() for t in out)
     up = lambda v: (v + 255) // 256 * 256
-    need = lib.mdcn_backward_workspace_bytes(ctypes.byref(bp)) - up(2 * 4 * 33 * 37 * 2) - up(640 * 4)
+    need = lib.mdcn_backward_workspace_bytes(ctypes.byref(bp)) - up(2 * 4 * 33 * 37 * 2) - up(640 * 4) - up(640 * 128 * 4)
     ws = torch.empty(need, dtype=torch.uint8, device='cuda')
     p.workspace, p.workspace_bytes = ws.data_ptr(), need
     stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
