@@ -459,7 +459,7 @@ int run_backward_matrix(const mdcn_bwd_params *bp, const Geom &g, const BwdPlan 
         pl.gpad_bytes ? up((long)g.N * g.Cout * (pl.P_pad / EPV), 256) : 0,
         gemm ? up(n_in, kPreZeroPerBlock) : 0,
         wgemm && pl.P_pad > plane_out ? up(a.col_rows * (pl.P_pad - plane_out), kPrePadPerBlock) : 0,
-        gemm ? up((long)g.G * pl.M_pad * pl.om.cgp, 256) + (wexp ? up((long)g.G * pl.M_pad, kPrePairRows) : 0) : 0,
+        gemm ? wexp ? up((long)g.G * pl.M_pad, kPrePairRows) : up((long)g.G * pl.M_pad * pl.om.cgp, 256) : 0,
         gemm && pl.fWH ? far_blocks : 0,
         early ? 0 : bias_blocks,
     };

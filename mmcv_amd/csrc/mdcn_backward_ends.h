@@ -44,7 +44,7 @@ constexpr int kPrePairRows = 8;              // rows of wT a block writes as fp1
 constexpr int kPreZeroPerBlock = 256 * 32;   // floats a block of the zero job clears
 constexpr int kPrePadPerBlock = 256 * 8;     // elements a block of the col-pad job clears
 
-// fp32 as fp16 pairs: wpair is wT, its rows scaled by a power of two that goes by the largest finite number of each, and split.  The 32 values of a slab are four
+// fp32 as fp16 pairs: wT, and wpair, which is wT with its rows scaled by a power of two that goes by the largest finite number of each, and split.  The 32 values of a slab are four
 // times eight, which a lane of the product takes at a time: the first halves of eight in one 16-byte piece, the second ones in the piece two behind
 // it.  32 lanes a row, eight output channels each.
 __device__ __forceinline__ void pack_weight_row_pairs(const BwdPreArgs &a, int b) {
@@ -89,15 +89,21 @@ __device__ __forceinline__ void pack_weight_row_pairs(const BwdPreArgs &a, int b
   const int e = pair_exponent(__uint_as_float(top));
   if (lane == 0) a.wexp[row] = e;
   uint4 *dst = (uint4 *)a.wpair + row * (a.om.cgp / 4);
+  float4 *whole = (float4 *)a.wT + row * (a.om.cgp / 4);
   for (int o = lane; o < eights; o += 32) {
     if (o != lane) load(o, v);
+    const int at = (o >> 2) * 8 + (o >> 1 & 1) * 4 + (o & 1);
     float x[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) x[j] = __builtin_amdgcn_ldexpf(o == lane ? first[j] : v[j], e);
+    for (int j = 0; j < 8; ++j) x[j] = o == lane ? first[j] : v[j];
+    whole[at] = make_float4(x[0], x[1], x[2], x[3]);
+    whole[at + 2] = make_float4(x[4], x[5], x[6], x[7]);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] = __builtin_amdgcn_ldexpf(x[j], e);
     uint2 lo[2], hi[2];
     split2({x[0], x[1], x[2], x[3]}, lo);
     split2({x[4], x[5], x[6], x[7]}, hi);
-    uint4 *d = dst + (o >> 2) * 8 + (o >> 1 & 1) * 4 + (o & 1);
+    uint4 *d = dst + at;
     d[0] = make_uint4(lo[0].x, lo[0].y, hi[0].x, hi[0].y);
     d[2] = make_uint4(lo[1].x, lo[1].y, hi[1].x, hi[1].y);
   }
@@ -199,14 +205,13 @@ __global__ __launch_bounds__(256) void bwd_prepass_kernel(BwdPreArgs a) {
     // either channel is padding and in the rows up to M_pad.  With wt_run it is [G][run][M_pad][wt_run], the last run what is left: what
     // bwd_fused_kernel copies at a time is one piece of memory for a tap (256 bytes of rows 1 KB apart, as with
     // 512 output channels, are in one of four channels of the L2).
-    const long total = (long)g.G * a.M_pad * a.om.cgp;
     if constexpr (sizeof(E) == 4) {
-      const int pairs_from = a.end[kPreColPad] + (int)((total + 255) / 256);
-      if (a.wexp && b >= pairs_from) {
-        pack_weight_row_pairs(a, b - pairs_from);
+      if (a.wexp) {
+        pack_weight_row_pairs(a, b - a.end[kPreColPad]);
         return;
       }
     }
+    const long total = (long)g.G * a.M_pad * a.om.cgp;
     const long idx = (long)(b - a.end[kPreColPad]) * 256 + tid;
     if (idx >= total) return;
     long r = idx;
