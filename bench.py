@@ -39,8 +39,8 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 sys.path.insert(0, os.path.join(ROOT, 'tests'))
 
-# (fp32: a product is six products of bf16 planes on the bf16 matrix pipe; the fp32 MFMAs, 157 TFLOP/s, are not what runs)
-PEAK_TFLOPS = {'bf16': 2500.0, 'f16': 2500.0, 'f32': 2500.0 / 6}
+# (fp32: a product is three products of fp16 pairs on the 16-bit matrix pipe; the fp32 MFMAs, 157 TFLOP/s, are not what runs)
+PEAK_TFLOPS = {'bf16': 2500.0, 'f16': 2500.0, 'f32': 2500.0 / 3}
 HBM_PEAK_GBS = 8000.0
 # (workload, dominant kernel) -> (HBM bytes per launch from rocprofv3 counters, the profile they are in)
 TRAFFIC = {
